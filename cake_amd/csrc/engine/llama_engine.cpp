@@ -68,6 +68,13 @@ long long cake_gemm_ws_floats(int cfg, int splits, int M, int N, int K, int gate
 int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long long lda, const void* b,
               long long ldb, void* c, long long ldc, const void* bias, void* resid,
               long long ldr, float* ws, const void* zeros, int M, int N, int K, hipStream_t st);
+int cake_gemm_rows_kind(int M, long long Nv, int K, int gated);
+long long cake_gemm_rows_ws_floats(int M);
+int cake_gemm_rows_ticks();
+int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long lda, const void* b,
+                   long long ldb, void* c, long long ldc, const void* bias, void* resid,
+                   long long ldr, float* ws, void* tick, const void* zeros, int M, int N, int K,
+                   float alpha, hipStream_t st);
 int cake_blaslt_gemm(int dt, int out, const void* a, long long lda, const void* w, long long ldw,
                      void* c, long long ldc, int M, int N, int K, void* ws, size_t ws_bytes,
                      hipStream_t st);
@@ -808,6 +815,7 @@ class Llama {
   int* scratch_i32_ = nullptr;  // warm-up snapshot: tok, pos, hist_len
   float* scratch_resid_ = nullptr;
   int32_t* zeros_ = nullptr;    // 64 zero words (GEMM LDS-DMA padding source)
+  int32_t* ticks_ = nullptr;    // arrival counters of the few-row products, zero between launches
   // prefill buffers (grown to the longest prompt)
   int pre_T_ = 0;
   float* hidden_ = nullptr;
@@ -1031,11 +1039,13 @@ class Llama {
     scratch_i32_ = dalloc<int>(4);
     scratch_resid_ = dalloc<float>(c.H + 4);  // + the hop header (self-tests)
     zeros_ = dalloc<int32_t>(64);
+    ticks_ = dalloc<int32_t>(cake_gemm_rows_ticks());
     hip_check(hipMemset(tickets_, 0, sizeof(unsigned int) * (2 * c.nkv + 2)), "memset");
     hip_check(hipMemset(part_, 0, sizeof(float) * 2 * c.nh * kAttnMaxSplit * (c.hd + 2)), "memset");
     hip_check(hipMemset(sel_ticket_, 0, sizeof(unsigned int)), "memset");
     hip_check(hipMemset(slot_, 0, sizeof(unsigned long long)), "memset");
     hip_check(hipMemset(zeros_, 0, sizeof(int32_t) * 64), "memset");
+    hip_check(hipMemset(ticks_, 0, sizeof(int32_t) * cake_gemm_rows_ticks()), "memset");
     hip_check(hipMemset(hist_, 0, sizeof(int) * S_), "memset");
     hip_check(hipMemset(resid_, 0, sizeof(float) * (c.H + 4)), "memset");
     // opt-in (CAKE_ATTN_OPROJ=1): measured slower than the attention + o_proj pair on
@@ -1176,12 +1186,25 @@ class Llama {
     pre_T_ = T;
   }
 
+  void grow_ws(size_t need) {
+    if (need <= ws_n_) return;
+    dfree(ws_);
+    ws_ = dalloc<float>(need);
+    ws_n_ = need;
+  }
+
   void gemm(int epi, const void* a, long long lda, const void* b, long long ldb, void* cptr,
             long long ldc, float* resid, long long ldr, int M, int N, int K, const char* what) {
     const bool gated = epi == kEpiSwiglu;
     const long long Nv = gated ? 2LL * N : N;
     static const char* names[] = {"store", "resid32", "add16", "swiglu", "geglu", "partial",
                                   "store32"};
+    if (const int kind = cake_gemm_rows_kind(M, Nv, K, gated ? 1 : 0)) {  // few rows
+      if (kind == 2) grow_ws((size_t)cake_gemm_rows_ws_floats(M));
+      k_check(cake_gemm_rows(dt_, epi, kind, a, lda, b, ldb, cptr, ldc, nullptr, resid, ldr, ws_,
+                             ticks_, zeros_, M, N, K, 1.f, st_), what);
+      return;
+    }
     auto p = planner_.plan(M, Nv, K, names[epi]);
     if (p.first == kGemmLib) {  // the table names the library GEMM (CAKE_GEMM_LIB=1 only)
       if ((epi != kEpiSwiglu || ldc == N) &&
@@ -1193,12 +1216,7 @@ class Llama {
     const int splits = p.second;
     float* ws = nullptr;
     if (splits > 1) {
-      const size_t need = (size_t)cake_gemm_ws_floats(p.first, splits, M, N, K, gated ? 1 : 0);
-      if (need > ws_n_) {
-        dfree(ws_);
-        ws_ = dalloc<float>(need);
-        ws_n_ = need;
-      }
+      grow_ws((size_t)cake_gemm_ws_floats(p.first, splits, M, N, K, gated ? 1 : 0));
       ws = ws_;
     }
     k_check(cake_gemm(dt_, epi, p.first, splits, a, lda, b, ldb, cptr, ldc, nullptr, resid, ldr,

@@ -36,6 +36,9 @@
 //     are read in a virtual order that interleaves 16-row blocks of the two
 //     halves, so gate and up of one feature land in the same lane.
 #include "gemm_kernel.h"
+#include "gemm_rows.h"
+
+#include <algorithm>
 
 namespace cake {
 // the launchers are instantiated in gemm_inst_{bf16,f16}_{a,b}.hip
@@ -47,6 +50,20 @@ CAKE_GEMM_EXTERN_ALL(kBF16)
 CAKE_GEMM_EXTERN_ALL(kF16)
 #undef CAKE_GEMM_EXTERN_ALL
 #undef CAKE_GEMM_EXTERN
+// ... and in gemm_inst_rows_{bf16,f16}.hip
+#define CAKE_ROWS_EXTERN(DT)                                                              \
+  extern template int launch_rows<DT, kEpiStore>(int, int, dim3, hipStream_t, const GemmArgs&);   \
+  extern template int launch_rows<DT, kEpiResid32>(int, int, dim3, hipStream_t, const GemmArgs&); \
+  extern template int launch_rows<DT, kEpiAdd16>(int, int, dim3, hipStream_t, const GemmArgs&);   \
+  extern template int launch_rows<DT, kEpiSwiglu>(int, int, dim3, hipStream_t, const GemmArgs&);  \
+  extern template int launch_rows<DT, kEpiGeglu>(int, int, dim3, hipStream_t, const GemmArgs&);   \
+  extern template int launch_rows<DT, kEpiStore32>(int, int, dim3, hipStream_t, const GemmArgs&); \
+  extern template int launch_rows<DT, kEpiSilu>(int, int, dim3, hipStream_t, const GemmArgs&);    \
+  extern template int launch_rows_grouped<DT, kEpiStore>(int, dim3, hipStream_t, const GemmArgs&); \
+  extern template int launch_rows_grouped<DT, kEpiSilu>(int, dim3, hipStream_t, const GemmArgs&);
+CAKE_ROWS_EXTERN(kBF16)
+CAKE_ROWS_EXTERN(kF16)
+#undef CAKE_ROWS_EXTERN
 }  // namespace cake
 
 using namespace cake;
@@ -220,4 +237,131 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
                        int K, hipStream_t st) {
   return cake_gemm_scaled(dt, epi, cfg, splits, a, lda, b, ldb, c, ldc, bias, resid, ldr, ws,
                           zeros, M, N, K, 1.f, st);
+}
+
+// ---- products of few rows (gemm_rows.h) -----------------------------------
+// Which form a product of M rows takes: 0 the tile kernels (cake_gemm_scaled), 1 direct, 2 stream.
+// The estimates (us) are fits to timings on weights that no cache holds, 5 .. 64 rows, weight
+// matrices of 8 .. 260 MB; both sides of the lines they draw, measured: 4096 x 4096 at 16 rows
+// direct 11.5, stream 14.4; 4096 x 14336 direct 35, stream 25; 28672 x 4096 at 45 rows stream 53,
+// tiles 58; 4096 x 4096 at 45 rows stream 19, tiles 17.
+static int rows_kind(int M, long long Nv, int K, bool gated) {
+  if (M > 64 || Nv > 128LL * kRowsTicks) return 0;
+  const double kb = K * 2e-3;   // KB of one row of k
+  const int mt = (M + 15) / 16;
+  const double tiles = 8 + Nv * kb / 4600;
+  const long long strips = (Nv + 127) / 128, ks = (K + 63) / 64, total = strips * ks;
+  const long long per = std::max<long long>((total + kRowsWgs - 1) / kRowsWgs, kRowsMinSteps);
+  const double stream = 7 + (ks > per || ks % per ? 0.7 * mt : 0.) + per * (16 + 2 * mt) / 27.;
+  double direct = 1e9;
+  if (M <= 32) {
+    const int nt = gated || Nv > 4096 ? 2 : 1;
+    const long long wgs = (Nv + 16 * nt - 1) / (16 * nt);
+    // a CU's share at 32 KB a us, all weights and half of the reads of x at 5.8 MB a us
+    direct = 4 + std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / 32,
+                          (Nv + 0.5 * wgs * M) * kb / 5800);
+  }
+  if (direct <= stream && direct <= tiles) return 1;
+  return stream < tiles ? 2 : 0;
+}
+CAKE_API int cake_gemm_rows_kind(int M, long long Nv, int K, int gated) {
+  return M < 1 || Nv < 1 || K < 1 ? 0 : rows_kind(M, Nv, K, gated != 0);
+}
+
+// stream form: f32 elements of ws (two parked strips per share) and counters of tick
+CAKE_API long long cake_gemm_rows_ws_floats(int M) { return (long long)kRowsWgs * 4096 * ((M + 15) / 16); }
+CAKE_API int cake_gemm_rows_ticks() { return kRowsTicks; }
+
+// cake_gemm_scaled for M <= 64 rows in the form `kind` (1 or 2).  The stream form needs ws
+// (cake_gemm_rows_ws_floats) and tick (cake_gemm_rows_ticks zeros, zero again when the launch is
+// done): both belong to one launch at a time, so to one stream.
+CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long lda, const void* b,
+                            long long ldb, void* c, long long ldc, const void* bias, void* resid,
+                            long long ldr, float* ws, void* tick, const void* zeros, int M, int N,
+                            int K, float alpha, hipStream_t st) {
+  if (alpha != 1.f && epi != kEpiResid32 && epi != kEpiStore32) return (int)hipErrorInvalidValue;
+  int act = 0;
+  if (epi >= 8 && epi <= 10) {
+    act = epi - 7;
+    epi = kEpiSilu;
+  }
+  const bool gated = (epi == kEpiSwiglu || epi == kEpiGeglu);
+  if (M < 1 || M > 64 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || (gated && N % 16) ||
+      !(kind == 1 || kind == 2) || (kind == 1 && M > 32) || (kind == 2 && (!ws || !tick || !zeros)))
+    return (int)hipErrorInvalidValue;
+  GemmArgs g{};
+  g.a = (const uint16_t*)a; g.b = (const uint16_t*)b; g.c = (uint16_t*)c;
+  g.bias = (const uint16_t*)bias;
+  g.r32 = (epi == kEpiResid32 || epi == kEpiStore32) ? (float*)resid : nullptr;
+  g.r16 = (epi == kEpiAdd16) ? (const uint16_t*)resid : nullptr;
+  g.ws = ws; g.tick = (unsigned*)tick; g.zeros = (const uint16_t*)zeros;
+  g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.ldr = ldr;
+  g.M = M; g.N = N; g.K = K;
+  g.gated = gated ? 1 : 0;
+  g.act = act;
+  g.alpha = alpha;
+  g.half = N;
+  g.Nv = gated ? 2 * N : N;
+  g.tiles_m = 1;
+  const int mt = (M + 15) / 16;
+  int form, wgs;
+  if (kind == 2) {
+    g.tiles_n = (g.Nv + 127) / 128;
+    if (g.tiles_n > kRowsTicks) return (int)hipErrorInvalidValue;
+    g.kps = kRowsMinSteps;
+    const long long total = (long long)g.tiles_n * ((K + 63) / 64);
+    form = 2;
+    wgs = (int)std::min<long long>(kRowsWgs, (total + kRowsMinSteps - 1) / kRowsMinSteps);
+  } else {
+    const int nt = gated || g.Nv > 4096 ? 2 : 1;   // one 16-row strip per CU, or two
+    form = nt - 1;
+    wgs = (g.Nv + 16 * nt - 1) / (16 * nt);
+  }
+  const auto run = [&](auto dtc) {
+    constexpr int DT = decltype(dtc)::value;
+    switch (epi) {
+      case kEpiStore: return launch_rows<DT, kEpiStore>(form, mt, dim3(wgs), st, g);
+      case kEpiResid32: return launch_rows<DT, kEpiResid32>(form, mt, dim3(wgs), st, g);
+      case kEpiAdd16: return launch_rows<DT, kEpiAdd16>(form, mt, dim3(wgs), st, g);
+      case kEpiSwiglu: return launch_rows<DT, kEpiSwiglu>(form, mt, dim3(wgs), st, g);
+      case kEpiGeglu: return launch_rows<DT, kEpiGeglu>(form, mt, dim3(wgs), st, g);
+      case kEpiStore32: return launch_rows<DT, kEpiStore32>(form, mt, dim3(wgs), st, g);
+      case kEpiSilu: return launch_rows<DT, kEpiSilu>(form, mt, dim3(wgs), st, g);
+    }
+    return (int)hipErrorInvalidValue;
+  };
+  return dt == kBF16 ? run(std::integral_constant<int, kBF16>{})
+         : dt == kF16 ? run(std::integral_constant<int, kF16>{}) : (int)hipErrorInvalidValue;
+}
+
+// cake_gemm_grouped in the stream form: tiles of at most 16 rows; ws and tick as above (ws of 16
+// rows), max_tiles strips of N within the counters
+CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long lda, const void* b,
+                                    long long ldb, long long b_group, void* c, long long ldc,
+                                    const void* tiles, int max_tiles, float* ws, void* tick,
+                                    const void* zeros, int N, int K, hipStream_t st) {
+  const long long strips = (long long)max_tiles * ((N + 127) / 128);
+  if (max_tiles <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || b_group % 8 ||
+      !(epi == 0 || (epi >= 7 && epi <= 10)) || !ws || !tick || !zeros || strips > kRowsTicks ||
+      strips * ((K + 63) / 64) >= 0x40000000LL)
+    return (int)hipErrorInvalidValue;
+  GemmArgs g{};
+  g.a = (const uint16_t*)a; g.b = (const uint16_t*)b; g.c = (uint16_t*)c;
+  g.ws = ws; g.tick = (unsigned*)tick; g.zeros = (const uint16_t*)zeros;
+  g.lda = lda; g.ldb = ldb; g.ldc = ldc;
+  g.N = N; g.K = K; g.Nv = N; g.half = N;
+  g.act = epi ? epi - 7 : 0;
+  g.tiles_m = max_tiles;
+  g.tiles_n = (N + 127) / 128;
+  g.kps = kRowsMinSteps;
+  g.groups = (const int4*)tiles;
+  g.b_group = b_group;
+  const dim3 grid(kRowsWgs);
+  if (epi == 0)
+    return dt == kBF16 ? launch_rows_grouped<kBF16, kEpiStore>(1, grid, st, g)
+           : dt == kF16 ? launch_rows_grouped<kF16, kEpiStore>(1, grid, st, g)
+                        : (int)hipErrorInvalidValue;
+  return dt == kBF16 ? launch_rows_grouped<kBF16, kEpiSilu>(1, grid, st, g)
+         : dt == kF16 ? launch_rows_grouped<kF16, kEpiSilu>(1, grid, st, g)
+                      : (int)hipErrorInvalidValue;
 }

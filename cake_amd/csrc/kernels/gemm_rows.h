@@ -1,0 +1,492 @@
+// Products of few rows (M <= 64): short prompts, one token of several sequences, routed experts.
+// The weights are read once and little is done with each of them, so the time is their bytes (and
+// a launch's fixed costs); two forms, chosen by gemm.hip rows_kind from the sizes.
+//
+// gemm_direct_kernel (M <= 32, weights up to some 60 MB): a workgroup owns 16 or 32 weight rows over
+//   the whole of k, its eight waves taking 64-element chunks of k in turn, operands straight into
+//   MFMA fragments; the waves' sums meet in LDS.  No partial sums in memory, no second launch, no
+//   barrier in the loop: 4096 x 4096 at 5 / 16 rows 9.7 / 11.5 us (tile kernel with split k and its
+//   finalize launch: 15-17 us), 2048 x 2048 6.1 / 7.1 us (14.6 us).  Every strip reads all of x
+//   from L2, which is what ends its range.
+// gemm_stream_kernel (M <= 64): 128 weight rows and the x tile go through LDS by DMA, 64 k per
+//   step; the steps of all strips form one sequence dealt out in equal contiguous shares, one
+//   workgroup per CU, so no last wave is left and the DMA never stops at a strip's end.  Strips
+//   that several shares cover meet in memory, the last to arrive sums in share order (the result
+//   does not hang on the order).  28672 x 4096 SwiGLU at 13 / 24 / 45 rows 44 / 46 / 53 us (tile
+//   kernels 58-60 us), 4096 x 23552 35 / 37 / 42 us (44-46 us).  The DMA moves 7 TB/s, L2 hits of
+//   x included, at any depth from three stages on, with 128 or 256 weight rows per strip and with
+//   one or two workgroups per CU alike: fewer x bytes per weight byte is what would speed it up.
+#pragma once
+#include "gemm_kernel.h"
+
+namespace cake {
+
+constexpr int kRowsWgs = 256;        // shares of the stream form (one per CU)
+constexpr int kRowsMinSteps = 8;     // steps of a share at least
+constexpr int kRowsTicks = 32768;    // strips of a launch at most (arrival counters)
+
+// the operand fragments of one 64-element chunk of k: a lane's two 16-byte pieces of each row are
+// neighbours, so the two MFMA steps read whole 128-byte lines (both operands use one order of k)
+template <int DT, int MT, int NT>
+struct DirectChunk {
+  uint4 w[NT][2], x[MT][2];
+
+  __device__ __forceinline__ void load(const uint16_t* const* wp, const uint16_t* const* xp, int k) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) w[j][h] = ld_nt16(reinterpret_cast<const uint4*>(wp[j] + k) + h);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) x[i][h] = reinterpret_cast<const uint4*>(xp[i] + k)[h];
+  }
+
+  // the last, short chunk: pieces past the end are zero in both operands
+  __device__ __forceinline__ void load_tail(const uint16_t* const* wp, const uint16_t* const* xp, int k,
+                                            int left) {
+    const uint4 z = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool in = h * 8 < left;   // left: elements of the row from this lane's first piece on
+#pragma unroll
+      for (int j = 0; j < NT; ++j) w[j][h] = in ? reinterpret_cast<const uint4*>(wp[j] + k)[h] : z;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) x[i][h] = in ? reinterpret_cast<const uint4*>(xp[i] + k)[h] : z;
+    }
+  }
+
+  __device__ __forceinline__ void mac(cf32x4 (&acc)[NT][MT]) const {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = cmfma<DT>(w[j][h], x[i][h], acc[j][i]);
+  }
+};
+
+template <int DT, int EPI, int MT, int NT>
+__global__ __launch_bounds__(512) void gemm_direct_kernel(GemmArgs g) {
+  constexpr bool GATED = (EPI == kEpiSwiglu || EPI == kEpiGeglu);
+  constexpr int NW = 8, D = 2;   // waves, chunks in flight of each
+  constexpr int TILES = NT * MT;
+  constexpr int GRP = TILES * NW <= 64 ? TILES : 64 / NW;   // tiles summed per round (<= 64 KB)
+  static_assert(TILES % GRP == 0 && (!GATED || (NT == 2 && GRP % 2 == 0)), "direct tile groups");
+  __shared__ float4 red[NW][GRP][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int v0 = blockIdx.x * NT * 16;
+
+  const int r = lane & 15, kq = (lane >> 4) * 16;
+  const uint16_t *wp[NT], *xp[MT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    wp[j] = g.b + (size_t)wrow(g, min(v0 + j * 16 + r, g.Nv - 1)) * g.ldb + kq;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xp[i] = g.a + (size_t)min(i * 16 + r, g.M - 1) * g.lda + kq;
+
+  cf32x4 acc[NT][MT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[j][i] = cf32x4{0.f, 0.f, 0.f, 0.f};
+
+  // wave w takes chunks w, w + NW, .. of the workgroup's whole ones, D of them in flight
+  const int nfull = g.K / 64;
+  const int mine = nfull > wave ? (nfull - wave + NW - 1) / NW : 0;
+  const int k = wave * 64;
+  DirectChunk<DT, MT, NT> buf[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < mine) buf[d].load(wp, xp, k + d * NW * 64);
+  int c = 0;
+  for (; c + 2 * D <= mine; c += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      buf[d].mac(acc);
+      buf[d].load(wp, xp, k + (c + D + d) * NW * 64);
+    }
+  }
+  for (; c < mine; c += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (c + d < mine) {
+        buf[d].mac(acc);
+        if (c + D + d < mine) buf[d].load(wp, xp, k + (c + D + d) * NW * 64);
+      }
+  }
+  const int rest = g.K - nfull * 64;
+  if (rest > 0 && wave == nfull % NW) {
+    DirectChunk<DT, MT, NT> t;
+    t.load_tail(wp, xp, nfull * 64, rest - kq);
+    t.mac(acc);
+  }
+
+  // the waves' sums meet in LDS; item = (tile, lane): token i * 16 + (lane & 15), four weight rows
+#pragma unroll
+  for (int t0 = 0; t0 < TILES; t0 += GRP) {
+    // tile t = i * NT + j, so the two halves of a gated pair are neighbours
+#pragma unroll
+    for (int t = 0; t < GRP; ++t) {
+      const cf32x4 a = acc[(t0 + t) % NT][(t0 + t) / NT];
+      red[wave][t][lane] = make_float4(a[0], a[1], a[2], a[3]);
+    }
+    __syncthreads();
+    constexpr int STEP = GATED ? 2 : 1;
+    for (int it = threadIdx.x; it < GRP / STEP * 64; it += NW * 64) {
+      const int t = it / 64 * STEP, l = it % 64;
+      float s[STEP][4];
+#pragma unroll
+      for (int q = 0; q < STEP; ++q) {
+        float4 a = red[0][t + q][l];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+          const float4 b = red[w][t + q][l];
+          a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+        }
+        s[q][0] = a.x; s[q][1] = a.y; s[q][2] = a.z; s[q][3] = a.w;
+      }
+      const int i = (t0 + t) / NT, j = (t0 + t) % NT;
+      const int m = i * 16 + (l & 15);
+      if (m >= g.M) continue;
+      const int n = (GATED ? blockIdx.x * 16 : v0 + j * 16) + (l >> 4) * 4;
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int nn = min(n + e, g.N - 1);
+        float a = s[0][e] + (g.bias != nullptr ? to_f32<DT>(g.bias[nn]) : 0.f);
+        if constexpr (GATED) {
+          const float b = s[STEP - 1][e] + (g.bias != nullptr ? to_f32<DT>(g.bias[g.half + nn]) : 0.f);
+          a = EPI == kEpiSwiglu ? silu(a) * b : a * gelu_tanh(b);
+        }
+        if constexpr (EPI == kEpiAdd16) a += to_f32<DT>(g.r16[(size_t)m * g.ldr + nn]);
+        if constexpr (EPI == kEpiSilu) a = gemm_act(g.act, a);
+        y[e] = a;
+      }
+      if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32) {
+        float* o = g.r32 + (size_t)m * g.ldr + n;
+        if (n + 4 <= g.N && ((g.ldr | n) & 3) == 0) {
+          float4 v = EPI == kEpiResid32 ? *reinterpret_cast<float4*>(o) : make_float4(0.f, 0.f, 0.f, 0.f);
+          v.x = fmaf(g.alpha, y[0], v.x); v.y = fmaf(g.alpha, y[1], v.y);
+          v.z = fmaf(g.alpha, y[2], v.z); v.w = fmaf(g.alpha, y[3], v.w);
+          *reinterpret_cast<float4*>(o) = v;
+        } else {
+          for (int e = 0; e < 4; ++e)
+            if (n + e < g.N) o[e] = fmaf(g.alpha, y[e], EPI == kEpiResid32 ? o[e] : 0.f);
+        }
+      } else {
+        uint16_t* o = g.c + (size_t)m * g.ldc + n;
+        for (int e = 0; e < 4; ++e)
+          if (n + e < g.N) o[e] = from_f32<DT>(y[e]);
+      }
+    }
+    if (t0 + GRP < TILES) __syncthreads();
+  }
+}
+
+// MT: 16-row tiles of x.  A stage holds 16 KB of weights and 2 MT KB of x.
+template <int MT> struct StreamShape {
+  static constexpr int NWV = 4;
+  static constexpr int BN = NWV * 32;               // weight rows of a strip
+  static constexpr int NS = 4;
+  static constexpr int XW = MT == 1 ? 2 : MT == 3 ? 3 : 4;   // waves that fetch x
+  static constexpr int XI = MT * 2 / XW;              // their x DMA instructions per step
+  static constexpr int IPW = 4 + XI;
+  static constexpr int STAGE = (BN + MT * 16) * 128;
+};
+
+// N 16-row fragments (both halves of k) at base + 2048 i; waits for them
+template <int N>
+__device__ __forceinline__ void stream_read(uint32_t lo, uint32_t hi, uint4 (&a)[N][2]) {
+  static_assert(N == 1 || N == 2, "fragments per read");
+  if constexpr (N == 2)
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:2048\n\t"
+                 "ds_read_b128 %3, %5 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1])
+                 : "v"(lo), "v"(hi) : "memory");
+  else
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[0][1]) : "v"(lo), "v"(hi) : "memory");
+}
+
+struct StreamStrip {   // one strip of the step sequence
+  const uint16_t *a, *b;
+  uint16_t* c;
+  int M, v0;
+};
+
+template <bool GRP, int BN>
+__device__ __forceinline__ StreamStrip stream_strip(const GemmArgs& g, int s) {
+  StreamStrip r{g.a, g.b, g.c, g.M, s * BN};
+  if constexpr (GRP) {
+    const int4 t = g.groups[s / g.tiles_n];
+    r.a += (size_t)t.y * g.lda;
+    r.c += (size_t)t.y * g.ldc;
+    r.b += (size_t)t.x * g.b_group;
+    r.M = t.z;
+    r.v0 = (s % g.tiles_n) * BN;
+  }
+  return r;
+}
+
+// epilogue of one wave's sums: acc[j][i][e] is token 16 i + (lane & 15), virtual weight row
+// v0 + 32 wave + 16 j + 4 (lane >> 4) + e
+template <int DT, int EPI, int MT>
+__device__ __forceinline__ void stream_store(const GemmArgs& g, const StreamStrip& s, int wave, int lane,
+                                             const cf32x4 (&acc)[2][MT]) {
+  constexpr bool GATED = (EPI == kEpiSwiglu || EPI == kEpiGeglu);
+  const int vw = s.v0 + wave * 32;
+#pragma unroll
+  for (int j = 0; j < (GATED ? 1 : 2); ++j) {
+    const int n = (GATED ? vw / 2 : vw + j * 16) + (lane >> 4) * 4;
+    if (n >= g.N) continue;
+    const bool full = n + 4 <= g.N;
+    float b0[4], b1[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int nn = min(n + e, g.N - 1);
+      b0[e] = g.bias != nullptr ? to_f32<DT>(g.bias[nn]) : 0.f;
+      b1[e] = GATED && g.bias != nullptr ? to_f32<DT>(g.bias[g.half + nn]) : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = i * 16 + (lane & 15);
+      if (m >= s.M) continue;
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float a = acc[j][i][e] + b0[e];
+        if constexpr (GATED) {
+          const float u = acc[1][i][e] + b1[e];
+          a = EPI == kEpiSwiglu ? silu(a) * u : a * gelu_tanh(u);
+        }
+        if constexpr (EPI == kEpiAdd16) a += to_f32<DT>(g.r16[(size_t)m * g.ldr + min(n + e, g.N - 1)]);
+        if constexpr (EPI == kEpiSilu) a = gemm_act(g.act, a);
+        y[e] = a;
+      }
+      if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32) {
+        constexpr bool ADD = EPI == kEpiResid32;
+        float* o = g.r32 + (size_t)m * g.ldr + n;
+        if (full && ((g.ldr | n) & 3) == 0) {
+          float4 v = ADD ? *reinterpret_cast<float4*>(o) : make_float4(0.f, 0.f, 0.f, 0.f);
+          v.x = fmaf(g.alpha, y[0], v.x); v.y = fmaf(g.alpha, y[1], v.y);
+          v.z = fmaf(g.alpha, y[2], v.z); v.w = fmaf(g.alpha, y[3], v.w);
+          *reinterpret_cast<float4*>(o) = v;
+        } else {
+          for (int e = 0; e < 4; ++e)
+            if (n + e < g.N) o[e] = fmaf(g.alpha, y[e], ADD ? o[e] : 0.f);
+        }
+      } else {
+        uint16_t* o = s.c + (size_t)m * g.ldc + n;
+        uint16_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = from_f32<DT>(y[e]);
+        if (full && ((g.ldc | n) & 3) == 0 && ((uintptr_t)s.c & 7) == 0)
+          *reinterpret_cast<uint2*>(o) = make_uint2(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16);
+        else
+          for (int e = 0; e < 4; ++e) if (n + e < g.N) o[e] = v[e];
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ void park(float* p, const cf32x4& v) {
+  const unsigned long long lo = (unsigned long long)__float_as_uint(v[1]) << 32 | __float_as_uint(v[0]);
+  const unsigned long long hi = (unsigned long long)__float_as_uint(v[3]) << 32 | __float_as_uint(v[2]);
+  unsigned long long* q = reinterpret_cast<unsigned long long*>(p);
+  __hip_atomic_store(q, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ cf32x4 unpark(const float* p) {
+  const unsigned long long* q = reinterpret_cast<const unsigned long long*>(p);
+  const unsigned long long lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return cf32x4{__uint_as_float((unsigned)lo), __uint_as_float((unsigned)(lo >> 32)),
+                __uint_as_float((unsigned)hi), __uint_as_float((unsigned)(hi >> 32))};
+}
+
+template <int DT, int EPI, int MT, bool GRP>
+__global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
+  using S = StreamShape<MT>;
+  constexpr int NWV = S::NWV;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[S::NS * S::STAGE];
+  __shared__ unsigned last;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int KS = (g.K + 63) / 64;
+  const int strips = (GRP ? g.groups[g.tiles_m].x : 1) * g.tiles_n;
+  const int total = strips * KS;
+  const int per = max((total + (int)gridDim.x - 1) / (int)gridDim.x, g.kps);
+  // neighbouring shares on one XCD (they read one strip's x and meet in its sums)
+  const int nwg = gridDim.x, q8 = nwg / 8, r8 = nwg % 8, x8 = blockIdx.x % 8;
+  const int wg = (x8 < r8 ? x8 * (q8 + 1) : r8 * (q8 + 1) + (x8 - r8) * q8) + blockIdx.x / 8;
+  const int u0 = wg * per, u1 = min(total, u0 + per);
+  if (u0 >= u1) return;
+
+  // ---- DMA: wave w fetches weight rows 32 w .. and its share of x ----
+  const int dr = lane >> 3;                 // row within an instruction's 8
+  int ds = u0 / KS, dk = u0 % KS, dnext = u0;
+  const uint16_t *wsrc[4], *xsrc[S::XI];
+  auto aim = [&](int s) {
+    const StreamStrip t = stream_strip<GRP, S::BN>(g, s);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = wave * 32 + i * 8 + dr;
+      const int v = t.v0 + row, ch = (lane & 7) ^ ((row >> 1) & 7);
+      wsrc[i] = v < g.Nv ? t.b + (size_t)wrow(g, v) * g.ldb + ch * 8 : nullptr;
+    }
+#pragma unroll
+    for (int i = 0; i < S::XI; ++i) {
+      const int row = (wave % S::XW * S::XI + i) * 8 + dr;
+      const int ch = (lane & 7) ^ ((row >> 1) & 7);
+      xsrc[i] = t.a + (size_t)min(row, t.M - 1) * g.lda + ch * 8;
+    }
+  };
+  aim(ds);
+  auto stage = [&](int buf) {
+    uint8_t* b = smem + buf * S::STAGE;
+    const bool live = dnext < u1;
+    const int k = dk * 64;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = wave * 32 + i * 8 + dr, ch = (lane & 7) ^ ((row >> 1) & 7);
+      const uint16_t* p = live && wsrc[i] != nullptr && k + ch * 8 < g.K ? wsrc[i] + k : g.zeros;
+      __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(b + (wave * 4 + i) * 1024), 16, 0, 2);
+    }
+    if (S::XW == NWV || wave < S::XW)
+#pragma unroll
+    for (int i = 0; i < S::XI; ++i) {
+      const int r0 = wave * S::XI + i;
+      const int row = r0 * 8 + dr, ch = (lane & 7) ^ ((row >> 1) & 7);
+      const uint16_t* p = live && k + ch * 8 < g.K ? xsrc[i] + k : g.zeros;
+      glds16(p, b + (NWV * 4 + r0) * 1024);
+    }
+    ++dnext;
+    if (++dk == KS) {
+      dk = 0;
+      ++ds;
+      if (dnext < u1) aim(ds);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < S::NS - 1; ++p) stage(p);
+
+  const int swz = (lane & 15) >> 1;
+  const uint32_t lrow = (uint32_t)(lane & 15) * 128;
+  const uint32_t off0 = (uint32_t)(((lane >> 4) ^ swz) * 16), off1 = (uint32_t)(((4 + (lane >> 4)) ^ swz) * 16);
+  const uint32_t lds0 = lds_off(smem) + lrow;
+
+  cf32x4 acc[2][MT];
+  int buf = 0, u = u0;
+  while (u < u1) {
+    const int s = u / KS, seg1 = min(u1, (s + 1) * KS);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[j][i] = cf32x4{0.f, 0.f, 0.f, 0.f};
+    for (; u < seg1; ++u) {
+      if (S::XW == NWV || wave < S::XW) __builtin_amdgcn_s_waitcnt(vm_wait((S::NS - 2) * S::IPW));
+      else __builtin_amdgcn_s_waitcnt(vm_wait((S::NS - 2) * 4));
+      asm volatile("s_barrier" ::: "memory");
+      // every wave has read the previous step's stage: it takes the step NS - 1 ahead
+      stage(buf == 0 ? S::NS - 1 : buf - 1);
+      const uint32_t b = lds0 + buf * S::STAGE;
+      uint4 w[2][2];
+      stream_read<2>(b + wave * 4096 + off0, b + wave * 4096 + off1, w);
+      constexpr int XR = MT % 2 ? 1 : 2;
+#pragma unroll
+      for (int i = 0; i < MT; i += XR) {
+        uint4 x[XR][2];
+        stream_read<XR>(b + NWV * 4096 + i * 2048 + off0, b + NWV * 4096 + i * 2048 + off1, x);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int p = 0; p < XR; ++p)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[j][i + p] = cmfma<DT>(w[j][h], x[p][h], acc[j][i + p]);
+      }
+      buf = buf + 1 == S::NS ? 0 : buf + 1;
+    }
+    const StreamStrip t = stream_strip<GRP, S::BN>(g, s);
+    const int lo = s * KS / per, hi = ((s + 1) * KS - 1) / per;   // shares with steps of this strip
+    bool mine = lo == hi;
+    if (lo != hi) {
+      auto slot = [&](int w) {   // a share's first strip, or its last
+        return g.ws + ((size_t)(2 * w + (w * per / KS == s ? 0 : 1)) * NWV + wave) * (2 * MT * 256) + lane * 4;
+      };
+      float* p = slot(wg);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          if (i * 16 + (lane & 15) < t.M) park(p + (j * MT + i) * 256, acc[j][i]);
+      __builtin_amdgcn_s_waitcnt(vm_wait(0));
+      asm volatile("s_barrier" ::: "memory");
+      if (tid == 0)
+        last = __hip_atomic_fetch_add(g.tick + s, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(hi - lo);
+      __syncthreads();
+      mine = last != 0;
+      if (mine) {
+        if (tid == 0) __hip_atomic_store(g.tick + s, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // in share order (the result does not hang on who came last), several shares in flight
+        constexpr int UN = MT <= 2 ? 8 : 4;
+        for (int w0 = lo; w0 <= hi; w0 += UN) {
+          cf32x4 o[UN][2][MT];
+#pragma unroll
+          for (int q = 0; q < UN; ++q) {
+            const float* p = slot(min(w0 + q, hi));
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int i = 0; i < MT; ++i)
+                o[q][j][i] = i * 16 + (lane & 15) < t.M ? unpark(p + (j * MT + i) * 256) : cf32x4{0.f, 0.f, 0.f, 0.f};
+          }
+#pragma unroll
+          for (int q = 0; q < UN; ++q)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int i = 0; i < MT; ++i) {
+                if (q == 0 && w0 == lo) acc[j][i] = o[0][j][i];
+                else if (w0 + q <= hi) acc[j][i] += o[q][j][i];
+              }
+        }
+      }
+      __syncthreads();
+    }
+    if (mine) stream_store<DT, EPI, MT>(g, t, wave, lane, acc);
+    // stores count with the DMA: drain them before the counted waits go on
+    if (u < u1) __builtin_amdgcn_s_waitcnt(vm_wait(0));
+  }
+  __builtin_amdgcn_s_waitcnt(vm_wait(0));
+}
+
+template <int DT, int EPI>
+int launch_rows(int kind, int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
+#define CAKE_STREAM(MT)                                                                             \
+  if (kind == 2 && mt == MT) {                                                                      \
+    hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI, MT, false>), grid, dim3(256), 0, st, g);        \
+    return (int)hipGetLastError();                                                                  \
+  }
+  CAKE_STREAM(1) CAKE_STREAM(2) CAKE_STREAM(3) CAKE_STREAM(4)
+#undef CAKE_STREAM
+  constexpr bool GATED = (EPI == kEpiSwiglu || EPI == kEpiGeglu);
+#define CAKE_DIRECT(KIND, MT, NT)                                                                   \
+  if constexpr (!GATED || NT == 2)                                                                  \
+    if (kind == KIND && mt == MT) {                                                                 \
+      hipLaunchKernelGGL((gemm_direct_kernel<DT, EPI, MT, NT>), grid, dim3(512), 0, st, g);         \
+      return (int)hipGetLastError();                                                                \
+    }
+  CAKE_DIRECT(0, 1, 1) CAKE_DIRECT(0, 2, 1) CAKE_DIRECT(1, 1, 2) CAKE_DIRECT(1, 2, 2)
+#undef CAKE_DIRECT
+  return (int)hipErrorInvalidValue;
+}
+
+// rows sorted by weight group (GemmArgs::groups), at most 16 MT of them per tile
+template <int DT, int EPI>
+int launch_rows_grouped(int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  if (mt != 1) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI, 1, true>), grid, dim3(256), 0, st, g);
+  return (int)hipGetLastError();
+}
+
+}  // namespace cake

@@ -46,7 +46,7 @@ def plan(ids, score, E: int, dtype) -> Plan:
     N, top = ids.shape
     _routing(E, top)
     M, dev = N * top, ids.device
-    cfg = G.grouped_cfg(M, E)
+    cfg = G.grouped_cfg(M, E, torch.cuda.is_current_stream_capturing())
     bm = BM32 if dtype == torch.float32 else G.GROUPED_CFGS[cfg]
     n = M // bm + min(E, M)
     i32 = torch.empty(2 * M + 4 * (n + 1) + 4, device=dev, dtype=torch.int32)

@@ -67,6 +67,17 @@ def _lib():
         lib.cake_gemm_ws_floats.restype = L
         lib.cake_gemm_grouped.argtypes = [I, I, I, P, L, P, L, L, P, L, P, I, P, I, I, P]
         lib.cake_gemm_grouped.restype = I
+        lib.cake_gemm_rows_kind.argtypes = [I, L, I, I]
+        lib.cake_gemm_rows_kind.restype = I
+        lib.cake_gemm_rows_ws_floats.argtypes = [I]
+        lib.cake_gemm_rows_ws_floats.restype = L
+        lib.cake_gemm_rows_ticks.argtypes = []
+        lib.cake_gemm_rows_ticks.restype = I
+        lib.cake_gemm_rows.argtypes = [I, I, I, P, L, P, L, P, L, P, P, L, P, P, P, I, I, I,
+                                       C.c_float, P]
+        lib.cake_gemm_rows.restype = I
+        lib.cake_gemm_rows_grouped.argtypes = [I, I, P, L, P, L, L, P, L, P, I, P, P, P, I, I, P]
+        lib.cake_gemm_rows_grouped.restype = I
         _bound = True
     return lib
 
@@ -100,6 +111,36 @@ def _workspace(dev, numel: int) -> torch.Tensor:
             _ws_keep.append(w)
         w = _ws[dev] = torch.empty(max(numel, 1 << 20), dtype=torch.float32, device=dev)
     return w
+
+
+ROWS_MAX = 64   # rows that the products of few rows take at most
+_rows_kinds: dict = {}
+_ticks: dict = {}   # (device, stream) -> arrival counters of the stream form, newest last
+
+
+def rows_kind(M: int, Nv: int, K: int, gated: bool) -> int:
+    """Form of a product of M rows (gemm.hip rows_kind): 0 tile kernels, 1 direct, 2 stream."""
+    if M > ROWS_MAX:
+        return 0
+    key = (M, Nv, K, gated)
+    kind = _rows_kinds.get(key)
+    if kind is None:
+        kind = _rows_kinds[key] = int(_lib().cake_gemm_rows_kind(M, Nv, K, int(gated)))
+    return kind
+
+
+def _rows_state(dev, M: int, st: int):
+    """(workspace, counters) of one launch of the stream form.  The counters are zero between
+    launches; two launches that run side by side need their own, so they belong to a stream.  A
+    captured graph may run beside any stream: none for it (the caller takes the tile kernels)."""
+    key = (dev, st)
+    t = _ticks.pop(key, None)
+    if t is None:
+        t = torch.zeros(_lib().cake_gemm_rows_ticks(), dtype=torch.int32, device=dev)
+        while len(_ticks) >= 16:   # freed in the order of its own stream
+            _ticks.pop(next(iter(_ticks)))
+    _ticks[key] = t
+    return torch.empty(int(_lib().cake_gemm_rows_ws_floats(M)), dtype=torch.float32, device=dev), t
 
 
 def _load_tuned() -> list:
@@ -297,11 +338,24 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
     f32_out = epi in ("resid32", "store32")
     if M == 0:
         return resid if f32_out else out
+    if alpha != 1.0 and not f32_out:
+        raise ValueError(f"{epi} takes no alpha")
+    if cfg is None and splits is None and M <= ROWS_MAX and (M, Nv, K, epi) not in _plans:
+        kind = rows_kind(M, Nv, K, gated)
+        if kind == 2 and torch.cuda.is_current_stream_capturing():
+            kind = 0
+        if kind:
+            st = torch.cuda.current_stream().cuda_stream
+            ws, tick = _rows_state(x.device, M, st) if kind == 2 else (None, None)
+            check(_lib().cake_gemm_rows(
+                _DT[x.dtype], EPI[epi], kind, x2.data_ptr(), lda, w.data_ptr(), ldb, cptr, ldc,
+                None if bias is None else bias.data_ptr(), rptr, ldr,
+                None if ws is None else ws.data_ptr(), None if tick is None else tick.data_ptr(),
+                _zeros16(x.device).data_ptr(), M, N, K, float(alpha), st), "gemm_rows")
+            return resid if f32_out else out
     c0, s0 = plan(M, Nv, K, epi)
     cfg = c0 if cfg is None else cfg
     lib_ok = epi != "swiglu" or (ldc == N and N % 8 == 0 and out2.data_ptr() % 16 == 0)
-    if alpha != 1.0 and not f32_out:
-        raise ValueError(f"{epi} takes no alpha")
     if cfg == LIB and bias is None and epi in LIB_EPIS and lib_ok and alpha == 1.0:
         _lib_gemm(x2, lda, w, ldb, epi, out2, ldc, r2 if f32_out else None, ldr, M, N, K)
         return resid if f32_out else out
@@ -319,12 +373,16 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
     return resid if f32_out else out
 
 
-GROUPED_CFGS = {0: 128, 4: 64, 5: 256}   # tile configuration of a grouped product -> its rows
+# tile configuration of a grouped product -> its rows (ROWS: the stream form)
+ROWS = 32
+GROUPED_CFGS = {0: 128, 4: 64, 5: 256, ROWS: 16}
 
 
-def grouped_cfg(rows: int, groups: int) -> int:
+def grouped_cfg(rows: int, groups: int, capturing: bool = False) -> int:
     """Tile configuration for `rows` sorted rows over `groups` weight groups."""
     mean = rows / groups
+    if mean <= 4 and not capturing:   # the stream form's counters stay out of graphs
+        return ROWS
     return 5 if mean >= 96 else 0 if mean >= 24 else 4
 
 
@@ -348,6 +406,14 @@ def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out
     if tiles.dtype != torch.int32 or not tiles.is_contiguous() or tiles.dim() != 2 or \
             tiles.shape[0] < 2 or tiles.shape[1] != 4 or not tiles.is_cuda or tiles.data_ptr() % 16:
         raise ValueError("grouped: tiles must be a contiguous int32 [n + 1, 4] device tensor")
+    if cfg == ROWS:
+        st = torch.cuda.current_stream().cuda_stream
+        ws, tick = _rows_state(x.device, 16, st)
+        check(_lib().cake_gemm_rows_grouped(
+            _DT[x.dtype], EPI[epi], x2.data_ptr(), lda, w.data_ptr(), K, N * K, o2.data_ptr(), ldc,
+            tiles.data_ptr(), tiles.shape[0] - 1, ws.data_ptr(), tick.data_ptr(),
+            _zeros16(x.device).data_ptr(), N, K, st), "gemm_rows_grouped")
+        return out
     check(_lib().cake_gemm_grouped(
         _DT[x.dtype], EPI[epi], int(cfg), x2.data_ptr(), lda, w.data_ptr(), K, N * K,
         o2.data_ptr(), ldc, tiles.data_ptr(), tiles.shape[0] - 1, _zeros16(x.device).data_ptr(), N, K,

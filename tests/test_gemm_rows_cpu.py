@@ -1,0 +1,24 @@
+"""Rule of the products of few rows (gemm.hip rows_kind): which form takes which sizes."""
+import pytest
+
+from cake_amd.build import GEMM_LIB
+
+pytestmark = pytest.mark.skipif(not GEMM_LIB.exists(), reason="native libraries not built")
+
+
+def test_rows_kind_lines():
+    from cake_amd.ops import gemm as G
+    assert G.rows_kind(5, 2048, 2048, False) == 1        # small weights: direct
+    assert G.rows_kind(16, 4096, 4096, False) == 1
+    assert G.rows_kind(16, 4096, 14336, False) == 2      # large ones: the stream
+    assert G.rows_kind(45, 28672, 4096, True) == 2
+    assert G.rows_kind(64, 4096, 4096, False) == 0       # tiles
+    assert G.rows_kind(65, 28672, 4096, True) == 0
+    assert all(G.rows_kind(M, Nv, K, False) != 1 for M in (33, 64) for Nv in (64, 4096)
+               for K in (64, 8192))
+
+
+def test_grouped_rows_stay_out_of_graphs():
+    from cake_amd.ops import gemm as G
+    assert G.grouped_cfg(78, 64) == G.ROWS and G.grouped_cfg(78, 64, capturing=True) == 4
+    assert G.grouped_cfg(64 * 5, 64) == 4
