@@ -41,26 +41,19 @@
 #include <algorithm>
 
 namespace cake {
-// the launchers are instantiated in gemm_inst_{bf16,f16}_{a,b}.hip
+// the launchers are instantiated in gemm_inst_{bf16,f16}_{a,b,c}.hip
 #define CAKE_GEMM_EXTERN(DT, E) extern template int launch_gemm<DT, E>(int, dim3, hipStream_t, const GemmArgs&);
 #define CAKE_GEMM_EXTERN_ALL(DT) CAKE_GEMM_EXTERN(DT, kEpiStore) CAKE_GEMM_EXTERN(DT, kEpiResid32) \
   CAKE_GEMM_EXTERN(DT, kEpiAdd16) CAKE_GEMM_EXTERN(DT, kEpiSwiglu) CAKE_GEMM_EXTERN(DT, kEpiGeglu) \
-  CAKE_GEMM_EXTERN(DT, kEpiPartial) CAKE_GEMM_EXTERN(DT, kEpiStore32) CAKE_GEMM_EXTERN(DT, kEpiSilu)
+  CAKE_GEMM_EXTERN(DT, kEpiPartial) CAKE_GEMM_EXTERN(DT, kEpiStore32) CAKE_GEMM_EXTERN(DT, kEpiSilu) \
+  CAKE_GEMM_EXTERN(DT, kEpiQuick) CAKE_GEMM_EXTERN(DT, kEpiGelu) CAKE_GEMM_EXTERN(DT, kEpiRelu2)
 CAKE_GEMM_EXTERN_ALL(kBF16)
 CAKE_GEMM_EXTERN_ALL(kF16)
 #undef CAKE_GEMM_EXTERN_ALL
 #undef CAKE_GEMM_EXTERN
 // ... and in gemm_inst_rows_{bf16,f16}.hip
-#define CAKE_ROWS_EXTERN(DT)                                                              \
-  extern template int launch_rows<DT, kEpiStore>(int, int, dim3, hipStream_t, const GemmArgs&);   \
-  extern template int launch_rows<DT, kEpiResid32>(int, int, dim3, hipStream_t, const GemmArgs&); \
-  extern template int launch_rows<DT, kEpiAdd16>(int, int, dim3, hipStream_t, const GemmArgs&);   \
-  extern template int launch_rows<DT, kEpiSwiglu>(int, int, dim3, hipStream_t, const GemmArgs&);  \
-  extern template int launch_rows<DT, kEpiGeglu>(int, int, dim3, hipStream_t, const GemmArgs&);   \
-  extern template int launch_rows<DT, kEpiStore32>(int, int, dim3, hipStream_t, const GemmArgs&); \
-  extern template int launch_rows<DT, kEpiSilu>(int, int, dim3, hipStream_t, const GemmArgs&);    \
-  extern template int launch_rows_grouped<DT, kEpiStore>(int, dim3, hipStream_t, const GemmArgs&); \
-  extern template int launch_rows_grouped<DT, kEpiSilu>(int, dim3, hipStream_t, const GemmArgs&);
+#define CAKE_ROWS_EXTERN(DT)                                                                      \
+  extern template struct Rows<DT>;
 CAKE_ROWS_EXTERN(kBF16)
 CAKE_ROWS_EXTERN(kF16)
 #undef CAKE_ROWS_EXTERN
@@ -108,6 +101,9 @@ static int dispatch_epi(int epi, int cfg, dim3 grid, hipStream_t st, const GemmA
     case kEpiPartial: return launch_gemm<DT, kEpiPartial>(cfg, grid, st, g);
     case kEpiStore32: return launch_gemm<DT, kEpiStore32>(cfg, grid, st, g);
     case kEpiSilu: return launch_gemm<DT, kEpiSilu>(cfg, grid, st, g);
+    case kEpiQuick: return launch_gemm<DT, kEpiQuick>(cfg, grid, st, g);
+    case kEpiGelu: return launch_gemm<DT, kEpiGelu>(cfg, grid, st, g);
+    case kEpiRelu2: return launch_gemm<DT, kEpiRelu2>(cfg, grid, st, g);
   }
   return (int)hipErrorInvalidValue;
 }
@@ -117,7 +113,7 @@ static int dispatch_finalize(int epi, dim3 grid, hipStream_t st, const GemmArgs&
   switch (epi) {
 #define F(E) case E: hipLaunchKernelGGL((gemm_splitk_finalize<DT, E>), grid, dim3(256), 0, st, g, splits); break;
     F(kEpiStore) F(kEpiResid32) F(kEpiAdd16) F(kEpiSwiglu) F(kEpiGeglu) F(kEpiStore32)
-    F(kEpiSilu)
+    F(kEpiSilu) F(kEpiQuick) F(kEpiGelu) F(kEpiRelu2)
 #undef F
     default: return (int)hipErrorInvalidValue;
   }
@@ -169,11 +165,6 @@ CAKE_API int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* 
                               const void* zeros, int M, int N, int K, float alpha,
                               hipStream_t st) {
   if (alpha != 1.f && epi != kEpiResid32 && epi != kEpiStore32) return (int)hipErrorInvalidValue;
-  int act = 0;
-  if (epi >= 8 && epi <= 10) {  // quick_gelu / GELU / relu^2: the activation epilogue, other act
-    act = epi - 7;
-    epi = kEpiSilu;
-  }
   int bm, bn;
   cfg_dims(cfg, bm, bn);
   if (bm == 0 || M <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || splits < 1)
@@ -196,7 +187,6 @@ CAKE_API int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* 
   g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.ldr = ldr;
   g.M = M; g.N = N; g.K = K;
   g.gated = gated ? 1 : 0;
-  g.act = act;
   g.alpha = alpha;
   g.half = N;
   g.Nv = gated ? 2 * N : N;
@@ -280,11 +270,6 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
                             long long ldr, float* ws, void* tick, const void* zeros, int M, int N,
                             int K, float alpha, hipStream_t st) {
   if (alpha != 1.f && epi != kEpiResid32 && epi != kEpiStore32) return (int)hipErrorInvalidValue;
-  int act = 0;
-  if (epi >= 8 && epi <= 10) {
-    act = epi - 7;
-    epi = kEpiSilu;
-  }
   const bool gated = (epi == kEpiSwiglu || epi == kEpiGeglu);
   if (M < 1 || M > 64 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || (gated && N % 16) ||
       !(kind == 1 || kind == 2) || (kind == 1 && M > 32) || (kind == 2 && (!ws || !tick || !zeros)))
@@ -298,7 +283,6 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
   g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.ldr = ldr;
   g.M = M; g.N = N; g.K = K;
   g.gated = gated ? 1 : 0;
-  g.act = act;
   g.alpha = alpha;
   g.half = N;
   g.Nv = gated ? 2 * N : N;
@@ -317,21 +301,8 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
     form = nt - 1;
     wgs = (g.Nv + 16 * nt - 1) / (16 * nt);
   }
-  const auto run = [&](auto dtc) {
-    constexpr int DT = decltype(dtc)::value;
-    switch (epi) {
-      case kEpiStore: return launch_rows<DT, kEpiStore>(form, mt, dim3(wgs), st, g);
-      case kEpiResid32: return launch_rows<DT, kEpiResid32>(form, mt, dim3(wgs), st, g);
-      case kEpiAdd16: return launch_rows<DT, kEpiAdd16>(form, mt, dim3(wgs), st, g);
-      case kEpiSwiglu: return launch_rows<DT, kEpiSwiglu>(form, mt, dim3(wgs), st, g);
-      case kEpiGeglu: return launch_rows<DT, kEpiGeglu>(form, mt, dim3(wgs), st, g);
-      case kEpiStore32: return launch_rows<DT, kEpiStore32>(form, mt, dim3(wgs), st, g);
-      case kEpiSilu: return launch_rows<DT, kEpiSilu>(form, mt, dim3(wgs), st, g);
-    }
-    return (int)hipErrorInvalidValue;
-  };
-  return dt == kBF16 ? run(std::integral_constant<int, kBF16>{})
-         : dt == kF16 ? run(std::integral_constant<int, kF16>{}) : (int)hipErrorInvalidValue;
+  return dt == kBF16 ? Rows<kBF16>::run(epi, form, mt, dim3(wgs), st, g)
+         : dt == kF16 ? Rows<kF16>::run(epi, form, mt, dim3(wgs), st, g) : (int)hipErrorInvalidValue;
 }
 
 // cake_gemm_grouped in the stream form: tiles of at most 16 rows; ws and tick as above (ws of 16
@@ -350,18 +321,11 @@ CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long ld
   g.ws = ws; g.tick = (unsigned*)tick; g.zeros = (const uint16_t*)zeros;
   g.lda = lda; g.ldb = ldb; g.ldc = ldc;
   g.N = N; g.K = K; g.Nv = N; g.half = N;
-  g.act = epi ? epi - 7 : 0;
   g.tiles_m = max_tiles;
   g.tiles_n = (N + 127) / 128;
   g.kps = kRowsMinSteps;
   g.groups = (const int4*)tiles;
   g.b_group = b_group;
-  const dim3 grid(kRowsWgs);
-  if (epi == 0)
-    return dt == kBF16 ? launch_rows_grouped<kBF16, kEpiStore>(1, grid, st, g)
-           : dt == kF16 ? launch_rows_grouped<kF16, kEpiStore>(1, grid, st, g)
-                        : (int)hipErrorInvalidValue;
-  return dt == kBF16 ? launch_rows_grouped<kBF16, kEpiSilu>(1, grid, st, g)
-         : dt == kF16 ? launch_rows_grouped<kF16, kEpiSilu>(1, grid, st, g)
-                      : (int)hipErrorInvalidValue;
+  return dt == kBF16 ? Rows<kBF16>::grouped(epi, dim3(kRowsWgs), st, g)
+         : dt == kF16 ? Rows<kF16>::grouped(epi, dim3(kRowsWgs), st, g) : (int)hipErrorInvalidValue;
 }

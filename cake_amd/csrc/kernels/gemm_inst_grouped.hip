@@ -39,18 +39,23 @@ CAKE_API int cake_gemm_grouped(int dt, int epi, int cfg, const void* a, long lon
   g.zeros = (const uint16_t*)zeros;
   g.lda = lda; g.ldb = ldb; g.ldc = ldc;
   g.N = N; g.K = K; g.Nv = N; g.half = N;
-  g.act = epi ? epi - 7 : 0;
   g.tiles_m = max_tiles;
   g.tiles_n = (N + bn - 1) / bn;
   g.kps = (K + kGBK - 1) / kGBK * kGBK;
   g.groups = (const int4*)tiles;
   g.b_group = b_group;
   const dim3 grid(g.tiles_m * g.tiles_n, 1);
-  if (epi == 0)
-    return dt == kBF16 ? launch_grouped<kBF16, kEpiStore>(cfg, grid, st, g)
-           : dt == kF16 ? launch_grouped<kF16, kEpiStore>(cfg, grid, st, g)
-                        : (int)hipErrorInvalidValue;
-  return dt == kBF16 ? launch_grouped<kBF16, kEpiSilu>(cfg, grid, st, g)
-         : dt == kF16 ? launch_grouped<kF16, kEpiSilu>(cfg, grid, st, g)
-                      : (int)hipErrorInvalidValue;
+  const auto run = [&](auto dtc) {
+    constexpr int DT = decltype(dtc)::value;
+    switch (epi) {
+      case kEpiStore: return launch_grouped<DT, kEpiStore>(cfg, grid, st, g);
+      case kEpiSilu: return launch_grouped<DT, kEpiSilu>(cfg, grid, st, g);
+      case kEpiQuick: return launch_grouped<DT, kEpiQuick>(cfg, grid, st, g);
+      case kEpiGelu: return launch_grouped<DT, kEpiGelu>(cfg, grid, st, g);
+      case kEpiRelu2: return launch_grouped<DT, kEpiRelu2>(cfg, grid, st, g);
+    }
+    return (int)hipErrorInvalidValue;
+  };
+  return dt == kBF16 ? run(std::integral_constant<int, kBF16>{})
+         : dt == kF16 ? run(std::integral_constant<int, kF16>{}) : (int)hipErrorInvalidValue;
 }

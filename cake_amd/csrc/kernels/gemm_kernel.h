@@ -20,11 +20,13 @@ enum GemmEpi : int {
   kEpiGeglu = 4,   // C16[:, f] = acc_h * gelu_tanh(acc_gate)
   kEpiPartial = 5, // W32[split] = acc (split-K slab, virtual column order)
   kEpiStore32 = 6, // R32 = acc (+ bias)              (f32 output, e.g. conv time biases)
-  kEpiSilu = 7,    // C16 = act(acc (+ bias)), act = GemmArgs::act: SiLU (time-embedding
-                   // MLP), quick_gelu / erf-GELU (CLIP MLP), relu^2; host ids 7 / 8 / 9 / 10
+  kEpiSilu = 7,    // C16 = act(acc (+ bias)): SiLU (time-embedding MLP),
+  kEpiQuick = 8,   //   quick_gelu, erf-GELU (CLIP MLP, hybrid feed-forwards), relu^2
+  kEpiGelu = 9,
+  kEpiRelu2 = 10,
 };
+constexpr bool act_epi(int epi) { return epi >= kEpiSilu; }
 
-// the activation of kEpiSilu (runtime-uniform: one kernel instance for all of them)
 // erf by Abramowitz & Stegun, formula 7.1.26 (|error| <= 1.5e-7): one exponential, one
 // reciprocal and a polynomial, no branch — the epilogue evaluates it once per output, where
 // erff's branches stood out (the result is rounded to 16 bits)
@@ -37,14 +39,19 @@ __device__ __forceinline__ float erf_as(float x) {
   return copysignf(fmaf(-p * t, __expf(-ax * ax), 1.f), x);
 }
 
-__device__ __forceinline__ float gemm_act(int act, float x) {
-  if (act == 1) return x * __frcp_rn(1.f + __expf(-1.702f * x));  // quick_gelu
-  if (act == 2) return 0.5f * x * (1.f + erf_as(x * 0.70710678118654752f));  // GELU (erf)
-  if (act == 3) {  // square of ReLU
+// the activation of an epilogue, a kernel instance each: picked per element at run time its
+// branches were a fifth of the kernel (6000 rows x 19456 x 4096 GELU, 256 x 192 tiles: 1031 us,
+// 849 us so)
+template <int EPI>
+__device__ __forceinline__ float gemm_act(float x) {
+  if constexpr (EPI == kEpiQuick) return x * __frcp_rn(1.f + __expf(-1.702f * x));
+  else if constexpr (EPI == kEpiGelu) return 0.5f * x * (1.f + erf_as(x * 0.70710678118654752f));
+  else if constexpr (EPI == kEpiRelu2) {
     const float r = fmaxf(x, 0.f);
     return r * r;
+  } else {
+    return silu(x);
   }
-  return silu(x);
 }
 
 struct GemmArgs {
@@ -61,7 +68,6 @@ struct GemmArgs {
   int Nv, half;          // gated: Nv = 2 * half, half = N
   int gated;             // B row order interleaves 16-row blocks of two halves
   int tiles_m, tiles_n, kps;  // k elements per split
-  int act;               // kEpiSilu activation: 0 SiLU, 1 quick_gelu, 2 GELU (erf), 3 relu^2
   float alpha = 1.f;     // kEpiResid32 / kEpiStore32: factor of the product (and bias)
   // in-kernel split-K pair (gemm_4w.h, splits == 2): the first split of a tile to finish
   // parks its accumulators in ws (one 256x256 f32 slab per tile), the second adds them and
@@ -341,9 +347,9 @@ __device__ __forceinline__ void epi_strip(const GemmArgs& g, const cf32x4 (&tile
 #pragma unroll
             for (int c = 0; c < CPL; ++c) v[c] += ops.res[B][c];
           }
-          if constexpr (EPI == kEpiSilu) {
+          if constexpr (act_epi(EPI)) {
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) v[c] = gemm_act(g.act, v[c]);
+            for (int c = 0; c < CPL; ++c) v[c] = gemm_act<EPI>(v[c]);
           }
           uint16_t outv[CPL];
 #pragma unroll
@@ -560,9 +566,9 @@ __device__ __forceinline__ void readout_strip_w(const GemmArgs& g, const float* 
 #pragma unroll
           for (int e = 0; e < CE; ++e) v[e] += ops.res[B][p * W::CPL + c * CE + e];
         }
-        if constexpr (EPI == kEpiSilu) {
+        if constexpr (act_epi(EPI)) {
 #pragma unroll
-          for (int e = 0; e < CE; ++e) v[e] = gemm_act(g.act, v[e]);
+          for (int e = 0; e < CE; ++e) v[e] = gemm_act<EPI>(v[e]);
         }
         uint16_t outv[CE];
 #pragma unroll
@@ -899,7 +905,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_finalize(GemmArgs g, int spli
     else {
       y = v[q] + (g.bias != nullptr ? to_f32<DT>(g.bias[fq]) : 0.f);
       if constexpr (EPI == kEpiAdd16) y += to_f32<DT>(g.r16[(size_t)m * g.ldr + fq]);
-      if constexpr (EPI == kEpiSilu) y = gemm_act(g.act, y);
+      if constexpr (act_epi(EPI)) y = gemm_act<EPI>(y);
     }
     if constexpr (EPI == kEpiResid32) {
       float* r = g.r32 + (size_t)m * g.ldr + fq;

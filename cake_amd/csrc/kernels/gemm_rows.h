@@ -160,7 +160,7 @@ __global__ __launch_bounds__(512) void gemm_direct_kernel(GemmArgs g) {
           a = EPI == kEpiSwiglu ? silu(a) * b : a * gelu_tanh(b);
         }
         if constexpr (EPI == kEpiAdd16) a += to_f32<DT>(g.r16[(size_t)m * g.ldr + nn]);
-        if constexpr (EPI == kEpiSilu) a = gemm_act(g.act, a);
+        if constexpr (act_epi(EPI)) a = gemm_act<EPI>(a);
         y[e] = a;
       }
       if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32) {
@@ -261,7 +261,7 @@ __device__ __forceinline__ void stream_store(const GemmArgs& g, const StreamStri
           a = EPI == kEpiSwiglu ? silu(a) * u : a * gelu_tanh(u);
         }
         if constexpr (EPI == kEpiAdd16) a += to_f32<DT>(g.r16[(size_t)m * g.ldr + min(n + e, g.N - 1)]);
-        if constexpr (EPI == kEpiSilu) a = gemm_act(g.act, a);
+        if constexpr (act_epi(EPI)) a = gemm_act<EPI>(a);
         y[e] = a;
       }
       if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32) {
@@ -481,12 +481,29 @@ int launch_rows(int kind, int mt, dim3 grid, hipStream_t st, const GemmArgs& g) 
   return (int)hipErrorInvalidValue;
 }
 
-// rows sorted by weight group (GemmArgs::groups), at most 16 MT of them per tile
-template <int DT, int EPI>
-int launch_rows_grouped(int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
-  if (mt != 1) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI, 1, true>), grid, dim3(256), 0, st, g);
-  return (int)hipGetLastError();
-}
+// every epilogue of a type; grouped: rows sorted by weight group (GemmArgs::groups), tiles of at most
+// 16 of them
+template <int DT> struct Rows {
+  static int run(int epi, int kind, int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
+    switch (epi) {
+#define X(E) case E: return launch_rows<DT, E>(kind, mt, grid, st, g);
+      X(kEpiStore) X(kEpiResid32) X(kEpiAdd16) X(kEpiSwiglu) X(kEpiGeglu) X(kEpiStore32)
+      X(kEpiSilu) X(kEpiQuick) X(kEpiGelu) X(kEpiRelu2)
+#undef X
+    }
+    return (int)hipErrorInvalidValue;
+  }
+  static int grouped(int epi, dim3 grid, hipStream_t st, const GemmArgs& g) {
+    switch (epi) {
+#define X(E)                                                                                  \
+  case E:                                                                                     \
+    hipLaunchKernelGGL((gemm_stream_kernel<DT, E, 1, true>), grid, dim3(256), 0, st, g);      \
+    return (int)hipGetLastError();
+      X(kEpiStore) X(kEpiSilu) X(kEpiQuick) X(kEpiGelu) X(kEpiRelu2)
+#undef X
+    }
+    return (int)hipErrorInvalidValue;
+  }
+};
 
 }  // namespace cake
