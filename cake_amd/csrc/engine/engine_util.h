@@ -97,6 +97,8 @@ inline bool gemm_lib_enabled() {
   return e && *e == '1';
 }
 
+extern "C" int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits);
+
 struct GemmPlanner {
   struct Tuned { long long M, Nv, K; std::string epi; int cfg, splits; };
   std::vector<Tuned> tuned;
@@ -127,6 +129,22 @@ struct GemmPlanner {
     for (const auto& e : tuned)
       if (e.cfg == kGemmLib) return true;
     return false;
+  }
+
+  // the plan that runs (ops/gemm.py resolve): the measured entry of this very size unless the
+  // kernel library's estimate puts it well behind, else the estimate's best; epi_id: its epilogue id
+  std::pair<int, int> resolve(long long M, long long Nv, long long K, const std::string& epi, int epi_id,
+                              bool big, bool mfma_only = false) const {
+    int cfg = -1, splits = 1;
+    for (const auto& e : tuned)
+      if (e.M == M && e.Nv == Nv && e.K == K && e.epi == epi && !(mfma_only && e.cfg == kGemmLib)) {
+        cfg = e.cfg;
+        splits = e.splits;
+        break;
+      }
+    if (cfg == kGemmLib && has_lib()) return {kGemmLib, 1};
+    cake_gemm_plan((int)M, Nv, (int)K, epi_id, big ? 1 : 0, &cfg, &splits);
+    return {cfg, splits};
   }
 
   // the MFMA kernel's plan: the measured entries other than the library GEMM's

@@ -1205,13 +1205,14 @@ class Llama {
                              ticks_, zeros_, M, N, K, 1.f, st_), what);
       return;
     }
-    auto p = planner_.plan(M, Nv, K, names[epi]);
+    const bool big = std::max((M - 1) * lda + K, (Nv - 1) * ldb + K) * 2 >= 0x7fffffffLL;
+    auto p = planner_.resolve(M, Nv, K, names[epi], epi, big);
     if (p.first == kGemmLib) {  // the table names the library GEMM (CAKE_GEMM_LIB=1 only)
       if ((epi != kEpiSwiglu || ldc == N) &&
           lib_gemm(epi, a, lda, b, ldb, cptr, ldc, resid, ldr, M, N, K, what))
         return;
       // a strided SwiGLU output or a library failure: the MFMA kernel's plan
-      p = planner_.plan_mfma(M, Nv, K, names[epi]);
+      p = planner_.resolve(M, Nv, K, names[epi], epi, big, true);
     }
     const int splits = p.second;
     float* ws = nullptr;

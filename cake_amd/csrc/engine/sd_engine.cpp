@@ -1473,7 +1473,8 @@ class SdEngine {
                              nullptr, zeros_, M, N, K, 1.f, st_), "gemm rows");
       return;
     }
-    const auto pl = planner_.plan_mfma(M, Nv, K, kEpiNames[epi]);  // no library path here
+    const bool big = std::max((M - 1) * lda + K, (Nv - 1LL) * K + K) * 2 >= 0x7fffffffLL;
+    const auto pl = planner_.resolve(M, Nv, K, kEpiNames[epi], epi, big, true);  // no library path here
     float* ws = pl.second > 1
                     ? gemm_ws((size_t)cake_gemm_ws_floats(pl.first, pl.second, M, N, K, gated ? 1 : 0))
                     : nullptr;

@@ -39,6 +39,7 @@
 #include "gemm_rows.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace cake {
 // the launchers are instantiated in gemm_inst_{bf16,f16}_{a,b,c}.hip
@@ -61,16 +62,29 @@ CAKE_ROWS_EXTERN(kF16)
 
 using namespace cake;
 
-// split-K pair tickets of gemm_4w (zero at load; every pair leaves its tile's zero)
-__device__ unsigned g_pair_tick[2 * kPairTiles];
+// Counters of the four-wave tiles' pieces (zero at load; every launch leaves its region zero).  A
+// launch has a region of its own: launches that run side by side (several streams, a graph beside
+// eager work) never meet in one.  Eager launches take turns through more regions than a device's
+// queues hold launches; a captured launch keeps its region for the life of the process, and when
+// those are used up it runs its tiles whole.
+constexpr unsigned kEagerRegions = 2048, kGraphRegions = 2048, kRegion = 2 * kPieceTiles;
+__device__ unsigned g_piece_tick[(size_t)(kEagerRegions + kGraphRegions) * kRegion];
 
-static unsigned* pair_ticks() {
-  static unsigned* p = nullptr;
-  if (!p) {
-    void* a = nullptr;
-    if (hipGetSymbolAddress(&a, HIP_SYMBOL(g_pair_tick)) == hipSuccess) p = static_cast<unsigned*>(a);
+static unsigned* piece_ticks(hipStream_t st) {
+  static std::atomic<unsigned> eager{0}, graph{0};
+  // the symbol's address on the current device (looked up per call: a few hundred ns, and right on
+  // every device)
+  void* base = nullptr;
+  if (hipGetSymbolAddress(&base, HIP_SYMBOL(g_piece_tick)) != hipSuccess) return nullptr;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) return nullptr;
+  unsigned r = eager.fetch_add(1, std::memory_order_relaxed) % kEagerRegions;
+  if (cap != hipStreamCaptureStatusNone) {
+    r = graph.fetch_add(1, std::memory_order_relaxed);
+    if (r >= kGraphRegions) return nullptr;
+    r += kEagerRegions;
   }
-  return p;
+  return static_cast<unsigned*>(base) + (size_t)r * kRegion;
 }
 
 static inline void cfg_dims(int cfg, int& bm, int& bn) {
@@ -120,38 +134,130 @@ static int dispatch_finalize(int epi, dim3 grid, hipStream_t st, const GemmArgs&
   return (int)hipGetLastError();
 }
 
-// Split plan of one call: the k split actually run (whole 64-element steps per split) and,
-// for a four-wave tile at splits 2, the in-kernel pair's tiles (0: the slab + finalize
-// form).  cake_gemm and cake_gemm_ws_floats both decide through this one function, so a
-// workspace sized by the query always covers the launch.
+// Split plan of one call: the k split actually run (whole 64-element steps per split) and, for a
+// four-wave tile, its pieces instead: the tiles past the last whole wave of 256 (all of them when
+// there are no more) in `splits` pieces each, or as many as one wave of 256 holds.
+// cake_gemm and cake_gemm_ws_floats both decide through this one function, so a workspace sized
+// by the query always covers the launch.
 struct SplitPlan {
-  int splits, kps, bm, bn, ntiles, npair;
+  int splits, kps, bm, bn, ntiles;
+  int rest, pieces;   // tiles that run in pieces (0: none), pieces of each
 };
 static SplitPlan split_plan(int cfg, int splits, int M, long long Nv, int K) {
   SplitPlan p{};
   cfg_dims(cfg, p.bm, p.bn);
+  if (p.bm != 0) p.ntiles = (int)(((M + p.bm - 1) / p.bm) * ((Nv + p.bn - 1) / p.bn));
+  const bool four = p.bm != 0 && four_wave_cfg(cfg);
+  const int rest = p.ntiles <= 256 ? p.ntiles : p.ntiles % 256;
+  if (four) splits = rest > 0 ? std::max(1, std::min(splits, 256 / rest)) : 1;
   int kps = (K + splits - 1) / splits;
   kps = (kps + kGBK - 1) / kGBK * kGBK;
   p.kps = kps;
   p.splits = (K + kps - 1) / kps;
-  if (p.bm == 0) return p;
-  p.ntiles = (int)(((M + p.bm - 1) / p.bm) * ((Nv + p.bn - 1) / p.bn));
-  const int npair = p.ntiles <= 256 ? p.ntiles : p.ntiles % 256;
-  if (four_wave_cfg(cfg) && p.splits == 2 && npair > 0 &&
-      npair <= 128 + (p.ntiles <= 256 ? 128 : 0) && p.ntiles <= kPairTiles &&
-      (long long)npair * p.bm * p.bn <= 2LL * M * Nv && pair_ticks())
-    p.npair = npair;
+  if (four && p.splits > 1) {
+    p.rest = rest;
+    p.pieces = p.splits;
+    p.splits = 1;
+  }
   return p;
 }
 
-// f32 workspace (elements) a cake_gemm call with these arguments needs: the pair's slabs
-// (npair x BM x BN) or splits x M x Nv partial rows, 0 when it runs unsplit
+// f32 workspace (elements) a cake_gemm call with these arguments needs: the pieces' slabs
+// (BM x BN each) or splits x M x Nv partial rows, 0 when it runs unsplit
 CAKE_API long long cake_gemm_ws_floats(int cfg, int splits, int M, int N, int K, int gated) {
   if (splits < 1 || M <= 0 || N <= 0 || K <= 0) return 0;
   const long long Nv = gated ? 2LL * N : N;
   const SplitPlan p = split_plan(cfg, splits, M, Nv, K);
-  if (p.npair > 0) return (long long)p.npair * p.bm * p.bn;
+  if (p.pieces > 0) return (long long)p.rest * p.pieces * p.bm * p.bn;
   return p.splits > 1 ? (long long)p.splits * M * Nv : 0;
+}
+
+// ---- tile plan of a size that has no measured entry ------------------------
+// t(us) = c0 + step (k steps of all rounds) + lone (k steps a thin round loses to latency)
+//         + epi[class] rounds + merge [split] + fin (split: MB of slabs written and read, or pieces)
+// fitted to timings of every tile and split on weights that no cache holds: 22 weight shapes (width
+// 512 .. 8192, k 512 .. 28672), 65 .. 6000 rows.  Over those 566 sizes the plan it picks is 2.4 %
+// off the best of all, at most 33 %; the nearest measured size with its split scaled was 16 % off
+// (777 x 4096 x 14336 184 us, 113 us so; 6000 rows 680, 550).  Left out: the tiles that were best
+// nowhere beyond what these reach.
+struct TileCost {
+  int cfg, bm, bn, slots;                  // slots: workgroups a CU holds
+  float c0, step, lone, epi[4], merge, fin;
+};
+static constexpr TileCost kTileCosts[] = {
+    {5, 256, 256, 1, 0.69f, 1.43f, 0.f, {5.52f, 7.84f, 9.9f, 6.58f}, 4.16f, 0.304f},
+    {6, 256, 128, 1, 0.844f, 0.802f, 0.f, {4.16f, 5.6f, 6.f, 4.4f}, 3.93f, 0.325f},
+    {7, 128, 128, 1, 2.77f, 0.539f, 0.f, {2.72f, 3.65f, 4.5f, 4.2f}, 3.6f, 0.382f},
+    {12, 64, 128, 2, 4.62f, 0.663f, 0.145f, {0.f, 0.598f, 1.92f, 1.93f}, 3.09f, 0.468f},
+    {13, 64, 64, 2, 3.41f, 0.427f, 0.107f, {0.79f, 1.37f, 2.48f, 2.18f}, 2.83f, 0.484f},
+    {18, 64, 160, 1, 2.28f, 0.467f, 0.f, {2.54f, 3.f, 0.f, 4.42f}, 3.53f, 0.353f},
+    {22, 256, 256, 1, 0.f, 1.26f, 0.f, {10.9f, 15.f, 14.f, 21.7f}, 13.2f, 10.2f},
+    {25, 256, 256, 1, 0.f, 1.49f, 0.f, {0.f, 0.f, 0.f, 0.f}, 20.8f, 13.2f},
+    {26, 256, 192, 1, 0.f, 1.13f, 0.f, {4.44f, 2.29f, 2.14f, 9.67f}, 16.1f, 6.33f},
+    {27, 128, 256, 1, 4.43f, 0.837f, 0.f, {0.0783f, 0.464f, 1.66f, 4.49f}, 13.7f, 4.33f},
+};
+static double tile_cost(const TileCost& c, int splits, long long M, long long Nv, int K, int epi) {
+  const long long ks = (K + kGBK - 1) / kGBK, t = ((M + c.bm - 1) / c.bm) * ((Nv + c.bn - 1) / c.bn);
+  const int cls = epi == kEpiResid32 || epi == kEpiStore32            ? 1
+                  : epi == kEpiSwiglu || epi == kEpiGeglu             ? 2
+                  : epi == kEpiSilu || epi == kEpiQuick || epi == kEpiGelu ? 3 : 0;
+  double steps, rounds, lone = 0, fin = 0;
+  bool split = false;
+  if (four_wave_cfg(c.cfg)) {
+    const SplitPlan p = split_plan(c.cfg, splits, (int)M, Nv, K);
+    if (splits > 1 && p.pieces != splits) return 1e30;   // it would run another split
+    const long long rest = t <= 256 ? t : t % 256;
+    const long long dp = (t - rest) / 256, per = p.pieces ? p.kps / kGBK : ks;
+    steps = (double)(dp * ks + (rest ? per : 0));
+    rounds = (double)(dp + (rest ? 1 : 0));
+    split = p.pieces > 0;
+    fin = p.pieces;
+  } else {
+    const long long kps = (ks + splits - 1) / splits, sp = (ks + kps - 1) / kps, n = t * sp;
+    const long long full = n / (256 * c.slots), rest = n % (256 * c.slots);
+    const double share = (double)((rest + 255) / 256) / c.slots;   // of a round's slots on a CU
+    steps = (double)kps * (full + share);
+    rounds = (double)(full + (rest ? 1 : 0));
+    lone = rest ? (1 - share) * kps : 0;
+    split = sp > 1;
+    if (split) fin = (double)(sp + 1) * M * Nv * 4e-6;
+  }
+  const double us = c.c0 + c.step * steps + c.lone * lone + c.epi[cls] * rounds +
+                    (split ? c.merge + c.fin * fin : 0.);
+  return std::max(us, ((double)Nv * K + (double)M * K) * 2 / 5e6 + 3);   // operands from memory
+}
+
+// (cfg, splits) for a product of M > 64 rows.  On entry *cfg, *splits: a measured plan of this very
+// size, or cfg -1; it stands unless it is modelled and 10 % behind the best.  big: an operand of
+// 2 GB or more (31-bit offsets of the four-wave tiles).
+CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits) {
+  if (M < 1 || Nv < 1 || K < 1 || !cfg || !splits) return (int)hipErrorInvalidValue;
+  const bool gated = epi == kEpiSwiglu || epi == kEpiGeglu;
+  const int ks = (K + kGBK - 1) / kGBK;
+  double best = 1e30, given = -1;
+  int bc = 0, bs = 1;
+  for (const TileCost& c : kTileCosts) {
+    const bool four = four_wave_cfg(c.cfg);
+    if (c.cfg == *cfg) given = tile_cost(c, *splits, M, Nv, K, epi);
+    if (four && (K % kGBK || big)) continue;
+    if (gated && c.cfg == 18) continue;               // 80-column wave tiles
+    // long rows of k: the three-barrier schedule of the 256 x 256 tile (8192 x 28672 at 2048 rows
+    // 726 against 800 us), else the two-stage one (8192 x 8192 199 against 206)
+    if ((c.cfg == k4WCfg && K > 8192) || (c.cfg == k4WCfg + k4WSched && K <= 8192)) continue;
+    for (int sp = 1; sp <= 16; sp *= 2) {
+      if (sp > 1 && (ks / sp < 4 || (four && M < 200))) break;
+      const double t = tile_cost(c, sp, M, Nv, K, epi);
+      if (t < best) {
+        best = t;
+        bc = c.cfg;
+        bs = sp;
+      }
+    }
+  }
+  if (*cfg >= 0 && (given < 0 || given <= 1.1 * best)) return 0;
+  *cfg = bc;
+  *splits = bs;
+  return 0;
 }
 
 // y = epilogue(x W^T).  N = output features (gated: W has 2N rows, gate rows
@@ -195,20 +301,15 @@ CAKE_API int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* 
   const SplitPlan sp = split_plan(cfg, splits, M, g.Nv, K);
   splits = sp.splits;
   g.kps = sp.kps;
-  const dim3 grid(g.tiles_m * g.tiles_n, splits);
-  // splits == 2 on a four-wave tile: the tiles past the last whole wave (all of them when
-  // there are at most 256) run as in-kernel k-half pairs, the rest whole; one slab per
-  // paired tile in ws (cake_gemm_ws_floats), no finalize launch
-  const int ntiles = g.tiles_m * g.tiles_n;
-  const int npair = sp.npair;
-  if (npair > 0 && ws != nullptr) {
-    g.pair = 1;
-    g.tick = pair_ticks();
-    g.dp_tiles = ntiles - npair;
-    const dim3 pgrid(g.dp_tiles + 2 * npair, 1);
-    return (dt == kBF16) ? dispatch_epi<kBF16>(epi, cfg, pgrid, st, g)
-           : (dt == kF16) ? dispatch_epi<kF16>(epi, cfg, pgrid, st, g)
-                          : (int)hipErrorInvalidValue;
+  dim3 grid(g.tiles_m * g.tiles_n, splits);
+  if (sp.pieces > 0) {
+    if (ws != nullptr && (g.tick = piece_ticks(st)) != nullptr) {
+      g.pieces = sp.pieces;
+      g.dp_tiles = sp.ntiles - sp.rest;
+      grid = dim3(g.dp_tiles + sp.rest * sp.pieces, 1);
+    } else {
+      g.kps = K;   // whole tiles
+    }
   }
   const int kernel_epi = splits > 1 ? (int)kEpiPartial : epi;
   if (splits > 1 && ws == nullptr) return (int)hipErrorInvalidValue;

@@ -107,32 +107,39 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   const int wr = wave >> 1, wc = wave & 1;
 
   // ---- XCD-aware grouped tile order (as gemm_kernel) ---------------------
-  // Paired split-K (g.pair): workgroups [0, dp_tiles) run whole tiles, the rest run the
-  // remaining tiles as pairs of k halves (2 workgroups per tile) — the last partial wave
-  // of a grid at half length instead of full (8B gate|up at 2048 tokens: 896 tiles =
-  // 3 full waves + 128 paired tiles), or every tile paired when there are too few.
+  // Pieces (g.pieces): workgroups [0, dp_tiles) run whole tiles, the rest run the remaining tiles
+  // in equal k pieces — the last partial wave of a grid at a fraction of its length (8B gate|up
+  // at 2048 tokens: 896 tiles = 3 full waves + 128 tiles in halves), or every tile in pieces
+  // when there are too few.  Equal pieces of all tiles walk k side by side and share their
+  // operands in L2; one line of k steps cut into 256 equal shares (a tile's pieces at any k)
+  // balanced better and ran at half the rate, every workgroup reading for itself.
   const int ntiles = g.tiles_m * g.tiles_n;
-  int id, split = blockIdx.y;
+  int id, split = blockIdx.y, piece = 0;
+  int kb = split * g.kps, ke = min(g.K, kb + g.kps);
   {
     const int bid = blockIdx.x;
-    const int dp = g.pair ? g.dp_tiles : ntiles;
+    const int dp = g.pieces ? g.dp_tiles : ntiles;
     if (bid < dp) {
       const int q = dp / 8, r = dp % 8, x = bid % 8, i = bid / 8;
       id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
-      if (g.pair) split = -1;  // a whole tile
+      if (g.pieces) {  // a whole tile
+        kb = 0;
+        ke = g.K;
+      }
     } else {
-      id = dp + (bid - dp) / 2;
-      split = (bid - dp) & 1;
+      id = dp + (bid - dp) / g.pieces;
+      piece = (bid - dp) % g.pieces;
+      kb = piece * g.kps;
+      ke = min(g.K, kb + g.kps);
     }
   }
+  const int pieces = (int)blockIdx.x >= (g.pieces ? g.dp_tiles : ntiles) ? g.pieces : 1;
   constexpr int GROUP = 8;
   const int per_group = GROUP * g.tiles_n;
   const int first_m = (id / per_group) * GROUP;
   const int gm = min(GROUP, g.tiles_m - first_m);
   const int m0 = (first_m + (id % per_group) % gm) * BM;
   const int n0 = ((id % per_group) / gm) * BN;
-  const int kb = split < 0 ? 0 : split * g.kps;
-  const int ke = split < 0 ? g.K : min(g.K, kb + g.kps);
   const int nk = (ke - kb) / kGBK;
 
   // ---- DMA: instruction i of this wave fills LDS rows i*32 + wave*8 + [0, 8) (A rows
@@ -304,6 +311,8 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
         }
       });
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      // the last MFMAs' results settle before the loop is left: a spill may read them first thing
+      if (t + 1 == nk) asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       buf = nbuf;
     }
@@ -372,6 +381,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
     });
     CAKE_STAMP(t3);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (t + 1 == nk) asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");  // (as above)
     __builtin_amdgcn_sched_barrier(0);
     buf = nbuf;
 #ifdef CAKE_GEMM_STAMPS
@@ -396,48 +406,48 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   for (int j = 0; j < FN; ++j) asm volatile("" : "+a"(acc[FM - 1][j]));
   __builtin_amdgcn_s_waitcnt(vm_wait(0));
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  const float4* padd = nullptr;
-  if (g.pair && split >= 0) {
-    // split-K pair: ticket per tile (agent scope).  The first arrival stores its
-    // accumulators to the tile's slab ([i][j][thread] float4, coalesced), releases and
-    // raises the ready flag, and is done; the second waits for the flag (the first is
-    // already past its ticket, so it is running: no residency assumption), acquires,
-    // adds the slab and runs the epilogue, then clears the tile's counters for the next
-    // launch.  a + b in either order: the same bits whichever split arrives first.
-    const int pid = id - g.dp_tiles;  // this pair's slot
-    unsigned* tk = g.tick + pid;
-    unsigned* fl = g.tick + kPairTiles + pid;
+  Pieces add{};
+  if (pieces > 1) {
+    // Counters per tile (agent scope).  Every piece but the last to arrive stores its
+    // accumulators to its slab ([i][j][thread] float4, coalesced; agent scope, so no fence has to
+    // write an XCD's L2 back), counts itself ready once they are there and is done; the last
+    // waits for the others (they are past their arrival, so they are running: no residency
+    // assumption), sums the pieces while it stages the strips, and clears the counters for the
+    // next launch.  Two pieces are summed in either
+    // order; of more the last parks its own too, and all are summed in piece order: the same
+    // bits whichever arrives last.
+    const int tile = id - g.dp_tiles;
+    unsigned* tk = g.tick + tile;
+    unsigned* fl = g.tick + kPieceTiles + tile;
     volatile uint32_t* bc = reinterpret_cast<volatile uint32_t*>(smem + 2 * BUF - 16);
     if (tid == 0) bc[0] = __hip_atomic_fetch_add(tk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    const bool first = bc[0] == 0;
-    float4* slab = reinterpret_cast<float4*>(g.ws + (size_t)pid * (BM * BN)) + tid;
-    if (first) {
+    const bool last = bc[0] == (uint32_t)(pieces - 1);
+    float4* slab = reinterpret_cast<float4*>(g.ws + (size_t)tile * pieces * (BM * BN)) + tid;
+    if (!last || pieces > 2) {
+      float4* to = slab + (size_t)piece * (BM * BN / 4);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
           const cf32x4 v = acc[i][j];
-          slab[(i * FN + j) * 256] = make_float4(v[0], v[1], v[2], v[3]);
+          st_agent16(to + (i * FN + j) * 256, v[0], v[1], v[2], v[3]);
         }
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-      if (tid == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __hip_atomic_store(fl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+    }
+    if (!last) {
+      if (tid == 0) __hip_atomic_fetch_add(fl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return;
     }
     if (tid == 0) {
-      while (__hip_atomic_load(fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+      while (__hip_atomic_load(fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)(pieces - 1))
         __builtin_amdgcn_s_sleep(2);
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __hip_atomic_store(tk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(fl, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    padd = slab;  // the epilogue strips add the first split's accumulators
+    add = Pieces{pieces > 2 ? slab : slab + (size_t)(1 - piece) * (BM * BN / 4),
+                 (size_t)(BM * BN / 4), pieces};
   }
   float* stg = reinterpret_cast<float*>(smem + wave * STG);
   const int row_m0 = m0 + wr * WTM;
@@ -456,14 +466,16 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
     // after the reads of the strip before it needs no wait)
     float* sg0 = reinterpret_cast<float*>(smem + (wave * 2) * STG);
     float* sg1 = reinterpret_cast<float*>(smem + (wave * 2 + 1) * STG);
-    stage_strip_w<FN>(acc[0], sg0, lane, padd);
+    const auto strip = [&](int i) {   // the pieces' float4s of strip i
+      return Pieces{add.base + i * FN * 256, add.stride, add.n};
+    };
+    stage_strip_w<FN>(acc[0], sg0, lane, add);
     static_for<0, FM>([&](auto ii) __attribute__((always_inline)) {
       constexpr int i = decltype(ii)::value;
       __builtin_amdgcn_s_waitcnt(0xc07f);
       __builtin_amdgcn_wave_barrier();
       if constexpr (i + 1 < FM) {
-        stage_strip_w<FN>(acc[i + 1], (i & 1) ? sg0 : sg1, lane,
-                          padd ? padd + (i + 1) * FN * 256 : nullptr);
+        stage_strip_w<FN>(acc[i + 1], (i & 1) ? sg0 : sg1, lane, strip(i + 1));
         ops.template load_res<(i + 1) & 1>(g, row_m0 + (i + 1) * 16, vcol0, lane);
       }
       readout_strip_w<DT, EPI, FN, i & 1>(g, (i & 1) ? sg1 : sg0, row_m0 + i * 16, vcol0, split,
@@ -482,7 +494,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       if constexpr (i + 1 < FM)
         ops.template load_res<(i + 1) & 1>(g, row_m0 + (i + 1) * 16 + (lane >> 2), vcol0, lane);
       epi_strip<DT, EPI, FN, i & 1>(g, acc[i], stg, row_m0 + i * 16, vcol0, split, lane, ops,
-                                    padd ? padd + i * FN * 256 : nullptr);
+                                    Pieces{add.base + i * FN * 256, add.stride, add.n});
     });
   }
 #ifdef CAKE_GEMM_STAMPS

@@ -69,19 +69,45 @@ struct GemmArgs {
   int gated;             // B row order interleaves 16-row blocks of two halves
   int tiles_m, tiles_n, kps;  // k elements per split
   float alpha = 1.f;     // kEpiResid32 / kEpiStore32: factor of the product (and bias)
-  // in-kernel split-K pair (gemm_4w.h, splits == 2): the first split of a tile to finish
-  // parks its accumulators in ws (one 256x256 f32 slab per tile), the second adds them and
-  // runs the epilogue; tick = [kPairTiles arrival counters | kPairTiles ready flags]
-  int pair;
-  unsigned* tick;
-  int dp_tiles;          // pair: tiles [0, dp_tiles) run whole, the rest as k-half pairs
+  // in-kernel split-K (gemm_4w.h): tiles [0, dp_tiles) run whole, the rest in `pieces` (0: none)
+  // pieces of kps k elements; every piece of a tile but the last to arrive parks its accumulators
+  // in ws, the last sums them in piece order and runs the epilogue; tick = [kPieceTiles arrival
+  // counters | kPieceTiles ready counters]
+  int pieces;
+  unsigned* tick;        // (gemm_rows.h: one arrival counter per strip)
+  int dp_tiles;
   // grouped products (gemm_inst_grouped.hip): row tile tm is [weight group, first row, rows, -]
   // of this list instead of rows tm BM .., its weights b + group b_group; entry tiles_m holds
   // the number of tiles
   const int4* groups;
   long long b_group;
 };
-constexpr int kPairTiles = 16384;
+constexpr int kPieceTiles = 256;
+
+// 16 bytes past the caches that other XCDs do not see (agent scope, two 8-byte accesses)
+__device__ __forceinline__ void st_agent16(float4* p, float x, float y, float z, float w) {
+  unsigned long long* q = reinterpret_cast<unsigned long long*>(p);
+  __hip_atomic_store(q, (unsigned long long)__float_as_uint(y) << 32 | __float_as_uint(x),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, (unsigned long long)__float_as_uint(w) << 32 | __float_as_uint(z),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float4 ld_agent16(const float4* p) {
+  const unsigned long long* q = reinterpret_cast<const unsigned long long*>(p);
+  const unsigned long long a = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long b = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return make_float4(__uint_as_float((unsigned)a), __uint_as_float((unsigned)(a >> 32)),
+                     __uint_as_float((unsigned)b), __uint_as_float((unsigned)(b >> 32)));
+}
+
+// a tile's pieces (gemm_4w.h): n 0, the tile is whole; 2, this wave's accumulators and the parked
+// ones at base; more, all parked, stride float4s apart.  base: this thread's float4s of the current
+// strip, tile j of it at base[j * 256]
+struct Pieces {
+  const float4* base;
+  size_t stride;
+  int n;
+};
 
 // virtual B row -> weight row (gated: [16 gate rows | 16 up rows] per 32-row block)
 __device__ __forceinline__ int wrow(const GemmArgs& g, int v) {
@@ -245,16 +271,54 @@ __device__ __forceinline__ void store16(uint16_t* dst, const uint16_t* v, bool f
   }
 }
 
+// a strip's accumulators (with the tile's other pieces, in piece order: the same bits whichever
+// arrived last) into the wave's staging slice
+template <int NF>
+__device__ __forceinline__ void stage_strip_w(const cf32x4 (&tiles)[NF], float* stg, int lane,
+                                              const Pieces& add) {
+  constexpr int STG_LD = NF * 16 + 4;
+  const auto put = [&](int j, float x, float y, float z, float w) {
+    float* at = stg + (lane >> 4) * 4 * STG_LD + j * 16 + (lane & 15);
+    at[0] = x;
+    at[STG_LD] = y;
+    at[2 * STG_LD] = z;
+    at[3 * STG_LD] = w;
+  };
+  if (add.n > 2) {   // all of them parked
+    float4 v[NF];
+#pragma unroll
+    for (int j = 0; j < NF; ++j) v[j] = ld_agent16(add.base + j * 256);
+    for (int q = 1; q < add.n; ++q) {
+      const float4* src = add.base + q * add.stride;
+#pragma unroll
+      for (int j = 0; j < NF; ++j) {
+        const float4 o = ld_agent16(src + j * 256);
+        v[j].x += o.x; v[j].y += o.y; v[j].z += o.z; v[j].w += o.w;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NF; ++j) put(j, v[j].x, v[j].y, v[j].z, v[j].w);
+  } else if (add.n == 2) {
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+      const float4 o = ld_agent16(add.base + j * 256);
+      put(j, tiles[j][0] + o.x, tiles[j][1] + o.y, tiles[j][2] + o.z, tiles[j][3] + o.w);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NF; ++j) put(j, tiles[j][0], tiles[j][1], tiles[j][2], tiles[j][3]);
+  }
+}
+
 // One 16-row strip of a wave's output (NF 16x16 accumulator tiles = NF*16 virtual
 // columns starting at vcol0), staged through the wave's LDS slice stg and written
 // with the epilogue EPI (bias / residual from ops, buffer B).
-// add (split-K pair, gemm_4w.h): this thread's parked partner accumulators of the strip,
-// float4 j at add[j * 256], summed in before staging
+// add: the tile's other pieces, summed in before staging
 template <int DT, int EPI, int NF, int B>
 __device__ __forceinline__ void epi_strip(const GemmArgs& g, const cf32x4 (&tiles)[NF], float* stg,
                                           int m_strip0, int vcol0, int split, int lane,
                                           const EpiOps<DT, EPI, NF>& ops,
-                                          const float4* add = nullptr) {
+                                          const Pieces add = {}) {
   constexpr int WTN = NF * 16;
   constexpr int STG_LD = WTN + 4;
   constexpr bool GATED = (EPI == kEpiSwiglu || EPI == kEpiGeglu);
@@ -262,22 +326,7 @@ __device__ __forceinline__ void epi_strip(const GemmArgs& g, const cf32x4 (&tile
   constexpr int CPL = OUTC / 4;                // columns per lane (4 lanes per row)
   const int er = lane >> 2, ec = (lane & 3) * CPL;
   {
-    if (add) {
-#pragma unroll
-      for (int j = 0; j < NF; ++j) {
-        const float4 o = add[j * 256];
-        const float ov[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          stg[((lane >> 4) * 4 + e) * STG_LD + j * 16 + (lane & 15)] = tiles[j][e] + ov[e];
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < NF; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          stg[((lane >> 4) * 4 + e) * STG_LD + j * 16 + (lane & 15)] = tiles[j][e];
-    }
+    stage_strip_w<NF>(tiles, stg, lane, add);
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
     const int m = m_strip0 + er;
@@ -448,29 +497,6 @@ template <int DT, int EPI, int NF> struct EpiW {
     }
   }
 };
-
-// a strip's accumulators (+ the split-K partner's, add) into the wave's staging slice
-template <int NF>
-__device__ __forceinline__ void stage_strip_w(const cf32x4 (&tiles)[NF], float* stg, int lane,
-                                              const float4* add) {
-  constexpr int STG_LD = NF * 16 + 4;
-  if (add) {
-#pragma unroll
-    for (int j = 0; j < NF; ++j) {
-      const float4 o = add[j * 256];
-      const float ov[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        stg[((lane >> 4) * 4 + e) * STG_LD + j * 16 + (lane & 15)] = tiles[j][e] + ov[e];
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < NF; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        stg[((lane >> 4) * 4 + e) * STG_LD + j * 16 + (lane & 15)] = tiles[j][e];
-  }
-}
 
 // a staged strip read out 8 lanes per row and written with the epilogue EPI
 template <int DT, int EPI, int NF, int B>
@@ -845,7 +871,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs g) {
     static_for<0, FM>([&](auto ii) __attribute__((always_inline)) {
       constexpr int i = decltype(ii)::value;
       if constexpr (i + 1 < FM) ops.template load_res<(i + 1) & 1>(g, row_m0 + (i + 1) * 16, vcol0, lane);
-      stage_strip_w<FN>(acc[i], stg, lane, nullptr);
+      stage_strip_w<FN>(acc[i], stg, lane, Pieces{});
       __builtin_amdgcn_s_waitcnt(0xc07f);
       __builtin_amdgcn_wave_barrier();
       readout_strip_w<DT, EPI, FN, i & 1>(g, stg, row_m0 + i * 16, vcol0, split, lane, ops);

@@ -291,18 +291,11 @@ __device__ __forceinline__ void stream_store(const GemmArgs& g, const StreamStri
 }
 
 __device__ __forceinline__ void park(float* p, const cf32x4& v) {
-  const unsigned long long lo = (unsigned long long)__float_as_uint(v[1]) << 32 | __float_as_uint(v[0]);
-  const unsigned long long hi = (unsigned long long)__float_as_uint(v[3]) << 32 | __float_as_uint(v[2]);
-  unsigned long long* q = reinterpret_cast<unsigned long long*>(p);
-  __hip_atomic_store(q, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(q + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  st_agent16(reinterpret_cast<float4*>(p), v[0], v[1], v[2], v[3]);
 }
 __device__ __forceinline__ cf32x4 unpark(const float* p) {
-  const unsigned long long* q = reinterpret_cast<const unsigned long long*>(p);
-  const unsigned long long lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const unsigned long long hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return cf32x4{__uint_as_float((unsigned)lo), __uint_as_float((unsigned)(lo >> 32)),
-                __uint_as_float((unsigned)hi), __uint_as_float((unsigned)(hi >> 32))};
+  const float4 v = ld_agent16(reinterpret_cast<const float4*>(p));
+  return cf32x4{v.x, v.y, v.z, v.w};
 }
 
 template <int DT, int EPI, int MT, bool GRP>

@@ -67,6 +67,8 @@ def _lib():
         lib.cake_gemm_ws_floats.restype = L
         lib.cake_gemm_grouped.argtypes = [I, I, I, P, L, P, L, L, P, L, P, I, P, I, I, P]
         lib.cake_gemm_grouped.restype = I
+        lib.cake_gemm_plan.argtypes = [I, L, I, I, I, P, P]
+        lib.cake_gemm_plan.restype = I
         lib.cake_gemm_rows_kind.argtypes = [I, L, I, I]
         lib.cake_gemm_rows_kind.restype = I
         lib.cake_gemm_rows_ws_floats.argtypes = [I]
@@ -103,13 +105,14 @@ _ws_keep: list = []
 
 
 def _workspace(dev, numel: int) -> torch.Tensor:
-    """Split-K slabs.  Superseded buffers are kept alive: a captured hipGraph may
-    still point at them."""
-    w = _ws.get(dev)
+    """Split-K slabs of the current stream (launches on two streams may run side by side).
+    Superseded buffers are kept alive: a captured hipGraph may still point at them."""
+    key = (dev, torch.cuda.current_stream(dev).cuda_stream)
+    w = _ws.get(key)
     if w is None or w.numel() < numel:
         if w is not None:
             _ws_keep.append(w)
-        w = _ws[dev] = torch.empty(max(numel, 1 << 20), dtype=torch.float32, device=dev)
+        w = _ws[key] = torch.empty(max(numel, 1 << 20), dtype=torch.float32, device=dev)
     return w
 
 
@@ -207,15 +210,41 @@ def set_plan(M: int, N: int, K: int, epi: str, cfg: int, splits: int) -> None:
 
 
 def plan(M: int, Nv: int, K: int, epi: str = "store") -> tuple[int, int]:
-    """(cfg, splits) for an M x Nv x K problem (Nv = weight rows read)."""
+    """(cfg, splits) by the measured table and its neighbours (Nv = weight rows read): the split
+    of a call that names its tile; :func:`resolve` plans the others."""
     p = _plans.get((M, Nv, K, epi))
     if p is not None:
         return p
     p = _tuned(M, Nv, K, epi)
+    return p if p is not None else _cost_plan(M, Nv, K)
+
+
+def resolve(M: int, Nv: int, K: int, epi: str, big: bool) -> tuple[int, int]:
+    """(cfg, splits) that :func:`linear` runs: a pinned plan, the measured one of this very size
+    unless the kernel library's estimate puts it well behind, else the estimate's best
+    (gemm.hip cake_gemm_plan, shared with the native engines)."""
+    p = _plans.get((M, Nv, K, epi))
     if p is not None:
-        _plans[(M, Nv, K, epi)] = p
         return p
-    return _cost_plan(M, Nv, K)
+    key = (M, Nv, K, epi, big)
+    p = _resolved.get(key)
+    if p is None:
+        if len(_resolved) >= 65536:   # as many sizes as a long-lived server meets
+            _resolved.clear()
+        e = next((e for e in _TUNED if e["M"] == M and e["Nv"] == Nv and e["K"] == K
+                  and e["epi"] == epi), None)
+        cfg, sp = C.c_int(-1 if e is None else e["cfg"]), C.c_int(1 if e is None else e["splits"])
+        if cfg.value == LIB and e is not None:
+            p = (LIB, 1)
+        else:
+            check(_lib().cake_gemm_plan(M, Nv, K, EPI[epi], int(big), C.addressof(cfg),
+                                        C.addressof(sp)), "gemm_plan")
+            p = (cfg.value, sp.value)
+        _resolved[key] = p
+    return p
+
+
+_resolved: dict = {}
 
 
 def _cost_plan(M: int, Nv: int, K: int) -> tuple[int, int]:
@@ -353,8 +382,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
                 None if ws is None else ws.data_ptr(), None if tick is None else tick.data_ptr(),
                 _zeros16(x.device).data_ptr(), M, N, K, float(alpha), st), "gemm_rows")
             return resid if f32_out else out
-    c0, s0 = plan(M, Nv, K, epi)
-    cfg = c0 if cfg is None else cfg
+    s0 = 1
+    if cfg is None:
+        big = max((M - 1) * lda + K, (Nv - 1) * ldb + K) * 2 >= 0x7fffffff
+        cfg, s0 = resolve(M, Nv, K, epi, big)
+    elif splits is None:
+        s0 = plan(M, Nv, K, epi)[1]
     lib_ok = epi != "swiglu" or (ldc == N and N % 8 == 0 and out2.data_ptr() % 16 == 0)
     if cfg == LIB and bias is None and epi in LIB_EPIS and lib_ok and alpha == 1.0:
         _lib_gemm(x2, lda, w, ldb, epi, out2, ldc, r2 if f32_out else None, ldr, M, N, K)

@@ -1,0 +1,50 @@
+"""Estimated tile plans (gemm.hip cake_gemm_plan): what they pick can run, at every size."""
+import random
+
+import pytest
+
+from cake_amd.build import GEMM_LIB
+
+pytestmark = pytest.mark.skipif(not GEMM_LIB.exists(), reason="native libraries not built")
+
+
+def test_estimated_plans_can_run():
+    from cake_amd.ops import gemm as G
+    rng = random.Random(4)
+    epis = list(G.EPI)
+    for _ in range(3000):
+        M = int(2 ** rng.uniform(0, 17))
+        Nv = 32 * int(2 ** rng.uniform(0, 12))
+        K = 8 * int(2 ** rng.uniform(0, 13))
+        epi, big = rng.choice(epis), rng.random() < 0.2
+        cfg, splits = G.resolve(M, Nv, K, epi, big)
+        assert cfg in G.CFG_TILES and 1 <= splits <= 16
+        if cfg in G.K64_ONLY:
+            assert K % 64 == 0 and not big
+        if epi in ("swiglu", "geglu"):
+            assert cfg not in G.NO_GATED
+        if splits > 1:
+            assert -(-K // 64) // splits >= 4
+
+
+def test_measured_entry_of_the_size_stands_unless_well_behind(monkeypatch):
+    from cake_amd.ops import gemm as G
+
+    def at(cfg, splits):
+        monkeypatch.setattr(G, "_TUNED", [{"M": 2048, "Nv": 4096, "K": 4096, "epi": "store",
+                                           "cfg": cfg, "splits": splits}])
+        monkeypatch.setattr(G, "_resolved", {})
+        return G.resolve(2048, 4096, 4096, "store", False)
+    assert at(27, 1) == (27, 1)     # close to the best estimate
+    assert at(13, 1) != (13, 1)     # 64 x 64 tiles of a large product
+    assert at(20, 1) == (20, 1)     # a tile the estimate does not cover
+
+
+def test_workspace_covers_the_pieces():
+    """Tiles in pieces need a slab each; whole tiles need none."""
+    from cake_amd.ops import gemm as G
+    L = G._lib()
+    assert L.cake_gemm_ws_floats(22, 4, 777, 4096, 14336, 0) == 64 * 4 * 256 * 256
+    assert L.cake_gemm_ws_floats(25, 8, 4500, 4096, 14336, 0) == 32 * 8 * 256 * 256   # 288 tiles
+    assert L.cake_gemm_ws_floats(27, 2, 1100, 4096, 14336, 0) == 0                     # 144 tiles
+    assert L.cake_gemm_ws_floats(22, 2, 2048, 8192, 8192, 0) == 0                      # one wave
