@@ -85,7 +85,11 @@ __device__ __forceinline__ void amfma_dma(cf32x4& acc, const uint4& a, const uin
 
 // SCHED 1 (cfg 25-27): the same tiles on a three-barrier schedule (the DMAs of step t+2
 // issued as soon as every wave has read the operand region they overwrite).
-template <int DT, int EPI, int BM, int BN, int SCHED = 0>
+// GRP: grouped row tiles (GemmArgs::groups), K any multiple of 8.  Bound by the matrix cores on
+// padded rows and, below some 200 rows a group, by reading the weights: 64 groups of 192 rows,
+// 4096 -> 3616 -> 4096 columns, 1102 -> 989 us against eight waves on the same tile (0.98 PFLOP/s
+// with the padding; the weights alone are 2 x 292 us).
+template <int DT, int EPI, int BM, int BN, int SCHED = 0, bool GRP = false>
 __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   static_assert((BM == 256 && (BN == 256 || BN == 192)) || (BM == 128 && BN == 256),
                 "four-wave tile shapes");
@@ -113,7 +117,12 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   // when there are too few.  Equal pieces of all tiles walk k side by side and share their
   // operands in L2; one line of k steps cut into 256 equal shares (a tile's pieces at any k)
   // balanced better and ran at half the rate, every workgroup reading for itself.
+  if constexpr (GRP) {
+    g.tiles_m = g.groups[g.tiles_m].x;
+    g.pieces = 0;
+  }
   const int ntiles = g.tiles_m * g.tiles_n;
+  if (GRP && (int)blockIdx.x >= ntiles) return;
   int id, split = blockIdx.y, piece = 0;
   int kb = split * g.kps, ke = min(g.K, kb + g.kps);
   {
@@ -134,25 +143,38 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
     }
   }
   const int pieces = (int)blockIdx.x >= (g.pieces ? g.dp_tiles : ntiles) ? g.pieces : 1;
-  constexpr int GROUP = 8;
+  // grouped products: most groups have one or two row tiles, so two of them walk all columns and
+  // their rows are read once (eight read every row four times over; 64 groups of 192 rows of 4096
+  // to 3616 columns 509 -> 483 us, back 543 -> 506)
+  constexpr int GROUP = GRP ? 2 : 8;
   const int per_group = GROUP * g.tiles_n;
   const int first_m = (id / per_group) * GROUP;
   const int gm = min(GROUP, g.tiles_m - first_m);
-  const int m0 = (first_m + (id % per_group) % gm) * BM;
+  const int tm = first_m + (id % per_group) % gm;
+  const int m0 = GRP ? 0 : tm * BM;
   const int n0 = ((id % per_group) / gm) * BN;
-  const int nk = (ke - kb) / kGBK;
+  if constexpr (GRP) {
+    const int4 t = g.groups[tm];
+    g.a += (size_t)t.y * g.lda;
+    g.c += (size_t)t.y * g.ldc;
+    g.b += (size_t)t.x * g.b_group + (size_t)n0 * g.ldb;
+    g.M = min(t.z, BM);
+  }
+  const int nk = GRP ? (ke - kb + kGBK - 1) / kGBK : (ke - kb) / kGBK;
 
   // ---- DMA: instruction i of this wave fills LDS rows i*32 + wave*8 + [0, 8) (A rows
   // for i < NA, B rows after); lane l -> row + l/8, slot l%8 holding source chunk
   // (l%8) ^ ((row >> 1) & 7), the same for every i
   const int rA = wave * 8 + (lane >> 3);
   const int chunk = (lane & 7) ^ ((rA >> 1) & 7);
-  const long long brows = g.gated ? 2LL * g.half : (long long)g.Nv;
+  // (grouped: weights from this tile's first row on, so that a tile, not a weight, is under 2 GB)
+  const long long brows = GRP ? min(BN, g.Nv - n0) : g.gated ? 2LL * g.half : (long long)g.Nv;
   const int nrec_a = (int)(((long long)(g.M - 1) * g.lda + g.K) * 2);
   const int nrec_b = (int)(((brows - 1) * g.ldb + g.K) * 2);
   const uint32_t voff_a = (uint32_t)(((long long)(m0 + rA) * g.lda + chunk * 8) * 2);
   long long brow0;  // weight row of this lane in B group 0
-  if (!g.gated) brow0 = n0 + rA;
+  if constexpr (GRP) brow0 = rA;
+  else if (!g.gated) brow0 = n0 + rA;
   else brow0 = (rA < 16 ? 0LL : (long long)g.half - 16) + n0 / 2 + rA;
   const uint32_t voff_b = (uint32_t)((brow0 * g.ldb + chunk * 8) * 2);
   // scalar byte offsets of each 32-row group (A: 32 rows; B: 32 virtual rows = 16
@@ -182,7 +204,17 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   auto dma_mb = [&](int buf) __attribute__((always_inline)) {
     return m0_base + (uint32_t)(buf * BUF);
   };
-  auto dma_voff = [&](int i) __attribute__((always_inline)) { return i < NA ? voff_a : voff_b; };
+  // GRP: the last step of a K that is no multiple of 64 reads its missing chunks out of range
+  // (the descriptors only bound the matrix, a row's end lies inside it)
+  uint32_t cur_a = voff_a, cur_b = voff_b;
+  auto tail_step = [&](int step) __attribute__((always_inline)) {
+    if constexpr (GRP) {
+      const bool in = step * kGBK + chunk * 8 < g.K;
+      cur_a = in ? voff_a : 0x80000000u;
+      cur_b = in ? voff_b : 0x80000000u;
+    }
+  };
+  auto dma_voff = [&](int i) __attribute__((always_inline)) { return i < NA ? cur_a : cur_b; };
   auto dma_soff = [&](int i) __attribute__((always_inline)) {
     return i < NA ? (uint32_t)i * gstride_a : (uint32_t)(i - NA) * gstride_b;
   };
@@ -199,6 +231,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   };
   auto stage = [&](int step, int buf) {
     const cu32x4 sa = src_a(step), sb = src_b(step);
+    tail_step(step);
     static_for<0, IPW>([&](auto I) __attribute__((always_inline)) { stage_one(sa, sb, buf, I); });
   };
 
@@ -247,6 +280,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       const int nbuf = buf ^ 1;
       const uint32_t na = a_base + nbuf * BUF, nb = b_base + nbuf * BUF;
       const cu32x4 sa = src_a(t + 2), sb = src_b(t + 2);
+      tail_step(t + 2);
       // ops k of n spread over MFMAs [lo, hi): op k after MFMA lo + floor(k (hi-lo) / n)
       static_for<0, NM>([&](auto mi) __attribute__((always_inline)) {
         constexpr int m = decltype(mi)::value;
@@ -362,6 +396,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
     CAKE_STAMP(t2);
     const uint32_t na = a_base + nbuf * BUF, nb = b_base + nbuf * BUF;
     const cu32x4 sa = src_a(t + 2), sb = src_b(t + 2);
+    tail_step(t + 2);
     static_for<0, NM>([&](auto mi) __attribute__((always_inline)) {
       constexpr int m = decltype(mi)::value;
       constexpr int l0 = (m * NL + NM - 1) / NM, l1 = ((m + 1) * NL + NM - 1) / NM;
@@ -407,7 +442,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   __builtin_amdgcn_s_waitcnt(vm_wait(0));
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   Pieces add{};
-  if (pieces > 1) {
+  if (!GRP && pieces > 1) {
     // Counters per tile (agent scope).  Every piece but the last to arrive stores its
     // accumulators to its slab ([i][j][thread] float4, coalesced; agent scope, so no fence has to
     // write an XCD's L2 back), counts itself ready once they are there and is done; the last

@@ -4,19 +4,24 @@
 
 namespace cake {
 
+constexpr long long kWide = 1 << 22;  // elements: 256 rows of this stride are 2 GB
+
+// Tiles by rows: 64 (cfg 4), 128 (0), 256 (5); the last two on four waves (gemm_4w.h).  Rows too
+// far apart for its 32-bit offsets take the 64-row tile, in passes.
 template <int DT, int EPI>
-static int launch_grouped(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
-#define X(id, BM, BN, WM, WN, NS, PR)                                                      \
-  if (cfg == id) {                                                                         \
-    hipLaunchKernelGGL((gemm_kernel<DT, BM, BN, WM, WN, NS, EPI, PR, true>), grid,         \
-                       dim3(64 * WM * WN), 0, st, g);                                      \
-    return (int)hipGetLastError();                                                         \
-  }
-  X(0, 128, 128, 2, 2, 2, 6)
-  X(4, 64, 64, 2, 2, 2, 6)
-  X(5, 256, 256, 2, 4, 2, 6)
-#undef X
-  return (int)hipErrorInvalidValue;
+static int launch_grouped(int cfg, int tiles, hipStream_t st, GemmArgs& g) {
+  const int bm = cfg == 4 ? 64 : cfg == 0 ? 128 : 256;
+  const bool wide = g.lda >= kWide || g.ldb >= kWide;
+  const int bn = bm == 64 || wide ? 64 : 256;
+  g.tiles_n = (g.N + bn - 1) / bn;
+  const dim3 grid(tiles * g.tiles_n, wide ? bm / 64 : 1);
+  if (bn == 64)
+    hipLaunchKernelGGL((gemm_kernel<DT, 64, 64, 2, 2, 2, EPI, 6, true>), grid, dim3(256), 0, st, g);
+  else if (bm == 128)
+    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 128, 256, 1, true>), grid, dim3(256), 0, st, g);
+  else
+    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 256, 256, 1, true>), grid, dim3(256), 0, st, g);
+  return (int)hipGetLastError();
 }
 
 }  // namespace cake
@@ -31,28 +36,25 @@ CAKE_API int cake_gemm_grouped(int dt, int epi, int cfg, const void* a, long lon
                                const void* tiles, int max_tiles, const void* zeros, int N, int K,
                                hipStream_t st) {
   if (max_tiles <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || b_group % 8 ||
-      !(epi == 0 || (epi >= 7 && epi <= 10)))
+      !(epi == 0 || (epi >= 7 && epi <= 10)) || !(cfg == 0 || cfg == 4 || cfg == 5))
     return (int)hipErrorInvalidValue;
-  const int bn = cfg == 4 ? 64 : cfg == 5 ? 256 : 128;
   GemmArgs g{};
   g.a = (const uint16_t*)a; g.b = (const uint16_t*)b; g.c = (uint16_t*)c;
   g.zeros = (const uint16_t*)zeros;
   g.lda = lda; g.ldb = ldb; g.ldc = ldc;
   g.N = N; g.K = K; g.Nv = N; g.half = N;
   g.tiles_m = max_tiles;
-  g.tiles_n = (N + bn - 1) / bn;
   g.kps = (K + kGBK - 1) / kGBK * kGBK;
   g.groups = (const int4*)tiles;
   g.b_group = b_group;
-  const dim3 grid(g.tiles_m * g.tiles_n, 1);
   const auto run = [&](auto dtc) {
     constexpr int DT = decltype(dtc)::value;
     switch (epi) {
-      case kEpiStore: return launch_grouped<DT, kEpiStore>(cfg, grid, st, g);
-      case kEpiSilu: return launch_grouped<DT, kEpiSilu>(cfg, grid, st, g);
-      case kEpiQuick: return launch_grouped<DT, kEpiQuick>(cfg, grid, st, g);
-      case kEpiGelu: return launch_grouped<DT, kEpiGelu>(cfg, grid, st, g);
-      case kEpiRelu2: return launch_grouped<DT, kEpiRelu2>(cfg, grid, st, g);
+      case kEpiStore: return launch_grouped<DT, kEpiStore>(cfg, max_tiles, st, g);
+      case kEpiSilu: return launch_grouped<DT, kEpiSilu>(cfg, max_tiles, st, g);
+      case kEpiQuick: return launch_grouped<DT, kEpiQuick>(cfg, max_tiles, st, g);
+      case kEpiGelu: return launch_grouped<DT, kEpiGelu>(cfg, max_tiles, st, g);
+      case kEpiRelu2: return launch_grouped<DT, kEpiRelu2>(cfg, max_tiles, st, g);
     }
     return (int)hipErrorInvalidValue;
   };

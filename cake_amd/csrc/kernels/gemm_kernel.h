@@ -654,12 +654,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs g) {
   const int m0 = GRP ? 0 : tm * BM, n0 = tn * BN;
   if constexpr (GRP) {
     const int4 t = g.groups[tm];
-    g.a += (size_t)t.y * g.lda;
-    g.c += (size_t)t.y * g.ldc;
+    const int r0 = blockIdx.y * BM;   // tiles of more rows in passes of BM
+    if (r0 >= t.z) return;
+    g.a += (size_t)(t.y + r0) * g.lda;
+    g.c += (size_t)(t.y + r0) * g.ldc;
     g.b += (size_t)t.x * g.b_group;
-    g.M = min(t.z, BM);
+    g.M = min(t.z - r0, BM);
   }
-  const int split = blockIdx.y;
+  const int split = GRP ? 0 : blockIdx.y;
   const int kb = split * g.kps, ke = min(g.K, kb + g.kps);
   const int nk = (ke - kb + kGBK - 1) / kGBK;
 

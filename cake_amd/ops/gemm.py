@@ -413,10 +413,15 @@ GROUPED_CFGS = {0: 128, 4: 64, 5: 256, ROWS: 16}
 
 def grouped_cfg(rows: int, groups: int, capturing: bool = False) -> int:
     """Tile configuration for `rows` sorted rows over `groups` weight groups."""
+    # up and down product of 64 experts 4096 x 3616, us in the stream form and at 64 / 128 / 256 rows
+    # a tile, by rows an expert: 3 561 / 651 / 646 / -, 6 644 / 688 / 669 / -, 9 680 / 705 / 672 / -,
+    # 16 938 / 739 / 683 / -, 24 - / 775 / 698 / -, 75 - / 1275 / 766 / 895, 112 - / 1412 / 888 / 937
+    # (skewed 1435 / 984 / 1029), 131 - / 1550 / 1100 / 954, 192 - / 1998 / 1130 / 989; of small
+    # experts the 64-row tile has more workgroups
     mean = rows / groups
     if mean <= 4 and not capturing:   # the stream form's counters stay out of graphs
         return ROWS
-    return 5 if mean >= 96 else 0 if mean >= 24 else 4
+    return 5 if mean >= 115 else 0 if mean >= 12 else 4
 
 
 def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out: torch.Tensor,
