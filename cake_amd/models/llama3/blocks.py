@@ -156,6 +156,13 @@ class LayerStack:
             self._decode_graph(hidden, layers, pos0, session)
             kv.length = max(kv.length, pos0 + 1)
             return hidden
+        if self.backend == "hip" and T > 1:
+            from ...ops.llama_rows import block_rows
+            if block_rows(hidden, [self.weights[li] for li in layers],
+                          [self.slot_of[li] for li in layers], kv.k, kv.v, self.inv_freq, self.cfg,
+                          pos0, self.scale):
+                kv.length = max(kv.length, pos0 + T)
+                return hidden
         for li in layers:
             w = self.weights[li]
             s = self.slot_of[li]

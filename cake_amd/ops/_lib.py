@@ -51,6 +51,7 @@ _SIGS = {
     "cake_embed": [I, P, P, I, I, P, P],
     "cake_rmsnorm": [I, P, P, F, I, I, P, P],
     "cake_rmsnorm_set_reg": [I],
+    "cake_block_rows": [P, P],
     "cake_rope_kv": [I, P, P, P, I, I, I, I, I, I, P, I, I, P, P, P],
     "cake_silu_mul": [I, P, P, Z, P, P],
     "cake_silu_mul_rows": [I, P, Z, I, P, P],

@@ -1,0 +1,100 @@
+"""A run of Llama blocks over several rows as one native call (csrc/driver/block_rows.cpp).
+
+:func:`block_rows` checks the tensors and plans the four products once for the whole run, by the
+rules of :func:`gemm.linear`; it returns False, with nothing launched, for what only the separate
+calls take (a library plan, sizes or layouts outside the kernels' fast forms)."""
+from __future__ import annotations
+
+import ctypes as C
+
+import torch
+
+from . import gemm as G
+from ._lib import check, kernels
+
+P, I, F = C.c_void_p, C.c_int, C.c_float
+
+
+class _Form(C.Structure):
+    _fields_ = [("kind", I), ("cfg", I), ("splits", I)]
+
+
+class _Run(C.Structure):
+    _fields_ = [(n, P) for n in ("blocks", "hidden", "x", "qkv", "att", "act", "inv_freq", "zeros",
+                                 "ws", "rows_ws", "rows_tick")] + \
+               [(n, _Form) for n in ("qkv_form", "o_form", "gu_form", "down_form")] + \
+               [(n, I) for n in ("n", "dt", "T", "H", "I", "nh", "nkv", "hd", "S", "pos0")] + \
+               [("eps", F), ("scale", F)]
+
+
+def _forms(T: int, products, capturing: bool):
+    """(kind, cfg, splits) of each (Nv, K, epi), as gemm.linear chooses them, and the slab floats
+    that the tile plans need; None if one of them is the library GEMM's."""
+    forms, floats = [], 0
+    for Nv, K, epi in products:
+        gated = epi == "swiglu"
+        kind = G.rows_kind(T, Nv, K, gated) if (T, Nv, K, epi) not in G._plans else 0
+        if kind == 2 and capturing:
+            kind = 0
+        cfg, splits = 0, 1
+        if not kind:
+            big = max(T, Nv) * K * 2 >= 0x7fffffff
+            cfg, splits = G.resolve(T, Nv, K, epi, big)
+            if cfg == G.LIB:
+                return None, 0
+            if splits > 1:
+                floats = max(floats, int(G._lib().cake_gemm_ws_floats(
+                    cfg, splits, T, Nv // 2 if gated else Nv, K, int(gated))))
+        forms.append(_Form(kind, cfg, splits))
+    return forms, floats
+
+
+def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Tensor,
+               v: torch.Tensor, inv_freq: torch.Tensor, cfg, pos0: int, scale: float) -> bool:
+    """hidden [T, H] f32 through `blocks` in place; k, v [layers, nkv, S, hd], block i's rows at
+    slots[i]."""
+    T, H = hidden.shape
+    nh, nkv, hd = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+    inter, S, dt = cfg.intermediate_size, k.shape[2], k.dtype
+    nq, nqkv = nh * hd, (nh + 2 * nkv) * hd
+    if dt not in G._DT or T < 1 or nh % nkv or hd % 8 or hd > 256 or H % 8 or inter % 16 or \
+            not hidden.is_cuda or not hidden.is_contiguous() or hidden.data_ptr() % 16 or \
+            not (k.is_contiguous() and v.is_contiguous()) or k.shape != v.shape or \
+            v.dtype != dt or tuple(k.shape[1:]) != (nkv, S, hd) or pos0 < 0 or pos0 + T > S or \
+            tuple(inv_freq.shape) != (hd // 2,) or inv_freq.dtype != torch.float32 or \
+            not inv_freq.is_contiguous():
+        return False
+    shapes = ((H,), (nqkv, H), (H, nq), (H,), (2 * inter, H), (H, inter))
+    kp, vp, step = k.data_ptr(), v.data_ptr(), nkv * S * hd * 2
+    table = (P * (8 * len(blocks)))()
+    for i, (b, s) in enumerate(zip(blocks, slots)):
+        if not 0 <= s < k.shape[0]:
+            return False
+        ptrs = []
+        for t, shape in zip((b.ln1, b.wqkv, b.wo, b.ln2, b.wgu, b.wd), shapes):
+            p = t.data_ptr()
+            if t.shape != shape or t.dtype != dt or not t.is_contiguous() or not t.is_cuda or \
+                    p % 16:
+                return False
+            ptrs.append(p)
+        table[8 * i:8 * i + 8] = [*ptrs, kp + s * step, vp + s * step]
+    capturing = torch.cuda.is_current_stream_capturing()
+    forms, floats = _forms(T, ((nqkv, H, "store"), (H, nq, "resid32"), (2 * inter, H, "swiglu"),
+                               (H, inter, "resid32")), capturing)
+    if forms is None:
+        return False
+    dev, st = hidden.device, torch.cuda.current_stream().cuda_stream
+    x = torch.empty((T, H), device=dev, dtype=dt)
+    qkv = torch.empty((T, nqkv), device=dev, dtype=dt)
+    att = torch.empty((T, nq), device=dev, dtype=dt)
+    act = torch.empty((T, inter), device=dev, dtype=dt)
+    ws = G._workspace(dev, floats) if floats else None
+    rows_ws = tick = None
+    if any(f.kind == 2 for f in forms):
+        rows_ws, tick = G._rows_state(dev, T, st)
+    ptr = [None if t is None else t.data_ptr() for t in (
+        hidden, x, qkv, att, act, inv_freq, G._zeros16(dev), ws, rows_ws, tick)]
+    run = _Run(C.addressof(table), *ptr, *forms, len(blocks), G._DT[dt], T, H, inter, nh, nkv, hd, S,
+               int(pos0), float(cfg.rms_norm_eps), float(scale))
+    check(kernels().cake_block_rows(C.addressof(run), st), "block_rows")
+    return True
