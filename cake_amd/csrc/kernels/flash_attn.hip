@@ -20,7 +20,7 @@
 // shares that row layout, so the rescale is a per-register multiply.  P goes
 // through a small per-wave LDS tile to become the A operand of P·V.
 // DP = head dim padded to a multiple of 32 (zero-filled, never stored).
-#include "common.h"
+#include "flash3.h"
 
 #include <cstdlib>
 
@@ -592,6 +592,57 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a) {
   *reinterpret_cast<uint2*>(a.o + b * a.o_sb + hq * a.o_sh + (long long)q * a.o_sn + d) = st;
 }
 
+// The causal prefill of 128-wide heads (flash3.h): q tile rows of 128 QS, whatever strides.
+template <int DT, int QS>
+__global__ __launch_bounds__(256, 1) void flash3_fwd_kernel(FlashArgs a) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[fl_lds<128>()];
+  const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // workgroups go to the XCDs in turn: the query heads of one key head to one XCD's L2 (8 key
+  // heads), the longest rows first
+  const int x = blockIdx.x % a.H, b = blockIdx.x / a.H;
+  const int hk = x % a.Hkv, hq = hk * (a.H / a.Hkv) + x / a.Hkv;
+  const int mblk = (gridDim.y - 1 - blockIdx.y) * (128 * QS), qw = mblk + wave * (32 * QS);
+  const uint16_t* qb = a.q + b * a.q_sb + hq * a.q_sh;
+  fu32x4 qf[QS][8];  // B operand: lane holds Q[row][16 ks + 8 h ..]
+#pragma unroll
+  for (int qs = 0; qs < QS; ++qs) {
+    const int row = min(qw + 32 * qs + l32, a.N - 1);
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+      qf[qs][ks] = *reinterpret_cast<const fu32x4*>(qb + (long long)row * a.q_sn + 16 * ks + 8 * h);
+  }
+  FlCore c{};
+  c.k = a.k + b * a.k_sb + hk * a.k_sh;
+  c.v = a.v + b * a.v_sb + hk * a.v_sh;
+  c.k_sn = a.k_sn;
+  c.v_sn = a.v_sn;
+  c.k_end = (unsigned)(((a.M - 1) * a.k_sn + 128) * 2);
+  c.v_end = (unsigned)(((a.M - 1) * a.v_sn + 128) * 2);
+  c.kend = min(a.M, a.pos0 + mblk + 128 * QS);
+  c.pos = a.pos0 + qw;
+  c.scale_log2 = a.scale_log2;
+  f32x16 o[QS][4];
+  float l[QS];
+  fl_core<DT, QS, 128, false, true>(smem, c, qf, o, l);
+#pragma unroll
+  for (int qs = 0; qs < QS; ++qs) {
+    const int qrow = qw + 32 * qs + l32;
+    if (qrow >= a.N) continue;
+    const float inv = l[qs] > 0.f ? 1.f / l[qs] : 0.f;
+    uint16_t* orow = a.o + b * a.o_sb + hq * a.o_sh + (long long)qrow * a.o_sn;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        uint2 st;
+        st.x = fl_cvt<DT>(o[qs][t][4 * g] * inv, o[qs][t][4 * g + 1] * inv);
+        st.y = fl_cvt<DT>(o[qs][t][4 * g + 2] * inv, o[qs][t][4 * g + 3] * inv);
+        *reinterpret_cast<uint2*>(orow + 32 * t + 8 * g + 4 * h) = st;
+      }
+  }
+}
+
 }  // namespace cake
 
 using namespace cake;
@@ -609,7 +660,7 @@ static int flash_ksplit() {
 }
 static int g_flash_impl = -1;  // -1: from CAKE_FLASH_IMPL (default 2)
 static long long g_flash_pair_min = 512;  // unpaired workgroups needed before pairing
-static int g_flash_nw = 0;                 // v2 waves per workgroup override (0 = auto)
+static int g_flash_nw = 0;                 // flash2 with these waves per workgroup (0 = auto)
 
 static int flash_impl() {
   if (g_flash_impl < 0) {
@@ -628,6 +679,20 @@ static int launch_flash(const FlashArgs& a, hipStream_t st) {
                   a.q_sh % 8 == 0 && a.k_sb % 8 == 0 && a.k_sh % 8 == 0 && a.v_sb % 8 == 0 &&
                   a.v_sh % 8 == 0 && a.o_sb % 4 == 0 && a.o_sh % 4 == 0 && al(a.q, 16) &&
                   al(a.k, 16) && al(a.v, 16) && al(a.o, 8);
+  // causal 128-wide heads: flash3.h (rows past M must lie past the last row's end, and 32-bit
+  // offsets reach it).  64 query rows a wave once 256-row workgroups fill the chip one and a half
+  // times (32 heads: 2500 rows, 320 of them, 88 us against 81 with 32 rows; 3000, 384, 98 / 102;
+  // 6000 327 / 342)
+  const auto end = [&](long long sn) { return sn >= 128 ? ((long long)a.M * sn + 128) * 2 : 1LL << 40; };
+  if (v2 && a.causal && a.D == 128 && flash_ksplit() <= 1 && g_flash_nw == 0 &&
+      end(a.k_sn) < 0x7fffffffLL && end(a.v_sn) < 0x7fffffffLL) {
+    const long long wgs = (long long)((a.N + 255) / 256) * a.H * a.B;
+    const int qs = wgs >= 384 ? 2 : 1;
+    const dim3 g3(a.H * a.B, (a.N + 128 * qs - 1) / (128 * qs));
+    if (qs == 2) hipLaunchKernelGGL((flash3_fwd_kernel<DT, 2>), g3, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((flash3_fwd_kernel<DT, 1>), g3, dim3(256), 0, st, a);
+    return (int)hipGetLastError();
+  }
   if (v2) {
     // rows per workgroup: 128 (4 waves); smaller only for tiny grids (measured:
     // 4-wave workgroups win even at 128 workgroups on 256 CUs)
@@ -696,7 +761,7 @@ static int launch_flash(const FlashArgs& a, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// 1 = the 16-row 16x16x32 kernel, 2 = the 32x32x16 swapped-QKᵀ kernel (when shapes allow)
+// 1 = the 16-row 16x16x32 kernel, 2 = the 32x32x16 swapped-QKᵀ kernels (when shapes allow)
 CAKE_API void cake_flash_set_impl(int v) { g_flash_impl = v; }
 CAKE_API void cake_flash_set_nw(int nw) { g_flash_nw = nw; }
 // causal q-tile pairing threshold (unpaired workgroups); <= 0 never pairs

@@ -5,6 +5,7 @@
 // (mixer_latent.hip), from the step's expansion of the latent, with the rotated key part read
 // from the latent cache.
 #pragma once
+#include "flash3.h"
 #include "mixer_common.h"
 
 namespace cake {
@@ -68,7 +69,7 @@ struct MixFlashArgs {
 
 // KC / VC: classes of the key and value sizes (EXACT: the sizes themselves)
 template <int DT, int KC> struct FlashGeo {
-  // keys per tile: 32 where 64 would spill the prefetched pieces (192: 198 -> 151 us)
+  // keys per tile: 32 where 64 would spill the prefetched pieces
   static constexpr int BN = DT == kF32 || KC == 192 ? 32 : 64;
   static constexpr int NBUF = KC <= 128 ? 2 : 1;     // LDS buffers
   static constexpr int WGS = KC <= 192 && (KC <= 128 || DT != kF32) ? 2 : 1;  // per CU
@@ -321,6 +322,118 @@ __global__ __launch_bounds__(256, (FlashGeo<DT, KC>::WGS)) void mixer_flash_kern
         }
       }
   }
+}
+
+// 16-bit types, keys of 128 columns (LAT: 128 and 64 rotated) and values of 128, on the shared
+// core (flash3.h), 128 rows a workgroup, the maximum exact as in the kernel above (the same rounding
+// of every probability).  32 heads over 8, us before / after: 300 rows 26.5 / 14.2, 1100 64 / 34,
+// 2048 110 / 65, 24 sequences of 60 47 / 32; latent 300 27 / 15, 1100 85 / 38, 2048 154 / 74.  (64
+// rows a wave: 1.05 - 1.15x faster from 3000 rows on with a deferred maximum, slower below.)
+template <int DT, bool LAT>
+__global__ __launch_bounds__(256, 1) void mixer_flash3_kernel(MixFlashArgs a) {
+  constexpr int QS = 1, KC = LAT ? 192 : 128, KS = KC / 16;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[fl_lds<KC>()];
+  const SeqRow sq = a.seq[blockIdx.z];
+  const int nqt = (sq.len + 128 * QS - 1) / (128 * QS);
+  if ((int)blockIdx.y >= nqt) return;
+  const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // the query heads of one key head to one XCD (8 key heads), the longest rows first
+  const int x = blockIdx.x, hk = LAT ? x : x % a.G, h = LAT ? x : hk * (a.H / a.G) + x / a.G;
+  const int m0 = (nqt - 1 - (int)blockIdx.y) * (128 * QS), qw = m0 + wave * (32 * QS);
+
+  fu32x4 qf[QS][KS];
+#pragma unroll
+  for (int qs = 0; qs < QS; ++qs) {
+    const int row = min(qw + 32 * qs + l32, sq.len - 1);
+    const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.qn) +
+        (LAT ? (sq.row0 + row) * a.lat.ldq + (long long)h * KC
+             : ((long long)(sq.row0 + row) * a.H + h) * KC);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      uint4 w = *reinterpret_cast<const uint4*>(qp + (2 * ks + hh) * 8);
+      if (ks >= 8)
+        rotate_piece<DT>(w, a.lat.cs + (long long)(sq.pos0 + row) * a.lat.rd2,
+                         (2 * (ks - 8) + hh) * 4, a.lat.rd2);
+      qf[qs][ks] = __builtin_bit_cast(fu32x4, w);
+    }
+  }
+  FlCore c{};
+  c.kend = sq.pos0 + min(sq.len, m0 + 128 * QS);
+  c.pos = sq.pos0 + qw;
+  c.scale_log2 = a.scale_log2;
+  c.sink = a.sink != 0;
+  const uint16_t *kc = reinterpret_cast<const uint16_t*>(a.kc),
+                 *vc = reinterpret_cast<const uint16_t*>(a.vc);
+  if constexpr (LAT) {
+    const int k0 = a.lat.koff[blockIdx.z];
+    c.k = kc + k0 * a.lat.ldk + (long long)h * 128;
+    c.k_sn = a.lat.ldk;
+    c.v = vc + (long long)h * 128 * a.lat.ldv + k0;
+    c.v_sn = a.lat.ldv;
+    c.v_end = (unsigned)((127 * a.lat.ldv + (c.kend + 63) / 64 * 64) * 2);
+    c.r = reinterpret_cast<const uint16_t*>(a.lat.rope) + sq.slot * a.lat.rope_slot;
+    c.r_sn = a.lat.ldr;
+    c.r_end = (unsigned)(((c.kend - 1) * c.r_sn + 64) * 2);
+  } else {
+    c.k = kc + sq.slot * a.k_slot + (long long)hk * a.S * 128;
+    c.k_sn = 128;
+    c.v = vc + sq.slot * a.v_slot + (long long)hk * 128 * a.S;
+    c.v_sn = a.S;
+    c.v_end = (unsigned)(256 * a.S);
+  }
+  c.k_end = (unsigned)(((c.kend - 1) * c.k_sn + 128) * 2);
+  ff32x16 o[QS][4];
+  float l[QS];
+  fl_core<DT, QS, KC, true, false>(smem, c, qf, o, l);
+
+#pragma unroll
+  for (int qs = 0; qs < QS; ++qs) {
+    const int row = qw + 32 * qs + l32;
+    if (row >= sq.len) continue;
+    const float inv = 1.f / l[qs];
+    const long long n = sq.row0 + row;
+    uint16_t* op = reinterpret_cast<uint16_t*>(a.out) + n * a.ldo + (long long)h * 128 + 4 * hh;
+    const uint16_t* gp = LAT || !a.gate ? nullptr
+        : reinterpret_cast<const uint16_t*>(a.gate) + n * a.ldg + (long long)h * 128 + 4 * hh;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = o[qs][t][4 * g + e] * inv;
+        if (!LAT && gp) {
+          const uint2 w = *reinterpret_cast<const uint2*>(gp + 32 * t + 8 * g);
+          y[0] *= sigmoid32(to_f32<DT>((uint16_t)(w.x & 0xffffu)));
+          y[1] *= sigmoid32(to_f32<DT>((uint16_t)(w.x >> 16)));
+          y[2] *= sigmoid32(to_f32<DT>((uint16_t)(w.y & 0xffffu)));
+          y[3] *= sigmoid32(to_f32<DT>((uint16_t)(w.y >> 16)));
+        }
+        *reinterpret_cast<uint2*>(op + 32 * t + 8 * g) =
+            make_uint2(fl_cvt<DT>(y[0], y[1]), fl_cvt<DT>(y[2], y[3]));
+      }
+  }
+}
+
+// Whether mixer_flash3_kernel takes a call: its head sizes, a scale that keeps the order of the
+// scores, 8-byte output and gate rows, a sequence's keys and values under 2 GB (rows: its most).
+inline bool flash3_ok(int dt, const MixFlashArgs& a, bool lat, long long rows) {
+  const auto al = [](const void* p, long long ld) { return (uintptr_t)p % 8 == 0 && ld % 4 == 0; };
+  const long long lim = 0x7fffffffLL / 2;
+  if ((dt != kBF16 && dt != kF16) || a.DVP != 128 || a.vdim != 128 || !(a.scale_log2 > 0.f) ||
+      !al(a.out, a.ldo) || (a.gate && !al(a.gate, a.ldg)))
+    return false;
+  if (!lat) return a.DP == 128 && 128LL * a.S < lim;
+  return a.DP == 192 && a.lat.dimp == 128 && a.lat.rotp == 64 && rows * a.lat.ldk < lim &&
+         rows * a.lat.ldr < lim && 127 * a.lat.ldv + rows + 64 < lim;
+}
+
+template <int DT, bool LAT>
+int launch_mix_flash3(const MixFlashArgs& a, int max_len, int B, hipStream_t st) {
+  const dim3 grid(a.H, (max_len + 127) / 128, B);
+  hipLaunchKernelGGL((mixer_flash3_kernel<DT, LAT>), grid, dim3(256), 0, st, a);
+  return (int)hipGetLastError();
 }
 
 template <int DT, int KC, int VC, bool EXACT, bool LAT>

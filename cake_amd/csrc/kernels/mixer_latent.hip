@@ -606,6 +606,12 @@ CAKE_API int cake_latent_flash(int dt, const void* q, long long ldq, const void*
   a.lat.ldq = ldq; a.lat.ldk = ldk; a.lat.ldv = ldv;
   a.lat.cs = (const float2*)cs;
   a.lat.rd2 = rd2;
+  if (dt != kF32) {
+    a.lat.rope = reinterpret_cast<const uint16_t*>(cache) + RP;
+    if (flash3_ok(dt, a, true, slot_stride / LD))
+      return dt == kBF16 ? launch_mix_flash3<kBF16, true>(a, max_len, B, st)
+                         : launch_mix_flash3<kF16, true>(a, max_len, B, st);
+  }
   const dim3 grid((max_len + 127) / 128, H, B);
   CAKE_MIX_DT(dt, {
     a.lat.rope = reinterpret_cast<const typename St<DT>::E*>(cache) + RP;

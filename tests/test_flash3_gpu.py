@@ -1,0 +1,136 @@
+"""Causal attention of 128-wide heads on the one-wave-per-SIMD core: row and key counts around its
+tiles, cached prefixes, ragged batches, sink and gate, the latent form; against float64 and beside
+the general kernel that takes what the core refuses."""
+import pytest
+import torch
+
+from cake_amd.ops import hip as K
+from cake_amd.ops import latent as L
+from cake_amd.ops import mixers as M
+
+pytestmark = pytest.mark.gpu
+
+# the probabilities and the result are rounded once each, half a unit in the last place (the sums
+# are float32)
+TOL = {torch.bfloat16: 2 * 2 ** -8, torch.float16: 2 * 2 ** -11}
+DTYPES = [torch.bfloat16, torch.float16]
+
+
+def _want(q, k, v, pos0, scale, sink=False, gate=None):
+    s = q.double() @ k.double().t().contiguous() * scale
+    n, T = s.shape
+    s.masked_fill_(torch.arange(T)[None] > torch.arange(n)[:, None] + pos0, float("-inf"))
+    v = v.double()
+    if sink:
+        s = torch.cat([s, s.new_zeros(n, 1)], 1)
+        v = torch.cat([v, v.new_zeros(1, v.shape[1])])
+    o = s.softmax(1) @ v
+    return o if gate is None else o * gate.double().sigmoid()
+
+
+def _close(got, want, dt):
+    assert bool(torch.isfinite(got).all())
+    assert float((got.double() - want).norm() / want.norm()) < TOL[dt]
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=str)
+@pytest.mark.parametrize("H,Hkv,N,pos0", [
+    (4, 2, 1, 0), (4, 1, 31, 33), (2, 2, 33, 0), (4, 2, 64, 64), (8, 8, 65, 3), (2, 1, 127, 1),
+    (2, 1, 129, 191), (3, 1, 256, 0), (2, 2, 641, 0), (192, 8, 257, 0), (192, 64, 300, 21)])
+def test_prefill(dt, H, Hkv, N, pos0):
+    """The last two have the workgroups for 64 rows a wave; keys past the live ones are NaN."""
+    g = torch.Generator().manual_seed(N)
+    S, Tk = pos0 + N + 37, pos0 + N
+    qkv = torch.randn(N, (H + 3) * 128, generator=g).to(dt)       # q is a column block of it
+    kc, vc = (torch.randn(Hkv, S, 128, generator=g).to(dt) for _ in range(2))
+    kc[:, Tk:], vc[:, Tk:] = float("nan"), float("nan")
+    qd, kd, vd = qkv.cuda(), kc.cuda(), vc.cuda()
+    out = torch.full((N + 1, H * 128), 7.0, device="cuda", dtype=dt)
+    K.flash_attn(qd[:, :H * 128].view(1, N, H, 128).transpose(1, 2), kd[None, :, :Tk],
+                 vd[None, :, :Tk], out[:N].view(1, N, H, 128).transpose(1, 2), 0.1, causal=True,
+                 pos0=pos0)
+    assert bool((out[N:] == 7.0).all())
+    for h in sorted({0, H // 2, H - 1}):
+        hk = h // (H // Hkv)
+        _close(out[:N, h * 128:h * 128 + 128].cpu(),
+               _want(qkv[:, h * 128:h * 128 + 128], kc[hk, :Tk], vc[hk, :Tk], pos0, 0.1), dt)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=str)
+def test_prefill_batch_and_standing_out_key(dt):
+    """Batched views; and a key far above the many others, whose share is of tiny probabilities."""
+    q, k, v = (torch.randn(3, n, 70, 128).to(dt) for n in (4, 2, 2))
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    out = torch.empty_like(qd)
+    K.flash_attn(qd, kd, vd, out, 0.2, causal=True)
+    for b in range(3):
+        _close(out[b, 3].cpu(), _want(q[b, 3], k[b, 1], v[b, 1], 0, 0.2), dt)
+    n, d = 3000, 9.0
+    q, k, v = torch.zeros(n, 128), torch.zeros(n, 128), torch.ones(n, 128)
+    q[:, 0], k[n // 2, 0], v[n // 2] = 1, d, 0
+    out = torch.empty(1, 1, n, 128, device="cuda", dtype=dt)
+    K.flash_attn(q.to(dt).cuda()[None, None], k.to(dt).cuda()[None, None],
+                 v.to(dt).cuda()[None, None], out, 1.0, causal=True)
+    _close(out[0, 0].cpu(), _want(q, k, v, 0, 1.0), dt)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=str)
+@pytest.mark.parametrize("sink,gated", [(True, True), (False, False)])
+@pytest.mark.parametrize("H,G,seqs", [
+    (8, 2, [(1, 0, 5), (0, 70, 300), (3, 0, 129)]), (4, 4, [(0, 0, 128), (2, 63, 1)]),
+    (2, 1, [(0, 1, 641)])])
+def test_ragged(dt, H, G, seqs, sink, gated):
+    sh, S = M.AttnShape(H, G, 128, 128), 704
+    rows = M.Rows.pack([(s, p, [0] * n) for s, p, n in seqs], "cuda")
+    g = torch.Generator().manual_seed(H)
+    kc, vc = (torch.randn(4, G, *d, generator=g).to(dt) for d in ((S, 128), (128, S)))
+    qn = torch.randn(rows.N, H, 128, generator=g).to(dt)
+    gate = torch.randn(rows.N, H * 128 + 8, generator=g).to(dt) if gated else None
+    dev = [None if t is None else t.cuda() for t in (qn, kc, vc, gate)]
+    outs = []
+    for ld in (H * 128 + 4, H * 128 + 1):    # the core; rows off 8 bytes: the general kernel
+        out = torch.full((rows.N, ld), 7.0, device="cuda", dtype=dt)
+        M.attn_prompt(sh, dev[0], dev[1], dev[2], rows, dev[3][:, :H * 128] if gated else None,
+                      out[:, :H * 128], 0.1, sink)
+        assert bool((out[:, H * 128:] == 7.0).all())
+        outs.append(out[:, :H * 128].cpu())
+    for r0, n, p0, s in rows.host:
+        for h in (0, H - 1):
+            c, hk = slice(h * 128, h * 128 + 128), h // (H // G)
+            w = _want(qn[r0:r0 + n, h], kc[s, hk, :p0 + n], vc[s, hk, :, :p0 + n].t(), p0, 0.1,
+                      sink, gate[r0:r0 + n, c] if gated else None)
+            for out in outs:
+                _close(out[r0:r0 + n, c], w, dt)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=str)
+@pytest.mark.parametrize("H,seqs", [(4, [(1, 0, 5), (0, 70, 300), (2, 0, 129)]), (2, [(0, 1, 513)])])
+def test_latent(dt, H, seqs):
+    S = 576
+    sh = L.LatentShape(H, 128, 64, 128, 96, 64, 30)
+    rows = M.Rows.pack([(s, p, [0] * n) for s, p, n in seqs], "cuda")
+    g = torch.Generator().manual_seed(H)
+    cache = torch.randn(3, S, sh.LD, generator=g).to(dt)
+    k = torch.randn(rows.n_keys, H * 128, generator=g).to(dt)
+    vt = torch.randn(H * 128, rows.n_keys, generator=g).to(dt)
+    q = torch.randn(rows.N, H * 192, generator=g).to(dt)
+    ang = torch.rand(S, 30, generator=g) * 6
+    cs = torch.stack([ang.cos(), ang.sin()], 2).reshape(S, 60).contiguous()
+    qd, kd, vd, cd, sd = (t.cuda() for t in (q, k, vt, cache, cs))
+    outs = []
+    for ld in (H * 128, H * 128 + 1):
+        out = torch.full((rows.N, ld), 7.0, device="cuda", dtype=dt)
+        L.prompt(sh, qd, kd, vd, rows, sd, cd, out[:, :H * 128], 0.08)
+        outs.append(out[:, :H * 128].cpu())
+    for i, (r0, n, p0, s) in enumerate(rows.host):
+        k0 = int(rows.key0[i])
+        for h in (0, H - 1):
+            qq = q[r0:r0 + n, h * 192:h * 192 + 192].float()
+            c, sn = ang[p0:p0 + n].cos(), ang[p0:p0 + n].sin()
+            x, y = qq[:, 128:188:2].clone(), qq[:, 129:188:2].clone()
+            qq[:, 128:188:2], qq[:, 129:188:2] = x * c - y * sn, y * c + x * sn
+            kk = torch.cat([k[k0:k0 + p0 + n, h * 128:h * 128 + 128],
+                            cache[s, :p0 + n, sh.RP:sh.RP + 64]], 1)
+            w = _want(qq.to(dt), kk, vt[h * 128:h * 128 + 128, k0:k0 + p0 + n].t(), p0, 0.08)
+            for out in outs:
+                _close(out[r0:r0 + n, h * 128:h * 128 + 128], w, dt)
