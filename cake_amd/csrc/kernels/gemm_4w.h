@@ -58,12 +58,12 @@ constexpr int alt_idx(int nr, int nd, int k) {
 
 // LDS-DMA of one 1 KiB piece (buffer_load_dwordx4 ... offen lds) with the M0 write in the
 // same statement (M0 is not preserved around inline asm); d = the buffer descriptor as an
-// SGPR quad.  amfma_dma issues an MFMA between the M0 write and the DMA, which covers the
+// SGPR quad; the add sets SCC, where the compiler may keep a comparison.  amfma_dma issues an MFMA between the M0 write and the DMA, which covers the
 // write's wait state (no s_nop) and keeps the DMA beside the MFMA it was scheduled with.
 template <int OFF>
 __device__ __forceinline__ void dma16(uint32_t mb, uint32_t voff, cu32x4 d, uint32_t soff) {
   asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(mb), "v"(voff), "s"(d), "s"(soff), "i"(OFF) : "memory");
+               :: "s"(mb), "v"(voff), "s"(d), "s"(soff), "i"(OFF) : "memory", "scc");
 }
 template <int DT, int OFF>
 __device__ __forceinline__ void amfma_dma(cf32x4& acc, const uint4& a, const uint4& b, uint32_t mb,
@@ -74,13 +74,13 @@ __device__ __forceinline__ void amfma_dma(cf32x4& acc, const uint4& a, const uin
                  "buffer_load_dwordx4 %4, %5, %6 offen lds"
                  : "+a"(acc)
                  : "v"(av), "v"(bv), "s"(mb), "v"(voff), "s"(d), "s"(soff), "i"(OFF)
-                 : "memory");
+                 : "memory", "scc");
   else
     asm volatile("s_add_u32 m0, %3, %7\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\t"
                  "buffer_load_dwordx4 %4, %5, %6 offen lds"
                  : "+a"(acc)
                  : "v"(av), "v"(bv), "s"(mb), "v"(voff), "s"(d), "s"(soff), "i"(OFF)
-                 : "memory");
+                 : "memory", "scc");
 }
 
 // SCHED 1 (cfg 25-27): the same tiles on a three-barrier schedule (the DMAs of step t+2
