@@ -147,7 +147,6 @@ struct MixDecArgs {
   unsigned int* ticket;  // [B][ngt], zero between launches
 };
 
-constexpr int kDecWaves = 4;
 
 // rotation + norm of one head by one wave: lane handles dims 4 lane .. +3 (dim <= 256)
 __device__ __forceinline__ void head_rot_norm(const float* src, int dim, int lane,
@@ -174,8 +173,8 @@ __device__ __forceinline__ void head_rot_norm(const float* src, int dim, int lan
   }
 }
 
-template <int DT, int CLS, bool EXACT>
-__global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDecArgs a) {
+template <int DT, int CLS, bool EXACT, int NW>
+__global__ __launch_bounds__(64 * NW) void mixer_attn_decode_kernel(MixDecArgs a) {
   using E = typename St<DT>::E;
   constexpr int EPC = St<DT>::EPC;
   constexpr int NKS = CLS / St<DT>::KSTEP, NVT = CLS / 16;
@@ -185,8 +184,8 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   __shared__ __attribute__((aligned(16))) E qs[16 * (CLS + EPC)];
   __shared__ __attribute__((aligned(16))) E kcur[CLS];
   __shared__ __attribute__((aligned(16))) E vcur[CLS];
-  __shared__ float red_m[kDecWaves][16], red_l[kDecWaves][16];
-  __shared__ float red_o[kDecWaves][16][CLS + 1];
+  __shared__ float red_m[NW][16], red_l[NW][16];
+  __shared__ float red_o[NW][16][CLS + 1];
   __shared__ int s_last;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
@@ -207,13 +206,16 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   E* kb = reinterpret_cast<E*>(a.kc) + slot * a.k_slot + (long long)hk * a.S * a.DP;
   E* vb = reinterpret_cast<E*>(a.vc) + slot * a.v_slot + (long long)hk * a.DVP * a.S;
 
-  // the wave's first block of keys is requested ahead of the prologue
+  // the wave's first block of keys is requested ahead of the prologue.  Row i of score block u is
+  // key 8 (i / 4) + 4 u + i % 4: the two blocks' accumulators of a lane group are then eight keys in
+  // a row, and a value piece is one 16-byte load (as two of 8 bytes 16 positions apart the loads of
+  // 256 keys took 2 us longer)
   uint4 kf[2][NKS];
   VFrag<DT> vf[NVT];
   auto load_k = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const E* kp = kb + (long long)(k0 + 16 * u + l15) * DP + g * EPC;
+      const E* kp = kb + (long long)(k0 + 8 * (l15 >> 2) + 4 * u + (l15 & 3)) * DP + g * EPC;
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks)
         if (EXACT || ks < nks) kf[u][ks] = *reinterpret_cast<const uint4*>(kp + ks * 4 * EPC);
@@ -222,7 +224,17 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   auto load_vs = [&](int k0) {
 #pragma unroll
     for (int t = 0; t < NVT; ++t)
-      if (EXACT || t < nvt) vf[t] = load_v<DT>(vb + (long long)(16 * t + l15) * a.S + k0, g);
+      if (EXACT || t < nvt) {
+        const E* vp = vb + (long long)(16 * t + l15) * a.S + k0 + 8 * g;
+        if constexpr (DT == kF32) {
+          vf[t].lo = *reinterpret_cast<const float4*>(vp);
+          vf[t].hi = *reinterpret_cast<const float4*>(vp + 4);
+        } else {
+          const uint4 w = *reinterpret_cast<const uint4*>(vp);
+          vf[t].lo = make_uint2(w.x, w.y);
+          vf[t].hi = make_uint2(w.z, w.w);
+        }
+      }
   };
   int k0 = kbeg + 32 * wave;
   if (kPrefetch && k0 < klim) { load_k(k0); load_vs(k0); }
@@ -233,11 +245,11 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   if (a.gated)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      if (tid + 64 * kDecWaves * i < nr * a.vdim) gpre[i] = gate[tid + 64 * kDecWaves * i];
+      if (tid + 64 * NW * i < nr * a.vdim) gpre[i] = gate[tid + 64 * NW * i];
 
   // rows past nr and value columns past vdim stay unwritten: they only reach accumulator
   // columns / rows that no output reads
-  for (int r = wave; r < nr + (owner ? 1 : 0); r += kDecWaves) {
+  for (int r = wave; r < nr + (owner ? 1 : 0); r += NW) {
     const bool isk = r == nr;
     const float* src = isk ? pj + (long long)(a.H + hk) * a.dim
                            : pj + (long long)(hk * R + r0 + r) * a.dim;
@@ -250,7 +262,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   }
   if (owner) {
     const float* vsrc = pj + (long long)(a.H + a.G) * a.dim + (long long)hk * a.vdim;
-    for (int d = tid; d < a.vdim; d += 64 * kDecWaves) {
+    for (int d = tid; d < a.vdim; d += 64 * NW) {
       const E v = St<DT>::st(vsrc[d]);
       vcur[d] = v;
       if (r0 == 0) vb[(long long)d * a.S + pos] = v;
@@ -258,7 +270,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   }
   __syncthreads();
   if (owner && r0 == 0)
-    for (int d = tid; d < DP; d += 64 * kDecWaves) kb[(long long)pos * DP + d] = kcur[d];
+    for (int d = tid; d < DP; d += 64 * NW) kb[(long long)pos * DP + d] = kcur[d];
 
   uint4 qf[NKS];
 #pragma unroll
@@ -286,7 +298,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[t][e] = St<DT>::ld(vcur[16 * t + 4 * g + e]);
   }
-  for (; k0 < klim; k0 += 32 * kDecWaves) {
+  for (; k0 < klim; k0 += 32 * NW) {
     if constexpr (!kPrefetch) { load_k(k0); load_vs(k0); }
     cf32x4 s[2];
 #pragma unroll
@@ -296,14 +308,14 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
       for (int ks = 0; ks < NKS; ++ks)
         if (EXACT || ks < nks) s[u] = mm_piece<DT>(kf[u][ks], qf[ks], s[u]);
     }
-    const int kn = k0 + 32 * kDecWaves;
+    const int kn = k0 + 32 * NW;
     if constexpr (kPrefetch) { if (kn < klim) load_k(kn); }
     float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const bool ok = k0 + 16 * u + 4 * g + e < klim;
+        const bool ok = k0 + 8 * g + 4 * u + e < klim;
         s[u][e] = ok ? s[u][e] * a.scale_log2 : -INFINITY;
         mx = fmaxf(mx, s[u][e]);
       }
@@ -346,18 +358,18 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   auto finish = [&](int i, float num, float den) {  // i = r vdim + d: heads are contiguous
     float y = num / den;
     if (a.gated)
-      y *= sigmoid32(i < 64 * kDecWaves ? gpre[0] : i < 128 * kDecWaves ? gpre[1] : gate[i]);
+      y *= sigmoid32(i < 64 * NW ? gpre[0] : i < 128 * NW ? gpre[1] : gate[i]);
     out[i] = St<DT>::st(y);
   };
-  for (int i = tid; i < nr * a.vdim; i += 64 * kDecWaves) {
+  for (int i = tid; i < nr * a.vdim; i += 64 * NW) {
     const int r = i / a.vdim, d = i - r * a.vdim;
     float M = red_m[0][r];
 #pragma unroll
-    for (int w = 1; w < kDecWaves; ++w) M = fmaxf(M, red_m[w][r]);
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, red_m[w][r]);
     if (nact == 1 && a.sink) M = fmaxf(M, 0.f);
     float num = 0.f, den = nact == 1 && a.sink ? __builtin_amdgcn_exp2f(-M) : 0.f;
 #pragma unroll
-    for (int w = 0; w < kDecWaves; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = __builtin_amdgcn_exp2f(red_m[w][r] - M);
       num = fmaf(f, red_o[w][r][d], num);
       den = fmaf(f, red_l[w][r], den);
@@ -392,7 +404,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
   float* wl = wm + 16 * 64;         // [nact][16] sums
   float* wd = &red_m[0][0];         // [16] denominators
   static_assert(sizeof(red_o) >= 2 * 16 * 64 * sizeof(float), "merge scratch");
-  for (int i = tid; i < nr * nact; i += 64 * kDecWaves) {
+  for (int i = tid; i < nr * nact; i += 64 * NW) {
     const int s = i / nr, r = i - s * nr;
     const float* pr = part + s * pstride + (long long)r * (DVP + 2);
     wm[s * 16 + r] = __hip_atomic_load(pr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -411,7 +423,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void mixer_attn_decode_kernel(MixDe
     wd[tid] = den;
   }
   __syncthreads();
-  for (int i = tid; i < nr * a.vdim; i += 64 * kDecWaves) {
+  for (int i = tid; i < nr * a.vdim; i += 64 * NW) {
     const int r = i / a.vdim, d = i - r * a.vdim;
     const float* pr = part + (long long)r * (DVP + 2) + 2 + d;
     float num = 0.f;
@@ -493,10 +505,22 @@ CAKE_API int cake_mixer_flash(int dt, const void* qn, const void* kc, const void
   return (int)hipErrorInvalidValue;
 }
 
+// Few keys: one workgroup's chain of loads (position, projections, keys, merge), so eight waves take
+// 256 keys in one pass of 32 each (16 heads over 4, 256 keys, 10.6 us with four waves, 8.4).  Key
+// splits only as far as the batch leaves compute units idle: 24 sequences of 8 key heads in 8 splits
+// took 27 us at 300 keys and 44.5 at 1000, unsplit 10.3 and 20.3 (2000 keys 56 / 38, 4000 102 / 85);
+// one sequence 1000 keys 10.4 in 8 splits, 18.2 unsplit.
 template <int DT, int CLS, bool EXACT>
-static int launch_mix_dec(const MixDecArgs& a, dim3 grid, hipStream_t st) {
-  hipLaunchKernelGGL((mixer_attn_decode_kernel<DT, CLS, EXACT>), grid, dim3(64 * kDecWaves), 0, st,
-                     a);
+static int launch_mix_dec(MixDecArgs a, dim3 grid, hipStream_t st) {
+  while (a.nsplit > 1 && (long long)grid.x * grid.z * a.nsplit > 256) a.nsplit /= 2;
+  grid.y = a.nsplit;
+  if constexpr (DT != kF32 && CLS <= 128) {
+    if (a.nsplit == 1) {
+      hipLaunchKernelGGL((mixer_attn_decode_kernel<DT, CLS, EXACT, 8>), grid, dim3(512), 0, st, a);
+      return (int)hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((mixer_attn_decode_kernel<DT, CLS, EXACT, 4>), grid, dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
 
