@@ -336,13 +336,19 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
 // matrices of 8 .. 260 MB; both sides of the lines they draw, measured: 4096 x 4096 at 16 rows
 // direct 11.5, stream 14.4; 4096 x 14336 direct 35, stream 25; 28672 x 4096 at 45 rows stream 53,
 // tiles 58; 4096 x 4096 at 45 rows stream 19, tiles 17.
+// (the stream form's shape, gemm_rows.h StreamShape)
+struct StreamPlan { int bn, kst, wgs; };
+static StreamPlan stream_plan(int mt, bool gated) {
+  return mt > 1 || gated ? StreamPlan{128, 64, 256} : StreamPlan{64, 128, 512};
+}
 static int rows_kind(int M, long long Nv, int K, bool gated) {
-  if (M > 64 || Nv > 128LL * kRowsTicks) return 0;
+  if (M > 64 || Nv > 64LL * kRowsTicks) return 0;
   const double kb = K * 2e-3;   // KB of one row of k
   const int mt = (M + 15) / 16;
   const double tiles = 8 + Nv * kb / 4600;
-  const long long strips = (Nv + 127) / 128, ks = (K + 63) / 64, total = strips * ks;
-  const long long per = std::max<long long>((total + kRowsWgs - 1) / kRowsWgs, kRowsMinSteps);
+  const StreamPlan sp = stream_plan(mt, gated);
+  const long long strips = (Nv + sp.bn - 1) / sp.bn, ks = (K + sp.kst - 1) / sp.kst, total = strips * ks;
+  const long long per = std::max<long long>((total + sp.wgs - 1) / sp.wgs, kRowsMinK / sp.kst);
   const double stream = 7 + (ks > per || ks % per ? 0.7 * mt : 0.) + per * (16 + 2 * mt) / 27.;
   double direct = 1e9;
   if (M <= 32) {
@@ -360,7 +366,7 @@ CAKE_API int cake_gemm_rows_kind(int M, long long Nv, int K, int gated) {
 }
 
 // stream form: f32 elements of ws (two parked strips per share) and counters of tick
-CAKE_API long long cake_gemm_rows_ws_floats(int M) { return (long long)kRowsWgs * 4096 * ((M + 15) / 16); }
+CAKE_API long long cake_gemm_rows_ws_floats(int M) { return 256LL * 4096 * ((M + 15) / 16); }
 CAKE_API int cake_gemm_rows_ticks() { return kRowsTicks; }
 
 // cake_gemm_scaled for M <= 64 rows in the form `kind` (1 or 2).  The stream form needs ws
@@ -391,12 +397,13 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
   const int mt = (M + 15) / 16;
   int form, wgs;
   if (kind == 2) {
-    g.tiles_n = (g.Nv + 127) / 128;
+    const StreamPlan sp = stream_plan(mt, gated);
+    g.tiles_n = (g.Nv + sp.bn - 1) / sp.bn;
     if (g.tiles_n > kRowsTicks) return (int)hipErrorInvalidValue;
-    g.kps = kRowsMinSteps;
-    const long long total = (long long)g.tiles_n * ((K + 63) / 64);
+    g.kps = kRowsMinK / sp.kst;   // steps of a share at least
+    const long long total = (long long)g.tiles_n * ((K + sp.kst - 1) / sp.kst);
     form = 2;
-    wgs = (int)std::min<long long>(kRowsWgs, (total + kRowsMinSteps - 1) / kRowsMinSteps);
+    wgs = (int)std::min<long long>(sp.wgs, (total + g.kps - 1) / g.kps);
   } else {
     const int nt = gated || g.Nv > 4096 ? 2 : 1;   // one 16-row strip per CU, or two
     form = nt - 1;
@@ -412,10 +419,11 @@ CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long ld
                                     long long ldb, long long b_group, void* c, long long ldc,
                                     const void* tiles, int max_tiles, float* ws, void* tick,
                                     const void* zeros, int N, int K, hipStream_t st) {
-  const long long strips = (long long)max_tiles * ((N + 127) / 128);
+  const StreamPlan sp = stream_plan(1, false);
+  const long long strips = (long long)max_tiles * ((N + sp.bn - 1) / sp.bn);
   if (max_tiles <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || b_group % 8 ||
       !(epi == 0 || (epi >= 7 && epi <= 10)) || !ws || !tick || !zeros || strips > kRowsTicks ||
-      strips * ((K + 63) / 64) >= 0x40000000LL)
+      strips * ((K + sp.kst - 1) / sp.kst) >= 0x40000000LL)
     return (int)hipErrorInvalidValue;
   GemmArgs g{};
   g.a = (const uint16_t*)a; g.b = (const uint16_t*)b; g.c = (uint16_t*)c;
@@ -423,10 +431,10 @@ CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long ld
   g.lda = lda; g.ldb = ldb; g.ldc = ldc;
   g.N = N; g.K = K; g.Nv = N; g.half = N;
   g.tiles_m = max_tiles;
-  g.tiles_n = (N + 127) / 128;
-  g.kps = kRowsMinSteps;
+  g.tiles_n = (N + sp.bn - 1) / sp.bn;
+  g.kps = kRowsMinK / sp.kst;
   g.groups = (const int4*)tiles;
   g.b_group = b_group;
-  return dt == kBF16 ? Rows<kBF16>::grouped(epi, dim3(kRowsWgs), st, g)
-         : dt == kF16 ? Rows<kF16>::grouped(epi, dim3(kRowsWgs), st, g) : (int)hipErrorInvalidValue;
+  return dt == kBF16 ? Rows<kBF16>::grouped(epi, dim3(sp.wgs), st, g)
+         : dt == kF16 ? Rows<kF16>::grouped(epi, dim3(sp.wgs), st, g) : (int)hipErrorInvalidValue;
 }

@@ -21,9 +21,8 @@
 
 namespace cake {
 
-constexpr int kRowsWgs = 256;        // shares of the stream form (one per CU)
-constexpr int kRowsMinSteps = 8;     // steps of a share at least
-constexpr int kRowsTicks = 32768;    // strips of a launch at most (arrival counters)
+constexpr int kRowsMinK = 512;       // k of a share at least
+constexpr int kRowsTicks = 65536;    // strips of a launch at most (arrival counters)
 
 // the operand fragments of one 64-element chunk of k: a lane's two 16-byte pieces of each row are
 // neighbours, so the two MFMA steps read whole 128-byte lines (both operands use one order of k)
@@ -184,26 +183,38 @@ __global__ __launch_bounds__(512) void gemm_direct_kernel(GemmArgs g) {
   }
 }
 
-// MT: 16-row tiles of x.  A stage holds 16 KB of weights and 2 MT KB of x.
-template <int MT> struct StreamShape {
-  static constexpr int NWV = 4;
-  static constexpr int BN = NWV * 32;               // weight rows of a strip
-  static constexpr int NS = 4;
-  static constexpr int XW = MT == 1 ? 2 : MT == 3 ? 3 : 4;   // waves that fetch x
-  static constexpr int XI = MT * 2 / XW;              // their x DMA instructions per step
+// MT: 16-row tiles of x.  A stage holds 16 KB of weights: WIDE 128 rows by 64 k, else 64 by 128.
+// What one workgroup of four waves can have outstanding moves 5.2 TB/s at any depth, two on a CU
+// 6.1; with 64-row strips the parked sums of 512 shares are as many as those of 256 shares of 128.
+// That pays while x is one tile (5 / 13 rows: 2048 x 8192 15.3 / 16.0 -> 13.6 / 13.9 us, 8192 x 8192
+// 35.7 / 36.3 -> 32.1 / 32.6, 4096 x 14336 25.1 / 25.6 -> 24.1 / 25.0); at 24 rows x is read twice as
+// often for it (4096 x 23552 38.7 -> 40.8).  Gated rows pair up within 32 of a wave.
+template <int MT, bool WIDE> struct StreamShape {
+  static constexpr int NWV = 4, RT = WIDE ? 2 : 1, KC = WIDE ? 1 : 2;   // row tiles, 64-element chunks
+  static constexpr int BN = NWV * 16 * RT, KST = 64 * KC;   // weight rows of a strip, k of a step
+  static constexpr int NS = WIDE ? 4 : 3, WGS = WIDE ? 256 : 512;
+  static constexpr int LPR = 8 * KC, RPI = 64 / LPR;   // lanes of a row's DMA, rows of an instruction
+  static constexpr int XT = 2 * MT * KC;               // x DMA instructions of a step
+  static constexpr int XW = XT % 4 == 0 ? 4 : XT % 3 == 0 ? 3 : 2;   // waves that issue them
+  static constexpr int XI = XT / XW;
   static constexpr int IPW = 4 + XI;
-  static constexpr int STAGE = (BN + MT * 16) * 128;
+  static constexpr int STAGE = (BN + MT * 16) * 128 * KC;
+  // 16-byte chunk c of row r is in slot c ^ swz(r)
+  static __device__ __forceinline__ int swz(int r) { return KC == 2 ? r & 15 : (r >> 1) & 7; }
 };
+template <int EPI, int MT> constexpr bool stream_wide() {
+  return MT > 1 || EPI == kEpiSwiglu || EPI == kEpiGeglu;
+}
 
-// N 16-row fragments (both halves of k) at base + 2048 i; waits for them
-template <int N>
+// N 16-row fragments (two 32-element chunks of k) at base + STRIDE i; waits for them
+template <int N, int STRIDE>
 __device__ __forceinline__ void stream_read(uint32_t lo, uint32_t hi, uint4 (&a)[N][2]) {
   static_assert(N == 1 || N == 2, "fragments per read");
   if constexpr (N == 2)
-    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:2048\n\t"
-                 "ds_read_b128 %3, %5 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:%6\n\t"
+                 "ds_read_b128 %3, %5 offset:%6\n\ts_waitcnt lgkmcnt(0)"
                  : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1])
-                 : "v"(lo), "v"(hi) : "memory");
+                 : "v"(lo), "v"(hi), "i"(STRIDE) : "memory");
   else
     asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
                  : "=&v"(a[0][0]), "=&v"(a[0][1]) : "v"(lo), "v"(hi) : "memory");
@@ -230,14 +241,15 @@ __device__ __forceinline__ StreamStrip stream_strip(const GemmArgs& g, int s) {
 }
 
 // epilogue of one wave's sums: acc[j][i][e] is token 16 i + (lane & 15), virtual weight row
-// v0 + 32 wave + 16 j + 4 (lane >> 4) + e
-template <int DT, int EPI, int MT>
+// v0 + 16 RT wave + 16 j + 4 (lane >> 4) + e
+template <int DT, int EPI, int MT, int RT>
 __device__ __forceinline__ void stream_store(const GemmArgs& g, const StreamStrip& s, int wave, int lane,
-                                             const cf32x4 (&acc)[2][MT]) {
+                                             const cf32x4 (&acc)[RT][MT]) {
   constexpr bool GATED = (EPI == kEpiSwiglu || EPI == kEpiGeglu);
-  const int vw = s.v0 + wave * 32;
+  static_assert(!GATED || RT == 2, "a gate row and its up row in one wave");
+  const int vw = s.v0 + wave * (16 * RT);
 #pragma unroll
-  for (int j = 0; j < (GATED ? 1 : 2); ++j) {
+  for (int j = 0; j < (GATED ? 1 : RT); ++j) {
     const int n = (GATED ? vw / 2 : vw + j * 16) + (lane >> 4) * 4;
     if (n >= g.N) continue;
     const bool full = n + 4 <= g.N;
@@ -257,7 +269,7 @@ __device__ __forceinline__ void stream_store(const GemmArgs& g, const StreamStri
       for (int e = 0; e < 4; ++e) {
         float a = acc[j][i][e] + b0[e];
         if constexpr (GATED) {
-          const float u = acc[1][i][e] + b1[e];
+          const float u = acc[RT - 1][i][e] + b1[e];
           a = EPI == kEpiSwiglu ? silu(a) * u : a * gelu_tanh(u);
         }
         if constexpr (EPI == kEpiAdd16) a += to_f32<DT>(g.r16[(size_t)m * g.ldr + min(n + e, g.N - 1)]);
@@ -299,13 +311,13 @@ __device__ __forceinline__ cf32x4 unpark(const float* p) {
 }
 
 template <int DT, int EPI, int MT, bool GRP>
-__global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
-  using S = StreamShape<MT>;
-  constexpr int NWV = S::NWV;
+__global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
+  using S = StreamShape<MT, stream_wide<EPI, MT>()>;
+  constexpr int NWV = S::NWV, RT = S::RT, KC = S::KC, KST = S::KST;
   __shared__ __attribute__((aligned(16))) uint8_t smem[S::NS * S::STAGE];
   __shared__ unsigned last;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int KS = (g.K + 63) / 64;
+  const int KS = (g.K + KST - 1) / KST;
   const int strips = (GRP ? g.groups[g.tiles_m].x : 1) * g.tiles_n;
   const int total = strips * KS;
   const int per = max((total + (int)gridDim.x - 1) / (int)gridDim.x, g.kps);
@@ -315,22 +327,22 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
   const int u0 = wg * per, u1 = min(total, u0 + per);
   if (u0 >= u1) return;
 
-  // ---- DMA: wave w fetches weight rows 32 w .. and its share of x ----
-  const int dr = lane >> 3;                 // row within an instruction's 8
+  // ---- DMA: wave w fetches weight rows 16 RT w .. and its share of x ----
+  const int dr = lane / S::LPR, dslot = lane % S::LPR;   // row within an instruction's, slot
   int ds = u0 / KS, dk = u0 % KS, dnext = u0;
   const uint16_t *wsrc[4], *xsrc[S::XI];
   auto aim = [&](int s) {
     const StreamStrip t = stream_strip<GRP, S::BN>(g, s);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = wave * 32 + i * 8 + dr;
-      const int v = t.v0 + row, ch = (lane & 7) ^ ((row >> 1) & 7);
+      const int row = wave * (16 * RT) + i * S::RPI + dr;
+      const int v = t.v0 + row, ch = dslot ^ S::swz(row);
       wsrc[i] = v < g.Nv ? t.b + (size_t)wrow(g, v) * g.ldb + ch * 8 : nullptr;
     }
 #pragma unroll
     for (int i = 0; i < S::XI; ++i) {
-      const int row = (wave % S::XW * S::XI + i) * 8 + dr;
-      const int ch = (lane & 7) ^ ((row >> 1) & 7);
+      const int row = (wave % S::XW * S::XI + i) * S::RPI + dr;
+      const int ch = dslot ^ S::swz(row);
       xsrc[i] = t.a + (size_t)min(row, t.M - 1) * g.lda + ch * 8;
     }
   };
@@ -338,10 +350,10 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
   auto stage = [&](int buf) {
     uint8_t* b = smem + buf * S::STAGE;
     const bool live = dnext < u1;
-    const int k = dk * 64;
+    const int k = dk * KST;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = wave * 32 + i * 8 + dr, ch = (lane & 7) ^ ((row >> 1) & 7);
+      const int ch = dslot ^ S::swz(wave * (16 * RT) + i * S::RPI + dr);
       const uint16_t* p = live && wsrc[i] != nullptr && k + ch * 8 < g.K ? wsrc[i] + k : g.zeros;
       __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(b + (wave * 4 + i) * 1024), 16, 0, 2);
     }
@@ -349,7 +361,7 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
 #pragma unroll
     for (int i = 0; i < S::XI; ++i) {
       const int r0 = wave * S::XI + i;
-      const int row = r0 * 8 + dr, ch = (lane & 7) ^ ((row >> 1) & 7);
+      const int ch = dslot ^ S::swz(r0 * S::RPI + dr);
       const uint16_t* p = live && k + ch * 8 < g.K ? xsrc[i] + k : g.zeros;
       glds16(p, b + (NWV * 4 + r0) * 1024);
     }
@@ -363,17 +375,17 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
 #pragma unroll
   for (int p = 0; p < S::NS - 1; ++p) stage(p);
 
-  const int swz = (lane & 15) >> 1;
-  const uint32_t lrow = (uint32_t)(lane & 15) * 128;
-  const uint32_t off0 = (uint32_t)(((lane >> 4) ^ swz) * 16), off1 = (uint32_t)(((4 + (lane >> 4)) ^ swz) * 16);
-  const uint32_t lds0 = lds_off(smem) + lrow;
+  uint32_t off[2 * KC];
+#pragma unroll
+  for (int h = 0; h < 2 * KC; ++h)
+    off[h] = lds_off(smem) + (uint32_t)((lane & 15) * 128 * KC + ((4 * h + (lane >> 4)) ^ S::swz(lane & 15)) * 16);
 
-  cf32x4 acc[2][MT];
+  cf32x4 acc[RT][MT];
   int buf = 0, u = u0;
   while (u < u1) {
     const int s = u / KS, seg1 = min(u1, (s + 1) * KS);
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < RT; ++j)
 #pragma unroll
       for (int i = 0; i < MT; ++i) acc[j][i] = cf32x4{0.f, 0.f, 0.f, 0.f};
     for (; u < seg1; ++u) {
@@ -382,20 +394,24 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
       asm volatile("s_barrier" ::: "memory");
       // every wave has read the previous step's stage: it takes the step NS - 1 ahead
       stage(buf == 0 ? S::NS - 1 : buf - 1);
-      const uint32_t b = lds0 + buf * S::STAGE;
-      uint4 w[2][2];
-      stream_read<2>(b + wave * 4096 + off0, b + wave * 4096 + off1, w);
-      constexpr int XR = MT % 2 ? 1 : 2;
+      const uint32_t b = buf * S::STAGE;
+      constexpr int XR = MT % 2 ? 1 : 2, T16 = 2048 * KC;   // bytes of 16 rows
 #pragma unroll
-      for (int i = 0; i < MT; i += XR) {
-        uint4 x[XR][2];
-        stream_read<XR>(b + NWV * 4096 + i * 2048 + off0, b + NWV * 4096 + i * 2048 + off1, x);
+      for (int c = 0; c < KC; ++c) {
+        const uint32_t lo = b + off[2 * c], hi = b + off[2 * c + 1];
+        uint4 w[RT][2];
+        stream_read<RT, T16>(lo + wave * (RT * T16), hi + wave * (RT * T16), w);
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int i = 0; i < MT; i += XR) {
+          uint4 x[XR][2];
+          stream_read<XR, T16>(lo + (NWV * RT + i) * T16, hi + (NWV * RT + i) * T16, x);
 #pragma unroll
-          for (int p = 0; p < XR; ++p)
+          for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[j][i + p] = cmfma<DT>(w[j][h], x[p][h], acc[j][i + p]);
+            for (int p = 0; p < XR; ++p)
+#pragma unroll
+              for (int j = 0; j < RT; ++j) acc[j][i + p] = cmfma<DT>(w[j][h], x[p][h], acc[j][i + p]);
+        }
       }
       buf = buf + 1 == S::NS ? 0 : buf + 1;
     }
@@ -404,11 +420,11 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
     bool mine = lo == hi;
     if (lo != hi) {
       auto slot = [&](int w) {   // a share's first strip, or its last
-        return g.ws + ((size_t)(2 * w + (w * per / KS == s ? 0 : 1)) * NWV + wave) * (2 * MT * 256) + lane * 4;
+        return g.ws + ((size_t)(2 * w + (w * per / KS == s ? 0 : 1)) * NWV + wave) * (RT * MT * 256) + lane * 4;
       };
       float* p = slot(wg);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < RT; ++j)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
           if (i * 16 + (lane & 15) < t.M) park(p + (j * MT + i) * 256, acc[j][i]);
@@ -423,12 +439,12 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
         // in share order (the result does not hang on who came last), several shares in flight
         constexpr int UN = MT <= 2 ? 8 : 4;
         for (int w0 = lo; w0 <= hi; w0 += UN) {
-          cf32x4 o[UN][2][MT];
+          cf32x4 o[UN][RT][MT];
 #pragma unroll
           for (int q = 0; q < UN; ++q) {
             const float* p = slot(min(w0 + q, hi));
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < RT; ++j)
 #pragma unroll
               for (int i = 0; i < MT; ++i)
                 o[q][j][i] = i * 16 + (lane & 15) < t.M ? unpark(p + (j * MT + i) * 256) : cf32x4{0.f, 0.f, 0.f, 0.f};
@@ -436,7 +452,7 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
 #pragma unroll
           for (int q = 0; q < UN; ++q)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < RT; ++j)
 #pragma unroll
               for (int i = 0; i < MT; ++i) {
                 if (q == 0 && w0 == lo) acc[j][i] = o[0][j][i];
@@ -446,7 +462,7 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmArgs g) {
       }
       __syncthreads();
     }
-    if (mine) stream_store<DT, EPI, MT>(g, t, wave, lane, acc);
+    if (mine) stream_store<DT, EPI, MT, RT>(g, t, wave, lane, acc);
     // stores count with the DMA: drain them before the counted waits go on
     if (u < u1) __builtin_amdgcn_s_waitcnt(vm_wait(0));
   }
