@@ -334,10 +334,11 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
 // Which form a product of M rows takes: 0 the tile kernels (cake_gemm_scaled), 1 direct, 2 stream.
 // The estimates (us) are fits to timings on weights that no cache holds, 5 .. 64 rows, weight
 // matrices of 8 .. 260 MB; both sides of the lines they draw, measured: 4096 x 4096 at 16 rows
-// direct 11.5, stream 14.4; 4096 x 14336 direct 35, stream 25; 28672 x 4096 at 45 rows stream 53,
-// tiles 58; 4096 x 4096 at 45 rows stream 19, tiles 17.
-// (the stream form's shape, gemm_rows.h StreamShape)
+// direct 12.6, stream 12.5; 4096 x 14336 direct 38, stream 25; 6144 x 4096 at 5 rows direct 16.9,
+// stream 14.5, 3072 x 2048 6.5, 7.9; 28672 x 4096 at 45 rows stream 53, tiles 58; 4096 x 4096 at 45
+// rows stream 19, tiles 17.
 struct StreamPlan { int bn, kst, wgs; };
+// the stream form's shape (gemm_rows.h StreamShape)
 static StreamPlan stream_plan(int mt, bool gated) {
   return mt > 1 || gated ? StreamPlan{128, 64, 256} : StreamPlan{64, 128, 512};
 }
@@ -349,13 +350,14 @@ static int rows_kind(int M, long long Nv, int K, bool gated) {
   const StreamPlan sp = stream_plan(mt, gated);
   const long long strips = (Nv + sp.bn - 1) / sp.bn, ks = (K + sp.kst - 1) / sp.kst, total = strips * ks;
   const long long per = std::max<long long>((total + sp.wgs - 1) / sp.wgs, kRowsMinK / sp.kst);
-  const double stream = 7 + (ks > per || ks % per ? 0.7 * mt : 0.) + per * (16 + 2 * mt) / 27.;
+  const double stream = sp.wgs == 512 ? 6.2 + 0.08 * M + 1.42 * per
+                        : 7 + (ks > per || ks % per ? 0.7 * mt : 0.) + per * (16 + 2 * mt) / 27.;
   double direct = 1e9;
   if (M <= 32) {
     const int nt = gated || Nv > 4096 ? 2 : 1;
     const long long wgs = (Nv + 16 * nt - 1) / (16 * nt);
-    // a CU's share at 32 KB a us, all weights and half of the reads of x at 5.8 MB a us
-    direct = 4 + std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / 32,
+    // a CU's share at 32 (of two strips 26) KB a us, all weights and half of the reads of x at 5.8 MB
+    direct = 4 + std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
                           (Nv + 0.5 * wgs * M) * kb / 5800);
   }
   if (direct <= stream && direct <= tiles) return 1;

@@ -8,14 +8,13 @@
 //   barrier in the loop: 4096 x 4096 at 5 / 16 rows 9.7 / 11.5 us (tile kernel with split k and its
 //   finalize launch: 15-17 us), 2048 x 2048 6.1 / 7.1 us (14.6 us).  Every strip reads all of x
 //   from L2, which is what ends its range.
-// gemm_stream_kernel (M <= 64): 128 weight rows and the x tile go through LDS by DMA, 64 k per
-//   step; the steps of all strips form one sequence dealt out in equal contiguous shares, one
-//   workgroup per CU, so no last wave is left and the DMA never stops at a strip's end.  Strips
-//   that several shares cover meet in memory, the last to arrive sums in share order (the result
-//   does not hang on the order).  28672 x 4096 SwiGLU at 13 / 24 / 45 rows 44 / 46 / 53 us (tile
-//   kernels 58-60 us), 4096 x 23552 35 / 37 / 42 us (44-46 us).  The DMA moves 7 TB/s, L2 hits of
-//   x included, at any depth from three stages on, with 128 or 256 weight rows per strip and with
-//   one or two workgroups per CU alike: fewer x bytes per weight byte is what would speed it up.
+// gemm_stream_kernel (M <= 64): 128 weight rows by 64 k (up to 16 rows of x 64 by 128) and the x tile
+//   go through LDS by DMA; the steps of all strips form one sequence dealt out in equal contiguous
+//   shares, one workgroup per CU (two), so no last wave is left and the DMA never stops at a strip's
+//   end.  Strips that several shares cover meet in memory, the last to arrive sums in share order
+//   (the result does not hang on the order).  28672 x 4096 SwiGLU at 13 / 24 / 45 rows 44 / 46 / 53
+//   us (tile kernels 58-60 us), 4096 x 23552 35 / 37 / 42 us (44-46 us).  What bounds it is how much
+//   the waves of a CU have outstanding (StreamShape) and, in short shares, the parked sums.
 #pragma once
 #include "gemm_kernel.h"
 
