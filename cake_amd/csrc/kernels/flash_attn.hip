@@ -680,12 +680,14 @@ static int launch_flash(const FlashArgs& a, hipStream_t st) {
                   a.v_sh % 8 == 0 && a.o_sb % 4 == 0 && a.o_sh % 4 == 0 && al(a.q, 16) &&
                   al(a.k, 16) && al(a.v, 16) && al(a.o, 8);
   // causal 128-wide heads: flash3.h (rows past M must lie past the last row's end, and 32-bit
-  // offsets reach it).  64 query rows a wave once 256-row workgroups fill the chip one and a half
-  // times (32 heads: 2500 rows, 320 of them, 88 us against 81 with 32 rows; 3000, 384, 98 / 102;
-  // 6000 327 / 342)
-  const auto end = [&](long long sn) { return sn >= 128 ? ((long long)a.M * sn + 128) * 2 : 1LL << 40; };
-  if (v2 && a.causal && a.D == 128 && flash_ksplit() <= 1 && g_flash_nw == 0 &&
-      end(a.k_sn) < 0x7fffffffLL && end(a.v_sn) < 0x7fffffffLL) {
+  // offsets reach the tiles requested ahead).  64 query rows a wave once 256-row workgroups fill the
+  // chip one and a half times (32 heads: 2500 rows, 320 of them, 88 us against 81 with 32 rows; 3000,
+  // 384, 98 / 102; 6000 327 / 342)
+  const auto fits = [&](long long sn) {
+    return sn >= 128 && (a.M * sn + 128) * 2 < 0x7fffffffLL && (a.M + 256LL) * sn * 2 < 0xffffffffLL;
+  };
+  if (v2 && a.causal && a.D == 128 && flash_ksplit() <= 1 && g_flash_nw == 0 && fits(a.k_sn) &&
+      fits(a.v_sn)) {
     const long long wgs = (long long)((a.N + 255) / 256) * a.H * a.B;
     const int qs = wgs >= 384 ? 2 : 1;
     const dim3 g3(a.H * a.B, (a.N + 128 * qs - 1) / (128 * qs));

@@ -420,13 +420,14 @@ __global__ __launch_bounds__(256, 1) void mixer_flash3_kernel(MixFlashArgs a) {
 // scores, 8-byte output and gate rows, a sequence's keys and values under 2 GB (rows: its most).
 inline bool flash3_ok(int dt, const MixFlashArgs& a, bool lat, long long rows) {
   const auto al = [](const void* p, long long ld) { return (uintptr_t)p % 8 == 0 && ld % 4 == 0; };
-  const long long lim = 0x7fffffffLL / 2;
+  const long long lim = 0x7fffffffLL / 2;   // elements; the tiles requested ahead: offsets of 32 bits
+  const auto rows_fit = [&](long long ld) { return rows * ld < lim && (rows + 256) * ld < 2 * lim; };
   if ((dt != kBF16 && dt != kF16) || a.DVP != 128 || a.vdim != 128 || !(a.scale_log2 > 0.f) ||
       !al(a.out, a.ldo) || (a.gate && !al(a.gate, a.ldg)))
     return false;
   if (!lat) return a.DP == 128 && 128LL * a.S < lim;
-  return a.DP == 192 && a.lat.dimp == 128 && a.lat.rotp == 64 && rows * a.lat.ldk < lim &&
-         rows * a.lat.ldr < lim && 127 * a.lat.ldv + rows + 64 < lim;
+  return a.DP == 192 && a.lat.dimp == 128 && a.lat.rotp == 64 && rows_fit(a.lat.ldk) &&
+         rows_fit(a.lat.ldr) && 127 * a.lat.ldv + rows + 64 < lim;
 }
 
 template <int DT, bool LAT>
