@@ -1,5 +1,6 @@
 // Grouped products: rows sorted by weight group (routed experts), every row tile reading its own
-// group's weight.  The plain GEMM's tiles (gemm_kernel.h) with the tile list as their row map.
+// group's weight.  The plain GEMM's tiles (gemm_kernel.h, gemm_4w.h) with the tile list as their row
+// map.
 #include "gemm_kernel.h"
 
 namespace cake {
