@@ -62,6 +62,11 @@ CAKE_ROWS_EXTERN(kF16)
 
 using namespace cake;
 
+extern "C" int cake_gemm_grouped(int dt, int epi, int cfg, const void* a, long long lda,
+                                 const void* b, long long ldb, long long b_group, void* c,
+                                 long long ldc, const void* tiles, int max_tiles,
+                                 const void* zeros, int N, int K, hipStream_t st);
+
 // Counters of the four-wave tiles' pieces (zero at load; every launch leaves its region zero).  A
 // launch has a region of its own: launches that run side by side (several streams, a graph beside
 // eager work) never meet in one.  Eager launches take turns through more regions than a device's
@@ -416,7 +421,8 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
 }
 
 // cake_gemm_grouped in the stream form: tiles of at most 16 rows; ws and tick as above (ws of 16
-// rows), max_tiles strips of N within the counters
+// rows).  More strips than counters, or steps than the kernel's indexes hold (1024 experts of 4096
+// columns with 1500 rows): the 64-row tile, which takes the same tile list.
 CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long lda, const void* b,
                                     long long ldb, long long b_group, void* c, long long ldc,
                                     const void* tiles, int max_tiles, float* ws, void* tick,
@@ -424,9 +430,11 @@ CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long ld
   const StreamPlan sp = stream_plan(1, false);
   const long long strips = (long long)max_tiles * ((N + sp.bn - 1) / sp.bn);
   if (max_tiles <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || b_group % 8 ||
-      !(epi == 0 || (epi >= 7 && epi <= 10)) || !ws || !tick || !zeros || strips > kRowsTicks ||
-      strips * ((K + sp.kst - 1) / sp.kst) >= 0x40000000LL)
+      !(epi == 0 || (epi >= 7 && epi <= 10)) || !ws || !tick || !zeros)
     return (int)hipErrorInvalidValue;
+  if (strips > kRowsTicks || strips * ((K + sp.kst - 1) / sp.kst) >= 0x40000000LL)
+    return cake_gemm_grouped(dt, epi, 4, a, lda, b, ldb, b_group, c, ldc, tiles, max_tiles, zeros, N,
+                             K, st);
   GemmArgs g{};
   g.a = (const uint16_t*)a; g.b = (const uint16_t*)b; g.c = (uint16_t*)c;
   g.ws = ws; g.tick = (unsigned*)tick; g.zeros = (const uint16_t*)zeros;

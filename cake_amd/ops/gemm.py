@@ -444,6 +444,8 @@ def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out
     if tiles.dtype != torch.int32 or not tiles.is_contiguous() or tiles.dim() != 2 or \
             tiles.shape[0] < 2 or tiles.shape[1] != 4 or not tiles.is_cuda or tiles.data_ptr() % 16:
         raise ValueError("grouped: tiles must be a contiguous int32 [n + 1, 4] device tensor")
+    if cfg == ROWS and torch.cuda.is_current_stream_capturing():
+        cfg = 4   # rows planned before the capture: the 64-row tile takes the same tile list
     if cfg == ROWS:
         st = torch.cuda.current_stream().cuda_stream
         ws, tick = _rows_state(x.device, 16, st)

@@ -1,5 +1,6 @@
 """Rule of the products of few rows (gemm.hip rows_kind): which form takes which sizes."""
 import pytest
+import torch
 
 from cake_amd.build import GEMM_LIB
 
@@ -22,3 +23,17 @@ def test_grouped_rows_stay_out_of_graphs():
     from cake_amd.ops import gemm as G
     assert G.grouped_cfg(78, 64) == G.ROWS and G.grouped_cfg(78, 64, capturing=True) == 4
     assert G.grouped_cfg(64 * 5, 64) == 4
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="makes launches without operands")
+@pytest.mark.parametrize("E,N,K,rows", [(1024, 4096, 64, 1500), (512, 8192, 64, 2048),
+                                        (1024, 4096, 4096, 4096), (1, 64, 64, 1)])
+def test_routed_products_of_any_width_pass_the_checks(E, N, K, rows):
+    """Tile lists with more strips than counters are not refused: without a device every call that
+    passes the checks ends at its launch, never with an invalid value."""
+    from cake_amd.ops import gemm as G
+    L, invalid = G._lib(), 1
+    tiles = rows // 16 + min(E, rows)
+    args = (64, K, 64, K, N * K, 64, N, 64, tiles, 64, 64, 64, N, K, None)
+    assert L.cake_gemm_rows_grouped(0, 0, *args) not in (0, invalid)
+    assert L.cake_gemm_rows_grouped(0, 1, *args) == invalid   # an epilogue that it does not carry

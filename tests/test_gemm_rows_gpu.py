@@ -132,7 +132,8 @@ def test_linear_takes_the_planned_form(cuda, M, N, K):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("N,K,top,E,tokens,act", [(1640, 2048, 6, 64, 13, "relu2"), (40, 72, 2, 5, 9, None),
-                                                  (128, 64, 1, 1024, 30, "gelu"), (272, 520, 3, 7, 1, None)])
+                                                  (128, 64, 1, 1024, 30, "gelu"), (272, 520, 3, 7, 1, None),
+                                                  (4160, 8, 2, 1024, 750, "silu")])   # strips past the counters
 def test_grouped_rows(cuda, dt, N, K, top, E, tokens, act):
     from cake_amd.ops import experts as X
     from cake_amd.ops import gemm as G
@@ -156,3 +157,28 @@ def test_grouped_rows(cuda, dt, N, K, top, E, tokens, act):
         want = getattr(torch.nn.functional, act)(want)
     scale = want.pow(2).mean().sqrt() + want.abs()
     assert bool(((out.double() - want).abs() <= (K * 2.0 ** -22 + STEP[dt]) * scale).all())
+
+
+def test_rows_planned_before_a_capture(cuda):
+    """A tile list of the stream form used under capture: no counters in the graph, and replays
+    equal the eager result."""
+    from cake_amd.ops import experts as X
+    from cake_amd.ops import gemm as G
+    E, N, K = 16, 200, 264
+    logits = torch.randn(20, E, device="cuda")
+    p = X.plan(*X.route(logits, 2), E, torch.bfloat16)
+    assert p.cfg == G.ROWS
+    x = torch.randn(40, K, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(E, N, K, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    want = X.product(x, w, p, torch.empty(40, N, device="cuda", dtype=torch.bfloat16)).float()
+    out = torch.empty(40, N, device="cuda", dtype=torch.bfloat16)
+    before, graph = set(G._ticks), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        X.product(x, w, p, out)
+    assert set(G._ticks) == before
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        torch.testing.assert_close(out.float(), want, rtol=2.0 ** -7, atol=2.0 ** -7)
+        X.product(x, w, p, torch.empty_like(out))
