@@ -24,8 +24,8 @@ int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long lda, cons
                    float alpha, hipStream_t st);
 int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* a, long long lda,
                      const void* b, long long ldb, void* c, long long ldc, const void* bias,
-                     void* resid, long long ldr, float* ws, const void* zeros, int M, int N, int K,
-                     float alpha, hipStream_t st);
+                     void* resid, long long ldr, float* ws, void* tick, const void* zeros, int M,
+                     int N, int K, float alpha, hipStream_t st);
 }
 
 namespace {
@@ -49,8 +49,8 @@ struct CakeBlockRun {
   const float* inv_freq;
   const void* zeros;
   float* ws;                    // split-k slabs of the tile plans
-  float* rows_ws;               // workspace and counters of the stream form
-  void* rows_tick;
+  float* rows_ws;               // workspace of the stream form
+  void* tick;                   // counters of either
   Form qkv_form, o_form, gu_form, down_form;
   int n, dt, T, H, I, nh, nkv, hd, S, pos0;
   float eps, scale;
@@ -70,10 +70,10 @@ CAKE_API int cake_block_rows(const CakeBlockRun* r, hipStream_t st) {
     void* resid = epi == kEpiResid32 ? r->hidden : nullptr;
     const long long ldr = resid ? N : 0, ldc = resid ? 0 : N;
     return f.kind ? cake_gemm_rows(r->dt, epi, f.kind, a, K, w, K, c, ldc, nullptr, resid, ldr,
-                                   r->rows_ws, r->rows_tick, r->zeros, T, N, K, 1.f, st)
+                                   r->rows_ws, r->tick, r->zeros, T, N, K, 1.f, st)
                   : cake_gemm_scaled(r->dt, epi, f.cfg, f.splits, a, K, w, K, c, ldc, nullptr,
-                                     resid, ldr, f.splits > 1 ? r->ws : nullptr, r->zeros, T, N, K,
-                                     1.f, st);
+                                     resid, ldr, f.splits > 1 ? r->ws : nullptr, r->tick, r->zeros, T,
+                                     N, K, 1.f, st);
   };
   uint16_t* q = static_cast<uint16_t*>(r->qkv);
   for (int i = 0; i < r->n; ++i) {

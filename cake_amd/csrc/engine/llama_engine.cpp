@@ -67,7 +67,9 @@ int cake_flash_attn(int dt, const void* q, const void* k, const void* v, void* o
 long long cake_gemm_ws_floats(int cfg, int splits, int M, int N, int K, int gated);
 int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long long lda, const void* b,
               long long ldb, void* c, long long ldc, const void* bias, void* resid,
-              long long ldr, float* ws, const void* zeros, int M, int N, int K, hipStream_t st);
+              long long ldr, float* ws, void* tick, const void* zeros, int M, int N, int K,
+              hipStream_t st);
+int cake_gemm_ticks();
 int cake_gemm_rows_kind(int M, long long Nv, int K, int gated);
 long long cake_gemm_rows_ws_floats(int M);
 int cake_gemm_rows_ticks();
@@ -815,7 +817,7 @@ class Llama {
   int* scratch_i32_ = nullptr;  // warm-up snapshot: tok, pos, hist_len
   float* scratch_resid_ = nullptr;
   int32_t* zeros_ = nullptr;    // 64 zero words (GEMM LDS-DMA padding source)
-  int32_t* ticks_ = nullptr;    // arrival counters of the few-row products, zero between launches
+  int32_t* ticks_ = nullptr;    // arrival counters of the products, zero between launches
   // prefill buffers (grown to the longest prompt)
   int pre_T_ = 0;
   float* hidden_ = nullptr;
@@ -1039,13 +1041,14 @@ class Llama {
     scratch_i32_ = dalloc<int>(4);
     scratch_resid_ = dalloc<float>(c.H + 4);  // + the hop header (self-tests)
     zeros_ = dalloc<int32_t>(64);
-    ticks_ = dalloc<int32_t>(cake_gemm_rows_ticks());
+    const int ticks = std::max(cake_gemm_rows_ticks(), cake_gemm_ticks());
+    ticks_ = dalloc<int32_t>(ticks);
     hip_check(hipMemset(tickets_, 0, sizeof(unsigned int) * (2 * c.nkv + 2)), "memset");
     hip_check(hipMemset(part_, 0, sizeof(float) * 2 * c.nh * kAttnMaxSplit * (c.hd + 2)), "memset");
     hip_check(hipMemset(sel_ticket_, 0, sizeof(unsigned int)), "memset");
     hip_check(hipMemset(slot_, 0, sizeof(unsigned long long)), "memset");
     hip_check(hipMemset(zeros_, 0, sizeof(int32_t) * 64), "memset");
-    hip_check(hipMemset(ticks_, 0, sizeof(int32_t) * cake_gemm_rows_ticks()), "memset");
+    hip_check(hipMemset(ticks_, 0, sizeof(int32_t) * ticks), "memset");
     hip_check(hipMemset(hist_, 0, sizeof(int) * S_), "memset");
     hip_check(hipMemset(resid_, 0, sizeof(float) * (c.H + 4)), "memset");
     // opt-in (CAKE_ATTN_OPROJ=1): measured slower than the attention + o_proj pair on
@@ -1221,7 +1224,7 @@ class Llama {
       ws = ws_;
     }
     k_check(cake_gemm(dt_, epi, p.first, splits, a, lda, b, ldb, cptr, ldc, nullptr, resid, ldr,
-                      ws, zeros_, M, N, K, st_), what);
+                      ws, ticks_, zeros_, M, N, K, st_), what);
   }
 
   // hipBLASLt's first call in a process costs ~175 ms (library init; a new shape after it

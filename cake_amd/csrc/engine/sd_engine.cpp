@@ -57,7 +57,9 @@ int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long lda, cons
                    float alpha, hipStream_t st);
 int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long long lda, const void* b,
               long long ldb, void* c, long long ldc, const void* bias, void* resid,
-              long long ldr, float* ws, const void* zeros, int M, int N, int K, hipStream_t st);
+              long long ldr, float* ws, void* tick, const void* zeros, int M, int N, int K,
+              hipStream_t st);
+int cake_gemm_ticks();
 int cake_flash_attn_ws(int dt, const void* q, const void* k, const void* v, void* o, int B, int H,
                        int Hkv, int N, int M, int D, const long long* strides, float scale,
                        int causal, int pos0, void* ws, long long ws_bytes, hipStream_t st);
@@ -512,6 +514,8 @@ class SdEngine {
     planner_.load(pkg_dir() + "/ops/gemm_tuned.json");
     zeros_ = dalloc(256);
     hip_check(hipMemset(zeros_, 0, 256), "memset");
+    ticks_ = dalloc(4 * cake_gemm_ticks());
+    hip_check(hipMemset(ticks_, 0, 4 * cake_gemm_ticks()), "memset");
     gn_tickets_ = static_cast<unsigned int*>(dalloc(256 * 4));
     hip_check(hipMemset(gn_tickets_, 0, 256 * 4), "memset");
     build_and_load();
@@ -1481,7 +1485,7 @@ class SdEngine {
     k_check(cake_gemm(dt_, epi, pl.first, pl.second, x, lda, w, K, f32out ? nullptr : out,
                       f32out ? 0 : ldc,
                       bias, f32out ? out : const_cast<void*>(resid), f32out ? ldc : ldr, ws,
-                      zeros_, M, N, K, st_), "gemm");
+                      ticks_, zeros_, M, N, K, st_), "gemm");
   }
 
   uint16_t* group_norm(Arena& A, const uint16_t* x, const uint16_t* x2, int Cx, int N, int HW,
@@ -2501,6 +2505,7 @@ class SdEngine {
   void* scratch_ = nullptr;
   size_t scratch_bytes_ = 0;
   void* zeros_ = nullptr;
+  void* ticks_ = nullptr;   // arrival counters of the products, zero between launches
   unsigned int* gn_tickets_ = nullptr;
   float* ws_ = nullptr;
   size_t ws_n_ = 0;

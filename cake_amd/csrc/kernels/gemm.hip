@@ -39,7 +39,6 @@
 #include "gemm_rows.h"
 
 #include <algorithm>
-#include <atomic>
 
 namespace cake {
 // the launchers are instantiated in gemm_inst_{bf16,f16}_{a,b,c}.hip
@@ -67,29 +66,12 @@ extern "C" int cake_gemm_grouped(int dt, int epi, int cfg, const void* a, long l
                                  long long ldc, const void* tiles, int max_tiles,
                                  const void* zeros, int N, int K, hipStream_t st);
 
-// Counters of the four-wave tiles' pieces (zero at load; every launch leaves its region zero).  A
-// launch has a region of its own: launches that run side by side (several streams, a graph beside
-// eager work) never meet in one.  Eager launches take turns through more regions than a device's
-// queues hold launches; a captured launch keeps its region for the life of the process, and when
-// those are used up it runs its tiles whole.
-constexpr unsigned kEagerRegions = 2048, kGraphRegions = 2048, kRegion = 2 * kPieceTiles;
-__device__ unsigned g_piece_tick[(size_t)(kEagerRegions + kGraphRegions) * kRegion];
-
-static unsigned* piece_ticks(hipStream_t st) {
-  static std::atomic<unsigned> eager{0}, graph{0};
-  // the symbol's address on the current device (looked up per call: a few hundred ns, and right on
-  // every device)
-  void* base = nullptr;
-  if (hipGetSymbolAddress(&base, HIP_SYMBOL(g_piece_tick)) != hipSuccess) return nullptr;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cap) != hipSuccess) return nullptr;
-  unsigned r = eager.fetch_add(1, std::memory_order_relaxed) % kEagerRegions;
-  if (cap != hipStreamCaptureStatusNone) {
-    r = graph.fetch_add(1, std::memory_order_relaxed);
-    if (r >= kGraphRegions) return nullptr;
-    r += kEagerRegions;
-  }
-  return static_cast<unsigned*>(base) + (size_t)r * kRegion;
+// Which capture records the stream's launches: 0 none, else an id of that capture, -1 an error.
+CAKE_API long long cake_stream_capture(hipStream_t st) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(st, &status, &id) != hipSuccess) return -1;
+  return status == hipStreamCaptureStatusNone ? 0 : (long long)(id + 1);
 }
 
 static inline void cfg_dims(int cfg, int& bm, int& bn) {
@@ -265,15 +247,20 @@ CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* c
   return 0;
 }
 
+// counters of tick below
+CAKE_API int cake_gemm_ticks() { return 2 * kPieceTiles; }
+
 // y = epilogue(x W^T).  N = output features (gated: W has 2N rows, gate rows
-// [0, N), up/gate-2 rows [N, 2N)).  splits > 1 needs ws = splits * M * Nv f32.
+// [0, N), up/gate-2 rows [N, 2N)).  splits > 1 needs ws (cake_gemm_ws_floats) and, for a four-wave
+// tile, tick (cake_gemm_ticks zeros, zero again when the launch is done): both belong to one launch
+// at a time, so to one stream, or to one graph.
 // Requirements (host-checked in ops/gemm.py): K % 8 == 0, lda/ldb % 8 == 0,
 // 16-byte aligned operand bases, gated => N % 16 == 0.
 // alpha (f32 epilogues only, 1 elsewhere): r32 (+)= alpha * (x W^T + bias).
 CAKE_API int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* a, long long lda,
                               const void* b, long long ldb, void* c, long long ldc,
                               const void* bias, void* resid, long long ldr, float* ws,
-                              const void* zeros, int M, int N, int K, float alpha,
+                              void* tick, const void* zeros, int M, int N, int K, float alpha,
                               hipStream_t st) {
   if (alpha != 1.f && epi != kEpiResid32 && epi != kEpiStore32) return (int)hipErrorInvalidValue;
   int bm, bn;
@@ -308,13 +295,11 @@ CAKE_API int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* 
   g.kps = sp.kps;
   dim3 grid(g.tiles_m * g.tiles_n, splits);
   if (sp.pieces > 0) {
-    if (ws != nullptr && (g.tick = piece_ticks(st)) != nullptr) {
-      g.pieces = sp.pieces;
-      g.dp_tiles = sp.ntiles - sp.rest;
-      grid = dim3(g.dp_tiles + sp.rest * sp.pieces, 1);
-    } else {
-      g.kps = K;   // whole tiles
-    }
+    if (ws == nullptr || tick == nullptr) return (int)hipErrorInvalidValue;
+    g.tick = static_cast<unsigned*>(tick);
+    g.pieces = sp.pieces;
+    g.dp_tiles = sp.ntiles - sp.rest;
+    grid = dim3(g.dp_tiles + sp.rest * sp.pieces, 1);
   }
   const int kernel_epi = splits > 1 ? (int)kEpiPartial : epi;
   if (splits > 1 && ws == nullptr) return (int)hipErrorInvalidValue;
@@ -329,9 +314,9 @@ CAKE_API int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* 
 
 CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long long lda,
                        const void* b, long long ldb, void* c, long long ldc, const void* bias,
-                       void* resid, long long ldr, float* ws, const void* zeros, int M, int N,
-                       int K, hipStream_t st) {
-  return cake_gemm_scaled(dt, epi, cfg, splits, a, lda, b, ldb, c, ldc, bias, resid, ldr, ws,
+                       void* resid, long long ldr, float* ws, void* tick, const void* zeros, int M,
+                       int N, int K, hipStream_t st) {
+  return cake_gemm_scaled(dt, epi, cfg, splits, a, lda, b, ldb, c, ldc, bias, resid, ldr, ws, tick,
                           zeros, M, N, K, 1.f, st);
 }
 

@@ -13,6 +13,7 @@ scripts/tune_gemm.py on the GPU box).
 from __future__ import annotations
 
 import ctypes as C
+import threading
 
 import torch
 
@@ -34,6 +35,7 @@ _SLOTS = {0: 2, 1: 2, 2: 1, 3: 1, 4: 4, 5: 1, 6: 1, 7: 1, 8: 2, 11: 1, 12: 2, 13
 NO_GATED = {14, 17, 18, 19}
 # register-staged / four-wave 256x256 (gemm_rs.h, gemm_4w.h): whole 64-element k steps only
 K64_ONLY = {21, 22, 23, 24, 25, 26, 27}
+FOUR_WAVE = {22, 23, 24, 25, 26, 27}   # split k in pieces of a tile (gemm_4w.h)
 # relative per-tile throughput (measured per-config sweep,
 # profiles/r2_gemm_sweep_agpr.jsonl): the AGPR-accumulator 128x128 tile (0) for most
 # shapes, the 8-wave 256x256 tile (11) where its tiles fill the chip, 64-wide tiles
@@ -60,9 +62,13 @@ def _lib():
     lib = library("gemm")
     if not _bound:
         P, I, L = C.c_void_p, C.c_int, C.c_longlong
-        lib.cake_gemm_scaled.argtypes = [I, I, I, I, P, L, P, L, P, L, P, P, L, P, P, I, I, I,
+        lib.cake_gemm_scaled.argtypes = [I, I, I, I, P, L, P, L, P, L, P, P, L, P, P, P, I, I, I,
                                          C.c_float, P]
         lib.cake_gemm_scaled.restype = I
+        lib.cake_gemm_ticks.argtypes = []
+        lib.cake_gemm_ticks.restype = I
+        lib.cake_stream_capture.argtypes = [P]
+        lib.cake_stream_capture.restype = L
         lib.cake_gemm_ws_floats.argtypes = [I, I, I, I, I, I]
         lib.cake_gemm_ws_floats.restype = L
         lib.cake_gemm_grouped.argtypes = [I, I, I, P, L, P, L, L, P, L, P, I, P, I, I, P]
@@ -118,7 +124,9 @@ def _workspace(dev, numel: int) -> torch.Tensor:
 
 ROWS_MAX = 64   # rows that the products of few rows take at most
 _rows_kinds: dict = {}
-_ticks: dict = {}   # (device, stream) -> arrival counters of the stream form, newest last
+_ticks: dict = {}         # (device, stream) -> arrival counters, newest last
+_graph_ticks: dict = {}   # (device, stream) -> (capture, counters) of its latest capture
+_lock = threading.RLock()
 
 
 def rows_kind(M: int, Nv: int, K: int, gated: bool) -> int:
@@ -132,18 +140,47 @@ def rows_kind(M: int, Nv: int, K: int, gated: bool) -> int:
     return kind
 
 
-def _rows_state(dev, M: int, st: int):
-    """(workspace, counters) of one launch of the stream form.  The counters are zero between
-    launches; two launches that run side by side need their own, so they belong to a stream.  A
-    captured graph may run beside any stream: none for it (the caller takes the tile kernels)."""
+def _newest(table: dict, key, value) -> None:
+    """table[key] = value, of the 16 newest streams (memory of the others is freed in the order of
+    its own stream)."""
+    table.pop(key, None)
+    while len(table) >= 16:
+        table.pop(next(iter(table)))
+    table[key] = value
+
+
+def _counters(dev, st: int) -> torch.Tensor:
+    """Arrival counters of a launch on stream `st`, the current one: zero between launches.
+    Launches of one stream run one after the other and share them; launches that may run side by
+    side never do.  A captured graph may run beside any stream, so its counters are its own: memory
+    of its pool, cleared by a fill at the head of every replay, as long-lived as the graph."""
     key = (dev, st)
-    t = _ticks.pop(key, None)
-    if t is None:
-        t = torch.zeros(_lib().cake_gemm_rows_ticks(), dtype=torch.int32, device=dev)
-        while len(_ticks) >= 16:   # freed in the order of its own stream
-            _ticks.pop(next(iter(_ticks)))
-    _ticks[key] = t
-    return torch.empty(int(_lib().cake_gemm_rows_ws_floats(M)), dtype=torch.float32, device=dev), t
+    lib = _lib()
+    with _lock:
+        if torch.cuda.is_current_stream_capturing():
+            capture = lib.cake_stream_capture(st)
+            if capture <= 0:
+                raise RuntimeError("gemm: the capture of the current stream is not to be told")
+            have = _graph_ticks.get(key)
+            if have is None or have[0] != capture:
+                have = (capture, torch.zeros(_n_ticks(), dtype=torch.int32, device=dev))
+                _newest(_graph_ticks, key, have)
+            return have[1]
+        t = _ticks.get(key)
+        if t is None:
+            t = torch.zeros(_n_ticks(), dtype=torch.int32, device=dev)
+        _newest(_ticks, key, t)
+        return t
+
+
+def _n_ticks() -> int:
+    return max(_lib().cake_gemm_rows_ticks(), _lib().cake_gemm_ticks())
+
+
+def _rows_state(dev, M: int, st: int):
+    """(workspace, counters) of one launch of the stream form."""
+    return torch.empty(int(_lib().cake_gemm_rows_ws_floats(M)), dtype=torch.float32,
+                       device=dev), _counters(dev, st)
 
 
 def _load_tuned() -> list:
@@ -395,14 +432,16 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
     if cfg == LIB:  # an epilogue / bias / strided output the library form does not carry
         cfg, s0 = plan_mfma(M, Nv, K, epi)
     splits = s0 if splits is None else max(1, int(splits))
-    # the kernel library sizes it (an in-kernel pair needs its slabs only)
+    # the kernel library sizes it (pieces of a tile need their slabs only)
+    st = torch.cuda.current_stream().cuda_stream
+    tick = _counters(x.device, st) if splits > 1 and cfg in FOUR_WAVE else None
     ws = _workspace(x.device, int(_lib().cake_gemm_ws_floats(
         int(cfg), int(splits), M, N, K, 1 if Nv != N else 0))) if splits > 1 else None
     check(_lib().cake_gemm_scaled(
         _DT[x.dtype], EPI[epi], int(cfg), int(splits), x2.data_ptr(), lda, w.data_ptr(), ldb, cptr,
         ldc, None if bias is None else bias.data_ptr(), rptr, ldr,
-        None if ws is None else ws.data_ptr(), _zeros16(x.device).data_ptr(), M, N, K,
-        float(alpha), torch.cuda.current_stream().cuda_stream), "gemm")
+        None if ws is None else ws.data_ptr(), None if tick is None else tick.data_ptr(),
+        _zeros16(x.device).data_ptr(), M, N, K, float(alpha), st), "gemm")
     return resid if f32_out else out
 
 

@@ -21,7 +21,7 @@ class _Form(C.Structure):
 
 class _Run(C.Structure):
     _fields_ = [(n, P) for n in ("blocks", "hidden", "x", "qkv", "att", "act", "inv_freq", "zeros",
-                                 "ws", "rows_ws", "rows_tick")] + \
+                                 "ws", "rows_ws", "tick")] + \
                [(n, _Form) for n in ("qkv_form", "o_form", "gu_form", "down_form")] + \
                [(n, I) for n in ("n", "dt", "T", "H", "I", "nh", "nkv", "hd", "S", "pos0")] + \
                [("eps", F), ("scale", F)]
@@ -92,6 +92,8 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
     rows_ws = tick = None
     if any(f.kind == 2 for f in forms):
         rows_ws, tick = G._rows_state(dev, T, st)
+    elif any(f.splits > 1 and f.cfg in G.FOUR_WAVE for f in forms):
+        tick = G._counters(dev, st)
     ptr = [None if t is None else t.data_ptr() for t in (
         hidden, x, qkv, att, act, inv_freq, G._zeros16(dev), ws, rows_ws, tick)]
     run = _Run(C.addressof(table), *ptr, *forms, len(blocks), G._DT[dt], T, H, inter, nh, nkv, hd, S,

@@ -32,23 +32,84 @@ def test_pieces_sum_to_the_product(cuda, cfg, M, N, K, splits, epi):
 
 
 def test_pieces_in_a_graph_beside_eager_work(cuda):
-    """A captured launch keeps counters of its own: replays beside eager launches of the same
-    product on another stream give the eager result, every time."""
+    """A captured launch keeps counters of its own: replays while eager launches of the same
+    product run on another stream give the eager result, every time, and so do those."""
     from cake_amd.ops import gemm as G
     x = torch.randn(500, 4096, device="cuda").to(torch.bfloat16)
     w = (torch.randn(4096, 4096, device="cuda") * 2.0 ** -6).to(torch.bfloat16)
     want = G.linear(x, w, cfg=27, splits=2)
-    out = torch.empty_like(want)
     graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    held = [torch.empty_like(want) for _ in range(4)]
+    outs = [[torch.zeros_like(want) for _ in range(12)] for _ in range(2)]
+    with torch.cuda.stream(side):
+        G.linear(x, w, cfg=27, splits=2)   # its workspace and counters
     G._workspace(x.device, 1 << 26)
     with torch.cuda.graph(graph):
-        G.linear(x, w, cfg=27, splits=2, out=out)
-    for _ in range(4):
-        out.zero_()
-        torch.cuda.synchronize()
+        for o in held:
+            G.linear(x, w, cfg=27, splits=2, out=o)
+    torch.cuda.synchronize()
+    for i in range(3):   # nothing waits between the two streams
+        graph.replay()
+        for o, h in zip(outs[0][4 * i:], held):
+            o.copy_(h)
+        with torch.cuda.stream(side):
+            for o in outs[1][4 * i:4 * i + 4]:
+                G.linear(x, w, cfg=27, splits=2, out=o)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for side_outs in outs for o in side_outs)
+
+
+def test_counters_are_of_a_stream_or_of_a_capture(cuda):
+    """Launches that may run side by side never share counters, however many there were; a stream's
+    stay its own and zero; the newest 16 streams keep theirs."""
+    from cake_amd.ops import gemm as G
+    dev = torch.empty(1, device="cuda").device
+
+    def here():
+        return G._counters(dev, torch.cuda.current_stream().cuda_stream)
+    streams = [torch.cuda.Stream() for _ in range(20)]
+    mine = here()
+    eager = []
+    for s in streams[:15]:
+        with torch.cuda.stream(s):
+            eager.append(here())
+    for _ in range(5000):
+        assert here() is mine
+    for s, t in zip(streams, eager):
+        with torch.cuda.stream(s):
+            assert here() is t
+    captured, graphs = [], [torch.cuda.CUDAGraph() for _ in range(3)]
+    for g in graphs:   # one after the other on PyTorch's one capture stream
+        with torch.cuda.graph(g):
+            captured.append(here())
+            assert here() is captured[-1]
+    ptrs = {t.data_ptr() for t in [mine, *eager, *captured]}
+    assert len(ptrs) == 1 + len(eager) + len(captured)
+    for s in streams:   # more streams than are kept
+        with torch.cuda.stream(s):
+            assert not bool(here().any())
+    assert len(G._ticks) <= 16 and here() is not mine and not bool(here().any())
+    captured[0].fill_(7)   # another use of the graph's pool: a replay starts from zero
+    graphs[0].replay()
+    torch.cuda.synchronize()
+    assert not bool(captured[0].any())
+
+
+def test_many_captures_keep_their_pieces(cuda):
+    """The thousandth capture runs the same kernel as the first: the same bits."""
+    from cake_amd.ops import gemm as G
+    x = torch.randn(130, 512, device="cuda").to(torch.bfloat16)
+    w = torch.randn(256, 512, device="cuda").to(torch.bfloat16)
+
+    def product(out, splits=3):
+        return G.linear(x, w, epi="store32", resid=out, cfg=27, splits=splits)
+    want = product(torch.empty(130, 256, device="cuda"))
+    assert not torch.equal(want, product(torch.empty_like(want), 1))   # sums in another order
+    for _ in range(5):
+        graph, outs = torch.cuda.CUDAGraph(), [torch.empty_like(want) for _ in range(500)]
+        with torch.cuda.graph(graph):
+            for o in outs:
+                product(o)
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out, want)
-        with torch.cuda.stream(side):
-            assert torch.equal(G.linear(x, w, cfg=27, splits=2), want)
-        torch.cuda.synchronize()
+        assert all(torch.equal(o, want) for o in outs)

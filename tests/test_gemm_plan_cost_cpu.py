@@ -2,6 +2,7 @@
 import random
 
 import pytest
+import torch
 
 from cake_amd.build import GEMM_LIB
 
@@ -48,3 +49,19 @@ def test_workspace_covers_the_pieces():
     assert L.cake_gemm_ws_floats(25, 8, 4500, 4096, 14336, 0) == 32 * 8 * 256 * 256   # 288 tiles
     assert L.cake_gemm_ws_floats(27, 2, 1100, 4096, 14336, 0) == 0                     # 144 tiles
     assert L.cake_gemm_ws_floats(22, 2, 2048, 8192, 8192, 0) == 0                      # one wave
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="makes launches without operands")
+@pytest.mark.parametrize("cfg,splits,M", [(22, 4, 777), (27, 2, 129)])
+def test_pieces_take_the_callers_counters(cfg, splits, M):
+    """Tiles in pieces need the workspace and the counters of the caller's stream: refused without
+    either; with both, and whole tiles without, the call ends at its launch (no device)."""
+    from cake_amd.ops import gemm as G
+    L, invalid = G._lib(), 1
+
+    def call(splits, ws, tick):
+        return L.cake_gemm_scaled(0, 0, cfg, splits, 64, 4096, 64, 4096, 64, 4096, None, None, 0, ws,
+                                  tick, 64, M, 4096, 4096, 1.0, None)
+    assert call(splits, 64, 64) not in (0, invalid) and call(1, None, None) not in (0, invalid)
+    assert call(splits, None, 64) == invalid and call(splits, 64, None) == invalid
+    assert 0 < L.cake_gemm_ticks() <= L.cake_gemm_rows_ticks()
