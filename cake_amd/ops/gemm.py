@@ -52,7 +52,10 @@ LIB_EPIS = ("store", "resid32", "store32", "swiglu")
 _LIB_WS_BYTES = 32 << 20
 _bound = False
 _plans: dict = {}
-_ws: dict = {}
+_ws: dict = {}            # (device, stream) -> split-K slabs, newest last
+_ticks: dict = {}         # (device, stream) -> arrival counters, newest last
+_graph_ticks: dict = {}   # (device, stream) -> (capture, counters) of its latest capture
+_lock = threading.RLock()
 _zeros: dict = {}
 
 
@@ -107,26 +110,32 @@ def _zeros16(dev) -> torch.Tensor:
     return z
 
 
-_ws_keep: list = []
+def _newest(table: dict, key, value) -> None:
+    """table[key] = value, of the 16 newest streams (memory of the others is freed in the order of
+    its own stream)."""
+    table.pop(key, None)
+    while len(table) >= 16:
+        table.pop(next(iter(table)))
+    table[key] = value
 
 
 def _workspace(dev, numel: int) -> torch.Tensor:
-    """Split-K slabs of the current stream (launches on two streams may run side by side).
-    Superseded buffers are kept alive: a captured hipGraph may still point at them."""
+    """Split-K slabs of one launch on the current stream: the stream's own (launches on two streams
+    may run side by side).  Under capture the graph's own, of its memory pool: graphs share a
+    capture stream and may be replayed side by side."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(numel, dtype=torch.float32, device=dev)
     key = (dev, torch.cuda.current_stream(dev).cuda_stream)
-    w = _ws.get(key)
-    if w is None or w.numel() < numel:
-        if w is not None:
-            _ws_keep.append(w)
-        w = _ws[key] = torch.empty(max(numel, 1 << 20), dtype=torch.float32, device=dev)
+    with _lock:
+        w = _ws.get(key)
+        if w is None or w.numel() < numel:
+            w = torch.empty(max(numel, 1 << 20), dtype=torch.float32, device=dev)
+        _newest(_ws, key, w)
     return w
 
 
 ROWS_MAX = 64   # rows that the products of few rows take at most
 _rows_kinds: dict = {}
-_ticks: dict = {}         # (device, stream) -> arrival counters, newest last
-_graph_ticks: dict = {}   # (device, stream) -> (capture, counters) of its latest capture
-_lock = threading.RLock()
 
 
 def rows_kind(M: int, Nv: int, K: int, gated: bool) -> int:
@@ -138,15 +147,6 @@ def rows_kind(M: int, Nv: int, K: int, gated: bool) -> int:
     if kind is None:
         kind = _rows_kinds[key] = int(_lib().cake_gemm_rows_kind(M, Nv, K, int(gated)))
     return kind
-
-
-def _newest(table: dict, key, value) -> None:
-    """table[key] = value, of the 16 newest streams (memory of the others is freed in the order of
-    its own stream)."""
-    table.pop(key, None)
-    while len(table) >= 16:
-        table.pop(next(iter(table)))
-    table[key] = value
 
 
 def _counters(dev, st: int) -> torch.Tensor:

@@ -43,7 +43,6 @@ def test_pieces_in_a_graph_beside_eager_work(cuda):
     outs = [[torch.zeros_like(want) for _ in range(12)] for _ in range(2)]
     with torch.cuda.stream(side):
         G.linear(x, w, cfg=27, splits=2)   # its workspace and counters
-    G._workspace(x.device, 1 << 26)
     with torch.cuda.graph(graph):
         for o in held:
             G.linear(x, w, cfg=27, splits=2, out=o)
@@ -57,6 +56,34 @@ def test_pieces_in_a_graph_beside_eager_work(cuda):
                 G.linear(x, w, cfg=27, splits=2, out=o)
     torch.cuda.synchronize()
     assert all(torch.equal(o, want) for side_outs in outs for o in side_outs)
+
+
+def test_graphs_side_by_side_keep_their_slabs(cuda):
+    """Two graphs, captured one after the other and replayed on two streams at once: pieces of a
+    tile (cfg 27) and slabs with a second launch (cfg 0), the eager result every time."""
+    from cake_amd.ops import gemm as G
+    x = torch.randn(2, 500, 4096, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(4096, 4096, device="cuda") * 2.0 ** -6).to(torch.bfloat16)
+    plans = [(27, 2), (0, 2)] * 3
+    want = [[G.linear(x[g], w, cfg=c, splits=s) for c, s in plans] for g in range(2)]
+    outs = [[torch.zeros_like(o) for o in row] for row in want]
+    graphs, streams = [torch.cuda.CUDAGraph() for _ in range(2)], [torch.cuda.Stream() for _ in range(2)]
+    for g, graph in enumerate(graphs):
+        with torch.cuda.graph(graph):
+            for (c, s), o in zip(plans, outs[g]):
+                G.linear(x[g], w, cfg=c, splits=s, out=o)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for _ in range(4):
+            for graph, st in zip(graphs, streams):
+                with torch.cuda.stream(st):
+                    graph.replay()
+        torch.cuda.synchronize()
+        for g in range(2):
+            assert all(torch.equal(o, e) for o, e in zip(outs[g], want[g]))
+            for o in outs[g]:
+                o.zero_()
+        torch.cuda.synchronize()
 
 
 def test_counters_are_of_a_stream_or_of_a_capture(cuda):

@@ -65,3 +65,29 @@ def test_pieces_take_the_callers_counters(cfg, splits, M):
     assert call(splits, 64, 64) not in (0, invalid) and call(1, None, None) not in (0, invalid)
     assert call(splits, None, 64) == invalid and call(splits, 64, None) == invalid
     assert 0 < L.cake_gemm_ticks() <= L.cake_gemm_rows_ticks()
+
+
+def test_workspaces_are_of_a_stream_or_of_a_graph(monkeypatch):
+    """An eager launch takes its stream's slabs, of the newest 16 streams; a captured one slabs of
+    its own, which nothing but the graph keeps (graphs share PyTorch's capture stream, and may be
+    replayed side by side)."""
+    from types import SimpleNamespace
+
+    from cake_amd.ops import gemm as G
+    state = SimpleNamespace(stream=1, capturing=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: SimpleNamespace(cuda_stream=state.stream))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state.capturing)
+    monkeypatch.setattr(G, "_ws", {})
+    dev = torch.device("cpu")
+    first = G._workspace(dev, 100)
+    assert G._workspace(dev, 50) is first
+    state.capturing = True
+    a, b = G._workspace(dev, 100), G._workspace(dev, 100)
+    assert a.numel() >= 100 and len({t.data_ptr() for t in (first, a, b)}) == 3
+    state.capturing = False
+    assert G._workspace(dev, 100) is first and len(G._ws) == 1
+    grown = G._workspace(dev, first.numel() + 1)
+    assert grown is not first and list(G._ws.values()) == [grown]
+    for state.stream in range(2, 40):
+        assert G._workspace(dev, 100) is not grown
+    assert len(G._ws) == 16
