@@ -10,8 +10,8 @@
 // without registers (buffer loads with LDS destination, swizzled through their source addresses);
 // row-major values are transposed by the LDS read.  One barrier per tile.
 // 32 heads over 8, causal, us before (two waves a SIMD, values transposed through registers) and
-// after: 777 rows 35.3 / 20.6, 1100 55 / 27, 2048 93 / 52, 6000 488 / 325 (906 TFLOP/s), 8192
-// 755 / 536 (1027).
+// after: 777 rows 35.3 / 20.2, 1100 55 / 26, 2048 93 / 52, 6000 488 / 319 (923 TFLOP/s), 8192
+// 755 / 526 (1045).
 #pragma once
 #include <type_traits>
 
@@ -62,6 +62,12 @@ template <bool AG>
 __device__ __forceinline__ void fl_settle(ff32x16& o) {
   if constexpr (AG) asm volatile("s_nop 7\n\ts_nop 7" : "+a"(o));
   else asm volatile("s_nop 7\n\ts_nop 7" : "+v"(o));
+}
+
+template <bool AG>
+__device__ __forceinline__ void fl_settle(ff32x16 (&o)[4]) {
+  if constexpr (AG) asm volatile("s_nop 7\n\ts_nop 7" : "+a"(o[0]), "+a"(o[1]), "+a"(o[2]), "+a"(o[3]));
+  else asm volatile("s_nop 7\n\ts_nop 7" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
 }
 
 // two f32 -> packed 16-bit pair, one instruction for either type
@@ -123,6 +129,12 @@ __device__ __forceinline__ void fl_core(uint8_t* smem, const FlCore& a,
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nt = (a.kend + 63) / 64;
+  // Of these a wave takes the nw that some row of it sees; of the last one, with 32 rows a wave, the
+  // upper 32 keys only if some row sees them (64 rows: the branch spills).  A product with
+  // probability 0 would still carry a later key's infinite or NaN value into this row.
+  const int seen = min(a.kend - 1, a.pos + 32 * QS - 1);
+  const int nw = max(1, (seen >> 6) + 1);
+  const bool upper = (seen & 63) >= 32;
 
   // staging of [.][128] rows: instruction i of a wave fills rows 16 i + 4 wave + lane / 16, 16-byte
   // slot lane % 16.  Slot s of a key row r holds chunk s ^ (r & 15) (a fragment read takes the same
@@ -339,7 +351,7 @@ __device__ __forceinline__ void fl_core(uint8_t* smem, const FlCore& a,
       }
       __builtin_amdgcn_sched_barrier(0);
     });
-    fl_for<0, 16>([&](auto I) __attribute__((always_inline)) {
+    const auto values = [&](auto I) __attribute__((always_inline)) {
       constexpr int i = decltype(I)::value;
       if constexpr (i + PF < 16)
         vf[(i + PF) % RG] = vfrag(vb, std::integral_constant<int, i + PF>{});
@@ -355,7 +367,18 @@ __device__ __forceinline__ void fl_core(uint8_t* smem, const FlCore& a,
       if constexpr (qk && i + PF >= 16)
         kf[i + PF - 16] = kfrag(j & 1, std::integral_constant<int, i + PF - 16>{});
       __builtin_amdgcn_sched_barrier(0);
-    });
+    };
+    fl_for<0, 8>(values);
+    if constexpr (qk || QS == 2) {
+      fl_for<8, 16>(values);
+    } else {
+      // settled on either side of the branch: a register may be copied there
+      fl_settle<AG>(o[0]);
+      if (upper) {
+        fl_for<8, 16>(values);
+        fl_settle<AG>(o[0]);
+      }
+    }
 #pragma unroll
     for (int qs = 0; qs < QS; ++qs)
       l[qs] += (rq[qs][0] + rq[qs][1]) + (rq[qs][2] + rq[qs][3]);
@@ -365,22 +388,28 @@ __device__ __forceinline__ void fl_core(uint8_t* smem, const FlCore& a,
   const std::true_type more{};
   const std::false_type last{};
   int j = 0;
-  for (; j + 2 < nt; j += 2) {
+  for (; j + 2 < nw; j += 2) {
     tile(more, j, sa, sb);
     tile(more, j + 1, sb, sa);
   }
-  if (j + 1 < nt) {
+  if (j + 1 < nw) {
     tile(more, j, sa, sb);
     tile(last, j + 1, sb, sa);
   } else {
     tile(last, j, sa, sb);
   }
+  // the barriers and requests of tiles that only later rows see (vbuf: tile i's values)
+  for (int i = nw; i < nt; ++i) {
+    landed();
+    stage_k(i + 2);
+    vbuf = vbuf == 2 ? 0 : vbuf + 1;
+    stage_v(i + 1, vbuf);
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // requests of tiles that are not there
 #pragma unroll
   for (int qs = 0; qs < QS; ++qs) {
     l[qs] += __shfl_xor(l[qs], 32, 64);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) fl_settle<AG>(o[qs][t]);
+    fl_settle<AG>(o[qs]);
   }
 }
 

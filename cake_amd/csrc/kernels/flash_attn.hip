@@ -681,8 +681,8 @@ static int launch_flash(const FlashArgs& a, hipStream_t st) {
                   al(a.k, 16) && al(a.v, 16) && al(a.o, 8);
   // causal 128-wide heads: flash3.h (rows past M must lie past the last row's end, and 32-bit
   // offsets reach the tiles requested ahead).  64 query rows a wave once 256-row workgroups fill the
-  // chip one and a half times (32 heads: 2500 rows, 320 of them, 88 us against 81 with 32 rows; 3000,
-  // 384, 98 / 102; 6000 327 / 342)
+  // chip one and a half times (32 heads: 2500 rows, 320 of them, 86 us against 83 with 32 rows; 3000,
+  // 384, 96 / 104; 6000 318 / 328; 64 heads, 384 of them: 1300 rows 56 / 52, 1490 57 / 59)
   const auto fits = [&](long long sn) {
     return sn >= 128 && (a.M * sn + 128) * 2 < 0x7fffffffLL && (a.M + 256LL) * sn * 2 < 0xffffffffLL;
   };

@@ -134,3 +134,61 @@ def test_latent(dt, H, seqs):
             w = _want(qq.to(dt), kk, vt[h * 128:h * 128 + 128, k0:k0 + p0 + n].t(), p0, 0.08)
             for out in outs:
                 _close(out[r0:r0 + n, h * 128:h * 128 + 128], w, dt)
+
+
+def _first_touched(n, p0, p, rows):
+    """First of n rows at positions p0.. that a value of probability 0 at key p may reach: of the
+    first wave (`rows` rows) that takes the key's run of `rows` keys."""
+    return next(r for r in range(0, n, rows) if p // rows * rows <= p0 + r + rows - 1)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=str)
+@pytest.mark.parametrize("H,Hkv,N,pos0,p,rows", [
+    (2, 1, 300, 0, 96, 32), (2, 1, 300, 0, 127, 32), (2, 2, 300, 13, 201, 32), (2, 1, 129, 0, 128, 32),
+    (192, 8, 300, 0, 192, 64), (192, 8, 300, 64, 290, 64)])
+def test_non_finite_values_stay_behind_prefill(dt, H, Hkv, N, pos0, p, rows):
+    """A row before an infinite or NaN value does not see it, save in the wave that takes its keys."""
+    g = torch.Generator().manual_seed(p)
+    q, k, v = (torch.randn(1, h, n, 128, generator=g).to(dt).cuda()
+               for h, n in ((H, N), (Hkv, pos0 + N), (Hkv, pos0 + N)))
+    clean, got = torch.empty_like(q), torch.empty_like(q)
+    K.flash_attn(q, k, v, clean, 0.1, causal=True, pos0=pos0)
+    for bad in (float("inf"), float("nan")):
+        v[:, :, p] = bad
+        K.flash_attn(q, k, v, got, 0.1, causal=True, pos0=pos0)
+        first = _first_touched(N, pos0, p, rows)
+        assert 0 < first < N
+        assert torch.equal(got[:, :, :first], clean[:, :, :first])
+        assert not bool(torch.isfinite(got[:, :, p - pos0:]).any())   # those that do see it
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=str)
+@pytest.mark.parametrize("p0,n,p", [(0, 300, 96), (0, 300, 130), (45, 129, 150)])
+def test_non_finite_values_stay_behind_hybrid(dt, p0, n, p):
+    """The same of the hybrid designs' form and the latent one; and values past a sequence's last run
+    of 32 keys (what an earlier sequence left in the slot) reach no row."""
+    sh, S = M.AttnShape(2, 1, 128, 128), 448
+    lat = L.LatentShape(2, 128, 64, 128, 96, 64, 30)
+    rows = M.Rows.pack([(0, p0, [0] * n)], "cuda")
+    g = torch.Generator().manual_seed(p)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(dt).cuda()
+    qn, kc, vc = rnd(n, 2, 128), rnd(1, 1, S, 128), rnd(1, 1, 128, S)
+    cache, lk, vt = rnd(1, S, lat.LD), rnd(rows.n_keys, 256), rnd(256, rows.n_keys)
+    lq, cs = rnd(n, 2 * 192), torch.rand(S, 60, generator=g).cuda()
+
+    def both():
+        a = torch.empty(n, 256, device="cuda", dtype=dt)
+        b = torch.empty_like(a)
+        M.attn_prompt(sh, qn, kc, vc, rows, None, a, 0.1, True)
+        L.prompt(lat, lq, lk, vt, rows, cs, cache, b, 0.08)
+        return torch.stack([a, b])
+    end = -(-(p0 + n) // 32) * 32
+    vc[..., end:], vt[:, end:] = float("nan"), float("nan")
+    clean = both()
+    assert bool(torch.isfinite(clean).all())
+    vc[..., p], vt[:, p] = float("inf"), float("nan")
+    got, first = both(), _first_touched(n, p0, p, 32)
+    assert first > 0 and torch.equal(got[:, :first], clean[:, :first])
+    assert not bool(torch.isfinite(got[:, p - p0:]).any())
