@@ -30,6 +30,7 @@ from __future__ import annotations
 import argparse
 import concurrent.futures as cf
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -59,10 +60,11 @@ def _newer(src: Path, deps: list[Path], out: Path) -> bool:
     return any(p.stat().st_mtime > t for p in [src, *deps] if p.exists())
 
 
-def _run(cmd: list[str]) -> None:
+def _run(cmd: list[str]) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"command failed ({r.returncode}): {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    return r.stderr
 
 
 # packed FP32 math stays off in every HIP object: some v_pk_*_f32 forms the compiler picks by
@@ -72,6 +74,26 @@ def _run(cmd: list[str]) -> None:
 # closures in scratch memory)
 NO_PK_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 HIP_EXTRA = {"gemm": ["-mllvm", "-inline-threshold=100000"]}  # gemm.hip and gemm_inst_*.hip
+# file -> kernels whose matrix instructions are written out in asm (csrc/kernels/flash3.h): the
+# compiler stores a spilled result without the wait states that it takes, so a spill ends the build
+NO_SPILL = {"flash_attn": "flash3_fwd_kernel", "mixer_attn": "mixer_flash3_kernel",
+            "mixer_latent": "mixer_flash3_kernel"}
+
+
+def check_spills(remarks: str, kernel: str) -> None:
+    """Raise if an instance of `kernel` uses scratch memory, by the compiler's resource remarks."""
+    name, seen = "", 0
+    for line in remarks.splitlines():
+        m = re.search(r"(Function Name|ScratchSize \[bytes/lane\]|[SV]GPRs Spill): (\S+)", line)
+        if m is None:
+            continue
+        if m.group(1) == "Function Name":
+            name = m.group(2)
+            seen += kernel in name
+        elif kernel in name and m.group(2) != "0":
+            raise RuntimeError(f"{name}: {m.group(1)} {m.group(2)}; its asm products allow none")
+    if not seen:
+        raise RuntimeError(f"no resource remarks of {kernel}")
 
 
 def _compile_hip(src: Path, force: bool) -> Path:
@@ -79,10 +101,18 @@ def _compile_hip(src: Path, force: bool) -> Path:
     out.parent.mkdir(parents=True, exist_ok=True)
     headers = sorted((CSRC / "kernels").glob("*.h"))
     if force or _newer(src, headers, out):
-        _run([HIPCC, "-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC",
-              "-Wno-unused-result", "-munsafe-fp-atomics", *NO_PK_FP32,
-              *HIP_EXTRA.get(src.stem.split("_")[0], []),
-              "-c", str(src), "-o", str(out)])
+        checked = NO_SPILL.get(src.stem)
+        remarks = _run([HIPCC, "-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC",
+                        "-Wno-unused-result", "-munsafe-fp-atomics", *NO_PK_FP32,
+                        *HIP_EXTRA.get(src.stem.split("_")[0], []),
+                        *(["-Rpass-analysis=kernel-resource-usage"] if checked else []),
+                        "-c", str(src), "-o", str(out)])
+        if checked:
+            try:
+                check_spills(remarks, checked)
+            except RuntimeError:
+                out.unlink()
+                raise
     return out
 
 

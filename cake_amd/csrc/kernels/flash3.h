@@ -27,7 +27,8 @@ typedef float ff32x16 __attribute__((ext_vector_type(16)));
 // them) and the output accumulators and queries in AGPRs.  What the compiler does not see then:
 // 11 wait states before a VALU instruction reads a result (the products of another phase always
 // lie between, or fl_settle), 2 before a product reads what a VALU instruction wrote (fl_mma_o's
-// s_nop).  A register spilled beside them would be read too early: no instance may spill.
+// s_nop).  A register spilled beside them would be read too early: no instance may spill (build.py
+// checks the compiler's remarks of each).
 template <int DT>
 __device__ __forceinline__ void fl_mma_s0(ff32x16& s, const uint4& k, const fu32x4& q) {
   const fu32x4 kv = __builtin_bit_cast(fu32x4, k);
