@@ -213,15 +213,12 @@ def _near_splits(splits: int, m_near: int, M: int) -> int:
     return p
 
 
-def _tuned(M: int, Nv: int, K: int, epi: str, mfma_only: bool = False):
+def _tuned(M: int, Nv: int, K: int, epi: str):
     """Exact measured shape, else the same (Nv, K, epilogue) measured at the nearest M
-    within 2x (its tile config, split-K scaled to this M).  mfma_only skips the library
-    GEMM's entries."""
+    within 2x (its tile config, split-K scaled to this M)."""
     near = None
     for e in _TUNED:
         if e["Nv"] != Nv or e["K"] != K or e["epi"] != epi:
-            continue
-        if mfma_only and e["cfg"] == LIB:
             continue
         if e["M"] == M:
             return e["cfg"], e["splits"]
@@ -232,13 +229,6 @@ def _tuned(M: int, Nv: int, K: int, epi: str, mfma_only: bool = False):
         return None
     e = near[1]
     return e["cfg"], (1 if e["cfg"] == LIB else _near_splits(e["splits"], e["M"], M))
-
-
-def plan_mfma(M: int, Nv: int, K: int, epi: str = "store") -> tuple[int, int]:
-    """The MFMA kernel's (cfg, splits) for a shape: its measured entries, else the cost
-    model (the library GEMM's entries ignored)."""
-    p = _tuned(M, Nv, K, epi, mfma_only=True)
-    return p if p is not None else _cost_plan(M, Nv, K)
 
 
 def set_plan(M: int, N: int, K: int, epi: str, cfg: int, splits: int) -> None:
@@ -256,20 +246,22 @@ def plan(M: int, Nv: int, K: int, epi: str = "store") -> tuple[int, int]:
     return p if p is not None else _cost_plan(M, Nv, K)
 
 
-def resolve(M: int, Nv: int, K: int, epi: str, big: bool) -> tuple[int, int]:
+def resolve(M: int, Nv: int, K: int, epi: str, big: bool = False,
+            mfma_only: bool = False) -> tuple[int, int]:
     """(cfg, splits) that :func:`linear` runs: a pinned plan, the measured one of this very size
     unless the kernel library's estimate puts it well behind, else the estimate's best
-    (gemm.hip cake_gemm_plan, shared with the native engines)."""
+    (gemm.hip cake_gemm_plan, shared with the native engines).  big: an operand of 2 GB or more;
+    mfma_only: as if no plan named the library GEMM."""
     p = _plans.get((M, Nv, K, epi))
-    if p is not None:
+    if p is not None and not (mfma_only and p[0] == LIB):
         return p
-    key = (M, Nv, K, epi, big)
+    key = (M, Nv, K, epi, big, mfma_only)
     p = _resolved.get(key)
     if p is None:
         if len(_resolved) >= 65536:   # as many sizes as a long-lived server meets
             _resolved.clear()
         e = next((e for e in _TUNED if e["M"] == M and e["Nv"] == Nv and e["K"] == K
-                  and e["epi"] == epi), None)
+                  and e["epi"] == epi and not (mfma_only and e["cfg"] == LIB)), None)
         cfg, sp = C.c_int(-1 if e is None else e["cfg"]), C.c_int(1 if e is None else e["splits"])
         if cfg.value == LIB and e is not None:
             p = (LIB, 1)
@@ -420,8 +412,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
                 _zeros16(x.device).data_ptr(), M, N, K, float(alpha), st), "gemm_rows")
             return resid if f32_out else out
     s0 = 1
+    big = max((M - 1) * lda + K, (Nv - 1) * ldb + K) * 2 >= 0x7fffffff
     if cfg is None:
-        big = max((M - 1) * lda + K, (Nv - 1) * ldb + K) * 2 >= 0x7fffffff
         cfg, s0 = resolve(M, Nv, K, epi, big)
     elif splits is None:
         s0 = plan(M, Nv, K, epi)[1]
@@ -430,7 +422,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
         _lib_gemm(x2, lda, w, ldb, epi, out2, ldc, r2 if f32_out else None, ldr, M, N, K)
         return resid if f32_out else out
     if cfg == LIB:  # an epilogue / bias / strided output the library form does not carry
-        cfg, s0 = plan_mfma(M, Nv, K, epi)
+        cfg, s0 = resolve(M, Nv, K, epi, big, mfma_only=True)
     splits = s0 if splits is None else max(1, int(splits))
     # the kernel library sizes it (pieces of a tile need their slabs only)
     st = torch.cuda.current_stream().cuda_stream

@@ -61,7 +61,7 @@ def main():
             for M in [int(m) for m in a.ms.split(",")]:
                 x = (torch.randn(M, K, device="cuda") * 0.5).bfloat16()
                 r0 = torch.randn(M, N, device="cuda") if epi in ("resid32", "store32") else None
-                cfg, spl = G.plan_mfma(M, Nv, K, epi)
+                cfg, spl = G.resolve(M, Nv, K, epi, mfma_only=True)
                 outs = {}
 
                 def run(kind):

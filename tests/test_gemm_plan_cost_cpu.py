@@ -41,6 +41,24 @@ def test_measured_entry_of_the_size_stands_unless_well_behind(monkeypatch):
     assert at(20, 1) == (20, 1)     # a tile the estimate does not cover
 
 
+def test_library_plan_falls_back_to_the_plan_without_it(monkeypatch):
+    """A call that the library form does not carry (a bias) runs what a table without the library's
+    entries plans, as the native engines do, not the nearest measured size."""
+    from cake_amd.ops import gemm as G
+    near = {"M": 1000, "Nv": 4096, "K": 4096, "epi": "store", "cfg": 13, "splits": 4}
+    lib = {**near, "M": 1100, "cfg": G.LIB, "splits": 1}
+    monkeypatch.setattr(G, "_TUNED", [near])
+    monkeypatch.setattr(G, "_resolved", {})
+    want = G.resolve(1100, 4096, 4096, "store")
+    assert want[0] != 13
+    monkeypatch.setattr(G, "_TUNED", [near, lib])
+    monkeypatch.setattr(G, "_resolved", {})
+    assert G.resolve(1100, 4096, 4096, "store") == (G.LIB, 1)
+    assert G.resolve(1100, 4096, 4096, "store", mfma_only=True) == want
+    monkeypatch.setattr(G, "_plans", {(1100, 4096, 4096, "store"): (G.LIB, 1)})
+    assert G.resolve(1100, 4096, 4096, "store", mfma_only=True) == want
+
+
 def test_workspace_covers_the_pieces():
     """Tiles in pieces need a slab each; whole tiles need none."""
     from cake_amd.ops import gemm as G

@@ -120,7 +120,9 @@ def test_nearest_measured_plan_scales_split_k(monkeypatch):
     assert G.plan(40, 4096, 14336, "resid32") == (13, 2)
     assert G.plan(20, 4096, 14336, "resid32") == (13, 4)   # 6.4 -> 4
     assert G.plan(1500, 4096, 14336, "resid32") == (G.LIB, 1)
-    assert G.plan_mfma(1500, 4096, 14336, "resid32")[0] in G.CFG_TILES
+    monkeypatch.setattr(G, "_resolved", {})
+    assert G.resolve(1024, 4096, 14336, "resid32") == (G.LIB, 1)
+    assert G.resolve(1024, 4096, 14336, "resid32", mfma_only=True)[0] in G.CFG_TILES
     eng = (ROOT / "cake_amd/csrc/engine/engine_util.h").read_text()
     assert "near->splits * near->M / std::max(M, 1LL)" in eng
 
