@@ -86,7 +86,7 @@ inline std::string read_file(const std::string& path) {
 }
 
 // ---------------------------------------------------------------------------
-// GEMM tile plan (ops/gemm.py plan(): measured table, else the cost model)
+// GEMM tile plan (ops/gemm.py resolve(): measured table, else the kernel library's estimate)
 // ---------------------------------------------------------------------------
 // plan cfg naming the library GEMM (hipBLASLt, driver/blaslt.cpp; ops/gemm.py LIB).
 // Off the default path: table entries naming it are read only under CAKE_GEMM_LIB=1
@@ -132,7 +132,8 @@ struct GemmPlanner {
   }
 
   // the plan that runs (ops/gemm.py resolve): the measured entry of this very size unless the
-  // kernel library's estimate puts it well behind, else the estimate's best; epi_id: its epilogue id
+  // kernel library's estimate puts it well behind, else the estimate's best; epi_id: its epilogue id;
+  // mfma_only: as if no plan named the library GEMM
   std::pair<int, int> resolve(long long M, long long Nv, long long K, const std::string& epi, int epi_id,
                               bool big, bool mfma_only = false) const {
     int cfg = -1, splits = 1;
@@ -145,60 +146,6 @@ struct GemmPlanner {
     if (cfg == kGemmLib && has_lib()) return {kGemmLib, 1};
     cake_gemm_plan((int)M, Nv, (int)K, epi_id, big ? 1 : 0, &cfg, &splits);
     return {cfg, splits};
-  }
-
-  // the MFMA kernel's plan: the measured entries other than the library GEMM's
-  std::pair<int, int> plan_mfma(long long M, long long Nv, long long K,
-                                const std::string& epi) const {
-    return plan(M, Nv, K, epi, true);
-  }
-
-  std::pair<int, int> plan(long long M, long long Nv, long long K, const std::string& epi,
-                           bool mfma_only = false) const {
-    const Tuned* near = nullptr;
-    double near_r = 0;
-    for (const auto& e : tuned) {
-      if (e.Nv != Nv || e.K != K || e.epi != epi) continue;
-      if (mfma_only && e.cfg == kGemmLib) continue;
-      if (e.M == M) return {e.cfg, e.splits};
-      const double r = (double)std::max(M, e.M) / (double)std::min(M, e.M);
-      if (r <= 2 && (!near || r < near_r)) { near = &e; near_r = r; }
-    }
-    if (near) {  // split-K scaled to this M (ops/gemm.py _near_splits)
-      if (near->cfg == kGemmLib) return {kGemmLib, 1};
-      long long sc = (long long)near->splits * near->M / std::max(M, 1LL);
-      int p = 1;
-      while ((long long)p * 2 <= sc) p *= 2;
-      return {near->cfg, p};
-    }
-    struct T { int cfg, bm, bn, slots; double eff; };
-    static const T tiles[] = {{0, 128, 128, 2, 1.0}, {1, 64, 128, 2, 0.8}, {4, 64, 64, 4, 0.7},
-                              {5, 256, 256, 1, 1.2}, {22, 256, 256, 1, 1.3}};
-    static const int small_c[] = {1, 4, 0}, big_c[] = {0, 1, 4, 5, 22};
-    const int* cands = M <= 64 ? small_c : big_c;
-    // the four-wave 256x256 tile (cfg 22) where it can run: whole 64-element k steps,
-    // operands under 2 GB (ops/gemm.py _cost_plan); unsplit
-    const bool four = M > 64 && K % 64 == 0 && M * K * 2 < (1LL << 31) && Nv * K * 2 < (1LL << 31);
-    const int nc = M <= 64 ? 3 : (four ? 5 : 4);
-    const long long ksteps = (K + 63) / 64;
-    double best = -1;
-    std::pair<int, int> out{0, 1};
-    for (int c = 0; c < nc; ++c) {
-      const T* t = nullptr;
-      for (const auto& x : tiles)
-        if (x.cfg == cands[c]) t = &x;
-      const long long tiles_n = ((M + t->bm - 1) / t->bm) * ((Nv + t->bn - 1) / t->bn);
-      for (int splits : {1, 2, 4, 8, 16}) {
-        if (splits > 1 && (t->cfg == 22 || ksteps / splits < 4 ||
-                           tiles_n * splits > 2LL * 256 * t->slots))
-          continue;
-        const long long waves = (tiles_n * splits + 256LL * t->slots - 1) / (256LL * t->slots);
-        double cost = (double)waves * t->slots * t->bm * t->bn * (double)((ksteps + splits - 1) / splits) / t->eff;
-        if (splits > 1) cost += (double)M * Nv * splits * 0.1;
-        if (best < 0 || cost < best) { best = cost; out = {t->cfg, splits}; }
-      }
-    }
-    return out;
   }
 };
 

@@ -1,5 +1,6 @@
-"""Causal flash attention (Llama prefill shapes) with and without q-tile pairing:
-µs per call and TFLOP/s (causal FLOPs), graph of back-to-back launches."""
+"""Causal flash attention (Llama prefill shapes) of the two-waves-a-SIMD kernel with and without
+q-tile pairing, beside what runs by itself ("auto": of 128-wide heads the core of flash3.h): µs per
+call and TFLOP/s (causal FLOPs), graph of back-to-back launches."""
 import json
 import math
 import os
@@ -23,7 +24,7 @@ def main():
         out = torch.empty(1, N, H, D, device=dev, dtype=dt).transpose(1, 2)
         rec = {"H": H, "D": D, "N": N}
         flops = 4.0 * N * N * D * H / 2
-        for name, pm, nw in (("unpaired", 0, 0), ("paired", 1, 0), ("nw2", 0, 2),
+        for name, pm, nw in (("unpaired", 0, 4), ("paired", 1, 4), ("nw2", 0, 2),
                              ("nw2_paired", 1, 2), ("auto", 512, 0)):
             K.flash_set_pair_min(pm)
             K.kernels().cake_flash_set_nw(nw)

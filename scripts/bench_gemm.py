@@ -97,7 +97,7 @@ def main():
             t_ours = to if t_ours is None else min(t_ours, to)
             t_lib = tl if t_lib is None else min(t_lib, tl)
             t_mm = tm if t_mm is None else min(t_mm, tm)
-        rec = {"shape": name, "M": M, "N": N, "K": K, "epi": epi, "plan": G.plan(M, Nw, K, epi),
+        rec = {"shape": name, "M": M, "N": N, "K": K, "epi": epi, "plan": G.resolve(M, Nw, K, epi),
                "ours_ms": round(t_ours, 4), "torch_fused_ms": round(t_lib, 4),
                "hipblaslt_gemm_ms": round(t_mm, 4),
                "ours_tflops": round(flops / t_ours / 1e9, 1),

@@ -43,16 +43,16 @@ def record_shapes(version, dt):
         unet.forward(w, x, tbuf, ctx, kv)  # first call: cross-attention k/v cache filled
         torch.cuda.synchronize()
         seen = collections.Counter()
-        orig = G.plan
+        orig = G.resolve
 
-        def spy(M, Nv, K, epi="store"):
+        def spy(M, Nv, K, epi, *a, **kw):
             seen[(M, Nv, K, epi)] += 1
-            return orig(M, Nv, K, epi)
-        G.plan = spy
+            return orig(M, Nv, K, epi, *a, **kw)
+        G.resolve = spy   # (products of few rows have forms of their own and no plan)
         try:
             unet.forward(w, x, tbuf, ctx, kv)
         finally:
-            G.plan = orig
+            G.resolve = orig
         torch.cuda.synchronize()
     del w, unet
     torch.cuda.empty_cache()
@@ -94,7 +94,7 @@ def tune(M, Nv, K, epi, dt, cfgs=None):
 
     def run(cfg, splits):
         return G.linear(x, w, b, epi=epi, resid=r, cfg=cfg, splits=splits)
-    cur = G.plan(M, Nv, K, epi)
+    cur = G.resolve(M, Nv, K, epi)
     res = {}
     for cfg, (bm, bn) in G.CFG_TILES.items():
         if gated and cfg in getattr(G, "NO_GATED", ()):
@@ -107,10 +107,9 @@ def tune(M, Nv, K, epi, dt, cfgs=None):
             continue
         tiles = -(-M // bm) * -(-Nv // bn)
         for splits in (1, 2, 4):
-            # four-wave tiles at splits 2 pair only the tiles past the last whole wave (the
-            # in-kernel pair, gemm.hip), whatever the tile count
-            pair = cfg in getattr(G, "K64_ONLY", ()) and cfg >= 22 and splits == 2
-            if splits > 1 and not pair and (tiles * splits > 2 * G.NUM_CUS or K // splits < 256):
+            # four-wave tiles split only the tiles past the last whole wave (in pieces, gemm.hip),
+            # whatever the tile count
+            if splits > 1 and cfg not in G.FOUR_WAVE and (tiles * splits > 2 * G.NUM_CUS or K // splits < 256):
                 continue
             try:
                 run(cfg, splits)

@@ -1,8 +1,8 @@
 """GEMM tile plans on the CPU: the measured table (ops/gemm_tuned.json) and the three places
 that name the tile configurations — the kernel table (csrc/kernels/gemm_kernel.h
 CAKE_GEMM_CFGS), the Python planner (ops/gemm.py CFG_TILES) and the native engine's planner
-(csrc/engine/engine_util.h, shared by the Llama and SD engines) — must agree, or a tuned plan launches a tile the library
-does not have."""
+(csrc/engine/engine_util.h, shared by the Llama and SD engines) — must agree, or a tuned plan
+launches a tile the library does not have."""
 import json
 import re
 from pathlib import Path
@@ -74,6 +74,9 @@ def test_plan_uses_measured_entries():
     table = json.loads((ROOT / "cake_amd/ops/gemm_tuned.json").read_text())["entries"]
     # (entries naming the library GEMM are read only under CAKE_GEMM_LIB=1)
     e = next(x for x in table if x["M"] >= 512 and x["cfg"] != G.LIB)
+    # the plan that runs: the entry, unless the estimate puts it well behind
+    assert G.resolve(e["M"], e["Nv"], e["K"], e["epi"])[0] in G.CFG_TILES
+    # the split of a call that names its tile
     assert G.plan(e["M"], e["Nv"], e["K"], e["epi"]) == (e["cfg"], e["splits"])
     # a nearby M (within 2x) reuses the measured tile without split-K
     cfg, splits = G.plan(e["M"] + 8, e["Nv"], e["K"], e["epi"])
@@ -96,21 +99,26 @@ def test_library_gemm_is_off_the_default_path(monkeypatch):
     assert set(re.findall(r'ep == "(\w+)"', body)) == set(G.LIB_EPIS)
     monkeypatch.setattr(G, "_plans", {})
     assert all(e["cfg"] != G.LIB for e in G._TUNED)
-    assert G.plan(2048, 28672, 4096, "swiglu")[0] in G.CFG_TILES   # 8B gate|up, 2048 tokens
-    assert G.plan(2048, 6144, 4096, "store")[0] in G.CFG_TILES     # 8B q|k|v
-    assert G.plan(2048, 1280, 5120, "add16")[0] in G.CFG_TILES     # SD shapes
+    monkeypatch.setattr(G, "_resolved", {})
+    for plan in (G.plan, G.resolve):
+        assert plan(2048, 28672, 4096, "swiglu")[0] in G.CFG_TILES   # 8B gate|up, 2048 tokens
+        assert plan(2048, 6144, 4096, "store")[0] in G.CFG_TILES     # 8B q|k|v
+        assert plan(2048, 1280, 5120, "add16")[0] in G.CFG_TILES     # SD shapes
     monkeypatch.setenv("CAKE_GEMM_LIB", "1")
     lib_table = G._load_tuned()
     assert any(e["cfg"] == G.LIB for e in lib_table)
     monkeypatch.setattr(G, "_TUNED", lib_table)
     monkeypatch.setattr(G, "_plans", {})
+    monkeypatch.setattr(G, "_resolved", {})
     assert G.plan(2048, 28672, 4096, "swiglu")[0] == G.LIB
+    assert any(G.resolve(e["M"], e["Nv"], e["K"], e["epi"]) == (G.LIB, 1) for e in lib_table
+               if e["cfg"] == G.LIB)
 
 
 def test_nearest_measured_plan_scales_split_k(monkeypatch):
-    """A shape measured at M with split-K s, asked at M' within 2x: the same tile with
-    s * M / M' splits (a power of two >= 1) — the grid fill the split was chosen for —
-    and a library entry stays a library plan; the engine planner applies the same rule."""
+    """Split of a call that names its tile.  A shape measured at M with split-K s, asked at M'
+    within 2x: the same tile with s * M / M' splits (a power of two >= 1) — the grid fill the
+    split was chosen for — and a library entry stays a library plan."""
     monkeypatch.setattr(G, "_TUNED", [
         {"M": 32, "Nv": 4096, "K": 14336, "epi": "resid32", "cfg": 13, "splits": 4},
         {"M": 1024, "Nv": 4096, "K": 14336, "epi": "resid32", "cfg": G.LIB, "splits": 1}])
@@ -123,8 +131,6 @@ def test_nearest_measured_plan_scales_split_k(monkeypatch):
     monkeypatch.setattr(G, "_resolved", {})
     assert G.resolve(1024, 4096, 14336, "resid32") == (G.LIB, 1)
     assert G.resolve(1024, 4096, 14336, "resid32", mfma_only=True)[0] in G.CFG_TILES
-    eng = (ROOT / "cake_amd/csrc/engine/engine_util.h").read_text()
-    assert "near->splits * near->M / std::max(M, 1LL)" in eng
 
 
 def test_kernel_library_exports_the_library_gemm():
