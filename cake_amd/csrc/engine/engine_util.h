@@ -139,11 +139,11 @@ struct GemmPlanner {
     int cfg = -1, splits = 1;
     for (const auto& e : tuned)
       if (e.M == M && e.Nv == Nv && e.K == K && e.epi == epi && !(mfma_only && e.cfg == kGemmLib)) {
+        if (e.cfg == kGemmLib) return {kGemmLib, 1};
         cfg = e.cfg;
         splits = e.splits;
         break;
       }
-    if (cfg == kGemmLib && has_lib()) return {kGemmLib, 1};
     cake_gemm_plan((int)M, Nv, (int)K, epi_id, big ? 1 : 0, &cfg, &splits);
     return {cfg, splits};
   }
