@@ -126,16 +126,18 @@ def _workspace(dev, numel: int) -> torch.Tensor:
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(numel, dtype=torch.float32, device=dev)
     key = (dev, torch.cuda.current_stream(dev).cuda_stream)
-    with _lock:
-        w = _ws.get(key)
-        if w is None or w.numel() < numel:
-            w = torch.empty(max(numel, 1 << 20), dtype=torch.float32, device=dev)
-        _newest(_ws, key, w)
+    w = _ws.get(key)
+    if w is None or w.numel() < numel or len(_ws) >= 16:
+        with _lock:
+            if w is None or w.numel() < numel:
+                w = torch.empty(max(numel, 1 << 20), dtype=torch.float32, device=dev)
+            _newest(_ws, key, w)
     return w
 
 
 ROWS_MAX = 64   # rows that the products of few rows take at most
 _rows_kinds: dict = {}
+_rows_floats: dict = {}   # rows -> workspace floats of the stream form
 
 
 def rows_kind(M: int, Nv: int, K: int, gated: bool) -> int:
@@ -154,23 +156,28 @@ def _counters(dev, st: int) -> torch.Tensor:
     Launches of one stream run one after the other and share them; launches that may run side by
     side never do.  A captured graph may run beside any stream, so its counters are its own: memory
     of its pool, cleared by a fill at the head of every replay, as long-lived as the graph."""
-    key = (dev, st)
-    lib = _lib()
+    if not torch.cuda.is_current_stream_capturing():
+        return _stream_counters(dev, st)
+    capture = _lib().cake_stream_capture(st)
+    if capture <= 0:
+        raise RuntimeError("gemm: the capture of the current stream is not to be told")
     with _lock:
-        if torch.cuda.is_current_stream_capturing():
-            capture = lib.cake_stream_capture(st)
-            if capture <= 0:
-                raise RuntimeError("gemm: the capture of the current stream is not to be told")
-            have = _graph_ticks.get(key)
-            if have is None or have[0] != capture:
-                have = (capture, torch.zeros(_n_ticks(), dtype=torch.int32, device=dev))
-                _newest(_graph_ticks, key, have)
-            return have[1]
-        t = _ticks.get(key)
-        if t is None:
-            t = torch.zeros(_n_ticks(), dtype=torch.int32, device=dev)
-        _newest(_ticks, key, t)
-        return t
+        have = _graph_ticks.get((dev, st))
+        if have is None or have[0] != capture:
+            have = (capture, torch.zeros(_n_ticks(), dtype=torch.int32, device=dev))
+            _newest(_graph_ticks, (dev, st), have)
+        return have[1]
+
+
+def _stream_counters(dev, st: int) -> torch.Tensor:
+    """:func:`_counters` outside of captures."""
+    t = _ticks.get((dev, st))
+    if t is None or len(_ticks) >= 16:
+        with _lock:
+            if t is None:
+                t = torch.zeros(_n_ticks(), dtype=torch.int32, device=dev)
+            _newest(_ticks, (dev, st), t)
+    return t
 
 
 def _n_ticks() -> int:
@@ -178,9 +185,11 @@ def _n_ticks() -> int:
 
 
 def _rows_state(dev, M: int, st: int):
-    """(workspace, counters) of one launch of the stream form."""
-    return torch.empty(int(_lib().cake_gemm_rows_ws_floats(M)), dtype=torch.float32,
-                       device=dev), _counters(dev, st)
+    """(workspace, counters) of one launch of the stream form, which graphs do not hold."""
+    n = _rows_floats.get(M)
+    if n is None:
+        n = _rows_floats[M] = int(_lib().cake_gemm_rows_ws_floats(M))
+    return torch.empty(n, dtype=torch.float32, device=dev), _stream_counters(dev, st)
 
 
 def _load_tuned() -> list:

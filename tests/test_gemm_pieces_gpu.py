@@ -86,10 +86,11 @@ def test_graphs_side_by_side_keep_their_slabs(cuda):
         torch.cuda.synchronize()
 
 
-def test_counters_are_of_a_stream_or_of_a_capture(cuda):
+def test_counters_are_of_a_stream_or_of_a_capture(cuda, monkeypatch):
     """Launches that may run side by side never share counters, however many there were; a stream's
     stay its own and zero; the newest 16 streams keep theirs."""
     from cake_amd.ops import gemm as G
+    monkeypatch.setattr(G, "_ticks", {})
     dev = torch.empty(1, device="cuda").device
 
     def here():
