@@ -192,3 +192,44 @@ def test_non_finite_values_stay_behind_hybrid(dt, p0, n, p):
     got, first = both(), _first_touched(n, p0, p, 32)
     assert first > 0 and torch.equal(got[:, :first], clean[:, :first])
     assert not bool(torch.isfinite(got[:, p - p0:]).any())
+
+
+@pytest.mark.parametrize("sn", [64, 1 << 22])
+def test_prefill_rows_outside_the_cores_offsets(sn):
+    """Key and value rows that overlap, or lie 2 GB apart in all: the general kernel, as ever."""
+    n, dt = 300, torch.bfloat16
+    buf = torch.zeros((n - 1) * sn + 512, device="cuda", dtype=dt)
+    rows = buf.as_strided((n, 512), (sn, 1))
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for r in range(n) if sn < 512 else [slice(None)]:
+        rows[r] = torch.randn(rows[r].shape, device="cuda", generator=g).to(dt)
+    k, v = (rows[:, c:c + 256].unflatten(1, (2, 128)).permute(1, 0, 2)[None] for c in (0, 256))
+    q = torch.randn(1, 4, n, 128, device="cuda", generator=g).to(dt)
+    out = torch.empty_like(q)
+    K.flash_attn(q, k, v, out, 0.1, causal=True)
+    for h in range(4):
+        _close(out[0, h].cpu(), _want(q[0, h].cpu(), k[0, h // 2].cpu(), v[0, h // 2].cpu(), 0, 0.1), dt)
+
+
+def test_ragged_caches_outside_the_cores_offsets():
+    """A sequence's keys or values of 2 GB, in the hybrid designs' form and the latent one."""
+    n, dt, S = 200, torch.bfloat16, 1 << 23
+    rows = M.Rows.pack([(0, 0, [0] * n)], "cuda")
+    g = torch.Generator(device="cuda").manual_seed(4)
+
+    def rnd(*s):
+        return torch.randn(*s, device="cuda", generator=g).to(dt)
+    kc, vc = (torch.zeros(1, 1, *d, device="cuda", dtype=dt) for d in ((S, 128), (128, S)))
+    kc[0, 0, :n], vc[0, 0, :, :n], qn = rnd(n, 128), rnd(128, n), rnd(n, 1, 128)
+    out = torch.empty(n, 128, device="cuda", dtype=dt)
+    M.attn_prompt(M.AttnShape(1, 1, 128, 128), qn, kc, vc, rows, None, out, 0.1, True)
+    _close(out.cpu(), _want(qn[:, 0].cpu(), kc[0, 0, :n].cpu(), vc[0, 0, :, :n].t().cpu(), 0, 0.1, True),
+           dt)
+    del kc, vc
+    lat = L.LatentShape(1, 128, 64, 128, 96, 64, 30)
+    cs = torch.tensor([1.0, 0.0], device="cuda").repeat(256, 30)   # no rotation
+    vt = torch.zeros(128, (1 << 23) + 69632, device="cuda", dtype=dt)
+    vt[:, :n], lk, q, cache = rnd(128, n), rnd(rows.n_keys, 128), rnd(n, 192), rnd(1, 256, lat.LD)
+    L.prompt(lat, q, lk, vt, rows, cs, cache, out, 0.08)
+    kk = torch.cat([lk[:n], cache[0, :n, lat.RP:lat.RP + 64]], 1).cpu()
+    _close(out.cpu(), _want(q.cpu(), kk, vt[:, :n].t().cpu(), 0, 0.08), dt)
