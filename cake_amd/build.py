@@ -1,7 +1,7 @@
 """Native build driver: HIP kernels (gfx950) and the C++ host runtime.
 
 Everything is compiled in-tree into ``cake_amd/lib/`` so the shared objects
-travel with the repository snapshot to the GPU box:
+travel with a copy of the repository:
 
 * ``libcake_gemm.so`` (``csrc/kernels/gemm*.hip``), ``libcake_mixers.so``
   (``csrc/kernels/mixer_*.hip``: the hybrid designs' layers) and
@@ -177,7 +177,7 @@ def build_kernels(force: bool = False, jobs: int = 8,
             "-Wl,-rpath,$ORIGIN"]
         if force or stale or any(_newer(o, [], lib) for o in mine):
             # --no-undefined: a kernel whose host stub the compiler dropped fails here, not at
-            # dlopen on the GPU box
+            # dlopen on a machine with a GPU
             tmp = lib.with_suffix(f".tmp{os.getpid()}")
             _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, mine),
                   "-o", str(tmp), f"-Wl,-soname,{lib.name}", *extra, "-Wl,--no-undefined"])

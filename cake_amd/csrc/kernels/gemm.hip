@@ -4,7 +4,7 @@
 // projections (cake-core/src/models/llama3/attention.rs:49-60 q/k/v, :120 o;
 // mlp.rs:14-18 gate/up/down) and every Stable Diffusion / CLIP linear
 // (candle-transformers stable_diffusion attention/FF/proj layers reached from
-// cake-core/src/models/sd/{unet,vae,clip}.rs), SURVEY K03 / K34-K36 / K40.
+// cake-core/src/models/sd/{unet,vae,clip}.rs).
 //
 //   A = x [M][K] (activations, row stride lda), B = W [N][K] (HF weight layout,
 //   row stride ldb): both operands are k-contiguous, so every MFMA fragment is
@@ -214,7 +214,9 @@ static double tile_cost(const TileCost& c, int splits, long long M, long long Nv
   return std::max(us, ((double)Nv * K + (double)M * K) * 2 / 5e6 + 3);   // operands from memory
 }
 
-// (cfg, splits) for a product of M > 64 rows.  On entry *cfg, *splits: a measured plan of this very
+// (cfg, splits) for a product on tiles.  The estimate is fitted from 65 rows on; captured products of
+// fewer, whose stream form stays out of graphs, take it too (2 .. 64 rows of 14 weight shapes in
+// graphs: 0.93 to 2.6 times as fast as the plan of the nearest measured size).  On entry *cfg, *splits: a measured plan of this very
 // size, or cfg -1; it stands unless it is modelled and 10 % behind the best.  big: an operand of
 // 2 GB or more (31-bit offsets of the four-wave tiles).
 CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits) {

@@ -58,8 +58,9 @@ constexpr int alt_idx(int nr, int nd, int k) {
 
 // LDS-DMA of one 1 KiB piece (buffer_load_dwordx4 ... offen lds) with the M0 write in the
 // same statement (M0 is not preserved around inline asm); d = the buffer descriptor as an
-// SGPR quad; the add sets SCC, where the compiler may keep a comparison.  amfma_dma issues an MFMA between the M0 write and the DMA, which covers the
-// write's wait state (no s_nop) and keeps the DMA beside the MFMA it was scheduled with.
+// SGPR quad; the add sets SCC, where the compiler may keep a comparison.  amfma_dma issues an
+// MFMA between the M0 write and the DMA, which covers the write's wait state (no s_nop) and
+// keeps the DMA beside the MFMA it was scheduled with.
 template <int OFF>
 __device__ __forceinline__ void dma16(uint32_t mb, uint32_t voff, cu32x4 d, uint32_t soff) {
   asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"

@@ -5,10 +5,10 @@ q|k|v, o (+residual), gate|up (+SwiGLU), down (+residual); every SD UNet / VAE /
 CLIP projection (+bias, +residual, +GEGLU).  Shapes and strides are validated
 on the host before launch; there is no library fallback.
 
-Tile choice: a cost model over the kernel's tile configurations (waves of
-tiles x per-tile work, split-K when the grid is smaller than the chip), with an
-optional measured override table (:func:`set_plan`, filled by
-scripts/tune_gemm.py on the GPU box).
+Tile choice: products of up to 64 rows take forms of their own (gemm.hip rows_kind); from 65 rows
+on, and where a captured graph keeps those out, :func:`resolve` asks the kernel library's fitted
+estimate, which a measured entry of the very size (gemm_tuned.json) or a pinned plan
+(:func:`set_plan`) goes before.
 """
 from __future__ import annotations
 
@@ -456,8 +456,9 @@ def grouped_cfg(rows: int, groups: int, capturing: bool = False) -> int:
     # up and down product of 64 experts 4096 x 3616, us in the stream form and at 64 / 128 / 256 rows
     # a tile, by rows an expert: 3 561 / 651 / 646 / -, 6 644 / 688 / 669 / -, 9 680 / 705 / 672 / -,
     # 16 938 / 739 / 683 / -, 24 - / 775 / 698 / -, 75 - / 1275 / 766 / 895, 112 - / 1412 / 888 / 937
-    # (skewed 1435 / 984 / 1029), 131 - / 1550 / 1100 / 954, 192 - / 1998 / 1130 / 989; of small
-    # experts the 64-row tile has more workgroups
+    # (skewed 1435 / 984 / 1029), 131 - / 1550 / 1100 / 954, 192 - / 1998 / 1130 / 989.  Only these
+    # were timed: from 4 to 12 rows the 64-row tile loses 3 - 7 % here and is taken for the smaller
+    # experts' sake, of which it makes four times the workgroups
     mean = rows / groups
     if mean <= 4 and not capturing:   # the stream form's counters stay out of graphs
         return ROWS
