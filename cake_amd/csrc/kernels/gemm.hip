@@ -51,6 +51,16 @@ CAKE_GEMM_EXTERN_ALL(kBF16)
 CAKE_GEMM_EXTERN_ALL(kF16)
 #undef CAKE_GEMM_EXTERN_ALL
 #undef CAKE_GEMM_EXTERN
+// ... and in gemm_inst_pieces_{bf16,f16}_{a,b}.hip
+#define CAKE_PIECES_EXTERN(DT, E) extern template int launch_pieces<DT, E>(int, dim3, hipStream_t, const GemmArgs&);
+#define CAKE_PIECES_EXTERN_ALL(DT) CAKE_PIECES_EXTERN(DT, kEpiStore) CAKE_PIECES_EXTERN(DT, kEpiResid32) \
+  CAKE_PIECES_EXTERN(DT, kEpiAdd16) CAKE_PIECES_EXTERN(DT, kEpiSwiglu) CAKE_PIECES_EXTERN(DT, kEpiGeglu) \
+  CAKE_PIECES_EXTERN(DT, kEpiStore32) CAKE_PIECES_EXTERN(DT, kEpiSilu) CAKE_PIECES_EXTERN(DT, kEpiQuick) \
+  CAKE_PIECES_EXTERN(DT, kEpiGelu) CAKE_PIECES_EXTERN(DT, kEpiRelu2)
+CAKE_PIECES_EXTERN_ALL(kBF16)
+CAKE_PIECES_EXTERN_ALL(kF16)
+#undef CAKE_PIECES_EXTERN_ALL
+#undef CAKE_PIECES_EXTERN
 // ... and in gemm_inst_rows_{bf16,f16}.hip
 #define CAKE_ROWS_EXTERN(DT)                                                                      \
   extern template struct Rows<DT>;
@@ -93,6 +103,15 @@ CAKE_API int cake_gemm_tile(int cfg, int* bm, int* bn) {
 // the gated epilogues pair 16-column gate / up blocks inside one wave: 32-column multiples
 template <int DT>
 static int dispatch_epi(int epi, int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  if (g.pieces > 0) {
+    switch (epi) {
+#define P(E) case E: return launch_pieces<DT, E>(cfg, grid, st, g);
+      P(kEpiStore) P(kEpiResid32) P(kEpiAdd16) P(kEpiSwiglu) P(kEpiGeglu) P(kEpiStore32)
+      P(kEpiSilu) P(kEpiQuick) P(kEpiGelu) P(kEpiRelu2)
+#undef P
+    }
+    return (int)hipErrorInvalidValue;
+  }
   switch (epi) {
     case kEpiStore: return launch_gemm<DT, kEpiStore>(cfg, grid, st, g);
     case kEpiResid32: return launch_gemm<DT, kEpiResid32>(cfg, grid, st, g);

@@ -90,7 +90,10 @@ __device__ __forceinline__ void amfma_dma(cf32x4& acc, const uint4& a, const uin
 // padded rows and, below some 200 rows a group, by reading the weights: 64 groups of 192 rows,
 // 4096 -> 3616 -> 4096 columns, 1102 -> 989 us against eight waves on the same tile (0.98 PFLOP/s
 // with the padding; the weights alone are 2 x 292 us).
-template <int DT, int EPI, int BM, int BN, int SCHED = 0, bool GRP = false>
+// PCS: the tiles past the last whole wave in k pieces (GemmArgs::pieces); an instance of its own,
+// since the sums of pieces spill twice the registers in the epilogue of whole tiles too (4096^3 with
+// the residual 113.3 us with them, 109.9 without).
+template <int DT, int EPI, int BM, int BN, int SCHED = 0, bool GRP = false, bool PCS = false>
 __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   static_assert((BM == 256 && (BN == 256 || BN == 192)) || (BM == 128 && BN == 256),
                 "four-wave tile shapes");
@@ -112,27 +115,24 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   const int wr = wave >> 1, wc = wave & 1;
 
   // ---- XCD-aware grouped tile order (as gemm_kernel) ---------------------
-  // Pieces (g.pieces): workgroups [0, dp_tiles) run whole tiles, the rest run the remaining tiles
+  // Pieces (PCS): workgroups [0, dp_tiles) run whole tiles, the rest run the remaining tiles
   // in equal k pieces — the last partial wave of a grid at a fraction of its length (8B gate|up
   // at 2048 tokens: 896 tiles = 3 full waves + 128 tiles in halves), or every tile in pieces
   // when there are too few.  Equal pieces of all tiles walk k side by side and share their
   // operands in L2; one line of k steps cut into 256 equal shares (a tile's pieces at any k)
   // balanced better and ran at half the rate, every workgroup reading for itself.
-  if constexpr (GRP) {
-    g.tiles_m = g.groups[g.tiles_m].x;
-    g.pieces = 0;
-  }
+  if constexpr (GRP) g.tiles_m = g.groups[g.tiles_m].x;
   const int ntiles = g.tiles_m * g.tiles_n;
   if (GRP && (int)blockIdx.x >= ntiles) return;
   int id, split = blockIdx.y, piece = 0;
   int kb = split * g.kps, ke = min(g.K, kb + g.kps);
   {
     const int bid = blockIdx.x;
-    const int dp = g.pieces ? g.dp_tiles : ntiles;
-    if (bid < dp) {
+    const int dp = PCS ? g.dp_tiles : ntiles;
+    if (!PCS || bid < dp) {
       const int q = dp / 8, r = dp % 8, x = bid % 8, i = bid / 8;
       id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
-      if (g.pieces) {  // a whole tile
+      if constexpr (PCS) {  // a whole tile
         kb = 0;
         ke = g.K;
       }
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       ke = min(g.K, kb + g.kps);
     }
   }
-  const int pieces = (int)blockIdx.x >= (g.pieces ? g.dp_tiles : ntiles) ? g.pieces : 1;
+  const int pieces = PCS && (int)blockIdx.x >= g.dp_tiles ? g.pieces : 1;
   // grouped products: most groups have one or two row tiles, so two of them walk all columns and
   // their rows are read once (eight read every row four times over; 64 groups of 192 rows of 4096
   // to 3616 columns 509 -> 483 us, back 543 -> 506)
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   __builtin_amdgcn_s_waitcnt(vm_wait(0));
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   Pieces add{};
-  if (!GRP && pieces > 1) {
+  if (pieces > 1) {
     // Counters per tile (agent scope).  Every piece but the last to arrive stores its
     // accumulators to its slab ([i][j][thread] float4, coalesced; agent scope, so no fence has to
     // write an XCD's L2 back), counts itself ready once they are there and is done; the last
@@ -461,16 +461,14 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
     if (tid == 0) bc[0] = __hip_atomic_fetch_add(tk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const bool last = bc[0] == (uint32_t)(pieces - 1);
-    float4* slab = reinterpret_cast<float4*>(g.ws + (size_t)tile * pieces * (BM * BN)) + tid;
+    constexpr uint32_t SLAB = BM * BN * 4;
+    add = Pieces{g.ws + (size_t)tile * pieces * (BM * BN), pieces * SLAB, (uint32_t)tid * 16u,
+                 pieces > 2 ? 0u : (1 - piece) * SLAB, SLAB, pieces};
     if (!last || pieces > 2) {
-      float4* to = slab + (size_t)piece * (BM * BN / 4);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const cf32x4 v = acc[i][j];
-          st_agent16(to + (i * FN + j) * 256, v[0], v[1], v[2], v[3]);
-        }
+        for (int j = 0; j < FN; ++j) add.store(piece * SLAB + (i * FN + j) * 4096u, acc[i][j]);
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     }
     if (!last) {
@@ -484,8 +482,6 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       __hip_atomic_store(fl, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    add = Pieces{pieces > 2 ? slab : slab + (size_t)(1 - piece) * (BM * BN / 4),
-                 (size_t)(BM * BN / 4), pieces};
   }
   float* stg = reinterpret_cast<float*>(smem + wave * STG);
   const int row_m0 = m0 + wr * WTM;
@@ -504,16 +500,13 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
     // after the reads of the strip before it needs no wait)
     float* sg0 = reinterpret_cast<float*>(smem + (wave * 2) * STG);
     float* sg1 = reinterpret_cast<float*>(smem + (wave * 2 + 1) * STG);
-    const auto strip = [&](int i) {   // the pieces' float4s of strip i
-      return Pieces{add.base + i * FN * 256, add.stride, add.n};
-    };
     stage_strip_w<FN>(acc[0], sg0, lane, add);
     static_for<0, FM>([&](auto ii) __attribute__((always_inline)) {
       constexpr int i = decltype(ii)::value;
       __builtin_amdgcn_s_waitcnt(0xc07f);
       __builtin_amdgcn_wave_barrier();
       if constexpr (i + 1 < FM) {
-        stage_strip_w<FN>(acc[i + 1], (i & 1) ? sg0 : sg1, lane, strip(i + 1));
+        stage_strip_w<FN>(acc[i + 1], (i & 1) ? sg0 : sg1, lane, add.strip(i + 1, FN));
         ops.template load_res<(i + 1) & 1>(g, row_m0 + (i + 1) * 16, vcol0, lane);
       }
       readout_strip_w<DT, EPI, FN, i & 1>(g, (i & 1) ? sg1 : sg0, row_m0 + i * 16, vcol0, split,
@@ -532,7 +525,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       if constexpr (i + 1 < FM)
         ops.template load_res<(i + 1) & 1>(g, row_m0 + (i + 1) * 16 + (lane >> 2), vcol0, lane);
       epi_strip<DT, EPI, FN, i & 1>(g, acc[i], stg, row_m0 + i * 16, vcol0, split, lane, ops,
-                                    Pieces{add.base + i * FN * 256, add.stride, add.n});
+                                    add.strip(i, FN));
     });
   }
 #ifdef CAKE_GEMM_STAMPS

@@ -101,12 +101,30 @@ __device__ __forceinline__ float4 ld_agent16(const float4* p) {
 }
 
 // a tile's pieces (gemm_4w.h): n 0, the tile is whole; 2, this wave's accumulators and the parked
-// ones at base; more, all parked, stride float4s apart.  base: this thread's float4s of the current
-// strip, tile j of it at base[j * 256]
+// ones at `at`; more, all parked, `stride` apart.  Bytes of the tile's slabs (uniform, `bytes` of
+// them): tile j of the current strip of this thread (`lane`) at + 4096 j.  16-byte accesses past the
+// caches that other XCDs do not see (sc1): as pairs of 8-byte atomics they took 128 tiles in two
+// pieces 16 us longer (2048 x 28672 x 4096 SwiGLU 385 us, 359 so), in four pieces a tenth of the
+// product (1100 x 4096 x 23552 282, 250)
 struct Pieces {
-  const float4* base;
-  size_t stride;
+  float* slabs;
+  uint32_t bytes, lane, at, stride;
   int n;
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  static constexpr int kSc1 = 16;
+  __device__ __forceinline__ float4 load(uint32_t off) const {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+        __builtin_amdgcn_make_buffer_rsrc(slabs, 0, (int)bytes, 0x00020000), (int)lane, (int)off, kSc1));
+  }
+  __device__ __forceinline__ void store(uint32_t off, const cf32x4& v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v),
+        __builtin_amdgcn_make_buffer_rsrc(slabs, 0, (int)bytes, 0x00020000), (int)lane, (int)off, kSc1);
+  }
+  __device__ __forceinline__ Pieces strip(int i, int nf) const {   // strip i of nf tiles each
+    Pieces p = *this;
+    p.at += (uint32_t)(i * nf) * 4096u;
+    return p;
+  }
 };
 
 // virtual B row -> weight row (gated: [16 gate rows | 16 up rows] per 32-row block)
@@ -287,23 +305,25 @@ __device__ __forceinline__ void stage_strip_w(const cf32x4 (&tiles)[NF], float* 
   if (add.n > 2) {   // all of them parked
     float4 v[NF];
 #pragma unroll
-    for (int j = 0; j < NF; ++j) v[j] = ld_agent16(add.base + j * 256);
+    for (int j = 0; j < NF; ++j) v[j] = add.load(add.at + j * 4096u);
     for (int q = 1; q < add.n; ++q) {
-      const float4* src = add.base + q * add.stride;
+      float4 o[NF];
+#pragma unroll
+      for (int j = 0; j < NF; ++j) o[j] = add.load(add.at + q * add.stride + j * 4096u);
 #pragma unroll
       for (int j = 0; j < NF; ++j) {
-        const float4 o = ld_agent16(src + j * 256);
-        v[j].x += o.x; v[j].y += o.y; v[j].z += o.z; v[j].w += o.w;
+        v[j].x += o[j].x; v[j].y += o[j].y; v[j].z += o[j].z; v[j].w += o[j].w;
       }
     }
 #pragma unroll
     for (int j = 0; j < NF; ++j) put(j, v[j].x, v[j].y, v[j].z, v[j].w);
   } else if (add.n == 2) {
+    float4 o[NF];
 #pragma unroll
-    for (int j = 0; j < NF; ++j) {
-      const float4 o = ld_agent16(add.base + j * 256);
-      put(j, tiles[j][0] + o.x, tiles[j][1] + o.y, tiles[j][2] + o.z, tiles[j][3] + o.w);
-    }
+    for (int j = 0; j < NF; ++j) o[j] = add.load(add.at + j * 4096u);
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+      put(j, tiles[j][0] + o[j].x, tiles[j][1] + o[j].y, tiles[j][2] + o[j].z, tiles[j][3] + o[j].w);
   } else {
 #pragma unroll
     for (int j = 0; j < NF; ++j) put(j, tiles[j][0], tiles[j][1], tiles[j][2], tiles[j][3]);
@@ -988,6 +1008,27 @@ constexpr bool gated_ok(int wave_cols) {
   return wave_cols % 32 == 0 || !(EPI == kEpiSwiglu || EPI == kEpiGeglu);
 }
 
+template <int DT, int EPI, bool PCS>
+int launch_4w(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
+#define X(ID, BM, BN, SCHED)                                                                   \
+  if (cfg == ID) {                                                                             \
+    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, BM, BN, SCHED, false, PCS>), grid, dim3(256),  \
+                       0, st, g);                                                              \
+    return (int)hipGetLastError();                                                             \
+  }
+  X(k4WCfg, 256, 256, 0) X(k4WCfg192, 256, 192, 0) X(k4WCfg128, 128, 256, 0)
+  X(k4WCfg + k4WSched, 256, 256, 1) X(k4WCfg192 + k4WSched, 256, 192, 1)
+  X(k4WCfg128 + k4WSched, 128, 256, 1)
+#undef X
+  return (int)hipErrorInvalidValue;
+}
+
+// four-wave tiles of which some run in pieces (GemmArgs::pieces)
+template <int DT, int EPI>
+int launch_pieces(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  return launch_4w<DT, EPI, true>(cfg, grid, st, g);
+}
+
 template <int DT, int EPI>
 int launch_gemm(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
   if (cfg == kPPCfg) {
@@ -998,30 +1039,7 @@ int launch_gemm(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
     hipLaunchKernelGGL((gemm_rs_kernel<DT, EPI>), grid, dim3(256), 0, st, g);
     return (int)hipGetLastError();
   }
-  if (cfg == k4WCfg) {
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 256, 256>), grid, dim3(256), 0, st, g);
-    return (int)hipGetLastError();
-  }
-  if (cfg == k4WCfg192) {
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 256, 192>), grid, dim3(256), 0, st, g);
-    return (int)hipGetLastError();
-  }
-  if (cfg == k4WCfg128) {
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 128, 256>), grid, dim3(256), 0, st, g);
-    return (int)hipGetLastError();
-  }
-  if (cfg == k4WCfg + k4WSched) {
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 256, 256, 1>), grid, dim3(256), 0, st, g);
-    return (int)hipGetLastError();
-  }
-  if (cfg == k4WCfg192 + k4WSched) {
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 256, 192, 1>), grid, dim3(256), 0, st, g);
-    return (int)hipGetLastError();
-  }
-  if (cfg == k4WCfg128 + k4WSched) {
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 128, 256, 1>), grid, dim3(256), 0, st, g);
-    return (int)hipGetLastError();
-  }
+  if (four_wave_cfg(cfg)) return launch_4w<DT, EPI, false>(cfg, grid, st, g);
 
 #define X(id, BM, BN, WM, WN, NS, PR)                                                        \
   if (cfg == id) {                                                                           \
