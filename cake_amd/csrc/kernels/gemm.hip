@@ -186,27 +186,41 @@ CAKE_API long long cake_gemm_ws_floats(int cfg, int splits, int M, int N, int K,
 // off the best of all, at most 33 %; the nearest measured size with its split scaled was 16 % off
 // (777 x 4096 x 14336 184 us, 113 us so; 6000 rows 680, 550).  Left out: the tiles that were best
 // nowhere beyond what these reach.
+// An image model's products are short (k from 128) or have a 16-bit residual or GEGLU: the tile's end
+// weighs as much as its k steps, so these have epilogue terms of their own, and three tiles more.
+// Over 123 sizes (width 256 .. 2048, 66 .. 18432 rows) 1.5 % off the best on the average, at most 15;
+// without the terms 5.5 %, at most 58 (12288 x 320 x 320 + residual 17.3 us, 11.0 so; 6144 x 5120 x
+// 640 GEGLU 59.6, 50.8).
 struct TileCost {
   int cfg, bm, bn, slots;                  // slots: workgroups a CU holds
-  float c0, step, lone, epi[4], merge, fin;
+  // epi: store, f32, SwiGLU, SiLU / GELU, 16-bit residual, GEGLU, store of k < 512; negative epi or
+  // merge: not modelled (that epilogue, that tile in splits)
+  float c0, step, lone, epi[7], merge, fin;
 };
 static constexpr TileCost kTileCosts[] = {
-    {5, 256, 256, 1, 0.69f, 1.43f, 0.f, {5.52f, 7.84f, 9.9f, 6.58f}, 4.16f, 0.304f},
-    {6, 256, 128, 1, 0.844f, 0.802f, 0.f, {4.16f, 5.6f, 6.f, 4.4f}, 3.93f, 0.325f},
-    {7, 128, 128, 1, 2.77f, 0.539f, 0.f, {2.72f, 3.65f, 4.5f, 4.2f}, 3.6f, 0.382f},
-    {12, 64, 128, 2, 4.62f, 0.663f, 0.145f, {0.f, 0.598f, 1.92f, 1.93f}, 3.09f, 0.468f},
-    {13, 64, 64, 2, 3.41f, 0.427f, 0.107f, {0.79f, 1.37f, 2.48f, 2.18f}, 2.83f, 0.484f},
-    {18, 64, 160, 1, 2.28f, 0.467f, 0.f, {2.54f, 3.f, 0.f, 4.42f}, 3.53f, 0.353f},
-    {22, 256, 256, 1, 0.f, 1.26f, 0.f, {10.9f, 15.f, 14.f, 21.7f}, 13.2f, 10.2f},
-    {25, 256, 256, 1, 0.f, 1.49f, 0.f, {0.f, 0.f, 0.f, 0.f}, 20.8f, 13.2f},
-    {26, 256, 192, 1, 0.f, 1.13f, 0.f, {4.44f, 2.29f, 2.14f, 9.67f}, 16.1f, 6.33f},
-    {27, 128, 256, 1, 4.43f, 0.837f, 0.f, {0.0783f, 0.464f, 1.66f, 4.49f}, 13.7f, 4.33f},
+    {4, 64, 64, 4, 1.48f, 0.787f, 0.263f, {-1.f, -1.f, -1.f, -1.f, 3.44f, 2.92f, 3.04f}, -1.f, 0.f},
+    {5, 256, 256, 1, 0.69f, 1.43f, 0.f, {5.52f, 7.84f, 9.9f, 6.58f, 11.7f, 9.55f, 8.55f}, 4.16f, 0.304f},
+    {6, 256, 128, 1, 0.844f, 0.802f, 0.f, {4.16f, 5.6f, 6.f, 4.4f, 7.42f, 6.68f, 6.1f}, 3.93f, 0.325f},
+    {7, 128, 128, 1, 2.77f, 0.539f, 0.f, {2.72f, 3.65f, 4.5f, 4.2f, 5.25f, 4.69f, 4.05f}, 3.6f, 0.382f},
+    {8, 128, 128, 2, 2.27f, 1.02f, 0.44f, {-1.f, -1.f, -1.f, -1.f, 5.46f, 4.78f, 4.01f}, -1.f, 0.f},
+    {12, 64, 128, 2, 4.62f, 0.663f, 0.145f, {0.f, 0.598f, 1.92f, 1.93f, 1.82f, 2.31f, -1.f}, 3.09f, 0.468f},
+    {13, 64, 64, 2, 3.41f, 0.427f, 0.107f, {0.79f, 1.37f, 2.48f, 2.18f, 2.f, 2.05f, 1.75f}, 2.83f, 0.484f},
+    {14, 64, 160, 2, 1.33f, 0.779f, 0.386f, {-1.f, -1.f, -1.f, -1.f, 5.97f, -1.f, 3.69f}, -1.f, 0.f},
+    {18, 64, 160, 1, 2.28f, 0.467f, 0.f, {2.54f, 3.f, 0.f, 4.42f, 5.07f, -1.f, 3.2f}, 3.53f, 0.353f},
+    {22, 256, 256, 1, 0.f, 1.26f, 0.f, {10.9f, 15.f, 14.f, 21.7f, 18.1f, 11.4f, 12.f}, 13.2f, 10.2f},
+    {25, 256, 256, 1, 0.f, 1.49f, 0.f, {0.f, 0.f, 0.f, 0.f, 14.9f, 9.6f, 10.8f}, 20.8f, 13.2f},
+    {26, 256, 192, 1, 0.f, 1.13f, 0.f, {4.44f, 2.29f, 2.14f, 9.67f, 13.1f, 9.73f, 9.91f}, 16.1f, 6.33f},
+    {27, 128, 256, 1, 4.43f, 0.837f, 0.f, {0.0783f, 0.464f, 1.66f, 4.49f, 6.33f, 4.58f, 3.86f}, 13.7f, 4.33f},
 };
 static double tile_cost(const TileCost& c, int splits, long long M, long long Nv, int K, int epi) {
   const long long ks = (K + kGBK - 1) / kGBK, t = ((M + c.bm - 1) / c.bm) * ((Nv + c.bn - 1) / c.bn);
-  const int cls = epi == kEpiResid32 || epi == kEpiStore32            ? 1
-                  : epi == kEpiSwiglu || epi == kEpiGeglu             ? 2
-                  : epi == kEpiSilu || epi == kEpiQuick || epi == kEpiGelu ? 3 : 0;
+  const int cls = epi == kEpiResid32 || epi == kEpiStore32                 ? 1
+                  : epi == kEpiSwiglu                                      ? 2
+                  : epi == kEpiSilu || epi == kEpiQuick || epi == kEpiGelu ? 3
+                  : epi == kEpiAdd16                                       ? 4
+                  : epi == kEpiGeglu                                       ? 5
+                  : epi == kEpiStore && K < 512                            ? 6 : 0;
+  if (c.epi[cls] < 0 || (splits > 1 && c.merge < 0)) return -1;   // not modelled
   double steps, rounds, lone = 0, fin = 0;
   bool split = false;
   if (four_wave_cfg(c.cfg)) {
@@ -230,14 +244,16 @@ static double tile_cost(const TileCost& c, int splits, long long M, long long Nv
   }
   const double us = c.c0 + c.step * steps + c.lone * lone + c.epi[cls] * rounds +
                     (split ? c.merge + c.fin * fin : 0.);
-  return std::max(us, ((double)Nv * K + (double)M * K) * 2 / 5e6 + 3);   // operands from memory
+  // operands from memory; of tiles that all wait for them the one with the least work (113 x 57344 x
+  // 8192 SwiGLU 193 us on 128 x 256, 209 on 128 x 128)
+  return std::max(us, ((double)Nv * K + (double)M * K) * 2 / 5e6 + 3) + 0.02 * us;
 }
 
 // (cfg, splits) for a product on tiles.  The estimate is fitted from 65 rows on; captured products of
 // fewer, whose stream form stays out of graphs, take it too (2 .. 64 rows of 14 weight shapes in
-// graphs: 0.93 to 2.6 times as fast as the plan of the nearest measured size).  On entry *cfg, *splits: a measured plan of this very
-// size, or cfg -1; it stands unless it is modelled and 10 % behind the best.  big: an operand of
-// 2 GB or more (31-bit offsets of the four-wave tiles).
+// graphs: 0.93 to 2.6 times as fast as the plan of the nearest measured size).  On entry *cfg,
+// *splits: a measured plan of this very size, or cfg -1; it stands unless it is modelled and 10 %
+// behind the best.  big: an operand of 2 GB or more (31-bit offsets of the four-wave tiles).
 CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits) {
   if (M < 1 || Nv < 1 || K < 1 || !cfg || !splits) return (int)hipErrorInvalidValue;
   const bool gated = epi == kEpiSwiglu || epi == kEpiGeglu;
@@ -255,7 +271,7 @@ CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* c
     for (int sp = 1; sp <= 16; sp *= 2) {
       if (sp > 1 && (ks / sp < 4 || (four && M < 200))) break;
       const double t = tile_cost(c, sp, M, Nv, K, epi);
-      if (t < best) {
+      if (t >= 0 && t < best) {
         best = t;
         bc = c.cfg;
         bs = sp;

@@ -41,6 +41,25 @@ def test_measured_entry_of_the_size_stands_unless_well_behind(monkeypatch):
     assert at(20, 1) == (20, 1)     # a tile the estimate does not cover
 
 
+@pytest.mark.parametrize("size,times", [
+    # us of the tiles (unsplit) on an MI355X: the estimate's choice is within a tenth of the best
+    ((12288, 320, 320, "add16"), {14: 11.6, 4: 11.8, 1: 13.0, 13: 13.2, 8: 13.4, 27: 18.4}),
+    ((7040, 640, 640, "add16"), {14: 16.3, 6: 18.7, 8: 19.0, 4: 20.6, 27: 21.5}),
+    ((7040, 640, 2560, "add16"), {14: 37.4, 6: 41.8, 27: 43.8, 8: 45.2}),
+    ((18432, 2560, 320, "geglu"), {5: 53.9, 22: 57.5, 8: 60.8, 26: 63.5, 27: 64.3}),
+    ((3200, 2560, 320, "geglu"), {27: 12.6, 8: 12.7, 12: 16.4, 4: 17.1, 26: 17.2}),
+    ((800, 5120, 640, "geglu"), {6: 15.1, 8: 15.2, 27: 15.6, 4: 17.5, 26: 20.0}),
+    ((18432, 960, 320, "store"), {8: 29.1, 14: 29.1, 26: 30.6, 6: 32.7, 27: 32.8, 12: 34.7}),
+    ((113, 57344, 8192, "swiglu"), {27: 193.0, 8: 204.7, 7: 209.5, 22: 221.2})], ids=str)
+def test_estimate_picks_a_measured_best(monkeypatch, size, times):
+    """Short products, residual and GEGLU epilogues, and tiles that all wait for the weights."""
+    from cake_amd.ops import gemm as G
+    monkeypatch.setattr(G, "_TUNED", [])
+    monkeypatch.setattr(G, "_resolved", {})
+    cfg, splits = G.resolve(*size)
+    assert splits == 1 and times[cfg] <= 1.1 * min(times.values())
+
+
 def test_library_plan_falls_back_to_the_plan_without_it(monkeypatch):
     """A call that the library form does not carry (a bias) runs what a table without the library's
     entries plans, as the native engines do, not the nearest measured size."""
