@@ -359,11 +359,14 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
 
 // ---- products of few rows (gemm_rows.h) -----------------------------------
 // Which form a product of M rows takes: 0 the tile kernels (cake_gemm_scaled), 1 direct, 2 stream.
-// The estimates (us) are fits to timings on weights that no cache holds, 5 .. 64 rows, weight
-// matrices of 8 .. 260 MB; both sides of the lines they draw, measured: 4096 x 4096 at 16 rows
-// direct 12.6, stream 12.5; 4096 x 14336 direct 38, stream 25; 6144 x 4096 at 5 rows direct 16.9,
-// stream 14.5, 3072 x 2048 6.5, 7.9; 28672 x 4096 at 45 rows stream 53, tiles 58; 4096 x 4096 at 45
-// rows stream 19, tiles 17.
+// The estimates (us) are fits to timings on weights that no cache holds, 2 .. 64 rows of 24 weight
+// shapes, 1 .. 940 MB: the form they pick is 0.7 % off the best of the three on the average.  Both
+// sides of the lines they draw, measured: 4096 x 4096 at 16 rows direct 11.8, stream 12.1; 4096 x 14336
+// direct 37, stream 23; 6144 x 4096 at 5 rows direct 16.9, stream 14.5, 3072 x 2048 6.5, 7.9; 28672 x
+// 4096 at 45 rows stream 52, tiles 55; 6144 x 4096 at 45 rows stream 22.0, tiles 19.4, 4096 x 11008
+// 31.0, 27.9.  Rows of k that start amid a 128-byte line (k no multiple of 64) cost a second line at
+// either end of a piece: 4096 x 10928 against 4096 x 11008, 5 rows direct 31.4 / 23.6, stream 23.5 /
+// 20.5, 33 rows stream 35.0 / 29.5, tiles 29.4 / 27.1.
 struct StreamPlan { int bn, kst, wgs; };
 // the stream form's shape (gemm_rows.h StreamShape)
 static StreamPlan stream_plan(int mt, bool gated) {
@@ -373,19 +376,29 @@ static int rows_kind(int M, long long Nv, int K, bool gated) {
   if (M > 64 || Nv > 64LL * kRowsTicks) return 0;
   const double kb = K * 2e-3;   // KB of one row of k
   const int mt = (M + 15) / 16;
-  const double tiles = 8 + Nv * kb / 4600;
+  const bool mid = K % 64 != 0;   // rows start amid a line
+  const double tiles = 6.7 + Nv * kb / 5590 + 0.0043 * M + 0.45e-3 * K;
   const StreamPlan sp = stream_plan(mt, gated);
   const long long strips = (Nv + sp.bn - 1) / sp.bn, ks = (K + sp.kst - 1) / sp.kst, total = strips * ks;
   const long long per = std::max<long long>((total + sp.wgs - 1) / sp.wgs, kRowsMinK / sp.kst);
-  const double stream = sp.wgs == 512 ? 6.2 + 0.08 * M + 1.42 * per
-                        : 7 + (ks > per || ks % per ? 0.7 * mt : 0.) + per * (16 + 2 * mt) / 27.;
+  double stream;
+  if (sp.wgs == 512) {
+    stream = 6.2 + 0.08 * M + (1.42 + (mid ? 0.11 : 0.)) * per;
+  } else {
+    // a strip's shares, parked and summed; equal shares of rows 16 KB apart start on the same
+    // channels of the memory (8192 x 8192 at 24 rows 35.6 us, 10240 x 8192 35.1)
+    const double shares = ks > per || ks % per ? (double)ks / per : 0.;
+    const bool camp = K % 8192 == 0 && ks % per == 0;
+    stream = (mt > 1 ? 3 : 4.3) + mt * (0.86 * std::min(shares, 1.) + 0.25 * shares) +
+             per * (0.65 + 0.027 * mt + (mid ? 0.19 : 0.) + (camp ? 0.2 : 0.));
+  }
   double direct = 1e9;
   if (M <= 32) {
     const int nt = gated || Nv > 4096 ? 2 : 1;
     const long long wgs = (Nv + 16 * nt - 1) / (16 * nt);
     // a CU's share at 32 (of two strips 26) KB a us, all weights and half of the reads of x at 5.8 MB
-    direct = 4 + std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
-                          (Nv + 0.5 * wgs * M) * kb / 5800);
+    direct = 4 + (mid ? 1.35 : 1.) * std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
+                                              (Nv + 0.5 * wgs * M) * kb / 5800);
   }
   if (direct <= stream && direct <= tiles) return 1;
   return stream < tiles ? 2 : 0;

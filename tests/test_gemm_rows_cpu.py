@@ -19,6 +19,19 @@ def test_rows_kind_lines():
                for K in (64, 8192))
 
 
+@pytest.mark.parametrize("M,Nv,K,kind", [
+    # us measured as tiles / direct / stream
+    (33, 6144, 4096, 0),     # 18.3 / - / 20.7
+    (24, 8192, 8192, 0),     # 32.2 / 38.2 / 35.6: equal shares on the same channels
+    (24, 10240, 8192, 2),    # 44.9 / 68.3 / 35.1
+    (45, 4096, 10928, 0),    # 31.3 / - / 36.6: rows that start amid a line
+    (5, 4096, 10928, 2),     # 28.9 / 31.4 / 23.5
+    (64, 10240, 8192, 2)])   # 52.3 / - / 40.9
+def test_rows_kind_takes_the_measured_best(M, Nv, K, kind):
+    from cake_amd.ops import gemm as G
+    assert G.rows_kind(M, Nv, K, False) == kind
+
+
 def test_grouped_rows_stay_out_of_graphs():
     from cake_amd.ops import gemm as G
     assert G.grouped_cfg(78, 64) == G.ROWS and G.grouped_cfg(78, 64, capturing=True) == 4
