@@ -42,11 +42,12 @@ class Plan:
     cfg: int              # grouped GEMM configuration (16-bit types)
 
 
-def plan(ids, score, E: int, dtype) -> Plan:
+def plan(ids, score, E: int, dtype, weight: int = 0) -> Plan:
+    """Rows sorted by expert, and their tiles; weight: elements of an expert's matrix."""
     N, top = ids.shape
     _routing(E, top)
     M, dev = N * top, ids.device
-    cfg = G.grouped_cfg(M, E, torch.cuda.is_current_stream_capturing())
+    cfg = G.grouped_cfg(M, E, torch.cuda.is_current_stream_capturing(), weight)
     bm = BM32 if dtype == torch.float32 else G.GROUPED_CFGS[cfg]
     n = M // bm + min(E, M)
     i32 = torch.empty(2 * M + 4 * (n + 1) + 4, device=dev, dtype=torch.int32)

@@ -451,18 +451,22 @@ ROWS = 32
 GROUPED_CFGS = {0: 128, 4: 64, 5: 256, ROWS: 16}
 
 
-def grouped_cfg(rows: int, groups: int, capturing: bool = False) -> int:
-    """Tile configuration for `rows` sorted rows over `groups` weight groups."""
+def grouped_cfg(rows: int, groups: int, capturing: bool = False, weight: int = 0) -> int:
+    """Tile configuration for `rows` sorted rows over `groups` weight groups of `weight` elements each
+    (0: small)."""
     # up and down product of 64 experts 4096 x 3616, us in the stream form and at 64 / 128 / 256 rows
     # a tile, by rows an expert: 3 561 / 651 / 646 / -, 6 644 / 688 / 669 / -, 9 680 / 705 / 672 / -,
     # 16 938 / 739 / 683 / -, 24 - / 775 / 698 / -, 75 - / 1275 / 766 / 895, 112 - / 1412 / 888 / 937
-    # (skewed 1435 / 984 / 1029), 131 - / 1550 / 1100 / 954, 192 - / 1998 / 1130 / 989.  Only these
-    # were timed: from 4 to 12 rows the 64-row tile loses 3 - 7 % here and is taken for the smaller
-    # experts' sake, of which it makes four times the workgroups
+    # (skewed 1435 / 984 / 1029), 131 - / 1550 / 1100 / 954, 192 - / 1998 / 1130 / 989.  From 4 to 12
+    # rows the 64-row tile loses 3 - 7 % here and is taken for the smaller experts' sake, of which it
+    # makes twice the workgroups: one product at 14 rows, 64 / 128 rows a tile, by millions of weights
+    # in all: 17 14.4 / 17.6 (8 of 1024 x 2048 24.4 / 29.3), 34 18.5 / 20.3, 101 47.6 / 50.1,
+    # 215 equal, 268 128.6 / 128.2
     mean = rows / groups
     if mean <= 4 and not capturing:   # the stream form's counters stay out of graphs
         return ROWS
-    return 5 if mean >= 115 else 0 if mean >= 12 else 4
+    big = groups * weight >= 200_000_000
+    return 5 if mean >= 115 else 0 if mean >= (12 if big else 24) else 4
 
 
 def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out: torch.Tensor,

@@ -38,6 +38,15 @@ def test_grouped_rows_stay_out_of_graphs():
     assert G.grouped_cfg(64 * 5, 64) == 4
 
 
+@pytest.mark.parametrize("E,N,K,cfg", [(8, 1024, 2048, 4), (32, 512, 1024, 4), (128, 256, 1024, 4),
+                                       (64, 768, 2048, 4), (64, 4096, 3616, 0), (64, 1640, 2048, 0)])
+def test_grouped_tiles_of_small_experts(E, N, K, cfg):
+    """Between 12 and 24 rows an expert: 128-row tiles only of weights that fill the chip with them."""
+    from cake_amd.ops import gemm as G
+    assert G.grouped_cfg(16 * E, E, weight=N * K) == cfg
+    assert G.grouped_cfg(16 * E, E) == 4 and G.grouped_cfg(24 * E, E, weight=N * K) == 0
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="makes launches without operands")
 @pytest.mark.parametrize("E,N,K,rows", [(1024, 4096, 64, 1500), (512, 8192, 64, 2048),
                                         (1024, 4096, 4096, 4096), (1, 64, 64, 1)])
