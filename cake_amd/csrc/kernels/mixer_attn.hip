@@ -497,7 +497,7 @@ CAKE_API int cake_mixer_flash(int dt, const void* qn, const void* kc, const void
     return (int)hipErrorInvalidValue;
   MixFlashArgs a{qn, kc, vc, k_slot, v_slot, (const SeqRow*)seq, gate, ldg, out, ldo,
                  H, G, DP, DVP, vdim, S, sink, scale * 1.4426950408889634f, {}};
-  if (flash3_ok(dt, a, false, S))
+  if (flash3_ok(dt, a, false, S, max_len, B))
     return dt == kBF16 ? launch_mix_flash3<kBF16, false>(a, max_len, B, st)
                        : launch_mix_flash3<kF16, false>(a, max_len, B, st);
   const dim3 grid((max_len + 127) / 128, H, B);

@@ -418,7 +418,13 @@ __global__ __launch_bounds__(256, 1) void mixer_flash3_kernel(MixFlashArgs a) {
 
 // Whether mixer_flash3_kernel takes a call: its head sizes, a scale that keeps the order of the
 // scores, 8-byte output and gate rows, a sequence's keys and values under 2 GB (rows: its most).
-inline bool flash3_ok(int dt, const MixFlashArgs& a, bool lat, long long rows) {
+// Not many sequences of a few rows: one wave of four has work then, and of the kernel above several
+// workgroups share a compute unit (us, this / the other: 24 sequences of 8 rows, 16 heads 9.2 / 7.9,
+// 32 heads 13.6 / 12.7, latent 14.0 / 9.2 and 20.8 / 15.3; 60 of 20 17.7 / 20.0 and 34.7 / 37.0, latent
+// 30.4 / 23.3 and 59 / 45; 40 of 33 14.4 / 17.4, latent 23.7 / 26.0; 8 of 20, 256 workgroups, latent
+// 8.4 / 10.4).
+inline bool flash3_ok(int dt, const MixFlashArgs& a, bool lat, long long rows, int max_len, int B) {
+  if (max_len <= (lat ? 32 : 12) && (long long)a.H * B > 256) return false;
   const auto al = [](const void* p, long long ld) { return (uintptr_t)p % 8 == 0 && ld % 4 == 0; };
   const long long lim = 0x7fffffffLL / 2;   // elements; the tiles requested ahead: offsets of 32 bits
   const auto rows_fit = [&](long long ld) { return rows * ld < lim && (rows + 256) * ld < 2 * lim; };

@@ -608,7 +608,7 @@ CAKE_API int cake_latent_flash(int dt, const void* q, long long ldq, const void*
   a.lat.rd2 = rd2;
   if (dt != kF32) {
     a.lat.rope = reinterpret_cast<const uint16_t*>(cache) + RP;
-    if (flash3_ok(dt, a, true, slot_stride / LD))
+    if (flash3_ok(dt, a, true, slot_stride / LD, max_len, B))
       return dt == kBF16 ? launch_mix_flash3<kBF16, true>(a, max_len, B, st)
                          : launch_mix_flash3<kF16, true>(a, max_len, B, st);
   }

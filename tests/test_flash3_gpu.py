@@ -136,6 +136,36 @@ def test_latent(dt, H, seqs):
                 _close(out[r0:r0 + n, h * 128:h * 128 + 128], w, dt)
 
 
+@pytest.mark.parametrize("dt", DTYPES, ids=str)
+@pytest.mark.parametrize("n", [1, 12, 13, 32, 33])
+def test_many_short_sequences(dt, n):
+    """Either side of the lines between the core and the general kernel, in both forms."""
+    H, B, S = 16, 17, 64
+    rows = M.Rows.pack([(i, 0, [0] * (n - i % 2 * (n > 1))) for i in range(B)], "cuda")
+    lat = L.LatentShape(H, 128, 64, 128, 96, 64, 30)
+    g = torch.Generator().manual_seed(n)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(dt)
+    qn, kc, vc = rnd(rows.N, H, 128), rnd(B, 4, S, 128), rnd(B, 4, 128, S)
+    lq, lk, vt, cache = rnd(rows.N, H * 192), rnd(rows.n_keys, H * 128), rnd(H * 128, rows.n_keys), rnd(B, S, lat.LD)
+    cs = torch.tensor([1.0, 0.0], device="cuda").repeat(S, 30)   # no rotation
+    out = torch.empty(2, rows.N, H * 128, device="cuda", dtype=dt)
+    M.attn_prompt(M.AttnShape(H, 4, 128, 128), qn.cuda(), kc.cuda(), vc.cuda(), rows, None, out[0], 0.1, True)
+    L.prompt(lat, lq.cuda(), lk.cuda(), vt.cuda(), rows, cs, cache.cuda(), out[1], 0.08)
+    got = out.cpu()
+    for i in (0, 9, B - 1):
+        r0, m, _, s = rows.host[i]
+        k0 = int(rows.key0[i])
+        for h in (0, H - 1):
+            c = slice(h * 128, h * 128 + 128)
+            _close(got[0, r0:r0 + m, c],
+                   _want(qn[r0:r0 + m, h], kc[s, h // 4, :m], vc[s, h // 4, :, :m].t(), 0, 0.1, True), dt)
+            kk = torch.cat([lk[k0:k0 + m, c], cache[s, :m, lat.RP:lat.RP + 64]], 1)
+            _close(got[1, r0:r0 + m, c],
+                   _want(lq[r0:r0 + m, h * 192:h * 192 + 192], kk, vt[c, k0:k0 + m].t(), 0, 0.08), dt)
+
+
 def _first_touched(n, p0, p, rows):
     """First of n rows at positions p0.. that a value of probability 0 at key p may reach: of the
     first wave (`rows` rows) that takes the key's run of `rows` keys."""
