@@ -404,8 +404,10 @@ CAKE_API int cake_expert_down(int dt, const void* in, const int* sel, int top, c
     hipLaunchKernelGGL(kern, dim3(g), dim3(64 * waves), lds, st, a, inv);
     return (int)hipGetLastError();
   };
-  // every workgroup stages the whole input row: eight waves a workgroup where they still reach every
-  // compute unit halve those reads (6 of 3616 columns to 4096 rows: 31.7 -> 30.2 us)
-  DISPATCH_DT(dt, return (W + 1) / 2 >= 2048 ? run(expert_down_kernel<DT, 8>, 8)
-                                             : run(expert_down_kernel<DT, 4>, 4));
+  // every workgroup stages the whole input row: eight waves a workgroup halve those reads where they
+  // still reach every compute unit (6 of 3616 columns to 4096 rows: 31.7 -> 30.2 us) and leave none
+  // with more row pairs than four would (4 of 2048 to 6000 rows, 375 workgroups: 16.7 -> 18.1)
+  const int n4 = ((W + 1) / 2 + 3) / 4, n8 = (n4 + 1) / 2;
+  const bool wide = (W + 1) / 2 >= 2048 && (n8 + 255) / 256 * 2 <= (n4 + 255) / 256;
+  DISPATCH_DT(dt, return wide ? run(expert_down_kernel<DT, 8>, 8) : run(expert_down_kernel<DT, 4>, 4));
 }
