@@ -325,8 +325,10 @@ __global__ __launch_bounds__(256, (FlashGeo<DT, KC>::WGS)) void mixer_flash_kern
 }
 
 // 16-bit types, keys of 128 columns (LAT: 128 and 64 rotated) and values of 128, on the shared
-// core (flash3.h), 128 rows a workgroup, the maximum exact as in the kernel above (the same rounding
-// of every probability).  32 heads over 8, us before / after: 300 rows 26.5 / 14.2, 1100 64 / 34,
+// core (flash3.h), 128 rows a workgroup, the maximum exact as in the kernel above.  Error against 64
+// bits as there, 0.00210 at 2048 rows; latent 0.00203 / 0.00202 (that kernel's tiles are of 32 keys:
+// twice as many find a new maximum, whose probability, 1, is not rounded).
+// 32 heads over 8, us before / after: 300 rows 26.5 / 14.2, 1100 64 / 34,
 // 2048 110 / 65, 24 sequences of 60 47 / 32; latent 300 27 / 16, 1100 85 / 36, 2048 154 / 71.  (64
 // rows a wave: 1.05 - 1.15x faster from 3000 rows on with a deferred maximum, slower below.)
 template <int DT, bool LAT>
