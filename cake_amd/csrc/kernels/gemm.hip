@@ -85,10 +85,14 @@ CAKE_API long long cake_stream_capture(hipStream_t st) {
 }
 
 static inline void cfg_dims(int cfg, int& bm, int& bn) {
-  if (cfg >= k4WCfg + k4WSched && cfg <= k4WCfg128 + k4WSched) cfg -= k4WSched;  // three-barrier twins
-  if (cfg == kPPCfg || cfg == kRSCfg || cfg == k4WCfg) { bm = bn = 256; return; }
+  if (cfg == kPPCfg || cfg == kRSCfg) { bm = bn = 256; return; }
+  if (cfg >= k4WCfg + k4WSched && cfg <= k4WCfg128 + k4WSched) cfg -= k4WSched;   // the same tiles
+  if (cfg == k4WCfg) { bm = bn = 256; return; }
   if (cfg == k4WCfg192) { bm = 256; bn = 192; return; }
   if (cfg == k4WCfg128) { bm = 128; bn = 256; return; }
+#define X(id, BM, BN, WM, WN, SCHED) if (cfg == id) { bm = BM; bn = BN; return; }
+  CAKE_GEMM_4W_TILES(X)
+#undef X
 #define X(id, BM, BN, WM, WN, NS, PR) if (cfg == id) { bm = BM; bn = BN; return; }
   CAKE_GEMM_CFGS(X)
 #undef X
@@ -179,13 +183,14 @@ CAKE_API long long cake_gemm_ws_floats(int cfg, int splits, int M, int N, int K,
 }
 
 // ---- tile plan of a size that has no measured entry ------------------------
-// t(us) = c0 + step (k steps of all rounds) + lone (k steps a thin round loses to latency)
+// t(us) = c0 + step (k steps of all rounds) + lone (k steps a thin round loses to latency; four-wave
+//         tiles: gains, its operands come faster; those steps at least at the memory's rate)
 //         + epi[class] rounds + merge [split] + fin (split: MB of slabs written and read, or pieces)
-// fitted to timings of every tile and split on weights that no cache holds: 22 weight shapes (width
-// 512 .. 8192, k 512 .. 28672), 65 .. 6000 rows.  Over those 566 sizes the plan it picks is 2.4 %
-// off the best of all, at most 33 %; the nearest measured size with its split scaled was 16 % off
-// (777 x 4096 x 14336 184 us, 113 us so; 6000 rows 680, 550).  Left out: the tiles that were best
-// nowhere beyond what these reach.
+// fitted to timings on weights that no cache holds.  The four-wave tiles: 38,000 of every tile and split
+// that fills up to 256 workgroups, 38 products (width 1024 .. 8192, k 512 .. 28672), 70 .. 6000 rows.
+// Over these the plan is 5 % off the best of all tiles at 70 and 100 rows, 2.5 % from 130, 1.4 % from
+// 700 (at most 48 %).  From 300 rows on the eight-wave tiles and the 160 columns are the best nowhere by
+// more than 1 %; where four-wave tiles can run they are left out there (with them, 2 - 4 % off).
 // An image model's products are short (k from 128) or have a 16-bit residual or GEGLU: the tile's end
 // weighs as much as its k steps, so these have epilogue terms of their own, and three tiles more.
 // Over 123 sizes (width 256 .. 2048, 66 .. 18432 rows) 1.5 % off the best on the average, at most 15;
@@ -207,19 +212,37 @@ static constexpr TileCost kTileCosts[] = {
     {13, 64, 64, 2, 3.41f, 0.427f, 0.107f, {0.79f, 1.37f, 2.48f, 2.18f, 2.f, 2.05f, 1.75f}, 2.83f, 0.484f},
     {14, 64, 160, 2, 1.33f, 0.779f, 0.386f, {-1.f, -1.f, -1.f, -1.f, 5.97f, -1.f, 3.69f}, -1.f, 0.f},
     {18, 64, 160, 1, 2.28f, 0.467f, 0.f, {2.54f, 3.f, 0.f, 4.42f, 5.07f, -1.f, 3.2f}, 3.53f, 0.353f},
-    {22, 256, 256, 1, 0.f, 1.26f, 0.f, {10.9f, 15.f, 14.f, 21.7f, 18.1f, 11.4f, 12.f}, 13.2f, 10.2f},
-    {25, 256, 256, 1, 0.f, 1.49f, 0.f, {0.f, 0.f, 0.f, 0.f, 14.9f, 9.6f, 10.8f}, 20.8f, 13.2f},
-    {26, 256, 192, 1, 0.f, 1.13f, 0.f, {4.44f, 2.29f, 2.14f, 9.67f, 13.1f, 9.73f, 9.91f}, 16.1f, 6.33f},
-    {27, 128, 256, 1, 4.43f, 0.837f, 0.f, {0.0783f, 0.464f, 1.66f, 4.49f, 6.33f, 4.58f, 3.86f}, 13.7f, 4.33f},
+    {22, 256, 256, 1, 6.44f, 1.47f, -0.358f, {1.47f, 6.92f, 1.39f, 13.4f, -1.f, -1.f, -1.f}, 7.49f, 4.03f},
+    {25, 256, 256, 1, 6.3f, 1.48f, -0.326f, {2.65f, 8.21f, 2.78f, 14.1f, -1.f, -1.f, -1.f}, 7.48f, 3.77f},
+    {26, 256, 192, 1, 4.95f, 1.16f, -0.257f, {3.58f, 6.84f, 2.4f, 9.04f, -1.f, -1.f, -1.f}, 4.28f, 3.64f},
+    {27, 128, 256, 1, 4.95f, 0.852f, -0.207f, {1.05f, 3.4f, 1.26f, 5.45f, -1.f, -1.f, -1.f}, 4.05f, 2.27f},
+    {28, 128, 128, 1, 3.28f, 0.524f, -0.165f, {1.86f, 3.55f, 1.92f, 3.92f, -1.f, -1.f, -1.f}, 2.48f, 1.91f},
+    {29, 128, 192, 1, 3.45f, 0.686f, -0.167f, {3.17f, 4.18f, 2.68f, 6.09f, -1.f, -1.f, -1.f}, 3.29f, 1.99f},
+    {30, 96, 256, 1, 5.21f, 0.765f, -0.157f, {0.277f, 1.17f, 0.662f, 3.95f, -1.f, -1.f, -1.f}, 3.01f, 1.9f},
+    {31, 160, 256, 1, 3.56f, 0.948f, -0.261f, {4.f, 7.49f, 3.83f, 9.4f, -1.f, -1.f, -1.f}, 3.91f, 2.7f},
+    {32, 192, 192, 1, 2.11f, 0.83f, -0.223f, {6.11f, 8.94f, 5.05f, 10.1f, -1.f, -1.f, -1.f}, 3.34f, 2.76f},
+    {33, 224, 192, 1, 2.17f, 0.923f, -0.265f, {7.53f, 11.f, 5.97f, 12.f, -1.f, -1.f, -1.f}, 3.06f, 3.14f},
+    {34, 192, 256, 1, 6.79f, 1.23f, -0.245f, {0.621f, 4.06f, 1.1f, 7.72f, -1.f, -1.f, -1.f}, 4.24f, 3.18f},
+    {35, 224, 256, 1, 6.34f, 1.35f, -0.274f, {1.79f, 6.43f, 2.28f, 10.1f, -1.f, -1.f, -1.f}, 4.48f, 3.65f},
+    // four-wave tiles, the classes from kImageClass on
+    {22, 256, 256, 1, 0.f, 1.26f, 0.f, {-1.f, -1.f, -1.f, -1.f, 18.1f, 11.4f, 12.f}, 13.2f, 10.2f},
+    {25, 256, 256, 1, 0.f, 1.49f, 0.f, {-1.f, -1.f, -1.f, -1.f, 14.9f, 9.6f, 10.8f}, 20.8f, 13.2f},
+    {26, 256, 192, 1, 0.f, 1.13f, 0.f, {-1.f, -1.f, -1.f, -1.f, 13.1f, 9.73f, 9.91f}, 16.1f, 6.33f},
+    {27, 128, 256, 1, 4.43f, 0.837f, 0.f, {-1.f, -1.f, -1.f, -1.f, 6.33f, 4.58f, 3.86f}, 13.7f, 4.33f},
 };
+// 0 .. 6, as TileCost::epi; from kImageClass on the products of image models
+static constexpr int kImageClass = 4;
+static int cost_class(int epi, int K) {
+  return epi == kEpiResid32 || epi == kEpiStore32                 ? 1
+         : epi == kEpiSwiglu                                      ? 2
+         : epi == kEpiSilu || epi == kEpiQuick || epi == kEpiGelu ? 3
+         : epi == kEpiAdd16                                       ? 4
+         : epi == kEpiGeglu                                       ? 5
+         : epi == kEpiStore && K < 512                            ? 6 : 0;
+}
 static double tile_cost(const TileCost& c, int splits, long long M, long long Nv, int K, int epi) {
   const long long ks = (K + kGBK - 1) / kGBK, t = ((M + c.bm - 1) / c.bm) * ((Nv + c.bn - 1) / c.bn);
-  const int cls = epi == kEpiResid32 || epi == kEpiStore32                 ? 1
-                  : epi == kEpiSwiglu                                      ? 2
-                  : epi == kEpiSilu || epi == kEpiQuick || epi == kEpiGelu ? 3
-                  : epi == kEpiAdd16                                       ? 4
-                  : epi == kEpiGeglu                                       ? 5
-                  : epi == kEpiStore && K < 512                            ? 6 : 0;
+  const int cls = cost_class(epi, K);
   if (c.epi[cls] < 0 || (splits > 1 && c.merge < 0)) return -1;   // not modelled
   double steps, rounds, lone = 0, fin = 0;
   bool split = false;
@@ -232,6 +255,7 @@ static double tile_cost(const TileCost& c, int splits, long long M, long long Nv
     rounds = (double)(dp + (rest ? 1 : 0));
     split = p.pieces > 0;
     fin = p.pieces;
+    if (rest) lone = per * (1 - (double)rest * std::max(p.pieces, 1) / 256);
   } else {
     const long long kps = (ks + splits - 1) / splits, sp = (ks + kps - 1) / kps, n = t * sp;
     const long long full = n / (256 * c.slots), rest = n % (256 * c.slots);
@@ -242,8 +266,9 @@ static double tile_cost(const TileCost& c, int splits, long long M, long long Nv
     split = sp > 1;
     if (split) fin = (double)(sp + 1) * M * Nv * 4e-6;
   }
-  const double us = c.c0 + c.step * steps + c.lone * lone + c.epi[cls] * rounds +
-                    (split ? c.merge + c.fin * fin : 0.);
+  double main = c.step * steps + c.lone * lone;
+  if (four_wave_cfg(c.cfg)) main = std::max(main, ((double)Nv * K + (double)M * K) * 2 / 5.2e6);
+  const double us = c.c0 + main + c.epi[cls] * rounds + (split ? c.merge + c.fin * fin : 0.);
   // operands from memory; of tiles that all wait for them the one with the least work (113 x 57344 x
   // 8192 SwiGLU 193 us on 128 x 256, 209 on 128 x 128)
   return std::max(us, ((double)Nv * K + (double)M * K) * 2 / 5e6 + 3) + 0.02 * us;
@@ -262,14 +287,18 @@ CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* c
   int bc = 0, bs = 1;
   for (const TileCost& c : kTileCosts) {
     const bool four = four_wave_cfg(c.cfg);
-    if (c.cfg == *cfg) given = tile_cost(c, *splits, M, Nv, K, epi);
+    if (c.cfg == *cfg) given = std::max(given, tile_cost(c, *splits, M, Nv, K, epi));
     if (four && (K % kGBK || big)) continue;
     if (gated && c.cfg == 18) continue;               // 80-column wave tiles
+    if (M >= 300 && K % kGBK == 0 && !big && cost_class(epi, K) < kImageClass &&
+        (c.cfg == 5 || c.cfg == 6 || c.cfg == 7 || c.cfg == 18))
+      continue;
     // long rows of k: the three-barrier schedule of the 256 x 256 tile (8192 x 28672 at 2048 rows
     // 726 against 800 us), else the two-stage one (8192 x 8192 199 against 206)
     if ((c.cfg == k4WCfg && K > 8192) || (c.cfg == k4WCfg + k4WSched && K <= 8192)) continue;
-    for (int sp = 1; sp <= 16; sp *= 2) {
+    for (int sp : {1, 2, 3, 4, 6, 8, 16}) {
       if (sp > 1 && (ks / sp < 4 || (four && M < 200))) break;
+      if (!four && (sp & (sp - 1))) continue;
       const double t = tile_cost(c, sp, M, Nv, K, epi);
       if (t >= 0 && t < best) {
         best = t;

@@ -1,5 +1,5 @@
-// Four-wave MFMA GEMM tiles 256x256 / 256x192 / 128x256 (plan cfg 22-24, and 25-27 on the
-// three-barrier schedule): the large Llama prefill projections.
+// Four-wave MFMA GEMM tiles (plan cfg 22-35; shapes and schedules below): the projections of
+// prompts.
 //
 // Included by gemm_kernel.h (launch_gemm dispatches cfg 22-27 here); same GemmArgs, tile
 // order, swizzled LDS image, fragment reads and epilogues as gemm_kernel's IL path.
@@ -9,8 +9,8 @@
 // staging, 32 fragment reads per k-step.  At one wave per SIMD every instruction beside
 // the MFMAs is paid in MFMA gaps (16 cycles, 8 of them free), so a DMA piece is three
 // instructions and nothing else (k-loop stamps: profiles/r6_gemm_stamps.jsonl):
-//   * buffer_load_dwordx4 ... offen lds with one per-lane byte offset VGPR per operand (the
-//     lane's row in its 32-row group and its swizzled 16-byte chunk) and the group's row
+//   * buffer_load_dwordx4 ... offen lds with two per-lane byte offset VGPRs per operand (the
+//     lane's row of an instruction's eight and its swizzled 16-byte chunk) and the rows'
 //     offset as a loop-invariant scalar soffset;
 //   * the k step in the descriptor: its base advanced and num_records shrunk per step (a
 //     handful of scalar ops per step, not per piece); rows past the matrix and steps past
@@ -44,8 +44,9 @@ constexpr int k4WCfg = 22;     // plan cfg id of the 256 x 256 tile
 constexpr int k4WCfg192 = 23;  // 256 x 192 (8B q|k|v: 6144 = 32 x 192 columns, 256 tiles at
                                // 2048 tokens instead of 192)
 constexpr int k4WCfg128 = 24;  // 128 x 256 (8B o / down at 2048 tokens: 256 tiles, not 128)
-constexpr int k4WSched = 3;    // cfg + 3: the same tiles on the three-barrier schedule (25-27)
-inline bool four_wave_cfg(int cfg) { return cfg >= k4WCfg && cfg <= k4WCfg128 + k4WSched; }
+constexpr int k4WSched = 3;    // cfg + 3: the same tiles on three barriers (25, 26), on one (27)
+constexpr int k4WLast = 35;    // 28 .. 35: the tiles of CAKE_GEMM_4W_TILES
+inline bool four_wave_cfg(int cfg) { return cfg >= k4WCfg && cfg <= k4WLast; }
 // op k of an alternating sequence of nr reads and nd DMAs (the longer list's tail last):
 // kind 0 = read, 1 = DMA, and its index within its list
 constexpr int alt_kind(int nr, int nd, int k) {
@@ -84,8 +85,12 @@ __device__ __forceinline__ void amfma_dma(cf32x4& acc, const uint4& a, const uin
                  : "memory", "scc");
 }
 
-// SCHED 1 (cfg 25-27): the same tiles on a three-barrier schedule (the DMAs of step t+2
-// issued as soon as every wave has read the operand region they overwrite).
+// SCHED 1: three barriers a k step (the DMAs of step t+2 issued as soon as every wave has read the
+// operand region they overwrite).  SCHED 2: one barrier, for tiles of which the LDS holds three or
+// four k steps.  A step of a small tile is bound by its waits, not by the matrix cores: 192 x 192 is
+// 0.49 us of MFMAs and took 0.75 us alone on the chip (0.63 with one barrier), 1.13 on all CUs (0.98);
+// 128 x 256 0.44, 0.72 (0.62), 1.11 (0.99).  More steps in flight alone changed neither.  Tiles of
+// two steps (256 x 192 and larger) are within 3 % either way.
 // GRP: grouped row tiles (GemmArgs::groups), K any multiple of 8.  Bound by the matrix cores on
 // padded rows and, below some 200 rows a group, by reading the weights: 64 groups of 192 rows,
 // 4096 -> 3616 -> 4096 columns, 1102 -> 989 us against eight waves on the same tile (0.98 PFLOP/s
@@ -95,16 +100,17 @@ __device__ __forceinline__ void amfma_dma(cf32x4& acc, const uint4& a, const uin
 // the residual 113.3 us with them, 109.9 without).
 template <int DT, int EPI, int BM, int BN, int SCHED = 0, bool GRP = false, bool PCS = false>
 __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
-  static_assert((BM == 256 && (BN == 256 || BN == 192)) || (BM == 128 && BN == 256),
-                "four-wave tile shapes");
+  static_assert(BM % 32 == 0 && BN % 64 == 0, "whole fragments, gated pairs within a wave");
   constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
-  constexpr int BUF = (BM + BN) * 128;  // 64 / 56 / 48 KB per k-step buffer
+  constexpr int BUF = (BM + BN) * 128;  // 64 KB at most per k-step buffer
+  constexpr int NBUF = SCHED != 2 ? 2 : 160 * 1024 / BUF > 4 ? 4 : 160 * 1024 / BUF;
+  static_assert(SCHED != 2 || NBUF > 2, "one barrier a step: three steps in the LDS");
   constexpr int IPW = (BM + BN) / 32;   // DMA wave-instructions per wave per k-step
   constexpr int NA = BM / 32;           // of which A
   static_assert(IPW == FM + FN, "the second half alternates one DMA with one fragment read");
   constexpr int STG_LD = WTN + 4, STG = 16 * STG_LD * 4;
-  static_assert(8 * STG <= 2 * BUF - 16, "epilogue staging (2 slices per wave) fits the operand buffers");
-  __shared__ __attribute__((aligned(16))) uint8_t smem[2 * BUF];
+  static_assert(8 * STG <= NBUF * BUF - 16, "epilogue staging (2 slices per wave) fits the operand buffers");
+  __shared__ __attribute__((aligned(16))) uint8_t smem[NBUF * BUF];
 
   const int tid = threadIdx.x, lane = tid & 63;
 #ifdef CAKE_GEMM_STAMPS
@@ -119,26 +125,24 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   // in equal k pieces — the last partial wave of a grid at a fraction of its length (8B gate|up
   // at 2048 tokens: 896 tiles = 3 full waves + 128 tiles in halves), or every tile in pieces
   // when there are too few.  Equal pieces of all tiles walk k side by side and share their
-  // operands in L2; one line of k steps cut into 256 equal shares (a tile's pieces at any k)
+  // operands in L2, so an XCD takes neighbouring tiles of one piece (with the pieces of a tile side
+  // by side it read most of both operands: 1100 x 4096 x 23552 in 224 x 192 tiles 203 us, 191 so); one line of k steps cut into 256 equal shares (a tile's pieces at any k)
   // balanced better and ran at half the rate, every workgroup reading for itself.
   if constexpr (GRP) g.tiles_m = g.groups[g.tiles_m].x;
   const int ntiles = g.tiles_m * g.tiles_n;
   if (GRP && (int)blockIdx.x >= ntiles) return;
-  int id, split = blockIdx.y, piece = 0;
-  int kb = split * g.kps, ke = min(g.K, kb + g.kps);
+  int id, piece = 0;
+  int kb = 0, ke = g.K;
   {
-    const int bid = blockIdx.x;
-    const int dp = PCS ? g.dp_tiles : ntiles;
-    if (!PCS || bid < dp) {
-      const int q = dp / 8, r = dp % 8, x = bid % 8, i = bid / 8;
-      id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
-      if constexpr (PCS) {  // a whole tile
-        kb = 0;
-        ke = g.K;
-      }
-    } else {
-      id = dp + (bid - dp) / g.pieces;
-      piece = (bid - dp) % g.pieces;
+    const int dp = PCS ? g.dp_tiles : ntiles;   // (a multiple of 8 where pieces follow)
+    const bool whole = !PCS || (int)blockIdx.x < dp;
+    const int n = whole ? dp : (int)gridDim.x - dp, bid = whole ? blockIdx.x : blockIdx.x - dp;
+    const int q = n / 8, r = n % 8, x = bid % 8, i = bid / 8;
+    id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
+    if (PCS && !whole) {   // the first pieces of all these tiles, then the second ones, ..
+      const int rest = n / g.pieces;
+      piece = id / rest;
+      id = dp + id % rest;
       kb = piece * g.kps;
       ke = min(g.K, kb + g.kps);
     }
@@ -163,25 +167,34 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   }
   const int nk = GRP ? (ke - kb + kGBK - 1) / kGBK : (ke - kb) / kGBK;
 
-  // ---- DMA: instruction i of this wave fills LDS rows i*32 + wave*8 + [0, 8) (A rows
-  // for i < NA, B rows after); lane l -> row + l/8, slot l%8 holding source chunk
-  // (l%8) ^ ((row >> 1) & 7), the same for every i
-  const int rA = wave * 8 + (lane >> 3);
-  const int chunk = (lane & 7) ^ ((rA >> 1) & 7);
+  // ---- DMA: an instruction fills 8 LDS rows, lane l row l/8, slot l%8 of it holding source chunk
+  // (l%8) ^ ((row >> 1) & 7).  A wave's instructions take rows side by side, 8 NA of A and 8 NB of B:
+  // with the waves' rows 8 apart (one 32-row group an instruction) the rows in flight at a time met on
+  // few channels of the memory where k is an odd multiple of 1024 or so (8 x 32 tiles of 128 x 256, k
+  // 5120 95 -> 77 us, 23552 364 -> 340, 28672 460 -> 402; 256 x 256 148 -> 130, 624 -> 588, 805 -> 699)
+  constexpr int NB = IPW - NA;
+  const int l8 = lane >> 3;
+  const int rA = wave * (NA * 8) + l8, rB = wave * (NB * 8) + l8;
+  const int chunk_a = (lane & 7) ^ ((rA >> 1) & 7), chunk_b = (lane & 7) ^ ((rB >> 1) & 7);
   // (grouped: weights from this tile's first row on, so that a tile, not a weight, is under 2 GB)
   const long long brows = GRP ? min(BN, g.Nv - n0) : g.gated ? 2LL * g.half : (long long)g.Nv;
   const int nrec_a = (int)(((long long)(g.M - 1) * g.lda + g.K) * 2);
   const int nrec_b = (int)(((brows - 1) * g.ldb + g.K) * 2);
-  const uint32_t voff_a = (uint32_t)(((long long)(m0 + rA) * g.lda + chunk * 8) * 2);
-  long long brow0;  // weight row of this lane in B group 0
-  if constexpr (GRP) brow0 = rA;
-  else if (!g.gated) brow0 = n0 + rA;
-  else brow0 = (rA < 16 ? 0LL : (long long)g.half - 16) + n0 / 2 + rA;
-  const uint32_t voff_b = (uint32_t)((brow0 * g.ldb + chunk * 8) * 2);
-  // scalar byte offsets of each 32-row group (A: 32 rows; B: 32 virtual rows = 16
-  // weight rows of each half when gated): loop-invariant SGPRs
-  const uint32_t gstride_a = (uint32_t)(32LL * g.lda * 2);
-  const uint32_t gstride_b = (uint32_t)((g.gated ? 16LL : 32LL) * g.ldb * 2);
+  // scalar byte offsets of each instruction's rows: loop-invariant SGPRs.  Gated: virtual rows 32 b ..
+  // are 16 gate rows from 16 b on and the 16 up rows beside them
+  const uint32_t gstride_a = (uint32_t)(8LL * g.lda * 2);
+  uint32_t soff_b[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int q = wave * NB + j;
+    const long long row = !g.gated ? 8 * j : q / 4 * 16 + q % 2 * 8 + (q % 4 < 2 ? 0 : g.half);
+    soff_b[j] = __builtin_amdgcn_readfirstlane((uint32_t)(row * g.ldb * 2));
+  }
+  const long long brow0 = GRP ? rB : g.gated ? n0 / 2 + l8 : n0 + rB;
+  // byte offsets of this lane, of the even and the odd instructions (rows 8 on: the chunk's bit 2)
+  const auto voff = [](long long row, long long ld, int chunk) { return (uint32_t)((row * ld + chunk * 8) * 2); };
+  const uint32_t voff_a[2] = {voff(m0 + rA, g.lda, chunk_a), voff(m0 + rA, g.lda, chunk_a ^ 4)};
+  const uint32_t voff_b[2] = {voff(brow0, g.ldb, chunk_b), voff(brow0, g.ldb, chunk_b ^ 4)};
   // The k step lives in the descriptors: base advanced to the step's first column and
   // num_records shrunk by as much (a step past the split's end: 0 records, every lane out
   // of range -> zeros, no memory traffic).  Per DMA that leaves the M0 write and the DMA
@@ -199,36 +212,42 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   };
   auto src_a = [&](int step) __attribute__((always_inline)) { return desc_at(g.a, nrec_a, step); };
   auto src_b = [&](int step) __attribute__((always_inline)) { return desc_at(g.b, nrec_b, step); };
-  const uint32_t m0_base = __builtin_amdgcn_readfirstlane(lds_off(smem) + (uint32_t)wave * 1024);
-  // M0 (= buffer base + 4 KiB per piece, the piece offset an immediate) / voffset / soffset
+  const uint32_t m0_a = __builtin_amdgcn_readfirstlane(lds_off(smem) + (uint32_t)wave * (NA * 1024));
+  const uint32_t m0_b = __builtin_amdgcn_readfirstlane(lds_off(smem) + BM * 128u + (uint32_t)wave * (NB * 1024));
+  // M0 (= buffer base + 1 KiB per piece, the piece offset an immediate) / voffset / soffset
   // of DMA I (A pieces for I < NA) into buffer buf
-  auto dma_mb = [&](int buf) __attribute__((always_inline)) {
-    return m0_base + (uint32_t)(buf * BUF);
+  auto dma_mb = [&](int buf, int i) __attribute__((always_inline)) {
+    return (i < NA ? m0_a : m0_b) + (uint32_t)(buf * BUF);
   };
   // GRP: the last step of a K that is no multiple of 64 reads its missing chunks out of range
   // (the descriptors only bound the matrix, a row's end lies inside it)
-  uint32_t cur_a = voff_a, cur_b = voff_b;
+  uint32_t cur_a[2] = {voff_a[0], voff_a[1]}, cur_b[2] = {voff_b[0], voff_b[1]};
   auto tail_step = [&](int step) __attribute__((always_inline)) {
     if constexpr (GRP) {
-      const bool in = step * kGBK + chunk * 8 < g.K;
-      cur_a = in ? voff_a : 0x80000000u;
-      cur_b = in ? voff_b : 0x80000000u;
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        cur_a[o] = step * kGBK + (chunk_a ^ 4 * o) * 8 < g.K ? voff_a[o] : 0x80000000u;
+        cur_b[o] = step * kGBK + (chunk_b ^ 4 * o) * 8 < g.K ? voff_b[o] : 0x80000000u;
+      }
     }
   };
-  auto dma_voff = [&](int i) __attribute__((always_inline)) { return i < NA ? cur_a : cur_b; };
+  auto dma_voff = [&](int i) __attribute__((always_inline)) {
+    return i < NA ? cur_a[i % 2] : cur_b[(i - NA) % 2];
+  };
   auto dma_soff = [&](int i) __attribute__((always_inline)) {
-    return i < NA ? (uint32_t)i * gstride_a : (uint32_t)(i - NA) * gstride_b;
+    return i < NA ? (uint32_t)i * gstride_a : soff_b[i < NA ? 0 : i - NA];
   };
   auto stage_one = [&](const cu32x4& sa, const cu32x4& sb, int buf, auto I)
                        __attribute__((always_inline)) {
     constexpr int i = decltype(I)::value;
-    dma16<i * 4096>(dma_mb(buf), dma_voff(i), i < NA ? sa : sb, dma_soff(i));
+    dma16<(i < NA ? i : i - NA) * 1024>(dma_mb(buf, i), dma_voff(i), i < NA ? sa : sb, dma_soff(i));
   };
   // MFMA with DMA I fused behind it
   auto mfma_dma = [&](cf32x4& c, const uint4& a, const uint4& b, const cu32x4& sa,
                       const cu32x4& sb, int buf, auto I) __attribute__((always_inline)) {
     constexpr int i = decltype(I)::value;
-    amfma_dma<DT, i * 4096>(c, a, b, dma_mb(buf), dma_voff(i), i < NA ? sa : sb, dma_soff(i));
+    amfma_dma<DT, (i < NA ? i : i - NA) * 1024>(c, a, b, dma_mb(buf, i), dma_voff(i), i < NA ? sa : sb,
+                                                dma_soff(i));
   };
   auto stage = [&](int step, int buf) {
     const cu32x4 sa = src_a(step), sb = src_b(step);
@@ -249,7 +268,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   const uint32_t lds0 = lds_off(smem);
   const uint32_t a_base = lds0 + (uint32_t)(wr * WTM) * 128 + lrow;
   const uint32_t b_base = lds0 + (uint32_t)(BM + wc * WTN) * 128 + lrow;
-  constexpr int NM = FM * FN, NR = FM + FN, NB = IPW - NA;
+  constexpr int NM = FM * FN, NR = FM + FN;
   uint4 af0[FM], bf0[FN], af1[FM], bf1[FN];
 
   if constexpr (SCHED == 1) {
@@ -349,6 +368,78 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       // the last MFMAs' results settle before the loop is left: a spill may read them first thing
       // (on every step: asked for on the last one only, the branch cost whole tiles that leave the
       // clock up to 9 %, 2048 x 4096 x 14336 281 us against 257)
+      asm volatile("s_nop 7" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      buf = nbuf;
+    }
+  } else if constexpr (SCHED == 2) {
+    // One barrier a k step, early in its second half: by then every wave has read all of step t (its
+    // buffer takes step t + NBUF) and waits for its own DMAs of step t+1.
+    //   first half: MFMAs of k 0..31, reads of k 32..63
+    //   second half: MFMAs of k 32..63, after the P-th of them vmcnt + barrier, then reads of
+    //     k 0..31 of t+1
+    // The reads end LAT MFMAs before their half does (their latency); the DMAs of a step are spread
+    // from barrier to barrier, ND2 of them before the next step begins.
+    constexpr int P = 2, LAT = NM >= 48 ? 9 : 7;
+    constexpr int R1 = NM - LAT, W2 = NM - P - 1, R2 = W2 - LAT;   // MFMAs that reads, DMAs follow
+    constexpr int ND2 = IPW / 2, ND1 = IPW - ND2;
+    static_assert(R2 >= NR / 2 && W2 >= ND2, "op density");
+    static_for<0, NBUF - 1>([&](auto i) __attribute__((always_inline)) { stage(i, i); });
+    {  // the first part of the last buffered step, as the loop leaves it
+      const cu32x4 sa = src_a(NBUF - 1), sb = src_b(NBUF - 1);
+      tail_step(NBUF - 1);
+      static_for<0, ND2>([&](auto I) __attribute__((always_inline)) { stage_one(sa, sb, NBUF - 1, I); });
+    }
+    __builtin_amdgcn_s_waitcnt(vm_wait((NBUF - 2) * IPW + ND2));
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < FM; ++i) af0[i] = ds_read16(a_base + i * 16 * 128 + off0);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) bf0[j] = ds_read16(b_base + j * 16 * 128 + off0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    int buf = 0;
+    cu32x4 sa = src_a(NBUF - 1), sb = src_b(NBUF - 1);
+    for (int t = 0; t < nk; ++t) {
+      const uint32_t ab = a_base + buf * BUF, bb = b_base + buf * BUF;
+      const int nbuf = buf + 1 == NBUF ? 0 : buf + 1, pbuf = buf == 0 ? NBUF - 1 : buf - 1;
+      const uint32_t na = a_base + nbuf * BUF, nb = b_base + nbuf * BUF;
+      tail_step(t + NBUF - 1);
+      static_for<0, NM>([&](auto mi) __attribute__((always_inline)) {
+        constexpr int m = decltype(mi)::value;
+        constexpr int d0 = (m * ND1 + NM - 1) / NM, d1 = ((m + 1) * ND1 + NM - 1) / NM;
+        if constexpr (d0 < d1) mfma_dma(acc[m / FN][m % FN], af0[m / FN], bf0[m % FN], sa, sb, pbuf, std::integral_constant<int, ND2 + d0>{});
+        else amfma_v<DT>(acc[m / FN][m % FN], af0[m / FN], bf0[m % FN]);
+        if constexpr (m < R1)
+          static_for<(m * NR + R1 - 1) / R1, ((m + 1) * NR + R1 - 1) / R1>([&](auto ri) __attribute__((always_inline)) {
+            constexpr int r = decltype(ri)::value;
+            if constexpr (r < FN) bf1[r] = ds_read16_off<r * 16 * 128>(bb + off1);
+            else af1[r - FN] = ds_read16_off<(r - FN) * 16 * 128>(ab + off1);
+          });
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      sa = src_a(t + NBUF);
+      sb = src_b(t + NBUF);
+      tail_step(t + NBUF);
+      static_for<0, NM>([&](auto mi) __attribute__((always_inline)) {
+        constexpr int m = decltype(mi)::value, mm = m - P - 1;
+        constexpr int d0 = mm < 0 ? 0 : (mm * ND2 + W2 - 1) / W2, d1 = mm < 0 ? 0 : ((mm + 1) * ND2 + W2 - 1) / W2;
+        if constexpr (d0 < d1) mfma_dma(acc[m / FN][m % FN], af1[m / FN], bf1[m % FN], sa, sb, buf, std::integral_constant<int, d0>{});
+        else amfma_v<DT>(acc[m / FN][m % FN], af1[m / FN], bf1[m % FN]);
+        if constexpr (m == P) {
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_waitcnt(vm_wait((NBUF - 2) * IPW));
+          asm volatile("s_barrier" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+        } else if constexpr (mm >= 0 && mm < R2)
+          static_for<(mm * NR + R2 - 1) / R2, ((mm + 1) * NR + R2 - 1) / R2>([&](auto ri) __attribute__((always_inline)) {
+            constexpr int r = decltype(ri)::value;
+            if constexpr (r < FN) bf0[r] = ds_read16_off<r * 16 * 128>(nb + off0);
+            else af0[r - FN] = ds_read16_off<(r - FN) * 16 * 128>(na + off0);
+          });
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       asm volatile("s_nop 7" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       buf = nbuf;
@@ -457,7 +548,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
     const int tile = id - g.dp_tiles;
     unsigned* tk = g.tick + tile;
     unsigned* fl = g.tick + kPieceTiles + tile;
-    volatile uint32_t* bc = reinterpret_cast<volatile uint32_t*>(smem + 2 * BUF - 16);
+    volatile uint32_t* bc = reinterpret_cast<volatile uint32_t*>(smem + NBUF * BUF - 16);
     if (tid == 0) bc[0] = __hip_atomic_fetch_add(tk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const bool last = bc[0] == (uint32_t)(pieces - 1);
@@ -509,7 +600,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
         stage_strip_w<FN>(acc[i + 1], (i & 1) ? sg0 : sg1, lane, add.strip(i + 1, FN));
         ops.template load_res<(i + 1) & 1>(g, row_m0 + (i + 1) * 16, vcol0, lane);
       }
-      readout_strip_w<DT, EPI, FN, i & 1>(g, (i & 1) ? sg1 : sg0, row_m0 + i * 16, vcol0, split,
+      readout_strip_w<DT, EPI, FN, i & 1>(g, (i & 1) ? sg1 : sg0, row_m0 + i * 16, vcol0, 0,
                                           lane, ops);
     });
 #ifdef CAKE_GEMM_STAMPS
@@ -524,7 +615,7 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       constexpr int i = decltype(ii)::value;
       if constexpr (i + 1 < FM)
         ops.template load_res<(i + 1) & 1>(g, row_m0 + (i + 1) * 16 + (lane >> 2), vcol0, lane);
-      epi_strip<DT, EPI, FN, i & 1>(g, acc[i], stg, row_m0 + i * 16, vcol0, split, lane, ops,
+      epi_strip<DT, EPI, FN, i & 1>(g, acc[i], stg, row_m0 + i * 16, vcol0, 0, lane, ops,
                                     add.strip(i, FN));
     });
   }

@@ -994,6 +994,20 @@ __global__ __launch_bounds__(256) void gemm_splitk_finalize(GemmArgs g, int spli
   X(17, 128, 160, 2, 2, 2, 6) \
   X(18, 64, 160, 2, 2, 3, 6) \
   X(19, 128, 160, 2, 2, 3, 6)
+// ... and of gemm_4w.h's further tiles (BM, BN, WM, WN, schedule).  Rows come in any number, and
+// padded rows and a last, partial wave of tiles cost as much as whole ones: 1100 x 4096 x 23552 in
+// 224 x 192 tiles 210 us, in 256 x 192 247; 777 x 6144 x 4096 in 128 x 192 45 us, in 256 x 128 55;
+// 777 x 4096 x 4096 in 128 x 128 36 us, 42 in cfg 7; 1455 x 4096 x 23552 in 192 x 256 269 us, in
+// 256 x 128 324; 300 x 14336 x 4096 SwiGLU in 160 x 256 79 us, in 256 x 256 106.
+#define CAKE_GEMM_4W_TILES(X) \
+  X(28, 128, 128, 2, 2, 2)    \
+  X(29, 128, 192, 2, 2, 2)    \
+  X(30, 96, 256, 2, 2, 2)     \
+  X(31, 160, 256, 2, 2, 2)    \
+  X(32, 192, 192, 2, 2, 2)    \
+  X(33, 224, 192, 2, 2, 2)    \
+  X(34, 192, 256, 2, 2, 1)    \
+  X(35, 224, 256, 2, 2, 1)
 
 }  // namespace cake
 
@@ -1008,22 +1022,47 @@ constexpr bool gated_ok(int wave_cols) {
   return wave_cols % 32 == 0 || !(EPI == kEpiSwiglu || EPI == kEpiGeglu);
 }
 
-template <int DT, int EPI, bool PCS>
-int launch_4w(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
-#define X(ID, BM, BN, SCHED)                                                                   \
+// PCS: some tiles run in pieces (GemmArgs::pieces)
+#define CAKE_LAUNCH_4W(ID, BM, BN, WM, WN, SCHED)                                                      \
   if (cfg == ID) {                                                                             \
     hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, BM, BN, SCHED, false, PCS>), grid, dim3(256),  \
                        0, st, g);                                                              \
     return (int)hipGetLastError();                                                             \
   }
-  X(k4WCfg, 256, 256, 0) X(k4WCfg192, 256, 192, 0) X(k4WCfg128, 128, 256, 0)
-  X(k4WCfg + k4WSched, 256, 256, 1) X(k4WCfg192 + k4WSched, 256, 192, 1)
-  X(k4WCfg128 + k4WSched, 128, 256, 1)
-#undef X
+// gemm_inst_tiles_*.hip
+template <int DT, int EPI, bool PCS>
+int launch_tiles(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  CAKE_GEMM_4W_TILES(CAKE_LAUNCH_4W)
+  return (int)hipErrorInvalidValue;
+}
+#define CAKE_TILES_EXTERN(DT, E)                                                              \
+  extern template int launch_tiles<DT, E, false>(int, dim3, hipStream_t, const GemmArgs&);     \
+  extern template int launch_tiles<DT, E, true>(int, dim3, hipStream_t, const GemmArgs&);
+#define CAKE_TILES_EXTERN_ALL(DT) CAKE_TILES_EXTERN(DT, kEpiStore) CAKE_TILES_EXTERN(DT, kEpiResid32) \
+  CAKE_TILES_EXTERN(DT, kEpiAdd16) CAKE_TILES_EXTERN(DT, kEpiSwiglu) CAKE_TILES_EXTERN(DT, kEpiGeglu) \
+  CAKE_TILES_EXTERN(DT, kEpiStore32) CAKE_TILES_EXTERN(DT, kEpiSilu) CAKE_TILES_EXTERN(DT, kEpiQuick) \
+  CAKE_TILES_EXTERN(DT, kEpiGelu) CAKE_TILES_EXTERN(DT, kEpiRelu2)
+CAKE_TILES_EXTERN_ALL(kBF16)
+CAKE_TILES_EXTERN_ALL(kF16)
+#undef CAKE_TILES_EXTERN_ALL
+#undef CAKE_TILES_EXTERN
+
+template <int DT, int EPI, bool PCS>
+int launch_4w(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  // (a four-wave tile's k split is its pieces: no partial slabs)
+  if constexpr (EPI != kEpiPartial) {
+    CAKE_LAUNCH_4W(k4WCfg, 256, 256, 2, 2, 0)
+    CAKE_LAUNCH_4W(k4WCfg192, 256, 192, 2, 2, 0)
+    CAKE_LAUNCH_4W(k4WCfg128, 128, 256, 2, 2, 0)
+    CAKE_LAUNCH_4W(k4WCfg + k4WSched, 256, 256, 2, 2, 1)
+    CAKE_LAUNCH_4W(k4WCfg192 + k4WSched, 256, 192, 2, 2, 1)
+    CAKE_LAUNCH_4W(k4WCfg128 + k4WSched, 128, 256, 2, 2, 2)
+    return launch_tiles<DT, EPI, PCS>(cfg, grid, st, g);
+  }
   return (int)hipErrorInvalidValue;
 }
 
-// four-wave tiles of which some run in pieces (GemmArgs::pieces)
+// four-wave tiles of which some run in pieces
 template <int DT, int EPI>
 int launch_pieces(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
   return launch_4w<DT, EPI, true>(cfg, grid, st, g);

@@ -1,0 +1,33 @@
+"""Four-wave tiles of every height and width (gemm_4w.h): edges, short k, pieces, gated pairs."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# one k step up to more than a buffer holds; rows and columns one off the tile's edge; in pieces
+@pytest.mark.parametrize("cfg", range(27, 36))
+@pytest.mark.parametrize("rows,cols,K,splits", [(-1, 1, 64, 1), (1, -3, 192, 1), (0, 0, 320, 1), (3, 5, 1088, 4)])
+@pytest.mark.parametrize("epi", ["store", "resid32", "swiglu"])
+def test_tile_edges(cuda, cfg, rows, cols, K, splits, epi):
+    """f32 sums of 16-bit products, in two orders, one rounding to bf16 (of gate, up and result in the
+    gated form); the same bits every time."""
+    from cake_amd.ops import gemm as G
+    bm, bn = G.CFG_TILES[cfg]
+    M, N = 2 * bm + rows, 3 * bn + cols
+    if epi == "swiglu":
+        N = 2 * (N // 32 * 16)
+    g = torch.Generator(device="cuda").manual_seed(cfg + K)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    y = x.float() @ w.float().t()
+    if epi == "swiglu":
+        y = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+    outs = []
+    for _ in range(2):
+        r = torch.zeros(M, N, device="cuda") if epi == "resid32" else None
+        outs.append(G.linear(x, w, epi=epi, resid=r, cfg=cfg, splits=splits))
+    assert torch.equal(outs[0], outs[1])
+    tol = K * 2.0 ** -21 + (2.0 ** -16 if epi == "resid32" else 2.0 ** -8)
+    scale = y.pow(2).mean().sqrt() + y.abs()
+    assert bool(((outs[0].float() - y).abs() <= tol * scale).all())
