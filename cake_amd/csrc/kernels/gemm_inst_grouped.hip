@@ -7,21 +7,31 @@ namespace cake {
 
 constexpr long long kWide = 1 << 22;  // elements: 256 rows of this stride are 2 GB
 
-// Tiles by rows: 64 (cfg 4), 128 (0), 256 (5); the last two on four waves (gemm_4w.h).  Rows too
-// far apart for its 32-bit offsets take the 64-row tile, in passes.
+// Tiles by rows, of 256 columns on four waves (gemm_4w.h); cfg 4: 64 x 64
+constexpr int grouped_rows(int cfg) {
+  return cfg == 4 ? 64 : cfg == 0 ? 128 : cfg == 1 ? 160 : cfg == 2 ? 192 : cfg == 5 ? 256 : 0;
+}
+
+// Rows too far apart for the four waves' 32-bit offsets take the 64-row tile, in passes.
 template <int DT, int EPI>
 static int launch_grouped(int cfg, int tiles, hipStream_t st, GemmArgs& g) {
-  const int bm = cfg == 4 ? 64 : cfg == 0 ? 128 : 256;
+  const int bm = grouped_rows(cfg);
   const bool wide = g.lda >= kWide || g.ldb >= kWide;
   const int bn = bm == 64 || wide ? 64 : 256;
   g.tiles_n = (g.N + bn - 1) / bn;
-  const dim3 grid(tiles * g.tiles_n, wide ? bm / 64 : 1);
-  if (bn == 64)
+  const dim3 grid(tiles * g.tiles_n, wide ? (bm + 63) / 64 : 1);
+  if (bn == 64) {
     hipLaunchKernelGGL((gemm_kernel<DT, 64, 64, 2, 2, 2, EPI, 6, true>), grid, dim3(256), 0, st, g);
-  else if (bm == 128)
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 128, 256, 1, true>), grid, dim3(256), 0, st, g);
-  else
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, 256, 256, 1, true>), grid, dim3(256), 0, st, g);
+    return (int)hipGetLastError();
+  }
+  switch (bm) {
+#define X(BM, SCHED)                                                                          \
+  case BM:                                                                                    \
+    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, BM, 256, SCHED, true>), grid, dim3(256), 0, st, g); \
+    break;
+    X(128, 2) X(160, 2) X(192, 1) X(256, 1)
+#undef X
+  }
   return (int)hipGetLastError();
 }
 
@@ -37,7 +47,7 @@ CAKE_API int cake_gemm_grouped(int dt, int epi, int cfg, const void* a, long lon
                                const void* tiles, int max_tiles, const void* zeros, int N, int K,
                                hipStream_t st) {
   if (max_tiles <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || b_group % 8 ||
-      !(epi == 0 || (epi >= 7 && epi <= 10)) || !(cfg == 0 || cfg == 4 || cfg == 5))
+      !(epi == 0 || (epi >= 7 && epi <= 10)) || grouped_rows(cfg) == 0)
     return (int)hipErrorInvalidValue;
   GemmArgs g{};
   g.a = (const uint16_t*)a; g.b = (const uint16_t*)b; g.c = (uint16_t*)c;

@@ -13,6 +13,8 @@ estimate, which a measured entry of the very size (gemm_tuned.json) or a pinned 
 from __future__ import annotations
 
 import ctypes as C
+import functools
+import math
 import threading
 
 import torch
@@ -452,25 +454,53 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
 
 # tile configuration of a grouped product -> its rows (ROWS: the stream form)
 ROWS = 32
-GROUPED_CFGS = {0: 128, 4: 64, 5: 256, ROWS: 16}
+GROUPED_CFGS = {0: 128, 1: 160, 2: 192, 4: 64, 5: 256, ROWS: 16}
 
 
 def grouped_cfg(rows: int, groups: int, capturing: bool = False, weight: int = 0) -> int:
     """Tile configuration for `rows` sorted rows over `groups` weight groups of `weight` elements each
     (0: small)."""
-    # up and down product of 64 experts 4096 x 3616, us in the stream form and at 64 / 128 / 256 rows
-    # a tile, by rows an expert: 3 561 / 651 / 646 / -, 6 644 / 688 / 669 / -, 9 680 / 705 / 672 / -,
-    # 16 938 / 739 / 683 / -, 24 - / 775 / 698 / -, 75 - / 1275 / 766 / 895, 112 - / 1412 / 888 / 937
-    # (skewed 1435 / 984 / 1029), 131 - / 1550 / 1100 / 954, 192 - / 1998 / 1130 / 989.  From 4 to 12
-    # rows the 64-row tile loses 3 - 7 % here and is taken for the smaller experts' sake, of which it
-    # makes twice the workgroups: one product at 14 rows, 64 / 128 rows a tile, by millions of weights
-    # in all: 17 14.4 / 17.6 (8 of 1024 x 2048 24.4 / 29.3), 34 18.5 / 20.3, 101 47.6 / 50.1,
-    # 215 equal, 268 128.6 / 128.2
+    # up and down product of 64 experts 4096 x 3616, us in the stream form and at 64 / 128 rows
+    # a tile, by rows an expert: 3 561 / 651 / 646, 6 644 / 688 / 669, 9 680 / 705 / 672, 16 938 / 739 /
+    # 683, 24 - / 775 / 698, 75 - / 1275 / 766.  From 4 to 12 rows the 64-row tile loses 3 - 7 % here and
+    # is taken for the smaller experts' sake, of which it makes twice the workgroups: one product at 14
+    # rows, 64 / 128 rows a tile, by millions of weights in all: 17 14.4 / 17.6 (8 of 1024 x 2048 24.4 /
+    # 29.3), 34 18.5 / 20.3, 101 47.6 / 50.1, 215 equal, 268 128.6 / 128.2
     mean = rows / groups
     if mean <= 4 and not capturing:   # the stream form's counters stay out of graphs
         return ROWS
     big = groups * weight >= 200_000_000
-    return 5 if mean >= 115 else 0 if mean >= (12 if big else 24) else 4
+    if mean < (12 if big else 24):
+        return 4
+    return 0 if mean < 64 else _tile_height(rows, groups)
+
+
+# configuration -> (rows, cost of an expert's weights for a pair of tiles, of a tile), us of both
+# products of 64 experts 4096 x 3648
+_HEIGHTS = {0: (128, 461, 279), 1: (160, 384, 390), 2: (192, 303, 522), 5: (256, 209, 715)}
+
+
+@functools.lru_cache(maxsize=1024)
+def _tile_height(rows: int, groups: int) -> int:
+    """Configuration whose tiles cost least over groups of rows / groups rows on the average.  Tokens
+    that choose independently spread by the root of that; trained routers more, and a group that
+    overflows its tile costs more than a taller tile does: four times as much is assumed (over 68
+    products of even and 68 of skewed groups 5 % and 1 % faster than 128 and 256 rows alone, at most 12 %
+    slower; without the factor 3 %, 0 and 28 %).  Even groups, the same experts, us at 128 / 160 / 192 /
+    256 rows a tile, by rows an expert: 90 739 / 749 / 783 / 840, 120 870 / 774 / 812 / 869, 150 1078 / 886 /
+    826 / 912, 170 977 / 1167 / 928 / 913, 210 1310 / 1104 / 1457 / 1023, 260 1479 / 1143 / 1324 / 1379,
+    300 1712 / 1324 / 1347 / 1711, 400 2051 / 1906 / 1965 / 1629, 500 2395 / 2359 / 2201 / 2025."""
+    mean = rows / groups
+    sd = 4 * math.sqrt(2 * mean)
+
+    def cost(bm: int, pair: float, tile: float) -> float:
+        out, n, more = 0.0, 1, 1.0   # more: share of the groups with an n-th tile
+        while more > 1e-3:
+            out += more * (tile + (pair if n % 2 else 0))
+            more = 0.5 * math.erfc((n * bm - mean) / sd)
+            n += 1
+        return out
+    return min(_HEIGHTS, key=lambda c: cost(*_HEIGHTS[c]))
 
 
 def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out: torch.Tensor,

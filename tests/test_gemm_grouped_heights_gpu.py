@@ -1,0 +1,31 @@
+"""Grouped products in tiles of 160 and 192 rows, and of 128 on one barrier a step (gemm_inst_grouped.hip)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cfg", [0, 1, 2])
+@pytest.mark.parametrize("N,K,ld", [(8, 8, 8), (257, 128, 136), (300, 200, 200), (520, 1096, 1104), (40, 72, 1 << 22)])
+def test_tile_heights(cuda, cfg, N, K, ld):
+    """Groups of none, of a tile and one row to either side, rows far apart: one rounding to bf16
+    (2^-8) of f32 sums; nothing beside the rows is written."""
+    from cake_amd.ops import gemm as G
+    bm = G.GROUPED_CFGS[cfg]
+    counts = [bm - 1, 0, bm, bm + 1, 1, 2 * bm + 33]
+    R = sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.empty((R - 1) * ld + K, dtype=torch.bfloat16, device="cuda").as_strided((R, K), (ld, 1))
+    x.copy_(torch.randn(R, K, device="cuda", generator=g))
+    w = (torch.randn(len(counts), N, K, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    tiles, r0, want = [], 0, []
+    for e, c in enumerate(counts):
+        tiles += [[e, r0 + t, min(bm, c - t), 0] for t in range(0, c, bm)]
+        want.append(x[r0:r0 + c].float() @ w[e].float().t())
+        r0 += c
+    t = torch.tensor(tiles + [[0, 0, 0, 0], [len(tiles), 0, 0, 0]], dtype=torch.int32, device="cuda")
+    out = torch.full((R, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    G.grouped(x, w, t, cfg, out[:, :N])
+    want = torch.cat(want)
+    assert bool((out[:, N:] == 7.0).all())
+    assert bool(((out[:, :N].float() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -20).all())
