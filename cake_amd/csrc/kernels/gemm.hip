@@ -39,6 +39,7 @@
 #include "gemm_rows.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace cake {
 // the launchers are instantiated in gemm_inst_{bf16,f16}_{a,b,c}.hip
@@ -389,44 +390,73 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
 // ---- products of few rows (gemm_rows.h) -----------------------------------
 // Which form a product of M rows takes: 0 the tile kernels (cake_gemm_scaled), 1 direct, 2 stream.
 // The estimates (us) are fits to timings on weights that no cache holds, 2 .. 64 rows of 24 weight
-// shapes, 1 .. 940 MB: the form they pick is 0.7 % off the best of the three on the average.  Both
-// sides of the lines they draw, measured: 4096 x 4096 at 16 rows direct 11.8, stream 12.1; 4096 x 14336
+// shapes, 1 .. 940 MB: the form they pick is 1.3 % off the best of the three on the average.  Both sides
+// of the lines they draw, measured: 4096 x 4096 at 16 rows direct 11.8, stream 12.1; 4096 x 14336
 // direct 37, stream 23; 6144 x 4096 at 5 rows direct 16.9, stream 14.5, 3072 x 2048 6.5, 7.9; 28672 x
-// 4096 at 45 rows stream 52, tiles 55; 6144 x 4096 at 45 rows stream 22.0, tiles 19.4, 4096 x 11008
+// 4096 at 45 rows stream 40, tiles 55; 6144 x 4096 at 45 rows stream 18.4, tiles 19.4, 4096 x 11008
 // 31.0, 27.9.  Rows of k that start amid a 128-byte line (k no multiple of 64) cost a second line at
 // either end of a piece: 4096 x 10928 against 4096 x 11008, 5 rows direct 31.4 / 23.6, stream 23.5 /
 // 20.5, 33 rows stream 35.0 / 29.5, tiles 29.4 / 27.1.
-struct StreamPlan { int bn, kst, wgs; };
-// the stream form's shape (gemm_rows.h StreamShape)
-static StreamPlan stream_plan(int mt, bool gated) {
-  return mt > 1 || gated ? StreamPlan{128, 64, 256} : StreamPlan{64, 128, 512};
+struct StreamPlan {
+  int bn, kst, most;   // weight rows of a strip, k of a step (gemm_rows.h StreamShape), workgroups at most
+  int wgs, per;        // workgroups, steps of each
+  double us;
+};
+// The shares: as many as there are workgroups at most, of equal length wherever that ends, or whole
+// strips, or equal parts of one.  The latter two park no sums, or one a share, and never wait for them
+// amid a share; with fewer workgroups a CU takes up to 42 KB a us of weights, all of them 7.0 MB.  At 24 /
+// 45 rows, 256 shares against the best of the others: 28672 x 4096 SwiGLU 46.8 / 50.5 -> 38.2 / 39.6 us
+// (224 whole strips), 19456 x 4096 37.9 / 42 -> 30.7 / 36.7 (152), 6144 x 4096 17.2 / 22.1 -> 16.0 / 18.4
+// (192 quarters), 2048 x 8192 18 / 25.6 -> 15.6 / 21.3 (128 eighths); 4096 x 14336 stays, 25.6 / 30.7
+// (128 quarters 32 / 38).
+static StreamPlan stream_plan(int M, long long Nv, int K, bool gated) {
+  const int mt = (M + 15) / 16;
+  StreamPlan p = mt > 1 || gated ? StreamPlan{128, 64, 256, 0, 0, 1e30} : StreamPlan{64, 128, 512, 0, 0, 1e30};
+  const long long strips = (Nv + p.bn - 1) / p.bn, ks = (K + p.kst - 1) / p.kst, total = strips * ks;
+  const int least = kRowsMinK / p.kst;
+  const bool mid = K % 64 != 0;   // rows start amid a line
+  const auto take = [&](long long wgs, long long per, double us) {
+    if (us < p.us) { p.wgs = (int)wgs; p.per = (int)per; p.us = us; }
+  };
+  // a strip's shares, parked and summed
+  const auto sums = [&](double shares) { return mt * (0.86 * std::min(shares, 1.) + 0.25 * shares); };
+  for (int most = p.most; most >= 256; most /= 2) {   // ends anywhere
+    const long long per = std::max<long long>((total + most - 1) / most, least);
+    const long long wgs = (total + per - 1) / per;
+    const double shares = (double)ks / per;
+    if (ks % per == 0 || per % ks == 0) continue;   // below
+    if (most == 512) take(wgs, per, 6.2 + 0.08 * M + (1.42 + (mid ? 0.11 : 0.)) * per);
+    else if (p.most == 512) take(wgs, per, 4.5 + 0.04 * M + sums(shares) + (0.62 + (mid ? 0.11 : 0.)) * per);
+    else take(wgs, per, (mt > 1 ? 3 : 4.3) + sums(shares) + mt * std::min(1., std::pow(4096. / K, 3)) +
+                  per * (0.65 + 0.027 * mt + (mid ? 0.19 : 0.)));
+  }
+  const double cu = mt == 1 ? 0.38 : mt == 2 ? 0.41 : mt == 3 ? 0.5 : 0.55;   // us of a step of a CU's own
+  const auto even = [&](long long wgs, long long per, int parts) {
+    const int on = (int)((wgs + 255) / 256);   // workgroups on a CU
+    // rows 16 KB apart: still the same channels (8192 x 8192 at 24 / 45 rows 31.6 / 33.9 us; up to 24 rows
+    // tiles, at 32.9, keep it)
+    const double camp = mt == 1 || K % 8192 != 0 ? 0. : mt == 2 ? 0.2235 : 0.13;
+    const double step = std::max(cu * on, wgs * 16.384e-3 / 7.0) + (mid ? 0.19 : 0.) + camp;
+    take(wgs, per, 3.5 + 0.5 * on + per * step + (parts > 1 ? (mt > 1 ? 1. : 1.6) + sums(parts) : 0.));
+  };
+  for (long long c = (strips + p.most - 1) / p.most, n = 0; n < 2; ++c, ++n)
+    even((strips + c - 1) / c, c * ks, 1);
+  for (int s = 2; s <= 16 && strips * s <= p.most; s *= 2)
+    if (ks % s == 0 && ks / s >= least) even(strips * s, ks / s, s);
+  return p;
 }
 static int rows_kind(int M, long long Nv, int K, bool gated) {
   if (M > 64 || Nv > 64LL * kRowsTicks) return 0;
   const double kb = K * 2e-3;   // KB of one row of k
-  const int mt = (M + 15) / 16;
   const bool mid = K % 64 != 0;   // rows start amid a line
-  const double tiles = 6.7 + Nv * kb / 5590 + 0.0043 * M + 0.45e-3 * K;
-  const StreamPlan sp = stream_plan(mt, gated);
-  const long long strips = (Nv + sp.bn - 1) / sp.bn, ks = (K + sp.kst - 1) / sp.kst, total = strips * ks;
-  const long long per = std::max<long long>((total + sp.wgs - 1) / sp.wgs, kRowsMinK / sp.kst);
-  double stream;
-  if (sp.wgs == 512) {
-    stream = 6.2 + 0.08 * M + (1.42 + (mid ? 0.11 : 0.)) * per;
-  } else {
-    // a strip's shares, parked and summed; equal shares of rows 16 KB apart start on the same
-    // channels of the memory (8192 x 8192 at 24 rows 35.6 us, 10240 x 8192 35.1)
-    const double shares = ks > per || ks % per ? (double)ks / per : 0.;
-    const bool camp = K % 8192 == 0 && ks % per == 0;
-    stream = (mt > 1 ? 3 : 4.3) + mt * (0.86 * std::min(shares, 1.) + 0.25 * shares) +
-             per * (0.65 + 0.027 * mt + (mid ? 0.19 : 0.) + (camp ? 0.2 : 0.));
-  }
+  const double tiles = 6.7 + Nv * kb / 5590 + 0.025 * M + 0.45e-3 * K;
+  const double stream = stream_plan(M, Nv, K, gated).us;
   double direct = 1e9;
   if (M <= 32) {
     const int nt = gated || Nv > 4096 ? 2 : 1;
     const long long wgs = (Nv + 16 * nt - 1) / (16 * nt);
     // a CU's share at 32 (of two strips 26) KB a us, all weights and half of the reads of x at 5.8 MB
-    direct = 4 + (mid ? 1.35 : 1.) * std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
+    direct = 3.4 + (mid ? 1.35 : 1.) * std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
                                               (Nv + 0.5 * wgs * M) * kb / 5800);
   }
   if (direct <= stream && direct <= tiles) return 1;
@@ -468,13 +498,12 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
   const int mt = (M + 15) / 16;
   int form, wgs;
   if (kind == 2) {
-    const StreamPlan sp = stream_plan(mt, gated);
+    const StreamPlan sp = stream_plan(M, g.Nv, K, gated);
     g.tiles_n = (g.Nv + sp.bn - 1) / sp.bn;
     if (g.tiles_n > kRowsTicks) return (int)hipErrorInvalidValue;
-    g.kps = kRowsMinK / sp.kst;   // steps of a share at least
-    const long long total = (long long)g.tiles_n * ((K + sp.kst - 1) / sp.kst);
+    g.kps = sp.per;
     form = 2;
-    wgs = (int)std::min<long long>(sp.wgs, (total + g.kps - 1) / g.kps);
+    wgs = sp.wgs;
   } else {
     const int nt = gated || g.Nv > 4096 ? 2 : 1;   // one 16-row strip per CU, or two
     form = nt - 1;
@@ -491,7 +520,7 @@ CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long ld
                                     long long ldb, long long b_group, void* c, long long ldc,
                                     const void* tiles, int max_tiles, float* ws, void* tick,
                                     const void* zeros, int N, int K, hipStream_t st) {
-  const StreamPlan sp = stream_plan(1, false);
+  const StreamPlan sp = stream_plan(1, N, K, false);
   const long long strips = (long long)max_tiles * ((N + sp.bn - 1) / sp.bn);
   if (max_tiles <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || b_group % 8 ||
       !(epi == 0 || (epi >= 7 && epi <= 10)) || !ws || !tick || !zeros)
@@ -509,6 +538,6 @@ CAKE_API int cake_gemm_rows_grouped(int dt, int epi, const void* a, long long ld
   g.kps = kRowsMinK / sp.kst;
   g.groups = (const int4*)tiles;
   g.b_group = b_group;
-  return dt == kBF16 ? Rows<kBF16>::grouped(epi, dim3(sp.wgs), st, g)
-         : dt == kF16 ? Rows<kF16>::grouped(epi, dim3(sp.wgs), st, g) : (int)hipErrorInvalidValue;
+  return dt == kBF16 ? Rows<kBF16>::grouped(epi, dim3(sp.most), st, g)
+         : dt == kF16 ? Rows<kF16>::grouped(epi, dim3(sp.most), st, g) : (int)hipErrorInvalidValue;
 }

@@ -10,11 +10,12 @@
 //   from L2, which is what ends its range.
 // gemm_stream_kernel (M <= 64): 128 weight rows by 64 k (up to 16 rows of x 64 by 128) and the x tile
 //   go through LDS by DMA; the steps of all strips form one sequence dealt out in equal contiguous
-//   shares, one workgroup per CU (two), so no last wave is left and the DMA never stops at a strip's
-//   end.  Strips that several shares cover meet in memory, the last to arrive sums in share order
-//   (the result does not hang on the order).  28672 x 4096 SwiGLU at 13 / 24 / 45 rows 44 / 46 / 53
-//   us (tile kernels 58-60 us), 4096 x 23552 35 / 37 / 42 us (44-46 us).  What bounds it is how much
-//   the waves of a CU have outstanding (StreamShape) and, in short shares, the parked sums.
+//   shares, at most one workgroup per CU (two): whole strips or equal parts of one where that pays, else
+//   ends anywhere (gemm.hip stream_plan).  Strips that several shares cover meet in memory, the last to
+//   arrive sums in share order (the result does not hang on the order).  28672 x 4096 SwiGLU at 5 / 24 /
+//   45 rows 38 / 38 / 40 us (tile kernels 58-60 us), 4096 x 23552 33 / 37 / 43 us (44-46 us), 57344 x 8192
+//   140 us (6.7 TB/s).  What bounds it is the memory in whole strips, in parts the parked sums; weight
+//   rings of a wave's own with a barrier every four steps only ran at the same rate.
 #pragma once
 #include "gemm_kernel.h"
 
@@ -329,6 +330,13 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
   // ---- DMA: wave w fetches weight rows 16 RT w .. and its share of x ----
   const int dr = lane / S::LPR, dslot = lane % S::LPR;   // row within an instruction's, slot
   int ds = u0 / KS, dk = u0 % KS, dnext = u0;
+  // shares of whole strips, or of equal parts of one, start at different k each: the strips lie the same
+  // distance apart, and in step they would ask the same channels of the memory at a time (28672 x 4096
+  // in 224 whole strips 46.8 us in step, 39.6 so; 32000 x 4096 in 250 56.8, 42.2)
+  const int seg = KS % per == 0 ? per : per % KS == 0 ? KS : 0;   // 0: other shares
+  const int seg0 = seg > 0 ? dk / seg * seg : 0;
+  if (seg > 0) dk = seg0 + wg * 5 % seg;
+  int left = seg;
   const uint16_t *wsrc[4], *xsrc[S::XI];
   auto aim = [&](int s) {
     const StreamStrip t = stream_strip<GRP, S::BN>(g, s);
@@ -365,7 +373,15 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
       glds16(p, b + (NWV * 4 + r0) * 1024);
     }
     ++dnext;
-    if (++dk == KS) {
+    ++dk;
+    if (seg > 0) {
+      if (dk == seg0 + seg) dk = seg0;
+      if (--left == 0) {
+        left = seg;
+        ++ds;
+        if (dnext < u1) aim(ds);
+      }
+    } else if (dk == KS) {
       dk = 0;
       ++ds;
       if (dnext < u1) aim(ds);
