@@ -17,10 +17,19 @@ import os
 import threading
 from pathlib import Path
 
+import torch
+
 _LIB_DIR = Path(__file__).resolve().parent.parent / "lib"
 _LIB_PATH = _LIB_DIR / "libcake_kernels.so"
 _lock = threading.Lock()
 _lib = None
+
+def current_stream() -> int:
+    """torch's current stream of the current device, as its handle.  Every launch asks for it:
+    ``torch.cuda.current_stream().cuda_stream`` makes an object and looks the device up three times,
+    2.5 us of the 17 that a launch of a batch's step took (1000 launches a pass, 13 sequences)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
 
 P = C.c_void_p
 I = C.c_int

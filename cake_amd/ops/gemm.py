@@ -19,7 +19,7 @@ import threading
 
 import torch
 
-from ._lib import check, kernels, library
+from ._lib import check, current_stream, kernels, library
 
 EPI = {"store": 0, "resid32": 1, "add16": 2, "swiglu": 3, "geglu": 4, "store32": 6, "silu": 7,
        "quick_gelu": 8, "gelu": 9, "relu2": 10}
@@ -418,7 +418,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
         if kind == 2 and torch.cuda.is_current_stream_capturing():
             kind = 0
         if kind:
-            st = torch.cuda.current_stream().cuda_stream
+            st = current_stream()
             ws, tick = _rows_state(x.device, M, st) if kind == 2 else (None, None)
             check(_lib().cake_gemm_rows(
                 _DT[x.dtype], EPI[epi], kind, x2.data_ptr(), lda, w.data_ptr(), ldb, cptr, ldc,
@@ -440,7 +440,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
         cfg, s0 = resolve(M, Nv, K, epi, big, mfma_only=True)
     splits = s0 if splits is None else max(1, int(splits))
     # the kernel library sizes it (pieces of a tile need their slabs only)
-    st = torch.cuda.current_stream().cuda_stream
+    st = current_stream()
     tick = _counters(x.device, st) if splits > 1 and cfg in FOUR_WAVE else None
     ws = _workspace(x.device, int(_lib().cake_gemm_ws_floats(
         int(cfg), int(splits), M, N, K, 1 if Nv != N else 0))) if splits > 1 else None
@@ -526,7 +526,7 @@ def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out
     if cfg == ROWS and torch.cuda.is_current_stream_capturing():
         cfg = 4   # rows planned before the capture: the 64-row tile takes the same tile list
     if cfg == ROWS:
-        st = torch.cuda.current_stream().cuda_stream
+        st = current_stream()
         ws, tick = _rows_state(x.device, 16, st)
         check(_lib().cake_gemm_rows_grouped(
             _DT[x.dtype], EPI[epi], x2.data_ptr(), lda, w.data_ptr(), K, N * K, o2.data_ptr(), ldc,
@@ -536,7 +536,7 @@ def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out
     check(_lib().cake_gemm_grouped(
         _DT[x.dtype], EPI[epi], int(cfg), x2.data_ptr(), lda, w.data_ptr(), K, N * K,
         o2.data_ptr(), ldc, tiles.data_ptr(), tiles.shape[0] - 1, _zeros16(x.device).data_ptr(), N, K,
-        torch.cuda.current_stream().cuda_stream), "gemm_grouped")
+        current_stream()), "gemm_grouped")
     return out
 
 
@@ -544,7 +544,7 @@ def _lib_gemm(x2, lda, w, ldb, epi, out2, ldc, r2, ldr, M, N, K) -> None:
     """The library GEMM (hipBLASLt) for a plan that names it.  Its workspace is one buffer
     per (device, stream), so library GEMMs on two streams never share one."""
     dev = x2.device
-    st = torch.cuda.current_stream().cuda_stream
+    st = current_stream()
     ws = _lib_ws.get((dev, st))
     if ws is None:
         ws = _lib_ws[(dev, st)] = torch.empty(_LIB_WS_BYTES, dtype=torch.uint8, device=dev)

@@ -10,7 +10,7 @@ import ctypes as C
 import torch
 
 from . import gemm as G
-from ._lib import check, kernels
+from ._lib import check, current_stream, kernels
 
 P, I, F = C.c_void_p, C.c_int, C.c_float
 
@@ -83,7 +83,7 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
                                (H, inter, "resid32")), capturing)
     if forms is None:
         return False
-    dev, st = hidden.device, torch.cuda.current_stream().cuda_stream
+    dev, st = hidden.device, current_stream()
     x = torch.empty((T, H), device=dev, dtype=dt)
     qkv = torch.empty((T, nqkv), device=dev, dtype=dt)
     att = torch.empty((T, nq), device=dev, dtype=dt)

@@ -12,6 +12,7 @@ from dataclasses import dataclass
 import torch
 
 from ._lib import check, library
+from ._lib import current_stream as _stream
 
 DT = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 MAX_HEAD = 256   # largest head size the kernels hold
@@ -24,10 +25,6 @@ ACTS = {"gelu": 0, "relu2": 1}   # feed-forward activations (erf GELU, square of
 
 def _lib():
     return library("mixers")
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def pad_to(n: int, m: int) -> int:
