@@ -471,15 +471,33 @@ __global__ __launch_bounds__(kDdThreads) void mixer_delta_decode_kernel(DeltaArg
   float* ring = a.ring + slot * a.r_slot;
   const int nch = 2 * a.dim + a.vdim;
   const bool own_qk = h % R == 0;
+  // everything else that is read, before the first use of any: one after the other they were six round
+  // trips to the memory (16 heads of 128 x 128, one row 7.9 -> 7.15 us)
+  const float* ab = a.ab + (long long)b * a.ldab;
+  const float a_log = a.a_log[h], a_in = ab[h] + a.dt_bias[h], b_in = ab[a.H + h];
+  float norm_w = 0.f, gate = 0.f;
+  if (tid < a.vdim) {
+    norm_w = a.norm_w[tid];
+    gate = pj[C + h * a.vdim + tid];
+  }
   for (int x = tid; x < nch; x += kDdThreads) {
     const bool isv = x >= 2 * a.dim;
     const int ch = isv ? 2 * a.G * a.dim + h * a.vdim + x - 2 * a.dim
                        : x < a.dim ? gh * a.dim + x : (a.G + gh) * a.dim + x - a.dim;
     const float cur = pj[ch];
     float y = a.conv[(long long)(a.taps - 1) * C + ch] * cur;
-    for (int j = 1; j < a.taps && j <= pos; ++j)
-      y = fmaf(a.conv[(long long)(a.taps - 1 - j) * C + ch],
-               ring[(long long)((pos - j) % a.taps) * C + ch], y);
+    for (int j0 = 1; j0 < a.taps; j0 += 3) {   // three earlier inputs at a time
+      float w[3], in[3];
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        const int j = min(j0 + e, a.taps - 1);
+        w[e] = a.conv[(long long)(a.taps - 1 - j) * C + ch];
+        in[e] = ring[(long long)((pos + a.taps - j) % a.taps) * C + ch];
+      }
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (j0 + e < a.taps && j0 + e <= pos) y = fmaf(w[e], in[e], y);
+    }
     y = silu32(y);
     if (isv) v[x - 2 * a.dim] = y;
     else if (x < a.dim) q[x] = y;
@@ -500,9 +518,8 @@ __global__ __launch_bounds__(kDdThreads) void mixer_delta_decode_kernel(DeltaArg
   }
   __syncthreads();
   const float rq = sn[0], rk = sn[1];
-  const float* ab = a.ab + (long long)b * a.ldab;
-  const float dec = expf(-expf(a.a_log[h]) * softplus32(ab[h] + a.dt_bias[h]));
-  const float beta = sigmoid32(ab[a.H + h]);
+  const float dec = expf(-expf(a_log) * softplus32(a_in));
+  const float beta = sigmoid32(b_in);
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
@@ -544,7 +561,7 @@ __global__ __launch_bounds__(kDdThreads) void mixer_delta_decode_kernel(DeltaArg
   const float rms = 1.f / sqrtf(block_sum(ov * ov, red) / (float)a.vdim + a.eps);
   if (tid < a.vdim)
     reinterpret_cast<E*>(a.out)[(long long)b * a.ldo + h * a.vdim + tid] =
-        St<DT>::st(ov * rms * a.norm_w[tid] * silu32(pj[C + h * a.vdim + tid]));
+        St<DT>::st(ov * rms * norm_w * silu32(gate));
 }
 
 }  // namespace cake
