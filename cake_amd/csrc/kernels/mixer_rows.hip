@@ -29,35 +29,51 @@ struct NormArgs {
   const float* x;       // [*][ldx], columns [W, ldo) zero
   long long ldx;
   const int* rows;      // row of x per output row (null: the same)
+  const int* where;     // or: output rows of each row of x, `copies` of them (else null, 1)
+  int copies;
   const float* scale;   // factor per output row (null: 1)
   const float* w;       // [ldo], zeros past W
   float off, eps;
   int ln, W, ldo;
   void* out;            // [N][ldo]
 };
+constexpr int kNormCopies = 32;
 
 // out[r] = scale[r] * norm(x[rows ? rows[r] : r]) * (off + w): the RMS norm x / rms, or (LN)
-// the layer norm (x - mean) / sqrt(variance + eps)
-template <int DT, bool LN>
+// the layer norm (x - mean) / sqrt(variance + eps).  Of a few rows a launch is its round trips to the
+// memory, so the weights are asked for with the row (24 rows of 4096 3.1 us, after the sums 3.6);
+// of many rows it is the bytes: a row that goes to several places is read and summed once (2048 rows
+// of 4096 to six places each 20.3 us, gathered six times over 46).
+template <int DT, bool LN, int NV>
 __global__ __launch_bounds__(256) void mixer_norm_kernel(NormArgs a) {
   using E = typename St<DT>::E;
-  __shared__ float red[16];
-  const long long r = blockIdx.x;
-  const int ldo = a.ldo, W = a.W;
-  const float* xr = a.x + (a.rows ? a.rows[r] : r) * a.ldx;
-  const float sc = a.scale ? a.scale[r] : 1.f;
-  float4 v[8];  // rows up to 8192 stay in registers (ldo % 8 == 0, zeros past W)
-  float ss = 0.f, sum = 0.f;
+  __shared__ float red[16], fac[kNormCopies];
+  __shared__ int dst[kNormCopies];
+  const long long n = blockIdx.x;
+  const int ldo = a.ldo, W = a.W, tid = threadIdx.x;
+  const float* xr = a.x + (a.rows ? a.rows[n] : n) * a.ldx;
+  float4 v[NV], wv[NV];  // rows up to 1024 NV stay in registers (ldo % 8 == 0, zeros past W)
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int i = (j * 256 + threadIdx.x) * 4;
+  for (int j = 0; j < NV; ++j) {
+    const int i = (j * 256 + tid) * 4;
+    v[j] = wv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (i < ldo) {
       v[j] = *reinterpret_cast<const float4*>(xr + i);
-      if constexpr (LN) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
-      else ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+      wv[j] = *reinterpret_cast<const float4*>(a.w + i);
     }
   }
-  for (int i = 8192 + threadIdx.x; i < ldo; i += 256) {
+  if (tid < a.copies) {   // read after the sums' barriers
+    const int r = a.where ? a.where[n * a.copies + tid] : (int)n;
+    dst[tid] = r;
+    fac[tid] = a.scale ? a.scale[r] : 1.f;
+  }
+  float ss = 0.f, sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    if constexpr (LN) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
+    else ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+  }
+  for (int i = 1024 * NV + tid; i < ldo; i += 256) {
     if constexpr (LN) sum += xr[i];
     else ss += xr[i] * xr[i];
   }
@@ -65,27 +81,26 @@ __global__ __launch_bounds__(256) void mixer_norm_kernel(NormArgs a) {
   if constexpr (LN) {
     mean = block_sum(sum, red) / (float)W;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int i = (j * 256 + threadIdx.x) * 4;
-      if (i < ldo) {
-        v[j].x = i < W ? v[j].x - mean : 0.f;
-        v[j].y = i + 1 < W ? v[j].y - mean : 0.f;
-        v[j].z = i + 2 < W ? v[j].z - mean : 0.f;
-        v[j].w = i + 3 < W ? v[j].w - mean : 0.f;
-        ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
-      }
+    for (int j = 0; j < NV; ++j) {
+      const int i = (j * 256 + tid) * 4;
+      v[j].x = i < W ? v[j].x - mean : 0.f;
+      v[j].y = i + 1 < W ? v[j].y - mean : 0.f;
+      v[j].z = i + 2 < W ? v[j].z - mean : 0.f;
+      v[j].w = i + 3 < W ? v[j].w - mean : 0.f;
+      ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
     }
-    for (int i = 8192 + threadIdx.x; i < W; i += 256) ss += (xr[i] - mean) * (xr[i] - mean);
+    for (int i = 1024 * NV + tid; i < W; i += 256) ss += (xr[i] - mean) * (xr[i] - mean);
   }
-  const float f = sc / sqrtf(block_sum(ss, red) / (float)W + a.eps);
-  E* o = reinterpret_cast<E*>(a.out) + r * ldo;
+  const float norm = sqrtf(block_sum(ss, red) / (float)W + a.eps);
+  for (int c = 0; c < a.copies; ++c) {
+    const float f = fac[c] / norm;
+    E* o = reinterpret_cast<E*>(a.out) + (long long)dst[c] * ldo;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int i = (j * 256 + threadIdx.x) * 4;
-    if (i < ldo) {
-      const float4 wv = *reinterpret_cast<const float4*>(a.w + i);
-      const float y[4] = {v[j].x * f * (a.off + wv.x), v[j].y * f * (a.off + wv.y),
-                          v[j].z * f * (a.off + wv.z), v[j].w * f * (a.off + wv.w)};
+    for (int j = 0; j < NV; ++j) {
+      const int i = (j * 256 + tid) * 4;
+      if (i >= ldo) continue;
+      const float y[4] = {v[j].x * f * (a.off + wv[j].x), v[j].y * f * (a.off + wv[j].y),
+                          v[j].z * f * (a.off + wv[j].z), v[j].w * f * (a.off + wv[j].w)};
       if constexpr (DT == kF32) {
         *reinterpret_cast<float4*>(o + i) = make_float4(y[0], y[1], y[2], y[3]);
       } else {
@@ -94,9 +109,9 @@ __global__ __launch_bounds__(256) void mixer_norm_kernel(NormArgs a) {
             (uint32_t)St<DT>::st(y[2]) | ((uint32_t)St<DT>::st(y[3]) << 16));
       }
     }
+    for (int i = 1024 * NV + tid; i < ldo; i += 256)
+      o[i] = St<DT>::st(i < W ? (xr[i] - mean) * f * (a.off + a.w[i]) : 0.f);
   }
-  for (int i = 8192 + threadIdx.x; i < ldo; i += 256)
-    o[i] = St<DT>::st(i < W ? (xr[i] - mean) * f * (a.off + a.w[i]) : 0.f);
 }
 
 // a[n] = [x[n] | x0[n] | 0] (storage type), y[n] = step (zeros past W)
@@ -152,18 +167,22 @@ CAKE_API int cake_mixer_embed(int dt, const void* table, const int* tok, int N, 
   return (int)hipGetLastError();
 }
 
-CAKE_API int cake_mixer_norm(int dt, const float* x, long long ldx, const int* rows,
-                             const float* scale, const float* w, float off, float eps, int ln,
-                             int N, int W, void* out, int ldo, hipStream_t st) {
+// rows: row of x per output row; or where [N][copies]: output rows of each of x's N rows
+CAKE_API int cake_mixer_norm(int dt, const float* x, long long ldx, const int* rows, const int* where,
+                             int copies, const float* scale, const float* w, float off, float eps,
+                             int ln, int N, int W, void* out, int ldo, hipStream_t st) {
   // w holds ldo f32 values (zeros past W); x has ldo readable columns
-  if (N < 0 || W <= 0 || W > ldo || ldo % 8 || ldx % 4 || ldx < ldo)
+  if (N < 0 || W <= 0 || W > ldo || ldo % 8 || ldx % 4 || ldx < ldo || copies < 1 ||
+      copies > kNormCopies || (where ? rows != nullptr : copies != 1))
     return (int)hipErrorInvalidValue;
   if (N == 0) return 0;
-  const NormArgs a{x, ldx, rows, scale, w, off, eps, ln, W, ldo, out};
-  CAKE_MIX_DT(dt, {
-    if (ln) hipLaunchKernelGGL((mixer_norm_kernel<DT, true>), dim3(N), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((mixer_norm_kernel<DT, false>), dim3(N), dim3(256), 0, st, a);
-  });
+  const NormArgs a{x, ldx, rows, where, copies, scale, w, off, eps, ln, W, ldo, out};
+#define CAKE_NORM(LN, NV) hipLaunchKernelGGL((mixer_norm_kernel<DT, LN, NV>), dim3(N), dim3(256), 0, st, a)
+#define CAKE_NORM_NV(LN) \
+  if (ldo <= 2048) CAKE_NORM(LN, 2); else if (ldo <= 4096) CAKE_NORM(LN, 4); else CAKE_NORM(LN, 8)
+  CAKE_MIX_DT(dt, { if (ln) { CAKE_NORM_NV(true); } else { CAKE_NORM_NV(false); } });
+#undef CAKE_NORM_NV
+#undef CAKE_NORM
   return (int)hipGetLastError();
 }
 

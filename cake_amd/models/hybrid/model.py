@@ -125,12 +125,13 @@ class HybridModel:
             t = self._rot[m.rot] = t.to(self.device).contiguous()
         return t
 
-    def norm_rows(self, x, w32, rows=None, scale=None, dtype=None) -> torch.Tensor:
-        """The model's norm of residual rows (of rows[r], times scale[r])."""
-        n = x.shape[0] if rows is None else rows.numel()
+    def norm_rows(self, x, w32, rows=None, scale=None, dtype=None, where=None) -> torch.Tensor:
+        """The model's norm of residual rows (of rows[r], times scale[r]; or each to the rows
+        where[r])."""
+        n = x.shape[0] if rows is None and where is None else (rows if where is None else where).numel()
         h = torch.empty((n, self.Wp), device=self.device, dtype=dtype or self.dtype)
         M.norm(x, w32, self.cfg.norm_offset, self.cfg.eps, self.W, h, rows=rows,
-               ln=self.cfg.layer_norm, scale=scale)
+               ln=self.cfg.layer_norm, scale=scale, where=where)
         return h
 
     def product(self, x, w, out):

@@ -203,7 +203,7 @@ _SIGS.update({
 _LIB_SIGS = {
     "mixers": {
         "cake_mixer_embed": [I, P, P, I, I, P, P, P],
-        "cake_mixer_norm": [I, P, L, P, P, P, F, F, I, I, I, P, I, P],
+        "cake_mixer_norm": [I, P, L, P, P, I, P, P, F, F, I, I, I, P, I, P],
         "cake_mixer_loop_rows": [I, P, P, I, P, I, I, P, I, P, P],
         "cake_mixer_act": [I, P, L, P, I, I, P, L, P],
         "cake_mixer_in": [I, P, P, F, F, I, I, P, I, I, I, P, I, P, P, P],

@@ -111,20 +111,26 @@ def embed(table, tok, x, x0=None):
 
 
 def norm(x, w, offset: float, eps: float, width: int, out, rows=None, ln: bool = False,
-         scale=None):
+         scale=None, where=None):
     """out[r] = scale[r] * x[rows[r] or r] / rms * (offset + w); ln: the layer norm
     (x - mean) / sqrt(variance + eps) instead.  x [*, >= ld] f32 (zeros in columns width .. ld),
-    w [ld] f32, out [R, ld], rows int32 [R], scale f32 [R]."""
+    w [ld] f32, out [R, ld], rows int32 [R], scale f32 [R].  where int32 [N, copies] instead of rows:
+    the output rows of each of x's N rows (at most 32 each), every one of the R named once."""
     R, ld = out.shape
-    xp, ldx = _mat(x, "x", torch.float32, 1 if rows is not None else R, ld)
+    N, copies = (R, 1) if where is None else where.shape
+    if where is not None and (rows is not None or N * copies != R or not 1 <= copies <= 32):
+        raise ValueError(f"norm: {tuple(where.shape)} output rows for {R}")
+    xp, ldx = _mat(x, "x", torch.float32, 1 if rows is not None else N, ld)
     ldx = max(ldx, ld)
     if not out.is_contiguous() or ld % 8 or ldx % 4 or xp % 16:
         raise ValueError("norm: rows of a multiple of 8 columns on 16-byte boundaries")
     check(_lib().cake_mixer_norm(DT[out.dtype], xp, ldx,
                                  None if rows is None else _vec(rows, "rows", torch.int32, R),
+                                 None if where is None else _vec(where, "where", torch.int32, R),
+                                 copies,
                                  None if scale is None else _vec(scale, "scale", torch.float32, R),
                                  _vec(w, "w", torch.float32, ld), float(offset), float(eps),
-                                 int(ln), R, int(width), out.data_ptr(), ld, _stream()),
+                                 int(ln), N, int(width), out.data_ptr(), ld, _stream()),
           "mixer_norm")
 
 
