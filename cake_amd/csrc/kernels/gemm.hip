@@ -390,7 +390,7 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
 // ---- products of few rows (gemm_rows.h) -----------------------------------
 // Which form a product of M rows takes: 0 the tile kernels (cake_gemm_scaled), 1 direct, 2 stream.
 // The estimates (us) are fits to timings on weights that no cache holds, 2 .. 64 rows of 24 weight
-// shapes, 1 .. 940 MB: the form they pick is 1.3 % off the best of the three on the average.  Both sides
+// shapes, 1 .. 940 MB: the form they pick is 1.1 % off the best of the three on the average.  Both sides
 // of the lines they draw, measured: 4096 x 4096 at 16 rows direct 11.8, stream 12.1; 4096 x 14336
 // direct 37, stream 23; 6144 x 4096 at 5 rows direct 16.9, stream 14.5, 3072 x 2048 6.5, 7.9; 28672 x
 // 4096 at 45 rows stream 40, tiles 55; 6144 x 4096 at 45 rows stream 18.4, tiles 19.4, 4096 x 11008
@@ -407,8 +407,8 @@ struct StreamPlan {
 // amid a share; with fewer workgroups a CU takes up to 42 KB a us of weights, all of them 7.0 MB.  At 24 /
 // 45 rows, 256 shares against the best of the others: 28672 x 4096 SwiGLU 46.8 / 50.5 -> 38.2 / 39.6 us
 // (224 whole strips), 19456 x 4096 37.9 / 42 -> 30.7 / 36.7 (152), 6144 x 4096 17.2 / 22.1 -> 16.0 / 18.4
-// (192 quarters), 2048 x 8192 18 / 25.6 -> 15.6 / 21.3 (128 eighths); 4096 x 14336 stays, 25.6 / 30.7
-// (128 quarters 32 / 38).
+// (192 quarters), 2048 x 8192 18 / 25.6 -> 15.6 / 21.3 (128 eighths); 4096 x 14336 stays at 24 rows, 25.6
+// (128 quarters 32), and takes tiles at 45, 30.4 (32.2).
 static StreamPlan stream_plan(int M, long long Nv, int K, bool gated) {
   const int mt = (M + 15) / 16;
   StreamPlan p = mt > 1 || gated ? StreamPlan{128, 64, 256, 0, 0, 1e30} : StreamPlan{64, 128, 512, 0, 0, 1e30};
@@ -419,15 +419,15 @@ static StreamPlan stream_plan(int M, long long Nv, int K, bool gated) {
     if (us < p.us) { p.wgs = (int)wgs; p.per = (int)per; p.us = us; }
   };
   // a strip's shares, parked and summed
-  const auto sums = [&](double shares) { return mt * (0.86 * std::min(shares, 1.) + 0.25 * shares); };
+  const auto sums = [&](double shares, double each) { return mt * (0.86 * std::min(shares, 1.) + each * shares); };
   for (int most = p.most; most >= 256; most /= 2) {   // ends anywhere
     const long long per = std::max<long long>((total + most - 1) / most, least);
     const long long wgs = (total + per - 1) / per;
     const double shares = (double)ks / per;
     if (ks % per == 0 || per % ks == 0) continue;   // below
     if (most == 512) take(wgs, per, 6.2 + 0.08 * M + (1.42 + (mid ? 0.11 : 0.)) * per);
-    else if (p.most == 512) take(wgs, per, 4.5 + 0.04 * M + sums(shares) + (0.62 + (mid ? 0.11 : 0.)) * per);
-    else take(wgs, per, (mt > 1 ? 3 : 4.3) + sums(shares) + mt * std::min(1., std::pow(4096. / K, 3)) +
+    else if (p.most == 512) take(wgs, per, 4.5 + 0.04 * M + sums(shares, 0.25) + (0.62 + (mid ? 0.11 : 0.)) * per);
+    else take(wgs, per, (mt > 1 ? 3 : 4.3) + sums(shares, 0.25) + mt * std::min(1., std::pow(4096. / K, 3)) +
                   per * (0.65 + 0.027 * mt + (mid ? 0.19 : 0.)));
   }
   const double cu = mt == 1 ? 0.38 : mt == 2 ? 0.41 : mt == 3 ? 0.5 : 0.55;   // us of a step of a CU's own
@@ -435,9 +435,9 @@ static StreamPlan stream_plan(int M, long long Nv, int K, bool gated) {
     const int on = (int)((wgs + 255) / 256);   // workgroups on a CU
     // rows 16 KB apart: still the same channels (8192 x 8192 at 24 / 45 rows 31.6 / 33.9 us; up to 24 rows
     // tiles, at 32.9, keep it)
-    const double camp = mt == 1 || K % 8192 != 0 ? 0. : mt == 2 ? 0.2235 : 0.13;
+    const double camp = mt == 1 || K % 8192 != 0 ? 0. : mt == 2 ? 0.1665 : 0.06;
     const double step = std::max(cu * on, wgs * 16.384e-3 / 7.0) + (mid ? 0.19 : 0.) + camp;
-    take(wgs, per, 3.5 + 0.5 * on + per * step + (parts > 1 ? (mt > 1 ? 1. : 1.6) + sums(parts) : 0.));
+    take(wgs, per, 3.5 + 0.5 * on + per * step + (parts <= 1 ? 0. : mt > 1 ? 1.4 + sums(parts, 0.4) : 2.65 + sums(parts, 0.1)));
   };
   for (long long c = (strips + p.most - 1) / p.most, n = 0; n < 2; ++c, ++n)
     even((strips + c - 1) / c, c * ks, 1);
@@ -449,14 +449,14 @@ static int rows_kind(int M, long long Nv, int K, bool gated) {
   if (M > 64 || Nv > 64LL * kRowsTicks) return 0;
   const double kb = K * 2e-3;   // KB of one row of k
   const bool mid = K % 64 != 0;   // rows start amid a line
-  const double tiles = 6.7 + Nv * kb / 5590 + 0.025 * M + 0.45e-3 * K;
+  const double tiles = 6.7 + Nv * kb / 5590 + 0.015 * M + 0.45e-3 * std::min(K, 8192);
   const double stream = stream_plan(M, Nv, K, gated).us;
   double direct = 1e9;
   if (M <= 32) {
     const int nt = gated || Nv > 4096 ? 2 : 1;
     const long long wgs = (Nv + 16 * nt - 1) / (16 * nt);
     // a CU's share at 32 (of two strips 26) KB a us, all weights and half of the reads of x at 5.8 MB
-    direct = 3.4 + (mid ? 1.35 : 1.) * std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
+    direct = 4 + (mid ? 1.35 : 1.) * std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
                                               (Nv + 0.5 * wgs * M) * kb / 5800);
   }
   if (direct <= stream && direct <= tiles) return 1;
