@@ -121,33 +121,59 @@ __global__ __launch_bounds__(1024) void expert_plan_kernel(const int* ids, const
   }
 }
 
-// x[n] += alpha * sum over k of y[where[n][k]]
+// x[n] += alpha * sum over k of y[where[n][k]].  Bound by its bytes at many tokens and by round trips
+// at few: the row of x and eight experts' rows are asked for at once (2048 x 4096, six each, 168 MB: 38.1 ->
+// 32.2 us, 5.2 TB/s; 13 x 2048 6.9 -> 6.3).
 template <int DT>
 __global__ __launch_bounds__(256) void expert_sum_kernel(const void* y, long long ldy,
                                                          const int* where, int top, int W,
                                                          float alpha, float* x, long long ldx) {
   using E = typename St<DT>::E;
+  using V = std::conditional_t<DT == kF32, float4, uint2>;
+  constexpr int U = 8;
   const long long n = blockIdx.x;
   const int* wp = where + n * top;
-  for (int i = threadIdx.x * 4; i < W; i += 1024) {  // ldy, ldx multiples of 4: whole reads
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < top; ++k) {
-      const E* src = reinterpret_cast<const E*>(y) + (long long)wp[k] * ldy + i;
-      if constexpr (DT == kF32) {
-        const float4 v = *reinterpret_cast<const float4*>(src);
-        s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
-      } else {
-        const uint2 v = *reinterpret_cast<const uint2*>(src);
-        s[0] += to_f32<DT>((uint16_t)(v.x & 0xffffu));
-        s[1] += to_f32<DT>((uint16_t)(v.x >> 16));
-        s[2] += to_f32<DT>((uint16_t)(v.y & 0xffffu));
-        s[3] += to_f32<DT>((uint16_t)(v.y >> 16));
-      }
-    }
+  const bool wide = ldx % 4 == 0 && ((uintptr_t)x & 15) == 0;
+  for (int i = threadIdx.x * 4; i < W; i += 1024) {  // ldy a multiple of 4: whole reads
     float* xr = x + n * ldx + i;
+    const bool whole = wide && i + 4 <= W;
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
+    if (whole) {
+      const float4 v = *reinterpret_cast<const float4*>(xr);
+      o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+    } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (i + e < W) xr[e] = fmaf(alpha, s[e], xr[e]);
+      for (int e = 0; e < 4; ++e)
+        if (i + e < W) o[e] = xr[e];
+    }
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < top; k0 += U) {
+      V v[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (k0 + k < top)
+          v[k] = *reinterpret_cast<const V*>(reinterpret_cast<const E*>(y) + (long long)wp[k0 + k] * ldy + i);
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (k0 + k < top) {
+          if constexpr (DT == kF32) {
+            s[0] += v[k].x; s[1] += v[k].y; s[2] += v[k].z; s[3] += v[k].w;
+          } else {
+            s[0] += to_f32<DT>((uint16_t)(v[k].x & 0xffffu));
+            s[1] += to_f32<DT>((uint16_t)(v[k].x >> 16));
+            s[2] += to_f32<DT>((uint16_t)(v[k].y & 0xffffu));
+            s[3] += to_f32<DT>((uint16_t)(v[k].y >> 16));
+          }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = fmaf(alpha, s[e], o[e]);
+    if (whole)
+      *reinterpret_cast<float4*>(xr) = make_float4(o[0], o[1], o[2], o[3]);
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i + e < W) xr[e] = o[e];
   }
 }
 
