@@ -1,7 +1,7 @@
 // Four-wave MFMA GEMM tiles (plan cfg 22-35; shapes and schedules below): the projections of
 // prompts.
 //
-// Included by gemm_kernel.h (launch_gemm dispatches cfg 22-27 here); same GemmArgs, tile
+// Included by gemm_kernel.h (launch_gemm dispatches them here); same GemmArgs, tile
 // order, swizzled LDS image, fragment reads and epilogues as gemm_kernel's IL path.
 //
 // The shape of the winning library kernel on this chip (hipBLASLt's 256x256x64 tile,
@@ -85,6 +85,29 @@ __device__ __forceinline__ void amfma_dma(cf32x4& acc, const uint4& a, const uin
                  : "memory", "scc");
 }
 
+// ... and with the piece's offset in a register
+__device__ __forceinline__ void dma16_at(uint32_t mb, uint32_t off, uint32_t voff, cu32x4 d, uint32_t soff) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(mb), "v"(voff), "s"(d), "s"(soff), "s"(off) : "memory", "scc");
+}
+template <int DT>
+__device__ __forceinline__ void amfma_dma_at(cf32x4& acc, const uint4& a, const uint4& b, uint32_t mb,
+                                             uint32_t off, uint32_t voff, cu32x4 d, uint32_t soff) {
+  const cu32x4 av = __builtin_bit_cast(cu32x4, a), bv = __builtin_bit_cast(cu32x4, b);
+  if constexpr (DT == kBF16)
+    asm volatile("s_add_u32 m0, %3, %7\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\t"
+                 "buffer_load_dwordx4 %4, %5, %6 offen lds"
+                 : "+a"(acc)
+                 : "v"(av), "v"(bv), "s"(mb), "v"(voff), "s"(d), "s"(soff), "s"(off)
+                 : "memory", "scc");
+  else
+    asm volatile("s_add_u32 m0, %3, %7\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\t"
+                 "buffer_load_dwordx4 %4, %5, %6 offen lds"
+                 : "+a"(acc)
+                 : "v"(av), "v"(bv), "s"(mb), "v"(voff), "s"(d), "s"(soff), "s"(off)
+                 : "memory", "scc");
+}
+
 // SCHED 1: three barriers a k step (the DMAs of step t+2 issued as soon as every wave has read the
 // operand region they overwrite).  SCHED 2: one barrier, for tiles of which the LDS holds three or
 // four k steps.  A step of a small tile is bound by its waits, not by the matrix cores: 192 x 192 is
@@ -126,7 +149,8 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   // at 2048 tokens: 896 tiles = 3 full waves + 128 tiles in halves), or every tile in pieces
   // when there are too few.  Equal pieces of all tiles walk k side by side and share their
   // operands in L2, so an XCD takes neighbouring tiles of one piece (with the pieces of a tile side
-  // by side it read most of both operands: 1100 x 4096 x 23552 in 224 x 192 tiles 203 us, 191 so); one line of k steps cut into 256 equal shares (a tile's pieces at any k)
+  // by side it read most of both operands: 1100 x 4096 x 23552 in 224 x 192 tiles 203 us, 191 so);
+  // one line of k steps cut into 256 equal shares (a tile's pieces at any k)
   // balanced better and ran at half the rate, every workgroup reading for itself.
   if constexpr (GRP) g.tiles_m = g.groups[g.tiles_m].x;
   const int ntiles = g.tiles_m * g.tiles_n;
@@ -172,9 +196,14 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   // with the waves' rows 8 apart (one 32-row group an instruction) the rows in flight at a time met on
   // few channels of the memory where k is an odd multiple of 1024 or so (8 x 32 tiles of 128 x 256, k
   // 5120 95 -> 77 us, 23552 364 -> 340, 28672 460 -> 402; 256 x 256 148 -> 130, 624 -> 588, 805 -> 699)
+  // SCHED 0 takes weight rows of 4096, 8192, .. the other way, since there the rows that waves have side by
+  // side are the ones that meet: 6000 x 28672 x 4096 SwiGLU 1063 us side by side, 1047 8 rows apart,
+  // plain 1094, 1062; 2048 x 16384 x 2048 103.9, 104.8.  (SCHED 1 is even there.)
   constexpr int NB = IPW - NA;
+  constexpr bool EITHER = SCHED == 0 && !GRP;
+  const bool apart = EITHER && g.ldb >= 4096 && (g.ldb & (g.ldb - 1)) == 0;
   const int l8 = lane >> 3;
-  const int rA = wave * (NA * 8) + l8, rB = wave * (NB * 8) + l8;
+  const int rA = wave * (apart ? 8 : NA * 8) + l8, rB = wave * (apart ? 8 : NB * 8) + l8;
   const int chunk_a = (lane & 7) ^ ((rA >> 1) & 7), chunk_b = (lane & 7) ^ ((rB >> 1) & 7);
   // (grouped: weights from this tile's first row on, so that a tile, not a weight, is under 2 GB)
   const long long brows = GRP ? min(BN, g.Nv - n0) : g.gated ? 2LL * g.half : (long long)g.Nv;
@@ -182,19 +211,20 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   const int nrec_b = (int)(((brows - 1) * g.ldb + g.K) * 2);
   // scalar byte offsets of each instruction's rows: loop-invariant SGPRs.  Gated: virtual rows 32 b ..
   // are 16 gate rows from 16 b on and the 16 up rows beside them
-  const uint32_t gstride_a = (uint32_t)(8LL * g.lda * 2);
+  const uint32_t gstride_a = (uint32_t)((apart ? 32LL : 8LL) * g.lda * 2);
   uint32_t soff_b[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
-    const int q = wave * NB + j;
-    const long long row = !g.gated ? 8 * j : q / 4 * 16 + q % 2 * 8 + (q % 4 < 2 ? 0 : g.half);
+    const int q = apart ? 4 * j + wave : wave * NB + j;
+    const long long row = !g.gated ? (apart ? 32 : 8) * j : q / 4 * 16 + q % 2 * 8 + (q % 4 < 2 ? 0 : g.half);
     soff_b[j] = __builtin_amdgcn_readfirstlane((uint32_t)(row * g.ldb * 2));
   }
   const long long brow0 = GRP ? rB : g.gated ? n0 / 2 + l8 : n0 + rB;
   // byte offsets of this lane, of the even and the odd instructions (rows 8 on: the chunk's bit 2)
+  const int odd = apart ? 0 : 4;
   const auto voff = [](long long row, long long ld, int chunk) { return (uint32_t)((row * ld + chunk * 8) * 2); };
-  const uint32_t voff_a[2] = {voff(m0 + rA, g.lda, chunk_a), voff(m0 + rA, g.lda, chunk_a ^ 4)};
-  const uint32_t voff_b[2] = {voff(brow0, g.ldb, chunk_b), voff(brow0, g.ldb, chunk_b ^ 4)};
+  const uint32_t voff_a[2] = {voff(m0 + rA, g.lda, chunk_a), voff(m0 + rA, g.lda, chunk_a ^ odd)};
+  const uint32_t voff_b[2] = {voff(brow0, g.ldb, chunk_b), voff(brow0, g.ldb, chunk_b ^ odd)};
   // The k step lives in the descriptors: base advanced to the step's first column and
   // num_records shrunk by as much (a step past the split's end: 0 records, every lane out
   // of range -> zeros, no memory traffic).  Per DMA that leaves the M0 write and the DMA
@@ -212,8 +242,9 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   };
   auto src_a = [&](int step) __attribute__((always_inline)) { return desc_at(g.a, nrec_a, step); };
   auto src_b = [&](int step) __attribute__((always_inline)) { return desc_at(g.b, nrec_b, step); };
-  const uint32_t m0_a = __builtin_amdgcn_readfirstlane(lds_off(smem) + (uint32_t)wave * (NA * 1024));
-  const uint32_t m0_b = __builtin_amdgcn_readfirstlane(lds_off(smem) + BM * 128u + (uint32_t)wave * (NB * 1024));
+  const uint32_t m0_a = __builtin_amdgcn_readfirstlane(lds_off(smem) + (uint32_t)wave * (apart ? 1024 : NA * 1024));
+  const uint32_t m0_b = __builtin_amdgcn_readfirstlane(lds_off(smem) + BM * 128u + (uint32_t)wave * (apart ? 1024 : NB * 1024));
+  const uint32_t piece_b = apart ? 4096 : 1024;   // LDS bytes from an instruction's rows to the next one's
   // M0 (= buffer base + 1 KiB per piece, the piece offset an immediate) / voffset / soffset
   // of DMA I (A pieces for I < NA) into buffer buf
   auto dma_mb = [&](int buf, int i) __attribute__((always_inline)) {
@@ -240,14 +271,19 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
   auto stage_one = [&](const cu32x4& sa, const cu32x4& sb, int buf, auto I)
                        __attribute__((always_inline)) {
     constexpr int i = decltype(I)::value;
-    dma16<(i < NA ? i : i - NA) * 1024>(dma_mb(buf, i), dma_voff(i), i < NA ? sa : sb, dma_soff(i));
+    constexpr int n = i < NA ? i : i - NA;
+    if constexpr (EITHER) dma16_at(dma_mb(buf, i), n * piece_b, dma_voff(i), i < NA ? sa : sb, dma_soff(i));
+    else dma16<n * 1024>(dma_mb(buf, i), dma_voff(i), i < NA ? sa : sb, dma_soff(i));
   };
   // MFMA with DMA I fused behind it
   auto mfma_dma = [&](cf32x4& c, const uint4& a, const uint4& b, const cu32x4& sa,
                       const cu32x4& sb, int buf, auto I) __attribute__((always_inline)) {
     constexpr int i = decltype(I)::value;
-    amfma_dma<DT, (i < NA ? i : i - NA) * 1024>(c, a, b, dma_mb(buf, i), dma_voff(i), i < NA ? sa : sb,
-                                                dma_soff(i));
+    constexpr int n = i < NA ? i : i - NA;
+    if constexpr (EITHER)
+      amfma_dma_at<DT>(c, a, b, dma_mb(buf, i), n * piece_b, dma_voff(i), i < NA ? sa : sb, dma_soff(i));
+    else
+      amfma_dma<DT, n * 1024>(c, a, b, dma_mb(buf, i), dma_voff(i), i < NA ? sa : sb, dma_soff(i));
   };
   auto stage = [&](int step, int buf) {
     const cu32x4 sa = src_a(step), sb = src_b(step);
