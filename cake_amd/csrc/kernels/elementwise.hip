@@ -152,57 +152,33 @@ __global__ __launch_bounds__(256) void rope_kv_vec_kernel(
   const int nrope = (nh + nkv) * hv, nv = nkv * (hd >> 3);
   // the token's rotation angles once (shared by its nh + nkv heads), not per head
   __shared__ float s_sn[128], s_cs[128];
-  // a block is one token's chain of request, angles and stores: two pieces a thread are asked for before
-  // the angles are worked out (32 + 8 heads of 128: 45 tokens 4.7 -> 3.8 us; 6000 tokens, bound by
-  // their 147 MB, 24.7 both ways)
-  constexpr int NP = 2;
-  uint4 xa[NP], xb[NP];
-  auto ask = [&](int e, int p) __attribute__((always_inline)) {
-    if (p < nrope) {
-      const int head = p / hv, i0 = (p - head * hv) * 8;
-      const uint16_t* src = head < nh ? q + (size_t)t * ldq + head * hd : k + (size_t)t * ld + (head - nh) * hd;
-      xa[e] = *reinterpret_cast<const uint4*>(src + i0);
-      xb[e] = *reinterpret_cast<const uint4*>(src + i0 + half);
-    } else if (p < nrope + nv) {
-      xa[e] = *reinterpret_cast<const uint4*>(v + (size_t)t * ld + (p - nrope) * 8);
-    }
-  };
-  auto put = [&](int e, int p) __attribute__((always_inline)) {
+  for (int i = threadIdx.x; i < half; i += blockDim.x) sincosf((float)pos * inv_freq[i], &s_sn[i], &s_cs[i]);
+  __syncthreads();
+  for (int p = threadIdx.x; p < nrope + nv; p += blockDim.x) {
     if (p < nrope) {
       const int head = p / hv, i0 = (p - head * hv) * 8;
       const bool isq = head < nh;
       const int hh = isq ? head : head - nh;
+      const uint16_t* src = isq ? q + (size_t)t * ldq + hh * hd : k + (size_t)t * ld + hh * hd;
       float a[8], b[8];
-      unpack8<DT>(xa[e], a);
-      unpack8<DT>(xb[e], b);
+      unpack8<DT>(*reinterpret_cast<const uint4*>(src + i0), a);
+      unpack8<DT>(*reinterpret_cast<const uint4*>(src + i0 + half), b);
       uint16_t oa[8], ob[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float sn = s_sn[i0 + j], cs = s_cs[i0 + j];
-        oa[j] = from_f32<DT>(a[j] * cs - b[j] * sn);
-        ob[j] = from_f32<DT>(a[j] * sn + b[j] * cs);
+      for (int e = 0; e < 8; ++e) {
+        const float sn = s_sn[i0 + e], cs = s_cs[i0 + e];
+        oa[e] = from_f32<DT>(a[e] * cs - b[e] * sn);
+        ob[e] = from_f32<DT>(a[e] * sn + b[e] * cs);
       }
       uint16_t* dst = isq ? q + (size_t)t * ldq + hh * hd : kc + ((size_t)hh * S + pos) * hd;
       *reinterpret_cast<uint4*>(dst + i0) = *reinterpret_cast<const uint4*>(oa);
       *reinterpret_cast<uint4*>(dst + i0 + half) = *reinterpret_cast<const uint4*>(ob);
-    } else if (p < nrope + nv) {
+    } else {
       const int pp = p - nrope, per = hd >> 3;
       const int head = pp / per, c = (pp - head * per) * 8;
-      *reinterpret_cast<uint4*>(vc + ((size_t)head * S + pos) * hd + c) = xa[e];
+      *reinterpret_cast<uint4*>(vc + ((size_t)head * S + pos) * hd + c) =
+          *reinterpret_cast<const uint4*>(v + (size_t)t * ld + head * hd + c);
     }
-  };
-  const int p0 = threadIdx.x, step = blockDim.x;
-#pragma unroll
-  for (int e = 0; e < NP; ++e) ask(e, p0 + e * step);
-  for (int i = threadIdx.x; i < half; i += blockDim.x) sincosf((float)pos * inv_freq[i], &s_sn[i], &s_cs[i]);
-  __syncthreads();
-  for (int p = p0; p < nrope + nv; p += NP * step) {
-    if (p != p0) {
-#pragma unroll
-      for (int e = 0; e < NP; ++e) ask(e, p + e * step);
-    }
-#pragma unroll
-    for (int e = 0; e < NP; ++e) put(e, p + e * step);
   }
 }
 
