@@ -184,68 +184,76 @@ CAKE_API long long cake_gemm_ws_floats(int cfg, int splits, int M, int N, int K,
 }
 
 // ---- tile plan of a size that has no measured entry ------------------------
-// t(us) = c0 + step (k steps of all rounds) + lone (k steps a thin round loses to latency; four-wave
-//         tiles: gains, its operands come faster; those steps at least at the memory's rate)
+// t(us) = c0 + step (1 + many (whole rounds, up to 4)) (k steps of all rounds) + lone (k steps a thin
+//         round loses to latency; four-wave tiles: gains), these at least mem (MB of operands)
 //         + epi[class] rounds + merge [split] + fin (split: MB of slabs written and read, or pieces)
-// fitted to timings on weights that no cache holds.  The four-wave tiles: 38,000 of every tile and split
-// that fills up to 256 workgroups, 38 products (width 1024 .. 8192, k 512 .. 28672), 70 .. 6000 rows.
-// Over these the plan is 5 % off the best of all tiles at 70 and 100 rows, 2.5 % from 130, 1.4 % from
-// 700 (at most 48 %).  From 300 rows on the eight-wave tiles and the 160 columns are the best nowhere by
-// more than 1 %; where four-wave tiles can run they are left out there (with them, 2 - 4 % off).
+// fitted to timings on weights that no cache holds, of every tile and split: 4,200 products (width 128 ..
+// 60000, k 512 .. 29000, 2 .. 6000 rows); wrong choices weighed more than wrong times.  Over these the
+// plan is 1 % off the best of all on the average, 0.7 % over the widths of named models.  Fitted
+// before tile 22 had its rows 8 apart and the slabs their 16-byte reads, and without the eight-wave
+// tiles from 300 rows on, it was 4 %: 6000 x 57344 x 8192 SwiGLU 4250 us on 224 x 192, 3970 on 256 x 256;
+// 350 x 2048 x 11776 43.4 on 128 x 128 in pieces, 34.9 on 256 x 128 in slabs; 113 x 57344 x 8192 SwiGLU,
+// where all wait for the weights, 186 on 128 x 128, 169 on 128 x 256.
 // An image model's products are short (k from 128) or have a 16-bit residual or GEGLU: the tile's end
-// weighs as much as its k steps, so these have epilogue terms of their own, and three tiles more.
+// weighs as much as its k steps, so these have rows of their own, and three tiles more.
 // Over 123 sizes (width 256 .. 2048, 66 .. 18432 rows) 1.5 % off the best on the average, at most 15;
 // without the terms 5.5 %, at most 58 (12288 x 320 x 320 + residual 17.3 us, 11.0 so; 6144 x 5120 x
 // 640 GEGLU 59.6, 50.8).
 struct TileCost {
   int cfg, bm, bn, slots;                  // slots: workgroups a CU holds
-  // epi: store, f32, SwiGLU, SiLU / GELU, 16-bit residual, GEGLU, store of k < 512; negative epi or
+  // epi: store, f32, SwiGLU, GELU, 16-bit residual, GEGLU, store of k < 512; negative epi or
   // merge: not modelled (that epilogue, that tile in splits)
-  float c0, step, lone, epi[7], merge, fin;
+  float c0, step, many, lone, mem, epi[7], merge, fin;
 };
 static constexpr TileCost kTileCosts[] = {
-    {4, 64, 64, 4, 1.48f, 0.787f, 0.263f, {-1.f, -1.f, -1.f, -1.f, 3.44f, 2.92f, 3.04f}, -1.f, 0.f},
-    {5, 256, 256, 1, 0.69f, 1.43f, 0.f, {5.52f, 7.84f, 9.9f, 6.58f, 11.7f, 9.55f, 8.55f}, 4.16f, 0.304f},
-    {6, 256, 128, 1, 0.844f, 0.802f, 0.f, {4.16f, 5.6f, 6.f, 4.4f, 7.42f, 6.68f, 6.1f}, 3.93f, 0.325f},
-    {7, 128, 128, 1, 2.77f, 0.539f, 0.f, {2.72f, 3.65f, 4.5f, 4.2f, 5.25f, 4.69f, 4.05f}, 3.6f, 0.382f},
-    {8, 128, 128, 2, 2.27f, 1.02f, 0.44f, {-1.f, -1.f, -1.f, -1.f, 5.46f, 4.78f, 4.01f}, -1.f, 0.f},
-    {12, 64, 128, 2, 4.62f, 0.663f, 0.145f, {0.f, 0.598f, 1.92f, 1.93f, 1.82f, 2.31f, -1.f}, 3.09f, 0.468f},
-    {13, 64, 64, 2, 3.41f, 0.427f, 0.107f, {0.79f, 1.37f, 2.48f, 2.18f, 2.f, 2.05f, 1.75f}, 2.83f, 0.484f},
-    {14, 64, 160, 2, 1.33f, 0.779f, 0.386f, {-1.f, -1.f, -1.f, -1.f, 5.97f, -1.f, 3.69f}, -1.f, 0.f},
-    {18, 64, 160, 1, 2.28f, 0.467f, 0.f, {2.54f, 3.f, 0.f, 4.42f, 5.07f, -1.f, 3.2f}, 3.53f, 0.353f},
-    {22, 256, 256, 1, 6.44f, 1.47f, -0.358f, {1.47f, 6.92f, 1.39f, 13.4f, -1.f, -1.f, -1.f}, 7.49f, 4.03f},
-    {25, 256, 256, 1, 6.3f, 1.48f, -0.326f, {2.65f, 8.21f, 2.78f, 14.1f, -1.f, -1.f, -1.f}, 7.48f, 3.77f},
-    {26, 256, 192, 1, 4.95f, 1.16f, -0.257f, {3.58f, 6.84f, 2.4f, 9.04f, -1.f, -1.f, -1.f}, 4.28f, 3.64f},
-    {27, 128, 256, 1, 4.95f, 0.852f, -0.207f, {1.05f, 3.4f, 1.26f, 5.45f, -1.f, -1.f, -1.f}, 4.05f, 2.27f},
-    {28, 128, 128, 1, 3.28f, 0.524f, -0.165f, {1.86f, 3.55f, 1.92f, 3.92f, -1.f, -1.f, -1.f}, 2.48f, 1.91f},
-    {29, 128, 192, 1, 3.45f, 0.686f, -0.167f, {3.17f, 4.18f, 2.68f, 6.09f, -1.f, -1.f, -1.f}, 3.29f, 1.99f},
-    {30, 96, 256, 1, 5.21f, 0.765f, -0.157f, {0.277f, 1.17f, 0.662f, 3.95f, -1.f, -1.f, -1.f}, 3.01f, 1.9f},
-    {31, 160, 256, 1, 3.56f, 0.948f, -0.261f, {4.f, 7.49f, 3.83f, 9.4f, -1.f, -1.f, -1.f}, 3.91f, 2.7f},
-    {32, 192, 192, 1, 2.11f, 0.83f, -0.223f, {6.11f, 8.94f, 5.05f, 10.1f, -1.f, -1.f, -1.f}, 3.34f, 2.76f},
-    {33, 224, 192, 1, 2.17f, 0.923f, -0.265f, {7.53f, 11.f, 5.97f, 12.f, -1.f, -1.f, -1.f}, 3.06f, 3.14f},
-    {34, 192, 256, 1, 6.79f, 1.23f, -0.245f, {0.621f, 4.06f, 1.1f, 7.72f, -1.f, -1.f, -1.f}, 4.24f, 3.18f},
-    {35, 224, 256, 1, 6.34f, 1.35f, -0.274f, {1.79f, 6.43f, 2.28f, 10.1f, -1.f, -1.f, -1.f}, 4.48f, 3.65f},
-    // four-wave tiles, the classes from kImageClass on
-    {22, 256, 256, 1, 0.f, 1.26f, 0.f, {-1.f, -1.f, -1.f, -1.f, 18.1f, 11.4f, 12.f}, 13.2f, 10.2f},
-    {25, 256, 256, 1, 0.f, 1.49f, 0.f, {-1.f, -1.f, -1.f, -1.f, 14.9f, 9.6f, 10.8f}, 20.8f, 13.2f},
-    {26, 256, 192, 1, 0.f, 1.13f, 0.f, {-1.f, -1.f, -1.f, -1.f, 13.1f, 9.73f, 9.91f}, 16.1f, 6.33f},
-    {27, 128, 256, 1, 4.43f, 0.837f, 0.f, {-1.f, -1.f, -1.f, -1.f, 6.33f, 4.58f, 3.86f}, 13.7f, 4.33f},
+    {5, 256, 256, 1, 1.315f, 1.423f, 0.0515f, 0.1f, 0.0978f, {8.12f, 12.76f, 9.355f, 10.28f, -1.f, -1.f, -1.f}, 0.465f, 0.211f},
+    {6, 256, 128, 1, 0.581f, 0.739f, 0.00913f, 0.1f, 0.0758f, {8.567f, 8.26f, 9.837f, 9.006f, -1.f, -1.f, -1.f}, 0.479f, 0.224f},
+    {7, 128, 128, 1, 2.447f, 0.492f, 0.00891f, 0.1f, 0.0668f, {5.312f, 5.424f, 5.552f, 6.45f, -1.f, -1.f, -1.f}, 0.791f, 0.198f},
+    {12, 64, 128, 2, 0.935f, 0.855f, -0.0328f, -0.0607f, 0.104f, {2.788f, 2.795f, 2.913f, 3.841f, -1.f, -1.f, -1.f}, 2.088f, 0.287f},
+    {13, 64, 64, 2, 0.356f, 0.547f, 0.1f, 0.0549f, 0.00984f, {0.416f, 0.656f, 0.489f, 1.683f, -1.f, -1.f, -1.f}, 2.649f, 0.448f},
+    {18, 64, 160, 1, 1.177f, 0.457f, 0.00266f, 0.1f, 0.0426f, {4.479f, 4.01f, -1.f, 4.044f, -1.f, -1.f, -1.f}, 1.721f, 0.209f},
+    {22, 256, 256, 1, 1.152f, 1.098f, 0.0174f, 0.128f, 0.176f, {9.638f, 16.22f, 10.07f, 19.8f, -1.f, -1.f, -1.f}, 13.95f, 7.829f},
+    {25, 256, 256, 1, 0.661f, 1.093f, 0.0424f, 0.209f, 0.0386f, {15.45f, 18.81f, 8.939f, 14.98f, -1.f, -1.f, -1.f}, 1.337f, 9.021f},
+    {26, 256, 192, 1, 0.12f, 0.916f, 0.0398f, 0.127f, 0.125f, {8.747f, 12.5f, 9.162f, 13.78f, -1.f, -1.f, -1.f}, 6.793f, 3.485f},
+    {27, 128, 256, 1, 0.489f, 0.657f, 0.11f, 0.169f, 0.113f, {4.901f, 7.49f, 4.916f, 11.28f, -1.f, -1.f, -1.f}, 3.05f, 3.666f},
+    {28, 128, 128, 1, 0.564f, 0.443f, 0.0724f, 0.0141f, 0.119f, {3.183f, 3.551f, 3.063f, 6.329f, -1.f, -1.f, -1.f}, 1.816f, 2.725f},
+    {29, 128, 192, 1, 0.158f, 0.513f, 0.11f, 0.237f, 0.18f, {6.195f, 6.798f, 5.003f, 8.104f, -1.f, -1.f, -1.f}, 6.417f, 2.032f},
+    {30, 96, 256, 1, 0.562f, 0.635f, 0.043f, 0.142f, 0.149f, {3.821f, 5.301f, 3.733f, 8.382f, -1.f, -1.f, -1.f}, 3.125f, 3.253f},
+    {31, 160, 256, 1, 0.797f, 0.711f, 0.0445f, 0.0764f, 0.127f, {7.909f, 11.57f, 7.589f, 13.52f, -1.f, -1.f, -1.f}, 3.749f, 3.796f},
+    {32, 192, 192, 1, 1.316f, 0.62f, 0.0623f, 0.0716f, 0.127f, {7.468f, 10.46f, 6.705f, 11.87f, -1.f, -1.f, -1.f}, 4.369f, 3.521f},
+    {33, 224, 192, 1, 0.846f, 0.777f, 0.0146f, -0.0934f, 0.144f, {10.04f, 12.63f, 8.565f, 13.22f, -1.f, -1.f, -1.f}, 4.312f, 3.47f},
+    {34, 192, 256, 1, 1.768f, 0.979f, 0.0472f, 0.0879f, 0.126f, {6.113f, 10.06f, 6.451f, 13.14f, -1.f, -1.f, -1.f}, 2.423f, 4.585f},
+    {35, 224, 256, 1, 1.053f, 1.076f, 0.045f, 0.148f, 0.113f, {7.659f, 11.94f, 7.822f, 13.64f, -1.f, -1.f, -1.f}, 6.25f, 4.798f},
+    // products of image models: the classes from kImageClass on
+    {4, 64, 64, 4, 1.48f, 0.787f, 0.f, 0.263f, 0.f, {-1.f, -1.f, -1.f, -1.f, 3.44f, 2.92f, 3.04f}, -1.f, 0.f},
+    {5, 256, 256, 1, 0.69f, 1.43f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 11.7f, 9.55f, 8.55f}, 4.16f, 0.304f},
+    {6, 256, 128, 1, 0.844f, 0.802f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 7.42f, 6.68f, 6.1f}, 3.93f, 0.325f},
+    {7, 128, 128, 1, 2.77f, 0.539f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 5.25f, 4.69f, 4.05f}, 3.6f, 0.382f},
+    {8, 128, 128, 2, 2.27f, 1.02f, 0.f, 0.44f, 0.f, {-1.f, -1.f, -1.f, -1.f, 5.46f, 4.78f, 4.01f}, -1.f, 0.f},
+    {12, 64, 128, 2, 4.62f, 0.663f, 0.f, 0.145f, 0.f, {-1.f, -1.f, -1.f, -1.f, 1.82f, 2.31f, -1.f}, 3.09f, 0.468f},
+    {13, 64, 64, 2, 3.41f, 0.427f, 0.f, 0.107f, 0.f, {-1.f, -1.f, -1.f, -1.f, 2.f, 2.05f, 1.75f}, 2.83f, 0.484f},
+    {14, 64, 160, 2, 1.33f, 0.779f, 0.f, 0.386f, 0.f, {-1.f, -1.f, -1.f, -1.f, 5.97f, -1.f, 3.69f}, -1.f, 0.f},
+    {18, 64, 160, 1, 2.28f, 0.467f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 5.07f, -1.f, 3.2f}, 3.53f, 0.353f},
+    {22, 256, 256, 1, 0.f, 1.26f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 18.1f, 11.4f, 12.f}, 13.2f, 10.2f},
+    {25, 256, 256, 1, 0.f, 1.49f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 14.9f, 9.6f, 10.8f}, 20.8f, 13.2f},
+    {26, 256, 192, 1, 0.f, 1.13f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 13.1f, 9.73f, 9.91f}, 16.1f, 6.33f},
+    {27, 128, 256, 1, 4.43f, 0.837f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 6.33f, 4.58f, 3.86f}, 13.7f, 4.33f},
 };
 // 0 .. 6, as TileCost::epi; from kImageClass on the products of image models
 static constexpr int kImageClass = 4;
 static int cost_class(int epi, int K) {
-  return epi == kEpiResid32 || epi == kEpiStore32                 ? 1
-         : epi == kEpiSwiglu                                      ? 2
-         : epi == kEpiSilu || epi == kEpiQuick || epi == kEpiGelu ? 3
-         : epi == kEpiAdd16                                       ? 4
-         : epi == kEpiGeglu                                       ? 5
-         : epi == kEpiStore && K < 512                            ? 6 : 0;
+  return epi == kEpiResid32 || epi == kEpiStore32 ? 1
+         : epi == kEpiSwiglu                      ? 2
+         : epi == kEpiGelu                        ? 3
+         : epi == kEpiAdd16                       ? 4
+         : epi == kEpiGeglu                       ? 5
+         : epi == kEpiStore && K < 512            ? 6 : 0;
 }
 static double tile_cost(const TileCost& c, int splits, long long M, long long Nv, int K, int epi) {
   const long long ks = (K + kGBK - 1) / kGBK, t = ((M + c.bm - 1) / c.bm) * ((Nv + c.bn - 1) / c.bn);
   const int cls = cost_class(epi, K);
   if (c.epi[cls] < 0 || (splits > 1 && c.merge < 0)) return -1;   // not modelled
-  double steps, rounds, lone = 0, fin = 0;
+  double steps, rounds, whole, lone = 0, fin = 0;
   bool split = false;
   if (four_wave_cfg(c.cfg)) {
     const SplitPlan p = split_plan(c.cfg, splits, (int)M, Nv, K);
@@ -254,6 +262,7 @@ static double tile_cost(const TileCost& c, int splits, long long M, long long Nv
     const long long dp = (t - rest) / 256, per = p.pieces ? p.kps / kGBK : ks;
     steps = (double)(dp * ks + (rest ? per : 0));
     rounds = (double)(dp + (rest ? 1 : 0));
+    whole = (double)dp;
     split = p.pieces > 0;
     fin = p.pieces;
     if (rest) lone = per * (1 - (double)rest * std::max(p.pieces, 1) / 256);
@@ -263,26 +272,29 @@ static double tile_cost(const TileCost& c, int splits, long long M, long long Nv
     const double share = (double)((rest + 255) / 256) / c.slots;   // of a round's slots on a CU
     steps = (double)kps * (full + share);
     rounds = (double)(full + (rest ? 1 : 0));
+    whole = (double)full;
     lone = rest ? (1 - share) * kps : 0;
     split = sp > 1;
     if (split) fin = (double)(sp + 1) * M * Nv * 4e-6;
   }
-  double main = c.step * steps + c.lone * lone;
-  if (four_wave_cfg(c.cfg)) main = std::max(main, ((double)Nv * K + (double)M * K) * 2 / 5.2e6);
-  const double us = c.c0 + main + c.epi[cls] * rounds + (split ? c.merge + c.fin * fin : 0.);
-  // operands from memory; of tiles that all wait for them the one with the least work (113 x 57344 x
-  // 8192 SwiGLU 193 us on 128 x 256, 209 on 128 x 128)
-  return std::max(us, ((double)Nv * K + (double)M * K) * 2 / 5e6 + 3) + 0.02 * us;
+  const double mb = ((double)Nv * K + (double)M * K) * 2e-6;
+  const bool image = cls >= kImageClass;
+  const double mem = !image ? c.mem * mb : four_wave_cfg(c.cfg) ? mb / 5.2 : 0.;
+  const double main = c.step * (1 + c.many * std::min(whole, 4.)) * steps + c.lone * lone;
+  const double us = c.c0 + std::max(main, mem) + c.epi[cls] * rounds +
+                    (split ? c.merge + c.fin * fin : 0.);
+  // operands from memory; of tiles that all wait for them the one with the least work
+  return image ? std::max(us, mb / 5 + 3) + 0.02 * us : us;
 }
 
-// (cfg, splits) for a product on tiles.  The estimate is fitted from 65 rows on; captured products of
-// fewer, whose stream form stays out of graphs, take it too (2 .. 64 rows of 14 weight shapes in
-// graphs: 0.93 to 2.6 times as fast as the plan of the nearest measured size).  On entry *cfg,
-// *splits: a measured plan of this very size, or cfg -1; it stands unless it is modelled and 10 %
-// behind the best.  big: an operand of 2 GB or more (31-bit offsets of the four-wave tiles).
+// (cfg, splits) for a product on tiles; of 64 rows and fewer captured ones, whose stream form stays out
+// of graphs.  On entry *cfg, *splits: a measured plan of this very size, or cfg -1; it stands unless it
+// is modelled and 10 % behind the best.  big: an operand of 2 GB or more (31-bit offsets of the
+// four-wave tiles).
 CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits) {
   if (M < 1 || Nv < 1 || K < 1 || !cfg || !splits) return (int)hipErrorInvalidValue;
   const bool gated = epi == kEpiSwiglu || epi == kEpiGeglu;
+  const bool image = cost_class(epi, K) >= kImageClass;
   const int ks = (K + kGBK - 1) / kGBK;
   double best = 1e30, given = -1;
   int bc = 0, bs = 1;
@@ -291,14 +303,13 @@ CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* c
     if (c.cfg == *cfg) given = std::max(given, tile_cost(c, *splits, M, Nv, K, epi));
     if (four && (K % kGBK || big)) continue;
     if (gated && c.cfg == 18) continue;               // 80-column wave tiles
-    if (M >= 300 && K % kGBK == 0 && !big && cost_class(epi, K) < kImageClass &&
-        (c.cfg == 5 || c.cfg == 6 || c.cfg == 7 || c.cfg == 18))
-      continue;
-    // long rows of k: the three-barrier schedule of the 256 x 256 tile (8192 x 28672 at 2048 rows
-    // 726 against 800 us), else the two-stage one (8192 x 8192 199 against 206)
-    if ((c.cfg == k4WCfg && K > 8192) || (c.cfg == k4WCfg + k4WSched && K <= 8192)) continue;
+    if (!image && c.bm > 2.2 * std::max(M, 64)) continue;   // mostly padding: not in the fit
+    // 256 x 256: three barriers a step for long rows of k, else two (k 8192 4.6 % faster, 11776 4.9, 14336
+    // 0.8 slower, 23552 2.4; an image model's line as fitted)
+    const bool three = K > (image ? 8192 : 12288);
+    if (c.cfg == (three ? k4WCfg : k4WCfg + k4WSched)) continue;
     for (int sp : {1, 2, 3, 4, 6, 8, 16}) {
-      if (sp > 1 && (ks / sp < 4 || (four && M < 200))) break;
+      if (sp > 1 && (ks / sp < 4 || (four && image && M < 200))) break;
       if (!four && (sp & (sp - 1))) continue;
       const double t = tile_cost(c, sp, M, Nv, K, epi);
       if (t >= 0 && t < best) {

@@ -60,6 +60,37 @@ def test_estimate_picks_a_measured_best(monkeypatch, size, times):
     assert splits == 1 and times[cfg] <= 1.1 * min(times.values())
 
 
+@pytest.mark.parametrize("size,times", [
+    # us of (tile, splits) on an MI355X, the fastest and some that an estimate has taken for them
+    ((6000, 57344, 8192, "swiglu"), {(22, 1): 3969, (25, 1): 4188, (33, 1): 4252}),
+    ((1800, 57344, 8192, "swiglu"), {(22, 1): 1275, (25, 1): 1306, (31, 2): 1354, (32, 1): 1393}),
+    ((3000, 10240, 8192, "store"), {(22, 1): 353, (31, 1): 374, (33, 1): 380}),
+    ((6000, 10240, 8192, "store"), {(22, 1): 746, (31, 1): 762, (33, 1): 775}),
+    ((1600, 8192, 8192, "resid32"), {(35, 1): 172.5, (22, 1): 178.8, (31, 4): 193.6}),
+    ((100, 57344, 8192, "swiglu"), {(27, 1): 169.5, (31, 1): 170.6, (28, 1): 179.2, (7, 1): 181.8}),
+    ((260, 4096, 14336, "resid32"), {(6, 4): 58.6, (28, 2): 59.7, (30, 4): 65.4}),
+    ((350, 2048, 11776, "resid32"), {(6, 8): 34.9, (7, 4): 38.0, (28, 4): 42.2}),
+    ((560, 1024, 4096, "resid32"), {(18, 4): 17.0, (7, 4): 18.8, (13, 1): 21.7}),
+    ((113, 16384, 2048, "swiglu"), {(12, 1): 21.9, (13, 1): 22.8, (28, 1): 24.2}),
+    ((512, 5120, 1280, "gelu"), {(18, 1): 17.9, (28, 1): 19.2, (7, 1): 20.5}),
+    ((1200, 5120, 1280, "gelu"), {(6, 1): 27.2, (32, 1): 27.6, (27, 1): 28.9})], ids=str)
+def test_estimate_picks_a_measured_best_of_all_splits(monkeypatch, size, times):
+    """Prompts of wide models, tiles that wait for the weights, short k: within 4 % of the best."""
+    from cake_amd.ops import gemm as G
+    monkeypatch.setattr(G, "_TUNED", [])
+    monkeypatch.setattr(G, "_resolved", {})
+    assert times[G.resolve(*size)] <= 1.04 * min(times.values())
+
+
+@pytest.mark.parametrize("M,Nv", [(3072, 57344), (2500, 57344), (1024, 28672), (1024, 14336)])
+def test_measured_eight_wave_tiles_behind_the_four_wave_ones(monkeypatch, M, Nv):
+    """3072 x 57344 x 8192 SwiGLU on 256 x 256: eight waves 2326 us, four 2056; 2500 rows 1902, 1688."""
+    from cake_amd.ops import gemm as G
+    monkeypatch.setattr(G, "_TUNED", [{"M": M, "Nv": Nv, "K": 8192, "epi": "swiglu", "cfg": 5, "splits": 1}])
+    monkeypatch.setattr(G, "_resolved", {})
+    assert G.resolve(M, Nv, 8192, "swiglu")[0] == 22
+
+
 def test_library_plan_falls_back_to_the_plan_without_it(monkeypatch):
     """A call that the library form does not carry (a bias) runs what a table without the library's
     entries plans, as the native engines do, not the nearest measured size."""
