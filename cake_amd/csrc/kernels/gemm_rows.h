@@ -330,12 +330,16 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
   // ---- DMA: wave w fetches weight rows 16 RT w .. and its share of x ----
   const int dr = lane / S::LPR, dslot = lane % S::LPR;   // row within an instruction's, slot
   int ds = u0 / KS, dk = u0 % KS, dnext = u0;
-  // shares of whole strips, or of equal parts of one, start at different k each: the strips lie the same
-  // distance apart, and in step they would ask the same channels of the memory at a time (28672 x 4096
-  // in 224 whole strips 46.8 us in step, 39.6 so; 32000 x 4096 in 250 56.8, 42.2)
+  // shares of whole strips start 5 steps on from the share before them, equal parts of one from the strip
+  // before: strips lie the same distance apart, and in step they would ask the same channels of the
+  // memory at a time (28672 x 4096 in 224 whole strips 46.8 us in step, 39.6 so; 12288 x 4096 in 192
+  // halves at 24 rows 28.1, 23.1; each half 5 steps on 25.5).  128-row parts that are no multiple of 4 KB apart spread by
+  // themselves, and in step read x together (4096 x 14336 in 256 eighths of 3.5 KB at 24 rows 25.9, 26.7
+  // turned; 8192 x 28672 at 64 rows 85.1, 86.7; of 64 rows, two on a CU, at 5 rows 88.3, 71.3 turned).
   const int seg = KS % per == 0 ? per : per % KS == 0 ? KS : 0;   // 0: other shares
+  const bool turn = seg == KS || S::KC == 2 || seg * KST * 2 % 4096 == 0;
   const int seg0 = seg > 0 ? dk / seg * seg : 0;
-  if (seg > 0) dk = seg0 + wg * 5 % seg;
+  if (seg > 0 && turn) dk = seg0 + u0 / max(per, KS) * 5 % seg;
   int left = seg;
   const uint16_t *wsrc[4], *xsrc[S::XI];
   auto aim = [&](int s) {
