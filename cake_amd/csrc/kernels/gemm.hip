@@ -400,14 +400,15 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
 
 // ---- products of few rows (gemm_rows.h) -----------------------------------
 // Which form a product of M rows takes: 0 the tile kernels (cake_gemm_scaled), 1 direct, 2 stream.
-// The estimates (us) are fits to timings on weights that no cache holds, 2 .. 64 rows of 24 weight
-// shapes, 1 .. 940 MB: the form they pick is 1.1 % off the best of the three on the average.  Both sides
-// of the lines they draw, measured: 4096 x 4096 at 16 rows direct 11.8, stream 12.1; 4096 x 14336
-// direct 37, stream 23; 6144 x 4096 at 5 rows direct 16.9, stream 14.5, 3072 x 2048 6.5, 7.9; 28672 x
-// 4096 at 45 rows stream 40, tiles 55; 6144 x 4096 at 45 rows stream 18.4, tiles 19.4, 4096 x 11008
-// 31.0, 27.9.  Rows of k that start amid a 128-byte line (k no multiple of 64) cost a second line at
-// either end of a piece: 4096 x 10928 against 4096 x 11008, 5 rows direct 31.4 / 23.6, stream 23.5 /
-// 20.5, 33 rows stream 35.0 / 29.5, tiles 29.4 / 27.1.
+// The estimates (us) are fits to timings on weights that no cache holds, 2 .. 64 rows of 80 weight
+// shapes, 0.2 .. 940 MB, every form and share; wrong choices weighed more than wrong times: what they pick
+// is 0.4 % off the best of all on the average, at most 16 %.  Both sides of the lines they draw, measured:
+// 3072 x 2048 at 5 rows direct 6.7, stream 8.4; 4096 x 4096 at 5 rows 10.3, 11.5, at 16 12.4, 11.7 (tiles
+// 12.1), at 24 tiles 12.4, stream 15.0; 4096 x 14336 at 24 rows stream 26.6, tiles 27.5, at 33 30.1, 27.8;
+// 6144 x 4096 at 16 rows stream 14.3, tiles 15.7, at 33 18.3, 16.7; 8192 x 8192 at 24 rows stream 29.6,
+// tiles 37.1; 28672 x 4096 SwiGLU at 64 rows 41.5, 51.8.  Rows of k that start amid a 128-byte line (k no
+// multiple of 64) cost a second line at either end of a piece: 4096 x 10928 against 4096 x 11008, 5 rows
+// direct 31.9 / 24.1, stream 21.0 / 20.1, 33 rows stream 36.1 / 30.9, tiles 26.3 / 25.2.
 struct StreamPlan {
   int bn, kst, most;   // weight rows of a strip, k of a step (gemm_rows.h StreamShape), workgroups at most
   int wgs, per;        // workgroups, steps of each
@@ -415,40 +416,43 @@ struct StreamPlan {
 };
 // The shares: as many as there are workgroups at most, of equal length wherever that ends, or whole
 // strips, or equal parts of one.  The latter two park no sums, or one a share, and never wait for them
-// amid a share; with fewer workgroups a CU takes up to 42 KB a us of weights, all of them 7.0 MB.  At 24 /
-// 45 rows, 256 shares against the best of the others: 28672 x 4096 SwiGLU 46.8 / 50.5 -> 38.2 / 39.6 us
-// (224 whole strips), 19456 x 4096 37.9 / 42 -> 30.7 / 36.7 (152), 6144 x 4096 17.2 / 22.1 -> 16.0 / 18.4
-// (192 quarters), 2048 x 8192 18 / 25.6 -> 15.6 / 21.3 (128 eighths); 4096 x 14336 stays at 24 rows, 25.6
-// (128 quarters 32), and takes tiles at 45, 30.4 (32.2).
+// amid a share; with fewer workgroups a CU takes up to 42 KB a us of weights, all of them 7.3 MB.
+// At 24 / 45 rows, 256 shares that end anywhere against the best of the others: 28672 x 4096 SwiGLU 45.8 /
+// 50.4, 38.9 / 39.9 us (224 whole strips), 19456 x 4096 37.5 / 41.4, 31.5 / 37.5 (152), 6144 x 4096 17.6 /
+// 22.3, 16.3 / 19.1 (192 quarters), 12288 x 4096 24.7 / 27.1, 23.5 / 26.8 (192 halves); 10240 x 8192 35.2 /
+// 38.7, 35.7 / 42.3 (160 halves).  8192 x 8192, 256 quarters: 29.6 / 30.9.
 static StreamPlan stream_plan(int M, long long Nv, int K, bool gated) {
   const int mt = (M + 15) / 16;
   StreamPlan p = mt > 1 || gated ? StreamPlan{128, 64, 256, 0, 0, 1e30} : StreamPlan{64, 128, 512, 0, 0, 1e30};
   const long long strips = (Nv + p.bn - 1) / p.bn, ks = (K + p.kst - 1) / p.kst, total = strips * ks;
   const int least = kRowsMinK / p.kst;
-  const bool mid = K % 64 != 0;   // rows start amid a line
+  const double mid = K % 64 != 0 ? 1 : 0;   // rows start amid a line
   const auto take = [&](long long wgs, long long per, double us) {
     if (us < p.us) { p.wgs = (int)wgs; p.per = (int)per; p.us = us; }
   };
-  // a strip's shares, parked and summed
-  const auto sums = [&](double shares, double each) { return mt * (0.86 * std::min(shares, 1.) + each * shares); };
-  for (int most = p.most; most >= 256; most /= 2) {   // ends anywhere
+  for (int most = p.most; most >= 256; most /= 2) {   // ends anywhere; a strip's shares are parked and summed
     const long long per = std::max<long long>((total + most - 1) / most, least);
     const long long wgs = (total + per - 1) / per;
-    const double shares = (double)ks / per;
+    const double shares = (double)ks / per, met = std::min(shares, 1.);
     if (ks % per == 0 || per % ks == 0) continue;   // below
-    if (most == 512) take(wgs, per, 6.2 + 0.08 * M + (1.42 + (mid ? 0.11 : 0.)) * per);
-    else if (p.most == 512) take(wgs, per, 4.5 + 0.04 * M + sums(shares, 0.25) + (0.62 + (mid ? 0.11 : 0.)) * per);
-    else take(wgs, per, (mt > 1 ? 3 : 4.3) + sums(shares, 0.25) + mt * std::min(1., std::pow(4096. / K, 3)) +
-                  per * (0.65 + 0.027 * mt + (mid ? 0.19 : 0.)));
+    if (most == 512)
+      take(wgs, per, 5.36 + 0.062 * M + (1.3 + 0.25 * mid) * per);
+    else if (p.most == 512)
+      take(wgs, per, 3.88 + 0.053 * M + 0.61 * met + 0.035 * shares + (0.594 + 0.08 * mid) * per);
+    else
+      take(wgs, per, (mt > 1 ? 5.37 : 6.05) +
+           mt * (0.73 * met + 0.273 * shares + 0.9 * std::min(1., std::pow(4096. / K, 3))) +
+           per * (0.636 - 0.0097 * mt + 0.4 * mid));
   }
-  const double cu = mt == 1 ? 0.38 : mt == 2 ? 0.41 : mt == 3 ? 0.5 : 0.55;   // us of a step of a CU's own
+  const double cu = mt == 1 ? 0.414 : mt == 2 ? 0.396 : mt == 3 ? 0.472 : 0.476;   // us of a step of a CU's own
   const auto even = [&](long long wgs, long long per, int parts) {
     const int on = (int)((wgs + 255) / 256);   // workgroups on a CU
-    // rows 16 KB apart: still the same channels (8192 x 8192 at 24 / 45 rows 31.6 / 33.9 us; up to 24 rows
-    // tiles, at 32.9, keep it)
-    const double camp = mt == 1 || K % 8192 != 0 ? 0. : mt == 2 ? 0.1665 : 0.06;
-    const double step = std::max(cu * on, wgs * 16.384e-3 / 7.0) + (mid ? 0.19 : 0.) + camp;
-    take(wgs, per, 3.5 + 0.5 * on + per * step + (parts <= 1 ? 0. : mt > 1 ? 1.4 + sums(parts, 0.4) : 2.65 + sums(parts, 0.1)));
+    const double step = std::max(cu * on, wgs * 16.384e-3 / 7.33) + 0.15 * mid;
+    const double sums = parts <= 1 ? 0.
+                        : mt > 1           ? 2.37 + mt * (0.53 + 0.262 * parts)
+                        : gated            ? 4.4
+                                           : 1.34 + 0.046 * parts;
+    take(wgs, per, 2.52 + 0.89 * on + per * step + sums);
   };
   for (long long c = (strips + p.most - 1) / p.most, n = 0; n < 2; ++c, ++n)
     even((strips + c - 1) / c, c * ks, 1);
@@ -460,15 +464,16 @@ static int rows_kind(int M, long long Nv, int K, bool gated) {
   if (M > 64 || Nv > 64LL * kRowsTicks) return 0;
   const double kb = K * 2e-3;   // KB of one row of k
   const bool mid = K % 64 != 0;   // rows start amid a line
-  const double tiles = 6.7 + Nv * kb / 5590 + 0.015 * M + 0.45e-3 * std::min(K, 8192);
+  const double tiles = 5.7 + Nv * kb / 5929 + 0.345e-3 * std::min(K, 8192);
   const double stream = stream_plan(M, Nv, K, gated).us;
   double direct = 1e9;
   if (M <= 32) {
     const int nt = gated || Nv > 4096 ? 2 : 1;
     const long long wgs = (Nv + 16 * nt - 1) / (16 * nt);
-    // a CU's share at 32 (of two strips 26) KB a us, all weights and half of the reads of x at 5.8 MB
-    direct = 4 + (mid ? 1.35 : 1.) * std::max((double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26 : 32),
-                                              (Nv + 0.5 * wgs * M) * kb / 5800);
+    // a CU's share at 30.4 (of two strips 26.4) KB a us, all weights and 0.65 of the reads of x at 5.8 MB
+    const double all = (Nv + 0.65 * wgs * M) * kb / 5844;
+    const double own = (double)((wgs + 255) / 256) * (16 * nt + M) * kb / (nt == 2 ? 26.4 : 30.4);
+    direct = 1.91 + (mid ? 1.56 : 1.) * std::max(own, all);
   }
   if (direct <= stream && direct <= tiles) return 1;
   return stream < tiles ? 2 : 0;

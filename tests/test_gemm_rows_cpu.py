@@ -10,7 +10,7 @@ pytestmark = pytest.mark.skipif(not GEMM_LIB.exists(), reason="native libraries 
 def test_rows_kind_lines():
     from cake_amd.ops import gemm as G
     assert G.rows_kind(5, 2048, 2048, False) == 1        # small weights: direct
-    assert G.rows_kind(16, 4096, 4096, False) == 1
+    assert G.rows_kind(5, 4096, 4096, False) == 1        # 10.3 us, stream 11.5
     assert G.rows_kind(16, 4096, 14336, False) == 2      # large ones: the stream
     assert G.rows_kind(45, 28672, 4096, True) == 2
     assert G.rows_kind(64, 4096, 4096, False) == 0       # tiles
@@ -21,12 +21,22 @@ def test_rows_kind_lines():
 
 @pytest.mark.parametrize("M,Nv,K,kind", [
     # us measured as tiles / direct / stream
-    (33, 6144, 4096, 0),     # 18.3 / - / 20.7
-    (24, 8192, 8192, 0),     # 32.2 / 38.2 / 35.6: equal shares on the same channels
-    (24, 10240, 8192, 2),    # 44.9 / 68.3 / 35.1
-    (45, 4096, 10928, 0),    # 31.3 / - / 36.6: rows that start amid a line
-    (5, 4096, 10928, 2),     # 28.9 / 31.4 / 23.5
-    (64, 10240, 8192, 2)])   # 52.3 / - / 40.9
+    (16, 4096, 4096, 2),     # 12.1 / 12.4 / 11.7
+    (24, 4096, 4096, 0),     # 12.4 / 14.4 / 15.0
+    (16, 6144, 4096, 2),     # 15.7 / 17.9 / 14.3
+    (33, 6144, 4096, 0),     # 16.7 / - / 18.3
+    (45, 6144, 4096, 0),     # 17.3 / - / 19.1
+    (24, 8192, 8192, 2),     # 37.1 / 39.4 / 29.6: parts that start by their strip
+    (64, 8192, 8192, 2),     # 39.3 / - / 32.5
+    (24, 8192, 16384, 2),    # 65.2 / 75.0 / 46.4
+    (24, 10240, 8192, 2),    # 43.3 / 68.2 / 35.2
+    (33, 4096, 14336, 0),    # 27.8 / - / 30.1
+    (45, 4096, 10928, 0),    # 27.4 / - / 37.6: rows that start amid a line
+    (5, 4096, 10928, 2),     # 23.7 / 31.9 / 21.0
+    (5, 3072, 2048, 1),      # 9.6 / 6.7 / 8.4
+    (24, 5120, 5120, 0),     # 17.2 / 27.6 / 18.3
+    (24, 10944, 2048, 0),    # 14.3 / 20.3 / 15.8
+    (64, 10240, 8192, 2)])   # 45.5 / - / 41.2
 def test_rows_kind_takes_the_measured_best(M, Nv, K, kind):
     from cake_amd.ops import gemm as G
     assert G.rows_kind(M, Nv, K, False) == kind
