@@ -121,19 +121,21 @@ __device__ __forceinline__ void amfma_dma_at(cf32x4& acc, const uint4& a, const 
 // PCS: the tiles past the last whole wave in k pieces (GemmArgs::pieces); an instance of its own,
 // since the sums of pieces spill twice the registers in the epilogue of whole tiles too (4096^3 with
 // the residual 113.3 us with them, 109.9 without).
-template <int DT, int EPI, int BM, int BN, int SCHED = 0, bool GRP = false, bool PCS = false>
-__global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
+template <int BM, int BN, int SCHED> struct FourWave {
+  static constexpr int BUF = (BM + BN) * 128;  // 64 KB at most per k-step buffer
+  static constexpr int NBUF = SCHED != 2 ? 2 : 160 * 1024 / BUF > 4 ? 4 : 160 * 1024 / BUF;
+};
+template <int DT, int EPI, int BM, int BN, int SCHED, bool GRP, bool PCS>
+__device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
   static_assert(BM % 32 == 0 && BN % 64 == 0, "whole fragments, gated pairs within a wave");
   constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
-  constexpr int BUF = (BM + BN) * 128;  // 64 KB at most per k-step buffer
-  constexpr int NBUF = SCHED != 2 ? 2 : 160 * 1024 / BUF > 4 ? 4 : 160 * 1024 / BUF;
+  constexpr int BUF = FourWave<BM, BN, SCHED>::BUF, NBUF = FourWave<BM, BN, SCHED>::NBUF;
   static_assert(SCHED != 2 || NBUF > 2, "one barrier a step: three steps in the LDS");
   constexpr int IPW = (BM + BN) / 32;   // DMA wave-instructions per wave per k-step
   constexpr int NA = BM / 32;           // of which A
   static_assert(IPW == FM + FN, "the second half alternates one DMA with one fragment read");
   constexpr int STG_LD = WTN + 4, STG = 16 * STG_LD * 4;
   static_assert(8 * STG <= NBUF * BUF - 16, "epilogue staging (2 slices per wave) fits the operand buffers");
-  __shared__ __attribute__((aligned(16))) uint8_t smem[NBUF * BUF];
 
   const int tid = threadIdx.x, lane = tid & 63;
 #ifdef CAKE_GEMM_STAMPS
@@ -667,6 +669,13 @@ __global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
       for (int i = 0; i < 8; ++i) g_gemm_stamps[((size_t)blockIdx.x * 4 + wave) * 8 + i] = st_[i];
   }
 #endif
+}
+
+template <int DT, int EPI, int BM, int BN, int SCHED = 0, bool PCS = false>
+__global__ __launch_bounds__(256) void gemm_4w_kernel(GemmArgs g) {
+  using F = FourWave<BM, BN, SCHED>;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[F::NBUF * F::BUF];
+  gemm_4w_tile<DT, EPI, BM, BN, SCHED, false, PCS>(g, smem);
 }
 
 }  // namespace cake

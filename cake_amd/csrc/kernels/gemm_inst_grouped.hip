@@ -7,9 +7,28 @@ namespace cake {
 
 constexpr long long kWide = 1 << 22;  // elements: 256 rows of this stride are 2 GB
 
-// Tiles by rows, of 256 columns on four waves (gemm_4w.h); cfg 4: 64 x 64
+// Tiles by rows, of 256 columns on four waves (gemm_4w.h); cfg 4: 64 x 64; cfg 6: as the tile list says
+constexpr int kByList = 6;
 constexpr int grouped_rows(int cfg) {
-  return cfg == 4 ? 64 : cfg == 0 ? 128 : cfg == 1 ? 160 : cfg == 2 ? 192 : cfg == 5 ? 256 : 0;
+  return cfg == 4 ? 64 : cfg == 0 ? 128 : cfg == 1 ? 160 : cfg == 2 ? 192 : cfg == 5 || cfg == kByList ? 256 : 0;
+}
+
+// One kernel for the four heights, so that the one that fits the groups can be chosen on the device, where
+// their sizes are known (mixer_experts.hip).  All of them fill a CU's LDS alone: a branch over whole
+// bodies costs none of them a workgroup (two products of 64 experts 4096 x 3648, 192 rows each: 932 us in
+// a kernel of its own, 938 so; over all heights and seven sizes 0.8 % more).
+template <int DT, int EPI>
+__global__ __launch_bounds__(256) void gemm_heights_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[FourWave<160, 256, 2>::NBUF * FourWave<160, 256, 2>::BUF];
+  const int rows = g.pieces > 0 ? g.pieces : __builtin_amdgcn_readfirstlane(g.groups[g.tiles_m].y);
+#define X(BM, SCHED)                                                                         \
+  if (rows == BM) {                                                                          \
+    static_assert(FourWave<BM, 256, SCHED>::NBUF * FourWave<BM, 256, SCHED>::BUF <= (int)sizeof(smem), "LDS"); \
+    gemm_4w_tile<DT, EPI, BM, 256, SCHED, true, false>(g, smem);                             \
+    return;                                                                                  \
+  }
+  X(128, 2) X(160, 2) X(192, 1) X(256, 1)
+#undef X
 }
 
 // Rows too far apart for the four waves' 32-bit offsets take the 64-row tile, in passes.
@@ -24,14 +43,8 @@ static int launch_grouped(int cfg, int tiles, hipStream_t st, GemmArgs& g) {
     hipLaunchKernelGGL((gemm_kernel<DT, 64, 64, 2, 2, 2, EPI, 6, true>), grid, dim3(256), 0, st, g);
     return (int)hipGetLastError();
   }
-  switch (bm) {
-#define X(BM, SCHED)                                                                          \
-  case BM:                                                                                    \
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, BM, 256, SCHED, true>), grid, dim3(256), 0, st, g); \
-    break;
-    X(128, 2) X(160, 2) X(192, 1) X(256, 1)
-#undef X
-  }
+  g.pieces = cfg == kByList ? 0 : bm;   // rows of a tile
+  hipLaunchKernelGGL((gemm_heights_kernel<DT, EPI>), grid, dim3(256), 0, st, g);
   return (int)hipGetLastError();
 }
 
@@ -40,7 +53,8 @@ static int launch_grouped(int cfg, int tiles, hipStream_t st, GemmArgs& g) {
 using namespace cake;
 
 // c[row0 + r] = act(a[row0 + r] W[group]^T) over the tiles [group, row0, rows, 0] (0 < rows <= the
-// configuration's BM), at most max_tiles of them; entry max_tiles of the list is [count, 0, 0, 0].
+// configuration's BM), at most max_tiles of them; entry max_tiles of the list is [count, BM, 0, 0] (BM, 128,
+// 160, 192 or 256, read in configuration 6 only).
 // epi 0: no activation, 7 .. 10 as cake_gemm_scaled.  K % 8 == 0.
 CAKE_API int cake_gemm_grouped(int dt, int epi, int cfg, const void* a, long long lda, const void* b,
                                long long ldb, long long b_group, void* c, long long ldc,

@@ -1061,7 +1061,7 @@ constexpr bool gated_ok(int wave_cols) {
 // PCS: some tiles run in pieces (GemmArgs::pieces)
 #define CAKE_LAUNCH_4W(ID, BM, BN, WM, WN, SCHED)                                                      \
   if (cfg == ID) {                                                                             \
-    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, BM, BN, SCHED, false, PCS>), grid, dim3(256),  \
+    hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, BM, BN, SCHED, PCS>), grid, dim3(256),  \
                        0, st, g);                                                              \
     return (int)hipGetLastError();                                                             \
   }

@@ -2,6 +2,7 @@
 grouped GEMM); shapes, dtypes and strides are validated on the host before every launch."""
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 
 import torch
@@ -38,25 +39,29 @@ class Plan:
     row: torch.Tensor     # [M] token of every sorted row
     scale: torch.Tensor   # [M] its score
     where: torch.Tensor   # [N, top] sorted row of every entry
-    tiles: torch.Tensor   # [n + 1, 4], the last entry their number
+    tiles: torch.Tensor   # [n + 1, 4], the last entry their number and height
     cfg: int              # grouped GEMM configuration (16-bit types)
 
 
-def plan(ids, score, E: int, dtype, weight: int = 0) -> Plan:
-    """Rows sorted by expert, and their tiles; weight: elements of an expert's matrix."""
+def plan(ids, score, E: int, dtype, weight: int = 0, up: int = 0) -> Plan:
+    """Rows sorted by expert, and their tiles; weight: elements of an expert's matrix, up: columns of
+    its up product (0: a square matrix)."""
     N, top = ids.shape
     _routing(E, top)
     M, dev = N * top, ids.device
     cfg = G.grouped_cfg(M, E, torch.cuda.is_current_stream_capturing(), weight)
-    bm = BM32 if dtype == torch.float32 else G.GROUPED_CFGS[cfg]
+    bm = BM32 if dtype == torch.float32 else G.GROUPED_CFGS[cfg]   # the least, of a height yet to choose
     n = M // bm + min(E, M)
+    up = up or math.isqrt(weight or 1 << 22)
+    wide = max(1, (weight or 1 << 22) // up)
     i32 = torch.empty(2 * M + 4 * (n + 1) + 4, device=dev, dtype=torch.int32)
     row, where = i32[:M], i32[M:2 * M].view(N, top)
     at = 2 * M + (-2 * M) % 4   # tiles are read whole, 16 bytes each
     tiles = i32[at:at + 4 * (n + 1)].view(n + 1, 4)
     scale = torch.empty(M, device=dev, dtype=torch.float32)
     check(_lib().cake_expert_plan(_vec(ids, "ids", torch.int32, M),
-                                  _vec(score, "score", torch.float32, M), N, top, E, bm,
+                                  _vec(score, "score", torch.float32, M), N, top, E,
+                                  0 if dtype != torch.float32 and cfg == G.BY_LIST else bm, up, wide,
                                   row.data_ptr(), scale.data_ptr(), where.data_ptr(),
                                   tiles.data_ptr(), n, _stream()), "expert_plan")
     return Plan(row, scale, where, tiles, cfg)

@@ -13,8 +13,6 @@ estimate, which a measured entry of the very size (gemm_tuned.json) or a pinned 
 from __future__ import annotations
 
 import ctypes as C
-import functools
-import math
 import threading
 
 import torch
@@ -452,9 +450,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
     return resid if f32_out else out
 
 
-# tile configuration of a grouped product -> its rows (ROWS: the stream form)
-ROWS = 32
-GROUPED_CFGS = {0: 128, 1: 160, 2: 192, 4: 64, 5: 256, ROWS: 16}
+# tile configuration of a grouped product -> its rows (ROWS: the stream form; BY_LIST: 128, 160, 192 or 256,
+# as the last entry of the tile list says: chosen on the device from the groups' sizes)
+ROWS, BY_LIST = 32, 6
+GROUPED_CFGS = {0: 128, 1: 160, 2: 192, 4: 64, 5: 256, BY_LIST: 128, ROWS: 16}
 
 
 def grouped_cfg(rows: int, groups: int, capturing: bool = False, weight: int = 0) -> int:
@@ -472,42 +471,14 @@ def grouped_cfg(rows: int, groups: int, capturing: bool = False, weight: int = 0
     big = groups * weight >= 200_000_000
     if mean < (12 if big else 24):
         return 4
-    return 0 if mean < 64 else _tile_height(rows, groups)
-
-
-# configuration -> (rows, cost of an expert's weights for a pair of tiles, of a tile), us of both
-# products of 64 experts 4096 x 3648
-_HEIGHTS = {0: (128, 461, 279), 1: (160, 384, 390), 2: (192, 303, 522), 5: (256, 209, 715)}
-
-
-@functools.lru_cache(maxsize=1024)
-def _tile_height(rows: int, groups: int) -> int:
-    """Configuration whose tiles cost least over groups of rows / groups rows on the average.  Tokens
-    that choose independently spread by the root of that; trained routers more, and a group that
-    overflows its tile costs more than a taller tile does: four times as much is assumed (over 68
-    products of even and 68 of skewed groups 5 % and 1 % faster than 128 and 256 rows alone, at most 12 %
-    slower; without the factor 3 %, 0 and 28 %).  Even groups, the same experts, us at 128 / 160 / 192 /
-    256 rows a tile, by rows an expert: 90 739 / 749 / 783 / 840, 120 870 / 774 / 812 / 869, 150 1078 / 886 /
-    826 / 912, 170 977 / 1167 / 928 / 913, 210 1310 / 1104 / 1457 / 1023, 260 1479 / 1143 / 1324 / 1379,
-    300 1712 / 1324 / 1347 / 1711, 400 2051 / 1906 / 1965 / 1629, 500 2395 / 2359 / 2201 / 2025."""
-    mean = rows / groups
-    sd = 4 * math.sqrt(2 * mean)
-
-    def cost(bm: int, pair: float, tile: float) -> float:
-        out, n, more = 0.0, 1, 1.0   # more: share of the groups with an n-th tile
-        while more > 1e-3:
-            out += more * (tile + (pair if n % 2 else 0))
-            more = 0.5 * math.erfc((n * bm - mean) / sd)
-            n += 1
-        return out
-    return min(_HEIGHTS, key=lambda c: cost(*_HEIGHTS[c]))
+    return 0 if mean < 64 else BY_LIST
 
 
 def grouped(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, cfg: int, out: torch.Tensor,
             epi: str = "store") -> torch.Tensor:
     """out[r] = act(x[r] @ w[g].T) for the rows of every tile of `tiles` (int32 [n + 1, 4] on the
-    device: weight group, first row, rows, 0; the last entry is the number of tiles in use), each
-    within x's rows and at most the configuration's row count.  x [R, K], w [groups, N, K] and
+    device: weight group, first row, rows, 0; the last entry is the number of tiles in use and, for
+    BY_LIST, their height), each within x's rows and at most the configuration's row count.  x [R, K], w [groups, N, K] and
     out [R, N] 16-bit; epi: store or one of the activations."""
     if epi not in ("store", "silu", "quick_gelu", "gelu", "relu2") or cfg not in GROUPED_CFGS:
         raise ValueError(f"grouped: epilogue {epi}, configuration {cfg}")
