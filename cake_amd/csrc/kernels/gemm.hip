@@ -341,6 +341,11 @@ CAKE_API int cake_gemm_scaled(int dt, int epi, int cfg, int splits, const void* 
                               void* tick, const void* zeros, int M, int N, int K, float alpha,
                               hipStream_t st) {
   if (alpha != 1.f && epi != kEpiResid32 && epi != kEpiStore32) return (int)hipErrorInvalidValue;
+  // tiles 28 on have no 16-bit residual and no GEGLU, 64 kernels that no plan takes: whole 128 x 256 tiles
+  if (cfg > k4WCfg128 + k4WSched && four_wave_cfg(cfg) && (epi == kEpiAdd16 || epi == kEpiGeglu)) {
+    cfg = k4WCfg128 + k4WSched;
+    splits = 1;
+  }
   int bm, bn;
   cfg_dims(cfg, bm, bn);
   if (bm == 0 || M <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || splits < 1)

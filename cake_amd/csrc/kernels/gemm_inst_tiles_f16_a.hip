@@ -1,4 +1,4 @@
-// Instantiates the four-wave tiles of CAKE_GEMM_4W_TILES (gemm_4w.h) for f16, epilogues Store, Resid32, Add16;
+// Instantiates the four-wave tiles of CAKE_GEMM_4W_TILES (gemm_4w.h) for f16, epilogues Store, Resid32;
 // split from gemm.hip so the heavy instantiations compile in parallel.
 #include "gemm_kernel.h"
 
@@ -7,6 +7,4 @@ template int launch_tiles<kF16, kEpiStore, false>(int, dim3, hipStream_t, const 
 template int launch_tiles<kF16, kEpiStore, true>(int, dim3, hipStream_t, const GemmArgs&);
 template int launch_tiles<kF16, kEpiResid32, false>(int, dim3, hipStream_t, const GemmArgs&);
 template int launch_tiles<kF16, kEpiResid32, true>(int, dim3, hipStream_t, const GemmArgs&);
-template int launch_tiles<kF16, kEpiAdd16, false>(int, dim3, hipStream_t, const GemmArgs&);
-template int launch_tiles<kF16, kEpiAdd16, true>(int, dim3, hipStream_t, const GemmArgs&);
 }  // namespace cake

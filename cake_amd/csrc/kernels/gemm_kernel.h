@@ -1075,9 +1075,8 @@ int launch_tiles(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
   extern template int launch_tiles<DT, E, false>(int, dim3, hipStream_t, const GemmArgs&);     \
   extern template int launch_tiles<DT, E, true>(int, dim3, hipStream_t, const GemmArgs&);
 #define CAKE_TILES_EXTERN_ALL(DT) CAKE_TILES_EXTERN(DT, kEpiStore) CAKE_TILES_EXTERN(DT, kEpiResid32) \
-  CAKE_TILES_EXTERN(DT, kEpiAdd16) CAKE_TILES_EXTERN(DT, kEpiSwiglu) CAKE_TILES_EXTERN(DT, kEpiGeglu) \
-  CAKE_TILES_EXTERN(DT, kEpiStore32) CAKE_TILES_EXTERN(DT, kEpiSilu) CAKE_TILES_EXTERN(DT, kEpiQuick) \
-  CAKE_TILES_EXTERN(DT, kEpiGelu) CAKE_TILES_EXTERN(DT, kEpiRelu2)
+  CAKE_TILES_EXTERN(DT, kEpiSwiglu) CAKE_TILES_EXTERN(DT, kEpiStore32) CAKE_TILES_EXTERN(DT, kEpiSilu) \
+  CAKE_TILES_EXTERN(DT, kEpiQuick) CAKE_TILES_EXTERN(DT, kEpiGelu) CAKE_TILES_EXTERN(DT, kEpiRelu2)
 CAKE_TILES_EXTERN_ALL(kBF16)
 CAKE_TILES_EXTERN_ALL(kF16)
 #undef CAKE_TILES_EXTERN_ALL
@@ -1093,7 +1092,7 @@ int launch_4w(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
     CAKE_LAUNCH_4W(k4WCfg + k4WSched, 256, 256, 2, 2, 1)
     CAKE_LAUNCH_4W(k4WCfg192 + k4WSched, 256, 192, 2, 2, 1)
     CAKE_LAUNCH_4W(k4WCfg128 + k4WSched, 128, 256, 2, 2, 2)
-    return launch_tiles<DT, EPI, PCS>(cfg, grid, st, g);
+    if constexpr (EPI != kEpiAdd16 && EPI != kEpiGeglu) return launch_tiles<DT, EPI, PCS>(cfg, grid, st, g);
   }
   return (int)hipErrorInvalidValue;
 }

@@ -31,3 +31,18 @@ def test_tile_edges(cuda, cfg, rows, cols, K, splits, epi):
     tol = K * 2.0 ** -21 + (2.0 ** -16 if epi == "resid32" else 2.0 ** -8)
     scale = y.pow(2).mean().sqrt() + y.abs()
     assert bool(((outs[0].float() - y).abs() <= tol * scale).all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("cfg", range(28, 36))
+@pytest.mark.parametrize("epi", ["add16", "geglu"])
+def test_image_epilogues_run_on_another_tile(cuda, dt, cfg, epi):
+    """Tiles without these epilogues: the call's result is the 128 x 256 tile's, pieces or none."""
+    from cake_amd.ops import gemm as G
+    M, N, K = 300, 288, 1088
+    g = torch.Generator(device="cuda").manual_seed(cfg)
+    x = torch.randn(M, K, device="cuda", generator=g).to(dt)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(dt)
+    kw = {"resid": torch.randn(M, N, device="cuda", generator=g).to(dt)} if epi == "add16" else {}
+    want = G.linear(x, w, epi=epi, cfg=27, splits=1, **kw)
+    assert all(torch.equal(G.linear(x, w, epi=epi, cfg=cfg, splits=s, **kw), want) for s in (1, 4))
