@@ -247,7 +247,7 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
   const uint32_t m0_a = __builtin_amdgcn_readfirstlane(lds_off(smem) + (uint32_t)wave * (apart ? 1024 : NA * 1024));
   const uint32_t m0_b = __builtin_amdgcn_readfirstlane(lds_off(smem) + BM * 128u + (uint32_t)wave * (apart ? 1024 : NB * 1024));
   const uint32_t piece_b = apart ? 4096 : 1024;   // LDS bytes from an instruction's rows to the next one's
-  // M0 (= buffer base + 1 KiB per piece, the piece offset an immediate) / voffset / soffset
+  // M0 = buffer base + piece_b per piece (an immediate where it is always 1 KiB) / voffset / soffset
   // of DMA I (A pieces for I < NA) into buffer buf
   auto dma_mb = [&](int buf, int i) __attribute__((always_inline)) {
     return (i < NA ? m0_a : m0_b) + (uint32_t)(buf * BUF);
@@ -418,7 +418,7 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
     //     k 0..31 of t+1
     // The reads end LAT MFMAs before their half does (their latency); the DMAs of a step are spread
     // from barrier to barrier, ND2 of them before the next step begins.
-    constexpr int P = 2, LAT = NM >= 48 ? 9 : 7;
+    constexpr int P = 2, LAT = 7;
     constexpr int R1 = NM - LAT, W2 = NM - P - 1, R2 = W2 - LAT;   // MFMAs that reads, DMAs follow
     constexpr int ND2 = IPW / 2, ND1 = IPW - ND2;
     static_assert(R2 >= NR / 2 && W2 >= ND2, "op density");

@@ -78,7 +78,7 @@ struct GemmArgs {
   int dp_tiles;
   // grouped products (gemm_inst_grouped.hip): row tile tm is [weight group, first row, rows, -]
   // of this list instead of rows tm BM .., its weights b + group b_group; entry tiles_m holds
-  // the number of tiles
+  // the number of tiles and, where `pieces` (here the tiles' rows) is 0, their rows
   const int4* groups;
   long long b_group;
 };

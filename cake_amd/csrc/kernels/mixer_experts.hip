@@ -88,13 +88,13 @@ __device__ inline int tile_height(const int (&tiles)[4], int E, int M, int F, in
   return kHeights[best];
 }
 
-// Entries (token, k) sorted by expert: row[p] = token, scale[p] = score, where[entry] = p; the
-// tile list [expert, first sorted row, rows, 0] of BM-row tiles (0: tile_height of an expert's F x W
-// up matrix), entry max_tiles [their number, BM, 0, 0].
+// Entries (token, k) sorted by expert: scale[p] = score of sorted row p, where[entry] = p; the tile
+// list [expert, first sorted row, rows, 0] of BM-row tiles (0: tile_height of an expert's F x W up
+// matrix), entry max_tiles [their number, BM, 0, 0].
 __global__ __launch_bounds__(1024) void expert_plan_kernel(const int* ids, const float* score,
                                                            int N, int top, int E, int BM, int F, int W,
-                                                           int* row, float* scale, int* where,
-                                                           int4* tiles, int max_tiles) {
+                                                           float* scale, int* where, int4* tiles,
+                                                           int max_tiles) {
   __shared__ int cnt[kMaxExperts], scan[2][kMaxExperts], fit[4];
   constexpr int U = 16;  // entries in flight per thread
   const int tid = threadIdx.x, M = N * top;
@@ -153,7 +153,6 @@ __global__ __launch_bounds__(1024) void expert_plan_kernel(const int* ids, const
     for (int u = 0; u < U; ++u)
       if (e[u] >= 0) {
         const int i = i0 + 1024 * u, p = atomicAdd(&cnt[e[u]], 1);
-        row[p] = i / top;
         scale[p] = s[u];
         where[i] = p;
       }
@@ -394,13 +393,12 @@ CAKE_API int cake_expert_route(const float* logits, long long ldl, int N, int E,
 // has one entry more (their number)
 // BM 0: the height that suits the groups, of experts of F x W (up) and W x F
 CAKE_API int cake_expert_plan(const int* ids, const float* score, int N, int top, int E, int BM, int F,
-                              int W, int* row, float* scale, int* where, void* tiles, int max_tiles,
-                              hipStream_t st) {
+                              int W, float* scale, int* where, void* tiles, int max_tiles, hipStream_t st) {
   if (!routing_ok(E, top) || N <= 0 || BM < 0 || (BM == 0 && (F <= 0 || W <= 0)) ||
       max_tiles < (long long)N * top / (BM > 0 ? BM : kHeights[0]) + (E < (long long)N * top ? E : N * top))
     return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(expert_plan_kernel, dim3(1), dim3(1024), 0, st, ids, score, N, top, E, BM, F, W, row,
-                     scale, where, (int4*)tiles, max_tiles);
+  hipLaunchKernelGGL(expert_plan_kernel, dim3(1), dim3(1024), 0, st, ids, score, N, top, E, BM, F, W, scale,
+                     where, (int4*)tiles, max_tiles);
   return (int)hipGetLastError();
 }
 

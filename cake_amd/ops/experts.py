@@ -36,11 +36,17 @@ def route(logits, top: int):
 @dataclass
 class Plan:
     """(token, choice) entries sorted by expert, and the row tiles of the grouped products."""
-    row: torch.Tensor     # [M] token of every sorted row
-    scale: torch.Tensor   # [M] its score
+    scale: torch.Tensor   # [M] score of every sorted row
     where: torch.Tensor   # [N, top] sorted row of every entry
     tiles: torch.Tensor   # [n + 1, 4], the last entry their number and height
     cfg: int              # grouped GEMM configuration (16-bit types)
+
+    @property
+    def row(self) -> torch.Tensor:
+        """[M] token of every sorted row."""
+        N, top = self.where.shape
+        token = torch.arange(N, dtype=torch.int32, device=self.where.device).repeat_interleave(top)
+        return torch.empty_like(token).scatter_(0, self.where.flatten().long(), token)
 
 
 def plan(ids, score, E: int, dtype, weight: int = 0, up: int = 0) -> Plan:
@@ -54,17 +60,17 @@ def plan(ids, score, E: int, dtype, weight: int = 0, up: int = 0) -> Plan:
     n = M // bm + min(E, M)
     up = up or math.isqrt(weight or 1 << 22)
     wide = max(1, (weight or 1 << 22) // up)
-    i32 = torch.empty(2 * M + 4 * (n + 1) + 4, device=dev, dtype=torch.int32)
-    row, where = i32[:M], i32[M:2 * M].view(N, top)
-    at = 2 * M + (-2 * M) % 4   # tiles are read whole, 16 bytes each
+    i32 = torch.empty(M + 4 * (n + 1) + 4, device=dev, dtype=torch.int32)
+    where = i32[:M].view(N, top)
+    at = M + -M % 4   # tiles are read whole, 16 bytes each
     tiles = i32[at:at + 4 * (n + 1)].view(n + 1, 4)
     scale = torch.empty(M, device=dev, dtype=torch.float32)
     check(_lib().cake_expert_plan(_vec(ids, "ids", torch.int32, M),
                                   _vec(score, "score", torch.float32, M), N, top, E,
                                   0 if dtype != torch.float32 and cfg == G.BY_LIST else bm, up, wide,
-                                  row.data_ptr(), scale.data_ptr(), where.data_ptr(),
-                                  tiles.data_ptr(), n, _stream()), "expert_plan")
-    return Plan(row, scale, where, tiles, cfg)
+                                  scale.data_ptr(), where.data_ptr(), tiles.data_ptr(), n, _stream()),
+          "expert_plan")
+    return Plan(scale, where, tiles, cfg)
 
 
 def product(x, w, p: Plan, out, act: str | None = None):
@@ -72,7 +78,7 @@ def product(x, w, p: Plan, out, act: str | None = None):
     E, N, K = w.shape
     if x.dtype != torch.float32:
         return G.grouped(x, w, p.tiles, p.cfg, out, epi=act or "store")
-    M = p.row.numel()
+    M = p.where.numel()
     xp, ldx = _mat(x, "x", torch.float32, M, K)
     op, ldo = _mat(out, "out", torch.float32, M, N)
     check(_lib().cake_expert_gemm32(xp, ldx, _vec(w, "w", torch.float32), K, N * K,

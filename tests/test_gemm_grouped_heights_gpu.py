@@ -29,3 +29,32 @@ def test_tile_heights(cuda, cfg, N, K, ld):
     want = torch.cat(want)
     assert bool((out[:, N:] == 7.0).all())
     assert bool(((out[:, :N].float() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -20).all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("cfg", [0, 1, 2, 5, 6])
+@pytest.mark.parametrize("epi", ["silu", "relu2"])
+def test_activations_of_every_height(cuda, dt, cfg, epi):
+    """As routed experts run them, 16-bit types and activations; configuration 6 by the list's height.  One
+    rounding (2^-8, 2^-11) of f32 sums, the activation's own 2^-10."""
+    from cake_amd.ops import gemm as G
+    N, K = 300, 200
+    for bm in ((128, 160, 192, 256) if cfg == 6 else (G.GROUPED_CFGS[cfg],)):
+        counts = [bm + 1, 3, 0, bm, bm - 1]
+        R = sum(counts)
+        g = torch.Generator(device="cuda").manual_seed(bm)
+        x = torch.randn(R, K, device="cuda", generator=g).to(dt)
+        w = (torch.randn(len(counts), N, K, device="cuda", generator=g) * K ** -0.5).to(dt)
+        tiles, r0, y = [], 0, []
+        for e, c in enumerate(counts):
+            tiles += [[e, r0 + t, min(bm, c - t), 0] for t in range(0, c, bm)]
+            y.append(x[r0:r0 + c].double() @ w[e].double().t())
+            r0 += c
+        t = torch.tensor(tiles + [[0, 0, 0, 0], [len(tiles), bm, 0, 0]], dtype=torch.int32, device="cuda")
+        out = torch.full((R, N + 8), 7.0, dtype=dt, device="cuda")
+        G.grouped(x, w, t, cfg, out[:, :N], epi=epi)
+        y = torch.cat(y)
+        want = torch.nn.functional.silu(y) if epi == "silu" else torch.relu(y).square()
+        size = 2.0 ** (-8 if dt == torch.bfloat16 else -11) + 2.0 ** -10
+        assert bool((out[:, N:] == 7.0).all())
+        assert bool(((out[:, :N].double() - want).abs() <= size * want.abs() + K * 2.0 ** -22 * (1 + y.abs()) * 2).all())

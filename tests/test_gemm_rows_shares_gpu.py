@@ -11,8 +11,9 @@ pytestmark = pytest.mark.gpu
                                  (2048, 8192), (4096, 3648), (70000, 192)])
 @pytest.mark.parametrize("epi", ["store32", "swiglu"])
 def test_shares(cuda, monkeypatch, M, N, K, epi):
-    """f32 sums in two orders, within K 2^-22 of the row's scale before a rounding to bf16 (gate, up
-    and their product in the gated form); a second launch finds clean counters, the same bits."""
+    """f32 sums of 16-bit products in two orders (either within K 2^-22 of the sums' scale of the exact
+    one: K 2^-21 apart), then 2^-16 for the f32 result (alpha and the oracle's own rounding) or one
+    rounding to bf16, 2^-8; a second launch finds clean counters, the same bits."""
     from cake_amd.ops import gemm as G
     monkeypatch.setattr(G, "rows_kind", lambda *a: 2)
     if epi == "swiglu":
