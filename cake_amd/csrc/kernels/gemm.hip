@@ -219,9 +219,9 @@ static constexpr TileCost kTileCosts[] = {
     {28, 128, 128, 1, 0.564f, 0.443f, 0.0724f, 0.0141f, 0.119f, {3.183f, 3.551f, 3.063f, 6.329f, -1.f, -1.f, -1.f}, 1.816f, 2.725f},
     {29, 128, 192, 1, 0.158f, 0.513f, 0.11f, 0.237f, 0.18f, {6.195f, 6.798f, 5.003f, 8.104f, -1.f, -1.f, -1.f}, 6.417f, 2.032f},
     {30, 96, 256, 1, 0.562f, 0.635f, 0.043f, 0.142f, 0.149f, {3.821f, 5.301f, 3.733f, 8.382f, -1.f, -1.f, -1.f}, 3.125f, 3.253f},
-    {31, 160, 256, 1, 0.797f, 0.711f, 0.0445f, 0.0764f, 0.127f, {7.909f, 11.57f, 7.589f, 13.52f, -1.f, -1.f, -1.f}, 3.749f, 3.796f},
+    {31, 160, 256, 1, 0.797f, 0.711f, 0.0445f, 0.0764f, 0.127f, {7.909f, 11.57f, 7.589f, 13.52f, -1.f, -1.f, -1.f}, 9.75f, 3.796f},
     {32, 192, 192, 1, 1.316f, 0.62f, 0.0623f, 0.0716f, 0.127f, {7.468f, 10.46f, 6.705f, 11.87f, -1.f, -1.f, -1.f}, 4.369f, 3.521f},
-    {33, 224, 192, 1, 0.846f, 0.777f, 0.0146f, -0.0934f, 0.144f, {10.04f, 12.63f, 8.565f, 13.22f, -1.f, -1.f, -1.f}, 4.312f, 3.47f},
+    {33, 224, 192, 1, 0.846f, 0.777f, 0.0146f, -0.0934f, 0.144f, {10.04f, 12.63f, 8.565f, 13.22f, -1.f, -1.f, -1.f}, 0.812f, 3.47f},
     {34, 192, 256, 1, 1.768f, 0.979f, 0.0472f, 0.0879f, 0.126f, {6.113f, 10.06f, 6.451f, 13.14f, -1.f, -1.f, -1.f}, 2.423f, 4.585f},
     {35, 224, 256, 1, 1.053f, 1.076f, 0.045f, 0.148f, 0.113f, {7.659f, 11.94f, 7.822f, 13.64f, -1.f, -1.f, -1.f}, 6.25f, 4.798f},
     // products of image models: the classes from kImageClass on
