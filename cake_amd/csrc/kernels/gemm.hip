@@ -291,8 +291,7 @@ static double tile_cost(const TileCost& c, int splits, long long M, long long Nv
 // of graphs.  On entry *cfg, *splits: a measured plan of this very size, or cfg -1; it stands unless it
 // is modelled and 10 % behind the best.  big: an operand of 2 GB or more (31-bit offsets of the
 // four-wave tiles).
-CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits) {
-  if (M < 1 || Nv < 1 || K < 1 || !cfg || !splits) return (int)hipErrorInvalidValue;
+static double tile_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits) {
   const bool gated = epi == kEpiSwiglu || epi == kEpiGeglu;
   const bool image = cost_class(epi, K) >= kImageClass;
   const int ks = (K + kGBK - 1) / kGBK;
@@ -319,9 +318,14 @@ CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* c
       }
     }
   }
-  if (*cfg >= 0 && (given < 0 || given <= 1.1 * best)) return 0;
+  if (*cfg >= 0 && (given < 0 || given <= 1.1 * best)) return given < 0 ? best : given;
   *cfg = bc;
   *splits = bs;
+  return best;
+}
+CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* cfg, int* splits) {
+  if (M < 1 || Nv < 1 || K < 1 || !cfg || !splits) return (int)hipErrorInvalidValue;
+  tile_plan(M, Nv, K, epi, big, cfg, splits);
   return 0;
 }
 
@@ -532,6 +536,126 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
   }
   return dt == kBF16 ? Rows<kBF16>::run(epi, form, mt, dim3(wgs), st, g)
          : dt == kF16 ? Rows<kF16>::run(epi, form, mt, dim3(wgs), st, g) : (int)hipErrorInvalidValue;
+}
+
+// ---- products that leave their sums in slabs ------------------------------
+// Which form such a product takes, and whether the launch that follows it gains from summing them
+// (gemm_slabs.hip).  The estimates (us) are fits to timings of product and norm or rotation on weights that no
+// cache holds, 2 .. 64 rows of 33 shapes, 2 .. 470 MB, every form: what they pick is 0.35 % off the best on the
+// average, at most 11 %.  The two launches take 0.9 of the three or two they replace at 2 .. 16 rows (4096 x
+// 14336 and norm at 5 rows 26.6 -> 25.0 us), 0.87 at 24 .. 64 (at 45 rows 32.6 -> 30.2, 4096 x 4096 16.0 ->
+// 13.9, 6144 x 4096 and rotation 20.3 -> 18.3, 10240 x 8192 44.4 -> 37.7, 4096 x 23552 48.5 -> 42.6).
+struct SlabStream { double c0, cu, step, rate, slab, mid; };   // by 16-row tiles of x
+static constexpr SlabStream kSlabStream[4] = {{3.02, 0.544, 0.518, 6.40, 1.05, 0.10},
+                                              {0.52, 3.394, 0.506, 6.71, 1.15, 0.15},
+                                              {1.77, 1.271, 0.587, 6.72, 1.14, 0.29},
+                                              {1.69, 2.506, 0.567, 6.90, 0.82, 0.24}};
+struct SlabTile { int cfg, least; double c0, step, mem, slab, wgs, mid; };   // least: rows
+static constexpr SlabTile kSlabTiles[] = {{7, 49, 5.20, 0.556, 0.172, 0.688, 1.02, 0.06},
+                                          {12, 1, 3.52, 1.167, 0.177, 0.380, 2.27, 0.08},
+                                          {13, 1, 3.79, 0.674, 0.178, 0.464, 1.01, 0.08},
+                                          {18, 1, 4.08, 0.551, 0.185, 0.462, 3.36, 0.17}};
+static constexpr double kSlabGain = 2.2;
+// 1 and the form in *kind, *cfg, *parts (as cake_gemm_slabs takes them); 0: the product with the epilogue
+// `epi`, and what follows it as a launch of its own
+CAKE_API int cake_gemm_slab_plan(int M, long long N, int K, int epi, int big, int* kind, int* cfg, int* parts) {
+  if (M < 1 || N < 1 || N > 64LL * kRowsTicks || K < 1 || !kind || !cfg || !parts) return 0;
+  const int k64 = (K + kGBK - 1) / kGBK;
+  const double mid = K % 64 != 0 ? 1 : 0;   // rows start amid a line
+  double best = 1e30;
+  const auto take = [&](double us, int f, int c, int p) {
+    if (us < best) { best = us; *kind = f; *cfg = c; *parts = p; }
+  };
+  if (M > 64) {
+    // of more rows the sum of a plan's splits (eight-wave tiles) goes into what follows, which saves the launch
+    // between them; other plans give way where that puts them behind: at 200 rows 4096 x 4096 28 -> 23 us,
+    // 4096 x 14336 the same plan, 8192 x 8192 at 300 rows stays on four-wave pieces (slabs 2 % slower)
+    int c = -1, s = 1;
+    const double plain = tile_plan(M, N, K, epi, big, &c, &s);
+    for (const TileCost& t : kTileCosts) {
+      if (four_wave_cfg(t.cfg) || t.bm > 2.2 * M) continue;
+      for (int sp : {2, 4, 8, 16}) {
+        if (k64 / sp < 4) break;
+        const double us = tile_cost(t, sp, M, N, K, epi);
+        if (us >= 0) take(us - kSlabGain, 0, t.cfg, sp);
+      }
+    }
+    return best < plain;
+  }
+  const int mt = (M + 15) / 16, bn = mt > 1 ? 128 : 64, kst = mt > 1 ? 64 : 128, most = mt > 1 ? 256 : 512;
+  const int ks = (K + kst - 1) / kst;
+  const long long strips = (N + bn - 1) / bn;
+  const SlabStream& c = kSlabStream[mt - 1];
+  for (int p : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16}) {
+    const int per = (ks + p - 1) / p;
+    if (p > 1 && (per * (p - 1) >= ks || ks / p < kRowsMinK / kst || strips * p > most)) continue;
+    const double wgs = (double)strips * p, on = std::ceil(wgs / 256);
+    take(c.c0 + c.cu * on + per * (std::max(c.step * on, wgs * 16.384e-3 / c.rate) + c.mid * mid) +
+             c.slab * p * M * N * 4e-6, 2, 0, p);
+  }
+  for (const SlabTile& t : kSlabTiles) {
+    int bm, bn2;
+    cfg_dims(t.cfg, bm, bn2);
+    for (int p : {2, 4, 8, 16}) {
+      if (M < t.least || k64 / p < 4) break;
+      const int kps = (k64 + p - 1) / p, sp = (k64 + kps - 1) / kps;
+      const double n = (double)((M + bm - 1) / bm) * ((N + bn2 - 1) / bn2) * sp / 256;
+      const int slots = t.cfg == 12 || t.cfg == 13 ? 2 : 1;
+      const double rounds = std::ceil(n - 1e-9) / slots;   // of the chip's slots
+      take(t.c0 + std::max(t.step * kps * rounds, t.mem * ((double)N * K + (double)M * K) * 2e-6) +
+               t.slab * sp * M * N * 4e-6 + t.wgs * n + t.mid * mid * kps, 0, t.cfg, p);
+    }
+  }
+  if (M <= 32) {   // as rows_kind
+    const int nt = N > 4096 ? 2 : 1;
+    const double kb = K * 2e-3, wgs = (double)((N + 16 * nt - 1) / (16 * nt));
+    take(1.91 + 1.36 + (mid ? 1.56 : 1.) * std::max(std::ceil(wgs / 256) * (16 * nt + M) * kb / (nt == 2 ? 26.4 : 30.4),
+                                                    (N + 0.65 * wgs * M) * kb / 5844), 1, 0, 1);
+  }
+  return 1;
+}
+
+// The product alone, as f32 slabs ws [slabs][M][N] that the launch behind it sums (gemm_slabs.hip).  kind 0:
+// tiles `cfg` (no four-wave tile) with k in `parts`; 1: the direct form; 2: the stream form, every strip in
+// `parts` of whole steps.  Returns the number of slabs, or minus a HIP error.
+CAKE_API int cake_gemm_slabs(int dt, int kind, int cfg, int parts, const void* a, long long lda, const void* b,
+                             long long ldb, float* ws, const void* zeros, int M, int N, int K, hipStream_t st) {
+  if (M < 1 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || parts < 1 || !ws || !zeros ||
+      !(dt == kBF16 || dt == kF16) || (kind != 0 && M > 64) || (kind == 1 && (M > 32 || parts != 1)) ||
+      (kind == 0 && (parts < 2 || four_wave_cfg(cfg) || cfg == kRSCfg)) || kind < 0 || kind > 2)
+    return -(int)hipErrorInvalidValue;
+  if (kind == 1) {
+    const int e = cake_gemm_rows(dt, kEpiStore32, 1, a, lda, b, ldb, nullptr, 0, nullptr, ws, N, nullptr, nullptr,
+                                 zeros, M, N, K, 1.f, st);
+    return e ? -e : 1;
+  }
+  GemmArgs g{};
+  g.a = (const uint16_t*)a; g.b = (const uint16_t*)b;
+  g.ws = ws; g.zeros = (const uint16_t*)zeros;
+  g.lda = lda; g.ldb = ldb;
+  g.M = M; g.N = g.Nv = g.half = N; g.K = K;
+  if (kind == 0) {
+    const SplitPlan sp = split_plan(cfg, parts, M, N, K);
+    if (sp.bm == 0 || sp.splits < 2) return -(int)hipErrorInvalidValue;
+    g.tiles_m = (M + sp.bm - 1) / sp.bm;
+    g.tiles_n = (N + sp.bn - 1) / sp.bn;
+    g.kps = sp.kps;
+    const dim3 grid(g.tiles_m * g.tiles_n, sp.splits);
+    const int e = dt == kBF16 ? dispatch_epi<kBF16>(kEpiPartial, cfg, grid, st, g)
+                              : dispatch_epi<kF16>(kEpiPartial, cfg, grid, st, g);
+    return e ? -e : sp.splits;
+  }
+  const int mt = (M + 15) / 16, bn = mt > 1 ? 128 : 64, kst = mt > 1 ? 64 : 128;
+  const int ks = (K + kst - 1) / kst;
+  g.tiles_m = 1;
+  g.tiles_n = (N + bn - 1) / bn;
+  g.kps = (ks + parts - 1) / parts;
+  g.pieces = (ks + g.kps - 1) / g.kps;   // no part without a step
+  const long long wgs = (long long)g.tiles_n * g.pieces;
+  if (wgs > 0x7fffff) return -(int)hipErrorInvalidValue;
+  const int e = dt == kBF16 ? Rows<kBF16>::run(kEpiPartial, 2, mt, dim3((unsigned)wgs), st, g)
+                            : Rows<kF16>::run(kEpiPartial, 2, mt, dim3((unsigned)wgs), st, g);
+  return e ? -e : g.pieces;
 }
 
 // cake_gemm_grouped in the stream form: tiles of at most 16 rows; ws and tick as above (ws of 16

@@ -25,7 +25,7 @@ enum GemmEpi : int {
   kEpiGelu = 9,
   kEpiRelu2 = 10,
 };
-constexpr bool act_epi(int epi) { return epi >= kEpiSilu; }
+constexpr bool act_epi(int epi) { return epi >= kEpiSilu && epi <= kEpiRelu2; }
 
 // erf by Abramowitz & Stegun, formula 7.1.26 (|error| <= 1.5e-7): one exponential, one
 // reciprocal and a polynomial, no branch — the epilogue evaluates it once per output, where

@@ -223,12 +223,14 @@ __device__ __forceinline__ void stream_read(uint32_t lo, uint32_t hi, uint4 (&a)
 struct StreamStrip {   // one strip of the step sequence
   const uint16_t *a, *b;
   uint16_t* c;
+  float* f;   // f32 output, rows ldf apart
+  long long ldf;
   int M, v0;
 };
 
 template <bool GRP, int BN>
 __device__ __forceinline__ StreamStrip stream_strip(const GemmArgs& g, int s) {
-  StreamStrip r{g.a, g.b, g.c, g.M, s * BN};
+  StreamStrip r{g.a, g.b, g.c, g.r32, g.ldr, g.M, s * BN};
   if constexpr (GRP) {
     const int4 t = g.groups[s / g.tiles_n];
     r.a += (size_t)t.y * g.lda;
@@ -276,10 +278,10 @@ __device__ __forceinline__ void stream_store(const GemmArgs& g, const StreamStri
         if constexpr (act_epi(EPI)) a = gemm_act<EPI>(a);
         y[e] = a;
       }
-      if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32) {
+      if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32 || EPI == kEpiPartial) {
         constexpr bool ADD = EPI == kEpiResid32;
-        float* o = g.r32 + (size_t)m * g.ldr + n;
-        if (full && ((g.ldr | n) & 3) == 0) {
+        float* o = s.f + (size_t)m * s.ldf + n;
+        if (full && ((s.ldf | n) & 3) == 0) {
           float4 v = ADD ? *reinterpret_cast<float4*>(o) : make_float4(0.f, 0.f, 0.f, 0.f);
           v.x = fmaf(g.alpha, y[0], v.x); v.y = fmaf(g.alpha, y[1], v.y);
           v.z = fmaf(g.alpha, y[2], v.z); v.w = fmaf(g.alpha, y[3], v.w);
@@ -320,11 +322,15 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
   const int KS = (g.K + KST - 1) / KST;
   const int strips = (GRP ? g.groups[g.tiles_m].x : 1) * g.tiles_n;
   const int total = strips * KS;
-  const int per = max((total + (int)gridDim.x - 1) / (int)gridDim.x, g.kps);
+  const int per = EPI == kEpiPartial ? g.kps : max((total + (int)gridDim.x - 1) / (int)gridDim.x, g.kps);
   // neighbouring shares on one XCD (they read one strip's x and meet in its sums)
   const int nwg = gridDim.x, q8 = nwg / 8, r8 = nwg % 8, x8 = blockIdx.x % 8;
   const int wg = (x8 < r8 ? x8 * (q8 + 1) : r8 * (q8 + 1) + (x8 - r8) * q8) + blockIdx.x / 8;
-  const int u0 = wg * per, u1 = min(total, u0 + per);
+  // slabs: every strip in g.pieces parts of g.kps steps (the last what is left), which do not meet
+  const bool parts = EPI == kEpiPartial && g.pieces > 1;
+  const int part = parts ? wg % g.pieces : 0;
+  const int u0 = parts ? wg / g.pieces * KS + part * per : wg * per;
+  const int u1 = parts ? min((wg / g.pieces + 1) * KS, u0 + per) : min(total, u0 + per);
   if (u0 >= u1) return;
 
   // ---- DMA: wave w fetches weight rows 16 RT w .. and its share of x ----
@@ -336,9 +342,9 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
   // halves at 24 rows 28.1, 23.1; each half 5 steps on 25.5).  128-row parts that are no multiple of 4 KB apart spread by
   // themselves, and in step read x together (4096 x 14336 in 256 eighths of 3.5 KB at 24 rows 25.9, 26.7
   // turned; 8192 x 28672 at 64 rows 85.1, 86.7; of 64 rows, two on a CU, at 5 rows 88.3, 71.3 turned).
-  const int seg = KS % per == 0 ? per : per % KS == 0 ? KS : 0;   // 0: other shares
+  const int seg = parts ? u1 - u0 : KS % per == 0 ? per : per % KS == 0 ? KS : 0;   // 0: other shares
   const bool turn = seg == KS || S::KC == 2 || seg * KST * 2 % 4096 == 0;
-  const int seg0 = seg > 0 ? dk / seg * seg : 0;
+  const int seg0 = parts ? dk : seg > 0 ? dk / seg * seg : 0;
   if (seg > 0 && turn) dk = seg0 + u0 / max(per, KS) * 5 % seg;
   int left = seg;
   const uint16_t *wsrc[4], *xsrc[S::XI];
@@ -434,10 +440,14 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
       }
       buf = buf + 1 == S::NS ? 0 : buf + 1;
     }
-    const StreamStrip t = stream_strip<GRP, S::BN>(g, s);
+    StreamStrip t = stream_strip<GRP, S::BN>(g, s);
+    if constexpr (EPI == kEpiPartial) {
+      t.f = g.ws + (size_t)part * g.M * g.Nv;
+      t.ldf = g.Nv;
+    }
     const int lo = s * KS / per, hi = ((s + 1) * KS - 1) / per;   // shares with steps of this strip
-    bool mine = lo == hi;
-    if (lo != hi) {
+    bool mine = EPI == kEpiPartial || lo == hi;
+    if (!mine) {
       auto slot = [&](int w) {   // a share's first strip, or its last
         return g.ws + ((size_t)(2 * w + (w * per / KS == s ? 0 : 1)) * NWV + wave) * (RT * MT * 256) + lane * 4;
       };
@@ -489,14 +499,20 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(GemmArgs g) {
 }
 
 template <int DT, int EPI>
-int launch_rows(int kind, int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
+int launch_stream(int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
 #define CAKE_STREAM(MT)                                                                             \
-  if (kind == 2 && mt == MT) {                                                                      \
+  if (mt == MT) {                                                                                   \
     hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI, MT, false>), grid, dim3(256), 0, st, g);        \
     return (int)hipGetLastError();                                                                  \
   }
   CAKE_STREAM(1) CAKE_STREAM(2) CAKE_STREAM(3) CAKE_STREAM(4)
 #undef CAKE_STREAM
+  return (int)hipErrorInvalidValue;
+}
+
+template <int DT, int EPI>
+int launch_rows(int kind, int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  if (kind == 2) return launch_stream<DT, EPI>(mt, grid, st, g);
   constexpr bool GATED = (EPI == kEpiSwiglu || EPI == kEpiGeglu);
 #define CAKE_DIRECT(KIND, MT, NT)                                                                   \
   if constexpr (!GATED || NT == 2)                                                                  \
@@ -518,6 +534,7 @@ template <int DT> struct Rows {
       X(kEpiStore) X(kEpiResid32) X(kEpiAdd16) X(kEpiSwiglu) X(kEpiGeglu) X(kEpiStore32)
       X(kEpiSilu) X(kEpiQuick) X(kEpiGelu) X(kEpiRelu2)
 #undef X
+      case kEpiPartial: return launch_stream<DT, kEpiPartial>(mt, grid, st, g);
     }
     return (int)hipErrorInvalidValue;
   }

@@ -357,21 +357,39 @@ class LayerStack:
         from ...ops import hip as K
         cfg = self.cfg
         T, H = hidden.shape
-        x = torch.empty((T, H), device=hidden.device, dtype=self.dtype)
-        K.rmsnorm(hidden, w.ln1, cfg.rms_norm_eps, x)
         nh, nkv, hd = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
-        nq, nk = nh * hd, nkv * hd
-        qkv = G.linear(x, w.wqkv)  # one GEMM for q|k|v
-        q, k, v = qkv[:, :nq], qkv[:, nq:nq + nk], qkv[:, nq + nk:]
-        K.rope_kv(q, k, v, self.inv_freq, pos0, kc, vc)
+        nq, nk, inter = nh * hd, nkv * hd, cfg.intermediate_size
+        nqkv, adds = nq + 2 * nk, H <= G.SLAB_NORM_MAX
+        # the products that leave slabs, as the native run of blocks chooses them (ops/llama_rows.py)
+        f_qkv = G.slab_form(T, nqkv, H, "store") if hd % 8 == 0 and hd <= 256 else None
+        f_o = G.slab_form(T, H, nq, "resid32") if adds else None
+        f_down = G.slab_form(T, H, inter, "resid32") if adds else None
+        x = torch.empty((T, H), device=hidden.device, dtype=self.dtype)
+        if f_down:
+            G.slab_norm(None, 0, hidden, w.ln1, cfg.rms_norm_eps, x)
+        else:
+            K.rmsnorm(hidden, w.ln1, cfg.rms_norm_eps, x)
+        if f_qkv:
+            q = torch.empty((T, nq), device=hidden.device, dtype=self.dtype)
+            G.slab_rope(*G.slabs(x, w.wqkv, f_qkv), q, nh, self.inv_freq, pos0, kc, vc)
+        else:
+            qkv = G.linear(x, w.wqkv)  # one GEMM for q|k|v
+            q, k, v = qkv[:, :nq], qkv[:, nq:nq + nk], qkv[:, nq + nk:]
+            K.rope_kv(q, k, v, self.inv_freq, pos0, kc, vc)
         att = torch.empty((T, nq), device=hidden.device, dtype=self.dtype)
         Tk = pos0 + T
         K.flash_attn(q.view(1, T, nh, hd).transpose(1, 2), kc[None, :, :Tk], vc[None, :, :Tk],
                      att.view(1, T, nh, hd).transpose(1, 2), self.scale, causal=True, pos0=pos0)
-        G.linear(att, w.wo, epi="resid32", resid=hidden)      # hidden += att @ wo^T
-        K.rmsnorm(hidden, w.ln2, cfg.rms_norm_eps, x)
+        if f_o:
+            G.slab_norm(*G.slabs(att, w.wo, f_o), hidden, w.ln2, cfg.rms_norm_eps, x)
+        else:
+            G.linear(att, w.wo, epi="resid32", resid=hidden)      # hidden += att @ wo^T
+            K.rmsnorm(hidden, w.ln2, cfg.rms_norm_eps, x)
         act = G.linear(x, w.wgu, epi="swiglu")                # silu(x wg^T) * (x wu^T)
-        G.linear(act, w.wd, epi="resid32", resid=hidden)      # hidden += act @ wd^T
+        if f_down:
+            G.slab_norm(*G.slabs(act, w.wd, f_down), hidden, w.ln1, cfg.rms_norm_eps, None)
+        else:
+            G.linear(act, w.wd, epi="resid32", resid=hidden)  # hidden += act @ wd^T
 
     # ------------------------------------------------------------------ torch path
     def _block_torch(self, hidden, w, kc, vc, pos0):

@@ -91,6 +91,15 @@ def _lib():
         lib.cake_gemm_rows.argtypes = [I, I, I, P, L, P, L, P, L, P, P, L, P, P, P, I, I, I,
                                        C.c_float, P]
         lib.cake_gemm_rows.restype = I
+        lib.cake_gemm_slab_plan.argtypes = [I, L, I, I, I, P, P, P]
+        lib.cake_gemm_slab_plan.restype = I
+        lib.cake_gemm_slabs.argtypes = [I, I, I, I, P, L, P, L, P, P, I, I, I, P]
+        lib.cake_gemm_slabs.restype = I
+        lib.cake_slab_norm.argtypes = [I, P, I, P, L, P, C.c_float, P, I, C.c_float, C.c_float, I, I,
+                                       I, P, L, P]
+        lib.cake_slab_norm.restype = I
+        lib.cake_slab_rope.argtypes = [I, P, I, P, I, I, I, I, I, P, I, I, P, P, P]
+        lib.cake_slab_rope.restype = I
         lib.cake_gemm_rows_grouped.argtypes = [I, I, P, L, P, L, L, P, L, P, I, P, P, P, I, I, P]
         lib.cake_gemm_rows_grouped.restype = I
         _bound = True
@@ -153,6 +162,28 @@ def rows_kind(M: int, Nv: int, K: int, gated: bool) -> int:
     if kind is None:
         kind = _rows_kinds[key] = int(_lib().cake_gemm_rows_kind(M, Nv, K, int(gated)))
     return kind
+
+
+SLAB_NORM_MAX = 8192   # columns of a row that slab_norm holds
+_slab_forms: dict = {}
+
+
+def slab_form(M: int, N: int, K: int, epi: str, big: bool = False):
+    """(kind, cfg, parts) of a product that leaves its sums in `parts` slabs or fewer for the launch
+    behind it (gemm.hip cake_gemm_slab_plan), or None: the product as :func:`linear` runs it with `epi`,
+    a launch of its own behind it.  Pinned plans run as pinned."""
+    if (M, N, K, epi) in _plans or N % 4 or K % 8:
+        return None
+    key = (M, N, K, epi, big)
+    f = _slab_forms.get(key, 0)
+    if f == 0:
+        if len(_slab_forms) >= 65536:
+            _slab_forms.clear()
+        k, c, p = C.c_int(0), C.c_int(0), C.c_int(1)
+        on = _lib().cake_gemm_slab_plan(M, N, K, EPI[epi], int(big), C.addressof(k), C.addressof(c),
+                                        C.addressof(p))
+        f = _slab_forms[key] = (k.value, c.value, p.value) if on else None
+    return f
 
 
 def _counters(dev, st: int) -> torch.Tensor:
@@ -448,6 +479,62 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
         None if ws is None else ws.data_ptr(), None if tick is None else tick.data_ptr(),
         _zeros16(x.device).data_ptr(), M, N, K, float(alpha), st), "gemm")
     return resid if f32_out else out
+
+
+def slabs(x: torch.Tensor, w: torch.Tensor, form) -> tuple[torch.Tensor, int]:
+    """x [M, K] w [N, K]^T as f32 slabs [n, M, N] of a workspace, form of :func:`slab_form`: (slabs, n)
+    for :func:`slab_norm` or :func:`slab_rope`."""
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.stride(1) != 1 or \
+            w.stride(1) != 1 or x.dtype not in _DT or w.dtype != x.dtype or not (x.is_cuda and w.is_cuda):
+        raise TypeError("gemm.slabs: 16-bit device matrices of one dtype expected")
+    (M, K), N = x.shape, w.shape[0]
+    lda = x.stride(0) if M > 1 else K
+    if lda < K or lda % 8 or w.stride(0) % 8 or x.data_ptr() % 16 or w.data_ptr() % 16:
+        raise ValueError("gemm.slabs: rows of a multiple of 8 on 16-byte boundaries")
+    kind, cfg, parts = form
+    ws = torch.empty(parts * M * N, device=x.device, dtype=torch.float32)
+    n = _lib().cake_gemm_slabs(_DT[x.dtype], kind, cfg, parts, x.data_ptr(), lda, w.data_ptr(), w.stride(0),
+                               ws.data_ptr(), _zeros16(x.device).data_ptr(), M, N, K, current_stream())
+    check(max(0, -n), "gemm_slabs")
+    return ws, n
+
+
+def slab_norm(ws, n: int, x: torch.Tensor, w, eps: float, out, *, bias=None, alpha: float = 1.0,
+              offset: float = 0.0, ln: bool = False) -> None:
+    """x [M, >= N] f32 [:, :N] += alpha (the sum of n slabs + bias [N]); then, with w [N] (f32 or the
+    storage type), out [M, N] = the RMS norm (ln: layer norm) of that times (offset + w).  n 0: of x as
+    it is.  out None: 16-bit type of w, no norm."""
+    N = (w if out is None else out).shape[-1]
+    M, t = x.shape[0], w if out is None else out
+    if x.dtype != torch.float32 or x.stride(1) != 1 or t.dtype not in _DT or not x.is_cuda or \
+            x.shape[1] < N or (n and ws.numel() < n * M * N) or (bias is not None and (
+                bias.dtype != t.dtype or bias.numel() != N or not bias.is_contiguous())):
+        raise ValueError("slab_norm: f32 rows, 16-bit output and bias expected")
+    ld = 0
+    if out is not None:
+        ld = out.stride(0) if M > 1 else N
+        if out.shape[0] != M or out.stride(1) != 1 or w.numel() < N or not w.is_contiguous() or \
+                w.dtype not in (torch.float32, out.dtype):
+            raise ValueError("slab_norm: norm weights of the output's columns expected")
+    check(_lib().cake_slab_norm(
+        _DT[t.dtype], ws.data_ptr() if n else None, n, x.data_ptr(), x.stride(0) if M > 1 else x.shape[1],
+        None if bias is None else bias.data_ptr(), float(alpha), None if out is None else w.data_ptr(),
+        int(w.dtype == torch.float32), float(offset), float(eps), int(ln), M, N,
+        None if out is None else out.data_ptr(), ld, current_stream()), "slab_norm")
+
+
+def slab_rope(ws, n: int, q: torch.Tensor, heads: int, inv_freq, pos0: int, kc, vc) -> None:
+    """hip.rope_kv of rows that are sums of n slabs [T, (heads + 2 nkv) hd]: rotated queries to q
+    [T, >= heads hd], keys and values to rows pos0 .. of kc, vc [nkv, S, hd]."""
+    T, (nkv, S, hd) = q.shape[0], kc.shape
+    if q.dtype not in _DT or kc.dtype != q.dtype or vc.dtype != q.dtype or q.stride(1) != 1 or \
+            q.shape[1] < heads * hd or not (kc.is_contiguous() and vc.is_contiguous()) or \
+            vc.shape != kc.shape or ws.numel() < n * T * (heads + 2 * nkv) * hd or \
+            inv_freq.dtype != torch.float32 or inv_freq.numel() != hd // 2:
+        raise ValueError("slab_rope: 16-bit rows and caches of one dtype expected")
+    check(_lib().cake_slab_rope(_DT[q.dtype], ws.data_ptr(), n, q.data_ptr(),
+                                q.stride(0) if T > 1 else q.shape[1], T, heads, nkv, hd, inv_freq.data_ptr(),
+                                int(pos0), S, kc.data_ptr(), vc.data_ptr(), current_stream()), "slab_rope")
 
 
 # tile configuration of a grouped product -> its rows (ROWS: the stream form; BY_LIST: 128, 160, 192 or 256,

@@ -16,37 +16,43 @@ P, I, F = C.c_void_p, C.c_int, C.c_float
 
 
 class _Form(C.Structure):
-    _fields_ = [("kind", I), ("cfg", I), ("splits", I)]
+    _fields_ = [("kind", I), ("cfg", I), ("splits", I), ("slabs", I)]
 
 
 class _Run(C.Structure):
     _fields_ = [(n, P) for n in ("blocks", "hidden", "x", "qkv", "att", "act", "inv_freq", "zeros",
-                                 "ws", "rows_ws", "tick")] + \
+                                 "ws", "slabs", "rows_ws", "tick")] + \
                [(n, _Form) for n in ("qkv_form", "o_form", "gu_form", "down_form")] + \
                [(n, I) for n in ("n", "dt", "T", "H", "I", "nh", "nkv", "hd", "S", "pos0")] + \
                [("eps", F), ("scale", F)]
 
 
 def _forms(T: int, products, capturing: bool):
-    """(kind, cfg, splits) of each (Nv, K, epi), as gemm.linear chooses them, and the slab floats
-    that the tile plans need; None if one of them is the library GEMM's."""
-    forms, floats = [], 0
-    for Nv, K, epi in products:
+    """(kind, cfg, splits) of each (Nv, K, epi), as gemm.linear chooses them or, of those that a sum of
+    slabs may follow, as gemm.slab_form does; the floats that the tile plans' slabs need, and those of
+    the products that leave them.  None if one of them is the library GEMM's."""
+    forms, floats, left = [], 0, 0
+    for Nv, K, epi, summed in products:
         gated = epi == "swiglu"
+        big = max(T, Nv) * K * 2 >= 0x7fffffff
+        slab = G.slab_form(T, Nv, K, epi, big) if summed else None
+        if slab is not None:
+            left = max(left, slab[2] * T * Nv)
+            forms.append(_Form(*slab, 1))
+            continue
         kind = G.rows_kind(T, Nv, K, gated) if (T, Nv, K, epi) not in G._plans else 0
         if kind == 2 and capturing:
             kind = 0
         cfg, splits = 0, 1
         if not kind:
-            big = max(T, Nv) * K * 2 >= 0x7fffffff
             cfg, splits = G.resolve(T, Nv, K, epi, big)
             if cfg == G.LIB:
-                return None, 0
+                return None, 0, 0
             if splits > 1:
                 floats = max(floats, int(G._lib().cake_gemm_ws_floats(
                     cfg, splits, T, Nv // 2 if gated else Nv, K, int(gated))))
-        forms.append(_Form(kind, cfg, splits))
-    return forms, floats
+        forms.append(_Form(kind, cfg, splits, 0))
+    return forms, floats, left
 
 
 def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Tensor,
@@ -79,8 +85,10 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
             ptrs.append(p)
         table[8 * i:8 * i + 8] = [*ptrs, kp + s * step, vp + s * step]
     capturing = torch.cuda.is_current_stream_capturing()
-    forms, floats = _forms(T, ((nqkv, H, "store"), (H, nq, "resid32"), (2 * inter, H, "swiglu"),
-                               (H, inter, "resid32")), capturing)
+    adds = H <= G.SLAB_NORM_MAX
+    forms, floats, left = _forms(T, ((nqkv, H, "store", True), (H, nq, "resid32", adds),
+                                     (2 * inter, H, "swiglu", False), (H, inter, "resid32", adds)),
+                                 capturing)
     if forms is None:
         return False
     dev, st = hidden.device, current_stream()
@@ -89,13 +97,14 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
     att = torch.empty((T, nq), device=dev, dtype=dt)
     act = torch.empty((T, inter), device=dev, dtype=dt)
     ws = G._workspace(dev, floats) if floats else None
+    slabs = torch.empty(left, device=dev, dtype=torch.float32) if left else None
     rows_ws = tick = None
-    if any(f.kind == 2 for f in forms):
+    if any(f.kind == 2 and not f.slabs for f in forms):
         rows_ws, tick = G._rows_state(dev, T, st)
-    elif any(f.splits > 1 and f.cfg in G.FOUR_WAVE for f in forms):
+    elif any(f.splits > 1 and f.cfg in G.FOUR_WAVE and not f.slabs for f in forms):
         tick = G._counters(dev, st)
     ptr = [None if t is None else t.data_ptr() for t in (
-        hidden, x, qkv, att, act, inv_freq, G._zeros16(dev), ws, rows_ws, tick)]
+        hidden, x, qkv, att, act, inv_freq, G._zeros16(dev), ws, slabs, rows_ws, tick)]
     run = _Run(C.addressof(table), *ptr, *forms, len(blocks), G._DT[dt], T, H, inter, nh, nkv, hd, S,
                int(pos0), float(cfg.rms_norm_eps), float(scale))
     check(kernels().cake_block_rows(C.addressof(run), st), "block_rows")
