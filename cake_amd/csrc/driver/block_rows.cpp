@@ -6,7 +6,7 @@
 // what is left per launch is the kernel library's own entry point (2 - 3 us).
 //
 // Of few rows the q/k/v, output and down products leave their sums in slabs, which the rotation and the next
-// norm add up: six launches a block instead of up to eleven (45 rows of an 8B block 130 us, 115 so).
+// norm add up: six launches a block instead of up to eleven (a block of 8B at 45 rows 122 us, 116 so).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -658,6 +658,30 @@ CAKE_API int cake_gemm_slabs(int dt, int kind, int cfg, int parts, const void* a
   return e ? -e : g.pieces;
 }
 
+// A layer's projections in one launch of the stream form, by columns: [0, n1) to c1 (16-bit), [n1, n2) to r32,
+// [n2, N) gelu to c.  n1, n2 multiples of 4; bases 16-byte aligned; ws, tick as above.
+CAKE_API int cake_gemm_rows_sections(int dt, const void* a, long long lda, const void* b, long long ldb, void* c1,
+                                     long long ldc1, float* r32, long long ldr, void* c, long long ldc, int n1,
+                                     int n2, float* ws, void* tick, const void* zeros, int M, int N, int K,
+                                     hipStream_t st) {
+  if (M < 1 || M > 64 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8 || n1 < 0 || n2 < n1 || n2 > N ||
+      n1 % 4 || n2 % 4 || (n1 > 0 && !c1) || (n2 > n1 && !r32) || (N > n2 && !c) || !ws || !tick || !zeros ||
+      (((uintptr_t)c1 | (uintptr_t)r32 | (uintptr_t)c) & 15))
+    return (int)hipErrorInvalidValue;
+  const StreamPlan sp = stream_plan(M, N, K, false);
+  GemmArgs g{};
+  g.a = (const uint16_t*)a; g.b = (const uint16_t*)b; g.c = (uint16_t*)c; g.c1 = (uint16_t*)c1;
+  g.r32 = r32; g.ws = ws; g.tick = (unsigned*)tick; g.zeros = (const uint16_t*)zeros;
+  g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.ldc1 = ldc1; g.ldr = ldr;
+  g.M = M; g.N = g.Nv = g.half = N; g.K = K; g.n1 = n1; g.n2 = n2;
+  g.tiles_m = 1;
+  g.tiles_n = (N + sp.bn - 1) / sp.bn;
+  if (g.tiles_n > kRowsTicks) return (int)hipErrorInvalidValue;
+  g.kps = sp.per;
+  return dt == kBF16 ? Rows<kBF16>::run(kEpiSections, 2, (M + 15) / 16, dim3(sp.wgs), st, g)
+         : dt == kF16 ? Rows<kF16>::run(kEpiSections, 2, (M + 15) / 16, dim3(sp.wgs), st, g) : (int)hipErrorInvalidValue;
+}
+
 // cake_gemm_grouped in the stream form: tiles of at most 16 rows; ws and tick as above (ws of 16
 // rows).  More strips than counters, or steps than the kernel's indexes hold (1024 experts of 4096
 // columns with 1500 rows): the 64-row tile, which takes the same tile list.

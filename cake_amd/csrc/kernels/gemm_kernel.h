@@ -24,6 +24,7 @@ enum GemmEpi : int {
   kEpiQuick = 8,   //   quick_gelu, erf-GELU (CLIP MLP, hybrid feed-forwards), relu^2
   kEpiGelu = 9,
   kEpiRelu2 = 10,
+  kEpiSections = 11,  // columns [0, n1) C1 16-bit, [n1, n2) R32, the others C16 = gelu (gemm_rows.h only)
 };
 constexpr bool act_epi(int epi) { return epi >= kEpiSilu && epi <= kEpiRelu2; }
 
@@ -81,6 +82,10 @@ struct GemmArgs {
   // the number of tiles and, where `pieces` (here the tiles' rows) is 0, their rows
   const int4* groups;
   long long b_group;
+  // kEpiSections
+  uint16_t* c1;
+  long long ldc1;
+  int n1, n2;
 };
 constexpr int kPieceTiles = 256;
 

@@ -278,7 +278,22 @@ __device__ __forceinline__ void stream_store(const GemmArgs& g, const StreamStri
         if constexpr (act_epi(EPI)) a = gemm_act<EPI>(a);
         y[e] = a;
       }
-      if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32 || EPI == kEpiPartial) {
+      if constexpr (EPI == kEpiSections) {   // a group of four columns lies in one section
+        const bool act = n >= g.n2;
+        if (!act && n >= g.n1) {
+          float* o = g.r32 + (size_t)m * g.ldr + (n - g.n1);
+          if ((g.ldr & 3) == 0) *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
+          else for (int e = 0; e < 4; ++e) o[e] = y[e];
+          continue;
+        }
+        uint16_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = from_f32<DT>(act ? gemm_act<kEpiGelu>(y[e]) : y[e]);
+        const long long ld = act ? g.ldc : g.ldc1;
+        uint16_t* o = (act ? g.c - g.n2 : g.c1) + (size_t)m * ld + n;
+        if (full && (ld & 3) == 0) *reinterpret_cast<uint2*>(o) = make_uint2(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16);
+        else for (int e = 0; e < 4; ++e) if (n + e < g.N) o[e] = v[e];
+      } else if constexpr (EPI == kEpiResid32 || EPI == kEpiStore32 || EPI == kEpiPartial) {
         constexpr bool ADD = EPI == kEpiResid32;
         float* o = s.f + (size_t)m * s.ldf + n;
         if (full && ((s.ldf | n) & 3) == 0) {
@@ -535,6 +550,7 @@ template <int DT> struct Rows {
       X(kEpiSilu) X(kEpiQuick) X(kEpiGelu) X(kEpiRelu2)
 #undef X
       case kEpiPartial: return launch_stream<DT, kEpiPartial>(mt, grid, st, g);
+      case kEpiSections: return launch_stream<DT, kEpiSections>(mt, grid, st, g);
     }
     return (int)hipErrorInvalidValue;
   }

@@ -8,7 +8,8 @@ position.  A parallel layer is three stages — norm + input projections, mixer,
 layer has its feed-forward (:mod:`.feedforward`) behind them.
 
 * prompt rows: MFMA GEMMs (ops/gemm.py; the feed-forward's activation and the scaled residual
-  sum in their epilogues), prompt kernels of the mixers (ops/mixers.py, ops/latent.py);
+  sum in their epilogues), prompt kernels of the mixers (ops/mixers.py, ops/latent.py); of up to 64
+  rows all projections of a layer are one product by sections (gemm.sections);
 * one token of one sequence, 16-bit: three launches per parallel layer run
   (:meth:`decode_layers`, the body of the captured decode graph, models/decoder.py);
 * one token of several sequences: the GEMMs over the batch, the mixers' decode kernels;
@@ -180,14 +181,22 @@ class HybridModel:
         h = self.norm_rows(x, w.norm32)
         new = torch.empty if w.mix_cols == w.shape.out_cols and w.ff % 8 == 0 else torch.zeros
         mix = new((N, w.out_cols), device=self.device, dtype=self.dtype)
-        if w.ff:
-            self.product_act(h, w.w_in[w.n_raw:], mix[:, w.mix_cols:w.mix_cols + w.ff])
         # the mixers' decode kernels read f32 projections, as the fused step leaves them; a latent
         # is normed before anything else reads it
         pdt = torch.float32 if decode or isinstance(m, LatentMixer) else self.dtype
         ncol = w.n_raw if decode else w.n_main
         proj = torch.empty((N, M.pad_to(ncol, 8)), device=self.device, dtype=pdt)
-        self.product(h, w.w_in[:ncol], proj[:, :ncol])
+        ab = None if decode or not w.n_ab else \
+            torch.empty((N, w.n_ab), device=self.device, dtype=torch.float32)
+        up = mix[:, w.mix_cols:w.mix_cols + w.ff]
+        if not (w.ff and self.dtype != torch.float32 and G.sections(
+                h, w.w_in, 0 if decode else w.n_main, w.n_raw, proj[:, :ncol],
+                proj[:, :ncol] if decode else ab, up)):
+            if w.ff:
+                self.product_act(h, w.w_in[w.n_raw:], up)
+            self.product(h, w.w_in[:ncol], proj[:, :ncol])
+            if ab is not None:
+                self.product(h, w.w_in[w.n_main:w.n_raw], ab)
         a, b = self.pool.bufs[run.index]
         if isinstance(m, LatentMixer):
             self._latent_rows(m, w, proj, rows, a, mix, LATENT_SPLITS[nsplit])
@@ -206,8 +215,6 @@ class HybridModel:
             M.delta_decode(w.shape, proj, proj[:, w.n_main:w.n_raw], rows.pos, rows.slot, cfg.eps,
                            **w.consts, state=a, ring=b, out=mix)
         else:
-            ab = torch.empty((N, w.n_ab), device=self.device, dtype=torch.float32)
-            self.product(h, w.w_in[w.n_main:w.n_raw], ab)
             M.delta_prompt(w.shape, proj, ab, rows, cfg.eps, **w.consts, state=a, ring=b, out=mix)
         self.product_add(mix, w.w_out, x, cfg.residual_mult)
         if w.post is not None:

@@ -100,6 +100,9 @@ def _lib():
         lib.cake_slab_norm.restype = I
         lib.cake_slab_rope.argtypes = [I, P, I, P, I, I, I, I, I, P, I, I, P, P, P]
         lib.cake_slab_rope.restype = I
+        lib.cake_gemm_rows_sections.argtypes = [I, P, L, P, L, P, L, P, L, P, L, I, I, P, P, P, I, I,
+                                                I, P]
+        lib.cake_gemm_rows_sections.restype = I
         lib.cake_gemm_rows_grouped.argtypes = [I, I, P, L, P, L, L, P, L, P, I, P, P, P, I, I, P]
         lib.cake_gemm_rows_grouped.restype = I
         _bound = True
@@ -479,6 +482,38 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
         None if ws is None else ws.data_ptr(), None if tick is None else tick.data_ptr(),
         _zeros16(x.device).data_ptr(), M, N, K, float(alpha), st), "gemm")
     return resid if f32_out else out
+
+
+def sections(x: torch.Tensor, w: torch.Tensor, n1: int, n2: int, out16, out32, act) -> bool:
+    """x [M, K] w [N, K]^T of few rows as one launch: columns [0, n1) to out16 (storage type), [n1, n2)
+    to out32 (f32), the others through the erf GELU to act; matrices with row strides, None where a
+    section is empty.  False, with nothing launched, where the stream form is not the product's."""
+    (M, K), N = x.shape, w.shape[0]
+    if M > ROWS_MAX or x.dtype not in _DT or n1 % 4 or n2 % 4 or K % 8 or \
+            rows_kind(M, N, K, False) != 2 or torch.cuda.is_current_stream_capturing():
+        return False
+    ptrs, lds = [], []
+    for t, n, dt in ((out16, n1, x.dtype), (out32, n2 - n1, torch.float32), (act, N - n2, x.dtype)):
+        if n == 0:
+            ptrs.append(None)
+            lds.append(0)
+            continue
+        if t.dtype != dt or tuple(t.shape) != (M, n) or t.stride(1) != 1:
+            raise ValueError(f"sections: {dt} [{M}, {n}] expected")
+        ptrs.append(t.data_ptr())
+        lds.append(t.stride(0) if M > 1 else n)
+    if x.stride(1) != 1 or w.stride(1) != 1 or w.shape[1] != K or w.dtype != x.dtype:
+        raise ValueError("sections: matrices of one 16-bit type expected")
+    lda = x.stride(0) if M > 1 else K
+    if lda % 8 or w.stride(0) % 8 or any((p or 0) % 16 for p in (x.data_ptr(), w.data_ptr(), *ptrs)):
+        return False
+    st = current_stream()
+    ws, tick = _rows_state(x.device, M, st)
+    check(_lib().cake_gemm_rows_sections(
+        _DT[x.dtype], x.data_ptr(), lda, w.data_ptr(), w.stride(0), ptrs[0], lds[0], ptrs[1], lds[1], ptrs[2],
+        lds[2], n1, n2, ws.data_ptr(), tick.data_ptr(), _zeros16(x.device).data_ptr(), M, N, K, st),
+        "gemm_rows_sections")
+    return True
 
 
 def slabs(x: torch.Tensor, w: torch.Tensor, form) -> tuple[torch.Tensor, int]:
