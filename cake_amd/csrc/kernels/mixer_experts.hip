@@ -215,6 +215,68 @@ __global__ __launch_bounds__(256) void expert_sum_kernel(const void* y, long lon
   }
 }
 
+// The same of 16-bit rows up to 4096 NV wide, and the norm of the new row for what reads it next: out[n] =
+// norm(x[n]) (off + w).  A thread has four columns (NV times), so that a row stays in registers between the
+// sum and the norm.
+template <int DT, int NV>
+__global__ __launch_bounds__(1024) void expert_sum_norm_kernel(const uint16_t* y, long long ldy, const int* where,
+                                                               int top, int W, float alpha, float* x, long long ldx,
+                                                               const float* w, float off, float eps, int ln,
+                                                               uint16_t* out, long long ldo) {
+  constexpr int U = 8;
+  __shared__ float red[16];
+  const long long n = blockIdx.x;
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int* wp = where + n * top;
+  float* xr = x + n * ldx;
+  float4 v[NV], wv[NV];
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int i = (j * nt + tid) * 4;
+    v[j] = wv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i >= W) continue;
+    const float4 old = *reinterpret_cast<const float4*>(xr + i);
+    wv[j] = *reinterpret_cast<const float4*>(w + i);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < top; k0 += U) {
+      uint2 p[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (k0 + k < top) p[k] = *reinterpret_cast<const uint2*>(y + (long long)wp[k0 + k] * ldy + i);
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (k0 + k < top) {
+          s[0] += to_f32<DT>((uint16_t)(p[k].x & 0xffffu));
+          s[1] += to_f32<DT>((uint16_t)(p[k].x >> 16));
+          s[2] += to_f32<DT>((uint16_t)(p[k].y & 0xffffu));
+          s[3] += to_f32<DT>((uint16_t)(p[k].y >> 16));
+        }
+    }
+    v[j] = make_float4(fmaf(alpha, s[0], old.x), fmaf(alpha, s[1], old.y), fmaf(alpha, s[2], old.z),
+                       fmaf(alpha, s[3], old.w));
+    *reinterpret_cast<float4*>(xr + i) = v[j];
+    sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
+  }
+  const float mean = ln ? block_sum(sum, red) / (float)W : 0.f;
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    if ((j * nt + tid) * 4 >= W) continue;
+    v[j].x -= mean; v[j].y -= mean; v[j].z -= mean; v[j].w -= mean;
+    ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+  }
+  const float f = 1.f / sqrtf(block_sum(ss, red) / (float)W + eps);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int i = (j * nt + tid) * 4;
+    if (i >= W) continue;
+    const uint16_t o[4] = {from_f32<DT>(v[j].x * f * (off + wv[j].x)), from_f32<DT>(v[j].y * f * (off + wv[j].y)),
+                           from_f32<DT>(v[j].z * f * (off + wv[j].z)), from_f32<DT>(v[j].w * f * (off + wv[j].w))};
+    *reinterpret_cast<uint2*>(out + n * ldo + i) = make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
+  }
+}
+
 // f32 grouped product: out[row0 + r] = act(a[row0 + r] W[expert]^T) for the tiles' rows (BM 32),
 // act < 0: none.  K % 8 == 0.
 __global__ __launch_bounds__(256) void expert_gemm32_kernel(const float* a, long long lda,
@@ -409,6 +471,25 @@ CAKE_API int cake_expert_sum(int dt, const void* y, long long ldy, const int* wh
   if (N == 0) return 0;
   CAKE_MIX_DT(dt, hipLaunchKernelGGL((expert_sum_kernel<DT>), dim3(N), dim3(256), 0, st, y, ldy,
                                      where, top, W, alpha, x, ldx));
+  return (int)hipGetLastError();
+}
+
+// ... and the norm of the new rows: 16-bit types, W % 4 == 0 up to 8192, w [W] f32, out [N][ldo]
+CAKE_API int cake_expert_sum_norm(int dt, const void* y, long long ldy, const int* where, int N, int top, int W,
+                                  float alpha, float* x, long long ldx, const float* w, float off, float eps, int ln,
+                                  void* out, long long ldo, hipStream_t st) {
+  if (N < 0 || top <= 0 || W <= 0 || W % 4 || W > 8192 || ldy < W || ldy % 4 || ldx < W || ldx % 4 || ldo < W ||
+      ldo % 4 || (((uintptr_t)x | (uintptr_t)w) & 15) || (((uintptr_t)y | (uintptr_t)out) & 7) ||
+      !(dt == kBF16 || dt == kF16))
+    return (int)hipErrorInvalidValue;
+  if (N == 0) return 0;
+  const int nt = W > 2048 ? 1024 : W > 1024 ? 512 : 256;
+#define CAKE_SUM_NORM(DT, NV)                                                                                   \
+  hipLaunchKernelGGL((expert_sum_norm_kernel<DT, NV>), dim3(N), dim3(nt), 0, st, (const uint16_t*)y, ldy, where, \
+                     top, W, alpha, x, ldx, w, off, eps, ln, (uint16_t*)out, ldo)
+  if (dt == kBF16) { if (W <= 4096) CAKE_SUM_NORM(kBF16, 1); else CAKE_SUM_NORM(kBF16, 2); }
+  else { if (W <= 4096) CAKE_SUM_NORM(kF16, 1); else CAKE_SUM_NORM(kF16, 2); }
+#undef CAKE_SUM_NORM
   return (int)hipGetLastError();
 }
 

@@ -71,11 +71,15 @@ class DenseFf:
 
     experts = top = 0
 
-    def rows(self, model, x: torch.Tensor) -> None:
-        h = model.norm_rows(x, self.norm32)
+    def rows(self, model, x: torch.Tensor, h=None, next_norm=None):
+        """h: the norm of x if it is there; returns the norm by next_norm of the new x if it is."""
+        h = model.norm_rows(x, self.norm32) if h is None else h
         a = torch.empty((x.shape[0], self.up.shape[0]), device=x.device, dtype=model.dtype)
         model.product_act(h, self.up, a, self.act, self.up_b)
+        if next_norm is not None:
+            return model.add_norm(a, self.down, x, model.cfg.residual_mult, next_norm, self.down_b)
         model.product_add(a, self.down, x, model.cfg.residual_mult, self.down_b)
+        return None
 
     def decode(self, model, b, x: torch.Tensor) -> None:
         cfg = model.cfg
@@ -117,13 +121,14 @@ class ExpertsFf:
     def act_elems(self) -> int:
         return self.top * self.up.shape[1]
 
-    def rows(self, model, x: torch.Tensor) -> None:
+    def rows(self, model, x: torch.Tensor, h=None, next_norm=None):
         """Router over all rows, then the chosen experts as grouped products over rows sorted by
-        expert; a row is normed, scaled by its score and rounded once on its way there."""
+        expert; a row is normed, scaled by its score and rounded once on its way there.  h: the norm of
+        x if it is there; returns the norm by next_norm of the new x if it is."""
         N, M_ = x.shape[0], x.shape[0] * self.top
         E, FP, Wp = self.up.shape
         logits = torch.empty((N, pad_to(E, 4)), device=x.device, dtype=torch.float32)[:, :E]
-        model.product(model.norm_rows(x, self.norm32), self.router, logits)
+        model.product(model.norm_rows(x, self.norm32) if h is None else h, self.router, logits)
         p = X.plan(*X.route(logits, self.top), E, model.dtype, FP * Wp, FP)
         h = model.norm_rows(x, self.norm32, where=p.where, scale=p.scale)
         a = torch.empty((M_, FP), device=x.device, dtype=model.dtype)
@@ -131,7 +136,13 @@ class ExpertsFf:
         W = self.down.shape[1]
         y = torch.empty((M_, pad_to(W, 8)), device=x.device, dtype=model.dtype)
         X.product(a, self.down, p, y[:, :W])
-        X.gather_sum(y, p, W, model.cfg.residual_mult, x)
+        cfg = model.cfg
+        if next_norm is None or model.dtype == torch.float32 or W != x.shape[1] or W > X.SUM_NORM_MAX:
+            X.gather_sum(y, p, W, cfg.residual_mult, x)
+            return None
+        h = torch.empty_like(x, dtype=model.dtype)
+        X.gather_sum_norm(y, p, W, cfg.residual_mult, x, next_norm, cfg.norm_offset, cfg.eps, cfg.layer_norm, h)
+        return h
 
     def decode(self, model, b, x: torch.Tensor) -> None:
         cfg = model.cfg

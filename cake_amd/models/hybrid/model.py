@@ -154,6 +154,20 @@ class HybridModel:
         else:
             G.linear(x, w, bias, epi="resid32", resid=y, alpha=alpha)
 
+    def add_norm(self, x, w, y, alpha: float, norm32, bias=None):
+        """:meth:`product_add`, and the norm of the new rows by norm32 where one launch does both (None: it
+        is left to what reads them): of few rows the product stops at its slabs and the norm sums them."""
+        W, cfg = w.shape[0], self.cfg
+        form = None if norm32 is None or self.dtype == torch.float32 or W != self.Wp or \
+            W > G.SLAB_NORM_MAX else G.slab_form(x.shape[0], W, x.shape[1], "resid32")
+        if form is None:
+            self.product_add(x, w, y, alpha, bias)
+            return None
+        h = torch.empty((x.shape[0], W), device=self.device, dtype=self.dtype)
+        G.slab_norm(*G.slabs(x, w, form), y, norm32, cfg.eps, h, bias=bias, alpha=alpha,
+                    offset=cfg.norm_offset, ln=cfg.layer_norm)
+        return h
+
     def product_act(self, x, w, out, act: str = "gelu", bias=None):
         """out = activation(x w^T + bias)."""
         if self.dtype == torch.float32:
@@ -174,11 +188,13 @@ class HybridModel:
         return self._part, self._ticket
 
     # ------------------------------------------------------------------ packed rows
-    def _layer_rows(self, run, x, rows: M.Rows, nsplit: int, observe) -> None:
+    def _layer_rows(self, run, x, h, rows: M.Rows, nsplit: int, observe, next_norm):
+        """One layer run of x; h: the norm of x if it is there.  Returns the norm by next_norm (None: of
+        no use) of the new x if it is there."""
         L, w = self.cfg.layers[run.layer], self.layers[run.layer]
         m, N, cfg = L.mixer, rows.N, self.cfg
         decode = rows.max_len == 1
-        h = self.norm_rows(x, w.norm32)
+        h = self.norm_rows(x, w.norm32) if h is None else h
         new = torch.empty if w.mix_cols == w.shape.out_cols and w.ff % 8 == 0 else torch.zeros
         mix = new((N, w.out_cols), device=self.device, dtype=self.dtype)
         # the mixers' decode kernels read f32 projections, as the fused step leaves them; a latent
@@ -216,11 +232,13 @@ class HybridModel:
                            **w.consts, state=a, ring=b, out=mix)
         else:
             M.delta_prompt(w.shape, proj, ab, rows, cfg.eps, **w.consts, state=a, ring=b, out=mix)
-        self.product_add(mix, w.w_out, x, cfg.residual_mult)
+        h = self.add_norm(mix, w.w_out, x, cfg.residual_mult,
+                          next_norm if w.post is None else w.post.norm32)
         if w.post is not None:
-            w.post.rows(self, x)
+            h = w.post.rows(self, x, h, next_norm)
         if observe is not None:
             observe(x[:, :self.W])
+        return h
 
     def _latent_rows(self, m: LatentMixer, w, proj, rows: M.Rows, cache, mix, nsplit: int) -> None:
         """Latent attention of projected rows into mix[:, :H vdim]."""
@@ -260,15 +278,19 @@ class HybridModel:
             if x0 is not None:
                 x0.copy_(x)
         nsplit = _splits(max(p0 + n for _, n, p0, _ in rows.host))
-        for run in self.runs:
+        h = None
+        for run, after in zip(self.runs, [*self.runs[1:], None]):
             if run.enter is not None:
                 pair = torch.empty((N, head.loop_in.shape[1]), device=self.device,
                                    dtype=self.dtype)
                 y = torch.empty_like(x)
                 M.loop_rows(x, x0, head.loop_step[run.enter], self.W, pair, y)
-                self.product_add(pair, head.loop_in, y, 1.0)
+                h = self.add_norm(pair, head.loop_in, y, 1.0, self.layers[run.layer].norm32)
                 x = y
-            self._layer_rows(run, x, rows, nsplit, observe)
+            # the last rows are gathered before their norm, an entered pass reads them as they are
+            next_norm = None if after is None or after.enter is not None else \
+                self.layers[after.layer].norm32
+            h = self._layer_rows(run, x, h, rows, nsplit, observe, next_norm)
         return x
 
     def _logits(self, x, take: list[int]) -> torch.Tensor:

@@ -223,6 +223,7 @@ _LIB_SIGS = {
         "cake_expert_route": [P, L, I, I, I, P, P, P],
         "cake_expert_plan": [P, P, I, I, I, I, I, I, P, P, P, I, P],
         "cake_expert_sum": [I, P, L, P, I, I, I, F, P, L, P],
+        "cake_expert_sum_norm": [I, P, L, P, I, I, I, F, P, L, P, F, F, I, P, L, P],
         "cake_expert_gemm32": [P, L, P, L, L, P, I, I, I, I, P, L, P],
         "cake_expert_up": [I, P, P, F, F, I, I, P, I, I, P, I, I, I, P, P, P],
         "cake_expert_down": [I, P, P, I, P, I, I, I, F, P, P, P],

@@ -13,6 +13,7 @@ from .mixers import ACTS, DT, _lib, _mat, _stream, _vec
 
 MAX_EXPERTS = 1024
 MAX_TOP = 32
+SUM_NORM_MAX = 8192   # columns of a row that gather_sum_norm holds
 BM32 = 32   # row tile of the f32 grouped product
 
 
@@ -95,6 +96,19 @@ def gather_sum(y, p: Plan, width: int, alpha: float, x):
     xp, ldx = _mat(x, "x", torch.float32, N, width)
     check(_lib().cake_expert_sum(DT[y.dtype], yp, ldy, p.where.data_ptr(), N, top, int(width),
                                  float(alpha), xp, max(ldx, width), _stream()), "expert_sum")
+
+
+def gather_sum_norm(y, p: Plan, width: int, alpha: float, x, w, offset: float, eps: float, ln: bool, out):
+    """:func:`gather_sum` of 16-bit rows up to 8192 wide (a multiple of 4), and out [N, width] = the norm
+    of the new rows (ln: layer norm) times (offset + w [width] f32)."""
+    N, top = p.where.shape
+    yp, ldy = _mat(y, "y", y.dtype, N * top, width)
+    xp, ldx = _mat(x, "x", torch.float32, N, width)
+    op, ldo = _mat(out, "out", y.dtype, N, width)
+    check(_lib().cake_expert_sum_norm(
+        DT[y.dtype], yp, ldy, p.where.data_ptr(), N, top, int(width), float(alpha), xp, max(ldx, width),
+        _vec(w, "w", torch.float32, width), float(offset), float(eps), int(ln), op, max(ldo, width), _stream()),
+        "expert_sum_norm")
 
 
 def up(resid, norm_w, eps: float, offset: float, ln: bool, width: int, logits, top: int, w,
