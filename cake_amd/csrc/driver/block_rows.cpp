@@ -5,6 +5,10 @@
 // allocations).  The caller checks and plans once per run, since every block has the same shapes;
 // what is left per launch is the kernel library's own entry point (2 - 3 us).
 //
+// Where the caller reads the last rows of the result only (a prompt's logits), the last block computes keys and
+// values of all rows, and what follows of those rows: no row reads another one's result there but through the
+// keys and values (6000 rows of an 8B block 2310 us, one of them 260).
+//
 // Of few rows the q/k/v, output and down products leave their sums in slabs, which the rotation and the next
 // norm add up: six launches a block instead of up to eleven (a block of 8B at 45 rows 122 us, 116 so).
 #include <hip/hip_runtime.h>
@@ -64,66 +68,110 @@ struct CakeBlockRun {
   float* rows_ws;               // workspace of the stream form
   void* tick;                   // counters of either
   Form qkv_form, o_form, gu_form, down_form;
+  Form kv_form, q1_form, o1_form, gu1_form, down1_form;   // of the last block, with a tail
   int n, dt, T, H, I, nh, nkv, hd, S, pos0;
+  int tail;                     // rows of the result that are wanted, the last ones (0: all)
   float eps, scale;
 };
 
+namespace {
+
+struct Run {
+  const CakeBlockRun* r;
+  hipStream_t st;
+  int nq = r->nh * r->hd, nk = r->nkv * r->hd, nqkv = nq + 2 * nk;
+  float* hidden = r->hidden;    // the rows at work: T of them from position pos0 on
+  uint16_t* x = static_cast<uint16_t*>(r->x);
+  uint16_t* qkv = static_cast<uint16_t*>(r->qkv);
+  int T = r->T, pos0 = r->pos0;
+
+  void only_last(int n) {
+    const size_t skip = T - n;
+    hidden += skip * r->H;
+    x += skip * r->H;
+    qkv += skip * nqkv;
+    pos0 += (int)skip;
+    T = n;
+  }
+  int product(const Form& f, int epi, const void* a, const void* w, void* c, long long ldc, int N, int K) const {
+    void* resid = epi == kEpiResid32 ? hidden : nullptr;
+    const long long ldr = resid ? N : 0;
+    return f.kind ? cake_gemm_rows(r->dt, epi, f.kind, a, K, w, K, c, ldc, nullptr, resid, ldr, r->rows_ws,
+                                   r->tick, r->zeros, T, N, K, 1.f, st)
+                  : cake_gemm_scaled(r->dt, epi, f.cfg, f.splits, a, K, w, K, c, ldc, nullptr, resid, ldr,
+                                     f.splits > 1 ? r->ws : nullptr, r->tick, r->zeros, T, N, K, 1.f, st);
+  }
+  // the product's slabs, their number (or minus an error)
+  int slabs(const Form& f, const void* a, const void* w, int N, int K) const {
+    return cake_gemm_slabs(r->dt, f.kind, f.cfg, f.splits, a, K, w, K, r->slabs, r->zeros, T, N, K, st);
+  }
+  // x = norm of the rows; one norm kernel at every place of a run
+  int norm(const void* ln, bool slab) const {
+    return slab ? cake_slab_norm(r->dt, nullptr, 0, hidden, r->H, nullptr, 1.f, ln, 0, 0.f, r->eps, 0, T, r->H, x,
+                                 r->H, st)
+                : cake_rmsnorm(r->dt, hidden, ln, r->eps, T, r->H, x, st);
+  }
+  // hidden += a w^T, and x = the norm of it by `ln` (null: none)
+  int add_norm(const Form& f, const void* a, const void* w, int K, const void* ln) const {
+    if (f.slabs) {
+      const int n = slabs(f, a, w, r->H, K);
+      return n < 0 ? -n : cake_slab_norm(r->dt, r->slabs, n, hidden, r->H, nullptr, 1.f, ln, 0, 0.f, r->eps, 0, T,
+                                         r->H, x, r->H, st);
+    }
+    const int e = product(f, kEpiResid32, a, w, nullptr, 0, r->H, K);
+    return e || !ln ? e : cake_rmsnorm(r->dt, hidden, ln, r->eps, T, r->H, x, st);
+  }
+  // rotated heads in qkv (q), keys and values in the cache
+  int project(const Block& b) const {
+    if (r->qkv_form.slabs) {
+      const int n = slabs(r->qkv_form, x, b.wqkv, nqkv, r->H);
+      return n < 0 ? -n : cake_slab_rope(r->dt, r->slabs, n, qkv, nqkv, T, r->nh, r->nkv, r->hd, r->inv_freq, pos0,
+                                         r->S, b.kc, b.vc, st);
+    }
+    const int e = product(r->qkv_form, kEpiStore, x, b.wqkv, qkv, nqkv, nqkv, r->H);
+    return e ? e : rope(b, r->nh, r->nkv);
+  }
+  int rope(const Block& b, int nh, int nkv) const {
+    return cake_rope_kv(r->dt, qkv, qkv + nq, qkv + nq + nk, nqkv, nqkv, T, nh, nkv, r->hd, r->inv_freq, pos0, r->S,
+                        b.kc, b.vc, st);
+  }
+  // the same, q of the last `tail` rows only, which are the rows at work from here on
+  int project_tail(const Block& b) {
+    const uint16_t* w = static_cast<const uint16_t*>(b.wqkv);
+    int e = product(r->kv_form, kEpiStore, x, w + (size_t)nq * r->H, qkv + nq, nqkv, 2 * nk, r->H);
+    if (!e) e = rope(b, 0, r->nkv);
+    only_last(r->tail);
+    if (!e) e = product(r->q1_form, kEpiStore, x, w, qkv, nqkv, nq, r->H);
+    return e ? e : rope(b, r->nh, 0);
+  }
+  int attend(const Block& b) const {
+    const long long Sh = (long long)r->S * r->hd, kv = r->nkv * Sh;
+    // [batch, head, row] strides of q (a column block of qkv), the cache twice, the output
+    const long long strides[12] = {(long long)T * nqkv, r->hd, nqkv, kv, Sh, r->hd, kv, Sh, r->hd,
+                                   (long long)T * nq, r->hd, nq};
+    return cake_flash_attn(r->dt, qkv, b.kc, b.vc, r->att, 1, r->nh, r->nkv, T, pos0 + T, r->hd, strides, r->scale,
+                           1, pos0, st);
+  }
+};
+
+}  // namespace
+
 // 0, or the HIP error of the first launch that failed (the blocks behind it are not launched)
 CAKE_API int cake_block_rows(const CakeBlockRun* r, hipStream_t st) {
-  if (!r || r->n < 0 || r->T < 1 || r->pos0 < 0 || r->pos0 + r->T > r->S)
+  if (!r || r->n < 0 || r->T < 1 || r->pos0 < 0 || r->pos0 + r->T > r->S || r->tail < 0 || r->tail > r->T)
     return (int)hipErrorInvalidValue;
-  const int T = r->T, H = r->H, nq = r->nh * r->hd, nk = r->nkv * r->hd, nqkv = nq + 2 * nk;
-  const long long Sh = (long long)r->S * r->hd;
-  // [batch, head, row] strides of q (a column block of qkv), the cache twice, the output
-  const long long strides[12] = {(long long)T * nqkv, r->hd, nqkv, r->nkv * Sh, Sh, r->hd,
-                                 r->nkv * Sh, Sh, r->hd, (long long)T * nq, r->hd, nq};
-  const auto product = [&](const Form& f, int epi, const void* a, const void* w, void* c, int N,
-                           int K) {
-    void* resid = epi == kEpiResid32 ? r->hidden : nullptr;
-    const long long ldr = resid ? N : 0, ldc = resid ? 0 : N;
-    return f.kind ? cake_gemm_rows(r->dt, epi, f.kind, a, K, w, K, c, ldc, nullptr, resid, ldr,
-                                   r->rows_ws, r->tick, r->zeros, T, N, K, 1.f, st)
-                  : cake_gemm_scaled(r->dt, epi, f.cfg, f.splits, a, K, w, K, c, ldc, nullptr,
-                                     resid, ldr, f.splits > 1 ? r->ws : nullptr, r->tick, r->zeros, T,
-                                     N, K, 1.f, st);
-  };
-  // the product's slabs, their number (or minus an error)
-  const auto slabs = [&](const Form& f, const void* a, const void* w, int N, int K) {
-    return cake_gemm_slabs(r->dt, f.kind, f.cfg, f.splits, a, K, w, K, r->slabs, r->zeros, T, N, K, st);
-  };
-  // hidden += a w^T, and x = the norm of it by `ln` (null: none)
-  const auto add_norm = [&](const Form& f, const void* a, const void* w, int K, const void* ln) {
-    if (f.slabs) {
-      const int n = slabs(f, a, w, H, K);
-      return n < 0 ? -n : cake_slab_norm(r->dt, r->slabs, n, r->hidden, H, nullptr, 1.f, ln, 0, 0.f, r->eps, 0, T, H,
-                                         r->x, H, st);
-    }
-    const int e = product(f, kEpiResid32, a, w, nullptr, H, K);
-    return e || !ln ? e : cake_rmsnorm(r->dt, r->hidden, ln, r->eps, T, H, r->x, st);
-  };
-  uint16_t* q = static_cast<uint16_t*>(r->qkv);
-  int e = r->n == 0 ? 0   // (one norm kernel at every place of the run)
-          : r->down_form.slabs ? cake_slab_norm(r->dt, nullptr, 0, r->hidden, H, nullptr, 1.f, r->blocks[0].ln1, 0,
-                                                0.f, r->eps, 0, T, H, r->x, H, st)
-                               : cake_rmsnorm(r->dt, r->hidden, r->blocks[0].ln1, r->eps, T, H, r->x, st);
+  Run g{r, st};
+  int e = r->n ? g.norm(r->blocks[0].ln1, r->down_form.slabs) : 0;
   for (int i = 0; !e && i < r->n; ++i) {
     const Block& b = r->blocks[i];
-    if (r->qkv_form.slabs) {
-      const int n = slabs(r->qkv_form, r->x, b.wqkv, nqkv, H);
-      e = n < 0 ? -n : cake_slab_rope(r->dt, r->slabs, n, q, nqkv, T, r->nh, r->nkv, r->hd, r->inv_freq, r->pos0,
-                                      r->S, b.kc, b.vc, st);
-    } else {
-      e = product(r->qkv_form, kEpiStore, r->x, b.wqkv, r->qkv, nqkv, H);
-      if (!e)
-        e = cake_rope_kv(r->dt, q, q + nq, q + nq + nk, nqkv, nqkv, T, r->nh, r->nkv, r->hd, r->inv_freq,
-                         r->pos0, r->S, b.kc, b.vc, st);
-    }
-    if (!e)
-      e = cake_flash_attn(r->dt, q, b.kc, b.vc, r->att, 1, r->nh, r->nkv, T, r->pos0 + T, r->hd,
-                          strides, r->scale, 1, r->pos0, st);
-    if (!e) e = add_norm(r->o_form, r->att, b.wo, nq, b.ln2);
-    if (!e) e = product(r->gu_form, kEpiSwiglu, r->x, b.wgu, r->act, r->I, H);
-    if (!e) e = add_norm(r->down_form, r->act, b.wd, r->I, i + 1 < r->n ? r->blocks[i + 1].ln1 : nullptr);
+    const bool last = i + 1 == r->n, tail = last && r->tail > 0;
+    const Form &o = tail ? r->o1_form : r->o_form, &gu = tail ? r->gu1_form : r->gu_form;
+    const Form& down = tail ? r->down1_form : r->down_form;
+    e = tail ? g.project_tail(b) : g.project(b);
+    if (!e) e = g.attend(b);
+    if (!e) e = g.add_norm(o, r->att, b.wo, g.nq, b.ln2);
+    if (!e) e = g.product(gu, kEpiSwiglu, g.x, b.wgu, r->act, r->I, r->I, r->H);
+    if (!e) e = g.add_norm(down, r->act, b.wd, r->I, last ? nullptr : r->blocks[i + 1].ln1);
   }
   return e;
 }

@@ -23,6 +23,7 @@ struct PrepArgs {
   const void* proj;      // [N][ldp] q | k | v | ... columns
   long long ldp;
   int N, H, G, dim, vdim, DP, DVP, S, rd2;  // rd2 = rotated pairs
+  int h0;                // the first head taken: 0, or H for the keys alone
   int qk_norm;
   float eps;
   const float2* cs;      // [positions][rd2] (cos, sin)
@@ -75,10 +76,10 @@ __global__ __launch_bounds__(256) void mixer_prep_kernel(PrepArgs a, int lph, in
   const int per = 256 / lph;  // (row, head) items per workgroup
   const int item = (blockIdx.x - nvb) * per + threadIdx.x / lph;
   const int l = threadIdx.x % lph, d0 = EPL * l;
-  const int nh = a.H + a.G;
+  const int nh = a.H + a.G - a.h0;
   const bool live = item < a.N * nh;  // lanes past the end shadow the last item
   const int it = live ? item : a.N * nh - 1;
-  const int n = it / nh, hh = it - n * nh;
+  const int n = it / nh, hh = it - n * nh + a.h0;
   const bool isq = hh < a.H;
   const int pos = a.row_pos[n];
   const E* src = reinterpret_cast<const E*>(a.proj) + (long long)n * a.ldp + (long long)hh * a.dim;
@@ -451,6 +452,7 @@ static bool mix_shape_ok(int H, int G, int dim, int vdim, int DP, int DVP, int S
          rd2 >= 0 && 2 * rd2 <= dim;
 }
 
+// (qn null: keys and values alone)
 CAKE_API int cake_mixer_prep(int dt, const void* proj, long long ldp, int N, int H, int G, int dim,
                              int vdim, int DP, int DVP, int S, int rd2, int qk_norm, float eps,
                              const void* cs, const int* row_pos, const int* row_slot, void* qn,
@@ -458,12 +460,13 @@ CAKE_API int cake_mixer_prep(int dt, const void* proj, long long ldp, int N, int
                              hipStream_t st) {
   if (!mix_shape_ok(H, G, dim, vdim, DP, DVP, S, rd2) || N < 0) return (int)hipErrorInvalidValue;
   if (N == 0) return 0;
-  PrepArgs a{proj, ldp, N, H, G, dim, vdim, DP, DVP, S, rd2, qk_norm, eps, (const float2*)cs,
+  const int h0 = qn ? 0 : H;
+  PrepArgs a{proj, ldp, N, H, G, dim, vdim, DP, DVP, S, rd2, h0, qk_norm, eps, (const float2*)cs,
              row_pos, row_slot, qn, kc, vc, k_slot, v_slot};
   int lph = 4;
   while (8 * lph < DP) lph <<= 1;  // <= 32
   const bool vec = dt != kF32 && dim % 8 == 0 && ldp % 8 == 0 && ((uintptr_t)proj % 16) == 0;
-  const long long items = (long long)N * (H + G);
+  const long long items = (long long)N * (H + G - h0);
   const int nvb = ((N + 63) / 64) * ((G * ((vdim + 7) / 8) + 3) / 4);
   const dim3 g((unsigned)(nvb + (items + 256 / lph - 1) / (256 / lph)));
   CAKE_MIX_DT(dt, {

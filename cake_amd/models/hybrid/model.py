@@ -37,6 +37,9 @@ SPLITS = ((256, 1), (1024, 8), (4096, 16), (1 << 30, 32))
 # the latent kernels' for the same buckets: a workgroup takes one 64-key tile while there are
 # splits for all of them
 LATENT_SPLITS = {n: min(M.MAX_SPLIT, -(-lim // 64)) for lim, n in SPLITS}
+# Rows of a step from which on the last run's unread ones are left out (:meth:`HybridModel._last_rows`);
+# fewer go through the products of few rows, which read the weights once either way
+LAST_LEAST = 65
 GEN_SLOT = 0  # the generator's own sequence
 
 
@@ -240,6 +243,70 @@ class HybridModel:
             observe(x[:, :self.W])
         return h
 
+    def _last_rows(self, run, x, h, rows: M.Rows, nsplit: int, sel) -> torch.Tensor:
+        """The last run of a prompt of which only the rows sel (one of a sequence at most) are read: all
+        rows leave keys and values or the state; what follows is that of one token per sequence, at the
+        place of its row.  Returns the wanted rows."""
+        L, w, cfg = self.cfg.layers[run.layer], self.layers[run.layer], self.cfg
+        m, N, n, dev = L.mixer, rows.N, sel.numel(), self.device
+        h = self.norm_rows(x, w.norm32) if h is None else h
+        x1, h1 = x.index_select(0, sel), h.index_select(0, sel)
+        pos, slot = rows.pos.index_select(0, sel), rows.slot.index_select(0, sel)
+        mix = torch.zeros((n, w.out_cols), device=dev, dtype=self.dtype)
+        up = mix[:, w.mix_cols:w.mix_cols + w.ff]
+        a, b = self.pool.bufs[run.index]
+        one = None   # the wanted rows' projections
+        if isinstance(m, AttentionMixer):
+            q, kv = w.shape.q_cols, w.shape.qkv_cols
+            q -= q % 8   # whole pieces of the rows
+            proj = torch.empty((N, M.pad_to(kv, 8)), device=dev, dtype=self.dtype)
+            self.product(h, w.w_in[q:kv], proj[:, q:kv])
+            M.attn_prep(w.shape, proj, rows, self._rotation(m), m.qk_norm, cfg.eps, None, a, b)
+            one = torch.empty((n, M.pad_to(w.n_raw, 8)), device=dev, dtype=torch.float32)[:, :w.n_raw]
+        if not (w.ff and one is not None and G.sections(h1, w.w_in, 0, w.n_raw, None, one, up)):
+            if w.ff:
+                self.product_act(h1, w.w_in[w.n_raw:], up)
+            if one is not None:
+                self.product(h1, w.w_in[:w.n_raw], one)
+        if isinstance(m, AttentionMixer):
+            # (not the steps' own: a captured step may run meanwhile)
+            part = torch.zeros(w.shape.part_floats(n, nsplit), device=dev, dtype=torch.float32)
+            ticket = torch.zeros(n * w.shape.tiles, device=dev, dtype=torch.int32)
+            M.attn_decode(w.shape, one, pos, slot, self._rotation(m), m.qk_norm, m.sink, m.gated,
+                          cfg.eps, m.scale, a, b, mix, nsplit, part, ticket)
+        elif isinstance(m, LatentMixer):
+            sh, c, cs, splits = w.shape, w.consts, self._rotation(m), LATENT_SPLITS[nsplit]
+            proj = torch.empty((N, w.n_main), device=dev, dtype=torch.float32)
+            self.product(h, w.w_in[:w.n_main], proj)
+            cq = torch.empty((N, sh.QP), device=dev, dtype=self.dtype)
+            LA.prep(sh, proj, rows, cs, cfg.eps, c["q_norm32"], c["kv_norm"], cq, a)
+            part = torch.zeros(sh.part_floats(n, splits), device=dev, dtype=torch.float32)
+            self._latent_tokens(m, w, cq.index_select(0, sel), pos, slot, a, mix, splits, part)
+        else:
+            proj = torch.empty((N, M.pad_to(w.n_main, 8)), device=dev, dtype=self.dtype)[:, :w.n_main]
+            ab = torch.empty((N, w.n_ab), device=dev, dtype=torch.float32)
+            self.product(h, w.w_in[:w.n_main], proj)
+            self.product(h, w.w_in[w.n_main:w.n_raw], ab)
+            out = torch.empty((N, w.mix_cols), device=dev, dtype=self.dtype)
+            M.delta_prompt(w.shape, proj, ab, rows, cfg.eps, **w.consts, state=a, ring=b, out=out)
+            cols = w.shape.out_cols
+            mix[:, :cols] = out[:, :cols].index_select(0, sel)
+        h1 = self.add_norm(mix, w.w_out, x1, cfg.residual_mult, None if w.post is None else w.post.norm32)
+        if w.post is not None:
+            w.post.rows(self, x1, h1)
+        return x1
+
+    def _latent_tokens(self, m: LatentMixer, w, cq, pos, slot, cache, mix, nsplit: int, part) -> None:
+        """Latent attention of one token per sequence, whose cache rows are there: cq [B, QP] their
+        normed query latents."""
+        sh, c, N = w.shape, w.consts, cq.shape[0]
+        q = torch.empty((N, sh.q_cols), device=self.device, dtype=torch.float32)
+        self.product(cq, c["uq"], q)
+        qa = torch.empty((N, sh.heads, sh.LD), device=self.device, dtype=self.dtype)
+        LA.absorb(sh, q, c["uk_t"], pos, slot, self._rotation(m), self.cfg.eps, c["kv_norm"], cache, qa)
+        LA.decode(sh, qa, pos, slot, cache, m.scale, nsplit, part)
+        LA.out(sh, part, pos, c["uv"], nsplit, mix)
+
     def _latent_rows(self, m: LatentMixer, w, proj, rows: M.Rows, cache, mix, nsplit: int) -> None:
         """Latent attention of projected rows into mix[:, :H vdim]."""
         sh, c, N, dev = w.shape, w.consts, rows.N, self.device
@@ -247,14 +314,8 @@ class HybridModel:
         cq = torch.empty((N, sh.QP), device=dev, dtype=self.dtype)
         LA.prep(sh, proj, rows, cs, self.cfg.eps, c["q_norm32"], c["kv_norm"], cq, cache)
         if rows.max_len == 1:   # on the latent rows themselves
-            q = torch.empty((N, sh.q_cols), device=dev, dtype=torch.float32)
-            self.product(cq, c["uq"], q)
-            qa = torch.empty((N, sh.heads, sh.LD), device=dev, dtype=self.dtype)
             part, _ = self._split_ws(N)
-            LA.absorb(sh, q, c["uk_t"], rows.pos, rows.slot, cs, self.cfg.eps, c["kv_norm"], cache,
-                      qa)
-            LA.decode(sh, qa, rows.pos, rows.slot, cache, m.scale, nsplit, part)
-            LA.out(sh, part, rows.pos, c["uv"], nsplit, mix)
+            self._latent_tokens(m, w, cq, rows.pos, rows.slot, cache, mix, nsplit, part)
             return
         q = torch.empty((N, sh.q_cols), device=dev, dtype=self.dtype)
         self.product(cq, c["uq"], q)
@@ -267,8 +328,8 @@ class HybridModel:
         self.product(c["uv"], lat, vt)
         LA.prompt(sh, q, k, vt, rows, cs, cache, mix, m.scale)
 
-    def _forward_rows(self, rows: M.Rows, observe=None) -> torch.Tensor:
-        """Residual rows [N, Wp] f32 after every layer run."""
+    def _forward_rows(self, rows: M.Rows, observe=None, sel=None) -> torch.Tensor:
+        """Residual rows [N, Wp] f32 after every layer run, of the rows sel alone if given."""
         N, head = rows.N, self.head
         x = torch.empty((N, self.Wp), device=self.device, dtype=torch.float32)
         x0 = torch.empty_like(x) if self.cfg.loop is not None else None
@@ -287,20 +348,28 @@ class HybridModel:
                 M.loop_rows(x, x0, head.loop_step[run.enter], self.W, pair, y)
                 h = self.add_norm(pair, head.loop_in, y, 1.0, self.layers[run.layer].norm32)
                 x = y
+            if after is None and sel is not None:
+                return self._last_rows(run, x, h, rows, nsplit, sel)
             # the last rows are gathered before their norm, an entered pass reads them as they are
             next_norm = None if after is None or after.enter is not None else \
                 self.layers[after.layer].norm32
             h = self._layer_rows(run, x, h, rows, nsplit, observe, next_norm)
         return x
 
-    def _logits(self, x, take: list[int]) -> torch.Tensor:
-        """Logits [len(take), V] f32 of the given residual rows."""
-        V = self.cfg.vocab_size
-        out = torch.empty((len(take), V), device=self.device, dtype=torch.float32)
-        if take:
-            sel = torch.tensor(take, dtype=torch.int32).to(self.device)
+    def _logits(self, x, sel) -> torch.Tensor:
+        """Logits [n, V] f32 of the residual rows sel [n] (None: of all)."""
+        n = x.shape[0] if sel is None else sel.numel()
+        out = torch.empty((n, self.cfg.vocab_size), device=self.device, dtype=torch.float32)
+        if n:
             self.product(self.norm_rows(x, self.head.norm32, rows=sel), self.head.lm_head, out)
         return out
+
+    def _reads_few(self, rows: M.Rows, entries, observe) -> bool:
+        """Whether the last run's results are read at few rows, one of a sequence (:meth:`_last_rows`)."""
+        n = sum(len(e.want) for e in entries)
+        return observe is None and self.dtype != torch.float32 and rows.max_len > 1 and \
+            rows.N >= LAST_LEAST and 0 < n <= min(G.ROWS_MAX, rows.N // 4) and \
+            all(len(e.want) <= 1 for e in entries)
 
     # ------------------------------------------------------------------ steps
     def open_sequence(self) -> int:
@@ -335,11 +404,16 @@ class HybridModel:
             self.decode_embed(b)
             with self.decode_eager(pos):
                 x = self.decode_layers(b, range(len(self.runs)))
-            return [self._logits(x.view(1, -1), [0] * len(entries[0].want))]
+            sel = torch.zeros(len(entries[0].want), dtype=torch.int32, device=self.device)
+            return [self._logits(x.view(1, -1), sel)]
         rows = M.Rows.pack(seqs, self.device)
-        x = self._forward_rows(rows, observe)
         take = [h[0] + w for h, e in zip(rows.host, entries) for w in e.want]
-        return list(self._logits(x, take).split([len(e.want) for e in entries]))
+        sel = torch.tensor(take, dtype=torch.int32).to(self.device)
+        if self._reads_few(rows, entries, observe):
+            logits = self._logits(self._forward_rows(rows, None, sel), None)
+        else:
+            logits = self._logits(self._forward_rows(rows, observe), sel)
+        return list(logits.split([len(e.want) for e in entries]))
 
     # ------------------------------------------------------------------ generator interface
     def reset(self) -> None:

@@ -144,8 +144,9 @@ class LayerStack:
 
     # ------------------------------------------------------------------ forward
     def forward(self, hidden: torch.Tensor, layers: list[int], pos0: int,
-                session: int = 0) -> torch.Tensor:
-        """Run `layers` (in order) over hidden [T, H] f32 at positions pos0.., in place."""
+                session: int = 0, tail: int = 0) -> torch.Tensor:
+        """Run `layers` (in order) over hidden [T, H] f32 at positions pos0.., in place.  tail: only
+        so many of the last rows of the result are wanted (0: all), the others may hold anything."""
         if hidden.dtype != torch.float32 or hidden.dim() != 2:
             raise ValueError("hidden must be f32 [T, H]")
         T = hidden.shape[0]
@@ -160,7 +161,7 @@ class LayerStack:
             from ...ops.llama_rows import block_rows
             if block_rows(hidden, [self.weights[li] for li in layers],
                           [self.slot_of[li] for li in layers], kv.k, kv.v, self.inv_freq, self.cfg,
-                          pos0, self.scale):
+                          pos0, self.scale, tail):
                 kv.length = max(kv.length, pos0 + T)
                 return hidden
         for li in layers:

@@ -83,10 +83,12 @@ class LlamaModel:
             return out
         return self.head.embed[ids.long()].float()
 
-    def forward_hidden(self, hidden: torch.Tensor, pos0: int) -> torch.Tensor:
-        for run in self.runs:
+    def forward_hidden(self, hidden: torch.Tensor, pos0: int, tail: int = 0) -> torch.Tensor:
+        """Hidden rows after all layers; tail: of so many of the last ones (0: all)."""
+        for i, run in enumerate(self.runs):
             if run.local:
-                self.stack.forward(hidden, run.layers, pos0, self.session)
+                self.stack.forward(hidden, run.layers, pos0, self.session,
+                                   tail if i + 1 == len(self.runs) else 0)
             else:
                 batch = [(layer_name(li), pos0, li) for li in run.layers]
                 hidden = run.forwarder.forward_batch(hidden, batch, self.session)
@@ -110,7 +112,7 @@ class LlamaModel:
     def forward(self, tokens: list[int], pos0: int) -> torch.Tensor:
         """Logits (f32 [V]) of the last of `tokens`, fed at positions pos0.."""
         h = self.embed(tokens)
-        h = self.forward_hidden(h, pos0)
+        h = self.forward_hidden(h, pos0, tail=1)
         return self.head_logits(h[-1])
 
     def reset(self) -> None:
@@ -189,7 +191,7 @@ class LlamaModel:
     def prefill_logits(self, prompt: list[int], out: torch.Tensor) -> None:
         """The whole prompt from position 0; logits of its last token into `out`."""
         self.stack.reset(self.session)
-        h = self.forward_hidden(self.embed(prompt), 0)
+        h = self.forward_hidden(self.embed(prompt), 0, tail=1)
         self.head_logits(h[-1], out=out)
 
     # ------------------------------------------------------------------ ragged steps
@@ -213,7 +215,8 @@ class LlamaModel:
             pos = self._seq_pos[e.seq]
             keep, self.session = self.session, e.seq
             try:
-                h = self.forward_hidden(self.embed(e.tokens), pos)
+                T = len(e.tokens)
+                h = self.forward_hidden(self.embed(e.tokens), pos, tail=T - min(e.want, default=T - 1))
             finally:
                 self.session = keep
             self._seq_pos[e.seq] = pos + len(e.tokens)

@@ -22,17 +22,18 @@ class _Form(C.Structure):
 class _Run(C.Structure):
     _fields_ = [(n, P) for n in ("blocks", "hidden", "x", "qkv", "att", "act", "inv_freq", "zeros",
                                  "ws", "slabs", "rows_ws", "tick")] + \
-               [(n, _Form) for n in ("qkv_form", "o_form", "gu_form", "down_form")] + \
-               [(n, I) for n in ("n", "dt", "T", "H", "I", "nh", "nkv", "hd", "S", "pos0")] + \
+               [(n, _Form) for n in ("qkv_form", "o_form", "gu_form", "down_form", "kv_form", "q1_form",
+                                     "o1_form", "gu1_form", "down1_form")] + \
+               [(n, I) for n in ("n", "dt", "T", "H", "I", "nh", "nkv", "hd", "S", "pos0", "tail")] + \
                [("eps", F), ("scale", F)]
 
 
-def _forms(T: int, products, capturing: bool):
-    """(kind, cfg, splits) of each (Nv, K, epi), as gemm.linear chooses them or, of those that a sum of
-    slabs may follow, as gemm.slab_form does; the floats that the tile plans' slabs need, and those of
-    the products that leave them.  None if one of them is the library GEMM's."""
+def _forms(products, capturing: bool):
+    """(kind, cfg, splits) of each (rows, Nv, K, epi, summed), as gemm.linear chooses them or, of those
+    that a sum of slabs may follow, as gemm.slab_form does; the floats that the tile plans' slabs need,
+    and those of the products that leave them.  None if one of them is the library GEMM's."""
     forms, floats, left = [], 0, 0
-    for Nv, K, epi, summed in products:
+    for T, Nv, K, epi, summed in products:
         gated = epi == "swiglu"
         big = max(T, Nv) * K * 2 >= 0x7fffffff
         slab = G.slab_form(T, Nv, K, epi, big) if summed else None
@@ -55,10 +56,18 @@ def _forms(T: int, products, capturing: bool):
     return forms, floats, left
 
 
+# A prompt of fewer rows goes through the last block whole: its products read the weights once either way
+# and the one row's are a launch more (nine blocks of 1B / 8B / 70B, whole and with one row at the end: 45
+# rows 540 / 978 / 2700 us, 544 / 984 / 2699; 80 rows 645 / 1240 / 3328, 642 / 1233 / 3271; 512 rows 1111 /
+# 2496 / 7538, 1071 / 2354 / 7023).
+TAIL_LEAST = 65
+
+
 def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Tensor,
-               v: torch.Tensor, inv_freq: torch.Tensor, cfg, pos0: int, scale: float) -> bool:
+               v: torch.Tensor, inv_freq: torch.Tensor, cfg, pos0: int, scale: float,
+               tail: int = 0) -> bool:
     """hidden [T, H] f32 through `blocks` in place; k, v [layers, nkv, S, hd], block i's rows at
-    slots[i]."""
+    slots[i].  tail: only so many of the last rows of the result are wanted (0: all)."""
     T, H = hidden.shape
     nh, nkv, hd = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
     inter, S, dt = cfg.intermediate_size, k.shape[2], k.dtype
@@ -86,11 +95,19 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
         table[8 * i:8 * i + 8] = [*ptrs, kp + s * step, vp + s * step]
     capturing = torch.cuda.is_current_stream_capturing()
     adds = H <= G.SLAB_NORM_MAX
-    forms, floats, left = _forms(T, ((nqkv, H, "store", True), (H, nq, "resid32", adds),
-                                     (2 * inter, H, "swiglu", False), (H, inter, "resid32", adds)),
-                                 capturing)
+    nk = nkv * hd
+    if T < TAIL_LEAST or tail * 4 > T or not blocks:
+        tail = 0
+
+    def behind(rows):   # the products behind the attention
+        return ((rows, H, nq, "resid32", adds), (rows, 2 * inter, H, "swiglu", False),
+                (rows, H, inter, "resid32", adds))
+    forms, floats, left = _forms(((T, nqkv, H, "store", True), *behind(T)) + (() if not tail else (
+        (T, 2 * nk, H, "store", False), (tail, nq, H, "store", False), *behind(tail))), capturing)
     if forms is None:
         return False
+    if not tail:
+        forms += [_Form()] * 5
     dev, st = hidden.device, current_stream()
     x = torch.empty((T, H), device=dev, dtype=dt)
     qkv = torch.empty((T, nqkv), device=dev, dtype=dt)
@@ -100,12 +117,12 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
     slabs = torch.empty(left, device=dev, dtype=torch.float32) if left else None
     rows_ws = tick = None
     if any(f.kind == 2 and not f.slabs for f in forms):
-        rows_ws, tick = G._rows_state(dev, T, st)
+        rows_ws, tick = G._rows_state(dev, min(T, G.ROWS_MAX), st)
     elif any(f.splits > 1 and f.cfg in G.FOUR_WAVE and not f.slabs for f in forms):
         tick = G._counters(dev, st)
     ptr = [None if t is None else t.data_ptr() for t in (
         hidden, x, qkv, att, act, inv_freq, G._zeros16(dev), ws, slabs, rows_ws, tick)]
     run = _Run(C.addressof(table), *ptr, *forms, len(blocks), G._DT[dt], T, H, inter, nh, nkv, hd, S,
-               int(pos0), float(cfg.rms_norm_eps), float(scale))
+               int(pos0), int(tail), float(cfg.rms_norm_eps), float(scale))
     check(kernels().cake_block_rows(C.addressof(run), st), "block_rows")
     return True

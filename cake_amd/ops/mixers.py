@@ -259,7 +259,8 @@ def _check_rows(rows: Rows, S: int, slots: int):
 
 
 def attn_prep(sh: AttnShape, proj, rows: Rows, cs, qk_norm: bool, eps: float, qn, kc, vc):
-    """Rotate / normalise q (-> qn [N, H, DP]) and k, v (-> cache) of packed prompt rows."""
+    """Rotate / normalise q (-> qn [N, H, DP]; None: q is left) and k, v (-> cache) of packed prompt
+    rows."""
     S, slots = _cache(sh, kc, vc, proj.dtype)
     _check_rows(rows, S, slots)
     pp, ldp = _mat(proj, "proj", proj.dtype, rows.N, sh.qkv_cols)
@@ -269,6 +270,7 @@ def attn_prep(sh: AttnShape, proj, rows: Rows, cs, qk_norm: bool, eps: float, qn
                                  sh.vdim, sh.DP, sh.DVP, S, sh.rot_pairs, int(qk_norm), float(eps),
                                  _vec(cs, "cs", torch.float32), rows.pos.data_ptr(),
                                  rows.slot.data_ptr(),
+                                 None if qn is None else
                                  _vec(qn, "qn", proj.dtype, rows.N * sh.heads * sh.DP),
                                  kc.data_ptr(), vc.data_ptr(), kc.stride(0), vc.stride(0),
                                  _stream()), "mixer_prep")
