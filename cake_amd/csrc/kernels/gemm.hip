@@ -224,6 +224,13 @@ static constexpr TileCost kTileCosts[] = {
     {33, 224, 192, 1, 0.846f, 0.777f, 0.0146f, -0.0934f, 0.144f, {10.04f, 12.63f, 8.565f, 13.22f, -1.f, -1.f, -1.f}, 0.812f, 3.47f},
     {34, 192, 256, 1, 1.768f, 0.979f, 0.0472f, 0.0879f, 0.126f, {6.113f, 10.06f, 6.451f, 13.14f, -1.f, -1.f, -1.f}, 2.423f, 4.585f},
     {35, 224, 256, 1, 1.053f, 1.076f, 0.045f, 0.148f, 0.113f, {7.659f, 11.94f, 7.822f, 13.64f, -1.f, -1.f, -1.f}, 6.25f, 4.798f},
+    // between 160 and 256 rows a tile the next larger one is padding and the next smaller one a partial wave
+    // more: of 2,275 products these are taken for a twelfth, 8 % faster each (SwiGLU of 777 x 28672 x 4096 172
+    // us on 192 x 192, 162 on 160 x 192; 777 x 4096 x 14336 98 in three pieces of 160 x 256, 93 in two of 224 x
+    // 128; 1100 x 6144 x 4096 57.6, 51.9).  Their estimates carry 1 or 2 % for the fit's own error.
+    {36, 160, 192, 1, 1.492f, 0.68f, 0.019f, 0.f, 0.162f, {6.568f, 8.877f, 5.377f, 9.642f, -1.f, -1.f, -1.f}, 3.255f, 2.515f},
+    {37, 160, 128, 1, 0.744f, 0.511f, 0.032f, 0.f, 0.163f, {5.184f, 7.988f, 4.123f, 7.683f, -1.f, -1.f, -1.f}, 3.312f, 3.9f},
+    {38, 224, 128, 1, 0.259f, 0.64f, 0.017f, 0.f, 0.162f, {6.65f, 10.33f, 5.431f, 11.4f, -1.f, -1.f, -1.f}, 1.852f, 3.237f},
     // products of image models: the classes from kImageClass on
     {4, 64, 64, 4, 1.48f, 0.787f, 0.f, 0.263f, 0.f, {-1.f, -1.f, -1.f, -1.f, 3.44f, 2.92f, 3.04f}, -1.f, 0.f},
     {5, 256, 256, 1, 0.69f, 1.43f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 11.7f, 9.55f, 8.55f}, 4.16f, 0.304f},

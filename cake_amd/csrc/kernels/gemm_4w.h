@@ -1,4 +1,4 @@
-// Four-wave MFMA GEMM tiles (plan cfg 22-35; shapes and schedules below): the projections of
+// Four-wave MFMA GEMM tiles (plan cfg 22-38; shapes and schedules below): the projections of
 // prompts.
 //
 // Included by gemm_kernel.h (launch_gemm dispatches them here); same GemmArgs, tile
@@ -45,7 +45,7 @@ constexpr int k4WCfg192 = 23;  // 256 x 192 (8B q|k|v: 6144 = 32 x 192 columns, 
                                // 2048 tokens instead of 192)
 constexpr int k4WCfg128 = 24;  // 128 x 256 (8B o / down at 2048 tokens: 256 tiles, not 128)
 constexpr int k4WSched = 3;    // cfg + 3: the same tiles on three barriers (25, 26), on one (27)
-constexpr int k4WLast = 35;    // 28 .. 35: the tiles of CAKE_GEMM_4W_TILES
+constexpr int k4WLast = 38;    // 28 .. 38: the tiles of CAKE_GEMM_4W_TILES
 inline bool four_wave_cfg(int cfg) { return cfg >= k4WCfg && cfg <= k4WLast; }
 // op k of an alternating sequence of nr reads and nd DMAs (the longer list's tail last):
 // kind 0 = read, 1 = DMA, and its index within its list

@@ -1048,7 +1048,10 @@ __global__ __launch_bounds__(256) void gemm_splitk_finalize(GemmArgs g, int spli
   X(32, 192, 192, 2, 2, 2)    \
   X(33, 224, 192, 2, 2, 2)    \
   X(34, 192, 256, 2, 2, 1)    \
-  X(35, 224, 256, 2, 2, 1)
+  X(35, 224, 256, 2, 2, 1)    \
+  X(36, 160, 192, 2, 2, 2)    \
+  X(37, 160, 128, 2, 2, 2)    \
+  X(38, 224, 128, 2, 2, 2)
 
 }  // namespace cake
 

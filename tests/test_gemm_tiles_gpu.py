@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 
 # one k step up to more than a buffer holds; rows and columns one off the tile's edge; in pieces
-@pytest.mark.parametrize("cfg", range(27, 36))
+@pytest.mark.parametrize("cfg", range(27, 39))
 @pytest.mark.parametrize("rows,cols,K,splits", [(-1, 1, 64, 1), (1, -3, 192, 1), (0, 0, 320, 1), (3, 5, 1088, 4)])
 @pytest.mark.parametrize("epi", ["store", "resid32", "swiglu"])
 def test_tile_edges(cuda, cfg, rows, cols, K, splits, epi):
@@ -35,7 +35,7 @@ def test_tile_edges(cuda, cfg, rows, cols, K, splits, epi):
 
 # the other type and the other epilogues that plans take: whole tiles and pieces, ragged edges
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
-@pytest.mark.parametrize("cfg", range(27, 36))
+@pytest.mark.parametrize("cfg", range(27, 39))
 @pytest.mark.parametrize("K,splits", [(192, 1), (1088, 4)])
 @pytest.mark.parametrize("epi", ["store", "swiglu", "store32", "silu", "quick_gelu", "gelu", "relu2"])
 def test_types_and_epilogues(cuda, dt, cfg, K, splits, epi):
@@ -63,7 +63,7 @@ def test_types_and_epilogues(cuda, dt, cfg, K, splits, epi):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
-@pytest.mark.parametrize("cfg", range(28, 36))
+@pytest.mark.parametrize("cfg", range(28, 39))
 @pytest.mark.parametrize("epi", ["add16", "geglu"])
 def test_image_epilogues_run_on_another_tile(cuda, dt, cfg, epi):
     """Tiles without these epilogues: the call's result is the 128 x 256 tile's, pieces or none."""
