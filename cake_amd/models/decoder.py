@@ -11,6 +11,8 @@ import os
 
 import torch
 
+from ..ops._lib import upload
+
 
 class DeviceDecoder:
     """Whole-step hipGraph decoder for an all-local model on the HIP backend.
@@ -187,8 +189,7 @@ class DeviceDecoder:
         if T + 1 > m.max_seq:
             raise ValueError("prompt longer than max_seq")
         m.prefill_logits(prompt, b.logits)
-        ids = torch.tensor(prompt, dtype=torch.int32)
-        b.hist[:T].copy_(ids.to(m.device))
+        b.hist[:T].copy_(upload(prompt, torch.int32, m.device))
         b.hist_len.fill_(T)
         b.pos.fill_(T - 1)
         b.slot.zero_()

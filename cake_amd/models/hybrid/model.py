@@ -27,6 +27,7 @@ import torch
 from ...ops import gemm as G
 from ...ops import latent as LA
 from ...ops import mixers as M
+from ...ops._lib import upload
 from ..base import StepEntry
 from .config import AttentionMixer, HybridConfig, LatentMixer, from_path
 from .state import StatePool
@@ -408,7 +409,7 @@ class HybridModel:
             return [self._logits(x.view(1, -1), sel)]
         rows = M.Rows.pack(seqs, self.device)
         take = [h[0] + w for h, e in zip(rows.host, entries) for w in e.want]
-        sel = torch.tensor(take, dtype=torch.int32).to(self.device)
+        sel = upload(take, torch.int32, self.device)
         if self._reads_few(rows, entries, observe):
             logits = self._logits(self._forward_rows(rows, None, sel), None)
         else:

@@ -20,6 +20,7 @@ from functools import partial
 import torch
 
 from ...ops import reference as R
+from ...ops._lib import upload
 from ..base import StepEntry
 from ..decoder import DeviceDecoder  # noqa: F401  (the all-local decoder of this family)
 from .blocks import DecodeBuffers, LayerStack
@@ -74,7 +75,7 @@ class LlamaModel:
 
     # ------------------------------------------------------------------ generic path
     def embed(self, tokens: list[int]) -> torch.Tensor:
-        ids = torch.tensor(tokens, dtype=torch.int32, device=self.device)
+        ids = upload(tokens, torch.int32, self.device)
         if self.backend == "hip":
             from ...ops import hip as K
             out = torch.empty((len(tokens), self.cfg.hidden_size), device=self.device,

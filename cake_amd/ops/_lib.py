@@ -154,6 +154,17 @@ def available() -> bool:
         return False
 
 
+def upload(values, dtype, device):
+    """Host numbers as a tensor of the device, through pinned memory: the copy is ordered on the current
+    stream and the host does not wait for it (a copy from pageable memory waits for all that the stream
+    still has to do, and the launches behind it then find the GPU idle)."""
+    import torch
+    device = torch.device(device)
+    if device.type != "cuda":
+        return torch.tensor(values, dtype=dtype, device=device)
+    return torch.tensor(values, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
+
+
 def check(rc: int, name: str) -> None:
     if rc != 0:
         raise KernelError(f"{name} failed with hipError {rc}")

@@ -11,7 +11,7 @@ from dataclasses import dataclass
 
 import torch
 
-from ._lib import check, library
+from ._lib import check, library, upload
 from ._lib import current_stream as _stream
 
 DT = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
@@ -94,7 +94,7 @@ class Rows:
         for p in parts:
             at.append(len(flat))
             flat += p + [0] * (-len(p) % 4)
-        flat = torch.tensor(flat, dtype=torch.int32).to(device)
+        flat = upload(flat, torch.int32, device)
         tok, pos, slot, first, chunk0, key0, seq, chunk = (flat[a:a + len(p)] for a, p in zip(at, parts))
         return cls(N, B, max(h[1] for h in host), tok, pos, slot, first, seq.view(B, 4),
                    chunk.view(-1, 2), chunk0, key0, n_keys, host)
