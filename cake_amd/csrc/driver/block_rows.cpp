@@ -10,7 +10,8 @@
 // keys and values (6000 rows of an 8B block 2310 us, one of them 260).
 //
 // Of few rows the q/k/v, output and down products leave their sums in slabs, which the rotation and the next
-// norm add up: six launches a block instead of up to eleven (a block of 8B at 45 rows 122 us, 116 so).
+// norm add up (a block of 8B at 45 rows 122 us, 116 so); of a prompt's first rows the rotation and the attention
+// are one launch too: seven a block instead of up to eleven.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -40,6 +41,8 @@ int cake_slab_norm(int dt, const float* ws, int slabs, float* x, long long ldx, 
                    hipStream_t st);
 int cake_slab_rope(int dt, const float* ws, int slabs, void* q, int ldq, int T, int nh, int nkv, int hd,
                    const float* inv_freq, int pos0, int S, void* kc, void* vc, hipStream_t st);
+int cake_slab_attn(int dt, const float* ws, int slabs, void* out, long long ldo, int T, int nh, int nkv, int hd,
+                   const float* inv_freq, int S, void* kc, void* vc, float scale, hipStream_t st);
 }
 
 namespace {
@@ -144,6 +147,15 @@ struct Run {
     if (!e) e = product(r->q1_form, kEpiStore, x, w, qkv, nqkv, nq, r->H);
     return e ? e : rope(b, r->nh, 0);
   }
+  // a short prompt's: projections left in slabs, rotation and attention in one launch
+  bool short_prompt() const {
+    return r->qkv_form.slabs && pos0 == 0 && T <= 64 && (r->hd == 64 || r->hd == 128);
+  }
+  int project_attend(const Block& b) const {
+    const int n = slabs(r->qkv_form, x, b.wqkv, nqkv, r->H);
+    return n < 0 ? -n : cake_slab_attn(r->dt, r->slabs, n, r->att, nq, T, r->nh, r->nkv, r->hd, r->inv_freq, r->S,
+                                       b.kc, b.vc, r->scale, st);
+  }
   int attend(const Block& b) const {
     const long long Sh = (long long)r->S * r->hd, kv = r->nkv * Sh;
     // [batch, head, row] strides of q (a column block of qkv), the cache twice, the output
@@ -167,8 +179,12 @@ CAKE_API int cake_block_rows(const CakeBlockRun* r, hipStream_t st) {
     const bool last = i + 1 == r->n, tail = last && r->tail > 0;
     const Form &o = tail ? r->o1_form : r->o_form, &gu = tail ? r->gu1_form : r->gu_form;
     const Form& down = tail ? r->down1_form : r->down_form;
-    e = tail ? g.project_tail(b) : g.project(b);
-    if (!e) e = g.attend(b);
+    if (!tail && g.short_prompt()) {
+      e = g.project_attend(b);
+    } else {
+      e = tail ? g.project_tail(b) : g.project(b);
+      if (!e) e = g.attend(b);
+    }
     if (!e) e = g.add_norm(o, r->att, b.wo, g.nq, b.ln2);
     if (!e) e = g.product(gu, kEpiSwiglu, g.x, b.wgu, r->act, r->I, r->I, r->H);
     if (!e) e = g.add_norm(down, r->act, b.wd, r->I, last ? nullptr : r->blocks[i + 1].ln1);

@@ -2,7 +2,8 @@
 // row's slabs goes straight into the work that reads the row next.
 //
 //   cake_slab_norm  x += alpha (sum + bias), and the norm of the new row (or the sum alone, or the norm);
-//   cake_slab_rope  q, k, v rows of a Llama block: rotation, keys and values into the cache.
+//   cake_slab_rope  q, k, v rows of a Llama block: rotation, keys and values into the cache;
+//   cake_slab_attn  the same and the rows' causal attention, for a short prompt from position 0.
 //
 // Of few rows a launch is its round trips to the memory, whatever it reads: the sum of eight slabs of 45
 // rows of 4096 (4.2 us) and the norm behind it (4.0) are one launch here, and neither a strip's parts in the
@@ -155,6 +156,166 @@ __global__ __launch_bounds__(256) void slab_rope_kernel(SlabRopeArgs a) {
   *reinterpret_cast<uint2*>(dst + i0 + half) = make_uint2(oh[0] | (uint32_t)oh[1] << 16, oh[2] | (uint32_t)oh[3] << 16);
 }
 
+struct SlabAttnArgs {
+  SlabRopeArgs r;        // (q, ldq unused)
+  uint16_t* out;         // [T][ldo]
+  long long ldo;
+  int T;
+  float scale_log2;
+};
+
+// Short prompts from position 0 (T <= 64): every key is one of these rows, so a workgroup of a query head sums
+// and rotates its q, k and v, keeps them in LDS and runs the attention at once.  Bound by a launch's round trips:
+// rotation and attention as two launches 9.2 us at 5 rows of 16 heads and 10.8 at 45 of 32, of which the
+// attention's 6 read back what the rotation had written.  The heads that share a key head sum its rows each.
+//
+// S^T = K Q^T with the keys of a 32-key group dealt to the two 16-row tiles so that a lane's scores are eight
+// keys in a row: they are the second operand of O^T = V^T P^T as they are.
+template <int DT, int HD, int SL>
+__global__ __launch_bounds__(512) void slab_attn_kernel(SlabAttnArgs b) {
+  constexpr int LQ = HD + 8, LV = 64 + 8, HV = HD / 8, NKS = HD / 32, NT = HD / 32;
+  __shared__ __attribute__((aligned(16))) uint16_t qs[64 * LQ], ks[64 * LQ], vt[HD * LV];
+  const SlabRopeArgs& a = b.r;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
+  const int h = blockIdx.x, rep = a.nh / a.nkv, kv = h / rep;
+  const bool writes = h % rep == 0;
+  const int cols = (a.nh + 2 * a.nkv) * HD;
+  const int head[3] = {h, a.nh + kv, a.nh + a.nkv + kv};
+
+  // ---- q, k, v: an item is four columns of both halves of a row's three heads ----
+  for (int p = tid; p < b.T * HV; p += 512) {
+    const int t = p / HV, i0 = (p - t * HV) * 4;
+    float4 x[3][2];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) x[n][0] = x[n][1] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float* row = a.ws + (size_t)t * cols + i0;
+    for (int s0 = 0; s0 < a.slabs; s0 += SL) {
+      float4 y[SL][3][2];
+#pragma unroll
+      for (int e = 0; e < SL; ++e)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+          const float* r = row + min(s0 + e, a.slabs - 1) * a.slab + head[n] * HD;
+          y[e][n][0] = *reinterpret_cast<const float4*>(r);
+          y[e][n][1] = *reinterpret_cast<const float4*>(r + HD / 2);
+        }
+#pragma unroll
+      for (int e = 0; e < SL; ++e)
+        if (s0 + e < a.slabs)
+#pragma unroll
+          for (int n = 0; n < 3; ++n)
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+              x[n][d].x += y[e][n][d].x; x[n][d].y += y[e][n][d].y;
+              x[n][d].z += y[e][n][d].z; x[n][d].w += y[e][n][d].w;
+            }
+    }
+    float c[4], s[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sincosf((float)t * a.inv_freq[i0 + e], &s[e], &c[e]);
+    uint2 w[3][2];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const float lo[4] = {x[n][0].x, x[n][0].y, x[n][0].z, x[n][0].w};
+      const float hi[4] = {x[n][1].x, x[n][1].y, x[n][1].z, x[n][1].w};
+      uint16_t ol[4], oh[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ol[e] = from_f32<DT>(n < 2 ? lo[e] * c[e] - hi[e] * s[e] : lo[e]);
+        oh[e] = from_f32<DT>(n < 2 ? lo[e] * s[e] + hi[e] * c[e] : hi[e]);
+        if (n == 2) {
+          vt[(i0 + e) * LV + t] = ol[e];
+          vt[(i0 + HD / 2 + e) * LV + t] = oh[e];
+        }
+      }
+      w[n][0] = make_uint2(ol[0] | (uint32_t)ol[1] << 16, ol[2] | (uint32_t)ol[3] << 16);
+      w[n][1] = make_uint2(oh[0] | (uint32_t)oh[1] << 16, oh[2] | (uint32_t)oh[3] << 16);
+    }
+    *reinterpret_cast<uint2*>(qs + t * LQ + i0) = w[0][0];
+    *reinterpret_cast<uint2*>(qs + t * LQ + i0 + HD / 2) = w[0][1];
+    *reinterpret_cast<uint2*>(ks + t * LQ + i0) = w[1][0];
+    *reinterpret_cast<uint2*>(ks + t * LQ + i0 + HD / 2) = w[1][1];
+    if (writes) {
+      uint16_t* kr = a.kc + ((size_t)kv * a.S + t) * HD + i0;
+      uint16_t* vr = a.vc + ((size_t)kv * a.S + t) * HD + i0;
+      *reinterpret_cast<uint2*>(kr) = w[1][0];
+      *reinterpret_cast<uint2*>(kr + HD / 2) = w[1][1];
+      *reinterpret_cast<uint2*>(vr) = w[2][0];
+      *reinterpret_cast<uint2*>(vr + HD / 2) = w[2][1];
+    }
+  }
+  // values past the rows meet probabilities of zero
+  const int pad = 64 - b.T;
+  for (int p = tid; p < HD * pad; p += 512) vt[p / pad * LV + b.T + p % pad] = 0;
+  __syncthreads();
+
+  // ---- a wave: 16 query rows, half of the value columns ----
+  const int q0 = (wave & 3) * 16, qi = q0 + l15, t0 = (wave >> 2) * NT;
+  if (q0 >= b.T) return;
+  const int groups = q0 < 32 ? 1 : 2;   // of 32 keys, up to the last query's own
+  cf32x4 sc[2][2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      sc[k][u] = cf32x4{0.f, 0.f, 0.f, 0.f};
+      if (k >= groups) continue;
+      const int key = 32 * k + 8 * (l15 >> 2) + 4 * u + (l15 & 3);
+#pragma unroll
+      for (int d = 0; d < NKS; ++d)
+        sc[k][u] = cmfma<DT>(*reinterpret_cast<const uint4*>(ks + key * LQ + 32 * d + 8 * g),
+                             *reinterpret_cast<const uint4*>(qs + qi * LQ + 32 * d + 8 * g), sc[k][u]);
+    }
+  float m = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool seen = k < groups && 32 * k + 8 * g + 4 * u + e <= qi;   // (a query past the rows sees some key)
+        sc[k][u][e] = seen ? sc[k][u][e] * b.scale_log2 : -INFINITY;
+        m = fmaxf(m, sc[k][u][e]);
+      }
+  m = fmaxf(m, __shfl_xor(m, 16));
+  m = fmaxf(m, __shfl_xor(m, 32));
+  float l = 0.f;
+  uint4 pf[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    uint32_t w[4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      uint16_t y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = __builtin_amdgcn_exp2f(sc[k][u][e] - m);
+        l += x;
+        y[e] = from_f32<DT>(x);
+      }
+      w[2 * u] = y[0] | (uint32_t)y[1] << 16;
+      w[2 * u + 1] = y[2] | (uint32_t)y[3] << 16;
+    }
+    pf[k] = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  const float inv = 1.f / l;
+  uint16_t* o = b.out + (size_t)qi * b.ldo + h * HD;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int d0 = 16 * (t0 + t);
+    cf32x4 acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (k < groups) acc = cmfma<DT>(*reinterpret_cast<const uint4*>(vt + (d0 + l15) * LV + 32 * k + 8 * g), pf[k], acc);
+    if (qi < b.T)
+      *reinterpret_cast<uint2*>(o + d0 + 4 * g) =
+          make_uint2(from_f32<DT>(acc[0] * inv) | (uint32_t)from_f32<DT>(acc[1] * inv) << 16,
+                     from_f32<DT>(acc[2] * inv) | (uint32_t)from_f32<DT>(acc[3] * inv) << 16);
+  }
+}
+
 template <int DT, int NV>
 static int launch_norm(const SlabNormArgs& a, int M, int threads, hipStream_t st) {
 #define CAKE_SLAB(SL) hipLaunchKernelGGL((slab_norm_kernel<DT, NV, SL>), dim3(M), dim3(threads), 0, st, a)
@@ -201,6 +362,26 @@ CAKE_API int cake_slab_rope(int dt, const float* ws, int slabs, void* q, int ldq
 #define CAKE_SLAB_DT(DT) if (slabs == 1) CAKE_SLAB(DT, 1); else if (slabs == 2) CAKE_SLAB(DT, 2); else CAKE_SLAB(DT, 4)
   if (dt == kBF16) { CAKE_SLAB_DT(kBF16); } else { CAKE_SLAB_DT(kF16); }
 #undef CAKE_SLAB_DT
+#undef CAKE_SLAB
+  return (int)hipGetLastError();
+}
+
+// cake_slab_rope of a prompt's first T <= 64 rows (position 0 on), and their causal attention to out [T][ldo];
+// head sizes of 64 and 128
+CAKE_API int cake_slab_attn(int dt, const float* ws, int slabs, void* out, long long ldo, int T, int nh, int nkv,
+                            int hd, const float* inv_freq, int S, void* kc, void* vc, float scale, hipStream_t st) {
+  if (T < 0 || T > 64 || slabs < 1 || !(hd == 64 || hd == 128) || nh < 1 || nkv < 1 || nh % nkv || T > S ||
+      ldo < (long long)nh * hd || ldo % 4 || ((uintptr_t)ws & 15) ||
+      (((uintptr_t)out | (uintptr_t)kc | (uintptr_t)vc) & 7) || !(dt == kBF16 || dt == kF16))
+    return (int)hipErrorInvalidValue;
+  if (T == 0) return 0;
+  const SlabAttnArgs a{{ws, nullptr, (uint16_t*)kc, (uint16_t*)vc, inv_freq, (long long)T * (nh + 2 * nkv) * hd, slabs,
+                        0, nh, nkv, hd, 0, S}, (uint16_t*)out, ldo, T, scale * 1.4426950408889634f};
+#define CAKE_SLAB(DT, HD) \
+  if (slabs <= 2) hipLaunchKernelGGL((slab_attn_kernel<DT, HD, 2>), dim3(nh), dim3(512), 0, st, a); \
+  else hipLaunchKernelGGL((slab_attn_kernel<DT, HD, 4>), dim3(nh), dim3(512), 0, st, a)
+  if (dt == kBF16) { if (hd == 128) { CAKE_SLAB(kBF16, 128); } else { CAKE_SLAB(kBF16, 64); } }
+  else { if (hd == 128) { CAKE_SLAB(kF16, 128); } else { CAKE_SLAB(kF16, 64); } }
 #undef CAKE_SLAB
   return (int)hipGetLastError();
 }

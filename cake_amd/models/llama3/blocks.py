@@ -370,17 +370,21 @@ class LayerStack:
             G.slab_norm(None, 0, hidden, w.ln1, cfg.rms_norm_eps, x)
         else:
             K.rmsnorm(hidden, w.ln1, cfg.rms_norm_eps, x)
-        if f_qkv:
+        att = torch.empty((T, nq), device=hidden.device, dtype=self.dtype)
+        q = None
+        if f_qkv and G.slab_attn_ok(T, pos0, hd):
+            G.slab_attn(*G.slabs(x, w.wqkv, f_qkv), att, nh, self.inv_freq, kc, vc, self.scale)
+        elif f_qkv:
             q = torch.empty((T, nq), device=hidden.device, dtype=self.dtype)
             G.slab_rope(*G.slabs(x, w.wqkv, f_qkv), q, nh, self.inv_freq, pos0, kc, vc)
         else:
             qkv = G.linear(x, w.wqkv)  # one GEMM for q|k|v
             q, k, v = qkv[:, :nq], qkv[:, nq:nq + nk], qkv[:, nq + nk:]
             K.rope_kv(q, k, v, self.inv_freq, pos0, kc, vc)
-        att = torch.empty((T, nq), device=hidden.device, dtype=self.dtype)
-        Tk = pos0 + T
-        K.flash_attn(q.view(1, T, nh, hd).transpose(1, 2), kc[None, :, :Tk], vc[None, :, :Tk],
-                     att.view(1, T, nh, hd).transpose(1, 2), self.scale, causal=True, pos0=pos0)
+        if q is not None:
+            Tk = pos0 + T
+            K.flash_attn(q.view(1, T, nh, hd).transpose(1, 2), kc[None, :, :Tk], vc[None, :, :Tk],
+                         att.view(1, T, nh, hd).transpose(1, 2), self.scale, causal=True, pos0=pos0)
         if f_o:
             G.slab_norm(*G.slabs(att, w.wo, f_o), hidden, w.ln2, cfg.rms_norm_eps, x)
         else:

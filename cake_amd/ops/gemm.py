@@ -100,6 +100,8 @@ def _lib():
         lib.cake_slab_norm.restype = I
         lib.cake_slab_rope.argtypes = [I, P, I, P, I, I, I, I, I, P, I, I, P, P, P]
         lib.cake_slab_rope.restype = I
+        lib.cake_slab_attn.argtypes = [I, P, I, P, L, I, I, I, I, P, I, P, P, C.c_float, P]
+        lib.cake_slab_attn.restype = I
         lib.cake_gemm_rows_sections.argtypes = [I, P, L, P, L, P, L, P, L, P, L, I, I, P, P, P, I, I,
                                                 I, P]
         lib.cake_gemm_rows_sections.restype = I
@@ -570,6 +572,26 @@ def slab_rope(ws, n: int, q: torch.Tensor, heads: int, inv_freq, pos0: int, kc, 
     check(_lib().cake_slab_rope(_DT[q.dtype], ws.data_ptr(), n, q.data_ptr(),
                                 q.stride(0) if T > 1 else q.shape[1], T, heads, nkv, hd, inv_freq.data_ptr(),
                                 int(pos0), S, kc.data_ptr(), vc.data_ptr(), current_stream()), "slab_rope")
+
+
+def slab_attn_ok(T: int, pos0: int, hd: int) -> bool:
+    """Rows that :func:`slab_attn` takes: a prompt's first ones."""
+    return pos0 == 0 and T <= ROWS_MAX and hd in (64, 128)
+
+
+def slab_attn(ws, n: int, out: torch.Tensor, heads: int, inv_freq, kc, vc, scale: float) -> None:
+    """:func:`slab_rope` of a prompt's first rows (position 0 on), and their causal attention to out
+    [T, >= heads hd]."""
+    T, (nkv, S, hd) = out.shape[0], kc.shape
+    if out.dtype not in _DT or kc.dtype != out.dtype or vc.dtype != out.dtype or out.stride(1) != 1 or \
+            out.shape[1] < heads * hd or not (kc.is_contiguous() and vc.is_contiguous()) or \
+            vc.shape != kc.shape or ws.numel() < n * T * (heads + 2 * nkv) * hd or \
+            inv_freq.dtype != torch.float32 or inv_freq.numel() != hd // 2:
+        raise ValueError("slab_attn: 16-bit rows and caches of one dtype expected")
+    check(_lib().cake_slab_attn(_DT[out.dtype], ws.data_ptr(), n, out.data_ptr(),
+                                out.stride(0) if T > 1 else out.shape[1], T, heads, nkv, hd,
+                                inv_freq.data_ptr(), S, kc.data_ptr(), vc.data_ptr(), float(scale),
+                                current_stream()), "slab_attn")
 
 
 # tile configuration of a grouped product -> its rows (ROWS: the stream form; BY_LIST: 128, 160, 192 or 256,

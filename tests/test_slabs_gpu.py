@@ -102,6 +102,45 @@ def test_slab_rope(dt, T, nh, nkv, hd, pos0, n):
         assert (c[:, :pos0] == 0).all() and (c[:, pos0 + T:] == 0).all()
 
 
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("T", [1, 2, 15, 16, 17, 31, 32, 33, 45, 48, 49, 64])
+@pytest.mark.parametrize("nh,nkv,hd,n", [(4, 2, 64, 1), (8, 1, 128, 3), (16, 16, 128, 8), (5, 5, 64, 2)])
+def test_slab_attn(dt, T, nh, nkv, hd, n):
+    g = torch.Generator("cuda").manual_seed(hd + n + T)
+    cols, S = (nh + 2 * nkv) * hd, 70
+    slabs = torch.randn(n, T, cols, device="cuda", generator=g) * n ** -0.5
+    inv = 1.0 / 10000.0 ** (torch.arange(0, hd, 2, device="cuda") / hd)
+    outs, caches = [], []
+    for _ in range(2):
+        out = torch.full((T, nh * hd + 8), 7.0, device="cuda", dtype=dt)
+        kc, vc = (torch.full((nkv, S, hd), 5.0, device="cuda", dtype=dt) for _ in range(2))
+        rc = G._lib().cake_slab_attn(G._DT[dt], slabs.data_ptr(), n, out.data_ptr(), nh * hd + 8, T, nh, nkv, hd,
+                                     inv.data_ptr(), S, kc.data_ptr(), vc.data_ptr(), hd ** -0.5,
+                                     torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        outs.append(out)
+        caches.append((kc, vc))
+    assert torch.equal(*outs) and (outs[0][:, nh * hd:] == 7).all()
+    # the cache of the rotation of its own, row for row
+    q = torch.zeros(T, cols, device="cuda", dtype=dt)
+    k2, v2 = (torch.full((nkv, S, hd), 5.0, device="cuda", dtype=dt) for _ in range(2))
+    assert G._lib().cake_slab_rope(G._DT[dt], slabs.data_ptr(), n, q.data_ptr(), cols, T, nh, nkv, hd,
+                                   inv.data_ptr(), 0, S, k2.data_ptr(), v2.data_ptr(),
+                                   torch.cuda.current_stream().cuda_stream) == 0
+    half = 2.0 ** (-8 if dt == torch.bfloat16 else -11)
+    for a, b in zip(caches[0], (k2, v2)):
+        assert ((a.double() - b.double()).abs() <= 2 * half * b.double().abs() + 1e-6).all()
+        assert (a[:, T:] == 5).all()
+    # and its rows' attention in 64 bits: probabilities and results are rounded once each
+    Q = q[:, :nh * hd].double().view(T, nh, hd)
+    K, V = (c[:, :T].double().transpose(0, 1).repeat_interleave(nh // nkv, 1) for c in caches[0])
+    s = torch.einsum("qhd,khd->hqk", Q, K) * hd ** -0.5
+    p = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device="cuda").triu(1), -float("inf")).softmax(-1)
+    want = torch.einsum("hqk,khd->qhd", p, V).reshape(T, -1)
+    size = torch.einsum("hqk,khd->qhd", p, V.abs()).reshape(T, -1)
+    assert ((outs[0][:, :nh * hd].double() - want).abs() <= 1.05 * half * (want.abs() + size) + 2 * half * size).all()
+
+
 def test_refused():
     z, st = torch.zeros(4096, device="cuda"), torch.cuda.current_stream().cuda_stream
     p = z.data_ptr()
@@ -113,3 +152,5 @@ def test_refused():
     assert L.cake_slab_norm(0, p, 1, p, 6, None, 1.0, None, 0, 0.0, 1e-5, 0, 1, 6, None, 0, st) != 0
     assert L.cake_slab_norm(0, p, 1, p, 8196, None, 1.0, None, 0, 0.0, 1e-5, 0, 1, 8196, None, 0, st) != 0
     assert L.cake_slab_rope(0, p, 1, p, 64, 1, 1, 1, 12, p, 0, 4, p, p, st) != 0
+    for T, nh, nkv, hd, S in ((65, 1, 1, 64, 70), (2, 3, 2, 64, 4), (2, 1, 1, 96, 4), (5, 1, 1, 64, 4)):
+        assert L.cake_slab_attn(0, p, 1, p, nh * hd, T, nh, nkv, hd, p, S, p, p, 1.0, st) != 0
