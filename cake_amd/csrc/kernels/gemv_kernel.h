@@ -101,14 +101,14 @@ __device__ __forceinline__ void stage_plain16(const uint16_t* __restrict__ x, in
 // plain prologue order — made the norm wait for the whole weight batch; in this
 // order the norm waits only for x, and its reduction / LDS round trips overlap
 // the weight stream.  K = 1024 NX (RMSNorm, f32 row) or 2048 NX (16-bit row).
-template <int DT, int NX> struct NormPre {  // K <= 1024 NX, K % 4 == 0
+template <int DT, int NX, int NT = kGemvThreads> struct NormPre {  // NT threads, K <= 4 NT NX, K % 4 == 0
   float4 x[NX];
   uint2 w[NX];
   __device__ __forceinline__ void load(const float* __restrict__ xg, const uint16_t* __restrict__ wg,
                                        int K) {
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
-      const int i = (j * kGemvThreads + threadIdx.x) * 4;
+      const int i = (j * NT + threadIdx.x) * 4;
       x[j] = i < K ? *reinterpret_cast<const float4*>(xg + i) : make_float4(0.f, 0.f, 0.f, 0.f);
       w[j] = i < K ? *reinterpret_cast<const uint2*>(wg + i) : make_uint2(0u, 0u);
     }
@@ -122,7 +122,7 @@ template <int DT, int NX> struct NormPre {  // K <= 1024 NX, K % 4 == 0
     const float r = rsqrtf(ss / (float)K + eps);
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
-      const int i = (j * kGemvThreads + threadIdx.x) * 4;
+      const int i = (j * NT + threadIdx.x) * 4;
       float4 v = x[j];
       v.x *= r * to_f32<DT>((uint16_t)(w[j].x & 0xffff));
       v.y *= r * to_f32<DT>((uint16_t)(w[j].x >> 16));
@@ -141,7 +141,7 @@ template <int DT, int NX> struct NormPre {  // K <= 1024 NX, K % 4 == 0
       for (int j = 0; j < NX; ++j) sum += (x[j].x + x[j].y) + (x[j].z + x[j].w);
       const float mean = block_sum(sum, red) / (float)Kn;
 #pragma unroll
-      for (int j = 0; j < NX; ++j) centre4(x[j], mean, (j * kGemvThreads + threadIdx.x) * 4, Kn);
+      for (int j = 0; j < NX; ++j) centre4(x[j], mean, (j * NT + threadIdx.x) * 4, Kn);
     }
     float ss = 0.f;
 #pragma unroll
@@ -150,7 +150,7 @@ template <int DT, int NX> struct NormPre {  // K <= 1024 NX, K % 4 == 0
     const float r = rsqrtf(ss / (float)Kn + eps);
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
-      const int i = (j * kGemvThreads + threadIdx.x) * 4;
+      const int i = (j * NT + threadIdx.x) * 4;
       float4 v = x[j];
       v.x *= r * (off + to_f32<DT>((uint16_t)(w[j].x & 0xffff)));
       v.y *= r * (off + to_f32<DT>((uint16_t)(w[j].x >> 16)));

@@ -4,49 +4,17 @@
 // concatenated rows [mixer projections | feed-forward up] (the norm is the prologue, the
 // feed-forward activation the epilogue of the up rows) and its output side ONE launch over
 // the concatenated columns [mixer output | feed-forward down] with the residual sum in the
-// epilogue; between them runs the mixer (mixer_attn.hip, mixer_delta.hip).  A serial layer runs
+// epilogue; between them runs the mixer (mixer_attn.hip, mixer_delta.hip; with the up rows beside it where
+// mixer_beside.hip takes them, the first launch is the mixer's rows then).  A serial layer runs
 // the same two kernels around its mixer and again around its feed-forward.
-#include "gemv_kernel.h"
-#include "mixer_common.h"
+#include "mixer_gemv.h"
 
 namespace cake {
 
-// rows [0, n_raw) -> out f32; rows [n_raw, N) -> act = actf(. + bias) in 16 bit.  ln: a layer
-// norm instead of the RMS norm; bias (the up rows') may be null.
 template <int DT, int U, int PFC, int NX>
-__global__ __launch_bounds__(kGemvThreads) void mixer_in_kernel(
-    const float* __restrict__ resid, const uint16_t* __restrict__ norm_w, float eps, float off,
-    int ln, int Kn, const uint16_t* __restrict__ w, int K, int N, int n_raw,
-    float* __restrict__ out, int actf, const uint16_t* __restrict__ bias,
-    uint16_t* __restrict__ act) {
+__global__ __launch_bounds__(kGemvThreads) void mixer_in_kernel(MixInArgs a) {
   extern __shared__ float xs[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int npairs = (N + 1) >> 1;
-  const int p0 = blockIdx.x * kGemvWaves + wave;
-  auto map = [&](int p, const uint16_t*& wa, const uint16_t*& wb) {
-    wa = w + (size_t)(2 * p) * K;
-    wb = w + (size_t)min(2 * p + 1, N - 1) * K;
-  };
-  Regs<PFC> pre;
-  NormPre<DT, NX> xp;
-  const uint16_t *wa0, *wb0;
-  map(p0 < npairs ? p0 : npairs - 1, wa0, wb0);
-  if constexpr (NX > 0) xp.load(resid, norm_w, K);
-  __builtin_amdgcn_sched_barrier(0);  // x loads strictly before the weights (in-order vmcnt)
-  if (NX > 0 || (PFC > 0 && p0 < npairs)) prefetch_rows<PFC>(wa0, wb0, pre);
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (NX > 0) xp.finish_off(eps, K, Kn, off, ln, xs);
-  else stage_norm_off<DT>(resid, norm_w, eps, K, Kn, off, ln, xs);
-  auto epi = [&](int p, float da, float db) {
-    if (lane > 1) return;  // lane 0 the pair's first row, lane 1 its second
-    const int r = 2 * p + lane;
-    const float d = lane == 0 ? da : db;
-    if (r >= N) return;
-    if (r < n_raw) out[r] = d;
-    else act[r - n_raw] =
-        from_f32<DT>(mix_act(actf, bias ? d + to_f32<DT>(bias[r - n_raw]) : d));
-  };
-  run_pairs<DT, true, U, PFC>(map, epi, xs, K, npairs, p0, gridDim.x * kGemvWaves, pre);
+  mixer_in_rows<DT, U, PFC, NX, kGemvThreads>(a, blockIdx.x, gridDim.x, xs);
 }
 
 // y[r] = x[r] + alpha ((W a)[r] + bias[r]), a 16-bit; bias may be null
@@ -142,10 +110,9 @@ CAKE_API int cake_mixer_in(int dt, const float* resid, const void* norm_w, float
       lds > 160 * 1024 || actf < 0 || actf >= kMixActs)
     return (int)hipErrorInvalidValue;
   const int g = grid_for((N + 1) / 2, 1024);
-#define CAKE_MIN(PF, NX)                                                                      \
-  CAKE_MIX_LAUNCH((mixer_in_kernel<DT, 2, PF, NX>), g, lds, resid, (const uint16_t*)norm_w, eps, \
-                  off, ln, Kn, (const uint16_t*)w, K, N, n_raw, out, actf, (const uint16_t*)bias, \
-                  (uint16_t*)act)
+  const MixInArgs a{resid, (const uint16_t*)norm_w, (const uint16_t*)w, out, (const uint16_t*)bias,
+                    (uint16_t*)act, eps, off, ln, Kn, K, N, n_raw, actf};
+#define CAKE_MIN(PF, NX) CAKE_MIX_LAUNCH((mixer_in_kernel<DT, 2, PF, NX>), g, lds, a)
   DISPATCH_DT(dt, if (K / 8 < 128) CAKE_MIN(0, 0); else if (K / 8 < 256) CAKE_MIN(2, 2);
               else if (K <= 4096) CAKE_MIN(4, 4);
               else if (K <= 8192) CAKE_MIN(4, 8); else CAKE_MIN(4, 0));

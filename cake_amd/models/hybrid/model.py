@@ -493,7 +493,13 @@ class HybridModel:
                 M.loop_in(x, x0, self.head.loop_step[run.enter], self.head.loop_in, self.W, y)
                 x = y
             mix = b.act[run.layer, :w.out_cols]
-            M.layer_in(x, w.norm, cfg.eps, cfg.norm_offset, self.W, w.w_in, w.n_raw, b.proj,
+            # the up rows go beside the mixer, which leaves most of the chip idle
+            rows, up = w.w_in, None
+            if w.ff and M.takes_up_rows(w.shape, rows.shape[1]):
+                rows = w.w_in[:w.n_raw]
+                up = M.UpRows(x, w.norm, cfg.eps, cfg.norm_offset, cfg.layer_norm, self.W,
+                              w.w_in[w.n_raw:], mix[w.mix_cols:])
+            M.layer_in(x, w.norm, cfg.eps, cfg.norm_offset, self.W, rows, w.n_raw, b.proj,
                        mix[w.mix_cols:], ln=cfg.layer_norm)
             ka, kb = self.pool.bufs[run.index]
             proj = b.proj[:w.n_raw].view(1, -1)
@@ -502,10 +508,10 @@ class HybridModel:
             elif isinstance(m, AttentionMixer):
                 M.attn_decode(w.shape, proj, b.pos, b.seq_slot, self._rotation(m), m.qk_norm,
                               m.sink, m.gated, cfg.eps, m.scale, ka, kb, mix.view(1, -1), nsplit,
-                              b.part, b.ticket)
+                              b.part, b.ticket, up)
             else:
                 M.delta_decode(w.shape, proj, proj[:, w.n_main:], b.pos, b.seq_slot, cfg.eps,
-                               **w.consts, state=ka, ring=kb, out=mix.view(1, -1))
+                               **w.consts, state=ka, ring=kb, out=mix.view(1, -1), up=up)
             y = b.xa if x is x0 else x
             M.layer_out(mix, w.w_out, cfg.residual_mult, x, y)
             x = y

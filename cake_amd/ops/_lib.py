@@ -242,5 +242,9 @@ _LIB_SIGS = {
                                      P, P, P, P, P, L, L, P, P, P, P, I, P, P, I, P, L, P],
         "cake_mixer_delta_decode": [I, P, L, P, L, I, I, I, I, I, I, I, F, P, P, P, P, P, P, L, L,
                                     P, P, P, L, P],
+        "cake_mixer_beside_attn": [I, P, P, P, P, I, I, I, I, F, F, P, P, L, L, P, I, I, I, I, I, I, I, I, P, P,
+                                   P, P, F, F, I, I, P, I, I, I, P, P],
+        "cake_mixer_beside_delta": [I, P, P, I, I, I, I, I, I, F, P, P, P, P, P, P, L, L, P, P, P,
+                                    P, P, F, F, I, I, P, I, I, I, P, P],
     },
 }

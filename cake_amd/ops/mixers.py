@@ -292,10 +292,42 @@ def attn_prompt(sh: AttnShape, qn, kc, vc, rows: Rows, gate, out, scale: float, 
           "mixer_flash")
 
 
+@dataclass(frozen=True)
+class UpRows:
+    """The feed-forward's up rows of a parallel layer's token, for the launch of its mixer: act [N] =
+    activation(w norm(resid)), w [N, K], the norm as :func:`layer_in` takes it."""
+    resid: torch.Tensor
+    norm_w: torch.Tensor
+    eps: float
+    offset: float
+    ln: bool
+    width: int
+    w: torch.Tensor
+    act: torch.Tensor
+    kind: str = "gelu"
+
+    def args(self, dtype):
+        N, K = self.w.shape
+        return (_vec(self.resid, "resid", torch.float32, K), _vec(self.norm_w, "norm_w", dtype, K),
+                float(self.eps), float(self.offset), int(self.ln), int(self.width),
+                _vec(self.w, "w", dtype), K, N, ACTS[self.kind], _vec(self.act, "act", dtype, N))
+
+
+def takes_up_rows(sh, K: int) -> bool:
+    """Whether a mixer's launch of one token takes rows of K columns along (mixer_beside.hip): 16-bit
+    storage, widths whose norm lies in registers, heads whose state or keys do."""
+    if not 2048 <= K <= 8192 or K % 8:
+        return False
+    if isinstance(sh, AttnShape):
+        return sh.DP == sh.DVP and sh.DP in (64, 128) and sh.tiles <= 256
+    return isinstance(sh, DeltaShape) and sh.heads <= 256 and -(-sh.dim // (512 // (sh.EP // 4))) <= 8
+
+
 def attn_decode(sh: AttnShape, proj, pos, slot, cs, qk_norm: bool, sink: bool, gated: bool,
-                eps: float, scale: float, kc, vc, out, nsplit: int, part, ticket):
+                eps: float, scale: float, kc, vc, out, nsplit: int, part, ticket, up: UpRows | None = None):
     """One token per sequence: proj [B, q|k|v(|gate)] f32, pos / slot int32 [B] on the device
-    (the caller keeps pos < S); writes the new key / value and out [B, >= H vdim]."""
+    (the caller keeps pos < S); writes the new key / value and out [B, >= H vdim].  up: rows to run
+    beside it, of one sequence (:func:`takes_up_rows`)."""
     S, _ = _cache(sh, kc, vc, out.dtype)
     B = proj.shape[0]
     cols = sh.qkv_cols + (sh.out_cols if gated else 0)
@@ -305,6 +337,18 @@ def attn_decode(sh: AttnShape, proj, pos, slot, cs, qk_norm: bool, sink: bool, g
         raise ValueError(f"nsplit {nsplit} outside 1..{MAX_SPLIT}")
     if sh.rot_pairs and (cs.shape[0] < S or cs.shape[1] != 2 * sh.rot_pairs):
         raise ValueError("rotation table does not cover the cache")
+    if up is not None:
+        if B != 1 or not takes_up_rows(sh, up.w.shape[1]):
+            raise ValueError(f"no rows beside {B} tokens of {sh}")
+        check(_lib().cake_mixer_beside_attn(
+            DT[out.dtype], pp, _vec(pos, "pos", torch.int32, B), _vec(slot, "slot", torch.int32, B),
+            _vec(cs, "cs", torch.float32), sh.rot_pairs, int(qk_norm), int(sink), int(gated), float(eps),
+            float(scale), kc.data_ptr(), vc.data_ptr(), kc.stride(0), vc.stride(0), op, sh.heads,
+            sh.kv_heads, sh.dim, sh.vdim, sh.DP, sh.DVP, S, int(nsplit),
+            _vec(part, "part", torch.float32, sh.part_floats(B, nsplit)),
+            _vec(ticket, "ticket", torch.int32, B * sh.tiles), *up.args(out.dtype), _stream()),
+            "mixer_beside_attn")
+        return
     check(_lib().cake_mixer_attn_decode(
         DT[out.dtype], pp, ldp, B, _vec(pos, "pos", torch.int32, B),
         _vec(slot, "slot", torch.int32, B), _vec(cs, "cs", torch.float32), sh.rot_pairs,
@@ -387,13 +431,23 @@ def delta_prompt(sh: DeltaShape, proj, ab, rows: Rows, eps: float, conv, a_log, 
 
 
 def delta_decode(sh: DeltaShape, proj, ab, pos, slot, eps: float, conv, a_log, dt_bias, norm_w,
-                 state, ring, out):
-    """One token per sequence: proj [B, q|k|v|gate] f32, ab [B, a|b] f32."""
+                 state, ring, out, up: UpRows | None = None):
+    """One token per sequence: proj [B, q|k|v|gate] f32, ab [B, a|b] f32.  up: rows to run beside it,
+    of one sequence (:func:`takes_up_rows`)."""
     B, f = proj.shape[0], torch.float32
     pp, ldp = _mat(proj, "proj", f, B, sh.channels + sh.out_cols)
     abp, ldab = _mat(ab, "ab", f, B, 2 * sh.heads)
     op, ldo = _mat(out, "out", out.dtype, B, sh.out_cols)
     sp, rp, s_slot, r_slot = _delta_state(sh, state, ring)
+    if up is not None:
+        if B != 1 or not takes_up_rows(sh, up.w.shape[1]):
+            raise ValueError(f"no rows beside {B} tokens of {sh}")
+        check(_lib().cake_mixer_beside_delta(
+            DT[out.dtype], pp, abp, sh.heads, sh.kv_heads, sh.dim, sh.vdim, sh.EP, sh.taps, float(eps),
+            *_delta_consts(sh, conv, a_log, dt_bias, norm_w), sp, rp, s_slot, r_slot,
+            _vec(pos, "pos", torch.int32, B), _vec(slot, "slot", torch.int32, B), op, *up.args(out.dtype),
+            _stream()), "mixer_beside_delta")
+        return
     check(_lib().cake_mixer_delta_decode(
         DT[out.dtype], pp, ldp, abp, ldab, B, sh.heads, sh.kv_heads, sh.dim, sh.vdim, sh.EP,
         sh.taps, float(eps), *_delta_consts(sh, conv, a_log, dt_bias, norm_w), sp, rp, s_slot,
