@@ -108,6 +108,16 @@ __device__ __forceinline__ void amfma_dma_at(cf32x4& acc, const uint4& a, const 
                  : "memory", "scc");
 }
 
+// Of a grouped product, workgroup bid's row tile and column tile (n x tiles_n of them): dealt out to the XCDs in
+// runs; most groups have one or two row tiles, so two of them walk all columns and their rows are read once (eight
+// read every row four times over; 64 groups of 192 rows of 4096 to 3616 columns 509 -> 483 us, back 543 -> 506)
+__device__ __forceinline__ int2 grouped_place(int n, int tiles_n, int bid) {
+  const int all = n * tiles_n, q = all / 8, r = all % 8, x = bid % 8;
+  const int id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + bid / 8;
+  const int per = 2 * tiles_n, first = id / per * 2, gm = min(2, n - first);
+  return make_int2(first + id % per % gm, id % per / gm);
+}
+
 // SCHED 1: three barriers a k step (the DMAs of step t+2 issued as soon as every wave has read the
 // operand region they overwrite).  SCHED 2: one barrier, for tiles of which the LDS holds three or
 // four k steps.  A step of a small tile is bound by its waits, not by the matrix cores: 192 x 192 is
@@ -174,16 +184,15 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
     }
   }
   const int pieces = PCS && (int)blockIdx.x >= g.dp_tiles ? g.pieces : 1;
-  // grouped products: most groups have one or two row tiles, so two of them walk all columns and
-  // their rows are read once (eight read every row four times over; 64 groups of 192 rows of 4096
-  // to 3616 columns 509 -> 483 us, back 543 -> 506)
-  constexpr int GROUP = GRP ? 2 : 8;
+  constexpr int GROUP = 8;
   const int per_group = GROUP * g.tiles_n;
   const int first_m = (id / per_group) * GROUP;
   const int gm = min(GROUP, g.tiles_m - first_m);
-  const int tm = first_m + (id % per_group) % gm;
+  const int2 at = GRP ? grouped_place(g.tiles_m, g.tiles_n, blockIdx.x)
+                      : make_int2(first_m + (id % per_group) % gm, (id % per_group) / gm);
+  const int tm = at.x;
   const int m0 = GRP ? 0 : tm * BM;
-  const int n0 = ((id % per_group) / gm) * BN;
+  const int n0 = at.y * BN;
   if constexpr (GRP) {
     const int4 t = g.groups[tm];
     g.a += (size_t)t.y * g.lda;

@@ -16,11 +16,19 @@ constexpr int grouped_rows(int cfg) {
 // One kernel for the four heights, so that the one that fits the groups can be chosen on the device, where
 // their sizes are known (mixer_experts.hip).  All of them fill a CU's LDS alone: a branch over whole
 // bodies costs none of them a workgroup (two products of 64 experts 4096 x 3648, 192 rows each: 932 us in
-// a kernel of its own, 938 so; over all heights and seven sizes 0.8 % more).
+// a kernel of its own, 938 so; over all heights and seven sizes 0.8 % more).  A tile runs at the least height
+// that holds its rows, the list's is what the longest of them needs: of 44 pairs of products, even and skewed groups of
+// 70 .. 600 rows, up to 12 % faster, 1.2 % on the average (64 of 4096 x 3648 at 170 rows 488 + 463 us, 451 + 429;
+// eight of 4096 x 4096 at 300 rows 93 + 91, 81 + 81), none slower by more than they vary.
 template <int DT, int EPI>
 __global__ __launch_bounds__(256) void gemm_heights_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[FourWave<160, 256, 2>::NBUF * FourWave<160, 256, 2>::BUF];
-  const int rows = g.pieces > 0 ? g.pieces : __builtin_amdgcn_readfirstlane(g.groups[g.tiles_m].y);
+  const int n = g.groups[g.tiles_m].x;
+  if ((int)blockIdx.x >= n * g.tiles_n) return;
+  const int most = g.pieces > 0 ? g.pieces : g.groups[g.tiles_m].y;
+  const int tm = grouped_place(n, g.tiles_n, blockIdx.x).x;
+  const int has = min(__builtin_amdgcn_readfirstlane(g.groups[tm].z), __builtin_amdgcn_readfirstlane(most));
+  const int rows = has <= 128 ? 128 : has <= 160 ? 160 : has <= 192 ? 192 : 256;
 #define X(BM, SCHED)                                                                         \
   if (rows == BM) {                                                                          \
     static_assert(FourWave<BM, 256, SCHED>::NBUF * FourWave<BM, 256, SCHED>::BUF <= (int)sizeof(smem), "LDS"); \
