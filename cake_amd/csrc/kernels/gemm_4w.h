@@ -193,8 +193,10 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
   const int tm = at.x;
   const int m0 = GRP ? 0 : tm * BM;
   const int n0 = at.y * BN;
+  int group = 0;
   if constexpr (GRP) {
     const int4 t = g.groups[tm];
+    group = t.x;
     g.a += (size_t)t.y * g.lda;
     g.c += (size_t)t.y * g.ldc;
     g.b += (size_t)t.x * g.b_group + (size_t)n0 * g.ldb;
@@ -241,8 +243,20 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
   // of range -> zeros, no memory traffic).  Per DMA that leaves the M0 write and the DMA
   // itself in the MFMA stream, the rest is a handful of scalar ops per k-step.
   // descriptor words: base (48 bits, stride 0), num_records, flags (raw, offen)
+  // GRP: weight rows of 4 KB meet on few channels of the memory while all tiles are at the same k, so each begins
+  // at a k of its own, those of the same weights at the same one.  64 groups 2048 -> 1984 at 70 / 130 / 170 / 192
+  // rows 137 / 150 / 160 / 166 us, 111 / 124 / 143 / 149 so.  Where most groups have two tiles, which read the
+  // weights together and x again, it gives from 6 % to -4 %; rows of 8 KB range from 0.8 to 1.08 by where they lie,
+  // longer ones lose the common reads of x (16 KB up to 14 %), and fewer tiles than units gain nothing.
+  int rot = 0;
+  if constexpr (GRP)
+    if (g.ldb == 2048 && ntiles >= 256 && 2 * g.tiles_m <= 3 * (g.groups[g.tiles_m - 1].x + 1))
+      rot = __builtin_amdgcn_readfirstlane((group * 7 + at.y) % nk);
+  auto place = [&](int step) __attribute__((always_inline)) {
+    return !GRP ? step : step >= nk ? nk : step + rot < nk ? step + rot : step + rot - nk;
+  };
   auto desc_at = [&](const uint16_t* base, int nrec, int step) __attribute__((always_inline)) {
-    const int k0 = kb + step * kGBK;
+    const int k0 = kb + place(step) * kGBK;
     const unsigned long long p = (unsigned long long)(base + k0);
     cu32x4 d;
     d[0] = __builtin_amdgcn_readfirstlane((unsigned)p);
@@ -268,8 +282,8 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
     if constexpr (GRP) {
 #pragma unroll
       for (int o = 0; o < 2; ++o) {
-        cur_a[o] = step * kGBK + (chunk_a ^ 4 * o) * 8 < g.K ? voff_a[o] : 0x80000000u;
-        cur_b[o] = step * kGBK + (chunk_b ^ 4 * o) * 8 < g.K ? voff_b[o] : 0x80000000u;
+        cur_a[o] = place(step) * kGBK + (chunk_a ^ 4 * o) * 8 < g.K ? voff_a[o] : 0x80000000u;
+        cur_b[o] = place(step) * kGBK + (chunk_b ^ 4 * o) * 8 < g.K ? voff_b[o] : 0x80000000u;
       }
     }
   };

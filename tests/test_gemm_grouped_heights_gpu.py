@@ -58,3 +58,29 @@ def test_activations_of_every_height(cuda, dt, cfg, epi):
         size = 2.0 ** (-8 if dt == torch.bfloat16 else -11) + 2.0 ** -10
         assert bool((out[:, N:] == 7.0).all())
         assert bool(((out[:, :N].double() - want).abs() <= size * want.abs() + K * 2.0 ** -22 * (1 + y.abs()) * 2).all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
+def test_a_k_of_their_own(cuda, dt):
+    """Weight rows of 4 KB and 256 tiles and more: every tile starts at another k and goes round.  One rounding
+    (2^-8, 2^-11) of f32 sums."""
+    from cake_amd.ops import gemm as G
+    N, K, bm = 520, 2048, 256
+    counts = [(7 * e) % 41 + (200 if e % 31 == 0 else 0) for e in range(90)]
+    R = sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(R, K, device="cuda", generator=g).to(dt)
+    w = (torch.randn(len(counts), N, K, device="cuda", generator=g) * K ** -0.5).to(dt)
+    tiles, r0, y = [], 0, []
+    for e, c in enumerate(counts):
+        tiles += [[e, r0 + t, min(bm, c - t), 0] for t in range(0, c, bm)]
+        y.append(x[r0:r0 + c].double() @ w[e].double().t())
+        r0 += c
+    assert len(tiles) * 3 >= 256
+    t = torch.tensor(tiles + [[0, 0, 0, 0], [len(tiles), bm, 0, 0]], dtype=torch.int32, device="cuda")
+    out = torch.full((R, N + 8), 7.0, dtype=dt, device="cuda")
+    G.grouped(x, w, t, 6, out[:, :N])
+    y = torch.cat(y)
+    size = 2.0 ** (-8 if dt == torch.bfloat16 else -11)
+    assert bool((out[:, N:] == 7.0).all())
+    assert bool(((out[:, :N].double() - y).abs() <= size * y.abs() + K * 2.0 ** -22 * (1 + y.abs())).all())
