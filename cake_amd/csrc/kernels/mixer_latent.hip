@@ -162,6 +162,22 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(AbsorbArgs a) {
     const int b = i / a.dimp, d = i - b * a.dimp;
     qs[b][d] = a.q[(b0 + b) * a.ldq + (long long)h * hd + d];
   }
+  if (blockIdx.y == 0) {
+    // the rotated part and the padding of all sequences at once: one after the other they were a chain of round
+    // trips longer than the products (13 sequences of 16 heads 9.2 us, 7.0 so)
+    const int n = LD - R;
+    for (int k = tid; k < nb * n; k += 256) {
+      const int b = k / n, i = R + k - b * n, j = i - a.p.RP;
+      const float* qr = a.q + (b0 + b) * a.ldq + (long long)h * hd + a.dimp;
+      float y = j >= 0 && j < a.p.rot ? qr[j] : 0.f;
+      if (j >= 0 && j < 2 * a.p.rd2) {
+        const float2 t = a.p.cs[(long long)a.p.pos[b0 + b] * a.p.rd2 + (j >> 1)];
+        const float o = qr[j ^ 1];
+        y = (j & 1) ? y * t.x + o * t.y : y * t.x - o * t.y;
+      }
+      reinterpret_cast<E*>(a.qa)[((long long)(b0 + b) * a.H + h) * LD + i] = St<DT>::st(y);
+    }
+  }
   __syncthreads();
   for (int b = 0; b < nb; ++b) {
     E* out = reinterpret_cast<E*>(a.qa) + ((long long)(b0 + b) * a.H + h) * LD;
@@ -187,20 +203,6 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(AbsorbArgs a) {
       acc = row16_sum(acc);
       const int row = blockIdx.y * kAbsRows + 16 * u + grp;
       if (l16 == 0 && row < R) out[row] = St<DT>::st(acc);
-    }
-    if (blockIdx.y == 0) {  // the rotated part and the padding
-      const float* qr = a.q + (b0 + b) * a.ldq + (long long)h * hd + a.dimp;
-      const float2* cs = a.p.cs + (long long)a.p.pos[b0 + b] * a.p.rd2;
-      for (int i = R + tid; i < LD; i += 256) {
-        const int j = i - a.p.RP;
-        float y = j >= 0 && j < a.p.rot ? qr[j] : 0.f;
-        if (j >= 0 && j < 2 * a.p.rd2) {
-          const float2 t = cs[j >> 1];
-          const float o = qr[j ^ 1];
-          y = (j & 1) ? y * t.x + o * t.y : y * t.x - o * t.y;
-        }
-        out[i] = St<DT>::st(y);
-      }
     }
   }
 }
