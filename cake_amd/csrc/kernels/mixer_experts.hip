@@ -90,14 +90,34 @@ __device__ inline int tile_height(const int (&tiles)[4], int E, int M, int F, in
 
 // Entries (token, k) sorted by expert: scale[p] = score of sorted row p, where[entry] = p; the tile
 // list [expert, first sorted row, rows, 0] of BM-row tiles (0: tile_height of an expert's F x W up
-// matrix), entry max_tiles [their number, BM, 0, 0].
-__global__ __launch_bounds__(1024) void expert_plan_kernel(const int* ids, const float* score,
-                                                           int N, int top, int E, int BM, int F, int W,
-                                                           float* scale, int* where, int4* tiles,
+// matrix), entry max_tiles [their number, BM, 0, 0].  VPL > 0: the choice of a few rows (kPlanEntries entries
+// at most) is made here from the logits, whose launch would be mostly its own time (13 rows of 64 experts 3.5 +
+// 5.8 us, 6.3 so).
+constexpr int kPlanEntries = 1024;
+template <int VPL>
+__global__ __launch_bounds__(1024) void expert_plan_kernel(const float* logits, long long ldl, const int* ids,
+                                                           const float* score, int N, int top, int E, int BM,
+                                                           int F, int W, float* scale, int* where, int4* tiles,
                                                            int max_tiles) {
   __shared__ int cnt[kMaxExperts], scan[2][kMaxExperts], fit[4];
-  constexpr int U = 16;  // entries in flight per thread
+  __shared__ int own_id[VPL > 0 ? kPlanEntries : 1];
+  __shared__ float own_score[VPL > 0 ? kPlanEntries : 1];
+  constexpr int U = VPL > 0 ? 1 : 16;  // entries in flight per thread
   const int tid = threadIdx.x, M = N * top;
+  if constexpr (VPL > 0) {
+    const int lane = tid & 63;
+    for (int n = tid >> 6; n < N; n += 16) {
+      int id;
+      float s;
+      wave_top<VPL>(logits + n * ldl, E, top, lane, id, s);
+      if (lane < top) {
+        own_id[n * top + lane] = id;
+        own_score[n * top + lane] = s;
+      }
+    }
+    ids = own_id;
+    score = own_score;
+  }
   cnt[tid] = 0;
   if (tid < 4) fit[tid] = 0;
   __syncthreads();
@@ -459,8 +479,23 @@ CAKE_API int cake_expert_plan(const int* ids, const float* score, int N, int top
   if (!routing_ok(E, top) || N <= 0 || BM < 0 || (BM == 0 && (F <= 0 || W <= 0)) ||
       max_tiles < (long long)N * top / (BM > 0 ? BM : kHeights[0]) + (E < (long long)N * top ? E : N * top))
     return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(expert_plan_kernel, dim3(1), dim3(1024), 0, st, ids, score, N, top, E, BM, F, W, scale,
-                     where, (int4*)tiles, max_tiles);
+  hipLaunchKernelGGL((expert_plan_kernel<0>), dim3(1), dim3(1024), 0, st, nullptr, 0, ids, score, N, top, E, BM, F, W,
+                     scale, where, (int4*)tiles, max_tiles);
+  return (int)hipGetLastError();
+}
+
+// cake_expert_route and cake_expert_plan of a few rows (N top <= 1024) in one launch
+CAKE_API int cake_expert_route_plan(const float* logits, long long ldl, int N, int top, int E, int BM, int F, int W,
+                                    float* scale, int* where, void* tiles, int max_tiles, hipStream_t st) {
+  if (!routing_ok(E, top) || N <= 0 || ldl < E || BM < 0 || (BM == 0 && (F <= 0 || W <= 0)) ||
+      (long long)N * top > kPlanEntries ||
+      max_tiles < N * top / (BM > 0 ? BM : kHeights[0]) + (E < N * top ? E : N * top))
+    return (int)hipErrorInvalidValue;
+#define CAKE_PLAN(VPL)                                                                                           \
+  hipLaunchKernelGGL((expert_plan_kernel<VPL>), dim3(1), dim3(1024), 0, st, logits, ldl, nullptr, nullptr, N, top, E, \
+                     BM, F, W, scale, where, (int4*)tiles, max_tiles)
+  if (E <= 64) CAKE_PLAN(1); else if (E <= 256) CAKE_PLAN(4); else CAKE_PLAN(16);
+#undef CAKE_PLAN
   return (int)hipGetLastError();
 }
 

@@ -129,7 +129,7 @@ class ExpertsFf:
         E, FP, Wp = self.up.shape
         logits = torch.empty((N, pad_to(E, 4)), device=x.device, dtype=torch.float32)[:, :E]
         model.product(model.norm_rows(x, self.norm32) if h is None else h, self.router, logits)
-        p = X.plan(*X.route(logits, self.top), E, model.dtype, FP * Wp, FP)
+        p = X.route_plan(logits, self.top, model.dtype, FP * Wp, FP)
         h = model.norm_rows(x, self.norm32, where=p.where, scale=p.scale)
         a = torch.empty((M_, FP), device=x.device, dtype=model.dtype)
         X.product(h, self.up, p, a, self.act)

@@ -232,6 +232,7 @@ _LIB_SIGS = {
         "cake_latent_flash": [I, P, L, P, L, P, L, P, P, L, I, I, P, I, I, P, I, I, I, I, I, I, I,
                               F, P, L, P],
         "cake_expert_route": [P, L, I, I, I, P, P, P],
+        "cake_expert_route_plan": [P, L, I, I, I, I, I, I, P, P, P, I, P],
         "cake_expert_plan": [P, P, I, I, I, I, I, I, P, P, P, I, P],
         "cake_expert_sum": [I, P, L, P, I, I, I, F, P, L, P],
         "cake_expert_sum_norm": [I, P, L, P, I, I, I, F, P, L, P, F, F, I, P, L, P],

@@ -14,6 +14,7 @@ from .mixers import ACTS, DT, _lib, _mat, _stream, _vec
 MAX_EXPERTS = 1024
 MAX_TOP = 32
 SUM_NORM_MAX = 8192   # columns of a row that gather_sum_norm holds
+PLAN_ENTRIES = 1024   # of a plan that makes its rows' choice
 BM32 = 32   # row tile of the f32 grouped product
 
 
@@ -50,12 +51,9 @@ class Plan:
         return torch.empty_like(token).scatter_(0, self.where.flatten().long(), token)
 
 
-def plan(ids, score, E: int, dtype, weight: int = 0, up: int = 0) -> Plan:
-    """Rows sorted by expert, and their tiles; weight: elements of an expert's matrix, up: columns of
-    its up product (0: a square matrix)."""
-    N, top = ids.shape
-    _routing(E, top)
-    M, dev = N * top, ids.device
+def _plan(N: int, top: int, E: int, dev, dtype, weight: int, up: int, launch) -> Plan:
+    """launch(BM, up, wide, scale, where, tiles, number of tiles) fills the plan."""
+    M = N * top
     cfg = G.grouped_cfg(M, E, torch.cuda.is_current_stream_capturing(), weight)
     bm = BM32 if dtype == torch.float32 else G.GROUPED_CFGS[cfg]   # the least, of a height yet to choose
     n = M // bm + min(E, M)
@@ -66,12 +64,31 @@ def plan(ids, score, E: int, dtype, weight: int = 0, up: int = 0) -> Plan:
     at = M + -M % 4   # tiles are read whole, 16 bytes each
     tiles = i32[at:at + 4 * (n + 1)].view(n + 1, 4)
     scale = torch.empty(M, device=dev, dtype=torch.float32)
-    check(_lib().cake_expert_plan(_vec(ids, "ids", torch.int32, M),
-                                  _vec(score, "score", torch.float32, M), N, top, E,
-                                  0 if dtype != torch.float32 and cfg == G.BY_LIST else bm, up, wide,
-                                  scale.data_ptr(), where.data_ptr(), tiles.data_ptr(), n, _stream()),
-          "expert_plan")
+    launch(0 if dtype != torch.float32 and cfg == G.BY_LIST else bm, up, wide,
+           scale.data_ptr(), where.data_ptr(), tiles.data_ptr(), n, _stream())
     return Plan(scale, where, tiles, cfg)
+
+
+def plan(ids, score, E: int, dtype, weight: int = 0, up: int = 0) -> Plan:
+    """Rows sorted by expert, and their tiles; weight: elements of an expert's matrix, up: columns of
+    its up product (0: a square matrix)."""
+    N, top = ids.shape
+    _routing(E, top)
+    ip, sp = _vec(ids, "ids", torch.int32, N * top), _vec(score, "score", torch.float32, N * top)
+    return _plan(N, top, E, ids.device, dtype, weight, up, lambda bm, up, wide, *out: check(
+        _lib().cake_expert_plan(ip, sp, N, top, E, bm, up, wide, *out), "expert_plan"))
+
+
+def route_plan(logits, top: int, dtype, weight: int = 0, up: int = 0) -> Plan:
+    """:func:`route` and :func:`plan`; of a few rows in one launch: while a wave has a row, or two
+    short ones, that one workgroup is no slower than many."""
+    N, E = logits.shape
+    _routing(E, top)
+    if not 0 < N <= (32 if E <= 64 else 16) or N * top > PLAN_ENTRIES:
+        return plan(*route(logits, top), E, dtype, weight, up)
+    lp, ldl = _mat(logits, "logits", torch.float32, N, E)
+    return _plan(N, top, E, logits.device, dtype, weight, up, lambda bm, up, wide, *out: check(
+        _lib().cake_expert_route_plan(lp, max(ldl, E), N, top, E, bm, up, wide, *out), "expert_route_plan"))
 
 
 def product(x, w, p: Plan, out, act: str | None = None):
