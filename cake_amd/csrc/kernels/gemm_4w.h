@@ -124,19 +124,15 @@ __device__ __forceinline__ int2 grouped_place(int n, int tiles_n, int bid) {
 // 0.49 us of MFMAs and took 0.75 us alone on the chip (0.63 with one barrier), 1.13 on all CUs (0.98);
 // 128 x 256 0.44, 0.72 (0.62), 1.11 (0.99).  More steps in flight alone changed neither.  Tiles of
 // two steps (256 x 192 and larger) are within 3 % either way.
-// GRP: grouped row tiles (GemmArgs::groups), K any multiple of 8.  Bound by the matrix cores on
-// padded rows and, below some 200 rows a group, by reading the weights: 64 groups of 192 rows,
-// 4096 -> 3616 -> 4096 columns, 1102 -> 989 us against eight waves on the same tile (0.98 PFLOP/s
-// with the padding; the weights alone are 2 x 292 us).
+// GRP: grouped row tiles (GemmArgs::groups), K any multiple of 8.
 // PCS: the tiles past the last whole wave in k pieces (GemmArgs::pieces); an instance of its own,
 // since the sums of pieces spill twice the registers in the epilogue of whole tiles too (4096^3 with
 // the residual 113.3 us with them, 109.9 without).
-// ROT: of grouped products, where a tile may begin at a k of its own (below).
 template <int BM, int BN, int SCHED> struct FourWave {
   static constexpr int BUF = (BM + BN) * 128;  // 64 KB at most per k-step buffer
   static constexpr int NBUF = SCHED != 2 ? 2 : 160 * 1024 / BUF > 4 ? 4 : 160 * 1024 / BUF;
 };
-template <int DT, int EPI, int BM, int BN, int SCHED, bool GRP, bool PCS, bool ROT = false>
+template <int DT, int EPI, int BM, int BN, int SCHED, bool GRP, bool PCS>
 __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
   static_assert(BM % 32 == 0 && BN % 64 == 0, "whole fragments, gated pairs within a wave");
   constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
@@ -244,22 +240,8 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
   // of range -> zeros, no memory traffic).  Per DMA that leaves the M0 write and the DMA
   // itself in the MFMA stream, the rest is a handful of scalar ops per k-step.
   // descriptor words: base (48 bits, stride 0), num_records, flags (raw, offen)
-  // GRP: weight rows of 4 KB meet on few channels of the memory while all tiles are at the same k, so each begins
-  // at a k of its own, those of the same weights at the same one.  64 groups 2048 -> 1984 at 70 / 130 / 170 / 192
-  // rows 137 / 150 / 160 / 166 us, 111 / 124 / 143 / 149 so.  Where most groups have two tiles, which read the
-  // weights together and x again, it gives from 6 % to -4 %; rows of 8 KB range from 0.8 to 1.08 by where they lie,
-  // longer ones lose the common reads of x (16 KB up to 14 %), and fewer tiles than units gain nothing.  An instance
-  // of its own (ROT): the steps' places cost the others up to 3 % (both products of eight groups of 4096 x 14336, 2048
-  // x 5632, 32 of 1024 x 2816, 250 .. 4000 tokens on two or six: 0.992 of the speed without them).
-  int rot = 0;
-  if constexpr (ROT)
-    if (ntiles >= 256 && 2 * g.tiles_m <= 3 * (g.groups[g.tiles_m - 1].x + 1))
-      rot = __builtin_amdgcn_readfirstlane((group * 7 + at.y) % nk);
-  auto place = [&](int step) __attribute__((always_inline)) {
-    return !ROT ? step : step + rot - (step < nk - rot ? 0 : nk);   // (steps past the last read nothing)
-  };
   auto desc_at = [&](const uint16_t* base, int nrec, int step) __attribute__((always_inline)) {
-    const int k0 = kb + place(step) * kGBK;
+    const int k0 = kb + step * kGBK;
     const unsigned long long p = (unsigned long long)(base + k0);
     cu32x4 d;
     d[0] = __builtin_amdgcn_readfirstlane((unsigned)p);
@@ -285,8 +267,8 @@ __device__ __forceinline__ void gemm_4w_tile(GemmArgs g, uint8_t* smem) {
     if constexpr (GRP) {
 #pragma unroll
       for (int o = 0; o < 2; ++o) {
-        cur_a[o] = place(step) * kGBK + (chunk_a ^ 4 * o) * 8 < g.K ? voff_a[o] : 0x80000000u;
-        cur_b[o] = place(step) * kGBK + (chunk_b ^ 4 * o) * 8 < g.K ? voff_b[o] : 0x80000000u;
+        cur_a[o] = step * kGBK + (chunk_a ^ 4 * o) * 8 < g.K ? voff_a[o] : 0x80000000u;
+        cur_b[o] = step * kGBK + (chunk_b ^ 4 * o) * 8 < g.K ? voff_b[o] : 0x80000000u;
       }
     }
   };

@@ -73,7 +73,7 @@ struct GemmArgs {
   // in-kernel split-K (gemm_4w.h): tiles [0, dp_tiles) run whole, the rest in `pieces` (0: none)
   // pieces of kps k elements; every piece of a tile but the last to arrive parks its accumulators
   // in ws, the last sums them in piece order and runs the epilogue; tick = [kPieceTiles arrival
-  // counters | kPieceTiles ready counters]
+  // counters | kPieceTiles ready counters] (gemm_ws.h: of each of a tile's eight waves)
   int pieces;
   unsigned* tick;        // (gemm_rows.h: one arrival counter per strip)
   int dp_tiles;
@@ -87,7 +87,7 @@ struct GemmArgs {
   long long ldc1;
   int n1, n2;
 };
-constexpr int kPieceTiles = 256;
+constexpr int kPieceTiles = 256, kPieceWaves = 8;
 
 // 16 bytes past the caches that other XCDs do not see (agent scope, two 8-byte accesses)
 __device__ __forceinline__ void st_agent16(float4* p, float x, float y, float z, float w) {
@@ -115,6 +115,7 @@ struct Pieces {
   float* slabs;
   uint32_t bytes, lane, at, stride;
   int n;
+  uint32_t tile = 4096;   // from a tile of a strip to the next
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   static constexpr int kSc1 = 16;
   __device__ __forceinline__ float4 load(uint32_t off) const {
@@ -127,7 +128,7 @@ struct Pieces {
   }
   __device__ __forceinline__ Pieces strip(int i, int nf) const {   // strip i of nf tiles each
     Pieces p = *this;
-    p.at += (uint32_t)(i * nf) * 4096u;
+    p.at += (uint32_t)(i * nf) * tile;
     return p;
   }
 };
@@ -296,10 +297,9 @@ __device__ __forceinline__ void store16(uint16_t* dst, const uint16_t* v, bool f
 
 // a strip's accumulators (with the tile's other pieces, in piece order: the same bits whichever
 // arrived last) into the wave's staging slice
-template <int NF>
+template <int NF, int STG_LD = NF * 16 + 4>
 __device__ __forceinline__ void stage_strip_w(const cf32x4 (&tiles)[NF], float* stg, int lane,
                                               const Pieces& add) {
-  constexpr int STG_LD = NF * 16 + 4;
   const auto put = [&](int j, float x, float y, float z, float w) {
     float* at = stg + (lane >> 4) * 4 * STG_LD + j * 16 + (lane & 15);
     at[0] = x;
@@ -310,11 +310,11 @@ __device__ __forceinline__ void stage_strip_w(const cf32x4 (&tiles)[NF], float* 
   if (add.n > 2) {   // all of them parked
     float4 v[NF];
 #pragma unroll
-    for (int j = 0; j < NF; ++j) v[j] = add.load(add.at + j * 4096u);
+    for (int j = 0; j < NF; ++j) v[j] = add.load(add.at + j * add.tile);
     for (int q = 1; q < add.n; ++q) {
       float4 o[NF];
 #pragma unroll
-      for (int j = 0; j < NF; ++j) o[j] = add.load(add.at + q * add.stride + j * 4096u);
+      for (int j = 0; j < NF; ++j) o[j] = add.load(add.at + q * add.stride + j * add.tile);
 #pragma unroll
       for (int j = 0; j < NF; ++j) {
         v[j].x += o[j].x; v[j].y += o[j].y; v[j].z += o[j].z; v[j].w += o[j].w;
@@ -325,7 +325,7 @@ __device__ __forceinline__ void stage_strip_w(const cf32x4 (&tiles)[NF], float* 
   } else if (add.n == 2) {
     float4 o[NF];
 #pragma unroll
-    for (int j = 0; j < NF; ++j) o[j] = add.load(add.at + j * 4096u);
+    for (int j = 0; j < NF; ++j) o[j] = add.load(add.at + j * add.tile);
 #pragma unroll
     for (int j = 0; j < NF; ++j)
       put(j, tiles[j][0] + o[j].x, tiles[j][1] + o[j].y, tiles[j][2] + o[j].z, tiles[j][3] + o[j].w);
@@ -524,12 +524,11 @@ template <int DT, int EPI, int NF> struct EpiW {
 };
 
 // a staged strip read out 8 lanes per row and written with the epilogue EPI
-template <int DT, int EPI, int NF, int B>
+template <int DT, int EPI, int NF, int B, int STG_LD = NF * 16 + 4>
 __device__ __forceinline__ void readout_strip_w(const GemmArgs& g, const float* stg, int m_strip0,
                                                 int vcol0, int split, int lane,
                                                 const EpiW<DT, EPI, NF>& ops) {
   using W = EpiW<DT, EPI, NF>;
-  constexpr int STG_LD = NF * 16 + 4;
   constexpr int CE = W::CE;
   // resid32: every chunk's residual requested before the first add / store (one memory
   // round trip per strip, not one per chunk: the stores could alias later loads)
@@ -1058,6 +1057,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_finalize(GemmArgs g, int spli
 #include "gemm_pp.h"
 #include "gemm_rs.h"
 #include "gemm_4w.h"
+#include "gemm_ws.h"
 
 namespace cake {
 

@@ -63,29 +63,46 @@ __global__ __launch_bounds__(256) void expert_route_kernel(const float* logits, 
   }
 }
 
-// Rows of a tile of the grouped products up (F columns) and down (W), of 256 columns on all CUs: the
-// height whose rounds cost least, by t = rounds (step k / 64 + end) us, at least the memory's.  Fitted to
-// seven expert sizes in even, independent and skewed groups of 60 .. 900 rows: 0.2 % off the best height
-// on the average, at most 6 %.  A height from the mean alone overflows its tiles: up and down of 64 experts
-// 2048 x 1856, 135 skewed rows each 291 us (192 rows a tile), 258 (256) by the counts; 240 even rows of
-// 4096 x 3648 1131 (160), 984 (256); 120 independent ones 898 at 256 rows, 780 at 160.
-constexpr int kHeights[4] = {128, 160, 192, 256};
+// Rows of a tile of the grouped products up (F columns) and down (W) on all CUs: the height whose rounds cost least.
+// A height from the mean alone overflows its tiles: up and down of 64 experts 2048 x 1856, 135 skewed rows each 291 us
+// (192 rows a tile), 258 (256) by the counts.
+//
+// Up rows of more than 1024 k take the tiles of gemm_ws.h: t = rounds (step k / 64 + end) us, at least the memory's (5.8
+// TB/s), a last round of less than an eighth of the CUs at less; of few tiles, of 128 columns, a share of the step.  Fitted
+// to 14 expert sizes in even, independent and skewed groups of 70 .. 600 rows: 0.2 % off the best height on the average.
+// Shorter ones the tiles of gemm_4w.h: t = rounds (step k / 64 + end), at least the memory's.
+constexpr int kHeights[4] = {160, 192, 224, 256}, kHeightsShort[4] = {128, 160, 192, 256};
+__device__ __forceinline__ int tile_rows(int W, int q) { return W > 1024 ? kHeights[q] : kHeightsShort[q]; }
+__device__ inline float height_us(int q, int tiles, int N, int K, float mem) {
+  constexpr float kStep[4] = {1.124f, 1.152f, 1.299f, 1.339f}, kEnd[4] = {5.53f, 7.80f, 7.07f, 8.42f};
+  const bool few = tiles * ((N + 255) / 256) <= (q == 0 ? 128 : 64);   // (gemm_inst_grouped.hip)
+  const int body = few && q > 0 ? 3 : q;
+  const float r = tiles * (few ? (N + 127) / 128 : (N + 255) / 256) / 256.f, whole = floorf(r), part = r - whole;
+  const float rounds = whole + (part > 0.f ? fminf(1.f, 0.82f + 1.42f * part) : 0.f);
+  return fmaxf(rounds * (kStep[body] * (few ? 0.448f : 1.f) * ((K + 63) / 64) + kEnd[body] * (few ? 1.54f : 1.f)), mem);
+}
 __device__ inline int tile_height(const int (&tiles)[4], int E, int M, int F, int W) {
   constexpr float kStep[4] = {1.106f, 1.161f, 1.38f, 1.547f}, kEnd[4] = {5.4f, 7.76f, 8.64f, 11.64f};
-  const float mem = ((float)E * F * W + (float)M * (F + W)) * 2 / 8.2e6f;
+  const bool ws = W > 1024;
+  const float mem = ((float)E * F * W + (float)M * (F + W)) * 2 / (ws ? 5.8e6f : 8.2e6f);
   int best = 0;
   float least = 0.f;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int up = (tiles[q] * ((F + 255) / 256) + 255) / 256, down = (tiles[q] * ((W + 255) / 256) + 255) / 256;
-    const float us = fmaxf(up * (kStep[q] * ((W + 63) / 64) + kEnd[q]), mem) +
-                     fmaxf(down * (kStep[q] * ((F + 63) / 64) + kEnd[q]), mem);
+    float us;
+    if (ws) {
+      us = height_us(q, tiles[q], F, W, mem) + height_us(q, tiles[q], W, F, mem);
+    } else {
+      const int up = (tiles[q] * ((F + 255) / 256) + 255) / 256, down = (tiles[q] * ((W + 255) / 256) + 255) / 256;
+      us = fmaxf(up * (kStep[q] * ((W + 63) / 64) + kEnd[q]), mem) +
+           fmaxf(down * (kStep[q] * ((F + 63) / 64) + kEnd[q]), mem);
+    }
     if (q == 0 || us < least) {
       best = q;
       least = us;
     }
   }
-  return kHeights[best];
+  return tile_rows(W, best);
 }
 
 // Entries (token, k) sorted by expert: scale[p] = score of sorted row p, where[entry] = p; the tile
@@ -134,7 +151,7 @@ __global__ __launch_bounds__(1024) void expert_plan_kernel(const float* logits, 
   if (BM == 0) {   // tiles of every height, over all experts
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      int n = (c + kHeights[q] - 1) / kHeights[q];
+      int n = (c + tile_rows(W, q) - 1) / tile_rows(W, q);
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
       if ((tid & 63) == 0) atomicAdd(&fit[q], n);
@@ -477,7 +494,7 @@ CAKE_API int cake_expert_route(const float* logits, long long ldl, int N, int E,
 CAKE_API int cake_expert_plan(const int* ids, const float* score, int N, int top, int E, int BM, int F,
                               int W, float* scale, int* where, void* tiles, int max_tiles, hipStream_t st) {
   if (!routing_ok(E, top) || N <= 0 || BM < 0 || (BM == 0 && (F <= 0 || W <= 0)) ||
-      max_tiles < (long long)N * top / (BM > 0 ? BM : kHeights[0]) + (E < (long long)N * top ? E : N * top))
+      max_tiles < (long long)N * top / (BM > 0 ? BM : kHeightsShort[0]) + (E < (long long)N * top ? E : N * top))
     return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL((expert_plan_kernel<0>), dim3(1), dim3(1024), 0, st, nullptr, 0, ids, score, N, top, E, BM, F, W,
                      scale, where, (int4*)tiles, max_tiles);
@@ -489,7 +506,7 @@ CAKE_API int cake_expert_route_plan(const float* logits, long long ldl, int N, i
                                     float* scale, int* where, void* tiles, int max_tiles, hipStream_t st) {
   if (!routing_ok(E, top) || N <= 0 || ldl < E || BM < 0 || (BM == 0 && (F <= 0 || W <= 0)) ||
       (long long)N * top > kPlanEntries ||
-      max_tiles < N * top / (BM > 0 ? BM : kHeights[0]) + (E < N * top ? E : N * top))
+      max_tiles < N * top / (BM > 0 ? BM : kHeightsShort[0]) + (E < N * top ? E : N * top))
     return (int)hipErrorInvalidValue;
 #define CAKE_PLAN(VPL)                                                                                           \
   hipLaunchKernelGGL((expert_plan_kernel<VPL>), dim3(1), dim3(1024), 0, st, logits, ldl, nullptr, nullptr, N, top, E, \

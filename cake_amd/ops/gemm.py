@@ -604,10 +604,10 @@ def slab_attn(ws, n: int, out: torch.Tensor, heads: int, inv_freq, kc, vc, scale
                                 current_stream()), "slab_attn")
 
 
-# tile configuration of a grouped product -> its rows (ROWS: the stream form; BY_LIST: 128, 160, 192 or 256,
+# tile configuration of a grouped product -> its rows (ROWS: the stream form; BY_LIST: 128 to 256,
 # as the last entry of the tile list says: chosen on the device from the groups' sizes)
 ROWS, BY_LIST = 32, 6
-GROUPED_CFGS = {0: 128, 1: 160, 2: 192, 4: 64, 5: 256, BY_LIST: 128, ROWS: 16}
+GROUPED_CFGS = {0: 128, 1: 160, 2: 192, 3: 224, 4: 64, 5: 256, BY_LIST: 128, ROWS: 16}
 
 
 def grouped_cfg(rows: int, groups: int, capturing: bool = False, weight: int = 0) -> int:
