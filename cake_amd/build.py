@@ -79,7 +79,8 @@ HIP_EXTRA = {"gemm": ["-mllvm", "-inline-threshold=100000"]}  # gemm.hip and gem
 NO_SPILL = {"flash_attn": "flash3_fwd_kernel", "mixer_attn": "mixer_flash3_kernel",
             "mixer_latent": "mixer_flash3_kernel"}
 # ... and in gemm_ws.h (an SGPR may go to a lane of a VGPR there: no result waits for that)
-NO_SPILL_TILES = {"gemm_inst_grouped": "gemm_groups_kernel"}
+NO_SPILL_TILES = {"gemm_inst_grouped": "gemm_groups_kernel", "gemm_inst_ws_bf16": "gemm_ws_kernel",
+                  "gemm_inst_ws_f16": "gemm_ws_kernel"}
 
 
 def check_spills(remarks: str, kernel: str, scalars: bool = True) -> None:

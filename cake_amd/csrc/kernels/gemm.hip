@@ -212,8 +212,8 @@ static constexpr TileCost kTileCosts[] = {
     {12, 64, 128, 2, 0.935f, 0.855f, -0.0328f, -0.0607f, 0.104f, {2.788f, 2.795f, 2.913f, 3.841f, -1.f, -1.f, -1.f}, 2.088f, 0.287f},
     {13, 64, 64, 2, 0.356f, 0.547f, 0.1f, 0.0549f, 0.00984f, {0.416f, 0.656f, 0.489f, 1.683f, -1.f, -1.f, -1.f}, 2.649f, 0.448f},
     {18, 64, 160, 1, 1.177f, 0.457f, 0.00266f, 0.1f, 0.0426f, {4.479f, 4.01f, -1.f, 4.044f, -1.f, -1.f, -1.f}, 1.721f, 0.209f},
-    {22, 256, 256, 1, 1.152f, 1.098f, 0.0174f, 0.128f, 0.176f, {9.638f, 16.22f, 10.07f, 19.8f, -1.f, -1.f, -1.f}, 13.95f, 7.829f},
-    {25, 256, 256, 1, 0.661f, 1.093f, 0.0424f, 0.209f, 0.0386f, {15.45f, 18.81f, 8.939f, 14.98f, -1.f, -1.f, -1.f}, 1.337f, 9.021f},
+    {22, 256, 256, 1, 1.152f, 1.098f, 0.0174f, 0.128f, 0.176f, {9.638f, -1.f, 10.07f, 19.8f, -1.f, -1.f, -1.f}, 13.95f, 7.829f},
+    {25, 256, 256, 1, 0.661f, 1.093f, 0.0424f, 0.209f, 0.0386f, {15.45f, -1.f, 8.939f, 14.98f, -1.f, -1.f, -1.f}, 1.337f, 9.021f},
     {26, 256, 192, 1, 0.12f, 0.916f, 0.0398f, 0.127f, 0.125f, {8.747f, 12.5f, 9.162f, 13.78f, -1.f, -1.f, -1.f}, 6.793f, 3.485f},
     {27, 128, 256, 1, 0.489f, 0.657f, 0.11f, 0.169f, 0.113f, {4.901f, 7.49f, 4.916f, 11.28f, -1.f, -1.f, -1.f}, 3.05f, 3.666f},
     {28, 128, 128, 1, 0.564f, 0.443f, 0.0724f, 0.0141f, 0.119f, {3.183f, 3.551f, 3.063f, 6.329f, -1.f, -1.f, -1.f}, 1.816f, 2.725f},
@@ -222,8 +222,8 @@ static constexpr TileCost kTileCosts[] = {
     {31, 160, 256, 1, 0.797f, 0.711f, 0.0445f, 0.0764f, 0.127f, {7.909f, 11.57f, 7.589f, 13.52f, -1.f, -1.f, -1.f}, 9.75f, 3.796f},
     {32, 192, 192, 1, 1.316f, 0.62f, 0.0623f, 0.0716f, 0.127f, {7.468f, 10.46f, 6.705f, 11.87f, -1.f, -1.f, -1.f}, 4.369f, 3.521f},
     {33, 224, 192, 1, 0.846f, 0.777f, 0.0146f, -0.0934f, 0.144f, {10.04f, 12.63f, 8.565f, 13.22f, -1.f, -1.f, -1.f}, 0.812f, 3.47f},
-    {34, 192, 256, 1, 1.768f, 0.979f, 0.0472f, 0.0879f, 0.126f, {6.113f, 10.06f, 6.451f, 13.14f, -1.f, -1.f, -1.f}, 2.423f, 4.585f},
-    {35, 224, 256, 1, 1.053f, 1.076f, 0.045f, 0.148f, 0.113f, {7.659f, 11.94f, 7.822f, 13.64f, -1.f, -1.f, -1.f}, 6.25f, 4.798f},
+    {34, 192, 256, 1, 1.768f, 0.979f, 0.0472f, 0.0879f, 0.126f, {6.113f, -1.f, 6.451f, 13.14f, -1.f, -1.f, -1.f}, 2.423f, 4.585f},
+    {35, 224, 256, 1, 1.053f, 1.076f, 0.045f, 0.148f, 0.113f, {7.659f, -1.f, 7.822f, 13.64f, -1.f, -1.f, -1.f}, 6.25f, 4.798f},
     // between 160 and 256 rows a tile the next larger one is padding and the next smaller one a partial wave
     // more: of 2,275 products these are taken for a twelfth, 8 % faster each (SwiGLU of 777 x 28672 x 4096 172
     // us on 192 x 192, 162 on 160 x 192; 777 x 4096 x 14336 98 in three pieces of 160 x 256, 93 in two of 224 x
@@ -231,6 +231,12 @@ static constexpr TileCost kTileCosts[] = {
     {36, 160, 192, 1, 1.492f, 0.68f, 0.019f, 0.f, 0.162f, {6.568f, 8.877f, 5.377f, 9.642f, -1.f, -1.f, -1.f}, 3.255f, 2.515f},
     {37, 160, 128, 1, 0.744f, 0.511f, 0.032f, 0.f, 0.163f, {5.184f, 7.988f, 4.123f, 7.683f, -1.f, -1.f, -1.f}, 3.312f, 3.9f},
     {38, 224, 128, 1, 0.259f, 0.64f, 0.017f, 0.f, 0.162f, {6.65f, 10.33f, 5.431f, 11.4f, -1.f, -1.f, -1.f}, 1.852f, 3.237f},
+    // f32 results on the tiles of gemm_ws.h, of 180 products (2048 .. 8192 columns, k 4096 .. 28672, 100 .. 6000 rows):
+    // 0.3 % off the best of all, 2.5 % faster than without them on the average, 5 to 16 % from 1300 rows on
+    {22, 256, 256, 1, 7.023f, 1.101f, 0.0578f, -0.3914f, 0.1106f, {-1.f, 12.87f, -1.f, -1.f, -1.f, -1.f, -1.f}, 1.22f, 5.201f},
+    {25, 256, 256, 1, 7.023f, 1.101f, 0.0578f, -0.3914f, 0.1106f, {-1.f, 12.87f, -1.f, -1.f, -1.f, -1.f, -1.f}, 1.22f, 5.201f},
+    {34, 192, 256, 1, 6.121f, 0.9357f, 0.0341f, -0.3562f, 0.1039f, {-1.f, 1.538f, -1.f, -1.f, -1.f, -1.f, -1.f}, 3.788f, 5.132f},
+    {35, 224, 256, 1, 6.214f, 1.06f, 0.0249f, -0.5244f, 0.0906f, {-1.f, 8.137f, -1.f, -1.f, -1.f, -1.f, -1.f}, 4.135f, 5.723f},
     // products of image models: the classes from kImageClass on
     {4, 64, 64, 4, 1.48f, 0.787f, 0.f, 0.263f, 0.f, {-1.f, -1.f, -1.f, -1.f, 3.44f, 2.92f, 3.04f}, -1.f, 0.f},
     {5, 256, 256, 1, 0.69f, 1.43f, 0.f, 0.f, 0.f, {-1.f, -1.f, -1.f, -1.f, 11.7f, 9.55f, 8.55f}, 4.16f, 0.304f},
@@ -337,7 +343,7 @@ CAKE_API int cake_gemm_plan(int M, long long Nv, int K, int epi, int big, int* c
 }
 
 // counters of tick below
-CAKE_API int cake_gemm_ticks() { return 2 * kPieceTiles; }
+CAKE_API int cake_gemm_ticks() { return 2 * kPieceTiles * kPieceWaves; }
 
 // y = epilogue(x W^T).  N = output features (gated: W has 2N rows, gate rows
 // [0, N), up/gate-2 rows [N, 2N)).  splits > 1 needs ws (cake_gemm_ws_floats) and, for a four-wave

@@ -1066,8 +1066,28 @@ constexpr bool gated_ok(int wave_cols) {
   return wave_cols % 32 == 0 || !(EPI == kEpiSwiglu || EPI == kEpiGeglu);
 }
 
+// The tiles of 192 rows and more whose f32 results gemm_ws.h runs, whole or in pieces (gemm_inst_ws_*.hip).
+constexpr bool ws_epi(int epi) { return epi == kEpiResid32 || epi == kEpiStore32; }
+constexpr bool ws_cfg(int cfg) { return cfg == k4WCfg || cfg == k4WCfg + k4WSched || cfg == 34 || cfg == 35; }
+template <int DT, int EPI>
+int launch_ws(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
+#define CAKE_LAUNCH_WS(BM)                                                                                     \
+  hipLaunchKernelGGL((gemm_ws_kernel<DT, EPI, BM, 256>), dim3(grid.x < 256 ? grid.x : 256),                     \
+                     dim3(WsTile<BM, 256>::THREADS), 0, st, g)
+  if (cfg == 34) CAKE_LAUNCH_WS(192);
+  else if (cfg == 35) CAKE_LAUNCH_WS(224);
+  else CAKE_LAUNCH_WS(256);
+#undef CAKE_LAUNCH_WS
+  return (int)hipGetLastError();
+}
+#define CAKE_WS_EXTERN(DT, E) extern template int launch_ws<DT, E>(int, dim3, hipStream_t, const GemmArgs&);
+CAKE_WS_EXTERN(kBF16, kEpiResid32) CAKE_WS_EXTERN(kBF16, kEpiStore32)
+CAKE_WS_EXTERN(kF16, kEpiResid32) CAKE_WS_EXTERN(kF16, kEpiStore32)
+#undef CAKE_WS_EXTERN
+
 // PCS: some tiles run in pieces (GemmArgs::pieces)
 #define CAKE_LAUNCH_4W(ID, BM, BN, WM, WN, SCHED)                                                      \
+  if constexpr (!(ws_epi(EPI) && ws_cfg(ID)))                                                  \
   if (cfg == ID) {                                                                             \
     hipLaunchKernelGGL((gemm_4w_kernel<DT, EPI, BM, BN, SCHED, PCS>), grid, dim3(256),  \
                        0, st, g);                                                              \
@@ -1092,6 +1112,8 @@ CAKE_TILES_EXTERN_ALL(kF16)
 
 template <int DT, int EPI, bool PCS>
 int launch_4w(int cfg, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  if constexpr (ws_epi(EPI))
+    if (ws_cfg(cfg)) return launch_ws<DT, EPI>(cfg, grid, st, g);
   // (a four-wave tile's k split is its pieces: no partial slabs)
   if constexpr (EPI != kEpiPartial) {
     CAKE_LAUNCH_4W(k4WCfg, 256, 256, 2, 2, 0)

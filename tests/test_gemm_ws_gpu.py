@@ -95,3 +95,28 @@ def test_height_of_the_groups(cuda, counts, F, W):
     costs = _height(counts, F, W)
     assert bm in [b for c, b in costs if c <= min(costs)[0] * (1 + 1e-4)]
     assert p.tiles[:n].tolist() == _tiles(counts, bm)
+
+
+# f32 results: fewer tiles than workgroups and more, pieces alone and behind whole tiles, bias and factor
+@pytest.mark.parametrize("dt", list(SIZE), ids=str)
+@pytest.mark.parametrize("cfg", [22, 25, 34, 35])
+@pytest.mark.parametrize("M,N,K,splits", [(1, 8, 64, 1), (700, 1000, 448, 3), (1500, 12300, 192, 1), (2100, 8200, 512, 2)])
+@pytest.mark.parametrize("epi", ["resid32", "store32"])
+def test_f32_results(cuda, dt, cfg, M, N, K, splits, epi):
+    """f32 sums of 16-bit products in two orders: K 2^-21 of the scale, twice that with the factor; the same bits
+    every time, and a second launch finds clean counters."""
+    from cake_amd.ops import gemm as G
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(dt)
+    w = torch.empty(N, K, device="cuda", dtype=dt).normal_(0, K ** -0.5, generator=g)
+    bias = torch.randn(N, device="cuda", generator=g).to(dt)
+    y = 0.5 * (x.float() @ w.float().t() + bias.float())
+    outs = []
+    for _ in range(3):
+        r = torch.full((M, N + 4), 3.0, device="cuda")
+        G.linear(x, w, bias, epi=epi, resid=r[:, :N], alpha=0.5, cfg=cfg, splits=splits)
+        assert bool((r[:, N:] == 3.0).all())
+        outs.append(r)
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    want = y + 3.0 if epi == "resid32" else y
+    assert bool(((outs[0][:, :N] - want).abs() <= K * 2.0 ** -20 + 2.0 ** -21 * want.abs()).all())
