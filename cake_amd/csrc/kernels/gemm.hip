@@ -510,7 +510,7 @@ CAKE_API int cake_gemm_rows_kind(int M, long long Nv, int K, int gated) {
 
 // stream form: f32 elements of ws (two parked strips per share) and counters of tick
 CAKE_API long long cake_gemm_rows_ws_floats(int M) { return 256LL * 4096 * ((M + 15) / 16); }
-CAKE_API int cake_gemm_rows_ticks() { return kRowsTicks; }
+CAKE_API int cake_gemm_rows_ticks() { return 4 * kRowsTicks; }
 
 // cake_gemm_scaled for M <= 64 rows in the form `kind` (1 or 2).  The stream form needs ws
 // (cake_gemm_rows_ws_floats) and tick (cake_gemm_rows_ticks zeros, zero again when the launch is
