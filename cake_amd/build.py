@@ -148,7 +148,7 @@ def _kernel_sources() -> dict[Path, list[Path]]:
     measured slower than the launch path: profiles/r4_mk_summary.md) only with
     CAKE_BUILD_EXPERIMENTAL=1."""
     hip = sorted((CSRC / "kernels").glob("*.hip"))
-    gemm = [p for p in hip if p.stem in ("gemm", "gemm_slabs") or p.stem.startswith("gemm_inst")]
+    gemm = [p for p in hip if p.stem in ("gemm", "gemm_slabs", "gemm_few") or p.stem.startswith("gemm_inst")]
     mixers = [p for p in hip if p.stem.startswith("mixer_")]
     rest = [p for p in hip if p not in gemm and p not in mixers]
     rest += sorted((CSRC / "driver").glob("*.cpp"))

@@ -11,7 +11,8 @@
 //
 // Of few rows the q/k/v, output and down products leave their sums in slabs, which the rotation and the next
 // norm add up (a block of 8B at 45 rows 122 us, 116 so); of a prompt's first rows the rotation and the attention
-// are one launch too: seven a block instead of up to eleven.
+// are one launch too: seven a block instead of up to eleven.  Of up to eight narrow rows the gated product norms them
+// itself: six.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -43,6 +44,10 @@ int cake_slab_rope(int dt, const float* ws, int slabs, void* q, int ldq, int T, 
                    const float* inv_freq, int pos0, int S, void* kc, void* vc, hipStream_t st);
 int cake_slab_attn(int dt, const float* ws, int slabs, void* out, long long ldo, int T, int nh, int nkv, int hd,
                    const float* inv_freq, int S, void* kc, void* vc, float scale, hipStream_t st);
+int cake_gemm_few_add(int dt, const void* a, long long lda, const void* b, long long ldb, float* r, long long ldr, int M,
+                      int N, int K, hipStream_t st);
+int cake_gemm_few_gated(int dt, const float* h, long long ldh, const void* ln, float eps, const void* b, long long ldb,
+                        void* c, long long ldc, int M, int N, int K, hipStream_t st);
 }
 
 namespace {
@@ -74,6 +79,7 @@ struct CakeBlockRun {
   Form kv_form, q1_form, o1_form, gu1_form, down1_form;   // of the last block, with a tail
   int n, dt, T, H, I, nh, nkv, hd, S, pos0;
   int tail;                     // rows of the result that are wanted, the last ones (0: all)
+  int few, few1;                // output and gate / up products as cake_gemm_few_*; of the last block, with a tail
   float eps, scale;
 };
 
@@ -123,6 +129,11 @@ struct Run {
     }
     const int e = product(f, kEpiResid32, a, w, nullptr, 0, r->H, K);
     return e || !ln ? e : cake_rmsnorm(r->dt, hidden, ln, r->eps, T, r->H, x, st);
+  }
+  // hidden += att wo^T, act = the gated product of its norm: up to eight rows
+  int few(const Block& b) const {
+    const int e = cake_gemm_few_add(r->dt, r->att, nq, b.wo, nq, hidden, r->H, T, r->H, nq, st);
+    return e ? e : cake_gemm_few_gated(r->dt, hidden, r->H, b.ln2, r->eps, b.wgu, r->H, r->act, r->I, T, r->I, r->H, st);
   }
   // rotated heads in qkv (q), keys and values in the cache
   int project(const Block& b) const {
@@ -185,8 +196,12 @@ CAKE_API int cake_block_rows(const CakeBlockRun* r, hipStream_t st) {
       e = tail ? g.project_tail(b) : g.project(b);
       if (!e) e = g.attend(b);
     }
-    if (!e) e = g.add_norm(o, r->att, b.wo, g.nq, b.ln2);
-    if (!e) e = g.product(gu, kEpiSwiglu, g.x, b.wgu, r->act, r->I, r->I, r->H);
+    if (tail ? r->few1 : r->few) {
+      if (!e) e = g.few(b);
+    } else {
+      if (!e) e = g.add_norm(o, r->att, b.wo, g.nq, b.ln2);
+      if (!e) e = g.product(gu, kEpiSwiglu, g.x, b.wgu, r->act, r->I, r->I, r->H);
+    }
     if (!e) e = g.add_norm(down, r->act, b.wd, r->I, last ? nullptr : r->blocks[i + 1].ln1);
   }
   return e;

@@ -385,12 +385,18 @@ class LayerStack:
             Tk = pos0 + T
             K.flash_attn(q.view(1, T, nh, hd).transpose(1, 2), kc[None, :, :Tk], vc[None, :, :Tk],
                          att.view(1, T, nh, hd).transpose(1, 2), self.scale, causal=True, pos0=pos0)
-        if f_o:
-            G.slab_norm(*G.slabs(att, w.wo, f_o), hidden, w.ln2, cfg.rms_norm_eps, x)
+        if G.few_pair(T, H, nq, inter) and all(t.is_contiguous() and t.data_ptr() % 16 == 0
+                                               for t in (hidden, w.wo, w.ln2, w.wgu)):
+            G.few_add(att, w.wo, hidden)                      # hidden += att @ wo^T
+            act = G.few_gated(hidden, w.ln2, cfg.rms_norm_eps, w.wgu,
+                              torch.empty((T, inter), device=hidden.device, dtype=self.dtype))
         else:
-            G.linear(att, w.wo, epi="resid32", resid=hidden)      # hidden += att @ wo^T
-            K.rmsnorm(hidden, w.ln2, cfg.rms_norm_eps, x)
-        act = G.linear(x, w.wgu, epi="swiglu")                # silu(x wg^T) * (x wu^T)
+            if f_o:
+                G.slab_norm(*G.slabs(att, w.wo, f_o), hidden, w.ln2, cfg.rms_norm_eps, x)
+            else:
+                G.linear(att, w.wo, epi="resid32", resid=hidden)      # hidden += att @ wo^T
+                K.rmsnorm(hidden, w.ln2, cfg.rms_norm_eps, x)
+            act = G.linear(x, w.wgu, epi="swiglu")                # silu(x wg^T) * (x wu^T)
         if f_down:
             G.slab_norm(*G.slabs(act, w.wd, f_down), hidden, w.ln1, cfg.rms_norm_eps, None)
         else:

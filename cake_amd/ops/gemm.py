@@ -102,6 +102,12 @@ def _lib():
         lib.cake_slab_rope.restype = I
         lib.cake_slab_attn.argtypes = [I, P, I, P, L, I, I, I, I, P, I, P, P, C.c_float, P]
         lib.cake_slab_attn.restype = I
+        lib.cake_gemm_few_pair.argtypes = [I, I, I, L]
+        lib.cake_gemm_few_pair.restype = I
+        lib.cake_gemm_few_add.argtypes = [I, P, L, P, L, P, L, I, I, I, P]
+        lib.cake_gemm_few_add.restype = I
+        lib.cake_gemm_few_gated.argtypes = [I, P, L, P, C.c_float, P, L, P, L, I, I, I, P]
+        lib.cake_gemm_few_gated.restype = I
         lib.cake_gemm_sections_gain.argtypes = [I, I, I, I, I]
         lib.cake_gemm_sections_gain.restype = I
         lib.cake_gemm_rows_sections.argtypes = [I, P, L, P, L, P, L, P, L, P, L, I, I, P, P, P, I, I,
@@ -194,6 +200,36 @@ def slab_form(M: int, N: int, K: int, epi: str, big: bool = False):
                                        C.addressof(p))
         f = _slab_forms[key] = (k.value, c.value, p.value) if on else None
     return f
+
+
+def few_pair(M: int, H: int, K: int, inter: int) -> bool:
+    """Whether a block's output product (rows of K to H, added to the residual rows) and its gated product of the
+    normed rows (H to `inter`) run as :func:`few_add` and :func:`few_gated` (gemm_few.hip); pinned plans run as pinned."""
+    return (M, H, K, "resid32") not in _plans and (M, 2 * inter, H, "swiglu") not in _plans and \
+        bool(_lib().cake_gemm_few_pair(M, H, K, inter))
+
+
+def few_add(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor) -> None:
+    """resid [M, N] f32 += x [M, K] w^T of up to eight rows."""
+    (M, K), N = x.shape, w.shape[0]
+    if x.dtype not in _DT or w.dtype != x.dtype or resid.dtype != torch.float32 or w.shape[1] != K or \
+            tuple(resid.shape) != (M, N) or x.stride(1) != 1 or w.stride(1) != 1 or resid.stride(1) != 1:
+        raise ValueError("few_add: 16-bit rows and weights, f32 sums of their shapes expected")
+    check(_lib().cake_gemm_few_add(_DT[x.dtype], x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
+                                   resid.data_ptr(), resid.stride(0), M, N, K, current_stream()), "few_add")
+
+
+def few_gated(h: torch.Tensor, ln: torch.Tensor, eps: float, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """out [M, N] = silu(x w[:N]^T) (x w[N:]^T), x the RMS norm of h [M, K] f32 with weights ln, of up to eight rows."""
+    (M, K), N = h.shape, w.shape[0] // 2
+    if w.dtype not in _DT or ln.dtype != w.dtype or out.dtype != w.dtype or h.dtype != torch.float32 or \
+            tuple(w.shape) != (2 * N, K) or tuple(ln.shape) != (K,) or tuple(out.shape) != (M, N) or \
+            h.stride(1) != 1 or w.stride(1) != 1 or out.stride(1) != 1 or not ln.is_contiguous():
+        raise ValueError("few_gated: f32 rows, 16-bit weights and output of their shapes expected")
+    check(_lib().cake_gemm_few_gated(_DT[w.dtype], h.data_ptr(), h.stride(0), ln.data_ptr(), float(eps),
+                                     w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), M, N, K,
+                                     current_stream()), "few_gated")
+    return out
 
 
 def _counters(dev, st: int) -> torch.Tensor:

@@ -24,7 +24,8 @@ class _Run(C.Structure):
                                  "ws", "slabs", "rows_ws", "tick")] + \
                [(n, _Form) for n in ("qkv_form", "o_form", "gu_form", "down_form", "kv_form", "q1_form",
                                      "o1_form", "gu1_form", "down1_form")] + \
-               [(n, I) for n in ("n", "dt", "T", "H", "I", "nh", "nkv", "hd", "S", "pos0", "tail")] + \
+               [(n, I) for n in ("n", "dt", "T", "H", "I", "nh", "nkv", "hd", "S", "pos0", "tail", "few",
+                              "few1")] + \
                [("eps", F), ("scale", F)]
 
 
@@ -133,6 +134,7 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
     ptr = [None if t is None else t.data_ptr() for t in (
         hidden, x, qkv, att, act, inv_freq, G._zeros16(dev), ws, slabs, rows_ws, tick)]
     run = _Run(C.addressof(table), *ptr, *forms, len(blocks), G._DT[dt], T, H, inter, nh, nkv, hd, S,
-               int(pos0), int(tail), float(cfg.rms_norm_eps), float(scale))
+               int(pos0), int(tail), int(G.few_pair(T, H, nq, inter)), int(G.few_pair(tail, H, nq, inter)),
+               float(cfg.rms_norm_eps), float(scale))
     check(kernels().cake_block_rows(C.addressof(run), st), "block_rows")
     return True
