@@ -11,10 +11,53 @@
 
 namespace cake {
 
-template <int DT, int U, int PFC, int NX>
-__global__ __launch_bounds__(kGemvThreads) void mixer_in_kernel(MixInArgs a) {
+template <int DT, int U, int PFC, int NX, int NT = kGemvThreads>
+__global__ __launch_bounds__(NT) void mixer_in_kernel(MixInArgs a) {
   extern __shared__ float xs[];
-  mixer_in_rows<DT, U, PFC, NX, kGemvThreads>(a, blockIdx.x, gridDim.x, xs);
+  mixer_in_rows<DT, U, PFC, NX, NT>(a, blockIdx.x, gridDim.x, xs);
+}
+
+// Few rows (a router's): a workgroup has one pair of them, each of its waves a quarter of k.  With a pair a wave, the
+// workgroups are as few as the rows are, and one CU reads 64 KB at 25 KB a us (64 / 512 / 1024 rows of 4096 4.9 / 5.4 /
+// 5.6 us, 3.2 / 4.0 / 4.5 so; 2048 6.6, 6.4; of 2048 columns 64 / 1024 3.5 / 3.9, 2.7 / 3.6, 4096 5.6, 6.2).
+template <int DT, int PFC, int NX>
+__global__ __launch_bounds__(kGemvThreads) void mixer_in_split_kernel(MixInArgs a) {
+  extern __shared__ float xs[];
+  __shared__ float part[2][kGemvWaves];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nch = a.K >> 3;
+  const uint4* wa = reinterpret_cast<const uint4*>(a.w + (size_t)(2 * blockIdx.x) * a.K);
+  const uint4* wb = reinterpret_cast<const uint4*>(a.w + (size_t)min(2 * (int)blockIdx.x + 1, a.N - 1) * a.K);
+  NormPre<DT, NX> xp;
+  xp.load(a.resid, a.norm_w, a.K);
+  __builtin_amdgcn_sched_barrier(0);
+  uint4 va[PFC], vb[PFC];
+#pragma unroll
+  for (int c = 0; c < PFC; ++c) {
+    const int i = min((c * kGemvWaves + wave) * 64 + lane, nch - 1);
+    va[c] = wa[i];
+    vb[c] = wb[i];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  xp.finish_off(a.eps, a.K, a.Kn, a.off, a.ln, xs);
+  float da = 0.f, db = 0.f;
+#pragma unroll
+  for (int c = 0; c < PFC; ++c) {
+    const int i = (c * kGemvWaves + wave) * 64 + lane;
+    if (i < nch) fma_chunk<DT, true>(xs, i, va[c], vb[c], da, db);
+  }
+  da = wave_sum(da);
+  db = wave_sum(db);
+  if (lane == 0) {
+    part[0][wave] = da;
+    part[1][wave] = db;
+  }
+  __syncthreads();
+  const int r = 2 * blockIdx.x + threadIdx.x;
+  if (threadIdx.x > 1 || r >= a.N) return;
+  const float* q = part[threadIdx.x];
+  const float d = (q[0] + q[1]) + (q[2] + q[3]);
+  if (r < a.n_raw) a.out[r] = d;
+  else a.act[r - a.n_raw] = from_f32<DT>(mix_act(a.actf, a.bias ? d + to_f32<DT>(a.bias[r - a.n_raw]) : d));
 }
 
 // y[r] = x[r] + alpha ((W a)[r] + bias[r]), a 16-bit; bias may be null
@@ -112,6 +155,23 @@ CAKE_API int cake_mixer_in(int dt, const float* resid, const void* norm_w, float
   const int g = grid_for((N + 1) / 2, 1024);
   const MixInArgs a{resid, (const uint16_t*)norm_w, (const uint16_t*)w, out, (const uint16_t*)bias,
                     (uint16_t*)act, eps, off, ln, Kn, K, N, n_raw, actf};
+  // few rows: above; up to a workgroup a CU: all of a pair is asked for before the norm, and of a few more pairs than
+  // those take, five waves have one each, so that no CU has two workgroups (2048 / 2112 / 2560 rows of 4096 6.6 / 6.8 /
+  // 7.2 us, 5.9 / 6.0 / 6.5 so; 3072 on five waves 8.4, on four with the whole pair asked for 7.6, 7.4 as below)
+  if (K / 8 >= 128 && K <= 4096 && N <= 1024) {
+    const int gs = (N + 1) / 2;
+    DISPATCH_DT(dt, if (K <= 2048) CAKE_MIX_LAUNCH((mixer_in_split_kernel<DT, 1, 2>), gs, lds, a);
+                else CAKE_MIX_LAUNCH((mixer_in_split_kernel<DT, 2, 4>), gs, lds, a));
+  }
+  if (K == 4096 && N <= 2048) DISPATCH_DT(dt, CAKE_MIX_LAUNCH((mixer_in_kernel<DT, 2, 8, 4>), g, lds, a));
+  if (K >= 2048 && K <= 4096 && N > 2048 && N <= 2560) {
+    const int g5 = ((N + 1) / 2 + 4) / 5;
+#define CAKE_MIN5(PF)                                                                                        \
+  hipLaunchKernelGGL((mixer_in_kernel<DT, 2, PF, 4, 320>), dim3(g5), dim3(320), lds, st, a);                 \
+  return (int)hipGetLastError()
+    DISPATCH_DT(dt, if (K == 4096) { CAKE_MIN5(8); } else { CAKE_MIN5(4); });
+#undef CAKE_MIN5
+  }
 #define CAKE_MIN(PF, NX) CAKE_MIX_LAUNCH((mixer_in_kernel<DT, 2, PF, NX>), g, lds, a)
   DISPATCH_DT(dt, if (K / 8 < 128) CAKE_MIN(0, 0); else if (K / 8 < 256) CAKE_MIN(2, 2);
               else if (K <= 4096) CAKE_MIN(4, 4);

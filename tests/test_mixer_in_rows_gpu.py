@@ -1,0 +1,34 @@
+"""Input products of one token: few rows (a pair a workgroup), and up to a workgroup a CU."""
+import pytest
+import torch
+
+from cake_amd.ops import mixers as M
+
+pytestmark = pytest.mark.gpu
+
+
+# odd and even rows to either side of each rule's ends; columns of whole and ragged rounds
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("N", [1, 2, 65, 1024, 1025, 2048, 2049, 2560, 2561])
+@pytest.mark.parametrize("K", [1016, 1024, 1032, 2048, 2056, 3000, 4088, 4096])
+@pytest.mark.parametrize("ln", [False, True])
+def test_rows(cuda, dt, N, K, ln):
+    """f32 dot products of f32 normed rows in another order: K 2^-22 of the scale; the activated rows rounded once."""
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    x = 2 * torch.randn(K, device="cuda", generator=g) + 0.5
+    nw = torch.rand(K, device="cuda", generator=g).to(dt)
+    w = torch.empty(N, K, device="cuda", dtype=dt).normal_(0, K ** -0.5, generator=g)
+    n_raw = (N + 1) // 2
+    out = torch.full((n_raw + 4,), 5.0, device="cuda")
+    act = torch.full((N - n_raw + 4,), 5.0, device="cuda", dtype=dt)
+    M.layer_in(x, nw, 1e-5, 1.0, K, w, n_raw, out[:n_raw], act[:N - n_raw], ln=ln)
+    h = x.double() - (x.double().mean() if ln else 0)
+    h = h * torch.rsqrt(h.square().mean() + 1e-5) * (1 + nw.double())
+    want = w.double() @ h
+    tol = K * 2.0 ** -22 * (1 + want.abs())
+    assert bool(((out[:n_raw].double() - want[:n_raw]).abs() <= tol[:n_raw]).all()) and bool((out[n_raw:] == 5.0).all())
+    a = want[n_raw:]
+    a = torch.nn.functional.gelu(a)
+    size = 2.0 ** (-8 if dt == torch.bfloat16 else -11)
+    assert bool(((act[:N - n_raw].double() - a).abs() <= 2 * tol[n_raw:] + size * a.abs()).all())
+    assert bool((act[N - n_raw:] == 5.0).all())
