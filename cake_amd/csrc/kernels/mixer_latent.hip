@@ -216,14 +216,14 @@ struct LatDecArgs {
   long long slot_stride;
   const int* pos;        // [B]
   const int* slot;
-  int H, LD, RP, nsplit;
+  int H, LD, RP, nsplit, tile;
   float scale_log2;
   float* part;           // [B][H][nsplit][RP + 4]: value sums, running max (log2), sum
 };
 
-// keys per split (whole 64-key tiles) and the splits that hold any
-__device__ __forceinline__ int latent_split_keys(int Tk, int nsplit) {
-  return ((Tk + nsplit - 1) / nsplit + 63) / 64 * 64;
+// keys per split (whole tiles of 32 or 64 keys) and the splits that hold any
+__device__ __forceinline__ int latent_split_keys(int Tk, int nsplit, int tile) {
+  return ((Tk + nsplit - 1) / nsplit + tile - 1) / tile * tile;
 }
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -241,10 +241,12 @@ __device__ __forceinline__ uint4 load_cols(const uint16_t* rows, int ld, int l15
 }
 
 // RC: class of the latent size, BK: keys per tile
+// 16-byte pieces of a tile per thread
+template <int DT, int RC, int BK> constexpr int lat_pieces() { return DT != kF32 && RC <= 512 && BK == 32 ? 10 : 20; }
 template <int DT, int RC, int BK>
 __global__ __launch_bounds__(256) void latent_decode_kernel(LatDecArgs a) {
   using E = typename St<DT>::E;
-  constexpr int EPC = St<DT>::EPC, NB = BK / 16, NVT = RC / 64, NLD = 20;
+  constexpr int EPC = St<DT>::EPC, NB = BK / 16, NVT = RC / 64, NLD = lat_pieces<DT, RC, BK>();
   constexpr int PLD = BK + EPC;
   extern __shared__ __attribute__((aligned(16))) unsigned char mixer_smem[];
   __shared__ float red_m[4][16], red_l[4][16];
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatDecArgs a) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
   const int h0 = blockIdx.x * 16, nr = min(16, a.H - h0), sp = blockIdx.y, b = blockIdx.z;
   const int Tk = a.pos[b] + 1;
-  const int kps = latent_split_keys(Tk, a.nsplit);
+  const int kps = latent_split_keys(Tk, a.nsplit, a.tile);
   const int kbeg = sp * kps, kend = min(kbeg + kps, Tk);
   if (kbeg >= kend) return;
   const E* rows = reinterpret_cast<const E*>(a.cache) + a.slot[b] * a.slot_stride;
@@ -414,7 +416,7 @@ struct LatOutArgs {
   const float* part;
   const int* pos;
   const void* uv;        // [H][DVP][RP]
-  int H, vdim, DVP, RP, nsplit;
+  int H, vdim, DVP, RP, nsplit, tile;
   void* out;             // [B][ldo], head h at h vdim
   long long ldo;
 };
@@ -437,7 +439,7 @@ __global__ __launch_bounds__(256) void latent_out_kernel(LatOutArgs a) {
     for (int c = 0; c < NCH; ++c)
       w[i][c] = lane + 64 * c < nch ? src[lane + 64 * c] : make_uint4(0u, 0u, 0u, 0u);
   }
-  const int Tk = a.pos[b] + 1, kps = latent_split_keys(Tk, a.nsplit);
+  const int Tk = a.pos[b] + 1, kps = latent_split_keys(Tk, a.nsplit, a.tile);
   const int nact = (Tk + kps - 1) / kps;
   const float* part = a.part + ((long long)b * a.H + h) * a.nsplit * PS;
   if (wave == 0) {
@@ -491,7 +493,7 @@ static int launch_latent_decode(const LatDecArgs& a, dim3 grid, hipStream_t st) 
   constexpr int EPC = St<DT>::EPC;
   const size_t lds = ((size_t)(BK + 16) * (a.LD + EPC) + 16 * (BK + EPC)) *
                      sizeof(typename St<DT>::E);
-  if (BK * (a.LD / EPC) > 256 * 20 || lds > 150 * 1024) return (int)hipErrorInvalidValue;
+  if (BK * (a.LD / EPC) > 256 * lat_pieces<DT, RC, BK>() || lds > 150 * 1024) return (int)hipErrorInvalidValue;
   static bool raised = false;
   if (!raised) {
     if (hipFuncSetAttribute((const void*)latent_decode_kernel<DT, RC, BK>,
@@ -550,31 +552,38 @@ CAKE_API int cake_latent_absorb(int dt, const float* q, long long ldq, const voi
   return (int)hipGetLastError();
 }
 
+// tile: 32 or 64 keys, as cake_latent_out takes it.  A CU reads some 25 KB a us and a tile of 64 keys is 74 KB: the
+// attention and value expansion of one sequence of 32 heads over 40 / 150 / 250 keys 12.2 / 12.9 / 13.3 us in up to four
+// 64-key tiles, 11.0 / 12.0 / 12.3 in eight of 32; of 13 sequences 18.9 / 22.5 / 23.0, 20.0 / 23.1 / 25.3.
 CAKE_API int cake_latent_decode(int dt, const void* qa, const void* cache, long long slot_stride,
                                 const int* pos, const int* slot, int B, int H, int LD, int RP,
-                                int nsplit, float scale, float* part, hipStream_t st) {
+                                int nsplit, int tile, float scale, float* part, hipStream_t st) {
   if (B <= 0 || H <= 0 || LD % 32 || RP % 16 || RP <= 0 || RP > 1024 || LD < RP || nsplit < 1 ||
-      nsplit > 64)
+      nsplit > 64 || (tile != 32 && tile != 64))
     return (int)hipErrorInvalidValue;
-  const LatDecArgs a{qa, cache, slot_stride, pos, slot, H, LD, RP, nsplit,
+  const LatDecArgs a{qa, cache, slot_stride, pos, slot, H, LD, RP, nsplit, tile,
                      scale * 1.4426950408889634f, part};
   const dim3 grid((H + 15) / 16, nsplit, B);
   CAKE_MIX_DT(dt, {
     constexpr bool F = DT == kF32;
-    if (RP <= 256 && LD <= (F ? 384 : 640)) return launch_latent_decode<DT, 256, F ? 32 : 64>(a, grid, st);
-    if (RP <= 512 && LD <= 640) return launch_latent_decode<DT, 512, F ? 32 : 64>(a, grid, st);
+    if (RP <= 256 && LD <= (F ? 384 : 640))
+      return F || tile == 32 ? launch_latent_decode<DT, 256, 32>(a, grid, st)
+                                    : launch_latent_decode<DT, 256, 64>(a, grid, st);
+    if (RP <= 512 && LD <= 640)
+      return F || tile == 32 ? launch_latent_decode<DT, 512, 32>(a, grid, st)
+                                    : launch_latent_decode<DT, 512, 64>(a, grid, st);
     return launch_latent_decode<DT, 1024, F ? 16 : 32>(a, grid, st);
   });
   return (int)hipErrorInvalidValue;
 }
 
 CAKE_API int cake_latent_out(int dt, const float* part, const int* pos, const void* uv, int B,
-                             int H, int vdim, int DVP, int RP, int nsplit, void* out,
+                             int H, int vdim, int DVP, int RP, int nsplit, int tile, void* out,
                              long long ldo, hipStream_t st) {
   if (B <= 0 || H <= 0 || vdim <= 0 || DVP < vdim || RP % 16 || RP <= 0 || RP > 1024 ||
-      nsplit < 1 || nsplit > 64 || ldo < (long long)H * vdim)
+      nsplit < 1 || nsplit > 64 || (tile != 32 && tile != 64) || ldo < (long long)H * vdim)
     return (int)hipErrorInvalidValue;
-  const LatOutArgs a{part, pos, uv, H, vdim, DVP, RP, nsplit, out, ldo};
+  const LatOutArgs a{part, pos, uv, H, vdim, DVP, RP, nsplit, tile, out, ldo};
   const dim3 grid((vdim + kOutRows - 1) / kOutRows, H, B);
   CAKE_MIX_DT(dt, hipLaunchKernelGGL((latent_out_kernel<DT>), grid, dim3(256), 0, st, a));
   return (int)hipGetLastError();

@@ -38,6 +38,8 @@ SPLITS = ((256, 1), (1024, 8), (4096, 16), (1 << 30, 32))
 # the latent kernels' for the same buckets: a workgroup takes one 64-key tile while there are
 # splits for all of them
 LATENT_SPLITS = {n: min(M.MAX_SPLIT, -(-lim // 64)) for lim, n in SPLITS}
+# ... (splits, tile) of a sequence alone: of short contexts 32-key tiles
+LATENT_ALONE = {n: (8, 32) if n == 1 else (s, 64) for n, s in LATENT_SPLITS.items()}
 # Rows of a step from which on the last run's unread ones are left out (:meth:`HybridModel._last_rows`);
 # fewer go through the products of few rows, which read the weights once either way
 LAST_LEAST = 65
@@ -513,7 +515,7 @@ class HybridModel:
             ka, kb = self.pool.bufs[run.index]
             proj = b.proj[:w.n_raw].view(1, -1)
             if isinstance(m, LatentMixer):
-                self._latent_decode(m, w, b, proj, ka, mix.view(1, -1), LATENT_SPLITS[nsplit])
+                self._latent_decode(m, w, b, proj, ka, mix.view(1, -1), *LATENT_ALONE[nsplit])
             elif isinstance(m, AttentionMixer):
                 M.attn_decode(w.shape, proj, b.pos, b.seq_slot, self._rotation(m), m.qk_norm,
                               m.sink, m.gated, cfg.eps, m.scale, ka, kb, mix.view(1, -1), nsplit,
@@ -530,7 +532,7 @@ class HybridModel:
         return x
 
     def _latent_decode(self, m: LatentMixer, w, b: DecodeState, proj, cache, mix,
-                       nsplit: int) -> None:
+                       nsplit: int, tile: int) -> None:
         """Latent attention of one token: query expansion (norm in the prologue), query into the
         latent space + cache row, attention over the latent rows, merge + value expansion."""
         sh, c, eps = w.shape, w.consts, self.cfg.eps
@@ -539,8 +541,8 @@ class HybridModel:
         qa = b.lat_qa[:sh.heads * sh.LD]
         LA.absorb(sh, q.view(1, -1), c["uk_t"], b.pos, b.seq_slot, self._rotation(m), eps,
                   c["kv_norm"], cache, qa, proj=proj)
-        LA.decode(sh, qa, b.pos, b.seq_slot, cache, m.scale, nsplit, b.part)
-        LA.out(sh, b.part, b.pos, c["uv"], nsplit, mix)
+        LA.decode(sh, qa, b.pos, b.seq_slot, cache, m.scale, nsplit, b.part, tile)
+        LA.out(sh, b.part, b.pos, c["uv"], nsplit, mix, tile)
 
     def decode_head(self, b: DecodeState) -> None:
         from ...ops import hip as K

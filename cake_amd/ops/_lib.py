@@ -227,8 +227,8 @@ _LIB_SIGS = {
         "cake_latent_prep": [I, P, L, I, I, I, I, I, I, I, I, F, P, P, P, P, P, P, P, L, P],
         "cake_latent_absorb": [I, P, L, P, I, I, I, I, I, P, L, I, I, I, I, I, I, F, P, P, P, P, P,
                                L, P, P],
-        "cake_latent_decode": [I, P, P, L, P, P, I, I, I, I, I, F, P, P],
-        "cake_latent_out": [I, P, P, P, I, I, I, I, I, I, P, L, P],
+        "cake_latent_decode": [I, P, P, L, P, P, I, I, I, I, I, I, F, P, P],
+        "cake_latent_out": [I, P, P, P, I, I, I, I, I, I, I, P, L, P],
         "cake_latent_flash": [I, P, L, P, L, P, L, P, P, L, I, I, P, I, I, P, I, I, I, I, I, I, I,
                               F, P, L, P],
         "cake_expert_route": [P, L, I, I, I, P, P, P],

@@ -143,9 +143,9 @@ def absorb(sh: LatentShape, q, uk_t, pos, slot, cs, eps: float, kv_norm, cache, 
         "latent_absorb")
 
 
-def decode(sh: LatentShape, qa, pos, slot, cache, scale: float, nsplit: int, part):
-    """Attention of one token per sequence over its cache rows 0 .. pos, split over the keys;
-    the splits' sums go to part."""
+def decode(sh: LatentShape, qa, pos, slot, cache, scale: float, nsplit: int, part, tile: int = 64):
+    """Attention of one token per sequence over its cache rows 0 .. pos, split over the keys in whole tiles
+    of 32 or 64; the splits' sums go to part."""
     B = pos.shape[0]
     cp, _, _ = _cache(sh, cache, qa.dtype)
     if not 1 <= nsplit <= MAX_SPLIT:
@@ -153,16 +153,16 @@ def decode(sh: LatentShape, qa, pos, slot, cache, scale: float, nsplit: int, par
     check(_lib().cake_latent_decode(
         DT[qa.dtype], _vec(qa, "qa", qa.dtype, B * sh.heads * sh.LD), cp, cache.stride(0),
         _vec(pos, "pos", torch.int32, B), _vec(slot, "slot", torch.int32, B), B, sh.heads, sh.LD,
-        sh.RP, int(nsplit), float(scale),
+        sh.RP, int(nsplit), int(tile), float(scale),
         _vec(part, "part", torch.float32, sh.part_floats(B, nsplit)), _stream()), "latent_decode")
 
 
-def out(sh: LatentShape, part, pos, uv, nsplit: int, y):
+def out(sh: LatentShape, part, pos, uv, nsplit: int, y, tile: int = 64):
     """y [B, >= H vdim] = the value expansion uv [H, DVP, RP] of the merged splits."""
     B = pos.shape[0]
     yp, ldy = _mat(y, "y", y.dtype, B, sh.out_cols)
     check(_lib().cake_latent_out(
         DT[y.dtype], _vec(part, "part", torch.float32, sh.part_floats(B, nsplit)),
         _vec(pos, "pos", torch.int32, B), _vec(uv, "uv", y.dtype, sh.heads * sh.DVP * sh.RP), B,
-        sh.heads, sh.vdim, sh.DVP, sh.RP, int(nsplit), yp, max(ldy, sh.out_cols), _stream()),
+        sh.heads, sh.vdim, sh.DVP, sh.RP, int(nsplit), int(tile), yp, max(ldy, sh.out_cols), _stream()),
         "latent_out")
