@@ -40,6 +40,17 @@ SPLITS = ((256, 1), (1024, 8), (4096, 16), (1 << 30, 32))
 LATENT_SPLITS = {n: min(M.MAX_SPLIT, -(-lim // 64)) for lim, n in SPLITS}
 # ... (splits, tile) of a sequence alone: of short contexts 32-key tiles
 LATENT_ALONE = {n: (8, 32) if n == 1 else (s, 64) for n, s in LATENT_SPLITS.items()}
+
+
+def latent_splits(nsplit: int, rows: M.Rows, heads: int) -> int:
+    """Splits of a step's sequences: no more workgroups at the longest one's length than CUs, since the value expansion
+    reads every split's sums (16 heads of 24 sequences at 600 / 3000 keys 38.6 us in 16 splits / 70.4 in 32, 30.5 / 44.4 in
+    8; 32 heads of 13 at 1000 45.4 in 16, 30.4 in 8; 32 heads of 2 at 3000 24.4 in 32, 25.1 in 16, 31.1 in 8)."""
+    keys = [p0 + n for _, n, p0, _ in rows.host]
+    groups = -(-sum(keys) // max(keys)) * -(-heads // 16)   # as many sequences of the longest one's length
+    return min(LATENT_SPLITS[nsplit], 1 << max(1, 256 // groups).bit_length() - 1)
+
+
 # Rows of a step from which on the last run's unread ones are left out (:meth:`HybridModel._last_rows`);
 # fewer go through the products of few rows, which read the weights once either way
 LAST_LEAST = 65
@@ -226,7 +237,7 @@ class HybridModel:
                 self.product(h, w.w_in[w.n_main:w.n_raw], ab)
         a, b = self.pool.bufs[run.index]
         if isinstance(m, LatentMixer):
-            self._latent_rows(m, w, proj, rows, a, mix, LATENT_SPLITS[nsplit])
+            self._latent_rows(m, w, proj, rows, a, mix, latent_splits(nsplit, rows, w.shape.heads))
         elif isinstance(m, AttentionMixer):
             cs = self._rotation(m)
             if decode:
@@ -285,7 +296,8 @@ class HybridModel:
             M.attn_decode(w.shape, one, pos, slot, self._rotation(m), m.qk_norm, m.sink, m.gated,
                           cfg.eps, m.scale, a, b, mix, nsplit, part, ticket, held=True)
         elif isinstance(m, LatentMixer):
-            sh, c, cs, splits = w.shape, w.consts, self._rotation(m), LATENT_SPLITS[nsplit]
+            sh, c, cs = w.shape, w.consts, self._rotation(m)
+            splits = latent_splits(nsplit, rows, sh.heads)
             proj = torch.empty((N, w.n_main), device=dev, dtype=torch.float32)
             self.product(h, w.w_in[:w.n_main], proj)
             cq = torch.empty((N, sh.QP), device=dev, dtype=self.dtype)
