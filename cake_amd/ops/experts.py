@@ -54,11 +54,11 @@ class Plan:
 def _plan(N: int, top: int, E: int, dev, dtype, weight: int, up: int, launch) -> Plan:
     """launch(BM, up, wide, scale, where, tiles, number of tiles) fills the plan."""
     M = N * top
-    cfg = G.grouped_cfg(M, E, torch.cuda.is_current_stream_capturing(), weight)
-    bm = BM32 if dtype == torch.float32 else G.GROUPED_CFGS[cfg]   # the least, of a height yet to choose
-    n = M // bm + min(E, M)
     up = up or math.isqrt(weight or 1 << 22)
     wide = max(1, (weight or 1 << 22) // up)
+    cfg = G.grouped_cfg(M, E, torch.cuda.is_current_stream_capturing(), weight, wide)
+    bm = BM32 if dtype == torch.float32 else G.GROUPED_CFGS[cfg]   # the least, of a height yet to choose
+    n = M // bm + min(E, M)
     i32 = torch.empty(M + 4 * (n + 1) + 4, device=dev, dtype=torch.int32)
     where = i32[:M].view(N, top)
     at = M + -M % 4   # tiles are read whole, 16 bytes each

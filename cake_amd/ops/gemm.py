@@ -646,18 +646,23 @@ ROWS, BY_LIST = 32, 6
 GROUPED_CFGS = {0: 128, 1: 160, 2: 192, 3: 224, 4: 64, 5: 256, BY_LIST: 128, ROWS: 16}
 
 
-def grouped_cfg(rows: int, groups: int, capturing: bool = False, weight: int = 0) -> int:
+def grouped_cfg(rows: int, groups: int, capturing: bool = False, weight: int = 0, width: int = 0) -> int:
     """Tile configuration for `rows` sorted rows over `groups` weight groups of `weight` elements each
-    (0: small)."""
-    # up and down product of 64 experts 4096 x 3616, us in the stream form and at 64 / 128 rows
-    # a tile, by rows an expert: 3 561 / 651 / 646, 6 644 / 688 / 669, 9 680 / 705 / 672, 16 938 / 739 /
-    # 683, 24 - / 775 / 698, 75 - / 1275 / 766.  From 4 to 12 rows the 64-row tile loses 3 - 7 % here and
-    # is taken for the smaller experts' sake, of which it makes twice the workgroups: one product at 14
-    # rows, 64 / 128 rows a tile, by millions of weights in all: 17 14.4 / 17.6 (8 of 1024 x 2048 24.4 /
-    # 29.3), 34 18.5 / 20.3, 101 47.6 / 50.1, 215 equal, 268 128.6 / 128.2
+    (0: small), `width` columns of the rows (0: few)."""
     mean = rows / groups
     if mean <= 4 and not capturing:   # the stream form's counters stay out of graphs
         return ROWS
+    if width > 1024:
+        # up and down product, us in the stream form and at 64 / 128 rows a tile (gemm_ws.h's), by rows an expert: 64 of 3648 x
+        # 4096 4 564 / 627 / 560, 8 595 / 656 / 584, 16 881 / 674 / 600, 48 2067 / 766 / 656; of 1856 x 2048 4 156 / 197 / 154, 8
+        # 164 / 208 / 160, 16 243 / 212 / 164; 128 of 768 x 2048 8 135 / 183 / 158, 12 154 / 185 / 159, 16 215 / 189 / 162; 8 of
+        # 2048 x 4096 8 55 / 91 / 71, 16 80 / 91 / 71; 32 of 1024 x 2048 8 50 / 67 / 60, 12 67 / 68 / 60
+        if mean <= 8 and not capturing and groups * weight < 220_000_000:
+            return ROWS
+        return 0 if mean < 64 else BY_LIST
+    # rows of up to 1024 columns are on 64-row tiles or gemm_4w.h's: the smaller make twice the workgroups.  One product at 14
+    # rows, 64 / 128 rows a tile, by millions of weights in all: 17 14.4 / 17.6 (8 of 1024 x 2048 24.4 /
+    # 29.3), 34 18.5 / 20.3, 101 47.6 / 50.1, 215 equal, 268 128.6 / 128.2
     big = groups * weight >= 200_000_000
     if mean < (12 if big else 24):
         return 4
