@@ -20,7 +20,7 @@
 //   * mixer_delta_prep: convolution, SiLU and unit norms of a chunk's rows.
 //   * mixer_delta_chunk: per chunk and head T = (I + A)^-1, P_ij = G_ij (q_i.k_j), g, beta.
 //   * mixer_delta_scan: walks the chunks of one sequence.  A workgroup takes 16 columns of one
-//     head's S; its four waves hold a quarter of the rows each, as accumulators that are the
+//     head's S; four of its waves hold a quarter of the rows each, as accumulators that are the
 //     next chunk's B operands; the partial S0^T k, S0^T q meet in LDS once per chunk.
 //   * mixer_delta_out: gated norm of the read-outs.
 //   * mixer_delta_decode: all of it for one token per sequence in one launch.
@@ -199,25 +199,127 @@ __global__ __launch_bounds__(256) void mixer_delta_chunk_kernel(DeltaArgs a) {
   }
 }
 
-// One chunk's operands of a scan lane.
+// A chunk's operands of a scan lane.
 template <int NI> struct ScanSet {
-  u32x4 kp[NI], qp[NI], t, p;
-  float kt[NI][4], v[4], g15;
-  cf32x4 gi, beta, ge;  // tokens 4 g .. 4 g + 3
+  uint4 kp[NI], qp[NI], t;
+  cf32x4 ka[NI], gi, beta, ge;  // tokens 4 g .. 4 g + 3
+  float v[4], g15;
+};
+
+// LDS bytes of a chunk's operands in a scan: 16 rows of k and of q (16-byte piece c of row t in place c ^ t, so that
+// neither the rows' pieces nor the columns meet in a bank), of the values' 16 columns, T and P, the factors.
+template <int NI> struct ScanLds {
+  static constexpr int DR = 64 * NI, KB = 64 * DR;
+  static constexpr int Q = KB, V = 2 * KB, T = V + 1024, GM = T + 2048, BUF = GM + 256;
+  static constexpr int IPC = 8 * NI + 7;   // DMA instructions of a chunk
 };
 
 // grid (H, ceil(vdim / 16), B) — the column blocks of a head land on one XCD and share its
-// rows in that L2 — 256 threads; wave w: rows [16 NI w, 16 NI (w + 1)), DR = 64 NI
+// rows in that L2 — 384 threads; wave w < 4: rows [16 NI w, 16 NI (w + 1)), DR = 64 NI; wave 4 asks, wave 5
+// finishes the read-outs.  What bounds a long prompt is a chunk's chain: products by the state, their sum over the
+// waves, T, the new state, 930 clocks of MFMAs a wave of some 2200.  All else is taken off it: operands come by LDS-DMA two
+// chunks ahead (loaded by the waves that use them, two times k and in 4-byte pieces, 32 heads of 128 x 128 over 1100 tokens
+// took 102 us, so 87) and to registers one ahead, and the read-outs, which the four waves took in turns while the others
+// waited, have a wave of their own (62).  24 sequences of 61 tokens 140 us either way.
 template <int DT, int NI>
-__global__ __launch_bounds__(256) void mixer_delta_scan_kernel(DeltaArgs a) {
+__global__ __launch_bounds__(384) void mixer_delta_scan_kernel(DeltaArgs a) {
   using E = typename St<DT>::E;
-  constexpr int DR = 64 * NI;
-  __shared__ __attribute__((aligned(16))) float ex[2][4][2][64][4];
+  using L = ScanLds<NI>;
+  constexpr int DR = L::DR, NBUF = 3;
+  __shared__ __attribute__((aligned(16))) float ex[2][4][2][64][4], us[2][64][4];
+  __shared__ __attribute__((aligned(16))) uint8_t ops[NBUF * L::BUF];
   const SeqRow sq = a.seq[blockIdx.z];
   const int h = blockIdx.x, R = a.H / a.G, gh = h / R, c0 = blockIdx.y * 16;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l15 = lane & 15, g = lane >> 4;
   const int col = c0 + l15;
   const bool cok = col < a.vdim;
+  const int nc = (sq.len + kChunk - 1) / kChunk;
+  if (wave == 4) {
+    // Rows past a sequence's end are another sequence's or zeros (prep) and count nothing: their beta is zero.
+    const unsigned krow = (unsigned)a.G * DR, vrow = (unsigned)a.H * a.vdim;
+    unsigned off[4 * NI], voff[4];
+#pragma unroll
+    for (int j = 0; j < 4 * NI; ++j) {
+      const int p = 64 * j + lane, t = p / (16 * NI), c = p - t * (16 * NI);
+      off[j] = t * krow + ((c ^ t) * 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) voff[e] = (4 * g + e) * vrow + (cok ? col : 0);
+    const float* kb = a.kn + ((long long)sq.row0 * a.G + gh) * DR;
+    const float* qb = a.qn + ((long long)sq.row0 * a.G + gh) * DR;
+    const float* vb = a.vv + (long long)sq.row0 * vrow + (long long)h * a.vdim;
+    const float* tb = a.tp + ((long long)a.chunk0[blockIdx.z] * a.H + h) * 512 + 4 * lane;
+    const float* gb = a.gm + ((long long)a.chunk0[blockIdx.z] * a.H + h) * 64 + lane;
+    int to = 0;
+    auto ask = [&]() __attribute__((always_inline)) {
+      uint8_t* b = ops + to * L::BUF;
+#pragma unroll
+      for (int j = 0; j < 4 * NI; ++j) {
+        glds16(kb + off[j], b + 1024 * j);
+        glds16(qb + off[j], b + L::Q + 1024 * j);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        __builtin_amdgcn_global_load_lds((gptr_t)(vb + voff[e]), (lptr_t)(b + L::V + 256 * e), 4, 0, 0);
+      glds16(tb, b + L::T);
+      glds16(tb + 256, b + L::T + 1024);
+      __builtin_amdgcn_global_load_lds((gptr_t)gb, (lptr_t)(b + L::GM), 4, 0, 0);
+      kb += (long long)kChunk * krow;
+      qb += (long long)kChunk * krow;
+      vb += (long long)kChunk * vrow;
+      tb += (long long)a.H * 512;
+      gb += (long long)a.H * 64;
+      to = to + 1 == NBUF ? 0 : to + 1;
+    };
+    ask();
+    if (nc > 1) {
+      ask();
+      __builtin_amdgcn_s_waitcnt(vm_wait(L::IPC));
+    } else {
+      __builtin_amdgcn_s_waitcnt(vm_wait(0));
+    }
+    asm volatile("s_barrier" ::: "memory");
+    for (int c = 0; c < nc; ++c) {
+      __builtin_amdgcn_s_waitcnt(vm_wait(0));   // chunk c + 1 has landed
+      asm volatile("s_barrier" ::: "memory");
+      if (c + 2 < nc) ask();                    // into chunk c - 1's buffer: every wave is past it
+    }
+    asm volatile("s_barrier" ::: "memory");
+    return;
+  }
+  if (wave == 5) {   // the read-outs, a chunk behind the others
+    const long long step = (long long)a.H * a.vdim;
+    float* o = a.o + ((long long)(sq.row0 + 4 * g) * a.H + h) * a.vdim + col;
+    uint4 p{};
+    cf32x4 gi{};
+    auto finish = [&](int c) __attribute__((always_inline)) {
+      const int buf = c & 1;
+      cf32x4 qs = *reinterpret_cast<const cf32x4*>(ex[buf][0][1][lane]);
+#pragma unroll
+      for (int w = 1; w < 4; ++w) qs += *reinterpret_cast<const cf32x4*>(ex[buf][w][1][lane]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qs[e] *= gi[e];
+      const cf32x4 y = mm_piece<kF32>(p, *reinterpret_cast<const uint4*>(us[buf][lane]), qs);
+      const int left = cok ? sq.len - kChunk * c - 4 * g : 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < left) o[e * step] = y[e];
+      o += kChunk * step;
+    };
+    asm volatile("s_barrier" ::: "memory");
+    int at = 0;
+    for (int c = 0; c < nc; ++c) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (c > 0) finish(c - 1);
+      const uint8_t* b = ops + at * L::BUF;
+      at = at + 1 == NBUF ? 0 : at + 1;
+      p = *reinterpret_cast<const uint4*>(b + L::T + 1024 + (16 * l15 + 4 * g) * 4);
+      gi = *reinterpret_cast<const cf32x4*>(b + L::GM + 16 * g);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    finish(nc - 1);
+    return;
+  }
   const int r0 = 16 * NI * wave;
   float* st = a.state + sq.slot * a.s_slot + (long long)h * a.dim * a.EP;
   cf32x4 S[NI];
@@ -228,106 +330,81 @@ __global__ __launch_bounds__(256) void mixer_delta_scan_kernel(DeltaArgs a) {
       const int r = r0 + 16 * i + 4 * g + e;
       S[i][e] = sq.pos0 > 0 && cok && r < a.dim ? st[(long long)r * a.EP + col] : 0.f;
     }
-  const int nc = (sq.len + kChunk - 1) / kChunk, ch0 = a.chunk0[blockIdx.z];
-  // A chunk's operands: a uniform base that moves with the chunk plus a lane offset that does
-  // not.  Rows past a sequence's end are another sequence's or zeros (prep) and count nothing:
-  // their beta is zero.
-  const unsigned krow = (unsigned)a.G * DR, vrow = (unsigned)a.H * a.vdim;
-  const unsigned koff = l15 * krow + r0 + 4 * g, toff = 16 * l15 + 4 * g;
-  unsigned ktoff[4], voff[4];
+  // places in a chunk's operands: rows of k and q as A of the products by the state, columns of k as A of its update
+  int kp[NI], kt[NI][4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    ktoff[e] = (4 * g + e) * krow + r0 + l15;
-    voff[e] = (4 * g + e) * vrow + (cok ? col : 0);
+  for (int i = 0; i < NI; ++i) {
+    kp[i] = l15 * DR * 4 + (((r0 + 16 * i) / 4 + g) ^ l15) * 16;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      kt[i][e] = (4 * g + e) * DR * 4 + (((r0 + 16 * i) / 4 + (l15 >> 2)) ^ (4 * g + e)) * 16 + (l15 & 3) * 4;
   }
-  const float* kbase = a.kn + ((long long)sq.row0 * a.G + gh) * DR;
-  const float* qbase = a.qn + ((long long)sq.row0 * a.G + gh) * DR;
-  const float* vbase = a.vv + (long long)sq.row0 * vrow + (long long)h * a.vdim;
-  const float* tbase = a.tp + ((long long)ch0 * a.H + h) * 512;
-  const float* gbase = a.gm + ((long long)ch0 * a.H + h) * 64;
-  auto load = [&](ScanSet<NI>& s, int c) __attribute__((always_inline)) {
-    const float* kb = kbase + (long long)c * kChunk * krow;
-    const float* qb = qbase + (long long)c * kChunk * krow;
-    const float* vb = vbase + (long long)c * kChunk * vrow;
-    const float* tb = tbase + (long long)c * a.H * 512;
-    const float* gb = gbase + (long long)c * a.H * 64;
+  int at = 0;
+  auto read = [&](ScanSet<NI>& s) __attribute__((always_inline)) {
+    const uint8_t* b = ops + at * L::BUF;
+    at = at + 1 == NBUF ? 0 : at + 1;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      s.kp[i] = *reinterpret_cast<const u32x4*>(kb + koff + 16 * i);
-      s.qp[i] = *reinterpret_cast<const u32x4*>(qb + koff + 16 * i);
+      s.kp[i] = *reinterpret_cast<const uint4*>(b + kp[i]);
+      s.qp[i] = *reinterpret_cast<const uint4*>(b + L::Q + kp[i]);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s.v[e] = vb[voff[e]];
-    s.gi = *reinterpret_cast<const cf32x4*>(gb + 4 * g);
-    s.beta = *reinterpret_cast<const cf32x4*>(gb + 16 + 4 * g);
-    s.t = *reinterpret_cast<const u32x4*>(tb + toff);
-    s.ge = *reinterpret_cast<const cf32x4*>(gb + 32 + 4 * g);
-    s.g15 = gb[48];
+    for (int e = 0; e < 4; ++e) {
+      s.v[e] = *reinterpret_cast<const float*>(b + L::V + 256 * e + 4 * lane);
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s.kt[i][e] = kb[ktoff[e] + 16 * i];
-    s.p = *reinterpret_cast<const u32x4*>(tb + 256 + toff);
+      for (int i = 0; i < NI; ++i) s.ka[i][e] = *reinterpret_cast<const float*>(b + kt[i][e]);
+    }
+    const float* gm = reinterpret_cast<const float*>(b + L::GM);
+    s.gi = *reinterpret_cast<const cf32x4*>(gm + 4 * g);
+    s.beta = *reinterpret_cast<const cf32x4*>(gm + 16 + 4 * g);
+    s.ge = *reinterpret_cast<const cf32x4*>(gm + 32 + 4 * g);
+    s.g15 = gm[48];
+    s.t = *reinterpret_cast<const uint4*>(b + L::T + (16 * l15 + 4 * g) * 4);
   };
-  auto chunk = [&](const ScanSet<NI>& s, int c) __attribute__((always_inline)) {
+  auto chunk = [&](const ScanSet<NI>& s, ScanSet<NI>& next, int c) __attribute__((always_inline)) {
     const int buf = c & 1;
     cf32x4 ks{0.f, 0.f, 0.f, 0.f}, qs{0.f, 0.f, 0.f, 0.f};
+    uint4 sb[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const uint4 sb = __builtin_bit_cast(uint4, S[i]);
-      ks = mm_piece<kF32>(__builtin_bit_cast(uint4, s.kp[i]), sb, ks);
-      qs = mm_piece<kF32>(__builtin_bit_cast(uint4, s.qp[i]), sb, qs);
+      sb[i] = __builtin_bit_cast(uint4, S[i]);
+      ks = mm_piece<kF32>(s.kp[i], sb[i], ks);
     }
     *reinterpret_cast<cf32x4*>(ex[buf][wave][0][lane]) = ks;
-    *reinterpret_cast<cf32x4*>(ex[buf][wave][1][lane]) = qs;
-    // the other waves' halves only need the LDS writes: a full barrier would also drain the
-    // operand loads in flight
+    // the other waves' parts of ks, the read-out's of the chunk before, and the next chunk's operands are there
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    ks = *reinterpret_cast<const cf32x4*>(ex[buf][0][0][lane]);
+    cf32x4 kw[4];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) ks += *reinterpret_cast<const cf32x4*>(ex[buf][w][0][lane]);
+    for (int w = 0; w < 4; ++w) kw[w] = *reinterpret_cast<const cf32x4*>(ex[buf][w][0][lane]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) qs = mm_piece<kF32>(s.qp[i], sb[i], qs);   // while the parts come in
+    __builtin_amdgcn_sched_barrier(0);
+    ks = ((kw[0] + kw[1]) + kw[2]) + kw[3];
     cf32x4 rhs;
 #pragma unroll
     for (int e = 0; e < 4; ++e) rhs[e] = s.beta[e] * (s.v[e] - s.gi[e] * ks[e]);
-    const cf32x4 u = mm_piece<kF32>(__builtin_bit_cast(uint4, s.t), __builtin_bit_cast(uint4, rhs),
-                                    cf32x4{0.f, 0.f, 0.f, 0.f});
+    const cf32x4 u = mm_piece<kF32>(s.t, __builtin_bit_cast(uint4, rhs), cf32x4{0.f, 0.f, 0.f, 0.f});
+    __builtin_amdgcn_sched_barrier(0);
+    *reinterpret_cast<cf32x4*>(ex[buf][wave][1][lane]) = qs;
+    if (c + 1 < nc) read(next);
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave == 0) *reinterpret_cast<cf32x4*>(us[buf][lane]) = u;
     cf32x4 ud;
 #pragma unroll
     for (int e = 0; e < 4; ++e) ud[e] = s.ge[e] * u[e];
     const uint4 ub = __builtin_bit_cast(uint4, ud);
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const cf32x4 ka = {s.kt[i][0], s.kt[i][1], s.kt[i][2], s.kt[i][3]};
-      S[i] = mm_piece<kF32>(__builtin_bit_cast(uint4, ka), ub, S[i] * s.g15);
-    }
-    if (wave == (c & 3)) {  // the read-outs of a chunk: the waves take turns
-      qs = *reinterpret_cast<const cf32x4*>(ex[buf][0][1][lane]);
-#pragma unroll
-      for (int w = 1; w < 4; ++w) qs += *reinterpret_cast<const cf32x4*>(ex[buf][w][1][lane]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) qs[e] *= s.gi[e];
-      const cf32x4 o = mm_piece<kF32>(__builtin_bit_cast(uint4, s.p), __builtin_bit_cast(uint4, u), qs);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = kChunk * c + 4 * g + e;
-        if (cok && t < sq.len) a.o[((long long)(sq.row0 + t) * a.H + h) * a.vdim + col] = o[e];
-      }
-    }
+    for (int i = 0; i < NI; ++i) S[i] = mm_piece<kF32>(__builtin_bit_cast(uint4, s.ka[i]), ub, S[i] * s.g15);
   };
-  // operands two chunks ahead (chunks past the end re-read the last one)
+  asm volatile("s_barrier" ::: "memory");
   ScanSet<NI> s0, s1;
-  load(s0, 0);
-  load(s1, min(1, nc - 1));
-  // once: with loads pending on the way in, the compiler waits for the newest loads in every
-  // round (its counts cover both ways into the loop)
-  __builtin_amdgcn_s_waitcnt(vm_wait(0));
+  read(s0);
   for (int c = 0; c < nc; c += 2) {
-    chunk(s0, c);
-    if (c + 1 >= nc) break;
-    load(s0, min(c + 2, nc - 1));
-    chunk(s1, c + 1);
-    load(s1, min(c + 3, nc - 1));
+    chunk(s0, s1, c);
+    if (c + 1 < nc) chunk(s1, s0, c + 1);
   }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if (cok)
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -448,10 +525,10 @@ CAKE_API int cake_mixer_delta_prefill(int dt, const void* proj, long long ldp, c
     if (taps <= 4) CAKE_PREP(4); else CAKE_PREP(8);
     hipLaunchKernelGGL(mixer_delta_chunk_kernel, dim3((unsigned)(((long long)NC * G + 3) / 4)),
                        dim3(256), 0, st, a);
-    if (ni == 1) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 1>), gs, dim3(256), 0, st, a);
-    else if (ni == 2) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 2>), gs, dim3(256), 0, st, a);
-    else if (ni == 3) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 3>), gs, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 4>), gs, dim3(256), 0, st, a);
+    if (ni == 1) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 1>), gs, dim3(384), 0, st, a);
+    else if (ni == 2) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 2>), gs, dim3(384), 0, st, a);
+    else if (ni == 3) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 3>), gs, dim3(384), 0, st, a);
+    else hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 4>), gs, dim3(384), 0, st, a);
     hipLaunchKernelGGL((mixer_delta_out_kernel<DT>), go, dim3(256), 0, st, a);
   });
   return (int)hipGetLastError();
