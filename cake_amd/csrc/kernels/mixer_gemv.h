@@ -48,7 +48,7 @@ __device__ __forceinline__ void mixer_in_rows(const MixInArgs& a, int blk, int n
     else a.act[r - a.n_raw] =
         from_f32<DT>(mix_act(a.actf, a.bias ? d + to_f32<DT>(a.bias[r - a.n_raw]) : d));
   };
-  run_pairs<DT, true, U, PFC>(map, epi, xs, a.K, npairs, p0, nblk * kWaves, pre);
+  run_pairs<DT, true, U, PFC, true>(map, epi, xs, a.K, npairs, p0, nblk * kWaves, pre);
 }
 
 }  // namespace cake

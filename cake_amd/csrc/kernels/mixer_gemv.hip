@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kGemvThreads) void mixer_out_kernel(
     const float d = (lane == 0 ? da : db) + (bias ? to_f32<DT>(bias[r]) : 0.f);
     y[r] = fmaf(alpha, d, p == p0 ? r0 : x[r]);
   };
-  run_pairs<DT, false, U, PFC>(map, epi, xs, K, npairs, p0, gridDim.x * kGemvWaves, pre);
+  run_pairs<DT, false, U, PFC, true>(map, epi, xs, K, npairs, p0, gridDim.x * kGemvWaves, pre);
 }
 
 // y = W [x ; x0] + step (x, x0 f32 [W] each; w [W][K], K = 2 W padded to 8); y is neither

@@ -32,3 +32,23 @@ def test_rows(cuda, dt, N, K, ln):
     size = 2.0 ** (-8 if dt == torch.bfloat16 else -11)
     assert bool(((act[:N - n_raw].double() - a).abs() <= 2 * tol[n_raw:] + size * a.abs()).all())
     assert bool((act[N - n_raw:] == 5.0).all())
+
+
+# whole rounds of 512 columns past the ones asked for ahead, one to three over, and pieces of a round
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("K", [2048, 2056, 2560, 3072, 3584, 4096, 4104, 6144, 11776, 29696, 30200])
+def test_rounds_left_over(cuda, dt, K):
+    """The output products of one token: 16-bit columns, f32 sums in another order (K 2^-22 of the scale)."""
+    from cake_amd.ops import hip as K32
+    N = 37
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a = torch.randn(K, device="cuda", generator=g).to(dt)
+    w = torch.empty(N, K, device="cuda", dtype=dt).normal_(0, K ** -0.5, generator=g)
+    x = torch.randn(N, device="cuda", generator=g)
+    y = torch.empty(N, device="cuda")
+    want = w.double() @ a.double()
+    M.layer_out(a, w, 0.5, x, y)
+    assert bool(((y.double() - x.double() - 0.5 * want).abs() <= K * 2.0 ** -22 * (1 + want.abs())).all())
+    r = x.clone()
+    K32.gemv(a, w, r, accumulate=True)
+    assert bool(((r.double() - x.double() - want).abs() <= K * 2.0 ** -22 * (1 + want.abs())).all())
