@@ -64,6 +64,20 @@ __global__ __launch_bounds__(AttnGeom2<NREP>::NT) void attn2_decode_kernel(AttnD
                                                                     lds, gridDim.x);
 }
 
+// NH of a kv head's PARTS NH heads a workgroup, all of a kv head on one XCD: what a workgroup takes longest for is the
+// value product of its heads (VALU), and there are CUs to spare.  Two heads; in launches for long contexts four of eight,
+// where the merge of more workgroups costs more than it gives.  Keys in a cold cache, whole groups and these: 64 heads over
+// 8 kv heads at 60 / 200 / 320 keys 8.4 / 11.7 / 12.5 us, 5.1 / 7.2 / 8.5 (halves 5.9 / 8.4 / 9.7), at 600 / 1500 / 2000 /
+// 4000 13.3 / 14.6 / 14.8 / 17.1, 9.4 / 10.1 / 10.3 / 13.0 (quarters 9.3 / 10.5 / 11.1 / 14.7); 32 over 8 at 60 / 320 / 600 /
+// 2000 / 4000 6.1 / 9.7 / 9.5 / 10.2 / 12.9, 5.1 / 8.3 / 7.9 / 8.7 / 11.2.
+template <int DT, int HD, int NH, int PARTS, int PFD>
+__global__ __launch_bounds__(AttnGeom2<NH>::NT) void attn2_parts_kernel(AttnDecArgs a) {
+  __shared__ __attribute__((aligned(16))) float lds[attn2_smem_floats<HD, NH, AttnGeom2<NH>::NW>()];
+  const int nkv = gridDim.x / PARTS, kv = blockIdx.x % nkv;
+  attn2_decode_block<DT, HD, NH, false, AttnGeom2<NH>::NW, PFD, NoHook, false, PARTS>(
+      a, PARTS * kv + blockIdx.x / nkv, blockIdx.y, lds, gridDim.x, NoHook(), kv);
+}
+
 // Head-parallel short-context decode: one workgroup per QUERY head (grid nh), NW waves
 // over the key blocks, the whole context as one split.  Against the per-kv-head launch
 // (nkv workgroups, each carrying its group's nrep heads) the same keys are read nrep
@@ -232,6 +246,17 @@ static int resident_splits(K kern, int threads, int heads, int splits) {
 template <int DT, int HD>
 static int launch_decode(int n_rep, dim3 grid, hipStream_t st, const AttnDecArgs& a) {
 #define CAKE_DEC2(NR, PF)                                                                     \
+  if constexpr (NR >= 4) {                                                                    \
+    constexpr int NH = NR < 4 ? 1 : PF == 1 ? 2 : NR / 2, PARTS = NR / NH;                    \
+    const auto parts = attn2_parts_kernel<DT, HD, NH, PARTS, PF>;                             \
+    const int fit = resident_splits(parts, AttnGeom2<NH>::NT, PARTS * (int)grid.x, (int)grid.y); \
+    if (fit > 0) {                                                                            \
+      AttnDecArgs a2 = a;                                                                     \
+      a2.maxsplit = fit;                                                                      \
+      hipLaunchKernelGGL(parts, dim3(PARTS * grid.x, fit), dim3(AttnGeom2<NH>::NT), 0, st, a2); \
+      return (int)hipGetLastError();                                                          \
+    }                                                                                         \
+  }                                                                                           \
   if (const int fit = resident_splits(attn2_decode_kernel<DT, HD, NR, PF>, AttnGeom2<NR>::NT,  \
                                       (int)grid.x, (int)grid.y)) {                            \
     AttnDecArgs a2 = a;                                                                       \

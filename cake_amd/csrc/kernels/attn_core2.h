@@ -114,8 +114,11 @@ struct NoHook {
 // front of them (attn_oproj.hip: the o_proj weight tile)
 // ONE: the head-parallel short-context launch (attn_head_kernel): one split, plain loads,
 // no epoch word (tickets untouched); g is then a QUERY head (NREP 1) and kvh its kv head.
+// PARTS: a kv head's group in so many parts (attn2_parts_kernel); ng = PARTS nkv, g one of them, kvh its kv head.
+// tickets has a word a kv head, so the epochs are every head's own, in the partials of its split 0, which no one
+// publishes: all advance by one a launch, in whatever parts it is.
 template <int DT, int HD, int NREP, bool FUSED = false, int NW = AttnGeom2<NREP>::NW,
-          int PFD = 2, class Hook = NoHook, bool ONE = false>
+          int PFD = 2, class Hook = NoHook, bool ONE = false, int PARTS = 1>
 __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, int s,
                                                    float* lds, int ng, const Hook& hook = Hook(),
                                                    int kvh = -1) {
@@ -218,7 +221,11 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
   }
   const int Tk = *a.pos + 1;
   unsigned int epoch = 0;
-  if constexpr (!ONE) epoch = a.tickets[ng + g];  // this launch's granule tag - 1
+  constexpr size_t kEpochs = 2 * (size_t)kMaxSplit * (HD + 2);   // words from a head's to the next
+  unsigned int* const epochs = PARTS > 1 ? reinterpret_cast<unsigned int*>(a.part) + (size_t)g * NREP * kEpochs
+                                         : a.tickets + ng + g;
+  unsigned int* const err = a.tickets + 2 * (ng / PARTS);
+  if constexpr (!ONE) epoch = *epochs;  // this launch's granule tag - 1
   ATTN_STAMP(1);
   int ns, kps;
   if constexpr (FUSED || ONE) {
@@ -383,11 +390,11 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
       if (idx < NOUT) a.out[(size_t)g * NOUT + idx] = from_f32<DT>(ao[i] / lo[i]);
     }
     if constexpr (!ONE) {
-      if (a.stamps != nullptr && tid == 0) {
-        unsigned long long* dd = a.stamps + ((size_t)s * ng + g) * 8;
+      if (a.stamps != nullptr && tid == 0 && g % PARTS == 0) {
+        unsigned long long* dd = a.stamps + ((size_t)s * (ng / PARTS) + g / PARTS) * 8;
         for (int k = 0; k < 8; ++k) dd[k] = (k < 6 || k == 6) ? stamp[k] : 0ull;
       }
-      if (tid == 0) a.tickets[ng + g] = epoch + 1u;
+      if (tid < (PARTS > 1 ? NREP : 1)) epochs[tid * kEpochs] = epoch + 1u;
     }
     return;
   }
@@ -415,8 +422,8 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
       }
     }
     ATTN_STAMP(5);
-    if (a.stamps != nullptr && tid == 0) {
-      unsigned long long* dd = a.stamps + ((size_t)s * ng + g) * 8;
+    if (a.stamps != nullptr && tid == 0 && g % PARTS == 0) {
+      unsigned long long* dd = a.stamps + ((size_t)s * (ng / PARTS) + g / PARTS) * 8;
       for (int k = 0; k < 8; ++k) dd[k] = k < 6 ? stamp[k] : 0ull;
     }
     return;
@@ -470,7 +477,7 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
       }
       if (__builtin_amdgcn_ballot_w64(!ok) == 0ull) break;
       if (tries > kAttnMaxPolls) {
-        if (lane == 0) attn_poll_timeout(a.tickets + 2 * ng);
+        if (lane == 0) attn_poll_timeout(err);
         break;
       }
       __builtin_amdgcn_s_sleep(1);
@@ -505,7 +512,7 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
         }
         if (__builtin_amdgcn_ballot_w64(!ok) == 0ull) break;
         if (tries > kAttnMaxPolls) {
-          if (lane == 0) attn_poll_timeout(a.tickets + 2 * ng);
+          if (lane == 0) attn_poll_timeout(err);
           break;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -517,9 +524,9 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
     for (int d = 0; d < DPL; ++d) dst[d] = from_f32<DT>(acc[d] * inv);
   }
   ATTN_STAMP(7);
-  if (tid == 0) a.tickets[ng + g] = epoch + 1u;  // the next launch's tag
-  if (a.stamps != nullptr && tid == 0) {
-    unsigned long long* dd = a.stamps + ((size_t)s * ng + g) * 8;
+  if (tid < (PARTS > 1 ? NREP : 1)) epochs[tid * kEpochs] = epoch + 1u;  // the next launch's tag
+  if (a.stamps != nullptr && tid == 0 && g % PARTS == 0) {
+    unsigned long long* dd = a.stamps + ((size_t)s * (ng / PARTS) + g / PARTS) * 8;
     for (int k = 0; k < 8; ++k) dd[k] = (k == 6) ? stamp[5] : stamp[k];
   }
 }

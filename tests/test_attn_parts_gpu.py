@@ -1,0 +1,41 @@
+"""Decode attention with a kv head's group in parts (attention.hip attn2_parts_kernel)."""
+import math
+
+import pytest
+import torch
+
+from cake_amd.ops import hip as K
+from cake_amd.ops import reference as R
+
+pytestmark = pytest.mark.gpu
+
+
+# two parts of two, halves and quarters of eight; launches for short and long contexts, in turns over one workspace
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (64, 8, 128), (8, 1, 64), (4, 1, 128)])
+def test_launches_in_turns(cuda, dt, nh, nkv, hd):
+    """Merged splits are this launch's own, whichever launch wrote the workspace before; a keys' block's ends; f32 attention
+    within a rounding of 16-bit queries and result."""
+    g = torch.Generator(device="cuda").manual_seed(nh)
+    S = 2048
+    kc = torch.randn(nkv, S, hd, device="cuda", generator=g).to(dt)
+    vc = torch.randn(nkv, S, hd, device="cuda", generator=g).to(dt)
+    part = torch.zeros(K.attn_workspace_numel(nh, hd, S), device="cuda")
+    tickets = torch.zeros(2 * nkv + 2, dtype=torch.int32, device="cuda")
+    out = torch.empty(nh * hd, device="cuda", dtype=dt)
+    size = 2.0 ** (-7 if dt == torch.bfloat16 else -10)
+    prev = K._ATTN_SINGLE[0]
+    K.attn_set_single_max(0)   # short contexts take the split and merge path too
+    try:
+        for turn, (cap, pos) in enumerate([(8, 100), (8, 101), (8, 300), (0, 300), (0, 1500), (8, 102), (0, 65), (8, 300),
+                                           (8, 15), (8, 16), (0, 2047), (0, 0), (8, 500), (8, 300), (0, 300), (8, 300)]):
+            K.check(K.kernels().cake_attn_set_split_cap(cap), "cap")
+            q = torch.randn(nh * hd, device="cuda", generator=g)
+            K.attn_decode(q, kc, vc, torch.tensor([pos], dtype=torch.int32, device="cuda"), hd ** -0.5, part, tickets, out)
+            want = R.attention(q.view(1, nh, hd), kc[:, :pos + 1].transpose(0, 1), vc[:, :pos + 1].transpose(0, 1),
+                               pos).reshape(-1)
+            assert not K.attn_error(tickets), turn
+            assert bool(((out.float() - want).abs() <= 2 * size * (1 + want.abs()) / math.sqrt(1 + pos / 64)).all()), turn
+    finally:
+        K.check(K.kernels().cake_attn_set_split_cap(0), "cap")
+        K.attn_set_single_max(prev)
