@@ -114,8 +114,8 @@ CAKE_API int cake_attn_set_impl(int impl) {
     else return (int)hipErrorInvalidValue;                                        \
   } while (0)
 
-// part: workspace [nh][64][hd+2] f32; tickets: [nkv] u32, zero-initialised
-// once (the kernel re-arms them).
+// part: workspace [nh][64][hd + 2] of 8-byte granules (core 1: f32); tickets: [nkv] arrivals (core 1), [nkv]
+// epochs (core 2), the error word.  Both zero-initialised once, together; the kernels maintain them.
 static inline int attn_max_split(int S) {
   const int n = (S + kChunk - 1) / kChunk;
   return n < kMaxSplit ? n : kMaxSplit;
@@ -243,26 +243,22 @@ static int resident_splits(K kern, int threads, int heads, int splits) {
   return fit;
 }
 
+template <int DT, int HD, int NH, int PARTS, int PF>
+static constexpr auto decode2_kernel() {
+  if constexpr (PARTS > 1) return attn2_parts_kernel<DT, HD, NH, PARTS, PF>;
+  else return attn2_decode_kernel<DT, HD, NH, PF>;
+}
+
 template <int DT, int HD>
 static int launch_decode(int n_rep, dim3 grid, hipStream_t st, const AttnDecArgs& a) {
 #define CAKE_DEC2(NR, PF)                                                                     \
-  if constexpr (NR >= 4) {                                                                    \
-    constexpr int NH = NR < 4 ? 1 : PF == 1 ? 2 : NR / 2, PARTS = NR / NH;                    \
-    const auto parts = attn2_parts_kernel<DT, HD, NH, PARTS, PF>;                             \
-    const int fit = resident_splits(parts, AttnGeom2<NH>::NT, PARTS * (int)grid.x, (int)grid.y); \
-    if (fit > 0) {                                                                            \
-      AttnDecArgs a2 = a;                                                                     \
-      a2.maxsplit = fit;                                                                      \
-      hipLaunchKernelGGL(parts, dim3(PARTS * grid.x, fit), dim3(AttnGeom2<NH>::NT), 0, st, a2); \
-      return (int)hipGetLastError();                                                          \
-    }                                                                                         \
-  }                                                                                           \
-  if (const int fit = resident_splits(attn2_decode_kernel<DT, HD, NR, PF>, AttnGeom2<NR>::NT,  \
-                                      (int)grid.x, (int)grid.y)) {                            \
+  constexpr int NH = NR < 4 ? NR : PF == 1 ? 2 : NR / 2, PARTS = NR / NH;                     \
+  const auto kern = decode2_kernel<DT, HD, NH, PARTS, PF>();                                  \
+  if (const int fit = resident_splits(kern, AttnGeom2<NH>::NT, PARTS * (int)grid.x,           \
+                                      (int)grid.y)) {                                         \
     AttnDecArgs a2 = a;                                                                       \
     a2.maxsplit = fit;                                                                        \
-    hipLaunchKernelGGL((attn2_decode_kernel<DT, HD, NR, PF>), dim3(grid.x, fit),              \
-                       dim3(AttnGeom2<NR>::NT), 0, st, a2);                                   \
+    hipLaunchKernelGGL(kern, dim3(PARTS * grid.x, fit), dim3(AttnGeom2<NH>::NT), 0, st, a2);  \
   } else                                                                                      \
     hipLaunchKernelGGL((attn_decode_kernel<DT, HD, NR>), grid, dim3(AttnGeom<NR>::NT), 0, st, a)
 #define CAKE_DEC(NR)                                                                          \

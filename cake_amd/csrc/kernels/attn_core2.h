@@ -115,8 +115,10 @@ struct NoHook {
 // ONE: the head-parallel short-context launch (attn_head_kernel): one split, plain loads,
 // no epoch word (tickets untouched); g is then a QUERY head (NREP 1) and kvh its kv head.
 // PARTS: a kv head's group in so many parts (attn2_parts_kernel); ng = PARTS nkv, g one of them, kvh its kv head.
-// tickets has a word a kv head, so the epochs are every head's own, in the partials of its split 0, which no one
-// publishes: all advance by one a launch, in whatever parts it is.
+// The kv head's epoch word advances by kEpoch a merging launch, a share of it by each part: while a part has not added its
+// own, the word is below this launch's end, whatever the others did, and rounded down it is this launch's in all of them.
+// So launches in any parts, groups and head sizes tag by one count and can share a workspace.
+constexpr unsigned int kEpoch = 4;
 template <int DT, int HD, int NREP, bool FUSED = false, int NW = AttnGeom2<NREP>::NW,
           int PFD = 2, class Hook = NoHook, bool ONE = false, int PARTS = 1>
 __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, int s,
@@ -221,11 +223,16 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
   }
   const int Tk = *a.pos + 1;
   unsigned int epoch = 0;
-  constexpr size_t kEpochs = 2 * (size_t)kMaxSplit * (HD + 2);   // words from a head's to the next
-  unsigned int* const epochs = PARTS > 1 ? reinterpret_cast<unsigned int*>(a.part) + (size_t)g * NREP * kEpochs
-                                         : a.tickets + ng + g;
+  static_assert(kEpoch % PARTS == 0, "whole shares");
+  unsigned int* const epochs = a.tickets + ng / PARTS + g / PARTS;
   unsigned int* const err = a.tickets + 2 * (ng / PARTS);
-  if constexpr (!ONE) epoch = *epochs;  // this launch's granule tag - 1
+  if constexpr (!ONE) epoch = *epochs & ~(kEpoch - 1u);  // this launch's granule tag - kEpoch
+  // by split 0 behind its poll, when every split that tags has read the epoch (a lone one tags nothing and leaves it)
+  auto advance = [&]() __attribute__((always_inline)) {
+    if (tid != 0) return;
+    if constexpr (PARTS == 1) *epochs = epoch + kEpoch;
+    else __hip_atomic_fetch_add(epochs, kEpoch / PARTS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   ATTN_STAMP(1);
   int ns, kps;
   if constexpr (FUSED || ONE) {
@@ -394,17 +401,16 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
         unsigned long long* dd = a.stamps + ((size_t)s * (ng / PARTS) + g / PARTS) * 8;
         for (int k = 0; k < 8; ++k) dd[k] = (k < 6 || k == 6) ? stamp[k] : 0ull;
       }
-      if (tid < (PARTS > 1 ? NREP : 1)) epochs[tid * kEpochs] = epoch + 1u;
     }
     return;
   }
   // Splits >= 1 publish their partial as 8-byte {value, tag} granules (one sc1 store
   // each; a reader that sees the tag sees the value: no fence, no drain, no ticket) and
   // exit.  Split 0 keeps its own partial in LDS and merges: one wave per head polls
-  // the other splits' granules until every tag is this launch's (tag = epoch + 1; the
-  // per-kv-head epoch lives in tickets[nkv + g] and is advanced by split 0 at the end,
+  // the other splits' granules until every tag is this launch's (tag = epoch + kEpoch; the
+  // kv head's epoch lives in tickets[nkv + kv head] and is advanced by split 0 behind its poll,
   // so stale granules of earlier launches never match).
-  const unsigned long long tagw = (unsigned long long)(epoch + 1u) << 32;
+  const unsigned long long tagw = (unsigned long long)(epoch + kEpoch) << 32;
   unsigned long long* gpart = reinterpret_cast<unsigned long long*>(a.part);
   if (s != 0) {
 #pragma unroll
@@ -482,6 +488,7 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
       }
       __builtin_amdgcn_s_sleep(1);
     }
+    advance();
     const float M = wave_max(mt);
     const float wt = lane < ns ? exp2f(mt - M) : 0.f;
     const float L = wave_sum(wt * lt);
@@ -524,7 +531,6 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
     for (int d = 0; d < DPL; ++d) dst[d] = from_f32<DT>(acc[d] * inv);
   }
   ATTN_STAMP(7);
-  if (tid < (PARTS > 1 ? NREP : 1)) epochs[tid * kEpochs] = epoch + 1u;  // the next launch's tag
   if (a.stamps != nullptr && tid == 0 && g % PARTS == 0) {
     unsigned long long* dd = a.stamps + ((size_t)s * (ng / PARTS) + g / PARTS) * 8;
     for (int k = 0; k < 8; ++k) dd[k] = (k == 6) ? stamp[5] : stamp[k];

@@ -39,3 +39,35 @@ def test_launches_in_turns(cuda, dt, nh, nkv, hd):
     finally:
         K.check(K.kernels().cake_attn_set_split_cap(0), "cap")
         K.attn_set_single_max(prev)
+
+
+@pytest.mark.parametrize("first,then", [(4, 2), (4, 1), (8, 2), (2, 4), (1, 8)])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_groups_of_two_sizes_share_a_workspace(cuda, first, then, hd):
+    """Launches of any group tag by one count: splits of the launch before, whose group was another, are not this one's.
+    Dropped ones end in the error word, whatever the workspace holds."""
+    nkv, S, pos = 2, 2048, 1500
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    kc = torch.randn(nkv, S, hd, device="cuda", generator=g).bfloat16()
+    vc = torch.randn(nkv, S, hd, device="cuda", generator=g).bfloat16()
+    p = torch.tensor([pos], dtype=torch.int32, device="cuda")
+    part = torch.zeros(K.attn_workspace_numel(nkv * max(first, then), hd, S), device="cuda")
+    tickets = torch.zeros(2 * nkv + 2, dtype=torch.int32, device="cuda")
+
+    def launch(n_rep):
+        nh = n_rep * nkv
+        q, out = torch.randn(nh * hd, device="cuda", generator=g), torch.empty(nh * hd, device="cuda", dtype=torch.bfloat16)
+        K.attn_decode(q, kc, vc, p, hd ** -0.5, part, tickets, out)
+        want = R.attention(q.view(1, nh, hd), kc[:, :pos + 1].transpose(0, 1), vc[:, :pos + 1].transpose(0, 1), pos)
+        return bool(((out.float() - want.reshape(-1)).abs() <= 2.0 ** -6 * (1 + want.reshape(-1).abs()) / math.sqrt(1 + pos / 64)).all())
+    for n_rep in (first, then, first, first, then):
+        assert launch(n_rep) and not K.attn_error(tickets)
+    K.attn_clear_error(tickets)
+    launch(first)
+    K.attn_debug_drop_partials(True)
+    try:
+        launch(then)
+        torch.cuda.synchronize()
+    finally:
+        K.attn_debug_drop_partials(False)
+    assert K.attn_error(tickets)
