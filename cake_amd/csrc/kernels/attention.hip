@@ -69,7 +69,9 @@ __global__ __launch_bounds__(AttnGeom2<NREP>::NT) void attn2_decode_kernel(AttnD
 // where the merge of more workgroups costs more than it gives.  Keys in a cold cache, whole groups and these: 64 heads over
 // 8 kv heads at 60 / 200 / 320 keys 8.4 / 11.7 / 12.5 us, 5.1 / 7.2 / 8.5 (halves 5.9 / 8.4 / 9.7), at 600 / 1500 / 2000 /
 // 4000 13.3 / 14.6 / 14.8 / 17.1, 9.4 / 10.1 / 10.3 / 13.0 (quarters 9.3 / 10.5 / 11.1 / 14.7); 32 over 8 at 60 / 320 / 600 /
-// 2000 / 4000 6.1 / 9.7 / 9.5 / 10.2 / 12.9, 5.1 / 8.3 / 7.9 / 8.7 / 11.2.
+// 2000 / 4000 6.1 / 9.7 / 9.5 / 10.2 / 12.9, 5.1 / 8.3 / 7.9 / 8.7 / 11.2.  Launches that are capped for lengths
+// past kLongKeys keep a group of eight whole: parts read the keys and values once each, and there their CUs read all the time
+// (64 heads over 8 at 48000 / 131000 keys in halves 51.3 / 132 us, whole 46.3 / 109; at 1500 9.6, 14.2).
 template <int DT, int HD, int NH, int PARTS, int PFD>
 __global__ __launch_bounds__(AttnGeom2<NH>::NT) void attn2_parts_kernel(AttnDecArgs a) {
   __shared__ __attribute__((aligned(16))) float lds[attn2_smem_floats<HD, NH, AttnGeom2<NH>::NW>()];
@@ -170,7 +172,8 @@ CAKE_API int cake_attn_splits(int Tk) {
   if (g_attn_impl == 2) {
     int ns, kps;
     if (Tk <= g_attn_single) return 1;
-    int keys = (Tk + g_attn_target - 1) / g_attn_target;
+    const int target = Tk > kLongKeys ? 2 * g_attn_target : g_attn_target;   // (of kLongHeads, else fewer)
+    int keys = (Tk + target - 1) / target;
     keys = (keys + 15) / 16 * 16;
     if (keys < g_attn_min_keys) keys = g_attn_min_keys;
     ns = (Tk + keys - 1) / keys;
@@ -243,23 +246,29 @@ static int resident_splits(K kern, int threads, int heads, int splits) {
   return fit;
 }
 
+// a core-2 launch in parts, with the splits that fit; false: not even one of each part does
 template <int DT, int HD, int NH, int PARTS, int PF>
-static constexpr auto decode2_kernel() {
-  if constexpr (PARTS > 1) return attn2_parts_kernel<DT, HD, NH, PARTS, PF>;
-  else return attn2_decode_kernel<DT, HD, NH, PF>;
+static bool launch_core2(dim3 grid, hipStream_t st, AttnDecArgs a) {
+  const auto kern = [] {
+    if constexpr (PARTS > 1) return attn2_parts_kernel<DT, HD, NH, PARTS, PF>;
+    else return attn2_decode_kernel<DT, HD, NH, PF>;
+  }();
+  a.maxsplit = resident_splits(kern, AttnGeom2<NH>::NT, PARTS * (int)grid.x, (int)grid.y);
+  if (a.maxsplit == 0) return false;
+  hipLaunchKernelGGL(kern, dim3(PARTS * grid.x, a.maxsplit), dim3(AttnGeom2<NH>::NT), 0, st, a);
+  return true;
 }
 
 template <int DT, int HD>
 static int launch_decode(int n_rep, dim3 grid, hipStream_t st, const AttnDecArgs& a) {
 #define CAKE_DEC2(NR, PF)                                                                     \
-  constexpr int NH = NR < 4 ? NR : PF == 1 ? 2 : NR / 2, PARTS = NR / NH;                     \
-  const auto kern = decode2_kernel<DT, HD, NH, PARTS, PF>();                                  \
-  if (const int fit = resident_splits(kern, AttnGeom2<NH>::NT, PARTS * (int)grid.x,           \
-                                      (int)grid.y)) {                                         \
-    AttnDecArgs a2 = a;                                                                       \
-    a2.maxsplit = fit;                                                                        \
-    hipLaunchKernelGGL(kern, dim3(PARTS * grid.x, fit), dim3(AttnGeom2<NH>::NT), 0, st, a2);  \
-  } else                                                                                      \
+  constexpr int NH = NR < 4 ? NR : PF == 1 ? 2 : NR / 2;                                      \
+  const bool whole = NR == 8 && PF == 2 && a.S > kLongKeys && (int)grid.y > a.target && (int)grid.y <= 2 * a.target; \
+  bool done = false;                                                                          \
+  if constexpr (NR == 8 && PF == 2)                                                           \
+    if (whole) done = launch_core2<DT, HD, NR, 1, PF>(grid, st, a);                           \
+  if (!whole) done = launch_core2<DT, HD, NH, NR / NH, PF>(grid, st, a);                      \
+  if (!done)                                                                                  \
     hipLaunchKernelGGL((attn_decode_kernel<DT, HD, NR>), grid, dim3(AttnGeom<NR>::NT), 0, st, a)
 #define CAKE_DEC(NR)                                                                          \
   if (g_attn_impl == 2 && (g_attn_prefetch == 2 || (g_attn_prefetch == 0 && grid.y > 8)))    \

@@ -68,14 +68,21 @@ template <int NREP> struct AttnGeom2 {
   static constexpr int NT = 64 * NW;
 };
 
+// live lengths past this take twice the splits aimed at, of up to kLongHeads kv heads: 16 of them leave half of the CUs
+// idle, and a CU reads some 30 KB a us.  16 / 32 splits of 64 heads over 8 at 48000 / 131000 keys 51.9 / 134 us, 46.3 / 109
+// (whole groups, attention.hip), of 32 over 8 45.2 / 124, 40.8 / 116, of 32 over 4 50.6 / 126, 37.9 / 71; at 16000 23.7 / 23.0 /
+// 20.4, 24.1 / 19.8 / 20.4; of 32 kv heads, which have them busy, at 48000 143, 153
+constexpr int kLongKeys = 24576, kLongHeads = 8;
+
 // host/device split policy of the v2 core (mirrored by ops.hip.attn_splits)
 __device__ __forceinline__ void attn2_splits(int Tk, int min_keys, int maxsplit, int target,
-                                             int single, int& ns, int& kps) {
+                                             int single, int nkv, int& ns, int& kps) {
   if (Tk <= single) {  // one split: no partials, no merge (cheaper up to ~320 keys)
     ns = 1;
     kps = (Tk + kBlk - 1) / kBlk * kBlk;
     return;
   }
+  if (Tk > kLongKeys && nkv <= kLongHeads) target *= 2;
   int keys = (Tk + target - 1) / target;
   keys = (keys + kBlk - 1) / kBlk * kBlk;
   if (keys < min_keys) keys = min_keys;
@@ -239,7 +246,7 @@ __device__ __forceinline__ void attn2_decode_block(const AttnDecArgs& a, int g, 
     ns = 1;
     kps = (Tk + kBlk - 1) / kBlk * kBlk;
   } else {
-    attn2_splits(Tk, a.min_keys, a.maxsplit, a.target, a.single, ns, kps);
+    attn2_splits(Tk, a.min_keys, a.maxsplit, a.target, a.single, ng / PARTS, ns, kps);
   }
   if (s >= ns) return;
   const int kb = s * kps, ke = min(Tk, kb + kps);

@@ -71,3 +71,26 @@ def test_groups_of_two_sizes_share_a_workspace(cuda, first, then, hd):
     finally:
         K.attn_debug_drop_partials(False)
     assert K.attn_error(tickets)
+
+
+# groups whole, in parts and of one head; as many kv heads as take more splits in long contexts, and one more
+@pytest.mark.parametrize("nh,nkv,hd", [(16, 2, 64), (64, 8, 128), (8, 2, 128), (8, 8, 64), (18, 9, 64)])
+def test_long_contexts(cuda, nh, nkv, hd):
+    """To either side of the length that takes twice the splits, in the graphs' caps and without; f32 attention within a
+    rounding of 16-bit queries and result."""
+    S, long = 28736, K._ATTN_LONG
+    g = torch.Generator(device="cuda").manual_seed(nh)
+    kc = torch.randn(nkv, S, hd, device="cuda", generator=g).bfloat16()
+    vc = torch.randn(nkv, S, hd, device="cuda", generator=g).bfloat16()
+    part = torch.zeros(K.attn_workspace_numel(nh, hd, S), device="cuda")
+    tickets = torch.zeros(2 * nkv + 2, dtype=torch.int32, device="cuda")
+    out = torch.empty(nh * hd, device="cuda", dtype=torch.bfloat16)
+    assert K.attn_split_caps(S) == [8, 16, 32] and K.attn_splits(long) <= 16 < K.attn_splits(long + 1)
+    for pos in (long - 1, long, S - 1, 700, long):
+        for cap in (16, 32, 0):
+            q = torch.randn(nh * hd, device="cuda", generator=g)
+            with K.attn_split_cap(cap):
+                K.attn_decode(q, kc, vc, torch.tensor([pos], dtype=torch.int32, device="cuda"), hd ** -0.5, part, tickets, out)
+            want = R.attention(q.view(1, nh, hd), kc[:, :pos + 1].transpose(0, 1), vc[:, :pos + 1].transpose(0, 1), pos).reshape(-1)
+            assert not K.attn_error(tickets)
+            assert bool(((out.float() - want).abs() <= 2.0 ** -6 * (1 + want.abs()) / math.sqrt(1 + pos / 64)).all()), (pos, cap)
