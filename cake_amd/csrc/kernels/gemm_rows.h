@@ -15,17 +15,19 @@
 //   arrive sums in share order (the result does not hang on the order).  28672 x 4096 SwiGLU at 5 / 24 /
 //   45 rows 38 / 38 / 40 us (tile kernels 58-60 us), 4096 x 23552 33 / 37 / 43 us (44-46 us), 57344 x 8192
 //   140 us (6.7 TB/s).  What bounds it is the memory in whole strips, in parts the parked sums; weight
-//   rings of a wave's own with a barrier every four steps only ran at the same rate.  Four waves ask, four multiply:
-//   loads go on while a strip's sums are parked, summed and stored, and every multiplying wave parks for itself
+//   rings of a wave's own with a barrier every four steps only ran at the same rate.  Of 128-row strips four waves ask and four
+//   multiply: loads go on while a strip's sums are parked, summed and stored, and every multiplying wave parks for itself
 //   (in one: 28672 x 4096 SwiGLU at 5 rows 39.9 -> 38.4 us, 6144 x 4096 in quarters at 45 15.0 -> 14.0, 4096 x 4096 in
-//   eighths 11.8 -> 11.1, 46 experts 1856 x 2048 61.2 -> 60.4; none slower).
+//   eighths 11.8 -> 11.1).  Strips of 64 rows are short and met by up to 60 shares: their four waves ask and multiply in turn
+//   (at 5 rows, in two kinds: 1024 x 4096 8.2, 8.9; 256 x 11008 10.6, 12.6; 1536 x 8960 14.0, 15.7; 2048 x 8192 10.7, 11.3;
+//   5120 x 5120 13.8, 13.4; 8192 x 28672 70.7, 70.5).
 #pragma once
 #include "gemm_kernel.h"
 
 namespace cake {
 
 constexpr int kRowsMinK = 512;       // k of a share at least
-constexpr int kRowsTicks = 65536;    // strips of a launch at most (an arrival counter for each of four waves)
+constexpr int kRowsTicks = 65536;    // strips of a launch at most (of 128 rows an arrival counter for each of four waves)
 
 // the operand fragments of one 64-element chunk of k: a lane's two 16-byte pieces of each row are
 // neighbours, so the two MFMA steps read whole 128-byte lines (both operands use one order of k)
@@ -196,6 +198,8 @@ template <int MT, bool WIDE> struct StreamShape {
   static constexpr int NWV = 4, RT = WIDE ? 2 : 1, KC = WIDE ? 1 : 2;   // row tiles, 64-element chunks
   static constexpr int BN = NWV * 16 * RT, KST = 64 * KC;   // weight rows of a strip, k of a step
   static constexpr int NS = WIDE ? 4 : 3, WGS = WIDE ? 256 : 512;
+  static constexpr bool ASK = WIDE;   // four more waves ask for what these multiply
+  static constexpr int THREADS = (ASK ? 2 : 1) * 64 * NWV;
   static constexpr int LPR = 8 * KC, RPI = 64 / LPR;   // lanes of a row's DMA, rows of an instruction
   static constexpr int XT = 2 * MT * KC;               // x DMA instructions of a step
   static constexpr int XW = XT % 4 == 0 ? 4 : XT % 3 == 0 ? 3 : 2;   // waves that issue them
@@ -331,10 +335,11 @@ __device__ __forceinline__ cf32x4 unpark(const float* p) {
 }
 
 template <int DT, int EPI, int MT, bool GRP>
-__global__ __launch_bounds__(512, (StreamShape<MT, stream_wide<EPI, MT>()>::WGS / 128)) void gemm_stream_kernel(GemmArgs g) {
+__global__ __launch_bounds__((StreamShape<MT, stream_wide<EPI, MT>()>::THREADS), 2) void gemm_stream_kernel(GemmArgs g) {
   using S = StreamShape<MT, stream_wide<EPI, MT>()>;
   constexpr int NWV = S::NWV, RT = S::RT, KC = S::KC, KST = S::KST;
   __shared__ __attribute__((aligned(16))) uint8_t smem[S::NS * S::STAGE];
+  __shared__ unsigned last;
   const int tid = threadIdx.x, who = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wave = who % NWV;
   const int KS = (g.K + KST - 1) / KST;
@@ -351,79 +356,85 @@ __global__ __launch_bounds__(512, (StreamShape<MT, stream_wide<EPI, MT>()>::WGS 
   const int u1 = parts ? min((wg / g.pieces + 1) * KS, u0 + per) : min(total, u0 + per);
   if (u0 >= u1) return;
 
-  if (who >= NWV) {   // ---- asking: wave w the rows 16 RT w .. of the weights and its share of x ----
-    const int dr = lane / S::LPR, dslot = lane % S::LPR;   // row within an instruction's, slot
-    int ds = u0 / KS, dk = u0 % KS, dnext = u0;
-    // shares of whole strips start 5 steps on from the share before them, equal parts of one from the strip
-    // before: strips lie the same distance apart, and in step they would ask the same channels of the
-    // memory at a time (28672 x 4096 in 224 whole strips 46.8 us in step, 39.6 so; 12288 x 4096 in 192
-    // halves at 24 rows 28.1, 23.1; each half 5 steps on 25.5).  128-row parts that are no multiple of 4 KB apart spread by
-    // themselves, and in step read x together (4096 x 14336 in 256 eighths of 3.5 KB at 24 rows 25.9, 26.7
-    // turned; 8192 x 28672 at 64 rows 85.1, 86.7; of 64 rows, two on a CU, at 5 rows 88.3, 71.3 turned).
-    const int seg = parts ? u1 - u0 : KS % per == 0 ? per : per % KS == 0 ? KS : 0;   // 0: other shares
-    const bool turn = seg == KS || S::KC == 2 || seg * KST * 2 % 4096 == 0;
-    const int seg0 = parts ? dk : seg > 0 ? dk / seg * seg : 0;
-    if (seg > 0 && turn) dk = seg0 + u0 / max(per, KS) * 5 % seg;
-    int left = seg;
-    const uint16_t *wsrc[4], *xsrc[S::XI];
-    auto aim = [&](int s) {
-      const StreamStrip t = stream_strip<GRP, S::BN>(g, s);
+  // ---- what is asked for: wave w the rows 16 RT w .. of the weights and its share of x ----
+  const int dr = lane / S::LPR, dslot = lane % S::LPR;   // row within an instruction's, slot
+  int ds = u0 / KS, dk = u0 % KS, dnext = u0;
+  // shares of whole strips start 5 steps on from the share before them, equal parts of one from the strip
+  // before: strips lie the same distance apart, and in step they would ask the same channels of the
+  // memory at a time (28672 x 4096 in 224 whole strips 46.8 us in step, 39.6 so; 12288 x 4096 in 192
+  // halves at 24 rows 28.1, 23.1; each half 5 steps on 25.5).  128-row parts that are no multiple of 4 KB apart spread by
+  // themselves, and in step read x together (4096 x 14336 in 256 eighths of 3.5 KB at 24 rows 25.9, 26.7
+  // turned; 8192 x 28672 at 64 rows 85.1, 86.7; of 64 rows, two on a CU, at 5 rows 88.3, 71.3 turned).
+  const int seg = parts ? u1 - u0 : KS % per == 0 ? per : per % KS == 0 ? KS : 0;   // 0: other shares
+  const bool turn = seg == KS || S::KC == 2 || seg * KST * 2 % 4096 == 0;
+  const int seg0 = parts ? dk : seg > 0 ? dk / seg * seg : 0;
+  if (seg > 0 && turn) dk = seg0 + u0 / max(per, KS) * 5 % seg;
+  int left = seg;
+  const uint16_t *wsrc[4], *xsrc[S::XI];
+  auto aim = [&](int s) {
+    const StreamStrip t = stream_strip<GRP, S::BN>(g, s);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = wave * (16 * RT) + i * S::RPI + dr;
-        const int v = t.v0 + row, ch = dslot ^ S::swz(row);
-        wsrc[i] = v < g.Nv ? t.b + (size_t)wrow(g, v) * g.ldb + ch * 8 : nullptr;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int row = wave * (16 * RT) + i * S::RPI + dr;
+      const int v = t.v0 + row, ch = dslot ^ S::swz(row);
+      wsrc[i] = v < g.Nv ? t.b + (size_t)wrow(g, v) * g.ldb + ch * 8 : nullptr;
+    }
 #pragma unroll
-      for (int i = 0; i < S::XI; ++i) {
-        const int row = (wave % S::XW * S::XI + i) * S::RPI + dr;
-        const int ch = dslot ^ S::swz(row);
-        xsrc[i] = t.a + (size_t)min(row, t.M - 1) * g.lda + ch * 8;
-      }
-    };
-    aim(ds);
-    auto stage = [&](int buf) {
-      uint8_t* b = smem + buf * S::STAGE;
-      const bool live = dnext < u1;
-      const int k = dk * KST;
+    for (int i = 0; i < S::XI; ++i) {
+      const int row = (wave % S::XW * S::XI + i) * S::RPI + dr;
+      const int ch = dslot ^ S::swz(row);
+      xsrc[i] = t.a + (size_t)min(row, t.M - 1) * g.lda + ch * 8;
+    }
+  };
+  auto stage = [&](int buf) {
+    uint8_t* b = smem + buf * S::STAGE;
+    const bool live = dnext < u1;
+    const int k = dk * KST;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int ch = dslot ^ S::swz(wave * (16 * RT) + i * S::RPI + dr);
-        const uint16_t* p = live && wsrc[i] != nullptr && k + ch * 8 < g.K ? wsrc[i] + k : g.zeros;
-        __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(b + (wave * 4 + i) * 1024), 16, 0, 2);
-      }
-      if (S::XW == NWV || wave < S::XW)
+    for (int i = 0; i < 4; ++i) {
+      const int ch = dslot ^ S::swz(wave * (16 * RT) + i * S::RPI + dr);
+      const uint16_t* p = live && wsrc[i] != nullptr && k + ch * 8 < g.K ? wsrc[i] + k : g.zeros;
+      __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(b + (wave * 4 + i) * 1024), 16, 0, 2);
+    }
+    if (S::XW == NWV || wave < S::XW)
 #pragma unroll
-      for (int i = 0; i < S::XI; ++i) {
-        const int r0 = wave * S::XI + i;
-        const int ch = dslot ^ S::swz(r0 * S::RPI + dr);
-        const uint16_t* p = live && k + ch * 8 < g.K ? xsrc[i] + k : g.zeros;
-        glds16(p, b + (NWV * 4 + r0) * 1024);
-      }
-      ++dnext;
-      ++dk;
-      if (seg > 0) {
-        if (dk == seg0 + seg) dk = seg0;
-        if (--left == 0) {
-          left = seg;
-          ++ds;
-          if (dnext < u1) aim(ds);
-        }
-      } else if (dk == KS) {
-        dk = 0;
+    for (int i = 0; i < S::XI; ++i) {
+      const int r0 = wave * S::XI + i;
+      const int ch = dslot ^ S::swz(r0 * S::RPI + dr);
+      const uint16_t* p = live && k + ch * 8 < g.K ? xsrc[i] + k : g.zeros;
+      glds16(p, b + (NWV * 4 + r0) * 1024);
+    }
+    ++dnext;
+    ++dk;
+    if (seg > 0) {
+      if (dk == seg0 + seg) dk = seg0;
+      if (--left == 0) {
+        left = seg;
         ++ds;
         if (dnext < u1) aim(ds);
       }
-    };
+    } else if (dk == KS) {
+      dk = 0;
+      ++ds;
+      if (dnext < u1) aim(ds);
+    }
+  };
+  // the step has landed; every wave has read the one before, whose stage takes the step NS - 1 ahead
+  auto feed = [&](int buf) __attribute__((always_inline)) {
+    if (S::XW == NWV || wave < S::XW) __builtin_amdgcn_s_waitcnt(vm_wait((S::NS - 2) * S::IPW));
+    else __builtin_amdgcn_s_waitcnt(vm_wait((S::NS - 2) * 4));
+    asm volatile("s_barrier" ::: "memory");
+    stage(buf == 0 ? S::NS - 1 : buf - 1);
+  };
+  if (!S::ASK || who >= NWV) {
+    aim(ds);
 #pragma unroll
     for (int p = 0; p < S::NS - 1; ++p) stage(p);
+  }
+  if (S::ASK && who >= NWV) {
     int buf = 0;
     for (int u = u0; u < u1; ++u) {
-      if (S::XW == NWV || wave < S::XW) __builtin_amdgcn_s_waitcnt(vm_wait((S::NS - 2) * S::IPW));
-      else __builtin_amdgcn_s_waitcnt(vm_wait((S::NS - 2) * 4));
-      asm volatile("s_barrier" ::: "memory");
-      // every wave has read the previous step's stage: it takes the step NS - 1 ahead
-      stage(buf == 0 ? S::NS - 1 : buf - 1);
+      feed(buf);
       buf = buf + 1 == S::NS ? 0 : buf + 1;
     }
     __builtin_amdgcn_s_waitcnt(vm_wait(0));
@@ -443,7 +454,8 @@ __global__ __launch_bounds__(512, (StreamShape<MT, stream_wide<EPI, MT>()>::WGS 
 #pragma unroll
       for (int i = 0; i < MT; ++i) acc[j][i] = cf32x4{0.f, 0.f, 0.f, 0.f};
     for (; u < seg1; ++u) {
-      asm volatile("s_barrier" ::: "memory");
+      if constexpr (S::ASK) asm volatile("s_barrier" ::: "memory");
+      else feed(buf);
       const uint32_t b = buf * S::STAGE;
       constexpr int XR = MT % 2 ? 1 : 2, T16 = 2048 * KC;   // bytes of 16 rows
 #pragma unroll
@@ -483,14 +495,22 @@ __global__ __launch_bounds__(512, (StreamShape<MT, stream_wide<EPI, MT>()>::WGS 
         for (int i = 0; i < MT; ++i)
           if (i * 16 + (lane & 15) < t.M) park(p + (j * MT + i) * 256, acc[j][i]);
       __builtin_amdgcn_s_waitcnt(vm_wait(0));
-      asm volatile("" ::: "memory");
-      unsigned* tick = g.tick + s * NWV + wave;
+      // (the waves of a workgroup that asks and multiplies in turn arrive as one)
+      unsigned* tick = g.tick + s * NWV + (S::ASK ? wave : 0);
       unsigned before = 0;
-      if (lane == 0) before = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if constexpr (S::ASK) {
+        asm volatile("" ::: "memory");
+        if (lane == 0) before = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::: "memory");
+      } else {
+        asm volatile("s_barrier" ::: "memory");
+        if (tid == 0) last = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        before = last;
+      }
       mine = __builtin_amdgcn_readfirstlane(before) == (unsigned)(hi - lo);
-      asm volatile("" ::: "memory");
       if (mine) {
-        if (lane == 0) __hip_atomic_store(tick, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (S::ASK ? lane == 0 : tid == 0) __hip_atomic_store(tick, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // in share order (the result does not hang on who came last), several shares in flight
         constexpr int UN = MT <= 2 ? 8 : 4;
         for (int w0 = lo; w0 <= hi; w0 += UN) {
@@ -515,16 +535,21 @@ __global__ __launch_bounds__(512, (StreamShape<MT, stream_wide<EPI, MT>()>::WGS 
               }
         }
       }
+      if constexpr (!S::ASK) __syncthreads();   // `last` is read
     }
     if (mine) stream_store<DT, EPI, MT, RT>(g, t, wave, lane, acc);
+    // stores count with the DMA: drain them before the counted waits go on
+    if (!S::ASK && u < u1) __builtin_amdgcn_s_waitcnt(vm_wait(0));
   }
+  if constexpr (!S::ASK) __builtin_amdgcn_s_waitcnt(vm_wait(0));
 }
 
 template <int DT, int EPI>
 int launch_stream(int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
 #define CAKE_STREAM(MT)                                                                             \
   if (mt == MT) {                                                                                   \
-    hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI, MT, false>), grid, dim3(512), 0, st, g);        \
+    hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI, MT, false>), grid,                              \
+                       dim3(StreamShape<MT, stream_wide<EPI, MT>()>::THREADS), 0, st, g);           \
     return (int)hipGetLastError();                                                                  \
   }
   CAKE_STREAM(1) CAKE_STREAM(2) CAKE_STREAM(3) CAKE_STREAM(4)
@@ -565,7 +590,8 @@ template <int DT> struct Rows {
     switch (epi) {
 #define X(E)                                                                                  \
   case E:                                                                                     \
-    hipLaunchKernelGGL((gemm_stream_kernel<DT, E, 1, true>), grid, dim3(512), 0, st, g);      \
+    hipLaunchKernelGGL((gemm_stream_kernel<DT, E, 1, true>), grid,                            \
+                       dim3(StreamShape<1, stream_wide<E, 1>()>::THREADS), 0, st, g);         \
     return (int)hipGetLastError();
       X(kEpiStore) X(kEpiSilu) X(kEpiQuick) X(kEpiGelu) X(kEpiRelu2)
 #undef X
