@@ -19,6 +19,10 @@ namespace cake {
 
 enum DType : int { kBF16 = 0, kF16 = 1, kF32 = 2 };
 
+// k of a grouped product up to which it takes the four-wave tiles: chosen at its launch (gemm_inst_grouped.hip), priced
+// by the plan (mixer_experts.hip)
+constexpr int kGroupedShort = 1024;
+
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
   return __uint_as_float(((uint32_t)h) << 16);
 }

@@ -36,7 +36,7 @@ __global__ __launch_bounds__((WsTile<160, 256>::THREADS)) void gemm_groups_kerne
   else ws_tiles<DT, EPI, 256, 256, true>(g, smem);
 }
 
-// The same on four waves (gemm_4w.h), for rows of 1024 k and fewer: 16 steps do not make up for the longer start of the
+// The same on four waves (gemm_4w.h), for rows of kGroupedShort k and fewer: 16 steps do not make up for the longer start of the
 // other (64 experts 1024 x 1024 at 100 rows 32 us, 34; 32 of 1024 -> 2816 47, 51).  All heights fill a CU's LDS alone: a
 // branch over whole bodies costs none of them a workgroup.  A tile runs at the least height that holds its rows.
 template <int DT, int EPI>
@@ -70,7 +70,7 @@ static int launch_grouped(int cfg, int tiles, hipStream_t st, GemmArgs& g) {
     return (int)hipGetLastError();
   }
   g.pieces = cfg == kByList ? 0 : bm;   // rows of a tile
-  if (g.K <= 1024) {
+  if (g.K <= kGroupedShort) {
     g.tiles_n = (g.N + 255) / 256;
     hipLaunchKernelGGL((gemm_heights_kernel<DT, EPI>), dim3(tiles * g.tiles_n), dim3(256), 0, st, g);
     return (int)hipGetLastError();

@@ -67,36 +67,37 @@ __global__ __launch_bounds__(256) void expert_route_kernel(const float* logits, 
 // A height from the mean alone overflows its tiles: up and down of 64 experts 2048 x 1856, 135 skewed rows each 291 us
 // (192 rows a tile), 258 (256) by the counts.
 //
-// Up rows of more than 1024 k take the tiles of gemm_ws.h: t = rounds (step k / 64 + end) us, at least the memory's (5.8
-// TB/s), a last round of less than an eighth of the CUs at less; of few tiles, of 128 columns, a share of the step.  Fitted
-// to 14 expert sizes in even, independent and skewed groups of 70 .. 600 rows: 0.2 % off the best height on the average.
-// Shorter ones the tiles of gemm_4w.h: t = rounds (step k / 64 + end), at least the memory's.
+// A product of more than kGroupedShort k takes the tiles of gemm_ws.h: t = rounds (step k / 64 + end) us, a last round of less
+// than an eighth of the CUs at less, at least the memory's (5.8 TB/s) and half of what the last round leaves idle; of few
+// tiles, of 128 columns, a share of the step.  A shorter one takes the tiles of gemm_4w.h: t = rounds (step k / 64 + end), at
+// least the memory's; tiles of a 224-row list run at 192 rows and fewer or at 256, in between.  The up product's k says which
+// heights there are.  Over 20 expert sizes in even and independent groups of 66 .. 500 rows 0.32 % off the best height on the
+// average where both k are long, 0.56 % where one or both are short (as if both products ran on the up product's tiles, without
+// the idle half, 0.37 and 0.72: 16 of 2816 x 1024 at 240 independent rows 94.0 us, 84.9 so; 256 of 512 x 4096 at 192 719, 653).
 constexpr int kHeights[4] = {160, 192, 224, 256}, kHeightsShort[4] = {128, 160, 192, 256};
-__device__ __forceinline__ int tile_rows(int W, int q) { return W > 1024 ? kHeights[q] : kHeightsShort[q]; }
-__device__ inline float height_us(int q, int tiles, int N, int K, float mem) {
+__device__ __forceinline__ int tile_rows(int W, int q) { return W > kGroupedShort ? kHeights[q] : kHeightsShort[q]; }
+__device__ inline float height_us(int rows, int tiles, int N, int K, float bytes) {
+  if (K <= kGroupedShort) {
+    constexpr float kStep[5] = {1.106f, 1.161f, 1.38f, 1.422f, 1.547f}, kEnd[5] = {5.4f, 7.76f, 8.64f, 9.39f, 11.64f};
+    const int q = rows / 32 - 4;
+    return fmaxf((tiles * ((N + 255) / 256) + 255) / 256 * (kStep[q] * ((K + 63) / 64) + kEnd[q]), bytes / 8.2e6f);
+  }
   constexpr float kStep[4] = {1.124f, 1.152f, 1.299f, 1.339f}, kEnd[4] = {5.53f, 7.80f, 7.07f, 8.42f};
+  const int q = max(rows / 32 - 5, 0);
   const bool few = tiles * ((N + 255) / 256) <= (q == 0 ? 128 : 64);   // (gemm_inst_grouped.hip)
   const int body = few && q > 0 ? 3 : q;
   const float r = tiles * (few ? (N + 127) / 128 : (N + 255) / 256) / 256.f, whole = floorf(r), part = r - whole;
-  const float rounds = whole + (part > 0.f ? fminf(1.f, 0.82f + 1.42f * part) : 0.f);
-  return fmaxf(rounds * (kStep[body] * (few ? 0.448f : 1.f) * ((K + 63) / 64) + kEnd[body] * (few ? 1.54f : 1.f)), mem);
+  const float rounds = whole + (part > 0.f ? fminf(1.f, 0.82f + 1.42f * part) : 0.f), mem = bytes / 5.8e6f;
+  const float one = kStep[body] * (few ? 0.448f : 1.f) * ((K + 63) / 64) + kEnd[body] * (few ? 1.54f : 1.f);
+  return fmaxf(rounds * one, whole > 0.f ? mem + 0.5f * (rounds - r) * one : mem);
 }
 __device__ inline int tile_height(const int (&tiles)[4], int E, int M, int F, int W) {
-  constexpr float kStep[4] = {1.106f, 1.161f, 1.38f, 1.547f}, kEnd[4] = {5.4f, 7.76f, 8.64f, 11.64f};
-  const bool ws = W > 1024;
-  const float mem = ((float)E * F * W + (float)M * (F + W)) * 2 / (ws ? 5.8e6f : 8.2e6f);
+  const float bytes = ((float)E * F * W + (float)M * (F + W)) * 2;
   int best = 0;
   float least = 0.f;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    float us;
-    if (ws) {
-      us = height_us(q, tiles[q], F, W, mem) + height_us(q, tiles[q], W, F, mem);
-    } else {
-      const int up = (tiles[q] * ((F + 255) / 256) + 255) / 256, down = (tiles[q] * ((W + 255) / 256) + 255) / 256;
-      us = fmaxf(up * (kStep[q] * ((W + 63) / 64) + kEnd[q]), mem) +
-           fmaxf(down * (kStep[q] * ((F + 63) / 64) + kEnd[q]), mem);
-    }
+    const float us = height_us(tile_rows(W, q), tiles[q], F, W, bytes) + height_us(tile_rows(W, q), tiles[q], W, F, bytes);
     if (q == 0 || us < least) {
       best = q;
       least = us;

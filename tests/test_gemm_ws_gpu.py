@@ -62,26 +62,35 @@ def test_groups_of_several_tiles(cuda):
 
 
 def _height(counts, F, W):
-    """(cost, height) of every height, in 64 bits."""
+    """(cost, height) of every height, in 64 bits: each product as on the tiles that its own k takes."""
     R, out = sum(counts), []
-    mem = (len(counts) * F * W + R * (F + W)) * 2 / 5.8e6
+    size = (len(counts) * F * W + R * (F + W)) * 2
 
-    def us(q, t, n, k):
+    def us(bm, t, n, k):
+        if k <= 1024:
+            step, end = {128: (1.106, 5.4), 160: (1.161, 7.76), 192: (1.38, 8.64), 224: (1.422, 9.39), 256: (1.547, 11.64)}[bm]
+            return max(-(-t * -(-n // 256) // 256) * (step * -(-k // 64) + end), size / 8.2e6)
+        q = max(bm // 32 - 5, 0)
         few = t * -(-n // 256) <= (128 if q == 0 else 64)
         body = 3 if few and q else q
-        whole, part = divmod(t * -(-n // (128 if few else 256)) / 256, 1)
+        r = t * -(-n // (128 if few else 256)) / 256
+        whole, part = divmod(r, 1)
         rounds = whole + (min(1.0, 0.82 + 1.42 * part) if part else 0.0)
         step, end = (1.124, 1.152, 1.299, 1.339)[body], (5.53, 7.80, 7.07, 8.42)[body]
-        return max(rounds * (step * (0.448 if few else 1) * -(-k // 64) + end * (1.54 if few else 1)), mem)
-    for q, bm in enumerate((160, 192, 224, 256)):
+        one = step * (0.448 if few else 1) * -(-k // 64) + end * (1.54 if few else 1)
+        return max(rounds * one, size / 5.8e6 + (0.5 * (rounds - r) * one if whole else 0))
+    for bm in (160, 192, 224, 256) if W > 1024 else (128, 160, 192, 256):
         t = sum(-(-c // bm) for c in counts)
-        out.append((us(q, t, F, W) + us(q, t, W, F), bm))
+        out.append((us(bm, t, F, W) + us(bm, t, W, F), bm))
     return out
 
 
 @pytest.mark.parametrize("counts,F,W", [([64], 72, 1032), ([161, 160, 159, 1], 300, 1160), ([192, 193, 191] * 20, 1096, 1100),
                                         ([220] * 64, 520, 2048), ([225, 224, 0, 223, 500] * 9, 1500, 1032),
-                                        ([250] * 40 + [1] * 30, 2000, 1536), ([150] * 64, 1856, 2048)])
+                                        ([250] * 40 + [1] * 30, 2000, 1536), ([150] * 64, 1856, 2048),
+                                         # a down product on the short rows' tiles under such an up product, and the other way
+                                         ([192, 206, 185, 210] * 64, 512, 4096), ([240, 251, 262, 228] * 4, 2816, 1024),
+                                         ([300] * 8, 4096, 1024), ([70] * 64, 1032, 1000)])
 def test_height_of_the_groups(cuda, counts, F, W):
     """The device lists tiles of the cheapest height (of two within 1e-4 either), every row in one of them."""
     from cake_amd.ops import experts as X
@@ -95,6 +104,40 @@ def test_height_of_the_groups(cuda, counts, F, W):
     costs = _height(counts, F, W)
     assert bm in [b for c, b in costs if c <= min(costs)[0] * (1 + 1e-4)]
     assert p.tiles[:n].tolist() == _tiles(counts, bm)
+
+
+# a list of 224 rows, by configuration and by itself, where no tile of that height is: 193 .. 224 rows run at 256
+@pytest.mark.parametrize("dt", list(SIZE), ids=str)
+@pytest.mark.parametrize("cfg", [3, 6])
+@pytest.mark.parametrize("N,K", [(8, 8), (300, 520), (1100, 1024)])
+def test_short_rows_in_lists_of_224(cuda, dt, cfg, N, K):
+    _groups(cuda, dt, cfg, [224, 0, 223, 225, 193, 192, 160, 1, 500], N, K, 224, K + 8)
+
+
+@pytest.mark.parametrize("dt", list(SIZE), ids=str)
+@pytest.mark.parametrize("F,W", [(768, 1160), (1024, 1032), (1032, 1024), (1304, 520)])
+def test_up_and_down_on_either_side_of_the_line(cuda, dt, F, W):
+    """Both products of a plan whose k lie to either side of the short rows' line: f32 sums of two orders, rounded once."""
+    from cake_amd.ops import experts as X
+    counts = [161, 0, 224, 193, 225, 256, 70, 129]
+    R, E = sum(counts), len(counts)
+    g = torch.Generator(device="cuda").manual_seed(F)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).int().cuda().view(R, 1)
+    p = X.plan(ids, torch.ones(R, 1, device="cuda"), E, dt, F * W, F)
+    x = torch.randn(R, W, device="cuda", generator=g).to(dt)
+    up = torch.empty(E, F, W, dtype=dt, device="cuda").normal_(0, W ** -0.5, generator=g)
+    down = torch.empty(E, W, F, dtype=dt, device="cuda").normal_(0, F ** -0.5, generator=g)
+    a = torch.empty(R, F, dtype=dt, device="cuda")
+    y = torch.empty(R, W, dtype=dt, device="cuda")
+    X.product(x, up, p, a)
+    X.product(a, down, p, y)
+    r0 = 0
+    for e, c in enumerate(counts):
+        for got, rows, w in ((a, x, up), (y, a, down)):
+            want = rows[r0:r0 + c].float() @ w[e].float().t()
+            tol = SIZE[dt] * want.abs() + max(F, W) * 2.0 ** -21 * (1 + want.abs())
+            assert bool(((got[r0:r0 + c].float() - want).abs() <= tol).all()), e
+        r0 += c
 
 
 # f32 results: fewer tiles than workgroups and more, pieces alone and behind whole tiles, bias and factor
