@@ -429,6 +429,162 @@ __global__ __launch_bounds__(384) void mixer_delta_scan_kernel(DeltaArgs a) {
   }
 }
 
+// One chunk's operands of a lane that loads them itself.
+template <int NI> struct ScanLane {
+  u32x4 kp[NI], qp[NI], t, p;
+  float kt[NI][4], v[4], g15;
+  cf32x4 gi, beta, ge;  // tokens 4 g .. 4 g + 3
+};
+
+// The same without waves of their own for operands and read-outs, four waves and 16 KB of LDS: of many sequences the chains
+// hide behind each other, and what counts is how many of them a CU holds (128 x 128 take six waves and 77 KB above); of one
+// chunk there is nothing to ask for ahead.  The same bits.  The mixer's prompt kernels with this scan and with the other, 32
+// heads of 128 x 128: 64 sequences of 10 / 40 / 300 tokens 160 / 319 / 1688 us, 212 / 363 / 1862; 8 of 300 211, 196; 16 heads of
+// 192 x 192, 64 of 10 / 40 / 300 197 / 365 / 1797, 264 / 402 / 1671; of 256 x 256 303 / 555 / 2703, 370 / 571 / 2541.
+template <int DT, int NI>
+__global__ __launch_bounds__(256) void mixer_delta_scan_many_kernel(DeltaArgs a) {
+  using E = typename St<DT>::E;
+  constexpr int DR = 64 * NI;
+  __shared__ __attribute__((aligned(16))) float ex[2][4][2][64][4];
+  const SeqRow sq = a.seq[blockIdx.z];
+  const int h = blockIdx.x, R = a.H / a.G, gh = h / R, c0 = blockIdx.y * 16;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
+  const int col = c0 + l15;
+  const bool cok = col < a.vdim;
+  const int r0 = 16 * NI * wave;
+  float* st = a.state + sq.slot * a.s_slot + (long long)h * a.dim * a.EP;
+  cf32x4 S[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = r0 + 16 * i + 4 * g + e;
+      S[i][e] = sq.pos0 > 0 && cok && r < a.dim ? st[(long long)r * a.EP + col] : 0.f;
+    }
+  const int nc = (sq.len + kChunk - 1) / kChunk, ch0 = a.chunk0[blockIdx.z];
+  // A chunk's operands: a uniform base that moves with the chunk plus a lane offset that does
+  // not.  Rows past a sequence's end are another sequence's or zeros (prep) and count nothing:
+  // their beta is zero.
+  const unsigned krow = (unsigned)a.G * DR, vrow = (unsigned)a.H * a.vdim;
+  const unsigned koff = l15 * krow + r0 + 4 * g, toff = 16 * l15 + 4 * g;
+  unsigned ktoff[4], voff[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    ktoff[e] = (4 * g + e) * krow + r0 + l15;
+    voff[e] = (4 * g + e) * vrow + (cok ? col : 0);
+  }
+  const float* kbase = a.kn + ((long long)sq.row0 * a.G + gh) * DR;
+  const float* qbase = a.qn + ((long long)sq.row0 * a.G + gh) * DR;
+  const float* vbase = a.vv + (long long)sq.row0 * vrow + (long long)h * a.vdim;
+  const float* tbase = a.tp + ((long long)ch0 * a.H + h) * 512;
+  const float* gbase = a.gm + ((long long)ch0 * a.H + h) * 64;
+  auto load = [&](ScanLane<NI>& s, int c) __attribute__((always_inline)) {
+    const float* kb = kbase + (long long)c * kChunk * krow;
+    const float* qb = qbase + (long long)c * kChunk * krow;
+    const float* vb = vbase + (long long)c * kChunk * vrow;
+    const float* tb = tbase + (long long)c * a.H * 512;
+    const float* gb = gbase + (long long)c * a.H * 64;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      s.kp[i] = *reinterpret_cast<const u32x4*>(kb + koff + 16 * i);
+      s.qp[i] = *reinterpret_cast<const u32x4*>(qb + koff + 16 * i);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s.v[e] = vb[voff[e]];
+    s.gi = *reinterpret_cast<const cf32x4*>(gb + 4 * g);
+    s.beta = *reinterpret_cast<const cf32x4*>(gb + 16 + 4 * g);
+    s.t = *reinterpret_cast<const u32x4*>(tb + toff);
+    s.ge = *reinterpret_cast<const cf32x4*>(gb + 32 + 4 * g);
+    s.g15 = gb[48];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s.kt[i][e] = kb[ktoff[e] + 16 * i];
+    s.p = *reinterpret_cast<const u32x4*>(tb + 256 + toff);
+  };
+  auto chunk = [&](const ScanLane<NI>& s, int c) __attribute__((always_inline)) {
+    const int buf = c & 1;
+    cf32x4 ks{0.f, 0.f, 0.f, 0.f}, qs{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const uint4 sb = __builtin_bit_cast(uint4, S[i]);
+      ks = mm_piece<kF32>(__builtin_bit_cast(uint4, s.kp[i]), sb, ks);
+      qs = mm_piece<kF32>(__builtin_bit_cast(uint4, s.qp[i]), sb, qs);
+    }
+    *reinterpret_cast<cf32x4*>(ex[buf][wave][0][lane]) = ks;
+    *reinterpret_cast<cf32x4*>(ex[buf][wave][1][lane]) = qs;
+    // the other waves' halves only need the LDS writes: a full barrier would also drain the
+    // operand loads in flight
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    ks = *reinterpret_cast<const cf32x4*>(ex[buf][0][0][lane]);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) ks += *reinterpret_cast<const cf32x4*>(ex[buf][w][0][lane]);
+    cf32x4 rhs;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rhs[e] = s.beta[e] * (s.v[e] - s.gi[e] * ks[e]);
+    const cf32x4 u = mm_piece<kF32>(__builtin_bit_cast(uint4, s.t), __builtin_bit_cast(uint4, rhs),
+                                    cf32x4{0.f, 0.f, 0.f, 0.f});
+    cf32x4 ud;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ud[e] = s.ge[e] * u[e];
+    const uint4 ub = __builtin_bit_cast(uint4, ud);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const cf32x4 ka = {s.kt[i][0], s.kt[i][1], s.kt[i][2], s.kt[i][3]};
+      S[i] = mm_piece<kF32>(__builtin_bit_cast(uint4, ka), ub, S[i] * s.g15);
+    }
+    if (wave == (c & 3)) {  // the read-outs of a chunk: the waves take turns
+      qs = *reinterpret_cast<const cf32x4*>(ex[buf][0][1][lane]);
+#pragma unroll
+      for (int w = 1; w < 4; ++w) qs += *reinterpret_cast<const cf32x4*>(ex[buf][w][1][lane]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qs[e] *= s.gi[e];
+      const cf32x4 o = mm_piece<kF32>(__builtin_bit_cast(uint4, s.p), __builtin_bit_cast(uint4, u), qs);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = kChunk * c + 4 * g + e;
+        if (cok && t < sq.len) a.o[((long long)(sq.row0 + t) * a.H + h) * a.vdim + col] = o[e];
+      }
+    }
+  };
+  // operands two chunks ahead (chunks past the end re-read the last one)
+  ScanLane<NI> s0, s1;
+  load(s0, 0);
+  load(s1, min(1, nc - 1));
+  // once: with loads pending on the way in, the compiler waits for the newest loads in every
+  // round (its counts cover both ways into the loop)
+  __builtin_amdgcn_s_waitcnt(vm_wait(0));
+  for (int c = 0; c < nc; c += 2) {
+    chunk(s0, c);
+    if (c + 1 >= nc) break;
+    load(s0, min(c + 2, nc - 1));
+    chunk(s1, c + 1);
+    load(s1, min(c + 3, nc - 1));
+  }
+  if (cok)
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = r0 + 16 * i + 4 * g + e;
+        if (r < a.dim) st[(long long)r * a.EP + col] = S[i][e];
+      }
+  // the ring entries of the last taps - 1 tokens (every prompt row has been convolved by now)
+  if (blockIdx.y != 0) return;
+  const int C = delta_channels(a);
+  float* ring = a.ring + sq.slot * a.r_slot;
+  const int keep = min(a.taps - 1, sq.len);
+  const int nq = h % R == 0 ? 2 * a.dim : 0;  // q and k channels: the group's first head
+  for (int i = tid; i < keep * (nq + a.vdim); i += 256) {
+    const int j = i / (nq + a.vdim), x = i - j * (nq + a.vdim);
+    const int cc = x < nq ? (x < a.dim ? gh * a.dim + x : (a.G + gh) * a.dim + x - a.dim)
+                          : 2 * a.G * a.dim + h * a.vdim + x - nq;
+    const int row = sq.len - 1 - j;
+    ring[(long long)((sq.pos0 + row) % a.taps) * C + cc] =
+        St<DT>::ld(reinterpret_cast<const E*>(a.proj)[(long long)(sq.row0 + row) * a.ldp + cc]);
+  }
+}
+
 // a wave per (row, head): o / rms(o) * norm_w * silu(gate)
 template <int DT>
 __global__ __launch_bounds__(256) void mixer_delta_out_kernel(DeltaArgs a) {
@@ -511,6 +667,11 @@ CAKE_API int cake_mixer_delta_prefill(int dt, const void* proj, long long ldp, c
   const dim3 gp((unsigned)(((long long)NC * (2 * G + H) + 3) / 4));
   const dim3 gs(H, (vdim + 15) / 16, B);
   const dim3 go((unsigned)(((long long)N * H + 3) / 4));
+  // mixer_delta_scan_many: one chunk a sequence; more workgroups than fit at once, where it fits more of them (128 wide) or the
+  // chains have up to three chunks
+  const long long wgs = (long long)H * gs.y * B;
+  const bool few_chunks = NC <= 3LL * B;
+  const bool many = NC == B || (ni == 2 && wgs > 4096) || (few_chunks && wgs > (ni == 2 || ni == 3 ? 2048 : 16384));
   const int widest = 64 * ni > vdim ? 64 * ni : vdim;
   const int vec = dim % 2 == 0 && vdim % 2 == 0 && ldp % 2 == 0 && ((uintptr_t)proj % 4) == 0;
 #define CAKE_PREP1(CPL, W) \
@@ -521,14 +682,16 @@ CAKE_API int cake_mixer_delta_prefill(int dt, const void* proj, long long ldp, c
     else if (widest <= 128) CAKE_PREP1(2, W); \
     else CAKE_PREP1(4, W);                  \
   } while (0)
+#define CAKE_SCAN(NI)                                                                               \
+  if (ni == NI) {                                                                                   \
+    if (many) hipLaunchKernelGGL((mixer_delta_scan_many_kernel<DT, NI>), gs, dim3(256), 0, st, a);  \
+    else hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, NI>), gs, dim3(384), 0, st, a);            \
+  }
   CAKE_MIX_DT(dt, {
     if (taps <= 4) CAKE_PREP(4); else CAKE_PREP(8);
     hipLaunchKernelGGL(mixer_delta_chunk_kernel, dim3((unsigned)(((long long)NC * G + 3) / 4)),
                        dim3(256), 0, st, a);
-    if (ni == 1) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 1>), gs, dim3(384), 0, st, a);
-    else if (ni == 2) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 2>), gs, dim3(384), 0, st, a);
-    else if (ni == 3) hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 3>), gs, dim3(384), 0, st, a);
-    else hipLaunchKernelGGL((mixer_delta_scan_kernel<DT, 4>), gs, dim3(384), 0, st, a);
+    CAKE_SCAN(1) CAKE_SCAN(2) CAKE_SCAN(3) CAKE_SCAN(4)
     hipLaunchKernelGGL((mixer_delta_out_kernel<DT>), go, dim3(256), 0, st, a);
   });
   return (int)hipGetLastError();
