@@ -11,10 +11,44 @@
 
 namespace cake {
 
-template <int DT, int U, int PFC, int NX, int NT = kGemvThreads>
-__global__ __launch_bounds__(NT) void mixer_in_kernel(MixInArgs a) {
+template <int DT, int U, int PFC, int NX>
+__global__ __launch_bounds__(kGemvThreads) void mixer_in_kernel(MixInArgs a) {
   extern __shared__ float xs[];
-  mixer_in_rows<DT, U, PFC, NX, NT>(a, blockIdx.x, gridDim.x, xs);
+  mixer_in_rows<DT, U, PFC, NX, kGemvThreads>(a, blockIdx.x, gridDim.x, xs);
+}
+
+// Up to a workgroup a CU: a wave has one pair, and all R rounds of 512 columns of it are asked for before the norm.  Rounds
+// behind it are round trips of their own, and with one workgroup on a CU nothing hides them.  A few more pairs than four
+// waves a CU take: five, so that no CU has two workgroups.  2048 rows of 1536 / 2560 / 3584 / 4096 columns, two or four rounds
+// before the norm, 3.9 / 4.8 / 5.9 / 6.7 us, 3.7 / 4.6 / 5.5 / 6.1 so; 2560 rows 4.3 / 5.6 / 6.6 / 7.1, 4.0 / 5.0 / 6.0 / 6.4; 3072
+// of 4096 on five waves 8.4, on four with the whole pair asked for 7.6, as mixer_in_kernel has them 7.4.
+template <int DT, int R, int NT>
+__global__ __launch_bounds__(NT) void mixer_in_pair_kernel(MixInArgs a) {
+  extern __shared__ float xs[];
+  constexpr int NX = (R * 512 + 4 * NT - 1) / (4 * NT);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nch = a.K >> 3, npairs = mixer_in_pairs(a);
+  const int p = blockIdx.x * (NT / 64) + wave, at = min(p, npairs - 1);
+  const uint4* wa = reinterpret_cast<const uint4*>(a.w + (size_t)(2 * at) * a.K);
+  const uint4* wb = reinterpret_cast<const uint4*>(a.w + (size_t)min(2 * at + 1, a.N - 1) * a.K);
+  NormPre<DT, NX, NT> xp;
+  xp.load(a.resid, a.norm_w, a.K);
+  __builtin_amdgcn_sched_barrier(0);
+  uint4 va[R], vb[R];
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    const int i = c + 1 < R ? c * 64 + lane : min(c * 64 + lane, nch - 1);
+    va[c] = ld_nt16(wa + i);
+    vb[c] = ld_nt16(wb + i);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  xp.finish_off(a.eps, a.K, a.Kn, a.off, a.ln, xs);
+  float da = 0.f, db = 0.f;
+#pragma unroll
+  for (int c = 0; c < R; ++c)
+    if (c + 1 < R || c * 64 + lane < nch) fma_chunk<DT, true>(xs, c * 64 + lane, va[c], vb[c], da, db);
+  da = wave_sum(da);
+  db = wave_sum(db);
+  if (p < npairs) mixer_in_store<DT>(a, p, da, db, lane);
 }
 
 // Few rows (a router's): a workgroup has one pair of them, each of its waves a quarter of k.  With a pair a wave, the
@@ -52,12 +86,8 @@ __global__ __launch_bounds__(kGemvThreads) void mixer_in_split_kernel(MixInArgs 
     part[1][wave] = db;
   }
   __syncthreads();
-  const int r = 2 * blockIdx.x + threadIdx.x;
-  if (threadIdx.x > 1 || r >= a.N) return;
-  const float* q = part[threadIdx.x];
-  const float d = (q[0] + q[1]) + (q[2] + q[3]);
-  if (r < a.n_raw) a.out[r] = d;
-  else a.act[r - a.n_raw] = from_f32<DT>(mix_act(a.actf, a.bias ? d + to_f32<DT>(a.bias[r - a.n_raw]) : d));
+  const float *qa = part[0], *qb = part[1];
+  mixer_in_store<DT>(a, blockIdx.x, (qa[0] + qa[1]) + (qa[2] + qa[3]), (qb[0] + qb[1]) + (qb[2] + qb[3]), threadIdx.x);
 }
 
 // y[r] = x[r] + alpha ((W a)[r] + bias[r]), a 16-bit; bias may be null
@@ -155,22 +185,25 @@ CAKE_API int cake_mixer_in(int dt, const float* resid, const void* norm_w, float
   const int g = grid_for((N + 1) / 2, 1024);
   const MixInArgs a{resid, (const uint16_t*)norm_w, (const uint16_t*)w, out, (const uint16_t*)bias,
                     (uint16_t*)act, eps, off, ln, Kn, K, N, n_raw, actf};
-  // few rows: above; up to a workgroup a CU: all of a pair is asked for before the norm, and of a few more pairs than
-  // those take, five waves have one each, so that no CU has two workgroups (2048 / 2112 / 2560 rows of 4096 6.6 / 6.8 /
-  // 7.2 us, 5.9 / 6.0 / 6.5 so; 3072 on five waves 8.4, on four with the whole pair asked for 7.6, 7.4 as below)
-  if (K / 8 >= 128 && K <= 4096 && N <= 1024) {
-    const int gs = (N + 1) / 2;
+  // few rows and up to a workgroup a CU: above
+  if (K >= 1024 && K <= 4096 && N <= 1024) {
+    const int gs = mixer_in_pairs(a);
     DISPATCH_DT(dt, if (K <= 2048) CAKE_MIX_LAUNCH((mixer_in_split_kernel<DT, 1, 2>), gs, lds, a);
                 else CAKE_MIX_LAUNCH((mixer_in_split_kernel<DT, 2, 4>), gs, lds, a));
   }
-  if (K == 4096 && N <= 2048) DISPATCH_DT(dt, CAKE_MIX_LAUNCH((mixer_in_kernel<DT, 2, 8, 4>), g, lds, a));
-  if (K >= 2048 && K <= 4096 && N > 2048 && N <= 2560) {
-    const int g5 = ((N + 1) / 2 + 4) / 5;
-#define CAKE_MIN5(PF)                                                                                        \
-  hipLaunchKernelGGL((mixer_in_kernel<DT, 2, PF, 4, 320>), dim3(g5), dim3(320), lds, st, a);                 \
-  return (int)hipGetLastError()
-    DISPATCH_DT(dt, if (K == 4096) { CAKE_MIN5(8); } else { CAKE_MIN5(4); });
-#undef CAKE_MIN5
+  if (K >= 1024 && K <= 4096 && N <= 2560) {
+    const int rounds = (K + 511) / 512, waves = N <= 2048 ? 4 : 5;
+#define CAKE_PAIR(R, W)                                                                                            \
+  if (rounds == R && waves == W) {                                                                                 \
+    hipLaunchKernelGGL((mixer_in_pair_kernel<DT, R, 64 * W>), dim3((mixer_in_pairs(a) + W - 1) / W), dim3(64 * W), \
+                       lds, st, a);                                                                                \
+    return (int)hipGetLastError();                                                                                 \
+  }
+#define CAKE_PAIRS(W) \
+  CAKE_PAIR(2, W) CAKE_PAIR(3, W) CAKE_PAIR(4, W) CAKE_PAIR(5, W) CAKE_PAIR(6, W) CAKE_PAIR(7, W) CAKE_PAIR(8, W)
+    DISPATCH_DT(dt, CAKE_PAIRS(4) CAKE_PAIRS(5));
+#undef CAKE_PAIRS
+#undef CAKE_PAIR
   }
 #define CAKE_MIN(PF, NX) CAKE_MIX_LAUNCH((mixer_in_kernel<DT, 2, PF, NX>), g, lds, a)
   DISPATCH_DT(dt, if (K / 8 < 128) CAKE_MIN(0, 0); else if (K / 8 < 256) CAKE_MIN(2, 2);

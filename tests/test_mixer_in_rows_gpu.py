@@ -34,6 +34,13 @@ def test_rows(cuda, dt, N, K, ln):
     assert bool((act[N - n_raw:] == 5.0).all())
 
 
+# every number of rounds that a pair has, their ends met and not
+@pytest.mark.parametrize("N", [1025, 2049, 2560])
+@pytest.mark.parametrize("K", [1536, 1544, 2552, 2560, 3064, 3072, 3576, 3584, 3592])
+def test_rounds_of_a_pair(cuda, N, K):
+    test_rows(cuda, torch.bfloat16, N, K, False)
+
+
 # whole rounds of 512 columns past the ones asked for ahead, one to three over, and pieces of a round
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
 @pytest.mark.parametrize("K", [2048, 2056, 2560, 3072, 3584, 4096, 4104, 6144, 11776, 29696, 30200])
