@@ -478,7 +478,7 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_x16_kernel(
     if (ACCUM) out[ra] = da + (p == p0 ? r0a : out[ra]); else out[ra] = da;
     if (rb < N) { if (ACCUM) out[rb] = db + (p == p0 ? r0b : out[rb]); else out[rb] = db; }
   };
-  run_pairs<DT, false, U, PFC, true>(map, epi, xs, K, npairs, p0, gridDim.x * kGemvWaves, pre);
+  run_pairs<DT, false, U, PFC, (U > 2)>(map, epi, xs, K, npairs, p0, gridDim.x * kGemvWaves, pre);
 }
 
 // Greedy token selection fused into the lm_head (SEL): repeat penalty on the logits of

@@ -23,7 +23,8 @@ CAKE_API int cake_gemv_x16(int dt, const void* x, const void* w, int K, int N, f
                            int accumulate, hipStream_t st) {
   if (K % 8) return (int)hipErrorInvalidValue;
   const size_t lds = (size_t)K * 2;
-  const GemvTune t = g_tune[K <= 8192 ? kX16S : kX16];
+  GemvTune t = g_tune[K <= 8192 ? kX16S : kX16];
+  if (K <= 1024) t.U = 2;   // (2048 rows of 512 / 1024 2.9 / 3.3 us, as left over of four 3.1 / 3.5)
   const int g = grid_for((N + 1) / 2, t.MB);
   if (accumulate) {
     DISPATCH_DT(dt, DISPATCH_TUNE(t, K, CAKE_NX_X16(K, hipLaunchKernelGGL((gemv_x16_kernel<DT, U, PF, NX, true>),

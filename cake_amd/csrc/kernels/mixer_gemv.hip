@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kGemvThreads) void mixer_out_kernel(
     const float d = (lane == 0 ? da : db) + (bias ? to_f32<DT>(bias[r]) : 0.f);
     y[r] = fmaf(alpha, d, p == p0 ? r0 : x[r]);
   };
-  run_pairs<DT, false, U, PFC, true>(map, epi, xs, K, npairs, p0, gridDim.x * kGemvWaves, pre);
+  run_pairs<DT, false, U, PFC, (U > 2)>(map, epi, xs, K, npairs, p0, gridDim.x * kGemvWaves, pre);
 }
 
 // y = W [x ; x0] + step (x, x0 f32 [W] each; w [W][K], K = 2 W padded to 8); y is neither
@@ -220,6 +220,10 @@ CAKE_API int cake_mixer_out(int dt, const void* a, const void* w, int K, int N, 
 #define CAKE_MOUT(PF, NX)                                                                   \
   CAKE_MIX_LAUNCH((mixer_out_kernel<DT, 4, PF, NX>), g, lds, (const uint16_t*)a,            \
                   (const uint16_t*)w, K, N, alpha, (const uint16_t*)bias, x, y)
+  // (one or two rounds of 512 columns: 2048 rows of 512 / 1024 2.6 / 3.0 us, as left over of four 2.8 / 3.2)
+  if (K <= 1024)
+    DISPATCH_DT(dt, CAKE_MIX_LAUNCH((mixer_out_kernel<DT, 2, 0, 0>), g, lds, (const uint16_t*)a, (const uint16_t*)w, K, N,
+                                    alpha, (const uint16_t*)bias, x, y));
   DISPATCH_DT(dt, if (K / 8 < 256) CAKE_MOUT(0, 0); else if (K <= 4096) CAKE_MOUT(4, 2);
               else if (K <= 8192) CAKE_MOUT(4, 4); else if (K <= 16384) CAKE_MOUT(4, 8);
               else if (K <= 28672) CAKE_MOUT(4, 14); else CAKE_MOUT(4, 0));

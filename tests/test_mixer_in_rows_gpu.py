@@ -59,3 +59,9 @@ def test_rounds_left_over(cuda, dt, K):
     r = x.clone()
     K32.gemv(a, w, r, accumulate=True)
     assert bool(((r.double() - x.double() - want).abs() <= K * 2.0 ** -22 * (1 + want.abs())).all())
+
+
+# columns of one and of two rounds, which are not asked for as left over
+@pytest.mark.parametrize("K", [8, 504, 512, 520, 1016, 1024, 1032])
+def test_up_to_two_rounds(cuda, K):
+    test_rounds_left_over(cuda, torch.bfloat16, K)
