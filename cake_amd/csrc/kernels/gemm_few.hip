@@ -251,13 +251,15 @@ static int run_few(int dt, const FewArgs& g, hipStream_t st) {
 
 using namespace cake;
 
-// Whether the output product [H][K] and the gated one [2 I][H] of M rows are better off here.  Of H 512 .. 3072, K
-// 512 .. 4096, I 2048 .. 14336 they always are (0.70 .. 0.99 of the time, 0.99 at 2048 x 4096 / 11008 and 3072 x 4096 / 14336
-// of 8 rows); 4096 wide ones at 5 rows are not (output 9.9 us and norm in the next, 8.2 and 3.5; 28672 x 4096 38.1 and its
-// norm, 37.6): a workgroup's x is as much as its weights, and the stream form moves those as fast.
+// Whether the output product [H][K] and the gated one [2 I][H] of M rows are better off here: of H 32 .. 3072, K 64 .. 4096,
+// I 64 .. 43000 within this line a block takes 0.79 .. 1.02 of the time.  Below 1024 columns some of a workgroup's eight waves
+// have none, and many narrow rows are many of its turns: a block of H 256, I 2048 / 8192 / 32768 at 5 rows 24.2 / 27.5 / 36.5
+// us in launches of its own, 23.5 / 28.8 / 43.9 here; H 512, I 4096 / 16384 27.9 / 34.4, 27.4 / 36.7.  4096 wide ones at 5 rows
+// are not better off (output 9.9 us and norm in the next, 8.2 and 3.5; 28672 x 4096 38.1 and its norm, 37.6): a workgroup's x
+// is as much as its weights, and the stream form moves those as fast.
 CAKE_API int cake_gemm_few_pair(int M, int H, int K, long long I) {
   return M >= 1 && M <= kFewRows && H >= 8 && H <= kFewNormK && H % 8 == 0 && K >= 8 && K <= 4096 && K % 8 == 0 && I >= 1 &&
-         I * H <= 44LL << 20;
+         I * H <= 44LL << 20 && (H >= 1024 || I <= 12LL * H);
 }
 
 // r [M][ldr] += a [M][lda] b^T, b [N][ldb]; M <= 8, rows of a and b on 16 bytes
