@@ -204,9 +204,11 @@ def slab_form(M: int, N: int, K: int, epi: str, big: bool = False):
 
 def few_pair(M: int, H: int, K: int, inter: int) -> bool:
     """Whether a block's output product (rows of K to H, added to the residual rows) and its gated product of the
-    normed rows (H to `inter`) run as :func:`few_add` and :func:`few_gated` (gemm_few.hip); pinned plans run as pinned."""
-    return (M, H, K, "resid32") not in _plans and (M, 2 * inter, H, "swiglu") not in _plans and \
-        bool(_lib().cake_gemm_few_pair(M, H, K, inter))
+    normed rows (H to `inter`) run as :func:`few_add` and :func:`few_gated` (gemm_few.hip); pinned plans run as pinned,
+    the library's as its own."""
+    both = ((M, H, K, "resid32"), (M, 2 * inter, H, "swiglu"))
+    return not any(p in _plans for p in both) and bool(_lib().cake_gemm_few_pair(M, H, K, inter)) and \
+        all(rows_kind(m, n, k, e == "swiglu") or resolve(m, n, k, e)[0] != LIB for m, n, k, e in both)
 
 
 def few_add(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor) -> None:

@@ -11,3 +11,12 @@ from cake_amd.ops import gemm as G
     (5, 1016, 1024, 12192, True), (5, 1016, 1024, 12208, False), (5, 1024, 1024, 16384, True), (5, 32, 32, 64, True)])
 def test_the_line(M, H, K, inter, takes):
     assert G.few_pair(M, H, K, inter) == takes
+
+
+def test_the_librarys_plan_is_its_own(monkeypatch):
+    """A measured plan that names the library GEMM stands, as for every product, where no form of few rows does."""
+    M, H, K, inter = 3, 64, 32, 128
+    assert G.few_pair(M, H, K, inter)
+    monkeypatch.setattr(G, "rows_kind", lambda *a: 0)
+    monkeypatch.setattr(G, "resolve", lambda m, n, k, epi, *a, **kw: (G.LIB if epi == "swiglu" else 4, 1))
+    assert not G.few_pair(M, H, K, inter)
