@@ -32,9 +32,14 @@ class _Run(C.Structure):
 def _forms(products, capturing: bool):
     """(kind, cfg, splits) of each (rows, Nv, K, epi, summed), as gemm.linear chooses them or, of those
     that a sum of slabs may follow, as gemm.slab_form does; the floats that the tile plans' slabs need,
-    and those of the products that leave them.  None if one of them is the library GEMM's."""
+    and those of the products that leave them.  None if one of them is the library GEMM's.  A product may be
+    None: it has no form."""
     forms, floats, left = [], 0, 0
-    for T, Nv, K, epi, summed in products:
+    for p in products:
+        if p is None:
+            forms.append(_Form())
+            continue
+        T, Nv, K, epi, summed = p
         gated = epi == "swiglu"
         big = max(T, Nv) * K * 2 >= 0x7fffffff
         slab = G.slab_form(T, Nv, K, epi, big) if summed else None
@@ -110,11 +115,13 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
     if not blocks or not takes_tail(T, tail, nqkv * H + H * nq + 3 * inter * H):
         tail = 0
 
-    def behind(rows):   # the products behind the attention
-        return ((rows, H, nq, "resid32", adds), (rows, 2 * inter, H, "swiglu", False),
-                (rows, H, inter, "resid32", adds))
-    forms, floats, left = _forms(((T, nqkv, H, "store", True), *behind(T)) + (() if not tail else (
-        (T, 2 * nk, H, "store", False), (tail, nq, H, "store", False), *behind(tail))), capturing)
+    few, few1 = G.few_pair(T, H, nq, inter), G.few_pair(tail, H, nq, inter)
+
+    def behind(rows, few):   # the products behind the attention
+        pair = (None, None) if few else ((rows, H, nq, "resid32", adds), (rows, 2 * inter, H, "swiglu", False))
+        return (*pair, (rows, H, inter, "resid32", adds))
+    forms, floats, left = _forms(((T, nqkv, H, "store", True), *behind(T, few)) + (() if not tail else (
+        (T, 2 * nk, H, "store", False), (tail, nq, H, "store", False), *behind(tail, few1))), capturing)
     if forms is None:
         return False
     if not tail:
@@ -134,7 +141,6 @@ def block_rows(hidden: torch.Tensor, blocks: list, slots: list[int], k: torch.Te
     ptr = [None if t is None else t.data_ptr() for t in (
         hidden, x, qkv, att, act, inv_freq, G._zeros16(dev), ws, slabs, rows_ws, tick)]
     run = _Run(C.addressof(table), *ptr, *forms, len(blocks), G._DT[dt], T, H, inter, nh, nkv, hd, S,
-               int(pos0), int(tail), int(G.few_pair(T, H, nq, inter)), int(G.few_pair(tail, H, nq, inter)),
-               float(cfg.rms_norm_eps), float(scale))
+               int(pos0), int(tail), int(few), int(few1), float(cfg.rms_norm_eps), float(scale))
     check(kernels().cake_block_rows(C.addressof(run), st), "block_rows")
     return True

@@ -20,3 +20,10 @@ def test_the_librarys_plan_is_its_own(monkeypatch):
     monkeypatch.setattr(G, "rows_kind", lambda *a: 0)
     monkeypatch.setattr(G, "resolve", lambda m, n, k, epi, *a, **kw: (G.LIB if epi == "swiglu" else 4, 1))
     assert not G.few_pair(M, H, K, inter)
+
+
+def test_products_of_the_pair_have_no_form():
+    """A native run forms no plan for products that the pair's kernels run, and holds no workspace for them."""
+    from cake_amd.ops import llama_rows as L
+    forms, floats, left = L._forms(((5, 3072, 2048, "store", True), None, None, (5, 2048, 8192, "resid32", True)), False)
+    assert [(f.kind, f.cfg, f.splits, f.slabs) for f in forms[1:3]] == [(0, 0, 0, 0)] * 2 and forms[0].slabs
