@@ -238,7 +238,8 @@ def _counters(dev, st: int) -> torch.Tensor:
     """Arrival counters of a launch on stream `st`, the current one: zero between launches.
     Launches of one stream run one after the other and share them; launches that may run side by
     side never do.  A captured graph may run beside any stream, so its counters are its own: memory
-    of its pool, cleared by a fill at the head of every replay, as long-lived as the graph."""
+    of its pool, cleared by a fill at the head of every replay, as long-lived as the graph, and no more than
+    tiles in pieces need: the stream form stays out of graphs."""
     if not torch.cuda.is_current_stream_capturing():
         return _stream_counters(dev, st)
     capture = _lib().cake_stream_capture(st)
@@ -247,7 +248,7 @@ def _counters(dev, st: int) -> torch.Tensor:
     with _lock:
         have = _graph_ticks.get((dev, st))
         if have is None or have[0] != capture:
-            have = (capture, torch.zeros(_n_ticks(), dtype=torch.int32, device=dev))
+            have = (capture, torch.zeros(_lib().cake_gemm_ticks(), dtype=torch.int32, device=dev))
             _newest(_graph_ticks, (dev, st), have)
         return have[1]
 

@@ -141,3 +141,28 @@ def test_many_captures_keep_their_pieces(cuda):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(o, want) for o in outs)
+
+
+def test_a_graph_holds_the_counters_of_pieces(cuda):
+    """A captured product's counters are as many as tiles in pieces have, not the stream form's, which every replay would
+    clear too; pieces of the most tiles find them zero and leave them so."""
+    from cake_amd.ops import gemm as G
+    M, N, K = 4096, 4096, 1024
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = torch.randn(N, K, device="cuda").bfloat16() * K ** -0.5
+    G._graph_ticks.clear()
+    outs = []
+    for cfg, splits in ((22, 1), (35, 3)):
+        want = G.linear(x, w, epi="store32", resid=torch.empty(M, N, device="cuda"), cfg=cfg, splits=splits)
+        graph, out = torch.cuda.CUDAGraph(), torch.zeros(M, N, device="cuda")
+        with torch.cuda.graph(graph):
+            G.linear(x, w, epi="store32", resid=out, cfg=cfg, splits=splits)
+        outs.append((graph, out, want))
+    (_, ticks), = G._graph_ticks.values()
+    assert ticks.numel() == G._lib().cake_gemm_ticks() < G._lib().cake_gemm_rows_ticks()
+    for _ in range(3):
+        for graph, out, want in outs:
+            out.zero_()
+            graph.replay()
+            assert torch.equal(out, want)
+    assert not bool(ticks.any())
