@@ -38,17 +38,31 @@ SPLITS = ((256, 1), (1024, 8), (4096, 16), (1 << 30, 32))
 # the latent kernels' for the same buckets: a workgroup takes one 64-key tile while there are
 # splits for all of them
 LATENT_SPLITS = {n: min(M.MAX_SPLIT, -(-lim // 64)) for lim, n in SPLITS}
-# ... (splits, tile) of a sequence alone: of short contexts 32-key tiles
-LATENT_ALONE = {n: (8, 32) if n == 1 else (s, 64) for n, s in LATENT_SPLITS.items()}
+MERGE_BYTES = 3 << 19   # of split sums that the value expansion of a sequence alone reads
 
 
-def latent_splits(nsplit: int, rows: M.Rows, heads: int) -> int:
+def latent_alone(nsplit: int, sh: LA.LatentShape) -> tuple[int, int]:
+    """(splits, tile) of a sequence alone: of short contexts 32-key tiles, unless their sums are as much to read as the
+    tiles (128 heads of rank 512 over 40 / 150 / 250 keys 12.4 / 13.9 / 15.3 us, 13.0 / 14.3 / 14.5 in 64-key tiles; 64 heads
+    11.2 / 12.3 / 12.7, 12.1 / 13.0 / 13.2)."""
+    return (8, 32) if nsplit == 1 and 4 * sh.part_floats(1, 8) <= MERGE_BYTES else (LATENT_SPLITS[nsplit], 64)
+
+
+def latent_splits(nsplit: int, rows: M.Rows, heads: int, per_cu: int = 1) -> int:
     """Splits of a step's sequences: no more workgroups at the longest one's length than CUs, since the value expansion
     reads every split's sums (16 heads of 24 sequences at 600 / 3000 keys 38.6 us in 16 splits / 70.4 in 32, 30.5 / 44.4 in
-    8; 32 heads of 13 at 1000 45.4 in 16, 30.4 in 8; 32 heads of 2 at 3000 24.4 in 32, 25.1 in 16, 31.1 in 8)."""
+    8; 32 heads of 13 at 1000 45.4 in 16, 30.4 in 8; 32 heads of 2 at 3000 24.4 in 32, 25.1 in 16, 31.1 in 8).  While splits
+    hold four tiles and more, as many as CUs with `per_cu` each hold, and a tenth of the longest's keys counts nothing
+    (128 heads of rank 256 of 3 at 30000 142.9 in 8, 94.9 in 16, of rank 512 of one at 30000 and 12 at 100 146 in 16, 120
+    in 32; of rank 256 of 2 at 3000, two tiles a split, 21.8 in 16, 25.0 in 32)."""
     keys = [p0 + n for _, n, p0, _ in rows.host]
-    groups = -(-sum(keys) // max(keys)) * -(-heads // 16)   # as many sequences of the longest one's length
-    return min(LATENT_SPLITS[nsplit], 1 << max(1, 256 // groups).bit_length() - 1)
+    most, total, groups = max(keys), sum(keys), -(-heads // 16)
+    # as many sequences of the longest one's length
+    n = min(LATENT_SPLITS[nsplit], 1 << max(1, 256 // (-(-total // most) * groups)).bit_length() - 1)
+    room = 256 * per_cu // (-(-(10 * total - most) // (10 * most)) * groups)
+    while 2 * n <= min(LATENT_SPLITS[nsplit], room) and -(-most // (2 * n)) > 192:
+        n *= 2
+    return n
 
 
 # Rows of a step from which on the last run's unread ones are left out (:meth:`HybridModel._last_rows`);
@@ -237,7 +251,8 @@ class HybridModel:
                 self.product(h, w.w_in[w.n_main:w.n_raw], ab)
         a, b = self.pool.bufs[run.index]
         if isinstance(m, LatentMixer):
-            self._latent_rows(m, w, proj, rows, a, mix, latent_splits(nsplit, rows, w.shape.heads))
+            self._latent_rows(m, w, proj, rows, a, mix, latent_splits(nsplit, rows, w.shape.heads,
+                                                                            LA.decode_per_cu(w.shape, self.dtype)))
         elif isinstance(m, AttentionMixer):
             cs = self._rotation(m)
             if decode:
@@ -297,7 +312,7 @@ class HybridModel:
                           cfg.eps, m.scale, a, b, mix, nsplit, part, ticket, held=True)
         elif isinstance(m, LatentMixer):
             sh, c, cs = w.shape, w.consts, self._rotation(m)
-            splits = latent_splits(nsplit, rows, sh.heads)
+            splits = latent_splits(nsplit, rows, sh.heads, LA.decode_per_cu(sh, self.dtype))
             proj = torch.empty((N, w.n_main), device=dev, dtype=torch.float32)
             self.product(h, w.w_in[:w.n_main], proj)
             cq = torch.empty((N, sh.QP), device=dev, dtype=self.dtype)
@@ -527,7 +542,7 @@ class HybridModel:
             ka, kb = self.pool.bufs[run.index]
             proj = b.proj[:w.n_raw].view(1, -1)
             if isinstance(m, LatentMixer):
-                self._latent_decode(m, w, b, proj, ka, mix.view(1, -1), *LATENT_ALONE[nsplit])
+                self._latent_decode(m, w, b, proj, ka, mix.view(1, -1), *latent_alone(nsplit, w.shape))
             elif isinstance(m, AttentionMixer):
                 M.attn_decode(w.shape, proj, b.pos, b.seq_slot, self._rotation(m), m.qk_norm,
                               m.sink, m.gated, cfg.eps, m.scale, ka, kb, mix.view(1, -1), nsplit,

@@ -143,6 +143,14 @@ def absorb(sh: LatentShape, q, uk_t, pos, slot, cs, eps: float, kv_norm, cache, 
         "latent_absorb")
 
 
+def decode_per_cu(sh: LatentShape, dtype) -> int:
+    """Workgroups of :func:`decode` in 64-key tiles that a CU's LDS holds (mixer_latent.hip launch_latent_decode)."""
+    f32 = dtype == torch.float32
+    size, piece = (4, 4) if f32 else (2, 8)
+    tile = (32 if f32 else 64) // (2 if sh.RP > 512 or sh.LD > 640 else 1)
+    return max(1, 160 * 1024 // (((tile + 16) * (sh.LD + piece) + 16 * (tile + piece)) * size))
+
+
 def decode(sh: LatentShape, qa, pos, slot, cache, scale: float, nsplit: int, part, tile: int = 64):
     """Attention of one token per sequence over its cache rows 0 .. pos, split over the keys in whole tiles
     of 32 or 64; the splits' sums go to part."""
