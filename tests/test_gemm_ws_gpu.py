@@ -49,6 +49,32 @@ def test_groups_of_every_height(cuda, dt, cfg, bm, N, K):
     _groups(cuda, dt, cfg, counts, N, K, bm, K + 8)
 
 
+@pytest.mark.parametrize("dt", list(SIZE), ids=str)
+@pytest.mark.parametrize("bm", [160, 192, 224, 256])
+@pytest.mark.parametrize("E", [2, 9], ids=["few", "many"])
+@pytest.mark.parametrize("epi", ["silu", "quick_gelu", "gelu", "relu2"])
+def test_activations(cuda, dt, bm, E, epi):
+    """As routed experts run them, on narrow tiles of few and on all of many: one rounding (2^-8, 2^-11) of f32 sums, the
+    activation's own 2^-10 and its factor of at most 2 on what the sums differ by."""
+    from cake_amd.ops import gemm as G
+    N, K = 2600, 1096
+    counts = [bm, bm - 1, bm + 1, 0, 3, 2 * bm, 17, 5 * bm, bm][:E]
+    R = sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(bm)
+    x = torch.randn(R, K, device="cuda", generator=g).to(dt)
+    w = torch.empty(E, N, K, dtype=dt, device="cuda").normal_(0, K ** -0.5, generator=g)
+    tiles = _tiles(counts, bm)
+    t = torch.tensor(tiles + [[0, 0, 0, 0], [len(tiles), bm, 0, 0]], dtype=torch.int32, device="cuda")
+    out = torch.full((R, N + 8), 7.0, dtype=dt, device="cuda")
+    G.grouped(x, w, t, 6, out[:, :N], epi=epi)
+    F = torch.nn.functional
+    act = {"silu": F.silu, "gelu": F.gelu, "quick_gelu": lambda y: y * torch.sigmoid(1.702 * y), "relu2": lambda y: F.relu(y).square()}[epi]
+    y = torch.cat([x[r:r + c].float() @ w[e].float().t() for e, (r, c) in enumerate(zip([sum(counts[:e]) for e in range(E)], counts))])
+    want = act(y.double())
+    tol = (SIZE[dt] + 2.0 ** -10) * want.abs() + 2 * K * 2.0 ** -21 * (1 + y.abs())
+    assert bool((out[:, N:] == 7.0).all()) and bool(((out[:, :N].double() - want).abs() <= tol).all())
+
+
 @pytest.mark.parametrize("bm", [160, 192, 224, 256])
 def test_more_tiles_than_workgroups_on_cold_weights(cuda, bm):
     """Several tiles a workgroup, one after the other, whose weights no cache holds (0.5 GB): all that a step
