@@ -15,12 +15,12 @@
 //   arrive sums in share order (the result does not hang on the order).  28672 x 4096 SwiGLU at 5 / 24 /
 //   45 rows 38 / 38 / 40 us (tile kernels 58-60 us), 4096 x 23552 33 / 37 / 43 us (44-46 us), 57344 x 8192
 //   140 us (6.7 TB/s).  What bounds it is the memory in whole strips, in parts the parked sums; weight
-//   rings of a wave's own with a barrier every four steps only ran at the same rate.  Of 128-row strips four waves ask and four
-//   multiply: loads go on while a strip's sums are parked, summed and stored, and every multiplying wave parks for itself
-//   (in one: 28672 x 4096 SwiGLU at 5 rows 39.9 -> 38.4 us, 6144 x 4096 in quarters at 45 15.0 -> 14.0, 4096 x 4096 in
-//   eighths 11.8 -> 11.1).  Strips of 64 rows are short and met by up to 60 shares: their four waves ask and multiply in turn
-//   (at 5 rows, in two kinds: 1024 x 4096 8.2, 8.9; 256 x 11008 10.6, 12.6; 1536 x 8960 14.0, 15.7; 2048 x 8192 10.7, 11.3;
-//   5120 x 5120 13.8, 13.4; 8192 x 28672 70.7, 70.5).
+//   rings of a wave's own with a barrier every four steps only ran at the same rate.  Of 128-row strips, and where sums stay in
+//   slabs, four waves ask and four multiply: loads go on while a strip's sums are parked, summed and stored, and every
+//   multiplying wave parks for itself (in one: 28672 x 4096 SwiGLU at 5 rows 39.9 -> 38.4 us, 6144 x 4096 in quarters at 45
+//   15.0 -> 14.0, 4096 x 4096 in eighths 11.8 -> 11.1).  Strips of 64 rows whose sums meet are short and met by up to 60 shares:
+//   their four waves ask and multiply in turn (at 5 rows, in two kinds: 1024 x 4096 8.2, 8.9; 256 x 11008 10.6, 12.6; 1536 x
+//   8960 14.0, 15.7; 2048 x 8192 10.7, 11.3; 5120 x 5120 13.8, 13.4; 8192 x 28672 70.7, 70.5).
 #pragma once
 #include "gemm_kernel.h"
 
@@ -198,8 +198,6 @@ template <int MT, bool WIDE> struct StreamShape {
   static constexpr int NWV = 4, RT = WIDE ? 2 : 1, KC = WIDE ? 1 : 2;   // row tiles, 64-element chunks
   static constexpr int BN = NWV * 16 * RT, KST = 64 * KC;   // weight rows of a strip, k of a step
   static constexpr int NS = WIDE ? 4 : 3, WGS = WIDE ? 256 : 512;
-  static constexpr bool ASK = WIDE;   // four more waves ask for what these multiply
-  static constexpr int THREADS = (ASK ? 2 : 1) * 64 * NWV;
   static constexpr int LPR = 8 * KC, RPI = 64 / LPR;   // lanes of a row's DMA, rows of an instruction
   static constexpr int XT = 2 * MT * KC;               // x DMA instructions of a step
   static constexpr int XW = XT % 4 == 0 ? 4 : XT % 3 == 0 ? 3 : 2;   // waves that issue them
@@ -212,6 +210,9 @@ template <int MT, bool WIDE> struct StreamShape {
 template <int EPI, int MT> constexpr bool stream_wide() {
   return MT > 1 || EPI == kEpiSwiglu || EPI == kEpiGeglu;
 }
+// four more waves ask for what these multiply
+template <int EPI, int MT> constexpr bool stream_ask() { return stream_wide<EPI, MT>() || EPI == kEpiPartial; }
+template <int EPI, int MT> constexpr int stream_threads() { return stream_ask<EPI, MT>() ? 512 : 256; }
 
 // N 16-row fragments (two 32-element chunks of k) at base + STRIDE i; waits for them
 template <int N, int STRIDE>
@@ -335,8 +336,11 @@ __device__ __forceinline__ cf32x4 unpark(const float* p) {
 }
 
 template <int DT, int EPI, int MT, bool GRP>
-__global__ __launch_bounds__((StreamShape<MT, stream_wide<EPI, MT>()>::THREADS), 2) void gemm_stream_kernel(GemmArgs g) {
+__global__ __launch_bounds__((stream_threads<EPI, MT>()),
+                             (stream_ask<EPI, MT>() ? StreamShape<MT, stream_wide<EPI, MT>()>::WGS / 128 : 2))
+    void gemm_stream_kernel(GemmArgs g) {
   using S = StreamShape<MT, stream_wide<EPI, MT>()>;
+  constexpr bool ASK = stream_ask<EPI, MT>();
   constexpr int NWV = S::NWV, RT = S::RT, KC = S::KC, KST = S::KST;
   __shared__ __attribute__((aligned(16))) uint8_t smem[S::NS * S::STAGE];
   __shared__ unsigned last;
@@ -426,12 +430,12 @@ __global__ __launch_bounds__((StreamShape<MT, stream_wide<EPI, MT>()>::THREADS),
     asm volatile("s_barrier" ::: "memory");
     stage(buf == 0 ? S::NS - 1 : buf - 1);
   };
-  if (!S::ASK || who >= NWV) {
+  if (!ASK || who >= NWV) {
     aim(ds);
 #pragma unroll
     for (int p = 0; p < S::NS - 1; ++p) stage(p);
   }
-  if (S::ASK && who >= NWV) {
+  if (ASK && who >= NWV) {
     int buf = 0;
     for (int u = u0; u < u1; ++u) {
       feed(buf);
@@ -454,7 +458,7 @@ __global__ __launch_bounds__((StreamShape<MT, stream_wide<EPI, MT>()>::THREADS),
 #pragma unroll
       for (int i = 0; i < MT; ++i) acc[j][i] = cf32x4{0.f, 0.f, 0.f, 0.f};
     for (; u < seg1; ++u) {
-      if constexpr (S::ASK) asm volatile("s_barrier" ::: "memory");
+      if constexpr (ASK) asm volatile("s_barrier" ::: "memory");
       else feed(buf);
       const uint32_t b = buf * S::STAGE;
       constexpr int XR = MT % 2 ? 1 : 2, T16 = 2048 * KC;   // bytes of 16 rows
@@ -496,9 +500,9 @@ __global__ __launch_bounds__((StreamShape<MT, stream_wide<EPI, MT>()>::THREADS),
           if (i * 16 + (lane & 15) < t.M) park(p + (j * MT + i) * 256, acc[j][i]);
       __builtin_amdgcn_s_waitcnt(vm_wait(0));
       // (the waves of a workgroup that asks and multiplies in turn arrive as one)
-      unsigned* tick = g.tick + s * NWV + (S::ASK ? wave : 0);
+      unsigned* tick = g.tick + s * NWV + (ASK ? wave : 0);
       unsigned before = 0;
-      if constexpr (S::ASK) {
+      if constexpr (ASK) {
         asm volatile("" ::: "memory");
         if (lane == 0) before = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("" ::: "memory");
@@ -510,7 +514,7 @@ __global__ __launch_bounds__((StreamShape<MT, stream_wide<EPI, MT>()>::THREADS),
       }
       mine = __builtin_amdgcn_readfirstlane(before) == (unsigned)(hi - lo);
       if (mine) {
-        if (S::ASK ? lane == 0 : tid == 0) __hip_atomic_store(tick, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (ASK ? lane == 0 : tid == 0) __hip_atomic_store(tick, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // in share order (the result does not hang on who came last), several shares in flight
         constexpr int UN = MT <= 2 ? 8 : 4;
         for (int w0 = lo; w0 <= hi; w0 += UN) {
@@ -535,13 +539,13 @@ __global__ __launch_bounds__((StreamShape<MT, stream_wide<EPI, MT>()>::THREADS),
               }
         }
       }
-      if constexpr (!S::ASK) __syncthreads();   // `last` is read
+      if constexpr (!ASK) __syncthreads();   // `last` is read
     }
     if (mine) stream_store<DT, EPI, MT, RT>(g, t, wave, lane, acc);
     // stores count with the DMA: drain them before the counted waits go on
-    if (!S::ASK && u < u1) __builtin_amdgcn_s_waitcnt(vm_wait(0));
+    if (!ASK && u < u1) __builtin_amdgcn_s_waitcnt(vm_wait(0));
   }
-  if constexpr (!S::ASK) __builtin_amdgcn_s_waitcnt(vm_wait(0));
+  if constexpr (!ASK) __builtin_amdgcn_s_waitcnt(vm_wait(0));
 }
 
 template <int DT, int EPI>
@@ -549,7 +553,7 @@ int launch_stream(int mt, dim3 grid, hipStream_t st, const GemmArgs& g) {
 #define CAKE_STREAM(MT)                                                                             \
   if (mt == MT) {                                                                                   \
     hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI, MT, false>), grid,                              \
-                       dim3(StreamShape<MT, stream_wide<EPI, MT>()>::THREADS), 0, st, g);           \
+                       dim3(stream_threads<EPI, MT>()), 0, st, g);                                  \
     return (int)hipGetLastError();                                                                  \
   }
   CAKE_STREAM(1) CAKE_STREAM(2) CAKE_STREAM(3) CAKE_STREAM(4)
@@ -591,7 +595,7 @@ template <int DT> struct Rows {
 #define X(E)                                                                                  \
   case E:                                                                                     \
     hipLaunchKernelGGL((gemm_stream_kernel<DT, E, 1, true>), grid,                            \
-                       dim3(StreamShape<1, stream_wide<E, 1>()>::THREADS), 0, st, g);         \
+                       dim3(stream_threads<E, 1>()), 0, st, g);                               \
     return (int)hipGetLastError();
       X(kEpiStore) X(kEpiSilu) X(kEpiQuick) X(kEpiGelu) X(kEpiRelu2)
 #undef X
