@@ -232,7 +232,9 @@ static constexpr TileCost kTileCosts[] = {
     {37, 160, 128, 1, 0.744f, 0.511f, 0.032f, 0.f, 0.163f, {5.184f, 7.988f, 4.123f, 7.683f, -1.f, -1.f, -1.f}, 3.312f, 3.9f},
     {38, 224, 128, 1, 0.259f, 0.64f, 0.017f, 0.f, 0.162f, {6.65f, 10.33f, 5.431f, 11.4f, -1.f, -1.f, -1.f}, 1.852f, 3.237f},
     // f32 results on the tiles of gemm_ws.h, of 180 products (2048 .. 8192 columns, k 4096 .. 28672, 100 .. 6000 rows):
-    // 0.3 % off the best of all, 2.5 % faster than without them on the average, 5 to 16 % from 1300 rows on
+    // 0.3 % off the best of all, 2.5 % faster than without them on the average, 5 to 16 % from 1300 rows on.  Of 170 others (1024
+    // .. 12288 columns, k 2048 .. 28672, 700 .. 8192 rows) 3.5 % faster, at most 5 % slower (12288 x 4096 at 1665 and 2600 rows
+    // 147 and 231 us on 224 x 192, 155 and 243).  22 and 25 are one kernel there; either id may be a plan's
     {22, 256, 256, 1, 7.023f, 1.101f, 0.0578f, -0.3914f, 0.1106f, {-1.f, 12.87f, -1.f, -1.f, -1.f, -1.f, -1.f}, 1.22f, 5.201f},
     {25, 256, 256, 1, 7.023f, 1.101f, 0.0578f, -0.3914f, 0.1106f, {-1.f, 12.87f, -1.f, -1.f, -1.f, -1.f, -1.f}, 1.22f, 5.201f},
     {34, 192, 256, 1, 6.121f, 0.9357f, 0.0341f, -0.3562f, 0.1039f, {-1.f, 1.538f, -1.f, -1.f, -1.f, -1.f, -1.f}, 3.788f, 5.132f},
@@ -423,8 +425,11 @@ CAKE_API int cake_gemm(int dt, int epi, int cfg, int splits, const void* a, long
 // ---- products of few rows (gemm_rows.h) -----------------------------------
 // Which form a product of M rows takes: 0 the tile kernels (cake_gemm_scaled), 1 direct, 2 stream.
 // The estimates (us) are fits to timings on weights that no cache holds, 2 .. 64 rows of 80 weight
-// shapes, 0.2 .. 940 MB, every form and share; wrong choices weighed more than wrong times: what they pick
-// is 0.4 % off the best of all on the average, at most 16 %.  Both sides of the lines they draw, measured:
+// shapes, 0.2 .. 940 MB, every form and share; wrong choices weighed more than wrong times: what they picked
+// was 0.4 % off the best of all on the average, at most 16 %.  The stream form was one of four waves in turn then; its
+// 128-row strips are 1 - 8 % faster since (gemm_rows.h) and not fitted again.  Of 35 narrow shapes (256 .. 3072 columns, k 2048
+// .. 28672) at 2 .. 16 rows they are 1.5 % off now, at most 19 (1024 x 8960, where 64 x 64 tiles in splits are the best, 11.2
+// for 13.3 us).  Both sides of the lines they draw, measured:
 // 3072 x 2048 at 5 rows direct 6.7, stream 8.4; 4096 x 4096 at 5 rows 10.3, 11.5, at 16 12.4, 11.7 (tiles
 // 12.1), at 24 tiles 12.4, stream 15.0; 4096 x 14336 at 24 rows stream 26.6, tiles 27.5, at 33 30.1, 27.8;
 // 6144 x 4096 at 16 rows stream 14.3, tiles 15.7, at 33 18.3, 16.7; 8192 x 8192 at 24 rows stream 29.6,
@@ -558,8 +563,8 @@ CAKE_API int cake_gemm_rows(int dt, int epi, int kind, const void* a, long long 
 // ---- products that leave their sums in slabs ------------------------------
 // Which form such a product takes, and whether the launch that follows it gains from summing them
 // (gemm_slabs.hip).  The estimates (us) are fits to timings of product and norm or rotation on weights that no
-// cache holds, 2 .. 64 rows of 33 shapes, 2 .. 470 MB, every form: what they pick is 0.35 % off the best on the
-// average, at most 11 %.  The two launches take 0.9 of the three or two they replace at 2 .. 16 rows (4096 x
+// cache holds, 2 .. 64 rows of 33 shapes, 2 .. 470 MB, every form: what they picked was 0.35 % off the best on the
+// average, at most 11 % (the stream form as above).  The two launches take 0.9 of the three or two they replace at 2 .. 16 rows (4096 x
 // 14336 and norm at 5 rows 26.6 -> 25.0 us), 0.87 at 24 .. 64 (at 45 rows 32.6 -> 30.2, 4096 x 4096 16.0 ->
 // 13.9, 6144 x 4096 and rotation 20.3 -> 18.3, 10240 x 8192 44.4 -> 37.7, 4096 x 23552 48.5 -> 42.6).
 struct SlabStream { double c0, cu, step, rate, slab, mid; };   // by 16-row tiles of x

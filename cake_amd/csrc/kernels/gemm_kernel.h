@@ -75,7 +75,7 @@ struct GemmArgs {
   // in ws, the last sums them in piece order and runs the epilogue; tick = [kPieceTiles arrival
   // counters | kPieceTiles ready counters] (gemm_ws.h: of each of a tile's eight waves)
   int pieces;
-  unsigned* tick;        // (gemm_rows.h: one arrival counter per strip)
+  unsigned* tick;        // (gemm_rows.h: four arrival counters a strip, one of a wave each or the first of them)
   int dp_tiles;
   // grouped products (gemm_inst_grouped.hip): row tile tm is [weight group, first row, rows, -]
   // of this list instead of rows tm BM .., its weights b + group b_group; entry tiles_m holds

@@ -3,9 +3,9 @@
 // Included by gemm_kernel.h; same GemmArgs, LDS image and epilogues as gemm_4w.h.
 //
 // Twelve waves, three on each SIMD: eight compute (2 x 4 of a tile, two a SIMD, so that one's LDS reads hide behind the
-// other's MFMAs), four ask for operands (LDS-DMA).  A CU has some 20 KB of loads under way, whatever it asks for: a step
-// takes its bytes times their latency (330 clocks from the L2, 1600 from the memory) / 20 KB at least, 1620 clocks on
-// 192 x 192 where the MFMAs are 1152, and a wave that asks for more stands still at that instruction with everything behind
+// other's MFMAs), four ask for operands (LDS-DMA).  A CU seems to have some 20 KB of loads under way, whatever it asks
+// for (an estimate from such kernels' times, no counter shows it): a step would take its bytes times their latency (330
+// clocks from the L2, 1600 from the memory) / 20 KB, 1620 clocks on 192 x 192 where the MFMAs are 1152, and a wave that asks for more stands still at that instruction with everything behind
 // it.  So large tiles, whose bytes the MFMAs cover, and the standing still left to waves that do nothing else (64 experts
 // 4096 x 3648 at 150 rows: MFMAs alone 190 us, weights alone 300, one after the other 425 on the four waves of gemm_4w.h,
 // 358 here).  192 x 256 is 144 KB of LDS and 168 registers a wave, 96 of them sums.

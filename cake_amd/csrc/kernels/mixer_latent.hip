@@ -240,9 +240,9 @@ __device__ __forceinline__ uint4 load_cols(const uint16_t* rows, int ld, int l15
   return make_uint4(a.x, a.y, b.x, b.y);
 }
 
-// RC: class of the latent size, BK: keys per tile
 // 16-byte pieces of a tile per thread
 template <int DT, int RC, int BK> constexpr int lat_pieces() { return DT != kF32 && RC <= 512 && BK == 32 ? 10 : 20; }
+// RC: class of the latent size, BK: keys per tile
 template <int DT, int RC, int BK>
 __global__ __launch_bounds__(256) void latent_decode_kernel(LatDecArgs a) {
   using E = typename St<DT>::E;

@@ -1,4 +1,5 @@
-"""Routed products whose tile height is chosen on the device (mixer_experts.hip, gemm_inst_grouped.hip)."""
+"""Routed products whose tile height is chosen on the device (mixer_experts.hip, gemm_inst_grouped.hip): both k short, on the
+four-wave tiles; long ones are in test_gemm_ws_gpu.py."""
 import pytest
 import torch
 

@@ -1,4 +1,5 @@
-"""Grouped products in tiles of 160 and 192 rows, and of 128 on one barrier a step (gemm_inst_grouped.hip)."""
+"""Grouped products by tile heights (gemm_inst_grouped.hip): rows of up to 1024 columns, on the four-wave tiles of gemm_4w.h,
+and some of more, on those of gemm_ws.h (which have their own tests too)."""
 import pytest
 import torch
 
@@ -35,7 +36,7 @@ def test_tile_heights(cuda, cfg, N, K, ld):
 @pytest.mark.parametrize("cfg", [0, 1, 2, 5, 6])
 @pytest.mark.parametrize("epi", ["silu", "relu2"])
 def test_activations_of_every_height(cuda, dt, cfg, epi):
-    """As routed experts run them, 16-bit types and activations; configuration 6 by the list's height.  One
+    """Short rows, the four-wave tiles: 16-bit types and activations; configuration 6 by the list's height.  One
     rounding (2^-8, 2^-11) of f32 sums, the activation's own 2^-10."""
     from cake_amd.ops import gemm as G
     N, K = 300, 200
